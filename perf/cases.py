@@ -113,7 +113,8 @@ def draw(rng):
         return {"kind": kind, "batch": batch, "channels": channels, "inner": inner, "over": over,
                 "op": rng.choice(["sum", "mean", "max"]), "dtype": dt}
     if kind == "dropout_norm":
-        cols = _width(rng, 512, 8192, 0.2)
+        # the dropout interface takes hidden sizes that are multiples of 8
+        cols = _width(rng, 512, 8192, 0.2) // 8 * 8
         return {"kind": kind, "rows": _rows(rng, 64, 16384, cols, 16384 * 4096, dt), "cols": cols, "dtype": dt}
     channels = _between(rng, 3, 1024)
     side = _between(rng, 4, 112)
