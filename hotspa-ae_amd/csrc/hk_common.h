@@ -200,6 +200,57 @@ __device__ __forceinline__ void buf_st16(BufferRsrc r, uint32_t byte_offset, con
   __builtin_amdgcn_raw_buffer_store_b128(v, r, int(byte_offset), 0, POLICY);
 }
 
+// Rows of any length at any element boundary ("ragged": cols is no multiple of the vector width, or a row does not
+// start on a 16-byte boundary).  A 16-byte access needs no more than the element's own alignment here, and costs
+// little: rows of 8190 bf16 elements (4-byte aligned) are read at the aligned rate (7.1 TB/s), rows of 8191 (2-byte
+// aligned) at 5.5 TB/s; read and written 5.9 / 5.3 TB/s against 6.2 aligned and 5.5 with the ends peeled off and the
+// middle aligned.  Vector v of such a row covers columns [v * N, v * N + N) as always; the last, partial one is loaded
+// as the row's LAST N elements, so every load is a whole vector inside the row: its first elements belong to the
+// vector before it and take no part in sums.  Rows shorter than a vector have no such load and stay with the
+// element-wise kernels.
+typedef u32x4 u32x4_on2 __attribute__((aligned(2)));
+typedef u32x4 u32x4_on4 __attribute__((aligned(4)));
+template <typename T> struct AnyBoundary {
+  using vec = typename std::conditional<sizeof(T) == 2, u32x4_on2, u32x4_on4>::type;
+};
+template <typename T>
+__device__ __forceinline__ u32x4 ld16_any(const T* p) {
+  return __builtin_nontemporal_load(reinterpret_cast<const typename AnyBoundary<T>::vec*>(p));
+}
+template <typename T>
+__device__ __forceinline__ u32x4 ld16_any_keep(const T* p) {
+  return *reinterpret_cast<const typename AnyBoundary<T>::vec*>(p);
+}
+template <typename T>
+__device__ __forceinline__ void st16_any(T* p, const u32x4& v) {
+  __builtin_nontemporal_store(v, reinterpret_cast<typename AnyBoundary<T>::vec*>(p));
+}
+// first column that vector v loads
+template <typename T, bool RAGGED>
+__device__ __forceinline__ int vec_column(int v, int cols) {
+  constexpr int N = VecIO<T>::N;
+  if constexpr (!RAGGED) return v * N;
+  return v * N + N <= cols ? v * N : cols - N;
+}
+// Stores vector v of a row.  SAME: an element that two vectors hold was computed to the same bits in both, so the
+// partial vector is stored whole over its neighbour's end; otherwise its own elements go out one by one.
+template <typename T, bool RAGGED, bool SAME>
+__device__ __forceinline__ void store_row_vec(T* row, int v, const float* f, int cols) {
+  constexpr int N = VecIO<T>::N;
+  if constexpr (!RAGGED) {
+    __builtin_nontemporal_store(VecIO<T>::pack(f), reinterpret_cast<u32x4*>(row + v * N));
+  } else if constexpr (SAME) {
+    st16_any(row + vec_column<T, true>(v, cols), VecIO<T>::pack(f));
+  } else if (v * N + N <= cols) {
+    st16_any(row + v * N, VecIO<T>::pack(f));
+  } else if (v * N < cols) {
+    const int skip = v * N + N - cols;
+#pragma unroll
+    for (int j = 1; j < N; ++j)
+      if (j >= skip) Cvt<T>::store(row + cols - N + j, f[j]);
+  }
+}
+
 __device__ __forceinline__ u32x4 ld16_stream(const void* p) {
   return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
 }
@@ -348,6 +399,37 @@ __device__ __forceinline__ P wave_allreduce_tuple(P a) {
   return P::merge(P::merge(r[0], r[1]), P::merge(r[2], r[3]));
 }
 
+// the same over groups of LPR neighbouring lanes (8, 16, 32 or the whole wavefront), each with a result of its own
+template <int LPR, typename P>
+__device__ __forceinline__ P lanes_allreduce_tuple(P a) {
+  static_assert(LPR == 8 || LPR == 16 || LPR == 32 || LPR == kWave, "group widths with a DPP butterfly");
+  if constexpr (LPR == kWave) {
+    return wave_allreduce_tuple<P>(a);
+  } else {
+    P b;
+#pragma unroll
+    for (int k = 0; k < P::K; ++k) b.v[k] = dpp_perm<kDppXor1>(a.v[k]);
+    a = P::merge(a, b);
+#pragma unroll
+    for (int k = 0; k < P::K; ++k) b.v[k] = dpp_perm<kDppXor2>(a.v[k]);
+    a = P::merge(a, b);
+#pragma unroll
+    for (int k = 0; k < P::K; ++k) b.v[k] = dpp_perm<kDppHalfMirror>(a.v[k]);
+    a = P::merge(a, b);
+    if constexpr (LPR >= 16) {
+#pragma unroll
+      for (int k = 0; k < P::K; ++k) b.v[k] = dpp_perm<kDppMirror>(a.v[k]);
+      a = P::merge(a, b);
+    }
+    if constexpr (LPR == 32) {
+#pragma unroll
+      for (int k = 0; k < P::K; ++k) b.v[k] = lane_xor<16>(a.v[k]);
+      a = P::merge(a, b);
+    }
+    return a;
+  }
+}
+
 // the cross-wave half of group_allreduce_tuple: `a` is already the same in every lane of a wave
 template <typename P>
 __device__ __forceinline__ P group_combine_tuple(P a, float* scratch, int first_wave, int nwaves);
@@ -435,6 +517,15 @@ struct SumTuple {
 #pragma unroll
     for (int k = 0; k < KK; ++k) a.v[k] += b.v[k];
     return a;
+  }
+};
+
+// a maximum
+struct MaxTuple {
+  static constexpr int K = 1;
+  float v[1];
+  static __device__ __forceinline__ MaxTuple merge(const MaxTuple& a, const MaxTuple& b) {
+    return MaxTuple{{fmaxf(a.v[0], b.v[0])}};
   }
 };
 

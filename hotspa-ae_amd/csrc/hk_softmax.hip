@@ -1,10 +1,11 @@
 // Softmax forward / backward for gfx950.
 //
-// Last-dimension softmax keeps the row in registers (one HBM read, one write):
-// every thread folds its elements into a (max, sum-of-exp) pair, the pairs are
-// merged online across lanes (DPP) and waves (LDS), and the stored exponentials
-// are rescaled on the way out, so exp is evaluated once per element.
-// One wavefront per row for short rows, one workgroup per row for long rows.
+// Last-dimension softmax keeps the row in registers (one HBM read, one write), whatever its length and alignment:
+// lanes of one wavefront agree on the row's maximum and then its sum (DPP); where a row takes a workgroup, every
+// thread folds its elements into a (max, sum-of-exp) pair and the pairs are merged online across wavefronts (LDS).
+// The stored exponentials are rescaled on the way out, so exp is evaluated once per element.
+// Bound by HBM: what a row costs is its bytes and, for ragged rows, the extra cache lines of misaligned accesses
+// (192 x 577 x 577 bf16, forward + backward: 508 us with element-wise passes, 118 us so).
 #include "hk_common.h"
 
 #include <algorithm>
@@ -26,26 +27,44 @@ struct SoftmaxArgs {
   int nvec;
 };
 
-template <typename T, int NV, bool WAVE_ROW>
-__global__ __launch_bounds__(WAVE_ROW ? 256 : 1024)
+// Which lanes hold a row.  LPR > 0: LPR neighbouring lanes of a wavefront (8, 16, 32 or all 64), 256 / LPR rows per
+// workgroup; LPR == 0: the whole workgroup.
+template <int LPR>
+struct RowLanes {
+  static __device__ __forceinline__ int count() { return LPR ? LPR : int(blockDim.x); }
+  static __device__ __forceinline__ int lane() { return LPR ? int(threadIdx.x) & (LPR - 1) : int(threadIdx.x); }
+  static __device__ __forceinline__ int64_t row() {
+    if constexpr (LPR == 0) return int64_t(blockIdx.x);
+    else if constexpr (LPR == kWave) return int64_t(blockIdx.x) * (256 / kWave) + wave_index();
+    else return int64_t(blockIdx.x) * (256 / LPR) + int(threadIdx.x) / LPR;
+  }
+  template <typename P>
+  static __device__ __forceinline__ P allreduce(P p, float* red) {
+    if constexpr (LPR == 0) return group_allreduce_tuple(p, red, 0, int(blockDim.x >> 6));
+    else return lanes_allreduce_tuple<LPR>(p);
+  }
+};
+
+template <typename T, int NV, int LPR, bool RAGGED>
+__global__ __launch_bounds__(LPR ? 256 : 1024)
 void softmax_fwd_kernel(SoftmaxArgs a) {
   constexpr int VEC = VecIO<T>::N;
+  using Lanes = RowLanes<LPR>;
   __shared__ float red[kMaxWaves * 2];
-  const int tpr = WAVE_ROW ? kWave : int(blockDim.x);
-  const int t = WAVE_ROW ? int(threadIdx.x & 63) : int(threadIdx.x);
-  const int64_t row = WAVE_ROW
-      ? int64_t(blockIdx.x) * (blockDim.x >> 6) + wave_index()
-      : int64_t(blockIdx.x);
-  if (WAVE_ROW && row >= a.n0) return;   // row counts within the innermost level
-  const int nwaves = WAVE_ROW ? 1 : int(blockDim.x >> 6);
+  const int tpr = Lanes::count(), t = Lanes::lane();
+  const int64_t row = Lanes::row();
+  if (LPR && row >= a.n0) return;   // row counts within the innermost level
 
   const T* xr = static_cast<const T*>(a.x) + row * a.x_pitch + outer_level_offset(a.x_lv);
-  // slots past the row's end hold -inf: they change neither the maximum nor the sum
+  // slots past the row's end hold -inf, which changes neither the maximum nor the sum; in a ragged row they hold
+  // elements of the row a second time, which the maximum may see and the sum leaves out
   u32x4 raw[NV];
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
     const int v = i * tpr + t;
-    if ((i + 1) * tpr <= a.nvec) {       // uniform: every thread's slot i is inside the row
+    if constexpr (RAGGED) {
+      raw[i] = ld16_any<T>(xr + vec_column<T, true>(v, a.cols));
+    } else if ((i + 1) * tpr <= a.nvec) {       // uniform: every thread's slot i is inside the row
       raw[i] = ld16(xr + v * VEC);
     } else {
       raw[i] = neg_inf_vec<T>();
@@ -59,19 +78,33 @@ void softmax_fwd_kernel(SoftmaxArgs a) {
   float m = fmaxf(e[0], e[1]);
 #pragma unroll
   for (int k = 2; k < NV * VEC; k += 2) m = max3(m, e[k], e[k + 1]);
-  // ml: this thread's maximum in the log2 domain, rounded once (see OnlineSoftmaxTuple)
+  // ml: the maximum in the log2 domain, rounded once (see OnlineSoftmaxTuple).  Lanes of one wavefront agree on the
+  // row's maximum first: its butterfly is cheaper than merging (maximum, sum) pairs, whose every step takes two
+  // exponentials, and an element held twice then comes out the same twice.  Across wavefronts each thread keeps its
+  // own maximum and the pairs are merged, which costs one barrier instead of two.
+  if constexpr (LPR > 0) m = Lanes::allreduce(MaxTuple{{m}}, red).v[0];
   const float ml = (m == kNegInf) ? 0.f : m * kLog2e;
   float s = 0.f;
 #pragma unroll
-  for (int k = 0; k < NV * VEC; ++k) {
-    e[k] = __builtin_amdgcn_exp2f(fmaf(e[k], kLog2e, -ml));
-    s += e[k];
+  for (int i = 0; i < NV; ++i) {
+    [[maybe_unused]] const int skip = (i * tpr + t + 1) * VEC - a.cols;   // elements of earlier vectors (ragged)
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) {
+      float& x = e[i * VEC + j];
+      x = __builtin_amdgcn_exp2f(fmaf(x, kLog2e, -ml));
+      s += (RAGGED && j < skip) ? 0.f : x;
+    }
   }
-  MaxSumTuple p;
-  p.v[0] = (m == kNegInf) ? kNegInf : ml; p.v[1] = s;
-  p = WAVE_ROW ? wave_allreduce_tuple(p) : group_allreduce_tuple(p, red, 0, nwaves);
-  const float ML = (p.v[0] == kNegInf) ? 0.f : p.v[0];
-  const float scale = __builtin_amdgcn_exp2f(ml - ML) / p.v[1];
+  float scale;
+  if constexpr (LPR > 0) {
+    scale = 1.0f / Lanes::allreduce(SumTuple<1>{{s}}, red).v[0];
+  } else {
+    MaxSumTuple p;
+    p.v[0] = (m == kNegInf) ? kNegInf : ml; p.v[1] = s;
+    p = Lanes::allreduce(p, red);
+    const float ML = (p.v[0] == kNegInf) ? 0.f : p.v[0];
+    scale = __builtin_amdgcn_exp2f(ml - ML) / p.v[1];
+  }
 
   T* yr = static_cast<T*>(a.out) + row * a.out_pitch + outer_level_offset(a.out_lv);
 #pragma unroll
@@ -80,24 +113,20 @@ void softmax_fwd_kernel(SoftmaxArgs a) {
     if (v < a.nvec) {
 #pragma unroll
       for (int j = 0; j < VEC; ++j) e[i * VEC + j] *= scale;
-      const u32x4 o = VecIO<T>::pack(&e[i * VEC]);
-      st16_stream(yr + v * VEC, o);
+      store_row_vec<T, RAGGED, (LPR > 0)>(yr, v, &e[i * VEC], a.cols);
     }
   }
 }
 
-template <typename T, int NV, bool WAVE_ROW>
-__global__ __launch_bounds__(WAVE_ROW ? 256 : 1024)
+template <typename T, int NV, int LPR, bool RAGGED>
+__global__ __launch_bounds__(LPR ? 256 : 1024)
 void softmax_bwd_kernel(SoftmaxArgs a) {
   constexpr int VEC = VecIO<T>::N;
+  using Lanes = RowLanes<LPR>;
   __shared__ float red[kMaxWaves];
-  const int tpr = WAVE_ROW ? kWave : int(blockDim.x);
-  const int t = WAVE_ROW ? int(threadIdx.x & 63) : int(threadIdx.x);
-  const int64_t row = WAVE_ROW
-      ? int64_t(blockIdx.x) * (blockDim.x >> 6) + wave_index()
-      : int64_t(blockIdx.x);
-  if (WAVE_ROW && row >= a.n0) return;   // row counts within the innermost level
-  const int nwaves = WAVE_ROW ? 1 : int(blockDim.x >> 6);
+  const int tpr = Lanes::count(), t = Lanes::lane();
+  const int64_t row = Lanes::row();
+  if (LPR && row >= a.n0) return;   // row counts within the innermost level
 
   const T* yr = static_cast<const T*>(a.x) + row * a.x_pitch + outer_level_offset(a.x_lv);
   const T* dyr = static_cast<const T*>(a.dy) + row * a.dy_pitch + outer_level_offset(a.dy_lv);
@@ -105,9 +134,15 @@ void softmax_bwd_kernel(SoftmaxArgs a) {
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
     const int v = i * tpr + t;
-    ry[i] = u32x4{0, 0, 0, 0};
-    rdy[i] = u32x4{0, 0, 0, 0};
-    if (v < a.nvec) { ry[i] = ld16(yr + v * VEC); rdy[i] = ld16(dyr + v * VEC); }
+    if constexpr (RAGGED) {
+      const int c = vec_column<T, true>(v, a.cols);
+      ry[i] = ld16_any<T>(yr + c);
+      rdy[i] = ld16_any<T>(dyr + c);
+    } else {
+      ry[i] = u32x4{0, 0, 0, 0};
+      rdy[i] = u32x4{0, 0, 0, 0};
+      if (v < a.nvec) { ry[i] = ld16(yr + v * VEC); rdy[i] = ld16(dyr + v * VEC); }
+    }
   }
   SumTuple<1> s;
   s.v[0] = 0.f;
@@ -116,10 +151,14 @@ void softmax_bwd_kernel(SoftmaxArgs a) {
     float y[VEC], d[VEC];
     VecIO<T>::unpack(ry[i], y);
     VecIO<T>::unpack(rdy[i], d);
+    [[maybe_unused]] const int skip = (i * tpr + t + 1) * VEC - a.cols;
 #pragma unroll
-    for (int j = 0; j < VEC; ++j) s.v[0] = fmaf(y[j], d[j], s.v[0]);  // padding is zero
+    for (int j = 0; j < VEC; ++j) {
+      if constexpr (RAGGED) s.v[0] = j < skip ? s.v[0] : fmaf(y[j], d[j], s.v[0]);
+      else s.v[0] = fmaf(y[j], d[j], s.v[0]);   // padding is zero
+    }
   }
-  s = WAVE_ROW ? wave_allreduce_tuple(s) : group_allreduce_tuple(s, red, 0, nwaves);
+  s = Lanes::allreduce(s, red);
   const float dot = s.v[0];
   T* dxr = static_cast<T*>(a.out) + row * a.out_pitch + outer_level_offset(a.out_lv);
 #pragma unroll
@@ -131,8 +170,7 @@ void softmax_bwd_kernel(SoftmaxArgs a) {
       VecIO<T>::unpack(rdy[i], d);
 #pragma unroll
       for (int j = 0; j < VEC; ++j) d[j] = y[j] * (d[j] - dot);
-      const u32x4 o = VecIO<T>::pack(d);
-      st16_stream(dxr + v * VEC, o);
+      store_row_vec<T, RAGGED, true>(dxr, v, d, a.cols);
     }
   }
 }
@@ -246,9 +284,18 @@ static inline int pow2_ceil_sm(int v) {
   return p;
 }
 
-// threads per row / vectors per thread for a row of nvec 16-byte vectors
-static bool pick_softmax_shape(int nvec, int max_nv_wave, int max_nv, bool bwd, int* threads, int* nv) {
+// lanes per row (threads of a workgroup per row when above 64) / vectors per lane for a row of nvec 16-byte vectors
+// (aligned: whole vectors on 16-byte boundaries; odd: rows on odd 2-byte boundaries)
+static bool pick_softmax_shape(int nvec, bool aligned, bool odd, int max_nv, bool bwd, int* threads, int* nv) {
   const int forced = tune_get(TUNE_SOFTMAX_THREADS);
+  // measured on MI355X at 2048 bf16 columns: forward is fastest with two
+  // vectors per thread (128 threads per row), backward with one (256 threads)
+  const int want = bwd ? 1 : 2;
+  if (forced > 0 && forced <= 64) {
+    *threads = forced;
+    *nv = (nvec + forced - 1) / forced;
+    return (forced == 8 || forced == 16 || forced == 32 || forced == 64) && *nv <= 4;
+  }
   if (forced > 0) {
     int t = std::min(1024, std::max(64, (forced + 63) / 64 * 64));
     int n = pow2_ceil_sm((nvec + t - 1) / t);
@@ -256,13 +303,28 @@ static bool pick_softmax_shape(int nvec, int max_nv_wave, int max_nv, bool bwd, 
     *threads = t; *nv = n;
     return true;
   }
-  // measured on MI355X at 2048 bf16 columns: forward is fastest with two
-  // vectors per thread (128 threads per row), backward with one (256 threads)
-  const int want = bwd ? 1 : 2;
-  if (nvec <= 64 * want) {
+  const bool whole_lines = aligned && nvec % 8 == 0;
+  // Short rows share a wavefront: one to itself leaves most lanes of a short row idle, and the launch is then bound by
+  // waves, not bytes.  Measured on arrays of 600 MB, bf16, forward / backward GB/s, one row per wavefront -> this
+  // choice: 32 columns 680 / 1055 -> 4710 / 5150, 64: 1300 / 1990 -> 6500 / 6490, 128: 2390 / 3720 -> 6540 / 6470,
+  // 256: 4440 / 5070 -> 6390 / 6490, 512: 6440 / 6440 -> 6380 / 6440.  What decides between the shapes:
+  //  - the backward streams best with one vector of each operand per lane (1024 columns, 128 lanes x 1: 6560, 64 x 2:
+  //    6180; 256 columns, 32 x 1: 6490, 16 x 2: 6200), the forward with two as long as no lane idles;
+  //  - two vectors in half the lanes cover a short row forward only where it ends on a 128-byte line (200 columns
+  //    5220 as 16 x 2, 5720 as 32 x 1);
+  //  - rows on odd 2-byte boundaries, whose every access straddles lines, want a wavefront of their own up to 256
+  //    vectors (2047 columns 5550 / 5950 against 5470 / 5410 with a workgroup); other backward rows do only where a
+  //    workgroup of one vector per lane would leave two fifths of its lanes idle (300 fp32 columns 6110 against 5400).
+  if (nvec <= 64) {
+    *threads = nvec <= 8 ? 8 : (nvec <= 16 || (nvec <= 32 && whole_lines && !bwd)) ? 16
+             : (nvec <= 40 || !bwd) ? 32 : 64;
+    *nv = (nvec + *threads - 1) / *threads;
+    return true;
+  }
+  if (nvec <= (odd ? 256 : bwd ? 76 : 192)) {
     *threads = 64;
-    *nv = pow2_ceil_sm((nvec + 63) / 64);
-    return *nv <= max_nv_wave;
+    *nv = (nvec + 63) / 64;
+    return true;
   }
   for (int n = want; n <= max_nv; n <<= 1) {
     int t = ((nvec + n - 1) / n + 63) / 64 * 64;
@@ -271,20 +333,38 @@ static bool pick_softmax_shape(int nvec, int max_nv_wave, int max_nv, bool bwd, 
   return false;
 }
 
-template <typename T, bool BWD, bool WAVE_ROW>
+template <typename T, bool BWD, int LPR, bool RAGGED>
 static int launch_softmax_nv(const SoftmaxArgs& a, int nv, dim3 grid, dim3 block, hipStream_t s) {
 #define HK_SM_CASE(N)                                                                      \
   case N:                                                                                  \
-    if constexpr (BWD) HK_LAUNCH((softmax_bwd_kernel<T, N, WAVE_ROW>), grid, block, 0, s, a); \
-    else HK_LAUNCH((softmax_fwd_kernel<T, N, WAVE_ROW>), grid, block, 0, s, a);   \
+    if constexpr (BWD) HK_LAUNCH((softmax_bwd_kernel<T, N, LPR, RAGGED>), grid, block, 0, s, a); \
+    else HK_LAUNCH((softmax_fwd_kernel<T, N, LPR, RAGGED>), grid, block, 0, s, a);   \
     break;
   profile_before(s);
   switch (nv) {
-    HK_SM_CASE(1) HK_SM_CASE(2) HK_SM_CASE(4) HK_SM_CASE(8)
-    case 16:
-      if constexpr (VecIO<T>::N == 4 && !BWD) {
-        HK_LAUNCH((softmax_fwd_kernel<T, 16, WAVE_ROW>), grid, block, 0, s, a);
+    HK_SM_CASE(1) HK_SM_CASE(2) HK_SM_CASE(4)
+    case 3:
+      if constexpr (LPR > 0) {
+        if constexpr (BWD) HK_LAUNCH((softmax_bwd_kernel<T, 3, LPR, RAGGED>), grid, block, 0, s, a);
+        else HK_LAUNCH((softmax_fwd_kernel<T, 3, LPR, RAGGED>), grid, block, 0, s, a);
         break;
+      }
+      [[fallthrough]];
+    case 8:
+      if constexpr (LPR == 0) {
+        if (nv == 8) {
+          if constexpr (BWD) HK_LAUNCH((softmax_bwd_kernel<T, 8, LPR, RAGGED>), grid, block, 0, s, a);
+          else HK_LAUNCH((softmax_fwd_kernel<T, 8, LPR, RAGGED>), grid, block, 0, s, a);
+          break;
+        }
+      }
+      [[fallthrough]];
+    case 16:
+      if constexpr (VecIO<T>::N == 4 && !BWD && LPR == 0) {
+        if (nv == 16) {
+          HK_LAUNCH((softmax_fwd_kernel<T, 16, LPR, RAGGED>), grid, block, 0, s, a);
+          break;
+        }
       }
       [[fallthrough]];
     default:
@@ -296,6 +376,22 @@ static int launch_softmax_nv(const SoftmaxArgs& a, int nv, dim3 grid, dim3 block
   return launch_check(BWD ? "softmax_bwd_kernel" : "softmax_fwd_kernel");
 }
 
+template <typename T, bool BWD, bool RAGGED>
+static int launch_softmax(const SoftmaxArgs& a, int threads, int nv, hipStream_t s) {
+  if (threads > 64) {
+    dim3 grid{unsigned(a.n0), unsigned(a.n1), unsigned(a.n2)}, block{unsigned(threads)};
+    return launch_softmax_nv<T, BWD, 0, RAGGED>(a, nv, grid, block, s);
+  }
+  const int rows_per_block = 256 / threads;
+  dim3 grid(unsigned((a.n0 + rows_per_block - 1) / rows_per_block), unsigned(a.n1), unsigned(a.n2)), block(256);
+  switch (threads) {
+    case 8: return launch_softmax_nv<T, BWD, 8, RAGGED>(a, nv, grid, block, s);
+    case 16: return launch_softmax_nv<T, BWD, 16, RAGGED>(a, nv, grid, block, s);
+    case 32: return launch_softmax_nv<T, BWD, 32, RAGGED>(a, nv, grid, block, s);
+    default: return launch_softmax_nv<T, BWD, 64, RAGGED>(a, nv, grid, block, s);
+  }
+}
+
 template <typename T, bool BWD>
 static int softmax_lastdim_typed(SoftmaxArgs a, hipStream_t s) {
   constexpr int VEC = VecIO<T>::N;
@@ -303,24 +399,22 @@ static int softmax_lastdim_typed(SoftmaxArgs a, hipStream_t s) {
   const bool vec_ok = a.cols % VEC == 0 && aligned16(a.x) && aligned16(a.dy) && aligned16(a.out) &&
                       steps_ok(a.x_pitch, a.x_lv) && steps_ok(a.out_pitch, a.out_lv) &&
                       (!BWD || steps_ok(a.dy_pitch, a.dy_lv));
-  a.nvec = a.cols / VEC;
+  a.nvec = (a.cols + VEC - 1) / VEC;
   // forward keeps NV*VEC exponentials per thread: at most 64 floats
   // backward holds y and dy: at most 4 vectors of each per thread
   const int max_nv = BWD ? 4 : 64 / VEC;
-  const int max_nv_wave = BWD ? 4 : std::min(8, 64 / VEC);
   int threads = 0, nv = 0;
-  if (vec_ok && pick_softmax_shape(a.nvec, max_nv_wave, max_nv, BWD, &threads, &nv)) {
-    if (threads == 64) {
-      dim3 grid(unsigned((a.n0 + 3) / 4), unsigned(a.n1), unsigned(a.n2)), block(256);
-      return launch_softmax_nv<T, BWD, true>(a, nv, grid, block, s);
-    }
-    dim3 grid{unsigned(a.n0), unsigned(a.n1), unsigned(a.n2)}, block{unsigned(threads)};
-    return launch_softmax_nv<T, BWD, false>(a, nv, grid, block, s);
-  }
+  const uintptr_t boundary = reinterpret_cast<uintptr_t>(a.x) | reinterpret_cast<uintptr_t>(a.dy) |
+                             reinterpret_cast<uintptr_t>(a.out) | uintptr_t(a.x_pitch * int64_t(sizeof(T))) |
+                             uintptr_t(a.out_pitch * int64_t(sizeof(T)));
+  const bool shaped = pick_softmax_shape(a.nvec, vec_ok, (boundary & 3) != 0, max_nv, BWD, &threads, &nv);
+  if (vec_ok && shaped) return launch_softmax<T, BWD, false>(a, threads, nv, s);
   if (a.n0 != a.rows) {
     set_last_error("softmax: rows on several levels need 16-byte aligned rows and steps");
     return HK_ERR_UNSUPPORTED;
   }
+  // any other length or alignment, down to rows of one vector
+  if (shaped && a.cols >= VEC) return launch_softmax<T, BWD, true>(a, threads, nv, s);
   if constexpr (BWD) {
     HK_LAUNCH((softmax_bwd_longrow_kernel<T, float>), dim3(unsigned(a.rows)), dim3(256), 0, s,
                        static_cast<const T*>(a.x), static_cast<const T*>(a.dy), static_cast<T*>(a.out),

@@ -1,0 +1,74 @@
+"""Rows of any length and alignment through the register kernels: row lengths at the edges of a vector, of a lane
+group and of a workgroup, bases that lie off the 16-byte grid by one element, and row pitches that are no multiple of
+a vector.  The outputs sit inside guarded buffers: nothing outside a row may be written."""
+import numpy as np
+import pytest
+
+import helpers
+import oracle
+
+pytestmark = pytest.mark.gpu
+
+ES = {"fp32": 4, "bf16": 2, "fp16": 2}
+GUARD = 16
+
+
+def _placed(cuda, a, dtype, offset, pitch, fill=None):
+    """(whole buffer, [rows, cols] view): `a` (or, without it, `fill`) laid `offset` elements into a buffer of rows
+    `pitch` apart, with guard elements of value 7 around and between the rows."""
+    import torch
+    rows, cols = a.shape
+    dt = {"fp32": torch.float32, "bf16": torch.bfloat16, "fp16": torch.float16}[dtype]
+    buf = torch.full((GUARD + rows * pitch + GUARD,), 7.0, dtype=dt, device=cuda)
+    view = torch.as_strided(buf, (rows, cols), (pitch, 1), GUARD + offset)
+    view.copy_(helpers.to_torch(a, dtype, cuda) if fill is None else torch.full_like(view, fill))
+    return buf, view
+
+
+def _guards_untouched(buf, view):
+    import torch
+    keep = buf.clone()
+    inside = torch.as_strided(keep, view.shape, view.stride(), view.storage_offset())
+    inside.fill_(7.0)
+    return bool((keep == 7.0).all())
+
+
+# vectors per row around 1, 8, 16, 32, 64, 128, 192, 256 and the workgroup widths above, and one element off each
+def _lengths(dtype):
+    vec = 16 // ES[dtype]
+    out = set()
+    for v in (1, 2, 8, 16, 32, 64, 96, 128, 192, 256, 300, 512):
+        out.update((v * vec, v * vec + 1, v * vec + vec - 1))
+    return sorted(out)
+
+
+@pytest.mark.parametrize("dtype", ["fp32", "bf16", "fp16"])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_softmax_any_length(hk, cuda, dtype, shift):
+    import torch
+    rows = 37
+    for cols in _lengths(dtype):
+        pitch = cols + (0 if shift == 0 else 5)
+        x = helpers.draw(3000 + cols, (rows, cols), dtype=dtype)
+        dy = helpers.draw(4000 + cols, (rows, cols), dtype=dtype)
+        ey = oracle.softmax_fwd(x)
+        _, tx = _placed(cuda, x, dtype, shift, pitch)
+        yb, ty = _placed(cuda, x, dtype, shift, pitch, 0.0)
+        hk.softmax_fwd(tx, ty)
+        torch.cuda.synchronize()
+        helpers.assert_close(ty.contiguous(), ey, dtype, "softmax y %d" % cols)
+        assert _guards_untouched(yb, ty), cols
+        y = helpers.to_numpy(ty.contiguous())
+        _, tdy = _placed(cuda, dy, dtype, shift, pitch)
+        db, tdx = _placed(cuda, x, dtype, shift, pitch, 0.0)
+        hk.softmax_bwd(ty, tdy, tdx)
+        torch.cuda.synchronize()
+        # dx = y (dy - sum dy y): a difference of terms of the size of y dy, which `scale` names
+        helpers.assert_close(tdx.contiguous(), oracle.softmax_bwd(y, dy), dtype, "softmax dx %d" % cols,
+                             scale=float(np.sqrt(np.mean(np.square(y * dy)))),
+                             ordinary_rtol=helpers.SOFTMAX_GRADIENT_ORDINARY_RTOL)
+        assert _guards_untouched(db, tdx), cols
+        # in place: the row's last vector overlaps the one before it
+        hk.softmax_fwd(tx, tx)
+        torch.cuda.synchronize()
+        assert torch.equal(tx.contiguous(), ty.contiguous()), cols
