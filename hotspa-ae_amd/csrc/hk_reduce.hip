@@ -3,8 +3,10 @@
 // The host merges neighbouring dimensions of the same kind (reduced / kept)
 // that are contiguous in memory, then picks one of three kernels:
 //   inner   [rows, C] -> [rows]   : the reduced extent is the unit-stride one;
-//           a wavefront or workgroup streams a row with 128-bit loads, DPP +
-//           LDS fold.  Long rows are split over several workgroups.
+//           some lanes, a wavefront or a workgroup stream a row with 128-bit
+//           loads at any boundary, DPP + LDS fold.  Long rows are split over
+//           several workgroups.  The same kernel takes rows that consist of
+//           several runs ([N, rows, C] -> [rows]).
 //   outer   [B, R, C] -> [B, C]   : the kept extent is the unit-stride one;
 //           every lane owns one 128-bit column vector, the waves of a
 //           workgroup take runs of consecutive rows, rows are split over many
@@ -147,67 +149,138 @@ __device__ __forceinline__ ACC block_reduce_lds(ACC v, ACC* lds) {
 
 // ---------------------------------------------------------------------------
 // inner reduction, vector path (fp32 / bf16 / fp16 input, fp32 accumulate)
-// grid = (row groups, nsplit); a group of `tpr` threads takes one row chunk
+// grid = (row groups, nsplit); `lanes` lanes of a wavefront (LANES) or a whole workgroup take one row chunk.
+//
+// A row is one run of `cols` contiguous elements or, with RUNS, `nruns` of them a fixed step apart (the sum over the
+// first and the last dimension of [N, C, H * W]: row = channel, run = image).  Rows start anywhere (see ld16_any in
+// hk_common.h); the last, partial vector of a run is loaded as the run's last whole one and the elements that the
+// vector before it holds are left out.  Bound by HBM: what counts is that every lane has eight 16-byte loads in
+// flight, so the (run, vector) place is advanced by additions (no division in the loop), and that the vectors left
+// over after the last full round of eight are loaded together too.  Measured, bf16: axes (0, 2) of [64, 256, 3136]
+// 87 ms (one thread per channel) -> 17.0 us (6.0 TB/s), of [12, 16, 16000] 72.7 ms -> 12.0 us; 16384 rows of 1021
+// elements (before: one workgroup per row, element by element) 20.9 -> 9.4 us, 524288 rows of 9 (9 MB) 364 -> 9.5 us,
+// 524288 aligned rows of 64 (a wavefront per row before) 93 -> 14.5 us; 32768 x 4096 unchanged at 40.1 us.
 // ---------------------------------------------------------------------------
 struct InnerArgs {
   const void* in;
   void* out;          // OUT_T [rows] when nsplit == 1, else float [rows, nsplit]
   int64_t rows;
   int64_t row_stride; // elements
-  int64_t cols;
-  int64_t chunk;      // columns per split (multiple of the vector width)
+  int64_t level_rows; // rows of the inner level; row r starts (r % level_rows) * row_stride + (r / level_rows) * level_stride
+  int64_t level_stride;
+  int64_t cols;       // at least one vector
+  int64_t nruns;
+  int64_t run_stride;
+  int64_t chunk;      // vectors per split, out of nruns * ceil(cols / vector)
   int nsplit;
+  int lanes;          // LANES: 1, 2, 4, ... 64 lanes take a row
   float factor;
   int is_mean;
 };
 
-template <typename T, typename OUT_T, bool WAVE_ROW, typename R>
-__global__ __launch_bounds__(WAVE_ROW ? 256 : 1024)
+template <typename R>
+__device__ __forceinline__ float lanes_reduce(float v, int lanes) {
+  if (lanes == kWave) return wave_allreduce<AsFloatOp<R>>(v);
+  if (lanes > 1) v = R::apply(v, dpp_perm<kDppXor1>(v));
+  if (lanes > 2) v = R::apply(v, dpp_perm<kDppXor2>(v));
+  if (lanes > 4) v = R::apply(v, dpp_perm<kDppHalfMirror>(v));
+  if (lanes > 8) v = R::apply(v, dpp_perm<kDppMirror>(v));
+  if (lanes > 16) v = R::apply(v, lane_xor<16>(v));
+  return v;
+}
+
+template <typename T, typename OUT_T, bool LANES, bool RUNS, typename R>
+__global__ __launch_bounds__(LANES ? 256 : 1024)
 void reduce_inner_vec_kernel(InnerArgs a) {
   constexpr int VEC = VecIO<T>::N;
   constexpr int U = 8;
   __shared__ float red[kMaxWaves];
-  const int tpr = WAVE_ROW ? kWave : int(blockDim.x);
-  const int t = WAVE_ROW ? int(threadIdx.x & 63) : int(threadIdx.x);
-  const int64_t row = WAVE_ROW
-      ? int64_t(blockIdx.x) * (blockDim.x >> 6) + wave_index()
-      : int64_t(blockIdx.x);
-  if (WAVE_ROW && row >= a.rows) return;
+  const int tpr = LANES ? a.lanes : int(blockDim.x);
+  const int t = LANES ? int(threadIdx.x) & (tpr - 1) : int(threadIdx.x);
+  const int64_t row = !LANES ? int64_t(blockIdx.x)
+                    : tpr == kWave ? int64_t(blockIdx.x) * (blockDim.x >> 6) + wave_index()
+                                   : (int64_t(blockIdx.x) * blockDim.x + threadIdx.x) >> __builtin_ctz(tpr);
+  if (LANES && row >= a.rows) return;   // whole groups of lanes leave
   const int split = blockIdx.y;
-  const int64_t c0 = int64_t(split) * a.chunk;
-  const int64_t c1 = (c0 + a.chunk < a.cols) ? c0 + a.chunk : a.cols;
-  const T* p = static_cast<const T*>(a.in) + row * a.row_stride + c0;
-  const int64_t nvec = (c1 - c0) / VEC;
+  int64_t base = row * a.row_stride;
+  if (a.level_rows != a.rows) {
+    const uint32_t q = uint32_t(row) / uint32_t(a.level_rows);
+    base = int64_t(uint32_t(row) - q * uint32_t(a.level_rows)) * a.row_stride + int64_t(q) * a.level_stride;
+  }
+  const T* p = static_cast<const T*>(a.in) + base;
+  const int64_t nvec = (a.cols + VEC - 1) / VEC;          // of one run
+  const int skip = int(nvec * VEC - a.cols);              // elements of a run's last load that the one before it holds
+  const int64_t total = RUNS ? a.nruns * nvec : nvec;
+  const int64_t end = (split + 1) * a.chunk < total ? (split + 1) * a.chunk : total;
+  int64_t i = split * a.chunk + t;                        // place in the row, in vectors
 
+  // the same place as (run, vector of the run), kept up by additions
+  int64_t v = i, off = i * VEC, dv = tpr, doff = int64_t(tpr) * VEC;
+  const int64_t wrap = RUNS ? a.run_stride - nvec * VEC : 0;
+  if constexpr (RUNS) {
+    const int64_t run = i / nvec, drun = tpr / nvec;
+    v = i - run * nvec;
+    off = run * a.run_stride + v * VEC;
+    dv = tpr - drun * nvec;
+    doff = drun * a.run_stride + dv * VEC;
+  }
+  auto load = [&]() {
+    const T* at = p + off;
+    if (skip != 0 && v == nvec - 1) at -= skip;
+    return ld16_any(at);
+  };
+  auto step = [&]() {
+    v += dv;
+    off += doff;
+    if constexpr (RUNS) {
+      if (v >= nvec) { v -= nvec; off += wrap; }
+    }
+  };
   float acc[U];
 #pragma unroll
   for (int u = 0; u < U; ++u) acc[u] = R::template identity<float>();
-  int64_t v = t;
-  for (; v + int64_t(U - 1) * tpr < nvec; v += int64_t(U) * tpr) {
-    u32x4 r[U];
+  auto add = [&](float& s, const u32x4& raw, bool last) {
+    float f[VEC];
+    VecIO<T>::unpack(raw, f);
+    if (last) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) r[u] = ld16(p + (v + int64_t(u) * tpr) * VEC);
+      for (int j = 0; j < VEC; ++j) s = R::apply(s, j >= skip ? R::pre(f[j], a.factor) : R::template identity<float>());
+    } else {
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) s = R::apply(s, R::pre(f[j], a.factor));
+    }
+  };
+  for (; i + int64_t(U - 1) * tpr < end; i += int64_t(U) * tpr) {
+    u32x4 r[U];
+    bool last[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      float f[VEC];
-      VecIO<T>::unpack(r[u], f);
-#pragma unroll
-      for (int j = 0; j < VEC; ++j) acc[u] = R::apply(acc[u], R::pre(f[j], a.factor));
+      last[u] = skip != 0 && v == nvec - 1;
+      r[u] = load();
+      step();
     }
-  }
-  for (; v < nvec; v += tpr) {
-    float f[VEC];
-    VecIO<T>::unpack(ld16(p + v * VEC), f);
 #pragma unroll
-    for (int j = 0; j < VEC; ++j) acc[0] = R::apply(acc[0], R::pre(f[j], a.factor));
+    for (int u = 0; u < U; ++u) add(acc[u], r[u], last[u]);
   }
-  // scalar tail of the last split
-  for (int64_t c = c0 + nvec * VEC + t; c < c1; c += tpr)
-    acc[1] = R::apply(acc[1], R::pre(Cvt<T>::load(static_cast<const T*>(a.in) + row * a.row_stride + c), a.factor));
+  if (i < end) {
+    // fewer than U are left: all of them in flight at once
+    u32x4 r[U - 1];
+    bool last[U - 1];
+#pragma unroll
+    for (int u = 0; u < U - 1; ++u) {
+      last[u] = skip != 0 && v == nvec - 1;
+      r[u] = u32x4{0, 0, 0, 0};
+      if (i + int64_t(u) * tpr < end) r[u] = load();
+      step();
+    }
+#pragma unroll
+    for (int u = 0; u < U - 1; ++u)
+      if (i + int64_t(u) * tpr < end) add(acc[u], r[u], last[u]);
+  }
   float s = R::apply(R::apply(R::apply(acc[0], acc[1]), R::apply(acc[2], acc[3])),
                      R::apply(R::apply(acc[4], acc[5]), R::apply(acc[6], acc[7])));
-  if constexpr (WAVE_ROW) {
-    s = wave_allreduce<AsFloatOp<R>>(s);
+  if constexpr (LANES) {
+    s = lanes_reduce<R>(s, tpr);
   } else {
     s = block_allreduce<AsFloatOp<R>>(s, red, int(blockDim.x >> 6));
   }
@@ -215,6 +288,25 @@ void reduce_inner_vec_kernel(InnerArgs a) {
     if (a.nsplit == 1) st_acc<OUT_T, float>(static_cast<OUT_T*>(a.out) + row, R::template post<float>(s, a.factor, a.is_mean));
     else static_cast<float*>(a.out)[row * a.nsplit + split] = s;
   }
+}
+
+// rows shorter than a vector: one row per thread
+template <typename T, typename OUT_T, typename R>
+__global__ __launch_bounds__(256)
+void reduce_inner_tiny_kernel(const T* in, OUT_T* out, int64_t rows, int64_t row_stride, int cols, float factor,
+                              int is_mean) {
+  constexpr int VEC = VecIO<T>::N;
+  const int64_t row = int64_t(blockIdx.x) * 256 + threadIdx.x;
+  if (row >= rows) return;
+  const T* p = in + row * row_stride;
+  float f[VEC - 1];
+#pragma unroll
+  for (int j = 0; j < VEC - 1; ++j) f[j] = j < cols ? Cvt<T>::load(p + j) : 0.f;
+  float s = R::template identity<float>();
+#pragma unroll
+  for (int j = 0; j < VEC - 1; ++j)
+    if (j < cols) s = R::apply(s, R::pre(f[j], factor));
+  st_acc<OUT_T, float>(out + row, R::template post<float>(s, factor, is_mean));
 }
 
 // inner reduction, scalar path: any dtype / alignment; one workgroup per row
@@ -246,6 +338,7 @@ struct OuterArgs {
   float factor;
   int is_mean;
   int split_major;      // grid = (row splits, column tiles, batch) instead of (column tiles, row splits, batch)
+  int partial;          // the sums go out as float [rsplit, B, C]; else (one split) finished, as OUT_T [B, C]
 };
 
 template <typename T, typename OUT_T, typename R>
@@ -267,8 +360,10 @@ void reduce_outer_vec_kernel(OuterArgs a) {
   const int split = a.split_major ? blockIdx.x : blockIdx.y;
   const int64_t tile = a.split_major ? blockIdx.y : blockIdx.x;
   const int64_t cv = (tile * wx + wc) * kWave + lane;   // column vector index
-  const int64_t c = cv * VEC;
-  const bool col_ok = c < a.C;                              // C is a multiple of VEC here
+  const bool col_ok = cv * VEC < a.C;
+  // the last, partial vector of a row is the row's last whole one: the columns that two lanes then hold come out of
+  // the same additions in both, and both store them (300 x 33300 bf16, before by the element-wise kernel: 72 -> 12 us)
+  const int64_t c = cv * VEC + VEC <= a.C ? cv * VEC : a.C - VEC;
   const int64_t b = blockIdx.z;
   const int64_t r0 = int64_t(split) * a.rows_per_split;
   const int64_t r1 = (r0 + a.rows_per_split < a.R) ? r0 + a.rows_per_split : a.R;
@@ -284,7 +379,7 @@ void reduce_outer_vec_kernel(OuterArgs a) {
     for (; r + U <= r1; r += int64_t(U) * wy) {
       u32x4 v[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) v[u] = ld16(p + (r + u) * a.r_stride);
+      for (int u = 0; u < U; ++u) v[u] = ld16_any(p + (r + u) * a.r_stride);
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         float f[VEC];
@@ -293,13 +388,44 @@ void reduce_outer_vec_kernel(OuterArgs a) {
         for (int j = 0; j < VEC; ++j) acc[j] = R::apply(acc[j], R::pre(f[j], a.factor));
       }
     }
-    // the last, partial run of rows of this wavefront (fewer than U)
-    for (; r < r1; ++r) {
-      float f[VEC];
-      VecIO<T>::unpack(ld16(p + r * a.r_stride), f);
+    // the last, partial run of rows of this wavefront (fewer than U), loaded together as well
+    if (r < r1) {
+      const int left = int(r1 - r) < U - 1 ? int(r1 - r) : U - 1;
+      u32x4 v[U - 1];
 #pragma unroll
-      for (int j = 0; j < VEC; ++j) acc[j] = R::apply(acc[j], R::pre(f[j], a.factor));
+      for (int u = 0; u < U - 1; ++u) {
+        v[u] = u32x4{0, 0, 0, 0};
+        if (u < left) v[u] = ld16_any(p + (r + u) * a.r_stride);
+      }
+#pragma unroll
+      for (int u = 0; u < U - 1; ++u) {
+        if (u < left) {
+          float f[VEC];
+          VecIO<T>::unpack(v[u], f);
+#pragma unroll
+          for (int j = 0; j < VEC; ++j) acc[j] = R::apply(acc[j], R::pre(f[j], a.factor));
+        }
+      }
     }
+  }
+  // one wavefront over the rows: a lane's columns are finished and go out as whole vectors (3 x 10^7 bf16, 2-byte
+  // stores from LDS before: 21.3 -> 14.2 us)
+  if (wy == 1) {
+    if (!col_ok) return;
+    const auto store = [&](auto* out) {
+      using O = typename std::remove_pointer<decltype(out)>::type;
+      constexpr int N = VecIO<O>::N;
+#pragma unroll
+      for (int j = 0; j < VEC; j += N) st16_any(out + c + j, VecIO<O>::pack(acc + j));
+    };
+    if (a.partial) {
+      store(static_cast<float*>(a.out) + (int64_t(split) * a.B + b) * a.C);
+    } else {
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) acc[j] = R::template post<float>(acc[j], a.factor, a.is_mean);
+      store(static_cast<OUT_T*>(a.out) + b * a.C);
+    }
+    return;
   }
   // fold the waves of the block: lane-major layout keeps LDS accesses conflict-free
 #pragma unroll
@@ -310,7 +436,7 @@ void reduce_outer_vec_kernel(OuterArgs a) {
     float s = R::template identity<float>();
     for (int k = 0; k < wy; ++k) s = R::apply(s, lds[((k * wx + wc) * VEC + j) * kWave + lane]);
     if (col_ok) {
-      if (a.rsplit == 1)
+      if (!a.partial)
         st_acc<OUT_T, float>(static_cast<OUT_T*>(a.out) + b * a.C + c + j, R::template post<float>(s, a.factor, a.is_mean));
       else
         static_cast<float*>(a.out)[(int64_t(split) * a.B + b) * a.C + c + j] = s;
@@ -347,6 +473,24 @@ void reduce_fold_partials_kernel(const float* part, OUT_T* out, int nparts, int6
     const float s = R::apply(R::apply(lds[0][lane], lds[1][lane]), R::apply(lds[2][lane], lds[3][lane]));
     st_acc<OUT_T, float>(out + i, R::template post<float>(s, factor, is_mean));
   }
+}
+
+// folds float partials [nparts, rows, cols] -> OUT_T [rows]: what is left of a row's elements after the column kernel
+// has folded the leading dimension; one wavefront per row
+template <typename OUT_T, typename R>
+__global__ __launch_bounds__(256)
+void reduce_fold_rows_kernel(const float* part, OUT_T* out, int nparts, int64_t rows, uint32_t cols, float factor,
+                             int is_mean) {
+  const int64_t row = int64_t(blockIdx.x) * 4 + wave_index();
+  if (row >= rows) return;
+  const uint32_t n = uint32_t(nparts) * cols;
+  float s = R::template identity<float>();
+  for (uint32_t i = threadIdx.x & 63; i < n; i += kWave) {
+    const uint32_t k = i / cols;
+    s = R::apply(s, part[(int64_t(k) * rows + row) * cols + (i - k * cols)]);
+  }
+  s = wave_allreduce<AsFloatOp<R>>(s);
+  if ((threadIdx.x & 63) == 0) st_acc<OUT_T, float>(out + row, R::template post<float>(s, factor, is_mean));
 }
 
 // outer reduction, scalar path: one thread per output column, any dtype
@@ -403,14 +547,15 @@ void reduce_generic_kernel(const T* in, OUT_T* out, GenericMeta m, float factor,
 // ---------------------------------------------------------------------------
 struct MergedDim { int64_t size, stride; bool reduce; };
 
-enum PlanKind { PLAN_EMPTY, PLAN_COPYLIKE, PLAN_INNER, PLAN_OUTER, PLAN_GENERIC };
+enum PlanKind { PLAN_EMPTY, PLAN_COPYLIKE, PLAN_INNER, PLAN_RUNS, PLAN_OUTER, PLAN_GENERIC };
 
 struct ReducePlan {
   PlanKind kind = PLAN_GENERIC;
   std::vector<MergedDim> dims;     // outermost first, extents > 1 only
   int64_t n_out = 1, n_red = 1;
-  // inner
+  // inner: one run per row, rows on one level; runs: several a step apart, or rows on two levels
   int64_t rows = 1, row_stride = 0, cols = 1;
+  int64_t level_rows = 1, level_stride = 0, nruns = 1, run_stride = 0;
   // outer
   int64_t B = 1, R = 1, C = 1, b_stride = 0, r_stride = 0;
 };
@@ -462,6 +607,20 @@ static int make_plan(int ndim, const int64_t* shape, const int64_t* strides, int
     plan->cols = rd[0].size;
     plan->rows = keep.empty() ? 1 : keep[0].size;
     plan->row_stride = keep.empty() ? 0 : keep[0].stride;
+    plan->level_rows = plan->rows;
+    return HK_OK;
+  }
+  // the unit-stride dimension is reduced, and at most one other is; at most two are kept
+  if (dims.back().reduce && dims.back().stride == 1 && rd.size() <= 2 && keep.size() <= 2 &&
+      plan->n_out <= 0x7fffffffLL) {
+    plan->kind = PLAN_RUNS;
+    plan->cols = rd.back().size;
+    plan->nruns = rd.size() == 2 ? rd[0].size : 1;
+    plan->run_stride = rd.size() == 2 ? rd[0].stride : 0;
+    plan->rows = plan->n_out;
+    plan->level_rows = keep.empty() ? 1 : keep.back().size;
+    plan->row_stride = keep.empty() ? 0 : keep.back().stride;
+    plan->level_stride = keep.size() == 2 ? keep[0].stride : 0;
     return HK_OK;
   }
   if (rd.size() == 1 && !dims.back().reduce && dims.back().stride == 1 && keep.size() <= 2 &&
@@ -478,48 +637,55 @@ static int make_plan(int ndim, const int64_t* shape, const int64_t* strides, int
   return HK_OK;
 }
 
-struct InnerShape { int tpr; int nsplit; int64_t chunk; bool vec; };
-struct OuterShape { int wy; int wx; int rsplit; int64_t rows_per_split; bool vec; };
+struct InnerShape { int tpr; int nsplit; int64_t chunk; };   // tpr <= 64: lanes of a wavefront; chunk in vectors
+struct OuterShape { int wy; int wx; int rsplit; int64_t rows_per_split; };
 
+// `split`: whether there is scratch for the partial results of rows that several workgroups share
 template <typename T>
-static InnerShape shape_inner(const ReducePlan& p, const void* in) {
+static InnerShape shape_inner(const ReducePlan& p, bool split) {
   constexpr int VEC = 16 / sizeof(T);
   InnerShape s{};
-  s.vec = aligned16(in) && (p.rows == 1 || p.row_stride % VEC == 0);
-  const int64_t nvec = p.cols / VEC;
+  const int64_t nvec = p.nruns * ((p.cols + VEC - 1) / VEC);
   int tpr = tune_get(TUNE_REDUCE_INNER_THREADS);
-  const int64_t want_blocks = int64_t(device_cu_count()) * 4;
+  const int64_t cus = device_cu_count(), want_blocks = cus * 4;
   if (tpr <= 0) {
-    tpr = nvec <= 64 * 32 ? 64 : (nvec <= 256 * 32 ? 256 : 1024);
-    // too few rows to fill the chip: widen the group until a thread has at most one round of 8 loads,
-    // so that a short row costs one memory round trip instead of several dependent ones
-    if (p.rows < want_blocks) tpr = int(std::max<int64_t>(tpr, std::min<int64_t>(1024, (nvec + 7) / 8)));
+    if (p.nruns > 1) {
+      // long rows, usually few of them: as many wavefronts as fill the chip (16 per compute unit) without sharing a
+      // row between workgroups, whose partial results would cost a second launch
+      tpr = p.rows >= cus * 4 ? 256 : (p.rows >= cus * 2 ? 512 : 1024);
+      while (tpr > 64 && nvec < int64_t(tpr) * 4) tpr >>= 1;
+    } else if (nvec <= 64) {
+      // short rows share a wavefront: two vectors per lane
+      tpr = 1;
+      while (int64_t(tpr) * 2 < nvec) tpr <<= 1;
+    } else {
+      tpr = nvec <= 64 * 32 ? 64 : (nvec <= 256 * 32 ? 256 : 1024);
+      // too few rows to fill the chip: widen the group until a thread has at most one round of 8 loads,
+      // so that a short row costs one memory round trip instead of several dependent ones
+      if (p.rows < want_blocks) tpr = int(std::max<int64_t>(tpr, std::min<int64_t>(1024, (nvec + 7) / 8)));
+    }
   }
-  tpr = std::min(1024, std::max(64, (tpr + 63) / 64 * 64));
+  if (tpr >= 64 || tune_get(TUNE_REDUCE_INNER_THREADS) > 0) tpr = std::min(1024, std::max(64, (tpr + 63) / 64 * 64));
   s.tpr = tpr;
-  // few long rows: split columns so that ~4 workgroups per CU exist
-  int64_t groups = tpr == 64 ? (p.rows + 3) / 4 : p.rows;
+  // few long rows: split columns so that ~4 workgroups per CU exist (of 1024 threads: one)
+  const int64_t groups = tpr <= 64 ? (p.rows * tpr + 255) / 256 : p.rows;
+  const int64_t want = p.nruns > 1 ? std::max<int64_t>(cus, want_blocks * 256 / std::max(tpr, 256)) : want_blocks;
+  const int64_t rounds = p.nruns > 1 ? 8 : 16;   // vectors per thread below which a split is not worth its fold
   int64_t nsplit = 1;
-  if (groups < want_blocks && nvec > int64_t(tpr) * 32) {
-    nsplit = std::min<int64_t>((want_blocks + groups - 1) / groups, nvec / (int64_t(tpr) * 16));
+  if (split && groups < want && nvec > int64_t(tpr) * rounds * 2) {
+    nsplit = std::min<int64_t>((want + groups - 1) / groups, nvec / (int64_t(tpr) * rounds));
     nsplit = std::max<int64_t>(1, std::min<int64_t>(nsplit, 1024));
   }
-  int64_t chunk_vec = (nvec + nsplit - 1) / nsplit;
-  if (chunk_vec == 0) chunk_vec = 1;
-  s.chunk = chunk_vec * VEC;
-  s.nsplit = int((p.cols + s.chunk - 1) / s.chunk);
-  if (s.nsplit < 1) s.nsplit = 1;
+  s.chunk = std::max<int64_t>(1, (nvec + nsplit - 1) / nsplit);
+  s.nsplit = int((nvec + s.chunk - 1) / s.chunk);
   return s;
 }
 
 template <typename T>
-static OuterShape shape_outer(const ReducePlan& p, const void* in) {
+static OuterShape shape_outer(const ReducePlan& p, bool split) {
   constexpr int VEC = 16 / sizeof(T);
   OuterShape s{};
-  s.vec = aligned16(in) && p.C % VEC == 0 && p.r_stride % VEC == 0 && (p.B == 1 || p.b_stride % VEC == 0);
-  s.wy = 1; s.wx = 1; s.rsplit = 1; s.rows_per_split = p.R;
-  if (!s.vec) return s;
-  int64_t col_tiles = std::max<int64_t>(1, (p.C / VEC + 63) / 64);
+  int64_t col_tiles = ((p.C + VEC - 1) / VEC + 63) / 64;
   // waves per block: enough rows per wave to keep 8 loads in flight
   // Measured at 32768 x 4096 bf16 (whole call, one workgroup per compute unit): 4 wavefronts 42.5 us, 8 wavefronts
   // 43.4 us, 16 wavefronts 44.3 us; putting 2, 4 or 8 of them side by side across columns (a workgroup then reads
@@ -538,7 +704,7 @@ static OuterShape shape_outer(const ReducePlan& p, const void* in) {
     const int64_t have = col_tiles * p.B;
     rsplit = int(std::max<int64_t>(1, (want_blocks + have - 1) / have));
   }
-  const int64_t max_split = std::max<int64_t>(1, p.R / (int64_t(wy) * 8));
+  const int64_t max_split = split ? std::max<int64_t>(1, p.R / (int64_t(wy) * 8)) : 1;
   rsplit = int(std::min<int64_t>(rsplit, max_split));
   rsplit = std::min(rsplit, 65535);
   s.rows_per_split = (p.R + rsplit - 1) / rsplit;
@@ -546,17 +712,50 @@ static OuterShape shape_outer(const ReducePlan& p, const void* in) {
   return s;
 }
 
+// Runs too short for the row kernel to read well (below 256 bytes: two lines of 128), in rows that lie next to each
+// other: the column kernel folds the leading dimension first, [nruns, rows * cols] -> [rows * cols] partial sums, and
+// a small kernel the rest.  The partial sums are what this costs (fp32, written and read once per row split), so at
+// least eight runs have to go into each.  Measured, bf16: [256, 512, 64] (128-byte runs) 7.1 ms (one thread per row)
+// -> 12.3 us, [256, 512, 7] 677 -> 12.8 us.
+static bool runs_by_columns(const ReducePlan& p, size_t es) {
+  return p.kind == PLAN_RUNS && p.level_rows == p.rows && p.row_stride == p.cols && p.nruns >= 8 &&
+         size_t(p.cols) * es < 256 && p.rows * p.cols * int64_t(es) >= 16;
+}
+static ReducePlan columns_of_runs(const ReducePlan& p) {
+  ReducePlan q = p;
+  q.kind = PLAN_OUTER;
+  q.B = 1; q.b_stride = 0;
+  q.R = p.nruns; q.r_stride = p.run_stride;
+  q.C = p.rows * p.cols;
+  return q;
+}
+
 template <typename T>
-static size_t workspace_for(const ReducePlan& p, const void* in) {
-  if (p.kind == PLAN_INNER) {
-    InnerShape s = shape_inner<T>(p, in);
-    return (s.vec && s.nsplit > 1) ? size_t(p.rows) * s.nsplit * sizeof(float) : 0;
+static size_t workspace_for(const ReducePlan& p) {
+  constexpr int VEC = 16 / sizeof(T);
+  if (runs_by_columns(p, sizeof(T))) {
+    const ReducePlan q = columns_of_runs(p);
+    return size_t(shape_outer<T>(q, true).rsplit) * q.C * sizeof(float);
   }
-  if (p.kind == PLAN_OUTER) {
-    OuterShape s = shape_outer<T>(p, in);
-    return (s.vec && s.rsplit > 1) ? size_t(s.rsplit) * p.B * p.C * sizeof(float) : 0;
+  if ((p.kind == PLAN_INNER || p.kind == PLAN_RUNS) && p.cols >= VEC) {
+    const InnerShape s = shape_inner<T>(p, true);
+    return s.nsplit > 1 ? size_t(p.rows) * s.nsplit * sizeof(float) : 0;
+  }
+  if (p.kind == PLAN_OUTER && p.C >= VEC) {
+    const OuterShape s = shape_outer<T>(p, true);
+    return s.rsplit > 1 ? size_t(s.rsplit) * p.B * p.C * sizeof(float) : 0;
   }
   return 0;
+}
+
+// Whether a call has to bring the scratch that hk_reduce_workspace_bytes asks for.  Whole vectors at 16-byte
+// boundaries always had to; the other layouts come without scratch, too, and then run unsplit.
+template <typename T>
+static bool scratch_required(const ReducePlan& p, const void* in) {
+  constexpr int VEC = 16 / sizeof(T);
+  if (!aligned16(in)) return false;
+  if (p.kind == PLAN_INNER) return p.rows == 1 || p.row_stride % VEC == 0;
+  return p.kind == PLAN_OUTER && p.C % VEC == 0 && p.r_stride % VEC == 0 && (p.B == 1 || p.b_stride % VEC == 0);
 }
 
 static GenericMeta generic_meta(const ReducePlan& p) {
@@ -573,34 +772,71 @@ static GenericMeta generic_meta(const ReducePlan& p) {
 
 // fast kernels: T in {float, bf16, fp16}, fp32 accumulation
 template <typename T, typename OUT_T, typename R>
+static int launch_inner(const ReducePlan& p, const InnerShape& s, const void* in, void* out, float factor, int is_mean,
+                        hipStream_t st) {
+  InnerArgs a{};
+  a.in = in; a.out = out; a.rows = p.rows; a.row_stride = p.row_stride; a.cols = p.cols; a.chunk = s.chunk;
+  a.level_rows = p.level_rows; a.level_stride = p.level_stride; a.nruns = p.nruns; a.run_stride = p.run_stride;
+  a.nsplit = s.nsplit; a.factor = factor; a.is_mean = is_mean; a.lanes = s.tpr;
+  const bool lanes = s.tpr <= kWave;
+  const int64_t groups = lanes ? (p.rows * s.tpr + 255) / 256 : p.rows;
+  dim3 grid(unsigned(groups), unsigned(s.nsplit)), block(lanes ? 256u : unsigned(s.tpr));
+  auto kernel = p.nruns > 1 ? (lanes ? reduce_inner_vec_kernel<T, OUT_T, true, true, R> : reduce_inner_vec_kernel<T, OUT_T, false, true, R>)
+                            : (lanes ? reduce_inner_vec_kernel<T, OUT_T, true, false, R> : reduce_inner_vec_kernel<T, OUT_T, false, false, R>);
+  profile_before(st);
+  HK_LAUNCH(kernel, grid, block, 0, st, a);
+  profile_after(st);
+  return launch_check("reduce_inner_vec_kernel");
+}
+
+template <typename T, typename OUT_T, typename R>
+static int launch_outer(const ReducePlan& p, const OuterShape& s, const void* in, void* out, bool partial, float factor,
+                        int is_mean, hipStream_t st) {
+  constexpr int VEC = 16 / sizeof(T);
+  OuterArgs a{};
+  a.in = in; a.out = out; a.B = p.B; a.R = p.R; a.C = p.C; a.b_stride = p.b_stride; a.r_stride = p.r_stride;
+  a.rows_per_split = s.rows_per_split; a.rsplit = s.rsplit; a.wx = s.wx; a.factor = factor; a.is_mean = is_mean;
+  a.partial = partial;
+  const int64_t col_tiles = (((p.C + VEC - 1) / VEC + 63) / 64 + s.wx - 1) / s.wx;
+  a.split_major = col_tiles <= 65535 ? 1 : 0;
+  dim3 grid(unsigned(col_tiles), unsigned(s.rsplit), unsigned(p.B)), block{unsigned(64 * s.wy * s.wx)};
+  if (a.split_major) grid = dim3(unsigned(s.rsplit), unsigned(col_tiles), unsigned(p.B));
+  const size_t lds = size_t(s.wy) * s.wx * 64 * VEC * sizeof(float);
+  profile_before(st);
+  HK_LAUNCH((reduce_outer_vec_kernel<T, OUT_T, R>), grid, block, lds, st, a);
+  profile_after(st);
+  return launch_check("reduce_outer_vec_kernel");
+}
+
+template <typename T, typename OUT_T, typename R>
 static int reduce_fast(const ReducePlan& p, const void* in, void* out, float factor, int is_mean,
                        void* ws, size_t ws_bytes, hipStream_t st, bool* handled) {
-  *handled = false;
-  if (p.kind == PLAN_INNER) {
-    InnerShape s = shape_inner<T>(p, in);
-    if (!s.vec) return HK_OK;
-    *handled = true;
-    InnerArgs a{};
-    a.in = in; a.rows = p.rows; a.row_stride = p.row_stride; a.cols = p.cols; a.chunk = s.chunk;
-    a.nsplit = s.nsplit; a.factor = factor; a.is_mean = is_mean;
-    if (s.nsplit > 1) {
-      const size_t need = size_t(p.rows) * s.nsplit * sizeof(float);
-      HK_REQUIRE(ws && ws_bytes >= need, HK_ERR_WORKSPACE, "hk_reduce: workspace of %zu bytes needed, %zu given", need, ws_bytes);
-      a.out = ws;
-    } else {
-      a.out = out;
-    }
+  constexpr int VEC = 16 / sizeof(T);
+  *handled = true;
+  const size_t need = workspace_for<T>(p);
+  const bool scratch = need == 0 || (ws && ws_bytes >= need);
+  HK_REQUIRE(scratch || !scratch_required<T>(p, in), HK_ERR_WORKSPACE,
+             "hk_reduce: workspace of %zu bytes needed, %zu given", need, ws_bytes);
+  if (scratch && runs_by_columns(p, sizeof(T))) {
+    const ReducePlan q = columns_of_runs(p);
+    const OuterShape s = shape_outer<T>(q, true);
+    int rc = launch_outer<T, float, R>(q, s, in, ws, true, factor, is_mean, st);
+    if (rc != HK_OK) return rc;
+    HK_LAUNCH((reduce_fold_rows_kernel<OUT_T, R>), dim3(unsigned((p.rows + 3) / 4)), dim3(256), 0, st,
+              static_cast<const float*>(ws), static_cast<OUT_T*>(out), s.rsplit, p.rows, uint32_t(p.cols), factor, is_mean);
+    return launch_check("reduce_fold_rows_kernel");
+  }
+  if (p.kind == PLAN_INNER || (p.kind == PLAN_RUNS && p.cols >= VEC)) {
     HK_REQUIRE(p.rows <= 0x7fffffffLL, HK_ERR_INVALID, "hk_reduce: too many rows");
-    profile_before(st);
-    if (s.tpr == 64) {
-      dim3 grid(unsigned((p.rows + 3) / 4), unsigned(s.nsplit)), block(256);
-      HK_LAUNCH((reduce_inner_vec_kernel<T, OUT_T, true, R>), grid, block, 0, st, a);
-    } else {
-      dim3 grid(unsigned(p.rows), unsigned(s.nsplit)), block{unsigned(s.tpr)};
-      HK_LAUNCH((reduce_inner_vec_kernel<T, OUT_T, false, R>), grid, block, 0, st, a);
+    if (p.cols < VEC) {
+      profile_before(st);
+      HK_LAUNCH((reduce_inner_tiny_kernel<T, OUT_T, R>), dim3(unsigned((p.rows + 255) / 256)), dim3(256), 0, st,
+                static_cast<const T*>(in), static_cast<OUT_T*>(out), p.rows, p.row_stride, int(p.cols), factor, is_mean);
+      profile_after(st);
+      return launch_check("reduce_inner_tiny_kernel");
     }
-    profile_after(st);
-    int rc = launch_check("reduce_inner_vec_kernel");
+    const InnerShape s = shape_inner<T>(p, scratch);
+    int rc = launch_inner<T, OUT_T, R>(p, s, in, s.nsplit > 1 ? ws : out, factor, is_mean, st);
     if (rc != HK_OK || s.nsplit == 1) return rc;
     // second pass over the fp32 partials [rows, nsplit]: combine and store only, the elements' own
     // transform (|x|, x^2, |x|^p of the p-norms) was applied when the partials were formed
@@ -609,37 +845,19 @@ static int reduce_fast(const ReducePlan& p, const void* in, void* out, float fac
                        int64_t(s.nsplit), factor, is_mean);
     return launch_check("reduce_inner_scalar_kernel");
   }
-  if (p.kind == PLAN_OUTER) {
-    OuterShape s = shape_outer<T>(p, in);
-    if (!s.vec) return HK_OK;
-    *handled = true;
-    constexpr int VEC = 16 / sizeof(T);
-    OuterArgs a{};
-    a.in = in; a.B = p.B; a.R = p.R; a.C = p.C; a.b_stride = p.b_stride; a.r_stride = p.r_stride;
-    a.rows_per_split = s.rows_per_split; a.rsplit = s.rsplit; a.wx = s.wx; a.factor = factor; a.is_mean = is_mean;
-    if (s.rsplit > 1) {
-      const size_t need = size_t(s.rsplit) * p.B * p.C * sizeof(float);
-      HK_REQUIRE(ws && ws_bytes >= need, HK_ERR_WORKSPACE, "hk_reduce: workspace of %zu bytes needed, %zu given", need, ws_bytes);
-      a.out = ws;
-    } else {
-      a.out = out;
-    }
+  // (a batch extent beyond the grid's third dimension stays with the kernel that numbers its outputs on one axis where
+  // that took it: everything but whole vectors at 16-byte boundaries)
+  if (p.kind == PLAN_OUTER && p.C >= VEC && (p.B <= 65535 || scratch_required<T>(p, in))) {
     HK_REQUIRE(p.B <= 65535, HK_ERR_UNSUPPORTED, "hk_reduce: batch extent %lld too large for the column kernel", (long long)p.B);
-    const int64_t col_tiles = ((p.C / VEC + 63) / 64 + s.wx - 1) / s.wx;
-    a.split_major = col_tiles <= 65535 ? 1 : 0;
-    dim3 grid(unsigned(col_tiles), unsigned(s.rsplit), unsigned(p.B)), block{unsigned(64 * s.wy * s.wx)};
-    if (a.split_major) grid = dim3(unsigned(s.rsplit), unsigned(col_tiles), unsigned(p.B));
-    const size_t lds = size_t(s.wy) * s.wx * 64 * VEC * sizeof(float);
-    profile_before(st);
-    HK_LAUNCH((reduce_outer_vec_kernel<T, OUT_T, R>), grid, block, lds, st, a);
-    profile_after(st);
-    int rc = launch_check("reduce_outer_vec_kernel");
+    const OuterShape s = shape_outer<T>(p, scratch);
+    int rc = launch_outer<T, OUT_T, R>(p, s, in, s.rsplit > 1 ? ws : out, s.rsplit > 1, factor, is_mean, st);
     if (rc != HK_OK || s.rsplit == 1) return rc;
     const int64_t n = p.B * p.C;
     HK_LAUNCH((reduce_fold_partials_kernel<OUT_T, R>), dim3(unsigned((n + 63) / 64)), dim3(256), 0, st,
                        static_cast<const float*>(ws), static_cast<OUT_T*>(out), s.rsplit, n, factor, is_mean);
     return launch_check("reduce_fold_partials_kernel");
   }
+  *handled = false;
   return HK_OK;
 }
 
@@ -849,11 +1067,9 @@ int hk_reduce_workspace_bytes(int in_dtype, int ndim, const int64_t* shape, cons
   ReducePlan p;
   int rc = make_plan(ndim, shape, strides, naxes, axes, &p, "hk_reduce_workspace_bytes");
   if (rc != HK_OK) return rc;
-  // alignment of the data pointer is unknown here: assume the vector path
-  const void* aligned = reinterpret_cast<const void*>(uintptr_t(16));
   switch (in_dtype) {
-    case HK_FLOAT32: *bytes = workspace_for<float>(p, aligned); break;
-    case HK_BFLOAT16: case HK_FLOAT16: *bytes = workspace_for<uint16_t>(p, aligned); break;
+    case HK_FLOAT32: *bytes = workspace_for<float>(p); break;
+    case HK_BFLOAT16: case HK_FLOAT16: *bytes = workspace_for<uint16_t>(p); break;
     default: break;
   }
   return HK_OK;

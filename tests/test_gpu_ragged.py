@@ -72,3 +72,43 @@ def test_softmax_any_length(hk, cuda, dtype, shift):
         hk.softmax_fwd(tx, tx)
         torch.cuda.synchronize()
         assert torch.equal(tx.contiguous(), ty.contiguous()), cols
+
+
+# (shape, axes, permutation of the dense array or None): runs of every length around a vector and the widths of the
+# lane groups and workgroups, few and many of them, rows that several workgroups share; rows shorter than a vector;
+# rows on two levels; columns that are no whole number of vectors, over few and many rows
+REDUCTIONS = [((b, c, n), (0, 2), None) for b, c, n in
+              [(2, 3, 8), (9, 5, 7), (8, 16, 1), (8, 33, 40), (8, 33, 63), (7, 33, 9), (8, 40, 127), (8, 40, 129),
+               (64, 3, 1000), (300, 20, 31), (5, 300, 257), (3, 2, 70001), (64, 1030, 130), (2, 1, 400003)]]
+REDUCTIONS += [((45, n), (1,), None) for n in list(range(2, 18)) + [31, 63, 65, 127, 129, 255, 257, 511, 513, 1021, 4099]]
+REDUCTIONS += [((3, 70001), (1,), None), ((1, 600011), (1,), None), ((70001, 3), (1,), None)]
+REDUCTIONS += [((4, 6, 50), (2,), (1, 0, 2)), ((5, 4, 6, 50), (1, 3), (0, 2, 1, 3)), ((5, 4, 6, 50), (0, 3), (2, 0, 1, 3))]
+REDUCTIONS += [((r, c), (0,), None) for r in (2, 7, 9, 300) for c in (3, 8, 9, 15, 513, 1025)]
+REDUCTIONS += [((3, 41, 77), (1,), None), ((2, 3000, 1001), (1,), None)]
+
+
+@pytest.mark.parametrize("dtype", ["fp32", "bf16", "fp16"])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_reduce_any_extent(hk, cuda, dtype, shift):
+    """Whole numbers of -3..3: their sums are exact in fp32 in any order, so the result is the rounded exact sum."""
+    import torch
+    dt = {"fp32": torch.float32, "bf16": torch.bfloat16, "fp16": torch.float16}[dtype]
+    for k, (shape, axes, perm) in enumerate(REDUCTIONS):
+        a = np.random.default_rng(5000 + k).integers(-3, 4, shape).astype(np.float32)
+        buf = torch.zeros(GUARD + a.size, dtype=dt, device=cuda)
+        x = torch.as_strided(buf, shape, torch.empty(shape).stride(), shift)
+        x.copy_(torch.from_numpy(a).to(dt))
+        if perm is not None:
+            x, a = x.permute(perm), a.transpose(perm)
+        kept = [n for i, n in enumerate(a.shape) if i not in axes]
+        for op, expected in (("sum", a.sum(axes, dtype=np.float64)), ("max", a.max(axes))):
+            # with the scratch asked for, and (where rows lie off the 16-byte grid) without any
+            for workspace in [None] + ([torch.empty(1, device=cuda)] if shift else []):
+                out = torch.full((GUARD + int(np.prod(kept)) + GUARD,), 77.0, dtype=dt, device=cuda)
+                view = out[GUARD:-GUARD].view(kept)
+                hk.reduce(x, view, list(axes), op, workspace=workspace)
+                torch.cuda.synchronize()
+                what = (shape, axes, op, workspace is None)
+                assert torch.equal(view.float().cpu().double(), torch.from_numpy(
+                    oracle.round_to(np.asarray(expected, np.float32), dtype).astype(np.float64))), what
+                assert bool((out[:GUARD] == 77.0).all()) and bool((out[-GUARD:] == 77.0).all()), what
