@@ -7,6 +7,9 @@
 // rescales the stored exponentials into (softmax - onehot) * grad_loss and
 // writes the row once.  Rows whose label equals the ignored index are not read
 // at all: loss 0 / a zero gradient row is written.
+//
+// Sparse labels take rows of any length and alignment this way (see RowSpan); rows longer than a workgroup's registers
+// hold are streamed (sce_long_kernel).
 #include "hk_common.h"
 
 #include <algorithm>
@@ -65,8 +68,108 @@ __device__ __forceinline__ void row_coords(const SceArgs& a, int& tpr, int& t, i
   nwaves = WAVE_ROW ? 1 : int(blockDim.x >> 6);
 }
 
+// Rows whose maximum lies at the type's lowest values (p.v[0] == kLowestLog2 after the reduction): the sum and the
+// gradient from the row itself.
+template <typename T, bool WAVE_ROW>
+__device__ __forceinline__ float sce_lowest_count(const T* xr, int cols, int t, int tpr, int nwaves, float* red, float& M) {
+  return row_max_count<T>(xr, cols, t, tpr, [&](auto v) {
+    if constexpr (WAVE_ROW) return wave_allreduce_tuple(v);
+    else { __syncthreads(); return group_allreduce_tuple(v, red, 0, nwaves); }   // red may still be read
+  }, M);
+}
+template <typename T, bool WAVE_ROW>
+__device__ __forceinline__ void sce_lowest_bwd(const T* xr, T* dxr, int cols, int lab, float g, int t, int tpr, int nwaves,
+                                               float* red) {
+  float M;
+  const float n = sce_lowest_count<T, WAVE_ROW>(xr, cols, t, tpr, nwaves, red, M);
+  const float scale = g / (M == kNegInf ? __builtin_nanf("") : n);   // a row of nothing but -inf has no softmax
+  for (int c = t; c < cols; c += tpr)
+    Cvt<T>::store(dxr + c, (Cvt<T>::load(xr + c) == M ? 1.f : 0.f) * scale - (c == lab ? g : 0.f));
+}
+
 // ------------------------------- sparse forward ----------------------------
-template <typename T, int NV, bool WAVE_ROW>
+// A row as the 16-byte vectors that lie on 16-byte boundaries of the logits, and up to 2 (N - 1) elements before and
+// after them, one of which each of the first 2 N threads takes.  The order of a row's elements does not matter to its
+// sum, and accesses that straddle cache lines cost more than the few single ones: 4096 x 50257 bf16, vectors counted
+// from the row's start (odd 2-byte boundaries) against this: forward 100 / 83 us, backward 216 / 160 us.
+// RAGGED == false: whole vectors on the grid, nothing else.
+template <typename T, bool RAGGED>
+struct RowSpan {
+  static constexpr int N = VecIO<T>::N;
+  int head, nvec, edge;   // elements before the vectors; vectors; column of this thread's single element, or -1
+  __device__ __forceinline__ RowSpan(const T* row, int cols, int t) : head(0), nvec(cols / N), edge(-1) {
+    if constexpr (RAGGED) {
+      const int past = int(reinterpret_cast<uintptr_t>(row) & 15u) / int(sizeof(T));
+      head = min((N - past) & (N - 1), cols);
+      nvec = (cols - head) / N;
+      const int rest = head + nvec * N, k = t - N;
+      if (t < head) edge = t;
+      else if (k >= 0 && k < cols - rest) edge = rest + k;
+    }
+  }
+  // vector v, -inf past the last one (inside: it is known to be there, uniform).  KEEP: the row is read again
+  template <bool KEEP>
+  __device__ __forceinline__ u32x4 load(const T* row, int v, bool inside) const {
+    u32x4 raw = neg_inf_vec<T>();
+    if (inside || v < nvec) {
+      if constexpr (RAGGED) raw = KEEP ? ld16_any_keep<T>(row + head + v * N) : ld16_any<T>(row + head + v * N);
+      else raw = KEEP ? ld16_keep(row + v * N) : ld16(row + v * N);
+    }
+    return raw;
+  }
+  // (the output may lie on another phase of the 16-byte grid than the logits)
+  __device__ __forceinline__ void store(T* row, int v, const float* f) const {
+    if constexpr (RAGGED) st16_any(row + head + v * N, VecIO<T>::pack(f));
+    else st16_stream(row + v * N, VecIO<T>::pack(f));
+  }
+  __device__ __forceinline__ float load_edge(const T* row) const {
+    return RAGGED && edge >= 0 ? Cvt<T>::load(row + edge) : kNegInf;
+  }
+  __device__ __forceinline__ void store_edge(T* row, float v) const {
+    if (RAGGED && edge >= 0) Cvt<T>::store(row + edge, v);
+  }
+};
+
+// what the forward writes for an ignored row, and for one whose (ML, sum, maximum) is p (one thread per row)
+template <typename T>
+__device__ __forceinline__ void sce_store_ignored(const SceArgs& a, int64_t row) {
+  if (a.stats) {
+    a.stats[row] = kNegInf;
+    a.stats[a.rows + row] = 0.f;
+    a.stats[2 * a.rows + row] = 0.f;
+  } else {
+    Cvt<T>::store(static_cast<T*>(a.out) + row, 0.f);
+  }
+}
+template <typename T>
+__device__ __forceinline__ void sce_store_loss(const SceArgs& a, int64_t row, int64_t label, const T* xr,
+                                               const MaxSumMaxTuple& p) {
+  const float M = p.v[2];
+  if (a.stats) {
+    // sum exp(x - M) = S * 2^(ML - M * log2e)
+    a.stats[row] = M;
+    a.stats[a.rows + row] = (M == kNegInf) ? 0.f
+        : p.v[0] == kLowestLog2 ? p.v[1] : p.v[1] * __builtin_amdgcn_exp2f(-fmaf(M, kLog2e, -p.v[0]));
+    const int64_t local = label - a.vocab_start;
+    a.stats[2 * a.rows + row] = (local >= 0 && local < a.cols) ? Cvt<T>::load(xr + local) : 0.f;
+    return;
+  }
+  float r;
+  if (label >= 0 && label < a.cols) {
+    const float xl = Cvt<T>::load(xr + label);
+    // sum exp(x - M) = S * 2^(ML - M * log2e); the fma recovers the rounding of ML exactly
+    // (a row of lowest values has its sum relative to M itself)
+    const float log2s = __builtin_amdgcn_logf(p.v[1]) - (p.v[0] == kLowestLog2 ? 0.f : fmaf(M, kLog2e, -p.v[0]));
+    // M - xl first: the difference of two logits is (nearly) exact however large their common offset is, and
+    // the sum then rounds at the size of the loss, not of the logits
+    r = log2s * kLn2 + (M - xl);
+  } else {
+    r = __builtin_nanf("");  // label outside [0, cols): no logit to gather
+  }
+  Cvt<T>::store(static_cast<T*>(a.out) + row, r);
+}
+
+template <typename T, int NV, bool WAVE_ROW, bool RAGGED>
 __global__ __launch_bounds__(WAVE_ROW ? 256 : 1024)
 void sce_sparse_fwd_kernel(SceArgs a) {
   constexpr int VEC = VecIO<T>::N;
@@ -76,75 +179,42 @@ void sce_sparse_fwd_kernel(SceArgs a) {
   row_coords<WAVE_ROW>(a, tpr, t, i0, row, nwaves);
   if (WAVE_ROW && i0 >= a.n0) return;
 
-  T* loss = static_cast<T*>(a.out);
   const int64_t label = a.labels[row];
   if (label == a.ignored_index) {          // uniform over the row's threads
-    if (t == 0) {
-      if (a.stats) {
-        a.stats[row] = kNegInf;
-        a.stats[a.rows + row] = 0.f;
-        a.stats[2 * a.rows + row] = 0.f;
-      } else {
-        Cvt<T>::store(loss + row, 0.f);
-      }
-    }
+    if (t == 0) sce_store_ignored<T>(a, row);
     return;
   }
   const T* xr = static_cast<const T*>(a.logits) + i0 * a.x_pitch + outer_level_offset(a.x_lv);
   // slots past the row's end hold -inf: they change neither the maximum nor the sum
+  const RowSpan<T, RAGGED> span(xr, a.cols, t);
   float f[NV * VEC];
+  float edge;
   {
     u32x4 raw[NV];
 #pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int v = i * tpr + t;
-      if ((i + 1) * tpr <= a.nvec) {       // uniform: every thread's slot i is inside the row
-        raw[i] = ld16(xr + v * VEC);
-      } else {
-        raw[i] = neg_inf_vec<T>();
-        if (v < a.nvec) raw[i] = ld16(xr + v * VEC);
-      }
-    }
+    for (int i = 0; i < NV; ++i)
+      raw[i] = span.template load<false>(xr, i * tpr + t, (i + 1) * tpr <= span.nvec);
+    edge = span.load_edge(xr);
 #pragma unroll
     for (int i = 0; i < NV; ++i) VecIO<T>::unpack(raw[i], &f[i * VEC]);
   }
-  float m = f[0];
   static_assert((NV * VEC) % 2 == 0, "pairs of elements per max3");
-  m = fmaxf(m, f[1]);
+  float m = RAGGED ? max3(edge, f[0], f[1]) : fmaxf(f[0], f[1]);
 #pragma unroll
   for (int e = 2; e < NV * VEC; e += 2) m = max3(m, f[e], f[e + 1]);
   // ml: this thread's maximum in the log2 domain, rounded once (see OnlineSoftmaxTuple)
-  const float ml = (m == kNegInf) ? 0.f : m * kLog2e;
+  const float ml = log2_of_max(m);
   // four independent chains: the exponential unit's latency is not serialised behind one accumulator
   float s4[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int e = 0; e < NV * VEC; ++e) s4[e & 3] += __builtin_amdgcn_exp2f(fmaf(f[e], kLog2e, -ml));
+  if constexpr (RAGGED) s4[0] += __builtin_amdgcn_exp2f(fmaf(edge, kLog2e, -ml));
   const float s = (s4[0] + s4[1]) + (s4[2] + s4[3]);
   MaxSumMaxTuple p;
-  p.v[0] = (m == kNegInf) ? kNegInf : ml; p.v[1] = s; p.v[2] = m;
+  p.v[0] = ml; p.v[1] = s; p.v[2] = m;
   p = WAVE_ROW ? wave_allreduce_tuple(p) : group_allreduce_tuple(p, red, 0, nwaves);
-  if (t == 0 && a.stats) {
-    const float M = p.v[2];
-    // sum exp(x - M) = S * 2^(ML - M * log2e)
-    a.stats[row] = M;
-    a.stats[a.rows + row] = (M == kNegInf) ? 0.f : p.v[1] * __builtin_amdgcn_exp2f(-fmaf(M, kLog2e, -p.v[0]));
-    const int64_t local = label - a.vocab_start;
-    a.stats[2 * a.rows + row] = (local >= 0 && local < a.cols) ? Cvt<T>::load(xr + local) : 0.f;
-  } else if (t == 0) {
-    float r;
-    if (label >= 0 && label < a.cols) {
-      const float xl = Cvt<T>::load(xr + label);
-      // sum exp(x - M) = S * 2^(ML - M * log2e); the fma recovers the rounding of ML exactly
-      const float M = p.v[2];
-      const float log2s = __builtin_amdgcn_logf(p.v[1]) - fmaf(M, kLog2e, -p.v[0]);
-      // M - xl first: the difference of two logits is (nearly) exact however large their common offset is, and
-      // the sum then rounds at the size of the loss, not of the logits
-      r = log2s * kLn2 + (M - xl);
-    } else {
-      r = __builtin_nanf("");  // label outside [0, cols): no logit to gather
-    }
-    Cvt<T>::store(loss + row, r);
-  }
+  if (p.v[0] == kLowestLog2) p.v[1] = sce_lowest_count<T, WAVE_ROW>(xr, a.cols, t, tpr, nwaves, red, p.v[2]);   // uniform
+  if (t == 0) sce_store_loss<T>(a, row, label, xr, p);
 }
 
 // ------------------------------- sparse backward ---------------------------
@@ -156,7 +226,21 @@ void sce_sparse_fwd_kernel(SceArgs a) {
 template <typename T, int NV>
 constexpr int sce_min_waves(bool wave_row) { return wave_row ? 1 : (sizeof(T) == 4 && NV == 8 ? 4 : 8); }
 
-template <typename T, int NV, bool WAVE_ROW>
+// the label's column if the row has it, else one that no vector holds
+__device__ __forceinline__ int sce_label_column(int64_t label, int cols) {
+  return label >= 0 && label < cols ? int(label) : -1;
+}
+
+// a zero gradient row for an ignored label
+template <typename T, bool RAGGED>
+__device__ __forceinline__ void sce_store_zero_row(T* dxr, int cols, int t, int tpr) {
+  const RowSpan<T, RAGGED> span(dxr, cols, t);
+  const float zero[VecIO<T>::N] = {};
+  for (int v = t; v < span.nvec; v += tpr) span.store(dxr, v, zero);
+  span.store_edge(dxr, 0.f);
+}
+
+template <typename T, int NV, bool WAVE_ROW, bool RAGGED>
 __global__ __launch_bounds__(WAVE_ROW ? 256 : 1024, (sce_min_waves<T, NV>(WAVE_ROW)))
 void sce_sparse_bwd_kernel(SceArgs a) {
   constexpr int VEC = VecIO<T>::N;
@@ -169,38 +253,26 @@ void sce_sparse_bwd_kernel(SceArgs a) {
   T* dxr = static_cast<T*>(a.out) + i0 * a.out_pitch + outer_level_offset(a.out_lv);
   const int64_t label = a.labels[row];
   if (label == a.ignored_index) {
-    const u32x4 z = {0, 0, 0, 0};
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int v = i * tpr + t;
-      if (v < a.nvec) {
-        st16_stream(dxr + v * VEC, z);
-      }
-    }
+    sce_store_zero_row<T, RAGGED>(dxr, a.cols, t, tpr);
     return;
   }
   const T* xr = static_cast<const T*>(a.logits) + i0 * a.x_pitch + outer_level_offset(a.x_lv);
   // slots past the row's end hold -inf: they change neither the maximum nor the sum
+  const RowSpan<T, RAGGED> span(xr, a.cols, t);
   u32x4 raw[NV];
 #pragma unroll
-  for (int i = 0; i < NV; ++i) {
-    const int v = i * tpr + t;
-    if ((i + 1) * tpr <= a.nvec) {       // uniform: every thread's slot i is inside the row
-      raw[i] = ld16(xr + v * VEC);
-    } else {
-      raw[i] = neg_inf_vec<T>();
-      if (v < a.nvec) raw[i] = ld16(xr + v * VEC);
-    }
-  }
+  for (int i = 0; i < NV; ++i)
+    raw[i] = span.template load<false>(xr, i * tpr + t, (i + 1) * tpr <= span.nvec);
+  [[maybe_unused]] float edge = span.load_edge(xr);
   const float g = sce_row_grad<T, float>(a, row);
   float e[NV * VEC];
 #pragma unroll
   for (int i = 0; i < NV; ++i) VecIO<T>::unpack(raw[i], &e[i * VEC]);
   static_assert((NV * VEC) % 2 == 0, "pairs of elements per max3");
-  float m = fmaxf(e[0], e[1]);
+  float m = RAGGED ? max3(edge, e[0], e[1]) : fmaxf(e[0], e[1]);
 #pragma unroll
   for (int k = 2; k < NV * VEC; k += 2) m = max3(m, e[k], e[k + 1]);
-  const float ml = (m == kNegInf) ? 0.f : m * kLog2e;
+  const float ml = log2_of_max(m);
   // four independent chains, as in the forward kernel
   float s4[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -208,27 +280,136 @@ void sce_sparse_bwd_kernel(SceArgs a) {
     e[k] = __builtin_amdgcn_exp2f(fmaf(e[k], kLog2e, -ml));
     s4[k & 3] += e[k];
   }
+  if constexpr (RAGGED) {
+    edge = __builtin_amdgcn_exp2f(fmaf(edge, kLog2e, -ml));
+    s4[0] += edge;
+  }
   const float s = (s4[0] + s4[1]) + (s4[2] + s4[3]);
   MaxSumTuple p;
-  p.v[0] = (m == kNegInf) ? kNegInf : ml; p.v[1] = s;
+  p.v[0] = ml; p.v[1] = s;
   p = WAVE_ROW ? wave_allreduce_tuple(p) : group_allreduce_tuple(p, red, 0, nwaves);
-  const float ML = (p.v[0] == kNegInf) ? 0.f : p.v[0];
-  const float scale = __builtin_amdgcn_exp2f(ml - ML) / p.v[1] * g;
-  const int lvec = int(label / VEC), lsub = int(label - int64_t(lvec) * VEC);
+  const int lab = sce_label_column(label, a.cols);
+  if (p.v[0] == kLowestLog2) {   // uniform
+    sce_lowest_bwd<T, WAVE_ROW>(xr, dxr, a.cols, lab, g, t, tpr, nwaves, red);
+    return;
+  }
+  const float scale = __builtin_amdgcn_exp2f(ml - p.v[0]) / p.v[1] * g;
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
     const int v = i * tpr + t;
-    if (v < a.nvec) {
+    if (v < span.nvec) {
 #pragma unroll
       for (int j = 0; j < VEC; ++j) e[i * VEC + j] *= scale;
-      if (label >= 0 && v == lvec) {
+      const int lsub = lab - (span.head + v * VEC);
+      if (uint32_t(lsub) < uint32_t(VEC)) {
 #pragma unroll
         for (int j = 0; j < VEC; ++j)
           if (j == lsub) e[i * VEC + j] -= g;
       }
-      const u32x4 o = VecIO<T>::pack(&e[i * VEC]);
-      st16_stream(dxr + v * VEC, o);
+      span.store(dxr, v, &e[i * VEC]);
     }
+  }
+  if constexpr (RAGGED) span.store_edge(dxr, edge * scale - (span.edge == lab ? g : 0.f));
+}
+
+// ------------------------------- long rows ---------------------------------
+// Sparse labels, rows that do not fit a workgroup's registers: the workgroup streams the row, kLongVecs vectors per
+// thread and step, and every thread keeps a running (maximum, sum of exponentials) that it re-bases once per step.
+// The backward reads the row a second time, from its end, so that what was read last is found in the nearest cache
+// (1024 x 128256 bf16 116 -> 111 us), and is bound by what that second read costs: 4096 x 50257 bf16 611 us by
+// elements -> 160 us (4.9 TB/s of row and gradient), forward 358 -> 83 us (4.7 TB/s).  Every step has as many threads
+// as its share of the row needs (1024 throughout: 167 and 86 us).
+constexpr int kLongThreads = 1024;
+constexpr int kLongVecs = 4;
+
+template <typename T, bool BWD>
+__global__ __launch_bounds__(kLongThreads, 8)
+void sce_long_kernel(SceArgs a) {
+  constexpr int VEC = VecIO<T>::N;
+  constexpr int U = kLongVecs, NE = U * VEC;
+  __shared__ float red[kMaxWaves * 3];
+  const int t = int(threadIdx.x), tpr = int(blockDim.x), nwaves = tpr >> 6;
+  const int64_t i0 = blockIdx.x, row = dense_row_index(i0, a.rn);
+  const int64_t label = a.labels[row];
+  T* dxr = BWD ? static_cast<T*>(a.out) + i0 * a.out_pitch + outer_level_offset(a.out_lv) : nullptr;
+  if (label == a.ignored_index) {
+    if constexpr (BWD) sce_store_zero_row<T, true>(dxr, a.cols, t, tpr);
+    else if (t == 0) sce_store_ignored<T>(a, row);
+    return;
+  }
+  const T* xr = static_cast<const T*>(a.logits) + i0 * a.x_pitch + outer_level_offset(a.x_lv);
+  const RowSpan<T, true> span(xr, a.cols, t);
+  const float edge = span.load_edge(xr);
+  float m = edge, ml = log2_of_max(m);
+  float s = edge == kNegInf ? 0.f : __builtin_amdgcn_exp2f(fmaf(edge, kLog2e, -ml));
+#pragma nounroll
+  for (int base = 0; base < span.nvec; base += U * tpr) {
+    u32x4 raw[U];
+    if (base + U * tpr <= span.nvec) {   // uniform
+#pragma unroll
+      for (int i = 0; i < U; ++i) raw[i] = span.template load<BWD>(xr, base + i * tpr + t, true);
+    } else {
+#pragma unroll
+      for (int i = 0; i < U; ++i) raw[i] = span.template load<BWD>(xr, base + i * tpr + t, false);
+    }
+    float f[NE];
+#pragma unroll
+    for (int i = 0; i < U; ++i) VecIO<T>::unpack(raw[i], &f[i * VEC]);
+    const float before = ml;
+#pragma unroll
+    for (int e = 0; e < NE; e += 2) m = max3(m, f[e], f[e + 1]);
+    ml = log2_of_max(m);
+    float s4[4] = {s * __builtin_amdgcn_exp2f(before - ml), 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int e = 0; e < NE; ++e) s4[e & 3] += __builtin_amdgcn_exp2f(fmaf(f[e], kLog2e, -ml));
+    s = (s4[0] + s4[1]) + (s4[2] + s4[3]);
+  }
+  if constexpr (!BWD) {
+    MaxSumMaxTuple p;
+    p.v[0] = ml; p.v[1] = s; p.v[2] = m;
+    p = group_allreduce_tuple(p, red, 0, nwaves);
+    if (p.v[0] == kLowestLog2) p.v[1] = sce_lowest_count<T, false>(xr, a.cols, t, tpr, nwaves, red, p.v[2]);   // uniform
+    if (t == 0) sce_store_loss<T>(a, row, label, xr, p);
+  } else {
+    const float g = sce_row_grad<T, float>(a, row);
+    MaxSumTuple p;
+    p.v[0] = ml; p.v[1] = s;
+    p = group_allreduce_tuple(p, red, 0, nwaves);
+    const int lab = sce_label_column(label, a.cols);
+    if (p.v[0] == kLowestLog2) {   // uniform
+      sce_lowest_bwd<T, false>(xr, dxr, a.cols, lab, g, t, tpr, nwaves, red);
+      return;
+    }
+    const float ML = p.v[0];
+    const float scale = g / p.v[1];
+    auto grad = [&](float x, bool at_label) {
+      const float o = __builtin_amdgcn_exp2f(fmaf(x, kLog2e, -ML)) * scale;
+      return at_label ? o - g : o;
+    };
+#pragma nounroll
+    for (int base = (span.nvec - 1) / (U * tpr) * (U * tpr); base >= 0; base -= U * tpr) {
+      u32x4 raw[U];
+#pragma unroll
+      for (int i = 0; i < U; ++i) raw[i] = span.template load<false>(xr, base + i * tpr + t, false);
+#pragma unroll
+      for (int i = 0; i < U; ++i) {
+        const int v = base + i * tpr + t;
+        if (v < span.nvec) {
+          float o[VEC];
+          VecIO<T>::unpack(raw[i], o);
+#pragma unroll
+          for (int j = 0; j < VEC; ++j) o[j] = grad(o[j], false);
+          const int lsub = lab - (span.head + v * VEC);
+          if (uint32_t(lsub) < uint32_t(VEC)) {
+#pragma unroll
+            for (int j = 0; j < VEC; ++j)
+              if (j == lsub) o[j] -= g;
+          }
+          span.store(dxr, v, o);
+        }
+      }
+    }
+    span.store_edge(dxr, grad(edge, span.edge == lab));
   }
 }
 
@@ -316,7 +497,7 @@ void sce_dense_kernel(SceArgs a) {
 }
 
 // ------------------------------- fallback ----------------------------------
-// Any cols / alignment / dtype: one workgroup per row, strided passes.
+// Dense labels of any cols / alignment, and fp64: one workgroup per row, strided passes.
 template <typename T, typename CT>
 struct SceIO {
   static __device__ __forceinline__ CT ld(const T* p) { return CT(Cvt<T>::load(p)); }
@@ -457,12 +638,12 @@ static bool pick_sce_shape(int nvec, int max_nv_wave, int max_nv, int* threads, 
 }
 
 // MODE as in sce_generic_kernel
-template <typename T, int MODE, bool WAVE_ROW>
+template <typename T, int MODE, bool WAVE_ROW, bool RAGGED>
 static int launch_sce_nv(const SceArgs& a, int nv, dim3 grid, dim3 block, hipStream_t s) {
 #define HK_SCE_LAUNCH(N)                                                                         \
   do {                                                                                           \
-    if constexpr (MODE == 0) HK_LAUNCH((sce_sparse_fwd_kernel<T, N, WAVE_ROW>), grid, block, 0, s, a); \
-    else if constexpr (MODE == 1) HK_LAUNCH((sce_sparse_bwd_kernel<T, N, WAVE_ROW>), grid, block, 0, s, a); \
+    if constexpr (MODE == 0) HK_LAUNCH((sce_sparse_fwd_kernel<T, N, WAVE_ROW, RAGGED>), grid, block, 0, s, a); \
+    else if constexpr (MODE == 1) HK_LAUNCH((sce_sparse_bwd_kernel<T, N, WAVE_ROW, RAGGED>), grid, block, 0, s, a); \
     else if constexpr (MODE == 2) HK_LAUNCH((sce_dense_kernel<T, N, WAVE_ROW, false>), grid, block, 0, s, a); \
     else HK_LAUNCH((sce_dense_kernel<T, N, WAVE_ROW, true>), grid, block, 0, s, a);       \
   } while (0)
@@ -490,18 +671,35 @@ static int sce_typed(SceArgs a, hipStream_t s) {
   const bool vec_ok = a.cols % VEC == 0 && aligned16(a.logits) && aligned16(a.dlabels) &&
                       (MODE == 0 || MODE == 2 || (aligned16(a.out) && steps_ok(a.out_pitch, a.out_lv))) &&
                       steps_ok(a.x_pitch, a.x_lv) && (MODE < 2 || steps_ok(a.lab_pitch, a.lab_lv));
-  a.nvec = a.cols / VEC;
+  a.nvec = (a.cols + VEC - 1) / VEC;
   // sparse forward only keeps the packed row; the others keep 32 floats or two rows
   const int max_nv = (MODE == 0) ? 8 : 32 / VEC;
   const int max_nv_wave = (MODE == 0) ? 8 : 32 / VEC;
   int threads = 0, nv = 0;
-  if (vec_ok && pick_sce_shape(a.nvec, max_nv_wave, max_nv, &threads, &nv)) {
+  bool shaped = pick_sce_shape(a.nvec, max_nv_wave, max_nv, &threads, &nv);
+  // the forward of long 16-bit rows is faster streamed than with 64 floats a thread in more than 512 threads
+  // (4096 x 50304 bf16 94 -> 82 us, x 65536 105 -> 89 us; 32000 columns, 512 threads, 155 us against 230 us)
+  if (MODE == 0 && VEC == 8 && a.nvec > 4096) shaped = false;
+  const dim3 levels{unsigned(a.n0), unsigned(a.n1), unsigned(a.n2)};
+  auto launch = [&](auto ragged) {
+    constexpr bool RAGGED = decltype(ragged)::value;
     if (threads == 64) {
       dim3 grid(unsigned((a.n0 + 3) / 4), unsigned(a.n1), unsigned(a.n2)), block(256);
-      return launch_sce_nv<T, MODE, true>(a, nv, grid, block, s);
+      return launch_sce_nv<T, MODE, true, RAGGED>(a, nv, grid, block, s);
     }
-    dim3 grid{unsigned(a.n0), unsigned(a.n1), unsigned(a.n2)}, block{unsigned(threads)};
-    return launch_sce_nv<T, MODE, false>(a, nv, grid, block, s);
+    return launch_sce_nv<T, MODE, false, RAGGED>(a, nv, levels, dim3{unsigned(threads)}, s);
+  };
+  if (vec_ok && shaped) return launch(std::false_type{});
+  if constexpr (MODE < 2) {
+    if (shaped) return launch(std::true_type{});
+    // equal steps: as many threads as the vectors of one step need
+    const int steps = (a.nvec + kLongVecs * kLongThreads - 1) / (kLongVecs * kLongThreads);
+    const int per_step = (a.nvec + steps * kLongVecs - 1) / (steps * kLongVecs);
+    threads = (per_step + 63) / 64 * 64;
+    profile_before(s);
+    HK_LAUNCH((sce_long_kernel<T, MODE == 1>), levels, dim3(unsigned(threads)), 0, s, a);
+    profile_after(s);
+    return launch_check("sce_long_kernel");
   }
   HK_LAUNCH((sce_generic_kernel<T, float, MODE>), dim3(unsigned(a.n0), unsigned(a.n1), unsigned(a.n2)), dim3(256), 0,
             s, a);

@@ -112,3 +112,77 @@ def test_reduce_any_extent(hk, cuda, dtype, shift):
                 assert torch.equal(view.float().cpu().double(), torch.from_numpy(
                     oracle.round_to(np.asarray(expected, np.float32), dtype).astype(np.float64))), what
                 assert bool((out[:GUARD] == 77.0).all()) and bool((out[-GUARD:] == 77.0).all()), what
+
+
+# vectors per row around 1, a wavefront, the widths of the workgroups, and (65536 16-bit / 32768 32-bit elements in the
+# forward, 32768 in the backward) past what a workgroup holds: whole vectors, one element more, one fewer
+def _class_counts(dtype):
+    vec = 16 // ES[dtype]
+    out = {v * vec + k for v in (1, 2, 63, 64, 65, 256, 512, 1000) for k in (0, 1, vec - 1)}
+    out.update(range(1, 2 * vec))
+    out.update((4096 * vec, 4096 * vec + 1, 8192 * vec - 1, 8192 * vec, 8192 * vec + 1, 9000 * vec + 3, 12289 * vec - 1))
+    return sorted(out)
+
+
+@pytest.mark.parametrize("dtype", ["fp32", "bf16", "fp16"])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_cross_entropy_any_length(hk, cuda, dtype, shift):
+    import torch
+    rows, ignored = 9, -100
+    for cols in _class_counts(dtype):
+        pitch = cols + (0 if shift == 0 else 5)
+        x = helpers.draw(6000 + cols, (rows, cols), dtype=dtype)
+        lab = np.array([0, cols - 1, ignored, cols // 2, cols - min(cols, 5), 1 % cols, -7, ignored, max(cols - 2, 0)], np.int64)
+        g = helpers.draw(7000 + cols, (rows,), dtype=dtype)
+        _, tx = _placed(cuda, x, dtype, shift, pitch)
+        tl, tg = torch.from_numpy(lab).to(cuda), helpers.to_torch(g, dtype, cuda)
+        loss = torch.empty(rows, dtype=tx.dtype, device=cuda)
+        hk.sce_sparse_fwd(tx, tl, loss, ignored)
+        db, dx = _placed(cuda, x, dtype, shift, pitch, 0.0)
+        hk.sce_sparse_bwd(tx, tl, tg, dx, ignored)
+        torch.cuda.synchronize()
+        inside = (lab >= 0) | (lab == ignored)     # -7 is no class: the loss is NaN, the gradient has no one-hot term
+        el = oracle.sce_sparse_fwd(x[inside], lab[inside], ignored)
+        helpers.assert_close(loss[torch.from_numpy(inside).to(cuda)], el, dtype, "loss %d" % cols)
+        assert bool(torch.isnan(loss[~torch.from_numpy(inside).to(cuda)]).all())
+        edx = oracle.sce_sparse_bwd(x[inside], lab[inside], g[inside], ignored)
+        helpers.assert_close(dx.contiguous()[torch.from_numpy(inside).to(cuda)], edx, dtype, "dlogits %d" % cols)
+        want = torch.softmax(tx[6].double(), -1) * tg[6].double()
+        helpers.assert_close(dx[6].contiguous(), want.cpu().numpy(), dtype, "dlogits of no class %d" % cols)
+        assert _guards_untouched(db, dx), cols
+        hk.sce_sparse_bwd(tx, tl, tg, tx, ignored)     # in place
+        torch.cuda.synchronize()
+        assert torch.equal(tx.contiguous(), dx.contiguous()), cols
+
+
+@pytest.mark.parametrize("dtype", ["fp32", "bf16", "fp16"])
+@pytest.mark.parametrize("cols", [40, 41, 1001, 4096, 50257, 70001])
+def test_cross_entropy_of_lowest_values(hk, cuda, dtype, cols):
+    """Logits masked with the type's lowest value (whole threads' share of a row, and whole rows), -inf, +inf and NaN."""
+    import torch
+    dt = {"fp32": torch.float32, "bf16": torch.bfloat16, "fp16": torch.float16}[dtype]
+    low = torch.finfo(dt).min
+    x = helpers.to_torch(helpers.draw(8000 + cols, (8, cols), dtype=dtype), dtype, cuda)
+    x[0, 3:] = low
+    x[1, : cols - 2] = -float("inf")
+    x[2, :] = low
+    x[3, :] = low
+    x[3, 5] = low / 1.25
+    x[4, :] = -float("inf")
+    x[5, cols // 2] = float("nan")
+    x[6, cols - 1] = float("inf")
+    lab = torch.tensor([1, cols - 1, 7, 5, 0, 0, 0, cols - 1], device=cuda)
+    g = torch.ones(8, dtype=dt, device=cuda)
+    loss, dx = torch.empty(8, dtype=dt, device=cuda), torch.empty_like(x)
+    hk.sce_sparse_fwd(x, lab, loss, -100)
+    hk.sce_sparse_bwd(x, lab, g, dx, -100)
+    torch.cuda.synchronize()
+    p = torch.softmax(x.double(), -1)
+    want = torch.nn.functional.cross_entropy(x.double(), lab, reduction="none")
+    p[torch.arange(8, device=cuda), lab] -= 1
+    for r in range(8):
+        assert bool(torch.isnan(loss[r])) == bool(torch.isnan(want[r])), r
+        assert torch.equal(torch.isnan(dx[r]), torch.isnan(p[r])), r
+    ok = [0, 1, 2, 3, 7]
+    helpers.assert_close(loss[ok], want[ok].cpu().numpy(), dtype, "loss")
+    helpers.assert_close(dx[ok], p[ok].cpu().numpy(), dtype, "dlogits")
