@@ -83,7 +83,12 @@ void softmax_fwd_kernel(SoftmaxArgs a) {
   // exponentials, and an element held twice then comes out the same twice.  Across wavefronts each thread keeps its
   // own maximum and the pairs are merged, which costs one barrier instead of two.
   if constexpr (LPR > 0) m = Lanes::allreduce(MaxTuple{{m}}, red).v[0];
-  const float ml = (m == kNegInf) ? 0.f : m * kLog2e;
+  // A row whose maximum lies at the type's lowest values (scores masked with it) would overflow in the log2 domain: two
+  // different values down there are so far apart that any base gives 1 at the maximum and 0 elsewhere, so lanes that
+  // agree on the row's maximum take base 2 for such a row.  A whole workgroup's threads have maxima of their own, kept
+  // finite by log2_of_max(), and the row is counted below.
+  const float k = (LPR > 0 && m < -2.3e38f) ? 1.0f : kLog2e;
+  const float ml = LPR > 0 ? m * k : log2_of_max(m);
   float s = 0.f;
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
@@ -91,22 +96,31 @@ void softmax_fwd_kernel(SoftmaxArgs a) {
 #pragma unroll
     for (int j = 0; j < VEC; ++j) {
       float& x = e[i * VEC + j];
-      x = __builtin_amdgcn_exp2f(fmaf(x, kLog2e, -ml));
+      x = __builtin_amdgcn_exp2f(fmaf(x, k, -ml));
       s += (RAGGED && j < skip) ? 0.f : x;
     }
   }
+  T* yr = static_cast<T*>(a.out) + row * a.out_pitch + outer_level_offset(a.out_lv);
   float scale;
   if constexpr (LPR > 0) {
     scale = 1.0f / Lanes::allreduce(SumTuple<1>{{s}}, red).v[0];
   } else {
     MaxSumTuple p;
-    p.v[0] = (m == kNegInf) ? kNegInf : ml; p.v[1] = s;
+    p.v[0] = ml; p.v[1] = s;
     p = Lanes::allreduce(p, red);
-    const float ML = (p.v[0] == kNegInf) ? 0.f : p.v[0];
-    scale = __builtin_amdgcn_exp2f(ml - ML) / p.v[1];
+    if (p.v[0] == kLowestLog2) {   // uniform: a row of the type's lowest values
+      float M;
+      const float n = row_max_count<T>(xr, a.cols, t, tpr, [&](auto v) {
+        __syncthreads();   // red may still be read
+        return Lanes::allreduce(v, red);
+      }, M);
+      const float inv = 1.0f / (M == kNegInf ? __builtin_nanf("") : n);   // nothing but -inf has no softmax
+      for (int c = t; c < a.cols; c += tpr) Cvt<T>::store(yr + c, (Cvt<T>::load(xr + c) == M ? 1.f : 0.f) * inv);
+      return;
+    }
+    scale = __builtin_amdgcn_exp2f(ml - p.v[0]) / p.v[1];
   }
 
-  T* yr = static_cast<T*>(a.out) + row * a.out_pitch + outer_level_offset(a.out_lv);
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
     const int v = i * tpr + t;

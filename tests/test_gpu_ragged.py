@@ -114,6 +114,34 @@ def test_reduce_any_extent(hk, cuda, dtype, shift):
                 assert bool((out[:GUARD] == 77.0).all()) and bool((out[-GUARD:] == 77.0).all()), what
 
 
+@pytest.mark.parametrize("dtype", ["fp32", "bf16", "fp16"])
+@pytest.mark.parametrize("cols", [3, 40, 41, 130, 1001, 2047, 2048, 4097])
+def test_softmax_of_lowest_values(hk, cuda, dtype, cols):
+    """Scores masked with the type's lowest value (whole threads' share of a row, and whole rows), -inf, +inf and NaN."""
+    import torch
+    dt = {"fp32": torch.float32, "bf16": torch.bfloat16, "fp16": torch.float16}[dtype]
+    low = torch.finfo(dt).min
+    x = helpers.to_torch(helpers.draw(9000 + cols, (8, cols), dtype=dtype), dtype, cuda)
+    x[0, 2:] = low
+    x[1, : cols - 2] = -float("inf")
+    x[2, :] = low
+    x[3, :] = low
+    x[3, 1] = low / 1.25
+    x[4, :] = -float("inf")
+    x[5, cols // 2] = float("nan")
+    x[6, cols - 1] = float("inf")
+    y = torch.empty_like(x)
+    hk.softmax_fwd(x, y)
+    torch.cuda.synchronize()
+    want = torch.softmax(x.double(), -1)
+    assert torch.equal(torch.isnan(y), torch.isnan(want))
+    ok = [0, 1, 2, 3, 7]
+    helpers.assert_close(y[ok], want[ok].cpu().numpy(), dtype, "softmax y")
+    hk.softmax_fwd(x, x)
+    torch.cuda.synchronize()
+    assert torch.equal(x[ok], y[ok])
+
+
 # vectors per row around 1, a wavefront, the widths of the workgroups, and (65536 16-bit / 32768 32-bit elements in the
 # forward, 32768 in the backward) past what a workgroup holds: whole vectors, one element more, one fewer
 def _class_counts(dtype):
