@@ -491,6 +491,24 @@ __device__ __forceinline__ P group_allreduce_tuple_fixed(P a, float* scratch) {
   return r;
 }
 
+// Which lanes hold a row.  LPR > 0: LPR neighbouring lanes of a wavefront (8, 16, 32 or all 64), 256 / LPR rows per
+// workgroup; LPR == 0: the whole workgroup.
+template <int LPR>
+struct RowLanes {
+  static __device__ __forceinline__ int count() { return LPR ? LPR : int(blockDim.x); }
+  static __device__ __forceinline__ int lane() { return LPR ? int(threadIdx.x) & (LPR - 1) : int(threadIdx.x); }
+  static __device__ __forceinline__ int64_t row() {
+    if constexpr (LPR == 0) return int64_t(blockIdx.x);
+    else if constexpr (LPR == kWave) return int64_t(blockIdx.x) * (256 / kWave) + wave_index();
+    else return int64_t(blockIdx.x) * (256 / LPR) + int(threadIdx.x) / LPR;
+  }
+  template <typename P>
+  static __device__ __forceinline__ P allreduce(P p, float* red) {
+    if constexpr (LPR == 0) return group_allreduce_tuple(p, red, 0, int(blockDim.x >> 6));
+    else return lanes_allreduce_tuple<LPR>(p);
+  }
+};
+
 // f(std::integral_constant<int, 0>{}), ..., f(std::integral_constant<int, N - 1>{}): a loop whose index is a
 // compile-time constant in every iteration
 template <typename F, int... D>

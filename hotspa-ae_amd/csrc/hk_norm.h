@@ -60,6 +60,7 @@ struct NormBwdArgs {
   LevelSteps dy_lv, x_lv, dx_lv, dxin_lv, dres_lv;
   int cols;
   int nvec;
+  int part_pitch;       // elements between partial rows: cols rounded up to whole vectors
   int tpr;              // threads per row (multiple of 64)
   float eps;
   float inv_cols;
@@ -70,6 +71,7 @@ struct NormBwdArgs {
 
 struct BwdPlan {
   bool reg_path;
+  bool any;             // the instance for rows of any length and alignment
   int tpr, nv, rpb, grid;
   int block;
   size_t lds_bytes;

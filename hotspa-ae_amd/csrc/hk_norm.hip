@@ -173,18 +173,20 @@ int hk_norm_bwd_workspace_bytes(int dtype, int64_t rows, int64_t cols, size_t* b
              "hk_norm_bwd_workspace_bytes: bad shape");
   *bytes = 0;
   if (rows == 0 || cols == 0) return HK_OK;
-  BwdPlan p{};
+  // for operands on the 16-byte grid and off it
+  auto need = [&](auto plan) {
+    const BwdPlan on = plan(rows, int(cols), true), off = plan(rows, int(cols), false);
+    return std::max(on.reg_path ? on.ws_bytes : 0, off.reg_path ? off.ws_bytes : 0);
+  };
   switch (dtype) {
-    case HK_FLOAT32: p = plan_norm_bwd<float>(rows, int(cols), true); break;
-    case HK_BFLOAT16: p = plan_norm_bwd<bf16>(rows, int(cols), true); break;
-    case HK_FLOAT16: p = plan_norm_bwd<fp16>(rows, int(cols), true); break;
+    case HK_FLOAT32: *bytes = need(plan_norm_bwd<float>); return HK_OK;
+    case HK_BFLOAT16: *bytes = need(plan_norm_bwd<bf16>); return HK_OK;
+    case HK_FLOAT16: *bytes = need(plan_norm_bwd<fp16>); return HK_OK;
     case HK_FLOAT64: return HK_OK;
     default:
       set_last_error("hk_norm_bwd_workspace_bytes: not implemented for dtype %d", dtype);
       return HK_ERR_UNSUPPORTED;
   }
-  *bytes = p.reg_path ? p.ws_bytes : 0;
-  return HK_OK;
 }
 
 int hk_layer_norm_bwd_strided_rows(int dtype, const void* dy, const int64_t dy_steps[3], const void* x_or_y,

@@ -55,11 +55,19 @@ __device__ __forceinline__ float clamp_by_magnitude(float g, float eps) {
 // issue is kept as a running (j0, j1, j2) in scalar registers and advanced by the split grid size with two
 // carries: no division in the loop, nothing on the vector unit.  The general instance takes levels too, with
 // optional operands, by splitting each row number with two divisions.
+//
+// RAGGED: rows of any length and alignment, see AnyBoundary.  The row's partial last vector is
+// read as its last whole one; the elements that it shares with the vector before it are zeroed in x and dy, add nothing
+// and are not stored.  The partial rows of the column sums keep whole vectors (part_pitch).  LayerNorm backward of
+// 8191 x 1021 bf16: 1114 us element by element -> 22.5 us, of 10000 x 8191 2121 -> 142 us (3.5 TB/s; 8192 columns on
+// the 16-byte grid 93 us: what is left is the extra cache lines of accesses on odd 2-byte boundaries), of
+// 8192 x 8191 fp32 1328 -> 150 us (5.4 TB/s).
 template <typename T, int NV, int MODE, int PF, bool EXACT, bool STATS_F32, bool EXTRA, int MAXT, bool FIXED,
-          bool CLAMP, bool LEVELS = false>
+          bool CLAMP, bool LEVELS = false, bool RAGGED = false>
 __global__ __launch_bounds__(MAXT)
 void norm_bwd_kernel(NormBwdArgs a) {
   static_assert(!LEVELS || (FIXED && !EXTRA && EXACT), "the running walk index is built for the lean instances");
+  static_assert(!RAGGED || (!FIXED && !EXACT), "rows of any boundary: any group width, a partial last vector");
   constexpr int VEC = VecIO<T>::N;
   constexpr int NE = NV * VEC;
   constexpr int KS = (MODE == BWD_RMS) ? 1 : 2;   // row sums to reduce: RMSNorm has no mean term
@@ -80,12 +88,23 @@ void norm_bwd_kernel(NormBwdArgs a) {
   // again and has its dy forced to zero, so it adds nothing and stores nothing
   int vidx[NV];
   bool vin[NV];
+  int col[NV];                            // first column that vector i loads
+  [[maybe_unused]] u32x4 own[NV];         // RAGGED: the bits of a loaded vector that belong to this thread
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
     const int v = i * tpr + t;
     vin[i] = EXACT || v < a.nvec;
     vidx[i] = vin[i] ? v : a.nvec - 1;
+    col[i] = vec_column<T, RAGGED>(vidx[i], a.cols);
+    if constexpr (RAGGED) {
+      const int skip = (v + 1) * VEC - a.cols;
+      constexpr int PER = 4 / int(sizeof(T));   // elements per dword
+#pragma unroll
+      for (int d = 0; d < 4; ++d) own[i][d] = skip >= (d + 1) * PER ? 0u : (skip <= d * PER ? 0xffffffffu : 0xffff0000u);
+    }
   }
+  auto ld_row = [](const T* p) { if constexpr (RAGGED) return ld16_any<T>(p); else return ld16(p); };
+  auto ld_par = [](const T* p) { if constexpr (RAGGED) return ld16_any_keep<T>(p); else return ld16_keep(p); };
 
   // gamma (and beta) of this thread's columns as fp32; a missing gamma is all ones
   float gm[NE];
@@ -97,11 +116,11 @@ void norm_bwd_kernel(NormBwdArgs a) {
     for (int i = 0; i < NV; ++i) {
 #pragma unroll
       for (int j = 0; j < VEC; ++j) gm[i * VEC + j] = 1.f;
-      if (gp) VecIO<T>::unpack(ld16_keep(gp + vidx[i] * VEC), &gm[i * VEC]);
+      if (gp) VecIO<T>::unpack(ld_par(gp + col[i]), &gm[i * VEC]);
       if constexpr (MODE == BWD_LN_MEMEFF) {
 #pragma unroll
         for (int j = 0; j < VEC; ++j) bt[i * VEC + j] = 0.f;
-        if (bp) VecIO<T>::unpack(ld16_keep(bp + vidx[i] * VEC), &bt[i * VEC]);
+        if (bp) VecIO<T>::unpack(ld_par(bp + col[i]), &bt[i * VEC]);
       }
     }
   }
@@ -162,8 +181,8 @@ void norm_bwd_kernel(NormBwdArgs a) {
     const T* dyr = static_cast<const T*>(a.dy) + dyo;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
-      nx[d][i] = ld16(xr + vidx[i] * VEC);
-      ndy[d][i] = ld16(dyr + vidx[i] * VEC);
+      nx[d][i] = ld_row(xr + col[i]);
+      ndy[d][i] = ld_row(dyr + col[i]);
     }
   };
   int64_t row0 = int64_t(blockIdx.x) * rpb + group;
@@ -179,9 +198,13 @@ void norm_bwd_kernel(NormBwdArgs a) {
     float xs[NE], ts[NE];                 // xc (x_hat in the memory-efficient mode) and dy * gamma
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
+      if constexpr (RAGGED) {
+        nx[d][i] &= own[i];
+        ndy[d][i] &= own[i];
+      }
       VecIO<T>::unpack(nx[d][i], &xs[i * VEC]);
       VecIO<T>::unpack(ndy[d][i], &ts[i * VEC]);
-      if (!EXACT) {
+      if (!EXACT && !RAGGED) {
 #pragma unroll
         for (int j = 0; j < VEC; ++j) ts[i * VEC + j] = vin[i] ? ts[i * VEC + j] : 0.f;
       }
@@ -276,15 +299,20 @@ void norm_bwd_kernel(NormBwdArgs a) {
           if constexpr (EXTRA) {
             if (dir) {
               float u[VEC];
-              VecIO<T>::unpack(ld16(dir + v * VEC), u);
+              VecIO<T>::unpack(ld_row(dir + col[i]), u);
 #pragma unroll
               for (int j = 0; j < VEC; ++j) o[j] += u[j];
             }
           }
-          const u32x4 pk = VecIO<T>::pack(o);
-          st16_stream(dxr + v * VEC, pk);
-          if constexpr (EXTRA) {
-            if (drr) st16(drr + v * VEC, pk);
+          if constexpr (RAGGED) {
+            store_row_vec<T, true, false>(dxr, v, o, a.cols);
+            if (drr) store_row_vec<T, true, false>(drr, v, o, a.cols);
+          } else {
+            const u32x4 pk = VecIO<T>::pack(o);
+            st16_stream(dxr + v * VEC, pk);
+            if constexpr (EXTRA) {
+              if (drr) st16(drr + v * VEC, pk);
+            }
           }
         }
       }
@@ -317,7 +345,7 @@ void norm_bwd_kernel(NormBwdArgs a) {
     for (int which = 0; which < (WITH_DB ? 2 : 1); ++which) {
       if (outs[which] == nullptr) continue;
       const float* acc = which == 0 ? dg : db;
-      float* dst = outs[which] + int64_t(blockIdx.x) * a.cols;
+      float* dst = outs[which] + int64_t(blockIdx.x) * a.cols;   // whole vectors: part_pitch == cols
 #pragma unroll
       for (int i = 0; i < NV; ++i) {
 #pragma unroll
@@ -341,13 +369,13 @@ void norm_bwd_kernel(NormBwdArgs a) {
         const int v = i * tpr + t;
         if (v < a.nvec) {
 #pragma unroll
-          for (int j = 0; j < VEC; ++j) lds[group * a.cols + v * VEC + j] = acc[i * VEC + j];
+          for (int j = 0; j < VEC; ++j) lds[group * a.part_pitch + v * VEC + j] = acc[i * VEC + j];
         }
       }
       __syncthreads();
     }
     if (group == 0) {
-      float* dst = outs[which] + int64_t(blockIdx.x) * a.cols;
+      float* dst = outs[which] + int64_t(blockIdx.x) * a.part_pitch;
 #pragma unroll
       for (int i = 0; i < NV; ++i) {
         const int v = i * tpr + t;
@@ -355,7 +383,7 @@ void norm_bwd_kernel(NormBwdArgs a) {
 #pragma unroll
           for (int j = 0; j < VEC; ++j) {
             float r = acc[i * VEC + j];
-            for (int g = 1; g < rpb; ++g) r += lds[g * a.cols + v * VEC + j];
+            for (int g = 1; g < rpb; ++g) r += lds[g * a.part_pitch + v * VEC + j];
             dst[v * VEC + j] = r;
           }
         }
@@ -364,7 +392,9 @@ void norm_bwd_kernel(NormBwdArgs a) {
   }
 }
 
-// Folds the [nparts, cols] fp32 partial rows into dgamma / dbeta of type T.
+// Folds the [nparts, pitch] fp32 partial rows into dgamma / dbeta of type T.  Rows of whole 16-byte vectors of T:
+// pitch == cols; otherwise the last vector of a partial row holds the row's last columns, the first pitch - cols of
+// its elements being another vector's.
 // blockIdx.y picks dgamma / dbeta; a block covers 128 columns as 32 float4
 // column groups x 16 row slices, every slice keeps 8 independent loads in
 // flight, slices are folded through LDS.
@@ -372,7 +402,7 @@ template <typename T>
 __global__ __launch_bounds__(512)
 void norm_bwd_finalize_kernel(const float* __restrict__ part_dgamma,
                               const float* __restrict__ part_dbeta, T* dgamma, T* dbeta,
-                              int nparts, int cols) {
+                              int nparts, int cols, int pitch) {
   constexpr int U = 8;
   __shared__ float lds[16][32][4];
   const float* part = blockIdx.y == 0 ? part_dgamma : part_dbeta;
@@ -381,19 +411,19 @@ void norm_bwd_finalize_kernel(const float* __restrict__ part_dgamma,
   const int cg = threadIdx.x & 31, slice = threadIdx.x >> 5;
   const int c = (blockIdx.x * 32 + cg) * 4;
   float acc[4] = {0.f, 0.f, 0.f, 0.f};
-  if (c < cols) {                                     // cols is a multiple of 4 on this path
+  if (c < pitch) {                                    // a multiple of 4
     int r = slice;
     for (; r + (U - 1) * 16 < nparts; r += U * 16) {
       u32x4 v[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) v[u] = ld16_keep(part + int64_t(r + u * 16) * cols + c);
+      for (int u = 0; u < U; ++u) v[u] = ld16_keep(part + int64_t(r + u * 16) * pitch + c);
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         acc[0] += u2f(v[u].x); acc[1] += u2f(v[u].y); acc[2] += u2f(v[u].z); acc[3] += u2f(v[u].w);
       }
     }
     for (; r < nparts; r += 16) {
-      const u32x4 v = ld16_keep(part + int64_t(r) * cols + c);
+      const u32x4 v = ld16_keep(part + int64_t(r) * pitch + c);
       acc[0] += u2f(v.x); acc[1] += u2f(v.y); acc[2] += u2f(v.z); acc[3] += u2f(v.w);
     }
   }
@@ -406,11 +436,14 @@ void norm_bwd_finalize_kernel(const float* __restrict__ part_dgamma,
     float s = 0.f;
 #pragma unroll
     for (int sl = 0; sl < 16; ++sl) s += lds[sl][g][k];
-    if (oc < cols) Cvt<T>::store(out + oc, s);
+    const int shift = pitch - cols, tail = pitch - VecIO<T>::N;   // shift > 0: the partial last vector
+    if (shift == 0 || oc < tail) { if (oc < cols) Cvt<T>::store(out + oc, s); }
+    else if (oc >= tail + shift && oc < pitch) Cvt<T>::store(out + oc - shift, s);
   }
 }
 
-// Fallback backward for rows the register kernel cannot take: one workgroup
+// Fallback backward for rows the register kernel cannot take (shorter than a 16-byte vector, more than 8192 columns,
+// no scratch given for rows off the 16-byte grid): one workgroup
 // per row for dx, then a column kernel for dgamma / dbeta (re-reads dy and x).
 template <typename T, typename CT>
 __global__ __launch_bounds__(256)
@@ -530,12 +563,38 @@ void norm_bwd_generic_cols_kernel(NormBwdArgs a, int mode, T* dgamma, T* dbeta) 
   }
 }
 
+// Rows that the aligned plan does not take: the general instance at 8 columns per thread (bf16, fp16; 4 for short fp32
+// rows), one 1024-thread workgroup per compute unit, as many rows per step as fit it.  The partial rows stay within
+// 16 MiB (what the library's own scratch holds) by using fewer workgroups for the longest rows.
+template <typename T>
+BwdPlan plan_norm_bwd_any(int64_t rows, int cols) {
+  constexpr int VEC = VecIO<T>::N;
+  BwdPlan p{};
+  if (cols < VEC) return p;
+  const int nvec = (cols + VEC - 1) / VEC, pitch = nvec * VEC;
+  const int nv = VEC == 4 && nvec > 1024 ? 2 : 1;
+  const int tpr = ((nvec + nv - 1) / nv + 63) / 64 * 64;
+  if (tpr > 1024) return p;
+  int rpb = std::max(1, 1024 / tpr);
+  while (rpb > 1 && size_t(rpb) * pitch * sizeof(float) > 65536) --rpb;
+  int64_t grid = tune_get(TUNE_NORM_BWD_BLOCKS);
+  if (grid <= 0) grid = device_cu_count();
+  grid = std::min<int64_t>(grid, (rows + rpb - 1) / rpb);
+  grid = std::min<int64_t>(grid, (int64_t(16) << 20) / (int64_t(2) * pitch * int64_t(sizeof(float))));
+  if (grid < 1) grid = 1;
+  p.reg_path = p.any = true;
+  p.tpr = tpr; p.nv = nv; p.rpb = rpb; p.grid = int(grid); p.block = tpr * rpb;
+  p.lds_bytes = rpb > 1 ? size_t(rpb) * pitch * sizeof(float) : 0;
+  p.ws_bytes = size_t(2) * size_t(grid) * pitch * sizeof(float);
+  return p;
+}
+
 template <typename T>
 BwdPlan plan_norm_bwd(int64_t rows, int cols, bool aligned) {
   constexpr int VEC = VecIO<T>::N;
   BwdPlan p{};
   p.reg_path = false;
-  if (!aligned || cols % VEC != 0) return p;
+  if (!aligned || cols % VEC != 0) return plan_norm_bwd_any<T>(rows, cols);
   const int nvec = cols / VEC;
   // column-owner kernel: the dgamma / dbeta accumulators of a thread must stay
   // in registers: 8 columns per thread by default, 16 when a thread count is forced
@@ -545,17 +604,17 @@ BwdPlan plan_norm_bwd(int64_t rows, int cols, bool aligned) {
   if (tpr > 0) {
     tpr = std::min(1024, std::max(64, (tpr + 63) / 64 * 64));
     nv = pow2_ceil((nvec + tpr - 1) / tpr);
-    if (nv > max_nv) return p;
+    if (nv > max_nv) return plan_norm_bwd_any<T>(rows, cols);
   } else {
     nv = max_nv;
     // short rows: fewer vectors per thread rather than a partly idle wavefront
     while (nv > 1 && (nvec + nv - 1) / nv < 64) nv >>= 1;
     tpr = ((nvec + nv - 1) / nv + 63) / 64 * 64;
-    if (tpr > 1024) return p;
+    if (tpr > 1024) return plan_norm_bwd_any<T>(rows, cols);
   }
   // kernels with more than one vector per thread are built for 512-thread blocks
   const int max_block = nv == 1 ? 1024 : 512;
-  if (tpr > max_block) return p;
+  if (tpr > max_block) return plan_norm_bwd_any<T>(rows, cols);
   int rpb = tune_get(TUNE_NORM_BWD_ROWS_PER_BLOCK);
   if (rpb <= 0) {
     rpb = std::max(1, max_block / tpr);
@@ -637,6 +696,42 @@ static int launch_norm_bwd_inst(const NormBwdArgs& a, const BwdPlan& p, int pf, 
 }
 
 template <typename T, int MODE>
+static int launch_norm_bwd_any(const NormBwdArgs& a, const BwdPlan& p, hipStream_t s) {
+  const dim3 grid{unsigned(p.grid)}, block{unsigned(p.block)};
+#define HK_BWD_ANY_P(P, NV, F, X) \
+  HK_LAUNCH((norm_bwd_kernel<T, NV, MODE, P, false, F, X, 1024, false, false, false, true>), grid, block, p.lds_bytes, s, a)
+#define HK_BWD_ANY(NV, F) HK_BWD_ANY_P(1, NV, F, true)
+  const bool extra = a.dx_in != nullptr || a.dres != nullptr || a.clamp_gamma != 0 || a.n0 != a.rows ||
+                     (MODE == BWD_RMS && a.part_dbeta != nullptr) || !a.stats_f32;
+  profile_before(s);
+  if constexpr (MODE != BWD_LN_MEMEFF) {
+    if (!extra) {
+      // two rows in flight where a workgroup holds few groups and is not full (16384 x 5001 bf16 LayerNorm 122 -> 109 us,
+      // x 3001 66 -> 61); one otherwise (x 2047 46 against 50 us, 10000 x 8191 142 against 148, 8192 x 8191 fp32 150
+      // against 190)
+      if constexpr (VecIO<T>::N == 4) {
+        if (p.nv == 2) HK_BWD_ANY_P(1, 2, true, false); else HK_BWD_ANY_P(1, 1, true, false);
+      } else {
+        if (p.tpr > 256 && p.tpr < 1024) HK_BWD_ANY_P(2, 1, true, false); else HK_BWD_ANY_P(1, 1, true, false);
+      }
+      profile_after(s);
+      return launch_check("norm_bwd_kernel");
+    }
+  }
+  if constexpr (VecIO<T>::N == 4) {
+    if (p.nv == 2) HK_BWD_ANY(2, true); else HK_BWD_ANY(1, true);   // statistics "in the data type" are the same
+  } else if constexpr (MODE == BWD_LN) {
+    if (a.stats_f32) HK_BWD_ANY(1, true); else HK_BWD_ANY(1, false);
+  } else {
+    HK_BWD_ANY(1, true);
+  }
+#undef HK_BWD_ANY
+#undef HK_BWD_ANY_P
+  profile_after(s);
+  return launch_check("norm_bwd_kernel");
+}
+
+template <typename T, int MODE>
 static int launch_norm_bwd_nv(const NormBwdArgs& a, const BwdPlan& p, hipStream_t s) {
   int pf = tune_get(TUNE_NORM_BWD_PREFETCH);
   // Rows in flight per thread group, measured on the lean instances: at 512 threads per row (4096 bf16 columns,
@@ -650,6 +745,7 @@ static int launch_norm_bwd_nv(const NormBwdArgs& a, const BwdPlan& p, hipStream_
     set_last_error("norm_bwd: this mode keeps its statistics in float32");
     return HK_ERR_INVALID;
   }
+  if (p.any) return launch_norm_bwd_any<T, MODE>(a, p, s);
   const int bound = bound_for(p.block);
   const bool have_kernel = p.nv == 1 || p.nv == 2 || (p.nv == 4 && VecIO<T>::N == 4);
   if (!have_kernel) {
@@ -685,6 +781,10 @@ int norm_bwd_typed(NormBwdArgs a, int mode, void* dgamma, void* dbeta, void* ws,
                        steps_ok(a.dy_pitch, a.dy_lv) && steps_ok(a.x_pitch, a.x_lv) && steps_ok(a.dx_pitch, a.dx_lv) &&
                        (!a.dx_in || steps_ok(a.dxin_pitch, a.dxin_lv)) && (!a.dres || steps_ok(a.dres_pitch, a.dres_lv));
   BwdPlan p = plan_norm_bwd<T>(a.rows, a.cols, aligned);
+  const bool want_cols = dgamma != nullptr || dbeta != nullptr;
+  // rows that once took no scratch do without it still
+  if (p.any && want_cols && (ws == nullptr || ws_bytes < p.ws_bytes || !aligned16(ws))) p.reg_path = false;
+  if (p.any && !a.stats_f32 && mode != BWD_LN) p.reg_path = false;
   if (!p.reg_path) {
     HK_LAUNCH((norm_bwd_generic_dx_kernel<T, float>), dim3(unsigned(a.n0), unsigned(a.n1), unsigned(a.n2)), dim3(256),
               0, s, a, mode);
@@ -697,19 +797,19 @@ int norm_bwd_typed(NormBwdArgs a, int mode, void* dgamma, void* dbeta, void* ws,
     }
     return rc;
   }
-  const bool want_cols = dgamma != nullptr || dbeta != nullptr;
+  a.nvec = (a.cols + VEC - 1) / VEC;
+  a.part_pitch = a.nvec * VEC;
   if (want_cols) {
     HK_REQUIRE(ws != nullptr && ws_bytes >= p.ws_bytes, HK_ERR_WORKSPACE,
                "norm_bwd: workspace of %zu bytes needed, %zu given", p.ws_bytes, ws_bytes);
     HK_REQUIRE(aligned16(ws), HK_ERR_INVALID, "norm_bwd: workspace must be 16-byte aligned");
     a.part_dgamma = dgamma ? static_cast<float*>(ws) : nullptr;
-    a.part_dbeta = dbeta ? static_cast<float*>(ws) + size_t(p.grid) * a.cols : nullptr;
+    a.part_dbeta = dbeta ? static_cast<float*>(ws) + size_t(p.grid) * a.part_pitch : nullptr;
   } else {
     a.part_dgamma = nullptr;
     a.part_dbeta = nullptr;
   }
   a.tpr = p.tpr;
-  a.nvec = a.cols / VecIO<T>::N;
   {
     // the walking kernel's row stride, split over the walk levels (used by the instances with a running walk index)
     const uint64_t stride = uint64_t(p.grid) * uint64_t(p.rpb);
@@ -725,9 +825,9 @@ int norm_bwd_typed(NormBwdArgs a, int mode, void* dgamma, void* dbeta, void* ws,
     default: rc = launch_norm_bwd_nv<T, BWD_LN_MEMEFF>(a, p, s); break;
   }
   if (rc != HK_OK || !want_cols) return rc;
-  HK_LAUNCH((norm_bwd_finalize_kernel<T>), dim3(unsigned((a.cols + 127) / 128), 2), dim3(512), 0, s,
+  HK_LAUNCH((norm_bwd_finalize_kernel<T>), dim3(unsigned((a.part_pitch + 127) / 128), 2), dim3(512), 0, s,
                      a.part_dgamma, a.part_dbeta, static_cast<T*>(dgamma), static_cast<T*>(dbeta),
-                     p.grid, a.cols);
+                     p.grid, a.cols, a.part_pitch);
   return launch_check("norm_bwd_finalize_kernel");
 }
 

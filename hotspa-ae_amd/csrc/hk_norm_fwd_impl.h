@@ -235,9 +235,127 @@ void norm_fwd_kernel(NormFwdArgs a) {
   else epilogue(std::false_type{}, std::false_type{});
 }
 
-// Fallback for rows that are not a whole number of 16-byte vectors, are not
-// 16-byte aligned, or do not fit the register file: one workgroup per row,
-// three strided passes (the re-reads hit L2).  CT is the arithmetic type.
+// Rows of any length and alignment (see AnyBoundary), and rows so short that several share a wavefront (LPR, see
+// RowLanes).  The row's partial last vector is read as its last whole one: the elements it shares with the vector
+// before it are left out of the sums and stored twice, to the same bits.  The residual sum goes out after the first
+// reduction: it may replace x or the residual in place, and every lane of the row has read its vectors by then.
+// Bound by HBM and, for odd rows, by the extra cache lines of accesses that straddle them (LayerNorm, bf16:
+// 8191 x 1021 30.7 us element by element -> 11.4 us, of which 10 are the call's own; 16384 x 2047 100 -> 30.5 us, 4.4
+// TB/s, 2048 columns 25 us; 10000 x 8191 290 -> 81 us; 8192 x 8191 fp32 219 -> 99 us, 5.4 TB/s).
+template <typename T, int NV, int LPR, bool HAS_RES, bool IS_RMS>
+__global__ __launch_bounds__(LPR ? 256 : 1024)
+void norm_fwd_any_kernel(NormFwdArgs a) {
+  constexpr int VEC = VecIO<T>::N;
+  using Lanes = RowLanes<LPR>;
+  __shared__ float red[2][kMaxWaves * 2];
+  const int tpr = Lanes::count(), t = Lanes::lane();
+  const int64_t row = Lanes::row();
+  if (LPR && row >= a.n0) return;   // row counts within the innermost level
+
+  float v[NV][VEC];
+  {
+    const T* xr = static_cast<const T*>(a.x) + row * a.x_pitch + outer_level_offset(a.x_lv);
+    const T* rr = HAS_RES ? static_cast<const T*>(a.residual) + row * a.res_pitch + outer_level_offset(a.res_lv) : nullptr;
+    u32x4 raw[NV];
+    [[maybe_unused]] u32x4 res[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int c = vec_column<T, true>(i * tpr + t, a.cols);
+      raw[i] = ld16_any<T>(xr + c);
+      if constexpr (HAS_RES) res[i] = ld16_any<T>(rr + c);
+    }
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      VecIO<T>::unpack(raw[i], v[i]);
+      if constexpr (HAS_RES) {
+        float f[VEC];
+        VecIO<T>::unpack(res[i], f);
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) v[i][j] += f[j];
+      }
+    }
+  }
+  // f(element) over the thread's elements, each element of the row once
+  auto each = [&](auto f) {
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      if ((i + 1) * tpr * VEC <= a.cols) {   // uniform: whole vectors in every lane
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) f(v[i][j]);
+      } else {
+        const int skip = (i * tpr + t + 1) * VEC - a.cols;   // elements of earlier vectors
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) f(j < skip ? 0.f : v[i][j]);
+      }
+    }
+  };
+  auto store_sum = [&] {
+    if constexpr (HAS_RES) {
+      if (a.x_out) {
+        T* xo = static_cast<T*>(a.x_out) + row * a.xout_pitch + outer_level_offset(a.xout_lv);
+#pragma unroll
+        for (int i = 0; i < NV; ++i)
+          if (i * tpr + t < a.nvec) store_row_vec<T, true, true>(xo, i * tpr + t, v[i], a.cols);
+      }
+    }
+  };
+
+  float mu, rs, var;
+  if constexpr (IS_RMS) {
+    SumTuple<2> both = SumTuple<2>::identity();
+    each([&](float x) { both.v[0] = fmaf(x, x, both.v[0]); both.v[1] += x; });
+    both = Lanes::allreduce(both, red[0]);
+    const float ms = both.v[0] * a.inv_cols;   // mean(x^2) = var + mu^2
+    mu = both.v[1] * a.inv_cols;
+    var = fmaxf(ms - mu * mu, 0.f);
+    rs = 1.0f / sqrtf(ms + a.eps);
+    store_sum();
+  } else {
+    // the mean first, then the sum of squares about it, as in norm_fwd_kernel
+    SumTuple<1> s = SumTuple<1>::identity();
+    each([&](float x) { s.v[0] += x; });
+    s = Lanes::allreduce(s, red[0]);
+    mu = s.v[0] * a.inv_cols;
+    store_sum();
+    s = SumTuple<1>::identity();
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) v[i][j] -= mu;
+    each([&](float x) { s.v[0] = fmaf(x, x, s.v[0]); });
+    s = Lanes::allreduce(s, red[1]);
+    var = s.v[0] * a.inv_cols;
+    rs = 1.0f / sqrtf(var + a.eps);
+  }
+  if (t == 0) {
+    const int64_t dense = dense_row_index(row, a.rn);
+    store_stat<T>(a.mean, dense, mu, a.stats_f32);
+    store_stat<T>(a.stat, dense, a.stat_kind == HK_STAT_VAR ? var : rs, a.stats_f32);
+  }
+
+  T* yr = static_cast<T*>(a.y) + row * a.y_pitch + outer_level_offset(a.y_lv);
+  const T* gp = static_cast<const T*>(a.gamma);
+  const T* bp = static_cast<const T*>(a.beta);
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int vec = i * tpr + t;
+    if (vec < a.nvec) {
+      const int c = vec_column<T, true>(vec, a.cols);
+      float g[VEC], b[VEC], f[VEC];
+      if (gp) VecIO<T>::unpack(ld16_any_keep<T>(gp + c), g);   // uniform
+      if (bp) VecIO<T>::unpack(ld16_any_keep<T>(bp + c), b);
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) {
+        const float n = rs * v[i][j];
+        f[j] = gp ? (bp ? fmaf(g[j], n, b[j]) : g[j] * n) : (bp ? n + b[j] : n);
+      }
+      store_row_vec<T, true, true>(yr, vec, f, a.cols);
+    }
+  }
+}
+
+// Fallback for rows shorter than a 16-byte vector or longer than the register file holds, and for double: one
+// workgroup per row, three strided passes (the re-reads hit L2).  CT is the arithmetic type.
 template <typename T, typename CT>
 __global__ __launch_bounds__(256)
 void norm_fwd_generic_kernel(NormFwdArgs a) {
@@ -429,6 +547,62 @@ static bool pick_row_shape(int nvec, int forced_threads, int max_nv, int wave_ro
   return false;
 }
 
+template <typename T, int LPR, bool HAS_RES, bool IS_RMS>
+static int launch_norm_fwd_any_nv(const NormFwdArgs& a, int nv, dim3 grid, dim3 block, hipStream_t s) {
+#define HK_ANY_CASE(N) case N: HK_LAUNCH((norm_fwd_any_kernel<T, N, LPR, HAS_RES, IS_RMS>), grid, block, 0, s, a); break;
+  profile_before(s);
+  if constexpr (LPR == kWave) {
+    switch (nv) { HK_ANY_CASE(1) HK_ANY_CASE(2) HK_ANY_CASE(3) default: HK_ANY_CASE(4) }
+  } else if constexpr (LPR == 0) {
+    switch (nv) { HK_ANY_CASE(2) HK_ANY_CASE(4) default: HK_ANY_CASE(8) }
+  } else {
+    HK_LAUNCH((norm_fwd_any_kernel<T, 1, LPR, HAS_RES, IS_RMS>), grid, block, 0, s, a);
+  }
+#undef HK_ANY_CASE
+  profile_after(s);
+  return launch_check("norm_fwd_any_kernel");
+}
+
+template <typename T, bool HAS_RES, bool IS_RMS>
+static int launch_norm_fwd_any(const NormFwdArgs& a, int lanes, int nv, hipStream_t s) {
+  if (lanes > kWave) {
+    const dim3 grid{unsigned(a.n0), unsigned(a.n1), unsigned(a.n2)};
+    return launch_norm_fwd_any_nv<T, 0, HAS_RES, IS_RMS>(a, nv, grid, dim3(unsigned(lanes)), s);
+  }
+  const int per_block = 256 / lanes;
+  const dim3 grid{unsigned((a.n0 + per_block - 1) / per_block), unsigned(a.n1), unsigned(a.n2)}, block{256};
+  switch (lanes) {
+    case 8: return launch_norm_fwd_any_nv<T, 8, HAS_RES, IS_RMS>(a, nv, grid, block, s);
+    case 16: return launch_norm_fwd_any_nv<T, 16, HAS_RES, IS_RMS>(a, nv, grid, block, s);
+    case 32: return launch_norm_fwd_any_nv<T, 32, HAS_RES, IS_RMS>(a, nv, grid, block, s);
+    default: return launch_norm_fwd_any_nv<T, kWave, HAS_RES, IS_RMS>(a, nv, grid, block, s);
+  }
+}
+
+// lanes per row (threads of a workgroup per row when above 64) and vectors per lane for norm_fwd_any_kernel: the fewest
+// lanes of a wavefront up to one vector each, then up to four vectors in a wavefront of their own, then a workgroup
+static bool pick_any_shape(int nvec, int* lanes, int* nv) {
+  if (nvec <= 64) {
+    *lanes = nvec <= 8 ? 8 : nvec <= 16 ? 16 : nvec <= 32 ? 32 : 64;
+    *nv = 1;
+    return true;
+  }
+  if (nvec <= 256) {
+    *lanes = 64;
+    *nv = (nvec + 63) / 64;
+    return true;
+  }
+  for (int n = 2; n <= 8; n <<= 1) {
+    const int t = ((nvec + n - 1) / n + 63) / 64 * 64;
+    if (t <= (n == 8 ? 1024 : 512)) {
+      *lanes = t;
+      *nv = n;
+      return true;
+    }
+  }
+  return false;
+}
+
 template <typename T>
 int norm_fwd_typed(NormFwdArgs a, hipStream_t s) {
   constexpr int VEC = VecIO<T>::N;
@@ -441,7 +615,7 @@ int norm_fwd_typed(NormFwdArgs a, hipStream_t s) {
                       (!a.residual || steps_ok(a.res_pitch, a.res_lv)) &&
                       (!a.x_out || steps_ok(a.xout_pitch, a.xout_lv));
   int threads = 0, nv = 0;
-  a.nvec = a.cols / VEC;
+  a.nvec = (a.cols + VEC - 1) / VEC;
   const bool has_res = a.residual != nullptr;
   // the row is held as at most 64 fp32 registers per thread (and at most 8 vectors when a residual row is in
   // flight next to it)
@@ -450,7 +624,10 @@ int norm_fwd_typed(NormFwdArgs a, hipStream_t s) {
   // large inputs take two rows per workgroup (below), which also changes the best width of some rows
   const int want_rows = tune_get(TUNE_NORM_FWD_ROWS);
   const bool many_rows = want_rows > 0 ? want_rows >= 2 : a.rows >= 16 * int64_t(device_cu_count());
-  if (vec_ok &&
+  // rows of up to 32 vectors share a wavefront (LayerNorm of 32768 rows of 256 bf16: 13.1 us with one to each, 10.7
+  // so); at 96 vectors norm_fwd_kernel is the faster one (20.1 against 25.5 us)
+  const bool short_rows = a.nvec <= 32 && tune_get(TUNE_NORM_FWD_THREADS) == 0;
+  if (vec_ok && !short_rows &&
       pick_row_shape(a.nvec, tune_get(TUNE_NORM_FWD_THREADS), max_nv, wave_nv, many_rows, &threads, &nv)) {
     if (threads == 64) {
       dim3 grid(unsigned((a.n0 + 3) / 4), unsigned(a.n1), unsigned(a.n2)), block(256);
@@ -467,6 +644,11 @@ int norm_fwd_typed(NormFwdArgs a, hipStream_t s) {
     dim3 grid{unsigned((a.n0 + rpb - 1) / rpb), unsigned(a.n1), unsigned(a.n2)}, block{unsigned(threads)};
     return has_res ? launch_norm_fwd_nv<T, false, true>(a, nv, rpb, grid, block, s)
                    : launch_norm_fwd_nv<T, false, false>(a, nv, rpb, grid, block, s);
+  }
+  int lanes = 0;
+  if (a.cols >= VEC && pick_any_shape(a.nvec, &lanes, &nv)) {
+    if (a.is_rms) return has_res ? launch_norm_fwd_any<T, true, true>(a, lanes, nv, s) : launch_norm_fwd_any<T, false, true>(a, lanes, nv, s);
+    return has_res ? launch_norm_fwd_any<T, true, false>(a, lanes, nv, s) : launch_norm_fwd_any<T, false, false>(a, lanes, nv, s);
   }
   HK_LAUNCH((norm_fwd_generic_kernel<T, float>), dim3(unsigned(a.n0), unsigned(a.n1), unsigned(a.n2)), dim3(256), 0,
             s, a);

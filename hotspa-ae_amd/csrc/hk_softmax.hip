@@ -27,24 +27,6 @@ struct SoftmaxArgs {
   int nvec;
 };
 
-// Which lanes hold a row.  LPR > 0: LPR neighbouring lanes of a wavefront (8, 16, 32 or all 64), 256 / LPR rows per
-// workgroup; LPR == 0: the whole workgroup.
-template <int LPR>
-struct RowLanes {
-  static __device__ __forceinline__ int count() { return LPR ? LPR : int(blockDim.x); }
-  static __device__ __forceinline__ int lane() { return LPR ? int(threadIdx.x) & (LPR - 1) : int(threadIdx.x); }
-  static __device__ __forceinline__ int64_t row() {
-    if constexpr (LPR == 0) return int64_t(blockIdx.x);
-    else if constexpr (LPR == kWave) return int64_t(blockIdx.x) * (256 / kWave) + wave_index();
-    else return int64_t(blockIdx.x) * (256 / LPR) + int(threadIdx.x) / LPR;
-  }
-  template <typename P>
-  static __device__ __forceinline__ P allreduce(P p, float* red) {
-    if constexpr (LPR == 0) return group_allreduce_tuple(p, red, 0, int(blockDim.x >> 6));
-    else return lanes_allreduce_tuple<LPR>(p);
-  }
-};
-
 template <typename T, int NV, int LPR, bool RAGGED>
 __global__ __launch_bounds__(LPR ? 256 : 1024)
 void softmax_fwd_kernel(SoftmaxArgs a) {

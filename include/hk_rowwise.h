@@ -186,7 +186,8 @@ HK_API int hk_layer_norm_fwd_strided_rows(int dtype, const void* x, const int64_
                                           hkStream_t stream);
 
 /* Bytes of scratch hk_layer_norm_bwd / hk_dropout_add_ln_bwd need for the
- * column-sum partials of dgamma / dbeta. */
+ * column-sum partials of dgamma / dbeta.  Rows that are no whole number of 16-byte vectors or do not start on 16-byte
+ * boundaries (and fp32 rows above 4096 columns) are also taken with less, or none, by slower kernels. */
 HK_API int hk_norm_bwd_workspace_bytes(int dtype, int64_t rows, int64_t cols, size_t* bytes);
 
 /* LayerNorm backward.  dy, x_or_y, dx: [rows, cols]; dgamma, dbeta: [cols] of

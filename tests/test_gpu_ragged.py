@@ -214,3 +214,100 @@ def test_cross_entropy_of_lowest_values(hk, cuda, dtype, cols):
     ok = [0, 1, 2, 3, 7]
     helpers.assert_close(loss[ok], want[ok].cpu().numpy(), dtype, "loss")
     helpers.assert_close(dx[ok], p[ok].cpu().numpy(), dtype, "dlogits")
+
+
+def _norm_lengths(dtype):
+    vec = 16 // ES[dtype]
+    out = {v * vec + k for v in (1, 2, 8, 16, 32, 64, 65, 128, 192, 256, 300, 512, 1024) for k in (0, 1, vec - 1)}
+    return sorted(out | {8192, 4097 * vec + 1})
+
+
+@pytest.mark.parametrize("dtype", ["fp32", "bf16", "fp16"])
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("is_rms", [True, False])
+def test_norm_any_length(hk, cuda, dtype, shift, is_rms):
+    """Forward with a residual (in place of it, and without), backward with an upstream gradient and a second output,
+    with the scratch that the library asks for and without any."""
+    import torch
+    eps = 1e-6
+    for cols in _norm_lengths(dtype):
+        rows = 37 if cols < 3000 else 5
+        pitch = cols + (0 if shift == 0 else 5)
+        x0, res, dz, dxin = (helpers.draw(s + cols, (rows, cols), dtype=dtype) for s in (100, 200, 300, 400))
+        gamma = helpers.draw(500 + cols, (cols,), "uniform", 0.5, 1.5, dtype)
+        beta = None if is_rms else helpers.draw(600 + cols, (cols,), "normal", 0.0, 0.1, dtype)
+        place = lambda a, fill=None: _placed(cuda, a, dtype, shift, pitch, fill)
+        vector = lambda a: None if a is None else _placed(cuda, a[None], dtype, shift, cols)[1][0]
+        tg, tb = vector(gamma), vector(beta)
+        tx0, tres = place(x0)[1], place(res)[1]
+        zb, tz = place(x0, 0.0)
+        xb, tx = place(x0, 0.0)
+        tmu, trs = torch.empty(rows, device=cuda), torch.empty(rows, device=cuda)
+        hk.dropout_add_ln_fwd(tx0, tres, tg, tb, tz, tx, tmu, trs, eps, is_rms)
+        torch.cuda.synchronize()
+        ez, ex, emu, ers = oracle.dropout_add_ln_fwd(x0, res, gamma, beta, eps, is_rms)
+        helpers.assert_close(tz.contiguous(), ez, dtype, "z %d" % cols)
+        helpers.assert_close(tx.contiguous(), ex, dtype, "x %d" % cols)
+        helpers.assert_close(trs, ers, "fp32", "rsigma %d" % cols)
+        helpers.assert_close(tmu, emu, "fp32", "mu %d" % cols, scale=1.0)
+        assert _guards_untouched(zb, tz) and _guards_untouched(xb, tx), cols
+        z2b, z2 = place(x0, 0.0)
+        hk.dropout_add_ln_fwd(tx0, tres, tg, tb, z2, tres, tmu, trs, eps, is_rms)     # the sum in place of the residual
+        torch.cuda.synchronize()
+        assert torch.equal(z2.contiguous(), tz.contiguous()) and torch.equal(tres.contiguous(), tx.contiguous()), cols
+        hk.dropout_add_ln_fwd(tx, None, tg, tb, z2, None, tmu, trs, eps, is_rms)      # no residual
+        torch.cuda.synchronize()
+        x = helpers.to_numpy(tx.contiguous())
+        ez, _, _, _ = oracle.dropout_add_ln_fwd(x, None, gamma, beta, eps, is_rms)
+        helpers.assert_close(z2.contiguous(), ez, dtype, "z %d" % cols)
+
+        mu32, rs32 = helpers.to_numpy(tmu), helpers.to_numpy(trs)
+        edx, edg, edb = oracle.dropout_add_ln_bwd(dz, dxin, x, mu32, rs32, gamma, is_rms)
+        tdz, tdxin = place(dz)[1], place(dxin)[1]
+        for workspace in (None, torch.empty(1, device=cuda)) if cols % (16 // ES[dtype]) or shift else (None,):
+            db, dx = place(x0, 0.0)
+            rb, dr = place(x0, 0.0)
+            (gb, dg), (bb, dbeta) = (_placed(cuda, gamma[None], dtype, shift, cols, 0.0) for _ in range(2))
+            hk.dropout_add_ln_bwd(tdz, tdxin, tx, tmu, trs, tg, dx, dr, dg[0], dbeta[0], is_rms, workspace=workspace)
+            torch.cuda.synchronize()
+            what = "%d %s" % (cols, workspace is None)
+            helpers.assert_close(dx.contiguous(), edx, dtype, "dx0 " + what)
+            assert torch.equal(dr.contiguous(), dx.contiguous())
+            helpers.assert_close(dg[0].contiguous(), edg, dtype, "dgamma " + what)
+            helpers.assert_close(dbeta[0].contiguous(), edb, dtype, "dbeta " + what)
+            for b, v in ((db, dx), (rb, dr), (gb, dg), (bb, dbeta)):
+                assert _guards_untouched(b, v), what
+        # in place of the upstream gradient
+        hk.dropout_add_ln_bwd(tdz, tdxin, tx, tmu, trs, tg, tdxin, None, None, None, is_rms)
+        torch.cuda.synchronize()
+        helpers.assert_close(tdxin.contiguous(), edx, dtype, "dx0 %d" % cols)
+
+
+@pytest.mark.parametrize("dtype", ["fp32", "bf16"])
+@pytest.mark.parametrize("cols", [9, 67, 1021, 3001, 8191])
+def test_layer_norm_bwd_any_length_modes(hk, cuda, dtype, cols):
+    """The plain backward from (mean, variance) in the data type, and the one that rebuilds x_hat from the output."""
+    import torch
+    rows, eps = 300, 1e-5
+    x, dy = (helpers.draw(s + cols, (rows, cols), dtype=dtype) for s in (700, 800))
+    gamma = helpers.draw(900 + cols, (cols,), "uniform", 0.5, 1.5, dtype)
+    beta = helpers.draw(950 + cols, (cols,), "normal", 0.0, 0.1, dtype)
+    y64, mean, var, rstd = oracle.layernorm_fwd(x, gamma, beta, eps)
+    tx, tg, tb, tdy = (helpers.to_torch(v, dtype, cuda) for v in (x, gamma, beta, dy))
+    tdx, tdg, tdb = torch.empty_like(tx), torch.empty_like(tg), torch.empty_like(tg)
+    # sums over 300 rows: their rounding error is that of the terms
+    many = float(np.sqrt(rows))
+    mean_s, var_s = oracle.round_to(mean, dtype), oracle.round_to(var, dtype)
+    edx, edg, edb = oracle.layernorm_bwd(dy, x, gamma, mean_s, 1.0 / np.sqrt(var_s.astype(np.float64) + eps), eps)
+    hk.layer_norm_bwd(tdy, tx, tg, tb, helpers.to_torch(mean_s, dtype, cuda), helpers.to_torch(var_s, dtype, cuda), tdx,
+                      tdg, tdb, eps, stat_kind=0)
+    torch.cuda.synchronize()
+    for got, want, what in ((tdx, edx, "dx"), (tdg, edg, "dgamma"), (tdb, edb, "dbeta")):
+        helpers.assert_close(got, want, dtype, what, scale=None if what == "dx" else many)
+    y, rstd32 = oracle.round_to(y64, dtype), rstd.astype(np.float32)
+    edx, edg, edb = oracle.layernorm_bwd_memeff(dy, y, gamma, beta, rstd32, eps)
+    hk.layer_norm_bwd(tdy, helpers.to_torch(y, dtype, cuda), tg, tb, None, helpers.to_torch(rstd32, "fp32", cuda), tdx,
+                      tdg, tdb, eps, memory_efficient=True)
+    torch.cuda.synchronize()
+    for got, want, what in ((tdx, edx, "dx"), (tdg, edg, "dgamma"), (tdb, edb, "dbeta")):
+        helpers.assert_close(got, want, dtype, what, scale=None if what == "dx" else many)
