@@ -3,12 +3,14 @@
 // cudnnBatchNormalizationBackward in CUDNN_BATCHNORM_SPATIAL mode (what the
 // reference calls): per channel over N, H, W.
 //
-// A channel's data is N runs of H*W contiguous elements, C*H*W apart.  Three
-// launches each way: (1) per-channel partial statistics from several workgroups
-// per channel, (2) a one-thread-per-channel merge that also writes the saved /
-// running statistics and the per-channel coefficients, (3) an element-wise pass,
-// one 16-byte vector per thread.  The input is read twice and the output written
-// once in the forward; the backward reads dy and x twice and writes dx once.
+// A channel's data is N runs of H*W contiguous elements, C*H*W apart.  Three forms:
+//  - a channel that fits a workgroup's registers (65536 16-bit or 32768 32-bit elements, half of that in the backward): one launch, one workgroup per
+//    channel reads it once, agrees on its statistics and writes the result;
+//  - longer ones: partial statistics from several workgroups per channel, then a pass whose workgroups merge their
+//    channel's partials themselves (the input is read twice, the second time from the memory-side cache where it fits);
+//  - fp64, planes shorter than a 16-byte vector and arrays past 2^31 elements: element by element, three launches.
+// The first two take planes of any length and alignment: the partial last vector of a run is read as the run's last whole
+// one, the elements it shares with the vector before it are left out of the sums.
 #include "hk_common.h"
 
 #include <algorithm>
@@ -19,60 +21,35 @@ namespace hk {
 template <typename T> struct BnCT { using type = float; };
 template <> struct BnCT<double> { using type = double; };
 
-// V elements starting at p as compute-type values (V == 1: any alignment)
-template <typename T, int V, typename CT>
-__device__ __forceinline__ void bn_load(const T* p, CT* f) {
-  if constexpr (V == 1) {
-    f[0] = CT(Cvt<T>::load(p));
-  } else {
-    float t[V];
-    VecIO<T>::unpack(ld16(p), t);
-#pragma unroll
-    for (int j = 0; j < V; ++j) f[j] = t[j];
-  }
-}
-template <typename T, int V, typename CT>
-__device__ __forceinline__ void bn_store(T* p, const CT* f) {
-  if constexpr (V == 1) {
-    Cvt<T>::store(p, f[0]);
-  } else {
-    float t[V];
-#pragma unroll
-    for (int j = 0; j < V; ++j) t[j] = f[j];
-    st16_stream(p, VecIO<T>::pack(t));
-  }
-}
-
 struct BnShape {
   int64_t N, C, HW;
-  int64_t hw_vec;         // HW / V
-  int64_t per_channel;    // N * hw_vec: loads of V elements per channel
+  int64_t per_channel;    // N * HW
   int splits;
 };
 
-// A thread's walk over the loads v0, v0 + stride, v0 + 2 stride, ... (< per_channel) of channel c: the element
-// offset of the current load, kept up by additions (one division per thread at the start, none per load).
+// A thread's walk over the elements v0, v0 + stride, v0 + 2 stride, ... (< per_channel) of channel c: the offset of the
+// current one, kept up by additions (one division per thread at the start, none per element).
 struct BnWalk {
-  int64_t off;        // element offset of the current load
-  int64_t in_plane;   // its load index inside its H*W plane
-  int64_t left;       // loads still to do, the current one included
-  int64_t step_off, step_in_plane, wrap_off, hw_vec;
-  __device__ __forceinline__ BnWalk(const BnShape& s, int64_t c, int64_t v0, int64_t stride, int V) {
-    const int64_t n = v0 / s.hw_vec;
-    in_plane = v0 - n * s.hw_vec;
-    off = (n * s.C + c) * s.HW + in_plane * V;
+  int64_t off;        // offset of the current element
+  int64_t in_plane;   // its index inside its H*W plane
+  int64_t left;       // elements still to do, the current one included
+  int64_t step_off, step_in_plane, wrap_off, hw;
+  __device__ __forceinline__ BnWalk(const BnShape& s, int64_t c, int64_t v0, int64_t stride) {
+    const int64_t n = v0 / s.HW;
+    in_plane = v0 - n * s.HW;
+    off = (n * s.C + c) * s.HW + in_plane;
     left = v0 < s.per_channel ? (s.per_channel - v0 + stride - 1) / stride : 0;
-    const int64_t q = stride / s.hw_vec;                 // whole planes per step
-    step_in_plane = stride - q * s.hw_vec;
-    step_off = q * s.C * s.HW + step_in_plane * V;
+    const int64_t q = stride / s.HW;                     // whole planes per step
+    step_in_plane = stride - q * s.HW;
+    step_off = q * s.C * s.HW + step_in_plane;
     wrap_off = (s.C - 1) * s.HW;                         // from the end of a plane to the same channel of the next image
-    hw_vec = s.hw_vec;
+    hw = s.HW;
   }
   __device__ __forceinline__ void next() {
     in_plane += step_in_plane;
     off += step_off;
-    const bool wrap = in_plane >= hw_vec;
-    in_plane -= wrap ? hw_vec : 0;
+    const bool wrap = in_plane >= hw;
+    in_plane -= wrap ? hw : 0;
     off += wrap ? wrap_off : 0;
     --left;
   }
@@ -93,32 +70,25 @@ __device__ __forceinline__ CT block_sum(CT v, CT* lds) {
 }
 
 // (count, mean, M2) of a slice of one channel -> part[(c * splits + split) * 3 ..]
-template <typename T, int V, typename CT>
+template <typename T, typename CT>
 __global__ __launch_bounds__(256)
 void bn_stats_kernel(const T* __restrict__ x, BnShape s, CT* __restrict__ part) {
   __shared__ CT lds[256];
   const int64_t c = blockIdx.x;
   const int split = blockIdx.y;
-  // per thread: sums of (x - K) and (x - K)^2 about a pivot K taken from the thread's first load, so that a
-  // large common offset of the channel never enters a sum; no division inside the loop
-  BnWalk w(s, c, int64_t(split) * 256 + threadIdx.x, int64_t(s.splits) * 256, V);
+  // per thread: sums of (x - K) and (x - K)^2 about a pivot K, the thread's first element, so that a large common
+  // offset of the channel never enters a sum; no division inside the loop
+  BnWalk w(s, c, int64_t(split) * 256 + threadIdx.x, int64_t(s.splits) * 256);
   CT cnt = 0, mean = 0, m2 = 0;
   if (w.left > 0) {
-    CT f[V];
-    bn_load<T, V, CT>(x + w.off, f);
-    CT K = 0;
-#pragma unroll
-    for (int j = 0; j < V; ++j) K += f[j];
-    K /= CT(V);
+    const CT K = CT(Cvt<T>::load(x + w.off));
     CT s1 = 0, s2 = 0;
-#pragma unroll
-    for (int j = 0; j < V; ++j) { const CT d = f[j] - K; s1 += d; s2 += d * d; }
-    cnt = CT(V);
+    cnt = 1;
     for (w.next(); w.left > 0; w.next()) {
-      bn_load<T, V, CT>(x + w.off, f);
-#pragma unroll
-      for (int j = 0; j < V; ++j) { const CT d = f[j] - K; s1 += d; s2 += d * d; }
-      cnt += CT(V);
+      const CT d = CT(Cvt<T>::load(x + w.off)) - K;
+      s1 += d;
+      s2 += d * d;
+      cnt += 1;
     }
     mean = K + s1 / cnt;
     m2 = s2 - s1 * (s1 / cnt);
@@ -133,6 +103,25 @@ void bn_stats_kernel(const T* __restrict__ x, BnShape s, CT* __restrict__ part) 
   if (threadIdx.x == 0) {
     CT* o = part + (c * s.splits + split) * 3;
     o[0] = bcnt; o[1] = bmean; o[2] = bm2;
+  }
+}
+
+// What the statistics of a channel leave behind; returns the inverse standard deviation.  (The running variance takes
+// the unbiased estimate, as cuDNN does.)
+template <typename PT, typename CT>
+__device__ __forceinline__ CT bn_invstd(CT var, double eps) {
+  if constexpr (std::is_same<CT, double>::value) return 1.0 / sqrt(var + eps);
+  else return 1.0f / sqrtf(var + float(eps));
+}
+template <typename PT, typename CT>
+__device__ __forceinline__ void bn_store_stats(int64_t c, CT cnt, CT mean, CT m2, CT invstd, double momentum,
+                                               PT* running_mean, PT* running_var, PT* save_mean, PT* save_invstd) {
+  if (save_mean) save_mean[c] = PT(mean);
+  if (save_invstd) save_invstd[c] = PT(invstd);
+  if (running_mean) running_mean[c] = PT((1.0 - momentum) * double(running_mean[c]) + momentum * double(mean));
+  if (running_var) {
+    const double unbiased = cnt > 1 ? double(m2) / (double(cnt) - 1.0) : double(cnt > 0 ? m2 / cnt : CT(0));
+    running_var[c] = PT((1.0 - momentum) * double(running_var[c]) + momentum * unbiased);
   }
 }
 
@@ -157,50 +146,19 @@ void bn_finalize_kernel(const CT* __restrict__ part, int64_t C, int splits, cons
     m2 += p[2] + delta * delta * (cnt * nb / n);
     cnt = n;
   }
-  const CT var = cnt > 0 ? m2 / cnt : CT(0);
-  CT invstd;
-  if constexpr (std::is_same<CT, double>::value) invstd = 1.0 / sqrt(var + eps);
-  else invstd = 1.0f / sqrtf(var + float(eps));
-  if (save_mean) save_mean[c] = PT(mean);
-  if (save_invstd) save_invstd[c] = PT(invstd);
-  if (running_mean) running_mean[c] = PT((1.0 - momentum) * double(running_mean[c]) + momentum * double(mean));
-  if (running_var) {
-    const double unbiased = cnt > 1 ? double(m2) / (double(cnt) - 1.0) : double(var);
-    running_var[c] = PT((1.0 - momentum) * double(running_var[c]) + momentum * unbiased);
-  }
+  const CT invstd = bn_invstd<PT, CT>(cnt > 0 ? m2 / cnt : CT(0), eps);
+  bn_store_stats<PT, CT>(c, cnt, mean, m2, invstd, momentum, running_mean, running_var, save_mean, save_invstd);
   coef[c] = CT(scale[c]) * invstd;
   coef[C + c] = mean;
   coef[2 * C + c] = CT(bias[c]);
 }
 
-// One load of V elements as it comes from memory; unpacked only after every load of the thread is issued.
-template <typename T, int V>
-struct BnRaw {
-  u32x4 vec;
-  T one;
-  __device__ __forceinline__ void load(const T* p) {
-    if constexpr (V == 1) one = *p;
-    else vec = ld16(p);
-  }
-  template <typename CT>
-  __device__ __forceinline__ void unpack(CT* f) const {
-    if constexpr (V == 1) {
-      f[0] = CT(Cvt<T>::load(&one));
-    } else {
-      float t[V];
-      VecIO<T>::unpack(vec, t);
-#pragma unroll
-      for (int j = 0; j < V; ++j) f[j] = t[j];
-    }
-  }
-};
-
-// Channel of load v of a dense [N, C, H*W] array, and whether the whole wavefront shares it (it does unless the
+// Channel of element v of a dense [N, C, H*W] array, and whether the whole wavefront shares it (it does unless the
 // wavefront crosses from one plane into the next): then the channel's coefficients are fetched once per
 // wavefront through the scalar unit instead of once per lane.
 template <typename IT>
-__device__ __forceinline__ IT bn_channel(IT v, IT hw_vec, IT C, bool& uniform) {
-  const IT plane = v / hw_vec;
+__device__ __forceinline__ IT bn_channel(IT v, IT hw, IT C, bool& uniform) {
+  const IT plane = v / hw;
   const IT plane0 = IT(__builtin_amdgcn_readfirstlane(uint32_t(plane)));
   uniform = __builtin_amdgcn_ballot_w64(plane != plane0) == 0;
   return uniform ? plane0 % C : plane % C;
@@ -209,15 +167,14 @@ __device__ __forceinline__ IT bn_channel(IT v, IT hw_vec, IT C, bool& uniform) {
 // y = (x - mean) * (scale * invstd) + bias; the mean is subtracted first: folding it into the constant term
 // would cancel badly for a channel whose mean is large against its spread.  IT: index type (32-bit when the
 // array allows it: the per-lane division is then a few instructions).
-template <typename T, int V, typename CT, typename IT>
+template <typename T, typename CT, typename IT>
 __global__ __launch_bounds__(256)
-void bn_apply_kernel(const T* x, T* y, const CT* __restrict__ coef, IT total_loads, IT hw_vec, IT C) {
+void bn_apply_kernel(const T* x, T* y, const CT* __restrict__ coef, IT total, IT hw, IT C) {
   const IT v = IT(blockIdx.x) * kStreamThreads + threadIdx.x;
-  if (v >= total_loads) return;
-  BnRaw<T, V> rx;
-  rx.load(x + size_t(v) * V);
+  if (v >= total) return;
+  const CT f = CT(Cvt<T>::load(x + size_t(v)));
   bool uniform;
-  const IT c = bn_channel<IT>(v, hw_vec, C, uniform);
+  const IT c = bn_channel<IT>(v, hw, C, uniform);
   CT a, mean, b;
   if (uniform) {
     const IT c0 = IT(__builtin_amdgcn_readfirstlane(uint32_t(c)));
@@ -225,15 +182,11 @@ void bn_apply_kernel(const T* x, T* y, const CT* __restrict__ coef, IT total_loa
   } else {
     a = coef[c]; mean = coef[size_t(C) + c]; b = coef[2 * size_t(C) + c];
   }
-  CT f[V];
-  rx.unpack(f);
-#pragma unroll
-  for (int j = 0; j < V; ++j) f[j] = (f[j] - mean) * a + b;
-  bn_store<T, V, CT>(y + size_t(v) * V, f);
+  Cvt<T>::store(y + size_t(v), (f - mean) * a + b);
 }
 
 // per-channel partial sums of dy and dy * (x - mean) * invstd -> part[(c * splits + split) * 2 ..]
-template <typename T, int V, typename PT, typename CT>
+template <typename T, typename PT, typename CT>
 __global__ __launch_bounds__(256)
 void bn_bwd_stats_kernel(const T* __restrict__ dy, const T* __restrict__ x, BnShape s,
                          const PT* __restrict__ save_mean, const PT* __restrict__ save_invstd,
@@ -243,12 +196,10 @@ void bn_bwd_stats_kernel(const T* __restrict__ dy, const T* __restrict__ x, BnSh
   const int split = blockIdx.y;
   const CT mean = CT(save_mean[c]), invstd = CT(save_invstd[c]);
   CT sdy = 0, sdyx = 0;
-  for (BnWalk w(s, c, int64_t(split) * 256 + threadIdx.x, int64_t(s.splits) * 256, V); w.left > 0; w.next()) {
-    CT g[V], f[V];
-    bn_load<T, V, CT>(dy + w.off, g);
-    bn_load<T, V, CT>(x + w.off, f);
-#pragma unroll
-    for (int j = 0; j < V; ++j) { sdy += g[j]; sdyx += g[j] * ((f[j] - mean) * invstd); }
+  for (BnWalk w(s, c, int64_t(split) * 256 + threadIdx.x, int64_t(s.splits) * 256); w.left > 0; w.next()) {
+    const CT g = CT(Cvt<T>::load(dy + w.off));
+    sdy += g;
+    sdyx += g * ((CT(Cvt<T>::load(x + w.off)) - mean) * invstd);
   }
   sdy = block_sum<CT>(sdy, lds);
   sdyx = block_sum<CT>(sdyx, lds);
@@ -282,17 +233,14 @@ void bn_bwd_finalize_kernel(const CT* __restrict__ part, int64_t C, int splits, 
   coef[3 * C + c] = mean;
 }
 
-template <typename T, int V, typename CT, typename IT>
+template <typename T, typename CT, typename IT>
 __global__ __launch_bounds__(256)
-void bn_bwd_apply_kernel(const T* dy, const T* x, T* dx, const CT* __restrict__ coef, IT total_loads, IT hw_vec,
-                         IT C) {
+void bn_bwd_apply_kernel(const T* dy, const T* x, T* dx, const CT* __restrict__ coef, IT total, IT hw, IT C) {
   const IT v = IT(blockIdx.x) * kStreamThreads + threadIdx.x;
-  if (v >= total_loads) return;
-  BnRaw<T, V> rg, rx;
-  rg.load(dy + size_t(v) * V);
-  rx.load(x + size_t(v) * V);
+  if (v >= total) return;
+  const CT g = CT(Cvt<T>::load(dy + size_t(v))), f = CT(Cvt<T>::load(x + size_t(v)));
   bool uniform;
-  const IT c = bn_channel<IT>(v, hw_vec, C, uniform);
+  const IT c = bn_channel<IT>(v, hw, C, uniform);
   CT k0, k1, k2, mean;
   if (uniform) {
     const IT c0 = IT(__builtin_amdgcn_readfirstlane(uint32_t(c)));
@@ -300,12 +248,361 @@ void bn_bwd_apply_kernel(const T* dy, const T* x, T* dx, const CT* __restrict__ 
   } else {
     k0 = coef[c]; k1 = coef[size_t(C) + c]; k2 = coef[2 * size_t(C) + c]; mean = coef[3 * size_t(C) + c];
   }
-  CT g[V], f[V];
-  rg.unpack(g);
-  rx.unpack(f);
+  Cvt<T>::store(dx + size_t(v), k0 * g + (k1 * (f - mean) + k2));
+}
+
+// ---------------------------------------------------------------------------
+// planes as 16-byte vectors
+// ---------------------------------------------------------------------------
+struct BnRuns {
+  int C, HW;
+  int run_vecs;        // vectors per run, the partial one included
+  int total;           // vectors per channel
+  int64_t image;       // C * HW
+};
+struct BnParams {
+  const float *scale, *bias;
+  float *running_mean, *running_var, *save_mean, *save_invstd;   // forward outputs (each may be null)
+  const float *mean, *invstd;                                    // backward inputs
+  float *dscale, *dbias;
+  double momentum, eps;
+  float count;
+};
+
+// A thread's walk over the vectors v0, v0 + stride, ... of a channel
+template <typename T>
+struct BnVecWalk {
+  static constexpr int VEC = VecIO<T>::N;
+  const BnRuns& r;
+  int index, v;          // vector in the channel, and in its run
+  int64_t plane;         // offset of the run from the channel's first
+  int stride, step_v;
+  int64_t step_plane;
+  __device__ __forceinline__ BnVecWalk(const BnRuns& runs, int v0, int by) : r(runs), index(v0), stride(by) {
+    const uint32_t n = uint32_t(v0) / uint32_t(r.run_vecs), q = uint32_t(by) / uint32_t(r.run_vecs);
+    v = v0 - int(n) * r.run_vecs;
+    plane = int64_t(n) * r.image;
+    step_v = by - int(q) * r.run_vecs;
+    step_plane = int64_t(q) * r.image;
+  }
+  __device__ __forceinline__ bool live() const { return index < r.total; }
+  // offset of the loaded vector (the channel's first one past the end), and how many of its elements belong to others
+  __device__ __forceinline__ int64_t off() const { return live() ? plane + vec_column<T, true>(v, r.HW) : 0; }
+  __device__ __forceinline__ int skip() const { return live() ? (v + 1) * VEC - r.HW : VEC; }
+  __device__ __forceinline__ void next() {
+    index += stride;
+    v += step_v;
+    plane += step_plane;
+    const bool wrap = v >= r.run_vecs;
+    v -= wrap ? r.run_vecs : 0;
+    plane += wrap ? r.image : 0;
+  }
+};
+// One workgroup per channel, NV vectors per thread in registers.  The mean first, as sums about the channel's first
+// element K (a large common offset never enters a sum), then the squares about it.  What the rounding of the mean
+// left out is kept as a second term, so that elements near the mean keep their digits.
+// Three launches and two reads of the input before (bf16, forward / backward): 64 x 256 x 196 24.4 / 23.6 us -> 11.2 /
+// 10.3, of which 10 are the call's own; 2 x 512 x 3969 27.9 / 27.0 -> 10.5 / 10.1.  Short odd planes are bound by cache
+// lines that neighbouring channels share (256 x 1024 x 49: 63 / 68 -> 34 / 44 us, 1.5 TB/s).
+template <typename T, int NV>
+__global__ __launch_bounds__(1024)
+void bn_fwd_channel_kernel(const T* x, T* y, BnRuns r, BnParams p) {
+  constexpr int VEC = VecIO<T>::N;
+  __shared__ float red[2][kMaxWaves * 2];
+  const int c = blockIdx.x, nwaves = int(blockDim.x >> 6);
+  const int64_t base = int64_t(c) * r.HW;
+  u32x4 raw[NV];
+  int off[NV], skip[NV];
+  BnVecWalk<T> w(r, int(threadIdx.x), int(blockDim.x));
 #pragma unroll
-  for (int j = 0; j < V; ++j) g[j] = k0 * g[j] + (k1 * (f[j] - mean) + k2);
-  bn_store<T, V, CT>(dx + size_t(v) * V, g);
+  for (int i = 0; i < NV; ++i, w.next()) {
+    off[i] = int(w.off());
+    skip[i] = w.skip();
+    raw[i] = ld16_any<T>(x + base + off[i]);
+  }
+  const float K = Cvt<T>::load(x + base);
+  SumTuple<1> s = SumTuple<1>::identity();
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    float f[VEC];
+    VecIO<T>::unpack(raw[i], f);
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) s.v[0] += j < skip[i] ? 0.f : f[j] - K;
+  }
+  const float near = K + group_allreduce_tuple(s, red[0], 0, nwaves).v[0] / p.count;
+  SumTuple<2> q = SumTuple<2>::identity();
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    float f[VEC];
+    VecIO<T>::unpack(raw[i], f);
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) {
+      const float d = j < skip[i] ? 0.f : f[j] - near;
+      q.v[0] += d;
+      q.v[1] = fmaf(d, d, q.v[1]);
+    }
+  }
+  q = group_allreduce_tuple(q, red[1], 0, nwaves);
+  const float rest = q.v[0] / p.count;   // mean = near + rest
+  const float m2 = fmaxf(q.v[1] - q.v[0] * rest, 0.f);
+  const float invstd = bn_invstd<float, float>(m2 / p.count, p.eps);
+  const float a = p.scale[c] * invstd, b = p.bias[c];
+  if (threadIdx.x == 0)
+    bn_store_stats<float, float>(c, p.count, near + rest, m2, invstd, p.momentum, p.running_mean, p.running_var,
+                                 p.save_mean, p.save_invstd);
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    if (skip[i] < VEC) {
+      float f[VEC];
+      VecIO<T>::unpack(raw[i], f);
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) f[j] = ((f[j] - near) - rest) * a + b;
+      st16_any(y + base + off[i], VecIO<T>::pack(f));   // shared elements: the same bits twice
+    }
+  }
+}
+
+// dx = scale * invstd * (dy - sum dy / m - xhat * sum(dy xhat) / m),  xhat = (x - mean) * invstd
+struct BnBwdCoef {
+  float k0, k1, k2, mean;
+  __device__ __forceinline__ BnBwdCoef(const BnParams& p, int c, float sdy, float sdyx, float mean_, float invstd) : mean(mean_) {
+    const float a = p.scale[c] * invstd;
+    k0 = a;
+    k1 = -a * invstd * sdyx / p.count;
+    k2 = -a * sdy / p.count;
+  }
+  __device__ __forceinline__ float operator()(float g, float x) const { return k0 * g + (k1 * (x - mean) + k2); }
+};
+
+template <typename T, int NV>
+__global__ __launch_bounds__(1024)
+void bn_bwd_channel_kernel(const T* dy, const T* x, T* dx, BnRuns r, BnParams p) {
+  constexpr int VEC = VecIO<T>::N;
+  __shared__ float red[kMaxWaves * 2];
+  const int c = blockIdx.x, nwaves = int(blockDim.x >> 6);
+  const int64_t base = int64_t(c) * r.HW;
+  u32x4 rg[NV], rx[NV];
+  int off[NV], skip[NV];
+  BnVecWalk<T> w(r, int(threadIdx.x), int(blockDim.x));
+#pragma unroll
+  for (int i = 0; i < NV; ++i, w.next()) {
+    off[i] = int(w.off());
+    skip[i] = w.skip();
+    rg[i] = ld16_any<T>(dy + base + off[i]);
+    rx[i] = ld16_any<T>(x + base + off[i]);
+  }
+  const float mean = p.mean[c], invstd = p.invstd[c];
+  SumTuple<2> s = SumTuple<2>::identity();
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    float g[VEC], f[VEC];
+    VecIO<T>::unpack(rg[i], g);
+    VecIO<T>::unpack(rx[i], f);
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) {
+      const float gj = j < skip[i] ? 0.f : g[j], xj = j < skip[i] ? mean : f[j];
+      s.v[0] += gj;
+      s.v[1] = fmaf(gj, (xj - mean) * invstd, s.v[1]);
+    }
+  }
+  s = group_allreduce_tuple(s, red, 0, nwaves);
+  if (threadIdx.x == 0) {
+    if (p.dscale) p.dscale[c] = s.v[1];
+    if (p.dbias) p.dbias[c] = s.v[0];
+  }
+  const BnBwdCoef k(p, c, s.v[0], s.v[1], mean, invstd);
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    if (skip[i] < VEC) {
+      float g[VEC], f[VEC];
+      VecIO<T>::unpack(rg[i], g);
+      VecIO<T>::unpack(rx[i], f);
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) g[j] = k(g[j], f[j]);
+      st16_any(dx + base + off[i], VecIO<T>::pack(g));
+    }
+  }
+}
+
+// Longer channels: kBnVecs vectors per thread in flight.  Bound by three (forward) and five (backward) streams at 6.3 to
+// 6.5 TB/s: 64 x 256 x 3136 bf16 55.7 / 83.2 -> 49.2 / 79.4 us, odd planes (32 x 100 x 3025 fp16, element by element
+// before) 63.9 / 57.2 -> 18.1 / 24.0 us.
+constexpr int kBnVecs = 4;
+
+// (count, mean, M2) of the slice blockIdx.y of channel blockIdx.x -> part[(c * splits + split) * 3 ..]
+template <typename T>
+__global__ __launch_bounds__(256)
+void bn_fwd_partial_kernel(const T* __restrict__ x, BnRuns r, int splits, float* __restrict__ part) {
+  constexpr int VEC = VecIO<T>::N, U = kBnVecs;
+  __shared__ float red[2][kMaxWaves * 2];
+  const int64_t c = blockIdx.x;
+  const T* base = x + c * r.HW;
+  BnVecWalk<T> w(r, int(blockIdx.y) * 256 + int(threadIdx.x), splits * 256);
+  // sums about a pivot K, the mean of the thread's first vector: a large common offset never enters a sum
+  float K = 0.f, s1 = 0.f, s2 = 0.f, cnt = 0.f;
+  while (w.live()) {
+    u32x4 raw[U];
+    int skip[U];
+#pragma unroll
+    for (int i = 0; i < U; ++i, w.next()) {
+      skip[i] = w.skip();
+      raw[i] = ld16_any_keep<T>(base + w.off());
+    }
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+      float f[VEC];
+      VecIO<T>::unpack(raw[i], f);
+      if (i == 0 && cnt == 0.f) {
+        float k = 0.f;
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) k += j < skip[0] ? 0.f : f[j];
+        K = k / float(VEC - max(skip[0], 0));
+      }
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) {
+        const float d = j < skip[i] ? 0.f : f[j] - K;
+        s1 += d;
+        s2 = fmaf(d, d, s2);
+      }
+      cnt += float(VEC - max(skip[i], 0));
+    }
+  }
+  const float mean = cnt > 0.f ? K + s1 / cnt : 0.f;
+  const float m2 = cnt > 0.f ? fmaxf(s2 - s1 * (s1 / cnt), 0.f) : 0.f;
+  // total count and mean first, then M2 about that mean
+  const SumTuple<2> t = group_allreduce_tuple(SumTuple<2>{{cnt, mean * cnt}}, red[0], 0, 4);
+  const float bmean = t.v[0] > 0.f ? t.v[1] / t.v[0] : 0.f, d = mean - bmean;
+  const SumTuple<1> q = group_allreduce_tuple(SumTuple<1>{{fmaf(d * d, cnt, m2)}}, red[1], 0, 4);
+  if (threadIdx.x == 0) {
+    float* o = part + (c * splits + blockIdx.y) * 3;
+    o[0] = t.v[0]; o[1] = bmean; o[2] = q.v[0];
+  }
+}
+
+// Workgroup (chunk, channel) = divmod(blockIdx.x, C): kBnVecs vectors per thread, loaded before the channel's partials
+// are merged; every wavefront merges them for itself.  The first chunk's workgroup writes the statistics.
+template <typename T>
+__global__ __launch_bounds__(256)
+void bn_fwd_merge_apply_kernel(const T* x, T* y, BnRuns r, BnParams p, int splits, const float* __restrict__ part) {
+  constexpr int VEC = VecIO<T>::N, U = kBnVecs;
+  const int chunk = int(blockIdx.x / uint32_t(r.C)), c = int(blockIdx.x - uint32_t(chunk) * uint32_t(r.C));
+  const int64_t base = int64_t(c) * r.HW;
+  u32x4 raw[U];
+  int v[U];
+  int64_t plane[U];
+  BnVecWalk<T> w(r, chunk * (256 * U) + int(threadIdx.x), 256);
+#pragma unroll
+  for (int i = 0; i < U; ++i, w.next()) {
+    raw[i] = ld16_any<T>(x + base + w.off());
+    v[i] = w.live() ? w.v : r.run_vecs;      // a vector past the run's end stores nothing
+    plane[i] = w.plane;
+  }
+  const float* mine = part + int64_t(c) * splits * 3;
+  const float near = mine[1];              // about the first slice's mean: mean = near + rest, as in bn_fwd_channel_kernel
+  float d1 = 0.f;
+  for (int k = int(threadIdx.x & 63); k < splits; k += kWave) d1 = fmaf(mine[k * 3], mine[k * 3 + 1] - near, d1);
+  const float rest = wave_allreduce_tuple(SumTuple<1>{{d1}}).v[0] / p.count;
+  SumTuple<1> q = SumTuple<1>::identity();
+  for (int k = int(threadIdx.x & 63); k < splits; k += kWave) {
+    const float d = (mine[k * 3 + 1] - near) - rest;
+    q.v[0] += fmaf(d * d, mine[k * 3], mine[k * 3 + 2]);
+  }
+  const float m2 = wave_allreduce_tuple(q).v[0];
+  const float invstd = bn_invstd<float, float>(m2 / p.count, p.eps);
+  if (chunk == 0 && threadIdx.x == 0)
+    bn_store_stats<float, float>(c, p.count, near + rest, m2, invstd, p.momentum, p.running_mean, p.running_var,
+                                 p.save_mean, p.save_invstd);
+  const float a = p.scale[c] * invstd, b = p.bias[c];
+#pragma unroll
+  for (int i = 0; i < U; ++i) {
+    float f[VEC];
+    VecIO<T>::unpack(raw[i], f);
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) f[j] = ((f[j] - near) - rest) * a + b;
+    // in place, a shared element may have been replaced before it was read here: only own ones go out
+    if (v[i] < r.run_vecs) store_row_vec<T, true, false>(y + base + plane[i], v[i], f, r.HW);
+  }
+}
+
+// sums of dy and dy * xhat of a slice -> part[(c * splits + split) * 2 ..]
+template <typename T>
+__global__ __launch_bounds__(256)
+void bn_bwd_partial_kernel(const T* __restrict__ dy, const T* __restrict__ x, BnRuns r, BnParams p, int splits,
+                           float* __restrict__ part) {
+  constexpr int VEC = VecIO<T>::N, U = kBnVecs / 2;
+  __shared__ float red[kMaxWaves * 2];
+  const int64_t c = blockIdx.x;
+  const int64_t base = c * r.HW;
+  const float mean = p.mean[c], invstd = p.invstd[c];
+  SumTuple<2> s = SumTuple<2>::identity();
+  BnVecWalk<T> w(r, int(blockIdx.y) * 256 + int(threadIdx.x), splits * 256);
+  while (w.live()) {
+    u32x4 rg[U], rx[U];
+    int skip[U];
+#pragma unroll
+    for (int i = 0; i < U; ++i, w.next()) {
+      const int64_t off = base + w.off();
+      skip[i] = w.skip();
+      rg[i] = ld16_any_keep<T>(dy + off);
+      rx[i] = ld16_any_keep<T>(x + off);
+    }
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+      float g[VEC], f[VEC];
+      VecIO<T>::unpack(rg[i], g);
+      VecIO<T>::unpack(rx[i], f);
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) {
+        const float gj = j < skip[i] ? 0.f : g[j], xj = j < skip[i] ? mean : f[j];
+        s.v[0] += gj;
+        s.v[1] = fmaf(gj, (xj - mean) * invstd, s.v[1]);
+      }
+    }
+  }
+  s = group_allreduce_tuple(s, red, 0, 4);
+  if (threadIdx.x == 0) {
+    float* o = part + (c * splits + blockIdx.y) * 2;
+    o[0] = s.v[0]; o[1] = s.v[1];
+  }
+}
+
+template <typename T>
+__global__ __launch_bounds__(256)
+void bn_bwd_merge_apply_kernel(const T* dy, const T* x, T* dx, BnRuns r, BnParams p, int splits,
+                               const float* __restrict__ part) {
+  constexpr int VEC = VecIO<T>::N, U = kBnVecs / 2;
+  const int chunk = int(blockIdx.x / uint32_t(r.C)), c = int(blockIdx.x - uint32_t(chunk) * uint32_t(r.C));
+  const int64_t base = int64_t(c) * r.HW;
+  u32x4 rg[U], rx[U];
+  int v[U];
+  int64_t plane[U];
+  BnVecWalk<T> w(r, chunk * (256 * U) + int(threadIdx.x), 256);
+#pragma unroll
+  for (int i = 0; i < U; ++i, w.next()) {
+    const int64_t off = base + w.off();
+    rg[i] = ld16_any<T>(dy + off);
+    rx[i] = ld16_any<T>(x + off);
+    v[i] = w.live() ? w.v : r.run_vecs;
+    plane[i] = w.plane;
+  }
+  const float* mine = part + int64_t(c) * splits * 2;
+  SumTuple<2> s = SumTuple<2>::identity();
+  for (int k = int(threadIdx.x & 63); k < splits; k += kWave) { s.v[0] += mine[k * 2]; s.v[1] += mine[k * 2 + 1]; }
+  s = wave_allreduce_tuple(s);
+  if (chunk == 0 && threadIdx.x == 0) {
+    if (p.dscale) p.dscale[c] = s.v[1];
+    if (p.dbias) p.dbias[c] = s.v[0];
+  }
+  const BnBwdCoef k(p, c, s.v[0], s.v[1], p.mean[c], p.invstd[c]);
+#pragma unroll
+  for (int i = 0; i < U; ++i) {
+    float g[VEC], f[VEC];
+    VecIO<T>::unpack(rg[i], g);
+    VecIO<T>::unpack(rx[i], f);
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) g[j] = k(g[j], f[j]);
+    if (v[i] < r.run_vecs) store_row_vec<T, true, false>(dx + base + plane[i], v[i], g, r.HW);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -319,20 +616,52 @@ static int bn_splits(int64_t C, int64_t per_channel) {
   return int(std::max<int64_t>(1, std::min<int64_t>(std::min(want, most), 1024)));
 }
 
-template <int V>
 static BnShape bn_shape(int64_t N, int64_t C, int64_t HW) {
   BnShape s{};
   s.N = N; s.C = C; s.HW = HW;
-  s.hw_vec = HW / V;
-  s.per_channel = N * s.hw_vec;
+  s.per_channel = N * HW;
   s.splits = bn_splits(C, s.per_channel);
   return s;
 }
 
 static size_t bn_ws_bytes(int64_t N, int64_t C, int64_t HW, size_t ct_size) {
-  // partials for the scalar decomposition (the larger one) + four coefficient rows
-  const BnShape s = bn_shape<1>(N, C, HW);
+  // partials for the element-wise decomposition (the largest one) + four coefficient rows
+  const BnShape s = bn_shape(N, C, HW);
   return (size_t(C) * size_t(s.splits) * 3 + size_t(C) * 4) * ct_size;
+}
+
+// How the vector kernels take an [N, C, HW] array; form 0: they don't
+struct BnPlan {
+  int form;            // 1: a workgroup per channel; 2: partials and merge
+  BnRuns runs;
+  int threads, nv;     // form 1
+  int splits;          // form 2
+};
+template <typename T>
+static BnPlan bn_plan(int64_t N, int64_t C, int64_t HW, int max_splits, int max_nv) {
+  constexpr int VEC = VecIO<T>::N;
+  BnPlan b{};
+  if (HW < VEC || N * C * HW > 0x7fffffffLL) return b;
+  b.runs.C = int(C); b.runs.HW = int(HW); b.runs.image = C * HW;
+  b.runs.run_vecs = int((HW + VEC - 1) / VEC);
+  const int64_t total = N * b.runs.run_vecs;
+  if (total > 0x3fffffff) return b;
+  b.runs.total = int(total);
+  for (int nv = 1; nv <= max_nv; nv <<= 1) {
+    // one vector a thread while there are fewer channels than two workgroups per compute unit, else two at least
+    if (total > int64_t(nv) * 1024 || (nv == 1 && total > 64 && C > 2 * device_cu_count())) continue;
+    b.form = 1;
+    b.nv = nv;
+    b.threads = int(((total + nv - 1) / nv + 63) / 64 * 64);
+    return b;
+  }
+  b.form = 2;
+  const int64_t want = (int64_t(device_cu_count()) * 8 + C - 1) / C, most = total / (256 * kBnVecs);
+  b.splits = int(std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(want, most), std::min(max_splits, 256))));
+  return b;
+}
+static inline unsigned bn_chunks(const BnRuns& r, int per_thread) {
+  return unsigned((int64_t(r.total) + 256 * per_thread - 1) / (256 * per_thread)) * unsigned(r.C);
 }
 
 template <typename T, typename PT>
@@ -343,41 +672,56 @@ static int bn_fwd_typed(const void* x, const void* scale, const void* bias, void
   CT* part = static_cast<CT*>(ws);
   const T* xp = static_cast<const T*>(x);
   T* yp = static_cast<T*>(y);
-  bool vec = false;
+  const BnShape s = bn_shape(N, C, HW);
   if constexpr (!std::is_same<T, double>::value) {
-    vec = HW % VecIO<T>::N == 0 && aligned16(x) && aligned16(y);
-  }
-  auto run = [&](auto vtag) -> int {
-    constexpr int V = decltype(vtag)::value;
-    const BnShape s = bn_shape<V>(N, C, HW);
-    CT* coef = part + size_t(C) * size_t(s.splits) * 3;
-    HK_REQUIRE(C <= 0x7fffffffLL && (N * C * s.hw_vec + kStreamThreads - 1) / kStreamThreads <= 0x7fffffffLL, HK_ERR_INVALID,
-               "hk_batch_norm_fwd: array too large");
-    HK_LAUNCH((bn_stats_kernel<T, V, CT>), dim3(unsigned(C), unsigned(s.splits)), dim3(256), 0, st, xp, s, part);
-    int rc = launch_check("bn_stats_kernel");
-    if (rc != HK_OK) return rc;
-    HK_LAUNCH((bn_finalize_kernel<PT, CT>), dim3(unsigned((C + 255) / 256)), dim3(256), 0, st, part, C,
-                       s.splits, static_cast<const PT*>(scale), static_cast<const PT*>(bias), momentum, eps,
-                       static_cast<PT*>(running_mean), static_cast<PT*>(running_var), static_cast<PT*>(save_mean),
-                       static_cast<PT*>(save_invstd), coef);
-    rc = launch_check("bn_finalize_kernel");
-    if (rc != HK_OK) return rc;
-    const int64_t loads = N * C * s.hw_vec;
-    profile_before(st);
-    if (loads < 0x7fffffffLL) {
-      HK_LAUNCH((bn_apply_kernel<T, V, CT, uint32_t>), dim3(unsigned((loads + kStreamThreads - 1) / kStreamThreads)), dim3(kStreamThreads), 0, st,
-                         xp, yp, coef, uint32_t(loads), uint32_t(s.hw_vec), uint32_t(C));
-    } else {
-      HK_LAUNCH((bn_apply_kernel<T, V, CT, int64_t>), dim3(unsigned((loads + kStreamThreads - 1) / kStreamThreads)), dim3(kStreamThreads), 0, st,
-                         xp, yp, coef, loads, s.hw_vec, C);
+    const BnPlan b = bn_plan<T>(N, C, HW, s.splits, 8);
+    BnParams p{};
+    p.scale = static_cast<const float*>(scale); p.bias = static_cast<const float*>(bias);
+    p.running_mean = static_cast<float*>(running_mean); p.running_var = static_cast<float*>(running_var);
+    p.save_mean = static_cast<float*>(save_mean); p.save_invstd = static_cast<float*>(save_invstd);
+    p.momentum = momentum; p.eps = eps; p.count = float(N * HW);
+    if (b.form == 1) {
+      const dim3 grid{unsigned(C)}, block{unsigned(b.threads)};
+      profile_before(st);
+      switch (b.nv) {
+        case 1: HK_LAUNCH((bn_fwd_channel_kernel<T, 1>), grid, block, 0, st, xp, yp, b.runs, p); break;
+        case 2: HK_LAUNCH((bn_fwd_channel_kernel<T, 2>), grid, block, 0, st, xp, yp, b.runs, p); break;
+        case 4: HK_LAUNCH((bn_fwd_channel_kernel<T, 4>), grid, block, 0, st, xp, yp, b.runs, p); break;
+        default: HK_LAUNCH((bn_fwd_channel_kernel<T, 8>), grid, block, 0, st, xp, yp, b.runs, p);
+      }
+      profile_after(st);
+      return launch_check("bn_fwd_channel_kernel");
     }
-    profile_after(st);
-    return launch_check("bn_apply_kernel");
-  };
-  if constexpr (!std::is_same<T, double>::value) {
-    if (vec) return run(std::integral_constant<int, VecIO<T>::N>{});
+    if (b.form == 2) {
+      HK_LAUNCH((bn_fwd_partial_kernel<T>), dim3(unsigned(C), unsigned(b.splits)), dim3(256), 0, st, xp, b.runs, b.splits, part);
+      const int rc = launch_check("bn_fwd_partial_kernel");
+      if (rc != HK_OK) return rc;
+      profile_before(st);
+      HK_LAUNCH((bn_fwd_merge_apply_kernel<T>), dim3(bn_chunks(b.runs, kBnVecs)), dim3(256), 0, st, xp, yp, b.runs, p, b.splits, part);
+      profile_after(st);
+      return launch_check("bn_fwd_merge_apply_kernel");
+    }
   }
-  return run(std::integral_constant<int, 1>{});
+  CT* coef = part + size_t(C) * size_t(s.splits) * 3;
+  const int64_t total = N * C * HW;
+  HK_REQUIRE(C <= 0x7fffffffLL && (total + kStreamThreads - 1) / kStreamThreads <= 0x7fffffffLL, HK_ERR_INVALID,
+             "hk_batch_norm_fwd: array too large");
+  HK_LAUNCH((bn_stats_kernel<T, CT>), dim3(unsigned(C), unsigned(s.splits)), dim3(256), 0, st, xp, s, part);
+  int rc = launch_check("bn_stats_kernel");
+  if (rc != HK_OK) return rc;
+  HK_LAUNCH((bn_finalize_kernel<PT, CT>), dim3(unsigned((C + 255) / 256)), dim3(256), 0, st, part, C, s.splits,
+            static_cast<const PT*>(scale), static_cast<const PT*>(bias), momentum, eps, static_cast<PT*>(running_mean),
+            static_cast<PT*>(running_var), static_cast<PT*>(save_mean), static_cast<PT*>(save_invstd), coef);
+  rc = launch_check("bn_finalize_kernel");
+  if (rc != HK_OK) return rc;
+  const dim3 grid{unsigned((total + kStreamThreads - 1) / kStreamThreads)}, block{kStreamThreads};
+  profile_before(st);
+  if (total < 0x7fffffffLL)
+    HK_LAUNCH((bn_apply_kernel<T, CT, uint32_t>), grid, block, 0, st, xp, yp, coef, uint32_t(total), uint32_t(HW), uint32_t(C));
+  else
+    HK_LAUNCH((bn_apply_kernel<T, CT, int64_t>), grid, block, 0, st, xp, yp, coef, total, HW, C);
+  profile_after(st);
+  return launch_check("bn_apply_kernel");
 }
 
 template <typename T, typename PT>
@@ -386,44 +730,58 @@ static int bn_bwd_typed(const void* dy, const void* x, const void* scale, void* 
                         hipStream_t st) {
   using CT = typename BnCT<T>::type;
   CT* part = static_cast<CT*>(ws);
-  bool vec = false;
+  const T *gp = static_cast<const T*>(dy), *xp = static_cast<const T*>(x);
+  T* op = static_cast<T*>(dx);
+  const BnShape s = bn_shape(N, C, HW);
   if constexpr (!std::is_same<T, double>::value) {
-    vec = HW % VecIO<T>::N == 0 && aligned16(x) && aligned16(dy) && aligned16(dx);
-  }
-  auto run = [&](auto vtag) -> int {
-    constexpr int V = decltype(vtag)::value;
-    const BnShape s = bn_shape<V>(N, C, HW);
-    CT* coef = part + size_t(C) * size_t(s.splits) * 3;
-    HK_REQUIRE(C <= 0x7fffffffLL && (N * C * s.hw_vec + kStreamThreads - 1) / kStreamThreads <= 0x7fffffffLL, HK_ERR_INVALID,
-               "hk_batch_norm_bwd: array too large");
-    HK_LAUNCH((bn_bwd_stats_kernel<T, V, PT, CT>), dim3(unsigned(C), unsigned(s.splits)), dim3(256), 0, st,
-                       static_cast<const T*>(dy), static_cast<const T*>(x), s, static_cast<const PT*>(save_mean),
-                       static_cast<const PT*>(save_invstd), part);
-    int rc = launch_check("bn_bwd_stats_kernel");
-    if (rc != HK_OK) return rc;
-    HK_LAUNCH((bn_bwd_finalize_kernel<PT, CT>), dim3(unsigned((C + 255) / 256)), dim3(256), 0, st, part, C,
-                       s.splits, CT(N * HW), static_cast<const PT*>(scale), static_cast<const PT*>(save_mean),
-                       static_cast<const PT*>(save_invstd), static_cast<PT*>(dscale), static_cast<PT*>(dbias), coef);
-    rc = launch_check("bn_bwd_finalize_kernel");
-    if (rc != HK_OK) return rc;
-    const int64_t loads = N * C * s.hw_vec;
-    profile_before(st);
-    if (loads < 0x7fffffffLL) {
-      HK_LAUNCH((bn_bwd_apply_kernel<T, V, CT, uint32_t>), dim3(unsigned((loads + kStreamThreads - 1) / kStreamThreads)), dim3(kStreamThreads), 0,
-                         st, static_cast<const T*>(dy), static_cast<const T*>(x), static_cast<T*>(dx), coef,
-                         uint32_t(loads), uint32_t(s.hw_vec), uint32_t(C));
-    } else {
-      HK_LAUNCH((bn_bwd_apply_kernel<T, V, CT, int64_t>), dim3(unsigned((loads + kStreamThreads - 1) / kStreamThreads)), dim3(kStreamThreads), 0,
-                         st, static_cast<const T*>(dy), static_cast<const T*>(x), static_cast<T*>(dx), coef, loads,
-                         s.hw_vec, C);
+    const BnPlan b = bn_plan<T>(N, C, HW, s.splits, 4);
+    BnParams p{};
+    p.scale = static_cast<const float*>(scale);
+    p.mean = static_cast<const float*>(save_mean); p.invstd = static_cast<const float*>(save_invstd);
+    p.dscale = static_cast<float*>(dscale); p.dbias = static_cast<float*>(dbias);
+    p.count = float(N * HW);
+    if (b.form == 1) {
+      const dim3 grid{unsigned(C)}, block{unsigned(b.threads)};
+      profile_before(st);
+      switch (b.nv) {
+        case 1: HK_LAUNCH((bn_bwd_channel_kernel<T, 1>), grid, block, 0, st, gp, xp, op, b.runs, p); break;
+        case 2: HK_LAUNCH((bn_bwd_channel_kernel<T, 2>), grid, block, 0, st, gp, xp, op, b.runs, p); break;
+        default: HK_LAUNCH((bn_bwd_channel_kernel<T, 4>), grid, block, 0, st, gp, xp, op, b.runs, p);
+      }
+      profile_after(st);
+      return launch_check("bn_bwd_channel_kernel");
     }
-    profile_after(st);
-    return launch_check("bn_bwd_apply_kernel");
-  };
-  if constexpr (!std::is_same<T, double>::value) {
-    if (vec) return run(std::integral_constant<int, VecIO<T>::N>{});
+    if (b.form == 2) {
+      HK_LAUNCH((bn_bwd_partial_kernel<T>), dim3(unsigned(C), unsigned(b.splits)), dim3(256), 0, st, gp, xp, b.runs, p, b.splits, part);
+      const int rc = launch_check("bn_bwd_partial_kernel");
+      if (rc != HK_OK) return rc;
+      profile_before(st);
+      HK_LAUNCH((bn_bwd_merge_apply_kernel<T>), dim3(bn_chunks(b.runs, kBnVecs / 2)), dim3(256), 0, st, gp, xp, op, b.runs, p, b.splits, part);
+      profile_after(st);
+      return launch_check("bn_bwd_merge_apply_kernel");
+    }
   }
-  return run(std::integral_constant<int, 1>{});
+  CT* coef = part + size_t(C) * size_t(s.splits) * 3;
+  const int64_t total = N * C * HW;
+  HK_REQUIRE(C <= 0x7fffffffLL && (total + kStreamThreads - 1) / kStreamThreads <= 0x7fffffffLL, HK_ERR_INVALID,
+             "hk_batch_norm_bwd: array too large");
+  HK_LAUNCH((bn_bwd_stats_kernel<T, PT, CT>), dim3(unsigned(C), unsigned(s.splits)), dim3(256), 0, st, gp, xp, s,
+            static_cast<const PT*>(save_mean), static_cast<const PT*>(save_invstd), part);
+  int rc = launch_check("bn_bwd_stats_kernel");
+  if (rc != HK_OK) return rc;
+  HK_LAUNCH((bn_bwd_finalize_kernel<PT, CT>), dim3(unsigned((C + 255) / 256)), dim3(256), 0, st, part, C, s.splits,
+            CT(N * HW), static_cast<const PT*>(scale), static_cast<const PT*>(save_mean),
+            static_cast<const PT*>(save_invstd), static_cast<PT*>(dscale), static_cast<PT*>(dbias), coef);
+  rc = launch_check("bn_bwd_finalize_kernel");
+  if (rc != HK_OK) return rc;
+  const dim3 grid{unsigned((total + kStreamThreads - 1) / kStreamThreads)}, block{kStreamThreads};
+  profile_before(st);
+  if (total < 0x7fffffffLL)
+    HK_LAUNCH((bn_bwd_apply_kernel<T, CT, uint32_t>), grid, block, 0, st, gp, xp, op, coef, uint32_t(total), uint32_t(HW), uint32_t(C));
+  else
+    HK_LAUNCH((bn_bwd_apply_kernel<T, CT, int64_t>), grid, block, 0, st, gp, xp, op, coef, total, HW, C);
+  profile_after(st);
+  return launch_check("bn_bwd_apply_kernel");
 }
 
 static int bn_check(const char* who, int dtype, int64_t N, int64_t C, int64_t HW, const void* ws, size_t ws_bytes,

@@ -115,3 +115,72 @@ def test_batch_norm_empty_shapes(hk, cuda, shape):
     hk.batch_norm_bwd(y, x, scale, dx, ds, db, sm, si)
     torch.cuda.synchronize()
     assert bool((rm == 3.0).all()) and bool((rv == 5.0).all())
+
+
+# planes around one vector, odd planes, channels on both sides of what a workgroup's registers hold (65536 16-bit, 32768
+# 32-bit elements; half of that backward), many and few of them, several splits per channel
+RUNS = [(3, 5, 8), (3, 5, 9), (7, 3, 15), (16, 1100, 17), (64, 4, 196), (1, 2, 32768), (1, 2, 65537), (5, 3, 13121),
+        (64, 8, 3136), (3, 700, 3969), (300, 2, 1021), (2, 1, 300007), (40, 1500, 49), (2048, 3, 20)]
+
+
+@pytest.mark.parametrize("dtype", ["fp32", "bf16", "fp16"])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_planes_of_any_length(hk, cuda, dtype, shift):
+    """Against the formulas in fp64 on the GPU; base addresses on and off the 16-byte grid; in place as well."""
+    import torch
+    dt = {"fp32": torch.float32, "bf16": torch.bfloat16, "fp16": torch.float16}[dtype]
+
+    def placed(a):
+        buf = torch.full((a.numel() + 32,), 7.0, dtype=dt, device=cuda)
+        view = buf[8 + shift:8 + shift + a.numel()].view(a.shape)
+        view.copy_(a)
+        return buf, view
+
+    def clean(buf, view):
+        return bool((buf[:8 + shift] == 7.0).all()) and bool((buf[8 + shift + view.numel():] == 7.0).all())
+
+    gen = torch.Generator(device="cuda").manual_seed(17)
+    for N, C, HW in RUNS:
+        shape, m = (N, C, HW), N * HW
+        rand = lambda *s: torch.randn(*s, generator=gen, device=cuda)
+        _, x = placed((rand(N, C, HW) * 2 + 3).to(dt))
+        _, dy = placed(rand(N, C, HW).to(dt))
+        scale, bias = rand(C).abs() + 0.5, rand(C)
+        rm, rv = rand(C), rand(C).abs() + 0.5
+        rm0, rv0 = rm.double(), rv.double()
+        yb, y = placed(torch.zeros(shape, device=cuda))
+        sm, si = torch.empty(C, device=cuda), torch.empty(C, device=cuda)
+        hk.batch_norm_fwd(x, scale, bias, y, 0.1, 1e-5, rm, rv, sm, si)
+        torch.cuda.synchronize()
+        xd, dyd = x.double(), dy.double()
+        mean = xd.mean((0, 2)); var = ((xd - mean[:, None]) ** 2).mean((0, 2))
+        inv = (var + 1e-5).rsqrt()
+        ey = (xd - mean[:, None]) * (scale.double() * inv)[:, None] + bias.double()[:, None]
+        num = lambda t: t.cpu().numpy()
+        helpers.assert_close(y.contiguous(), num(ey), dtype, "y %s" % (shape,))
+        helpers.assert_close(sm, num(mean), "fp32", "save_mean")
+        helpers.assert_close(si, num(inv), "fp32", "save_invstd")
+        helpers.assert_close(rm, num(0.9 * rm0 + 0.1 * mean), "fp32", "running_mean", scale=1.0)
+        helpers.assert_close(rv, num(0.9 * rv0 + 0.1 * var * m / max(m - 1, 1)), "fp32", "running_var")
+        assert clean(yb, y), shape
+        xb, x2 = placed(x)
+        hk.batch_norm_fwd(x2, scale, bias, x2, 0.1, 1e-5, None, None, None, None)
+        torch.cuda.synchronize()
+        assert torch.equal(x2, y) and clean(xb, x2), shape
+        smd, sid = sm.double()[:, None], si.double()[:, None]
+        xhat = (xd - smd) * sid
+        eb, es = dyd.sum((0, 2)), (dyd * xhat).sum((0, 2))
+        edx = scale.double()[:, None] * sid * (dyd - eb[:, None] / m - xhat * es[:, None] / m)
+        db_, dx = placed(torch.zeros(shape, device=cuda))
+        ds, db = torch.empty(C, device=cuda), torch.empty(C, device=cuda)
+        hk.batch_norm_bwd(dy, x, scale, dx, ds, db, sm, si)
+        torch.cuda.synchronize()
+        helpers.assert_close(dx.contiguous(), num(edx), dtype, "dx %s" % (shape,), rtol=1e-4 if dtype == "fp32" else None)
+        # sums of m terms of both signs: the rounding error is that of the terms
+        helpers.assert_close(ds, num(es), "fp32", "dscale", scale=float(np.sqrt(m)))
+        helpers.assert_close(db, num(eb), "fp32", "dbias", scale=float(np.sqrt(m)))
+        assert clean(db_, dx), shape
+        gb, g2 = placed(dy)
+        hk.batch_norm_bwd(g2, x, scale, g2, None, None, sm, si)
+        torch.cuda.synchronize()
+        assert torch.equal(g2, dx) and clean(gb, g2), shape
