@@ -171,7 +171,159 @@ void softmax_bwd_kernel(SoftmaxArgs a) {
   }
 }
 
-// Softmax along a dimension of extent `dim` with element stride `inner`
+// Softmax along a dimension other than the last, [outer, dim, inner].  A lane holds one 16-byte vector of neighbouring
+// inner positions; the dimension is cut into slices of NK entries, LX lanes per slice, so that the whole column stays in
+// registers: one read, one write.  Slices agree on the maximum and the sum through LDS.  The partial last vector of a
+// plane is read as its last whole one, its own elements are stored one by one (in place, a neighbour may have replaced
+// the others before they were read).  The exponentials are formed twice, once for the sum and once on the way out:
+// holding them in fp32 would cost twice the registers.
+// Bound by HBM and, on odd planes, by the extra cache lines of accesses that straddle them; one thread per column that
+// passed over it three times measured (forward / backward, us) 150 / 160 at 8 x 21 x 263169 fp32, now 81 / 113 (4.4 and 4.7
+// TB/s; 5.3 and 5.5 at 263168); 81 / 77 at 8 x 21 x 263168 bf16, now 34.6 / 48.8; 143 / 103 at 16 x 150 x 16384 bf16, now
+// 44 / 46.5; 447 / 356 at 8 x 256 x 40000 fp32, now 124 / 183.
+constexpr int kDimVecs = 8;      // most entries per lane
+template <int N> __device__ __forceinline__ void slices_share(float* f, float* lds, int lx, int lane, int slices, bool take_max) {
+  // lds: [slices][N / 4][lx] 16-byte vectors
+  u32x4* mine = reinterpret_cast<u32x4*>(lds);
+#pragma unroll
+  for (int q = 0; q < N / 4; ++q)
+    mine[(int(threadIdx.y) * (N / 4) + q) * lx + lane] = u32x4{f2u(f[4 * q]), f2u(f[4 * q + 1]), f2u(f[4 * q + 2]), f2u(f[4 * q + 3])};
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < N; ++j) f[j] = take_max ? kNegInf : 0.f;
+  for (int s = 0; s < slices; ++s) {   // the same order in every slice
+#pragma unroll
+    for (int q = 0; q < N / 4; ++q) {
+      const u32x4 o = mine[(s * (N / 4) + q) * lx + lane];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) f[4 * q + j] = take_max ? fmaxf(f[4 * q + j], u2f(o[j])) : f[4 * q + j] + u2f(o[j]);
+    }
+  }
+}
+
+struct SoftmaxDimArgs {
+  const void* x;       // forward: input;  backward: y
+  const void* dy;
+  void* out;
+  int64_t inner, total;   // total: vectors of all planes, outer * run_vecs
+  int dim, run_vecs, slices;
+};
+// this lane's column: element offset of its vector in entry 0 of the plane, its place in the run, whether it exists
+template <typename T, int LX>
+struct DimColumn {
+  int64_t base;
+  int v, first, count;
+  bool live;
+  __device__ __forceinline__ DimColumn(const SoftmaxDimArgs& a, int nk) {
+    const int64_t id = int64_t(blockIdx.x) * LX + int(threadIdx.x);
+    live = id < a.total;
+    const uint32_t i = uint32_t(live ? id : a.total - 1), o = i / uint32_t(a.run_vecs);
+    v = int(i - o * uint32_t(a.run_vecs));
+    base = int64_t(o) * a.dim * a.inner + vec_column<T, true>(v, int(a.inner));
+    // a slice of a whole wavefront: its entries' addresses are scalar
+    first = (LX == kWave ? __builtin_amdgcn_readfirstlane(int(threadIdx.y)) : int(threadIdx.y)) * nk;
+    count = min(nk, a.dim - first);        // entries of this slice, at least one
+  }
+};
+
+template <typename T, int NK, int LX>
+__global__ __launch_bounds__(1024)
+void softmax_fwd_dim_kernel(SoftmaxDimArgs a) {
+  constexpr int VEC = VecIO<T>::N;
+  extern __shared__ __align__(16) float shared[];   // two [slices][LX][VEC] arrays
+  const DimColumn<T, LX> c(a, NK);
+  const T* xp = static_cast<const T*>(a.x) + c.base;
+  u32x4 raw[NK];
+  // entries past the slice's end are its last one again: no change to the maximum, left out of the sum
+#pragma unroll
+  for (int k = 0; k < NK; ++k) raw[k] = ld16_any<T>(xp + int64_t(c.first + min(k, c.count - 1)) * a.inner);
+  float m[VEC];
+  VecIO<T>::unpack(raw[0], m);
+#pragma unroll
+  for (int k = 1; k < NK; k += 2) {
+    float f[VEC], g[VEC];
+    VecIO<T>::unpack(raw[k], f);
+    VecIO<T>::unpack(raw[k + 1 < NK ? k + 1 : k], g);
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) m[j] = max3(m[j], f[j], g[j]);
+  }
+  if (a.slices > 1) slices_share<VEC>(m, shared, LX, int(threadIdx.x), a.slices, true);
+  float base2[VEC], ml[VEC], s[VEC];
+#pragma unroll
+  for (int j = 0; j < VEC; ++j) {
+    base2[j] = m[j] < -2.3e38f ? 1.0f : kLog2e;   // a column of the type's lowest values, as in softmax_fwd_kernel
+    ml[j] = m[j] * base2[j];
+    s[j] = 0.f;
+  }
+#pragma unroll
+  for (int k = 0; k < NK; ++k) {
+    float f[VEC];
+    VecIO<T>::unpack(raw[k], f);
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) {
+      const float e = __builtin_amdgcn_exp2f(fmaf(f[j], base2[j], -ml[j]));
+      s[j] += k < c.count ? e : 0.f;
+    }
+  }
+  if (a.slices > 1) slices_share<VEC>(s, shared + a.slices * LX * VEC, LX, int(threadIdx.x), a.slices, false);
+  if (!c.live) return;
+#pragma unroll
+  for (int j = 0; j < VEC; ++j) s[j] = 1.0f / s[j];
+  T* yp = static_cast<T*>(a.out) + c.base - vec_column<T, true>(c.v, int(a.inner));   // the run's start
+#pragma unroll
+  for (int k = 0; k < NK; ++k) {
+    if (k < c.count) {
+      float f[VEC];
+      VecIO<T>::unpack(raw[k], f);
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) f[j] = __builtin_amdgcn_exp2f(fmaf(f[j], base2[j], -ml[j])) * s[j];
+      store_row_vec<T, true, false>(yp + int64_t(c.first + k) * a.inner, c.v, f, int(a.inner));
+    }
+  }
+}
+
+template <typename T, int NK, int LX>
+__global__ __launch_bounds__(1024)
+void softmax_bwd_dim_kernel(SoftmaxDimArgs a) {
+  constexpr int VEC = VecIO<T>::N;
+  extern __shared__ __align__(16) float shared[];   // [slices][LX][VEC]
+  const DimColumn<T, LX> c(a, NK);
+  const T* yp = static_cast<const T*>(a.x) + c.base;
+  const T* dyp = static_cast<const T*>(a.dy) + c.base;
+  u32x4 ry[NK], rd[NK];
+#pragma unroll
+  for (int k = 0; k < NK; ++k) {
+    const int64_t at = int64_t(c.first + min(k, c.count - 1)) * a.inner;
+    ry[k] = ld16_any<T>(yp + at);
+    rd[k] = ld16_any<T>(dyp + at);
+  }
+  float dot[VEC] = {};
+#pragma unroll
+  for (int k = 0; k < NK; ++k) {
+    float y[VEC], d[VEC];
+    VecIO<T>::unpack(ry[k], y);
+    VecIO<T>::unpack(rd[k], d);
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) dot[j] = k < c.count ? fmaf(y[j], d[j], dot[j]) : dot[j];
+  }
+  if (a.slices > 1) slices_share<VEC>(dot, shared, LX, int(threadIdx.x), a.slices, false);
+  if (!c.live) return;
+  T* dxp = static_cast<T*>(a.out) + c.base - vec_column<T, true>(c.v, int(a.inner));
+#pragma unroll
+  for (int k = 0; k < NK; ++k) {
+    if (k < c.count) {
+      float y[VEC], d[VEC];
+      VecIO<T>::unpack(ry[k], y);
+      VecIO<T>::unpack(rd[k], d);
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) d[j] = y[j] * (d[j] - dot[j]);
+      store_row_vec<T, true, false>(dxp + int64_t(c.first + k) * a.inner, c.v, d, int(a.inner));
+    }
+  }
+}
+
+// Softmax along a dimension of extent `dim` with element stride `inner`, longer or with shorter planes than the kernels
+// above take, and fp64
 // (inner == 1: rows too long or too unaligned for the register kernels).
 // One thread walks one (outer, inner) position, threads of a wave sit on
 // neighbouring inner positions; for inner == 1 one workgroup takes one row.
@@ -423,6 +575,23 @@ static int softmax_lastdim_typed(SoftmaxArgs a, hipStream_t s) {
   }
 }
 
+template <typename T, bool BWD, int LX>
+static void launch_softmax_dim(const SoftmaxDimArgs& a, int nk, hipStream_t s) {
+  const dim3 grid{unsigned((a.total + LX - 1) / LX)}, block{unsigned(LX), unsigned(a.slices)};
+  const size_t lds = a.slices > 1 ? size_t(BWD ? 1 : 2) * a.slices * LX * VecIO<T>::N * sizeof(float) : 0;
+#define HK_DIM_CASE(N)                                                              \
+  case N:                                                                           \
+    if constexpr (BWD) HK_LAUNCH((softmax_bwd_dim_kernel<T, N, LX>), grid, block, lds, s, a); \
+    else HK_LAUNCH((softmax_fwd_dim_kernel<T, N, LX>), grid, block, lds, s, a);     \
+    break;
+  profile_before(s);
+  switch (nk) {
+    HK_DIM_CASE(1) HK_DIM_CASE(2) HK_DIM_CASE(3) HK_DIM_CASE(4) HK_DIM_CASE(5) HK_DIM_CASE(6) HK_DIM_CASE(7) HK_DIM_CASE(8)
+  }
+#undef HK_DIM_CASE
+  profile_after(s);
+}
+
 template <typename T, typename CT, bool BWD>
 static int softmax_strided_typed(const void* x, const void* dy, void* out, int64_t outer, int64_t dim,
                                  int64_t inner, int64_t x_pitch, int64_t dy_pitch, int64_t out_pitch,
@@ -437,6 +606,26 @@ static int softmax_strided_typed(const void* x, const void* dy, void* out, int64
                          static_cast<const T*>(x), static_cast<T*>(out), dim, x_pitch, out_pitch);
     }
     return launch_check("softmax_longrow_kernel");
+  }
+  if constexpr (!std::is_same<T, double>::value) {
+    constexpr int VEC = VecIO<T>::N;
+    if (inner >= VEC && inner <= 0x7fffffff && dim <= 32 * kDimVecs) {
+      SoftmaxDimArgs a{};
+      a.x = x; a.dy = dy; a.out = out; a.inner = inner; a.dim = int(dim);
+      a.run_vecs = int((inner + VEC - 1) / VEC);
+      a.total = outer * a.run_vecs;
+      // 8 entries a lane; 6 where that holds two 16-bit operands in fewer registers (8 x 21 x 263168 bf16 backward
+      // 56.1 -> 48.8 us, 16 x 150 x 16384 86.7 -> 46.5; forward 34.6 / 34.1 and 43.8 / 47.4 us), if 32 slices do then
+      const int most = std::max(BWD && VEC == 8 ? 6 : kDimVecs, int(dim + 31) / 32);
+      const int slices = int((dim + most - 1) / most), nk = int((dim + slices - 1) / slices);
+      a.slices = int((dim + nk - 1) / nk);
+      if (a.total <= 0x7fffffffLL) {
+        // up to 16 slices of a wavefront each, up to 32 of half a wavefront
+        if (a.slices <= 16) launch_softmax_dim<T, BWD, 64>(a, nk, s);
+        else launch_softmax_dim<T, BWD, 32>(a, nk, s);
+        return launch_check("softmax_dim_kernel");
+      }
+    }
   }
   const int64_t npos = outer * inner;
   const int64_t blocks = (npos + 255) / 256;

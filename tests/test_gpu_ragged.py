@@ -74,6 +74,60 @@ def test_softmax_any_length(hk, cuda, dtype, shift):
         assert torch.equal(tx.contiguous(), ty.contiguous()), cols
 
 
+# entries around one lane's share, a wavefront's and half a wavefront's slices and the most of both; planes around a
+# vector and a workgroup's vectors
+DIM_SHAPES = [(2, d, n) for d in (2, 3, 7, 8, 9, 16, 17, 21, 33, 128, 129, 150, 255, 256, 257) for n in (7, 8, 9, 67)] + \
+             [(1, 5, 1), (1, 5, 3), (3, 21, 515), (2, 40, 1031), (300, 11, 49), (1, 256, 600)]
+
+
+@pytest.mark.parametrize("dtype", ["fp32", "bf16", "fp16"])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_softmax_over_a_leading_dimension(hk, cuda, dtype, shift):
+    import torch
+    dt = {"fp32": torch.float32, "bf16": torch.bfloat16, "fp16": torch.float16}[dtype]
+    low = torch.finfo(dt).min
+    for shape in DIM_SHAPES:
+        n = int(np.prod(shape))
+        x, dy = (helpers.to_torch(helpers.draw(s + n, shape, dtype=dtype), dtype, cuda) for s in (10, 20))
+        x[0, :, -1] = low                         # masked: all of a column, all but one entry, -inf, NaN
+        if shape[2] > 3:
+            x[0, 1:, 0] = low
+            x[0, 0, 1] = -float("inf")
+            x[-1, :, 2] = -float("inf")
+            x[-1, 0, 3] = float("nan")
+
+        def placed(a):
+            buf = torch.full((n + 32,), 7.0, dtype=dt, device=cuda)
+            view = buf[8 + shift:8 + shift + n].view(shape)
+            view.copy_(a)
+            return buf, view
+
+        def clean(buf):
+            return bool((buf[:8 + shift] == 7.0).all()) and bool((buf[8 + shift + n:] == 7.0).all())
+
+        (_, tx), (_, tdy) = placed(x), placed(dy)
+        (yb, ty), (db, tdx) = placed(torch.zeros_like(x)), placed(torch.zeros_like(x))
+        hk.softmax_fwd(tx, ty, 1)
+        torch.cuda.synchronize()
+        ey = torch.softmax(x.double(), 1)
+        assert torch.equal(torch.isnan(ty), torch.isnan(ey)), shape
+        helpers.assert_close(ty.nan_to_num().contiguous(), ey.nan_to_num().cpu().numpy(), dtype, "softmax y %s" % (shape,))
+        y = ty.nan_to_num()
+        (_, ty2) = placed(y)
+        hk.softmax_bwd(ty2, tdy, tdx, 1)
+        torch.cuda.synchronize()
+        yd = y.double() * dy.double()
+        edx = yd - y.double() * yd.sum(1, keepdim=True)
+        helpers.assert_close(tdx.contiguous(), edx.cpu().numpy(), dtype, "softmax dx %s" % (shape,),
+                             scale=float(yd.square().mean().sqrt()), ordinary_rtol=helpers.SOFTMAX_GRADIENT_ORDINARY_RTOL)
+        assert clean(yb) and clean(db), shape
+        (xb, x2), (gb, g2) = placed(x), placed(dy)
+        hk.softmax_fwd(x2, x2, 1)                 # in place
+        hk.softmax_bwd(ty2, g2, g2, 1)
+        torch.cuda.synchronize()
+        assert torch.equal(x2.nan_to_num(), ty.nan_to_num()) and torch.equal(g2, tdx) and clean(xb) and clean(gb), shape
+
+
 # (shape, axes, permutation of the dense array or None): runs of every length around a vector and the widths of the
 # lane groups and workgroups, few and many of them, rows that several workgroups share; rows shorter than a vector;
 # rows on two levels; columns that are no whole number of vectors, over few and many rows
