@@ -368,12 +368,41 @@ struct DalBwdArgs {
   void* dx0;
   void* dx1;
   void* dresidual;
-  float* part[kMaxParts];   // [groups of the grid, cols] each; nullptr: not wanted
+  float* part[kMaxParts];   // [blocks of the grid, cols] each; nullptr: not wanted
   int64_t rows, x0_numrows, z_numrows;
   int cols, nchunks, tpr;
   float inv_cols, scale, rowscale_const;
   int is_rms, dropout;
 };
+
+// A thread's column sums acc -> the partial row of its block.  The block's row groups are folded through LDS first: one
+// partial row per group took the fold kernel longer than the backward itself (16384 x 768 bf16 73 us, 30 us now,
+// with the rows that do not fill their threads on the streaming kernel; 8192 x 4104 110 -> 70 us).
+// Every thread of the block calls (barriers); stage: [rows per block, cols] floats when a block holds several groups.
+__device__ __forceinline__ void put_column_sums(float* part, float* acc, float* stage, int group, int rpb, bool in, int cols,
+                                                int col) {
+  if (part == nullptr) return;   // uniform
+  if (rpb > 1) {
+    __syncthreads();
+    if (in && group > 0) {
+      float* mine = stage + group * cols + col;
+#pragma unroll
+      for (int j = 0; j < kChunk; ++j) mine[j] = acc[j];
+    }
+    __syncthreads();
+    if (in && group == 0) {
+      for (int g = 1; g < rpb; ++g) {
+#pragma unroll
+        for (int j = 0; j < kChunk; ++j) acc[j] += stage[g * cols + col + j];
+      }
+    }
+  }
+  if (in && group == 0) {
+    float* out = part + int64_t(blockIdx.x) * cols + col;
+    st16(out, VecIO<float>::pack(acc));
+    st16(out + 4, VecIO<float>::pack(acc + 4));
+  }
+}
 
 // One chunk of 8 columns per thread.  COLSCALE: per-column scaling (and its gradient); G1: a second
 // affine output (dz1 / gamma1 and their gradients).
@@ -381,6 +410,7 @@ template <typename IT, typename RT, typename WT, bool COLSCALE, bool G1>
 __global__ __launch_bounds__(1024)
 void dal_bwd_kernel(DalBwdArgs a) {
   __shared__ float red[2][kMaxWaves * 2];   // double-buffered by step parity
+  extern __shared__ __align__(16) float stage[];
   const int tpr = a.tpr;
   const int group = __builtin_amdgcn_readfirstlane(int(threadIdx.x) / tpr);
   const int t = int(threadIdx.x) - group * tpr;
@@ -515,13 +545,7 @@ void dal_bwd_kernel(DalBwdArgs a) {
     }
   }
 
-  if (!in) return;
-  const int64_t prow = (int64_t(blockIdx.x) * rpb + group) * a.cols + col;
-  auto put = [&](float* part, const float* acc) {
-    if (part == nullptr) return;
-    st16(part + prow, VecIO<float>::pack(acc));
-    st16(part + prow + 4, VecIO<float>::pack(acc + 4));
-  };
+  auto put = [&](float* part, float* acc) { put_column_sums(part, acc, stage, group, rpb, in, a.cols, col); };
   put(a.part[0], dg0);
   put(a.part[1], db0);
   if constexpr (G1) { put(a.part[2], dg1); put(a.part[3], db1); }
@@ -529,11 +553,12 @@ void dal_bwd_kernel(DalBwdArgs a) {
 }
 
 // The pre-norm residual block's backward, the shape a transformer layer calls: dropout on, the gradient of
-// the residual stream coming in (dx) and going out (dresidual), no scaling, no subsets, one affine pair, and
-// a row that fills every thread's chunk exactly.  With nothing optional left, the row loop holds no branch
+// the residual stream coming in (dx) and going out (dresidual), no scaling, no subsets, one affine pair.  With nothing
+// optional left, the row loop holds no branch
 // around a memory instruction, so the compiler counts outstanding loads exactly and PF rows stay in flight
 // per thread group (a ring of register slots refilled as soon as a slot has been unpacked); rows past the
-// end are clamped to the last row and their results dropped.
+// end are clamped to the last row and their results dropped.  A thread past the row's last chunk works on that chunk with
+// a zero gradient and stores nothing.
 // TPR: the group width when the one group of a block is the whole block and its size is known at compile time
 // (512 threads = 4096 columns), else 0: the launch bound and the cross-wavefront step of the row sums follow it.
 template <typename IT, typename RT, typename WT, int PF, int TPR>
@@ -548,7 +573,9 @@ void dal_bwd_stream_kernel(DalBwdArgs a) {
   const int rpb = TPR ? 1 : int(blockDim.x) / tpr;
   const int wpg = tpr >> 6;
   const int first_wave = group * wpg;
-  const int col = t * kChunk;
+  const bool in = TPR || t < a.nchunks;
+  const int col = (in ? t : a.nchunks - 1) * kChunk;
+  extern __shared__ __align__(16) float stage[];
 
   float g0[kChunk];
   load8_keep<WT>(static_cast<const WT*>(a.gamma) + col, g0);
@@ -603,7 +630,7 @@ void dal_bwd_stream_kernel(DalBwdArgs a) {
     float dy[kChunk];
 #pragma unroll
     for (int j = 0; j < kChunk; ++j) {
-      const float d0 = (GUARD && !valid) ? 0.f : dz[j];
+      const float d0 = ((GUARD && !valid) || !in) ? 0.f : dz[j];
       y[j] = rs * (y[j] - mu);
       dy[j] = g0[j] * d0;
       dg0[j] = fmaf(d0, y[j], dg0[j]);
@@ -614,7 +641,7 @@ void dal_bwd_stream_kernel(DalBwdArgs a) {
     if constexpr (TPR != 0) s = group_allreduce_tuple_fixed<SumTuple<2>, TPR / 64>(s, red[parity]);
     else s = group_allreduce_tuple(s, red[parity], first_wave, wpg);
     parity ^= 1;
-    if (valid) {
+    if (valid && in) {
       const float mdy = a.is_rms ? 0.f : s.v[0] * a.inv_cols;
       const float mdyy = s.v[1] * a.inv_cols;
       float o[kChunk];
@@ -644,15 +671,8 @@ void dal_bwd_stream_kernel(DalBwdArgs a) {
     row0 += round;
   }
 
-  const int64_t prow = (int64_t(blockIdx.x) * rpb + group) * a.cols + col;
-  if (a.part[0]) {
-    st16(a.part[0] + prow, VecIO<float>::pack(dg0));
-    st16(a.part[0] + prow + 4, VecIO<float>::pack(dg0 + 4));
-  }
-  if (a.part[1]) {
-    st16(a.part[1] + prow, VecIO<float>::pack(db0));
-    st16(a.part[1] + prow + 4, VecIO<float>::pack(db0 + 4));
-  }
+  put_column_sums(a.part[0], dg0, stage, group, rpb, in, a.cols, col);
+  put_column_sums(a.part[1], db0, stage, group, rpb, in, a.cols, col);
 }
 
 // Folds [nparts, cols] fp32 partial rows into a [cols] vector of WT; blockIdx.y picks which of the
@@ -674,7 +694,18 @@ void dal_fold_kernel(DalFoldArgs a) {
   const int c = (blockIdx.x * 32 + cg) * 4;
   float acc[4] = {0.f, 0.f, 0.f, 0.f};
   if (c < a.cols) {
-    for (int r = slice; r < a.nparts; r += 16) {
+    constexpr int U = 8;   // loads in flight
+    int r = slice;
+    for (; r + (U - 1) * 16 < a.nparts; r += U * 16) {
+      u32x4 v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) v[u] = ld16_keep(part + int64_t(r + u * 16) * a.cols + c);
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        acc[0] += u2f(v[u].x); acc[1] += u2f(v[u].y); acc[2] += u2f(v[u].z); acc[3] += u2f(v[u].w);
+      }
+    }
+    for (; r < a.nparts; r += 16) {
       const u32x4 v = ld16_keep(part + int64_t(r) * a.cols + c);
       acc[0] += u2f(v.x); acc[1] += u2f(v.y); acc[2] += u2f(v.z); acc[3] += u2f(v.w);
     }
@@ -740,7 +771,7 @@ static BwdShape plan_dal_bwd(int64_t rows, int cols) {
   if (grid > useful) grid = useful;
   if (grid < 1) grid = 1;
   p.grid = int(grid);
-  p.nparts = grid * p.rpb;
+  p.nparts = grid;
   return p;
 }
 
@@ -918,14 +949,15 @@ int hk_dropout_add_ln_bwd_ex(const hkDropoutAddLnBwdParams* pp, hkStream_t strea
   }
 
   BwdShape sh = plan_dal_bwd(p.rows, int(p.cols));
-  // the pre-norm residual block with full rows has a kernel of its own; it keeps two rows in flight per
+  // the pre-norm residual block has a kernel of its own; it keeps two rows in flight per
   // thread group and runs best with one workgroup per compute unit (measured: 264 us against 283 us with
-  // two at [32768 x 4096] bf16).  The workspace was sized for the larger grid.
+  // two at [32768 x 4096] bf16, 29.6 against 32.3 us at
+  // [16384 x 768]).  The workspace was sized for the larger grid.
   const bool stream_form = dropout && p.dx && p.dresidual && !subset && !p.rowscale && !colscale && !parallel &&
-                           int(p.cols) / kChunk == sh.tpr && tune_get(TUNE_NORM_BWD_PREFETCH) != 1;
+                           tune_get(TUNE_NORM_BWD_PREFETCH) != 1;
   if (stream_form && tune_get(TUNE_NORM_BWD_BLOCKS) <= 0 && sh.grid > device_cu_count()) {
     sh.grid = device_cu_count();
-    sh.nparts = int64_t(sh.grid) * sh.rpb;
+    sh.nparts = sh.grid;
   }
   const int nslots = count_parts(p);
   const size_t slot_floats = size_t(sh.nparts) * size_t(p.cols);
@@ -962,11 +994,13 @@ int hk_dropout_add_ln_bwd_ex(const hkDropoutAddLnBwdParams* pp, hkStream_t strea
     profile_before(s);
     // two rows in flight where the ring fits the registers (a 16-bit residual stream), else one
     constexpr int PF = sizeof(RT) == 2 ? 2 : 1;
-    if (stream_form && sh.tpr == 512 && sh.block == 512) HK_LAUNCH((dal_bwd_stream_kernel<IT, RT, WT, PF, 512>), grid, block, 0, s, a);
-    else if (stream_form) HK_LAUNCH((dal_bwd_stream_kernel<IT, RT, WT, PF, 0>), grid, block, 0, s, a);
-    else if (g1) HK_LAUNCH((dal_bwd_kernel<IT, RT, WT, false, true>), grid, block, 0, s, a);
-    else if (colscale) HK_LAUNCH((dal_bwd_kernel<IT, RT, WT, true, false>), grid, block, 0, s, a);
-    else HK_LAUNCH((dal_bwd_kernel<IT, RT, WT, false, false>), grid, block, 0, s, a);
+    const bool full = int(p.cols) / kChunk == sh.tpr;
+    const size_t lds = sh.rpb > 1 ? size_t(sh.rpb) * size_t(p.cols) * sizeof(float) : 0;
+    if (stream_form && full && sh.tpr == 512 && sh.block == 512) HK_LAUNCH((dal_bwd_stream_kernel<IT, RT, WT, PF, 512>), grid, block, lds, s, a);
+    else if (stream_form) HK_LAUNCH((dal_bwd_stream_kernel<IT, RT, WT, PF, 0>), grid, block, lds, s, a);
+    else if (g1) HK_LAUNCH((dal_bwd_kernel<IT, RT, WT, false, true>), grid, block, lds, s, a);
+    else if (colscale) HK_LAUNCH((dal_bwd_kernel<IT, RT, WT, true, false>), grid, block, lds, s, a);
+    else HK_LAUNCH((dal_bwd_kernel<IT, RT, WT, false, false>), grid, block, lds, s, a);
     profile_after(s);
     int r = launch_check("dal_bwd_kernel");
     if (r != HK_OK || nslots == 0) return r;
