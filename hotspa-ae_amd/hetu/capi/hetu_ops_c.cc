@@ -108,6 +108,27 @@ void copy_out(const NDArray& result, HtArray* out, const Stream& stream) {
   stream.Sync();   // the caller owns dst and may read it right away
 }
 
+// The caller's buffer as the place of an accelerator's loss, if the loss can be written there directly (the copy of one
+// value from a pool array took longer than the kernels of a 256 x 1000 loss): dense, of the loss's type and extent, apart
+// from the inputs.  Undefined otherwise: the loss goes through copy_out() and its checks.
+NDArray loss_buffer(const NDArray& preds, const NDArray& labels, const HtArray* out, ReductionType reduction,
+                    const Stream& stream) {
+  if (!stream.device().is_cuda() || out == nullptr || !preds.is_defined() || !labels.is_defined() || preds->ndim() == 0)
+    return NDArray();
+  NDArray dst = wrap(out);
+  size_t rows = 1;
+  for (size_t i = 0; i + 1 < preds->ndim(); ++i) rows *= size_t(preds->shape(i));
+  const size_t numel = reduction == kNONE ? rows : 1;
+  if (numel == 0 || dst->numel() != numel || dst->ndim() != 1 || !dst->is_contiguous() || dst->dtype() != preds->dtype() ||
+      dst->device() != preds->device())
+    return NDArray();
+  auto first = [](const NDArray& a) { return reinterpret_cast<uintptr_t>(a->storage()->data_ptr().ptr); };
+  auto past = [&](const NDArray& a) { return first(a) + a->storage()->data_ptr().size; };
+  for (const NDArray* in : {&preds, &labels})
+    if (first(dst) < past(*in) && first(*in) < past(dst)) return NDArray();
+  return dst;
+}
+
 hetu::impl::CachingMemoryPool& caching_pool(int device_index) {
   auto pool = GetMemoryPool(Device(kCUDA, DeviceIndex(device_index)));
   auto* cp = dynamic_cast<hetu::impl::CachingMemoryPool*>(pool.get());
@@ -535,9 +556,14 @@ int ht_ndarray_sceloss(const HtArray* preds, const HtArray* labels, int sparse, 
                        int reduction, HtArray* out, int stream_index) {
   return guarded([&] {
     const auto red = static_cast<ReductionType>(reduction);
-    NDArray r = sparse ? NDArray::sceloss(wrap(preds), wrap(labels), ignored_index, red, stream_index)
-                       : NDArray::sceloss(wrap(preds), wrap(labels), red, stream_index);
-    copy_out(r, out, stream_of(preds, stream_index));
+    const NDArray p = wrap(preds), l = wrap(labels);
+    const Stream st = stream_of(preds, stream_index);
+    NDArray direct = loss_buffer(p, l, out, red, st);
+    const bool in_place = direct.is_defined();
+    NDArray r = sparse ? NDArray::sceloss(p, l, ignored_index, red, stream_index, direct)
+                       : NDArray::sceloss(p, l, red, stream_index, direct);
+    if (in_place) st.Sync();   // the caller owns out and may read it right away
+    else copy_out(r, out, st);
   });
 }
 

@@ -1122,3 +1122,27 @@ def test_permuted_views_run_in_place(ops, cuda, dtype):
     ops.stream_sync()
     assert ops.pool_stats()["alloc_cnt"] == before and torch.equal(loss_v, loss_d), "sparse CE"
     both(lambda a, d, out: ops.softmax_cross_entropy_sparse_gradient(a, labels, gl, out, -100), "sparse CE gradient")
+
+
+@pytest.mark.parametrize("reduction", ["none", "mean", "sum"])
+def test_ndarray_sceloss_buffers(ops, cuda, reduction):
+    """The loss goes straight into a dense buffer of its own; a buffer of another rank, and one that lies in the labels or
+    in the predictions, get the same values by way of a copy; one that does not fit is refused."""
+    import torch
+    rows, cols = 12, 40
+    x = helpers.draw(77, (rows, cols), dtype="fp32")
+    lab = np.arange(rows, dtype=np.int64) * 3
+    tx = helpers.to_torch(x, "fp32", cuda)
+    want = oracle.sce_sparse_fwd(x, lab, -100)
+    want = want if reduction == "none" else np.array([want.mean() if reduction == "mean" else want.sum()])
+    n = want.size
+    tl = torch.from_numpy(lab).to(cuda)
+    inside_labels, inside_preds = torch.from_numpy(lab).to(cuda), tx.clone()
+    for out, labels, preds in ((torch.empty(n, device=cuda), tl, tx), (torch.empty(1, n, device=cuda), tl, tx),
+                               (inside_labels.view(torch.float32)[:n], inside_labels, tx),
+                               (inside_preds.view(-1)[5:5 + n], tl, inside_preds)):
+        ops.ndarray_sceloss(preds, labels, out, reduction, ignored_index=-100)
+        helpers.assert_close(out.view(-1), want, "fp32", "loss")
+    for bad in (torch.empty(n + 1, device=cuda), torch.empty(n, device=cuda, dtype=torch.bfloat16)):
+        with pytest.raises(Exception):
+            ops.ndarray_sceloss(tx, tl, bad, reduction, ignored_index=-100)
