@@ -8,8 +8,8 @@
 // writes the row once.  Rows whose label equals the ignored index are not read
 // at all: loss 0 / a zero gradient row is written.
 //
-// Sparse labels take rows of any length and alignment this way (see RowSpan); rows longer than a workgroup's registers
-// hold are streamed (sce_long_kernel).
+// Sparse labels take rows of any length and alignment this way (see RowSpan); 16-bit rows of 32768 to 65536 columns are
+// kept packed (sce_packed_kernel), longer ones are streamed (sce_long_kernel).
 #include "hk_common.h"
 
 #include <algorithm>
@@ -313,12 +313,13 @@ void sce_sparse_bwd_kernel(SceArgs a) {
 }
 
 // ------------------------------- long rows ---------------------------------
-// Sparse labels, rows that do not fit a workgroup's registers: the workgroup streams the row, kLongVecs vectors per
+// Sparse labels, rows that do not fit a workgroup's registers (65536 16-bit elements, 32768 fp32): the workgroup streams the row, kLongVecs vectors per
 // thread and step, and every thread keeps a running (maximum, sum of exponentials) that it re-bases once per step.
 // The backward reads the row a second time, from its end, so that what was read last is found in the nearest cache
-// (1024 x 128256 bf16 116 -> 111 us), and is bound by what that second read costs: 4096 x 50257 bf16 611 us by
-// elements -> 160 us (4.9 TB/s of row and gradient), forward 358 -> 83 us (4.7 TB/s).  Every step has as many threads
-// as its share of the row needs (1024 throughout: 167 and 86 us).
+// (1024 x 128256 bf16 116 -> 111 us), and is bound by what that second read costs: 1024 x 128256 bf16 679 us by
+// elements -> 111 us (4.7 TB/s of row and gradient), forward 307 -> 48 us (5.5 TB/s).  Every step has as many threads
+// as its share of the row needs (4096 x 50257 bf16, which sce_packed_kernel takes now: 160 and 83 us, with 1024
+// throughout 167 and 86 us).
 constexpr int kLongThreads = 1024;
 constexpr int kLongVecs = 4;
 
@@ -410,6 +411,102 @@ void sce_long_kernel(SceArgs a) {
       }
     }
     span.store_edge(dxr, grad(edge, span.edge == lab));
+  }
+}
+
+// --------------------------- rows kept as loaded ---------------------------
+// Sparse labels, 16-bit rows of more than kLongVecs and up to kPackedVecs vectors per thread of a 1024-thread workgroup:
+// the vectors stay in registers as they were loaded and are unpacked three times (maximum, sum, gradient), so that twice
+// the elements fit the 64 registers at which two such workgroups share a compute unit (43 forward, 56 backward), and the
+// row is read once.  Bound by HBM and by the two rows that a compute unit has under way, whose loads, arithmetic and
+// stores overlap less than four would.  Against sce_long_kernel, bf16, forward / backward: 4096 x 50257 83.9 / 164.5 ->
+// 78.3 / 152.9 us (5.4 TB/s backward), x 50304 81.6 / 159.7 -> 78.0 / 146.8, x 65536 88.5 / 202.5 -> 88.6 / 182.4,
+// x 33000 49.2 / 106.6 -> 47.0 / 99.6.
+constexpr int kPackedVecs = 8;
+
+// The compiler would keep the unpacked elements from one pass to the next otherwise: twice the registers.
+template <int NV>
+__device__ __forceinline__ void unpack_again(u32x4 (&raw)[NV]) {
+#pragma unroll
+  for (int i = 0; i < NV; ++i) asm volatile("" : "+v"(raw[i]));
+}
+
+template <typename T, bool BWD>
+__global__ __launch_bounds__(1024, 8)
+void sce_packed_kernel(SceArgs a) {
+  constexpr int VEC = VecIO<T>::N, NV = kPackedVecs;
+  __shared__ float red[kMaxWaves * 3];
+  const int t = int(threadIdx.x), tpr = int(blockDim.x), nwaves = tpr >> 6;
+  const int64_t i0 = blockIdx.x, row = dense_row_index(i0, a.rn);
+  const int64_t label = a.labels[row];
+  T* dxr = BWD ? static_cast<T*>(a.out) + i0 * a.out_pitch + outer_level_offset(a.out_lv) : nullptr;
+  if (label == a.ignored_index) {
+    if constexpr (BWD) sce_store_zero_row<T, true>(dxr, a.cols, t, tpr);
+    else if (t == 0) sce_store_ignored<T>(a, row);
+    return;
+  }
+  const T* xr = static_cast<const T*>(a.logits) + i0 * a.x_pitch + outer_level_offset(a.x_lv);
+  const RowSpan<T, true> span(xr, a.cols, t);
+  u32x4 raw[NV];
+#pragma unroll
+  for (int i = 0; i < NV; ++i)
+    raw[i] = span.template load<false>(xr, i * tpr + t, (i + 1) * tpr <= span.nvec);
+  const float edge = span.load_edge(xr);
+  float m = edge;
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    float f[VEC];
+    VecIO<T>::unpack(raw[i], f);
+#pragma unroll
+    for (int j = 0; j < VEC; j += 2) m = max3(m, f[j], f[j + 1]);
+  }
+  const float ml = log2_of_max(m);
+  unpack_again(raw);
+  float s4[4] = {__builtin_amdgcn_exp2f(fmaf(edge, kLog2e, -ml)), 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    float f[VEC];
+    VecIO<T>::unpack(raw[i], f);
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) s4[j & 3] += __builtin_amdgcn_exp2f(fmaf(f[j], kLog2e, -ml));
+  }
+  const float s = (s4[0] + s4[1]) + (s4[2] + s4[3]);
+  if constexpr (!BWD) {
+    MaxSumMaxTuple p;
+    p.v[0] = ml; p.v[1] = s; p.v[2] = m;
+    p = group_allreduce_tuple(p, red, 0, nwaves);
+    if (p.v[0] == kLowestLog2) p.v[1] = sce_lowest_count<T, false>(xr, a.cols, t, tpr, nwaves, red, p.v[2]);   // uniform
+    if (t == 0) sce_store_loss<T>(a, row, label, xr, p);
+  } else {
+    const float g = sce_row_grad<T, float>(a, row);
+    MaxSumTuple p;
+    p.v[0] = ml; p.v[1] = s;
+    p = group_allreduce_tuple(p, red, 0, nwaves);
+    const int lab = sce_label_column(label, a.cols);
+    if (p.v[0] == kLowestLog2) {   // uniform
+      sce_lowest_bwd<T, false>(xr, dxr, a.cols, lab, g, t, tpr, nwaves, red);
+      return;
+    }
+    const float ML = p.v[0], scale = g / p.v[1];
+    unpack_again(raw);
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int v = i * tpr + t;
+      if (v < span.nvec) {
+        float o[VEC];
+        VecIO<T>::unpack(raw[i], o);
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) o[j] = __builtin_amdgcn_exp2f(fmaf(o[j], kLog2e, -ML)) * scale;
+        const int lsub = lab - (span.head + v * VEC);
+        if (uint32_t(lsub) < uint32_t(VEC)) {
+#pragma unroll
+          for (int j = 0; j < VEC; ++j)
+            if (j == lsub) o[j] -= g;
+        }
+        span.store(dxr, v, o);
+      }
+    }
+    span.store_edge(dxr, __builtin_amdgcn_exp2f(fmaf(edge, kLog2e, -ML)) * scale - (span.edge == lab ? g : 0.f));
   }
 }
 
@@ -676,10 +773,7 @@ static int sce_typed(SceArgs a, hipStream_t s) {
   const int max_nv = (MODE == 0) ? 8 : 32 / VEC;
   const int max_nv_wave = (MODE == 0) ? 8 : 32 / VEC;
   int threads = 0, nv = 0;
-  bool shaped = pick_sce_shape(a.nvec, max_nv_wave, max_nv, &threads, &nv);
-  // the forward of long 16-bit rows is faster streamed than with 64 floats a thread in more than 512 threads
-  // (4096 x 50304 bf16 94 -> 82 us, x 65536 105 -> 89 us; 32000 columns, 512 threads, 155 us against 230 us)
-  if (MODE == 0 && VEC == 8 && a.nvec > 4096) shaped = false;
+  const bool shaped = pick_sce_shape(a.nvec, max_nv_wave, max_nv, &threads, &nv);
   const dim3 levels{unsigned(a.n0), unsigned(a.n1), unsigned(a.n2)};
   auto launch = [&](auto ragged) {
     constexpr bool RAGGED = decltype(ragged)::value;
@@ -689,6 +783,19 @@ static int sce_typed(SceArgs a, hipStream_t s) {
     }
     return launch_sce_nv<T, MODE, false, RAGGED>(a, nv, levels, dim3{unsigned(threads)}, s);
   };
+  if constexpr (MODE < 2 && VEC == 8) {
+    // The forward with 64 floats a thread in more than 512 threads is slower (4096 x 50304 bf16 94 us, kept packed 78,
+    // x 65536 105 against 89; 32000 columns, 512 threads, stay with it: 155 us, streamed 230), the backward does not fit
+    // that.  fp32 vectors have nothing to unpack: 4096 x 32000 78.0 / 177.7 us against 79.0 / 177.4, x 20001 48.3 / 114.9
+    // against 48.5 / 116.2, so they stay with the kernels above.
+    if (a.nvec > kLongVecs * 1024 && a.nvec <= kPackedVecs * 1024 && tune_get(TUNE_SCE_THREADS) <= 0) {
+      threads = ((a.nvec + kPackedVecs - 1) / kPackedVecs + 63) / 64 * 64;
+      profile_before(s);
+      HK_LAUNCH((sce_packed_kernel<T, MODE == 1>), levels, dim3(unsigned(threads)), 0, s, a);
+      profile_after(s);
+      return launch_check("sce_packed_kernel");
+    }
+  }
   if (vec_ok && shaped) return launch(std::false_type{});
   if constexpr (MODE < 2) {
     if (shaped) return launch(std::true_type{});
