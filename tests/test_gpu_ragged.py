@@ -196,8 +196,8 @@ def test_softmax_of_lowest_values(hk, cuda, dtype, cols):
     assert torch.equal(x[ok], y[ok])
 
 
-# vectors per row around 1, a wavefront, the widths of the workgroups, and (65536 16-bit / 32768 32-bit elements in the
-# forward, 32768 in the backward) past what a workgroup holds: whole vectors, one element more, one fewer
+# vectors per row around 1, a wavefront, the widths of the workgroups, and (65536 16-bit / 32768 32-bit elements)
+# past what a workgroup holds: whole vectors, one element more, one fewer
 def _class_counts(dtype):
     vec = 16 // ES[dtype]
     out = {v * vec + k for v in (1, 2, 63, 64, 65, 256, 512, 1000) for k in (0, 1, vec - 1)}
