@@ -613,28 +613,33 @@ struct OnlineSoftmaxTuple {
 using MaxSumTuple = OnlineSoftmaxTuple<2>;
 using MaxSumMaxTuple = OnlineSoftmaxTuple<3>;
 
-// The maximum of a thread's elements in the log2 domain, kept finite: a maximum near the type's lowest value (logits
-// masked with it) would overflow to -inf and turn 0 * inf into the row's sum, an empty maximum would need a select.
-// Elements at such a maximum come out as 0, as they should next to any ordinary element of the row; a row whose own
-// maximum is that low is what row_max_count() is for.
-constexpr float kLowestLog2 = -3.402823466e38f;
-__device__ __forceinline__ float log2_of_max(float m) { return fmaxf(m * 1.4426950408889634f, kLowestLog2); }
+// The maximum of a thread's elements in the log2 domain, kept finite.  Below: a maximum near the type's lowest value
+// (logits masked with it) would overflow to -inf and turn 0 * inf into the row's sum, an empty maximum would need a
+// select; elements at such a maximum come out as 0, as they should next to any ordinary element of the row.  Above: a
+// maximum near the type's highest value would overflow to +inf, which leaves no element of the row a weight.  A row
+// whose own maximum is that low or that high (past_log2_range() of the row's) is what row_max_count() is for.
+constexpr float kLog2Bound = 3.402823466e38f;
+__device__ __forceinline__ float log2_of_max(float m) {
+  return fminf(fmaxf(m * 1.4426950408889634f, -kLog2Bound), kLog2Bound);
+}
+__device__ __forceinline__ bool past_log2_range(float ml) { return fabsf(ml) == kLog2Bound; }
 
-// Rows whose maximum is below kLowestLog2 / log2(e): two different values down there lie so far apart that the softmax
-// is 1 / count at the maximum and 0 elsewhere.  M = the row's maximum, returned: how many elements equal it (NaN if
-// the row holds a NaN).  Reads the row again, element by element; `allred` merges over the row's lanes and may be
-// called twice.
+// Rows whose maximum's magnitude is past kLog2Bound / log2(e): two different values out there lie so far apart that the
+// softmax is 1 / count at the maximum and 0 elsewhere.  M = the row's maximum, returned: how many elements equal it (NaN
+// if the row holds a NaN or +inf).  Reads the row again, element by element; `allred` merges over the row's lanes and
+// may be called twice.
 template <typename T, typename AllRed>
 __device__ __forceinline__ float row_max_count(const T* row, int cols, int t, int tpr, AllRed allred, float& M) {
   float m = -__builtin_huge_valf();
-  for (int c = t; c < cols; c += tpr) m = fmaxf(m, Cvt<T>::load(row + c));
+  for (int64_t c = t; c < cols; c += tpr) m = fmaxf(m, Cvt<T>::load(row + c));
   M = allred(MaxTuple{{m}}).v[0];
   SumTuple<1> n = SumTuple<1>::identity();
-  for (int c = t; c < cols; c += tpr) {
+  for (int64_t c = t; c < cols; c += tpr) {
     const float x = Cvt<T>::load(row + c);
     n.v[0] += x == M ? 1.f : (x != x ? x : 0.f);
   }
-  return allred(n).v[0];
+  const float count = allred(n).v[0];
+  return M <= kLog2Bound ? count : __builtin_nanf("");
 }
 
 // ---------------------------------------------------------------------------

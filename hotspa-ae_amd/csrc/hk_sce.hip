@@ -68,22 +68,22 @@ __device__ __forceinline__ void row_coords(const SceArgs& a, int& tpr, int& t, i
   nwaves = WAVE_ROW ? 1 : int(blockDim.x >> 6);
 }
 
-// Rows whose maximum lies at the type's lowest values (p.v[0] == kLowestLog2 after the reduction): the sum and the
-// gradient from the row itself.
+// Rows whose maximum lies at the type's lowest or highest values (past_log2_range(p.v[0]) after the reduction): the sum
+// and the gradient from the row itself.
 template <typename T, bool WAVE_ROW>
-__device__ __forceinline__ float sce_lowest_count(const T* xr, int cols, int t, int tpr, int nwaves, float* red, float& M) {
+__device__ __forceinline__ float sce_extreme_count(const T* xr, int cols, int t, int tpr, int nwaves, float* red, float& M) {
   return row_max_count<T>(xr, cols, t, tpr, [&](auto v) {
     if constexpr (WAVE_ROW) return wave_allreduce_tuple(v);
     else { __syncthreads(); return group_allreduce_tuple(v, red, 0, nwaves); }   // red may still be read
   }, M);
 }
 template <typename T, bool WAVE_ROW>
-__device__ __forceinline__ void sce_lowest_bwd(const T* xr, T* dxr, int cols, int lab, float g, int t, int tpr, int nwaves,
-                                               float* red) {
+__device__ __forceinline__ void sce_extreme_bwd(const T* xr, T* dxr, int cols, int lab, float g, int t, int tpr, int nwaves,
+                                                float* red) {
   float M;
-  const float n = sce_lowest_count<T, WAVE_ROW>(xr, cols, t, tpr, nwaves, red, M);
+  const float n = sce_extreme_count<T, WAVE_ROW>(xr, cols, t, tpr, nwaves, red, M);
   const float scale = g / (M == kNegInf ? __builtin_nanf("") : n);   // a row of nothing but -inf has no softmax
-  for (int c = t; c < cols; c += tpr)
+  for (int64_t c = t; c < cols; c += tpr)
     Cvt<T>::store(dxr + c, (Cvt<T>::load(xr + c) == M ? 1.f : 0.f) * scale - (c == lab ? g : 0.f));
 }
 
@@ -149,7 +149,7 @@ __device__ __forceinline__ void sce_store_loss(const SceArgs& a, int64_t row, in
     // sum exp(x - M) = S * 2^(ML - M * log2e)
     a.stats[row] = M;
     a.stats[a.rows + row] = (M == kNegInf) ? 0.f
-        : p.v[0] == kLowestLog2 ? p.v[1] : p.v[1] * __builtin_amdgcn_exp2f(-fmaf(M, kLog2e, -p.v[0]));
+        : past_log2_range(p.v[0]) ? p.v[1] : p.v[1] * __builtin_amdgcn_exp2f(-fmaf(M, kLog2e, -p.v[0]));
     const int64_t local = label - a.vocab_start;
     a.stats[2 * a.rows + row] = (local >= 0 && local < a.cols) ? Cvt<T>::load(xr + local) : 0.f;
     return;
@@ -158,8 +158,8 @@ __device__ __forceinline__ void sce_store_loss(const SceArgs& a, int64_t row, in
   if (label >= 0 && label < a.cols) {
     const float xl = Cvt<T>::load(xr + label);
     // sum exp(x - M) = S * 2^(ML - M * log2e); the fma recovers the rounding of ML exactly
-    // (a row of lowest values has its sum relative to M itself)
-    const float log2s = __builtin_amdgcn_logf(p.v[1]) - (p.v[0] == kLowestLog2 ? 0.f : fmaf(M, kLog2e, -p.v[0]));
+    // (a row of extreme values has its sum relative to M itself)
+    const float log2s = __builtin_amdgcn_logf(p.v[1]) - (past_log2_range(p.v[0]) ? 0.f : fmaf(M, kLog2e, -p.v[0]));
     // M - xl first: the difference of two logits is (nearly) exact however large their common offset is, and
     // the sum then rounds at the size of the loss, not of the logits
     r = log2s * kLn2 + (M - xl);
@@ -213,7 +213,7 @@ void sce_sparse_fwd_kernel(SceArgs a) {
   MaxSumMaxTuple p;
   p.v[0] = ml; p.v[1] = s; p.v[2] = m;
   p = WAVE_ROW ? wave_allreduce_tuple(p) : group_allreduce_tuple(p, red, 0, nwaves);
-  if (p.v[0] == kLowestLog2) p.v[1] = sce_lowest_count<T, WAVE_ROW>(xr, a.cols, t, tpr, nwaves, red, p.v[2]);   // uniform
+  if (past_log2_range(p.v[0])) p.v[1] = sce_extreme_count<T, WAVE_ROW>(xr, a.cols, t, tpr, nwaves, red, p.v[2]);   // uniform
   if (t == 0) sce_store_loss<T>(a, row, label, xr, p);
 }
 
@@ -289,8 +289,8 @@ void sce_sparse_bwd_kernel(SceArgs a) {
   p.v[0] = ml; p.v[1] = s;
   p = WAVE_ROW ? wave_allreduce_tuple(p) : group_allreduce_tuple(p, red, 0, nwaves);
   const int lab = sce_label_column(label, a.cols);
-  if (p.v[0] == kLowestLog2) {   // uniform
-    sce_lowest_bwd<T, WAVE_ROW>(xr, dxr, a.cols, lab, g, t, tpr, nwaves, red);
+  if (past_log2_range(p.v[0])) {   // uniform
+    sce_extreme_bwd<T, WAVE_ROW>(xr, dxr, a.cols, lab, g, t, tpr, nwaves, red);
     return;
   }
   const float scale = __builtin_amdgcn_exp2f(ml - p.v[0]) / p.v[1] * g;
@@ -369,7 +369,7 @@ void sce_long_kernel(SceArgs a) {
     MaxSumMaxTuple p;
     p.v[0] = ml; p.v[1] = s; p.v[2] = m;
     p = group_allreduce_tuple(p, red, 0, nwaves);
-    if (p.v[0] == kLowestLog2) p.v[1] = sce_lowest_count<T, false>(xr, a.cols, t, tpr, nwaves, red, p.v[2]);   // uniform
+    if (past_log2_range(p.v[0])) p.v[1] = sce_extreme_count<T, false>(xr, a.cols, t, tpr, nwaves, red, p.v[2]);   // uniform
     if (t == 0) sce_store_loss<T>(a, row, label, xr, p);
   } else {
     const float g = sce_row_grad<T, float>(a, row);
@@ -377,8 +377,8 @@ void sce_long_kernel(SceArgs a) {
     p.v[0] = ml; p.v[1] = s;
     p = group_allreduce_tuple(p, red, 0, nwaves);
     const int lab = sce_label_column(label, a.cols);
-    if (p.v[0] == kLowestLog2) {   // uniform
-      sce_lowest_bwd<T, false>(xr, dxr, a.cols, lab, g, t, tpr, nwaves, red);
+    if (past_log2_range(p.v[0])) {   // uniform
+      sce_extreme_bwd<T, false>(xr, dxr, a.cols, lab, g, t, tpr, nwaves, red);
       return;
     }
     const float ML = p.v[0];
@@ -475,7 +475,7 @@ void sce_packed_kernel(SceArgs a) {
     MaxSumMaxTuple p;
     p.v[0] = ml; p.v[1] = s; p.v[2] = m;
     p = group_allreduce_tuple(p, red, 0, nwaves);
-    if (p.v[0] == kLowestLog2) p.v[1] = sce_lowest_count<T, false>(xr, a.cols, t, tpr, nwaves, red, p.v[2]);   // uniform
+    if (past_log2_range(p.v[0])) p.v[1] = sce_extreme_count<T, false>(xr, a.cols, t, tpr, nwaves, red, p.v[2]);   // uniform
     if (t == 0) sce_store_loss<T>(a, row, label, xr, p);
   } else {
     const float g = sce_row_grad<T, float>(a, row);
@@ -483,8 +483,8 @@ void sce_packed_kernel(SceArgs a) {
     p.v[0] = ml; p.v[1] = s;
     p = group_allreduce_tuple(p, red, 0, nwaves);
     const int lab = sce_label_column(label, a.cols);
-    if (p.v[0] == kLowestLog2) {   // uniform
-      sce_lowest_bwd<T, false>(xr, dxr, a.cols, lab, g, t, tpr, nwaves, red);
+    if (past_log2_range(p.v[0])) {   // uniform
+      sce_extreme_bwd<T, false>(xr, dxr, a.cols, lab, g, t, tpr, nwaves, red);
       return;
     }
     const float ML = p.v[0], scale = g / p.v[1];

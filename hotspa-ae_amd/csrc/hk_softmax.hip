@@ -65,11 +65,11 @@ void softmax_fwd_kernel(SoftmaxArgs a) {
   // exponentials, and an element held twice then comes out the same twice.  Across wavefronts each thread keeps its
   // own maximum and the pairs are merged, which costs one barrier instead of two.
   if constexpr (LPR > 0) m = Lanes::allreduce(MaxTuple{{m}}, red).v[0];
-  // A row whose maximum lies at the type's lowest values (scores masked with it) would overflow in the log2 domain: two
-  // different values down there are so far apart that any base gives 1 at the maximum and 0 elsewhere, so lanes that
-  // agree on the row's maximum take base 2 for such a row.  A whole workgroup's threads have maxima of their own, kept
-  // finite by log2_of_max(), and the row is counted below.
-  const float k = (LPR > 0 && m < -2.3e38f) ? 1.0f : kLog2e;
+  // A row whose maximum lies at the type's lowest values (scores masked with it) or at its highest would overflow in the
+  // log2 domain: two different values out there are so far apart that any base gives 1 at the maximum and 0 elsewhere, so
+  // lanes that agree on the row's maximum take base 2 for such a row.  A whole workgroup's threads have maxima of their
+  // own, kept finite by log2_of_max(), and the row is counted below.
+  const float k = (LPR > 0 && fabsf(m) > 2.3e38f) ? 1.0f : kLog2e;
   const float ml = LPR > 0 ? m * k : log2_of_max(m);
   float s = 0.f;
 #pragma unroll
@@ -90,7 +90,7 @@ void softmax_fwd_kernel(SoftmaxArgs a) {
     MaxSumTuple p;
     p.v[0] = ml; p.v[1] = s;
     p = Lanes::allreduce(p, red);
-    if (p.v[0] == kLowestLog2) {   // uniform: a row of the type's lowest values
+    if (past_log2_range(p.v[0])) {   // uniform
       float M;
       const float n = row_max_count<T>(xr, a.cols, t, tpr, [&](auto v) {
         __syncthreads();   // red may still be read
@@ -251,7 +251,7 @@ void softmax_fwd_dim_kernel(SoftmaxDimArgs a) {
   float base2[VEC], ml[VEC], s[VEC];
 #pragma unroll
   for (int j = 0; j < VEC; ++j) {
-    base2[j] = m[j] < -2.3e38f ? 1.0f : kLog2e;   // a column of the type's lowest values, as in softmax_fwd_kernel
+    base2[j] = fabsf(m[j]) > 2.3e38f ? 1.0f : kLog2e;   // lowest or highest values, as in softmax_fwd_kernel
     ml[j] = m[j] * base2[j];
     s[j] = 0.f;
   }

@@ -365,3 +365,81 @@ def test_layer_norm_bwd_any_length_modes(hk, cuda, dtype, cols):
     torch.cuda.synchronize()
     for got, want, what in ((tdx, edx, "dx"), (tdg, edg, "dgamma"), (tdb, edb, "dbeta")):
         helpers.assert_close(got, want, dtype, what, scale=None if what == "dx" else many)
+
+
+def _highest_rows(torch, cuda, seed, cols, dt):
+    """Six rows: one element of the type's highest value, two of them, all of them, one above a second highest, highest
+    beside lowest, and +inf beside the highest.  softmax is 1 / count at the row's maximum but for the last, all NaN."""
+    x = torch.from_numpy(helpers.draw(seed, (6, cols))).to(dt).to(cuda)
+    high = torch.finfo(dt).max
+    x[0, cols // 2] = high
+    x[1, 0] = x[1, cols - 1] = high
+    x[2, :] = high
+    x[3, :] = high / 1.25
+    x[3, 1] = high
+    x[4, :] = -high
+    x[4, cols - 2] = high
+    x[5, :] = high
+    x[5, 1] = float("inf")
+    return x
+
+
+# rows that some lanes of a wavefront, a wavefront and a workgroup hold, whole vectors and ragged ones
+@pytest.mark.parametrize("dtype", ["fp32", "bf16", "fp16"])
+@pytest.mark.parametrize("cols", [3, 40, 41, 130, 1001, 2047, 2048, 4097, 9000])
+def test_softmax_of_highest_values(hk, cuda, dtype, cols):
+    """Finite scores whose product with log2(e) is past fp32."""
+    import torch
+    dt = {"fp32": torch.float32, "bf16": torch.bfloat16, "fp16": torch.float16}[dtype]
+    x = _highest_rows(torch, cuda, 9100 + cols, cols, dt)
+    y = torch.empty_like(x)
+    hk.softmax_fwd(x, y)
+    torch.cuda.synchronize()
+    want = torch.softmax(x.double(), -1)
+    assert bool(torch.isnan(y[5]).all()) and bool(torch.isnan(want[5]).all())
+    helpers.assert_close(y[:5], want[:5].cpu().numpy(), dtype, "softmax y")
+    hk.softmax_fwd(x, x)
+    torch.cuda.synchronize()
+    assert torch.equal(x[:5], y[:5])
+
+
+@pytest.mark.parametrize("dtype", ["fp32", "bf16", "fp16"])
+@pytest.mark.parametrize("dim,inner", [(3, 9), (21, 8), (21, 67), (150, 40), (256, 33), (257, 9)])
+def test_softmax_of_highest_values_over_a_leading_dimension(hk, cuda, dtype, dim, inner):
+    """The rows above as columns, ordinary ones between them."""
+    import torch
+    dt = {"fp32": torch.float32, "bf16": torch.bfloat16, "fp16": torch.float16}[dtype]
+    x = torch.from_numpy(helpers.draw(9200 + dim, (2, dim, inner))).to(dt).to(cuda)
+    x[1, :, :6] = _highest_rows(torch, cuda, 9300 + dim, dim, dt).t()
+    y = torch.empty_like(x)
+    hk.softmax_fwd(x, y, 1)
+    torch.cuda.synchronize()
+    want = torch.softmax(x.double(), 1)
+    assert torch.equal(torch.isnan(y), torch.isnan(want))
+    helpers.assert_close(y.nan_to_num(), want.nan_to_num().cpu().numpy(), dtype, "softmax y")
+
+
+# a wavefront's and a workgroup's rows, 16-bit rows kept packed, streamed ones; whole vectors and ragged ones
+@pytest.mark.parametrize("dtype", ["fp32", "bf16", "fp16"])
+@pytest.mark.parametrize("cols", [40, 41, 1001, 4096, 40001, 50257, 70001])
+def test_cross_entropy_of_highest_values(hk, cuda, dtype, cols):
+    import torch
+    dt = {"fp32": torch.float32, "bf16": torch.bfloat16, "fp16": torch.float16}[dtype]
+    x = _highest_rows(torch, cuda, 8100 + cols, cols, dt)
+    lab = torch.tensor([cols // 2, cols - 1, 7, 1, cols - 2, 0], device=cuda)
+    g = torch.ones(6, dtype=dt, device=cuda)
+    loss, dx = torch.empty(6, dtype=dt, device=cuda), torch.empty_like(x)
+    stats = torch.empty(3, 6, device=cuda)
+    hk.sce_sparse_fwd(x, lab, loss, -100)
+    hk.sce_sparse_bwd(x, lab, g, dx, -100)
+    hk.vocab_parallel_ce_stats(x, lab, stats, 0, -100)
+    torch.cuda.synchronize()
+    p = torch.softmax(x.double(), -1)
+    want = torch.nn.functional.cross_entropy(x.double(), lab, reduction="none")
+    p[torch.arange(6, device=cuda), lab] -= 1
+    assert bool(torch.isnan(loss[5])) and bool(torch.isnan(dx[5]).all()) and bool(torch.isnan(stats[1, 5]))
+    helpers.assert_close(loss[:5], want[:5].cpu().numpy(), dtype, "loss")
+    helpers.assert_close(dx[:5], p[:5].cpu().numpy(), dtype, "dlogits")
+    top = x[:5].double().max(-1).values
+    assert torch.equal(stats[0, :5].double(), top)
+    helpers.assert_close(stats[1, :5], (x[:5].double() - top[:, None]).exp().sum(-1).cpu().numpy(), "fp32", "stats")
