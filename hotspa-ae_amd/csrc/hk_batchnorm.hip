@@ -344,7 +344,7 @@ void bn_fwd_channel_kernel(const T* x, T* y, BnRuns r, BnParams p) {
   }
   q = group_allreduce_tuple(q, red[1], 0, nwaves);
   const float rest = q.v[0] / p.count;   // mean = near + rest
-  const float m2 = fmaxf(q.v[1] - q.v[0] * rest, 0.f);
+  const float about = q.v[1] - q.v[0] * rest, m2 = about < 0.f ? 0.f : about;   // (a NaN stays one)
   const float invstd = bn_invstd<float, float>(m2 / p.count, p.eps);
   const float a = p.scale[c] * invstd, b = p.bias[c];
   if (threadIdx.x == 0)
@@ -468,7 +468,7 @@ void bn_fwd_partial_kernel(const T* __restrict__ x, BnRuns r, int splits, float*
     }
   }
   const float mean = cnt > 0.f ? K + s1 / cnt : 0.f;
-  const float m2 = cnt > 0.f ? fmaxf(s2 - s1 * (s1 / cnt), 0.f) : 0.f;
+  const float about = cnt > 0.f ? s2 - s1 * (s1 / cnt) : 0.f, m2 = about < 0.f ? 0.f : about;   // (a NaN stays one)
   // total count and mean first, then M2 about that mean
   const SumTuple<2> t = group_allreduce_tuple(SumTuple<2>{{cnt, mean * cnt}}, red[0], 0, 4);
   const float bmean = t.v[0] > 0.f ? t.v[1] / t.v[0] : 0.f, d = mean - bmean;

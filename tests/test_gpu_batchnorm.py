@@ -184,3 +184,34 @@ def test_planes_of_any_length(hk, cuda, dtype, shift):
         hk.batch_norm_bwd(g2, x, scale, g2, None, None, sm, si)
         torch.cuda.synchronize()
         assert torch.equal(g2, dx) and clean(gb, g2), shape
+
+
+# one workgroup per channel, several with a second launch, element by element
+@pytest.mark.parametrize("dtype", ["fp32", "bf16", "fp16"])
+@pytest.mark.parametrize("shape", [(3, 6, 121), (64, 6, 196), (64, 6, 3136), (3, 6, 3)])
+def test_channels_that_hold_a_nan_or_an_infinity(hk, cuda, dtype, shape):
+    """Their variance, saved and running, and every output are NaN and their mean is not finite, whatever the channel's
+    size; the channels beside them are as if alone."""
+    import torch
+    dt = {"fp32": torch.float32, "bf16": torch.bfloat16, "fp16": torch.float16}[dtype]
+    gen = torch.Generator(device="cuda").manual_seed(23)
+    clean = torch.randn(shape, generator=gen, device="cuda").to(dt)
+    dirty = clean.clone()
+    dirty[-1, 1, shape[2] // 2] = float("nan")
+    dirty[0, 2, 0] = float("inf")
+    dirty[-1, 3, -1] = -float("inf")
+    dirty[0, 4, 1], dirty[-1, 4, 2] = float("inf"), -float("inf")
+    C, hit = shape[1], torch.tensor([False, True, True, True, True, False], device="cuda")
+    scale, bias = torch.rand(C, generator=gen, device="cuda") + 0.5, torch.randn(C, generator=gen, device="cuda")
+    out = []
+    for x in (clean, dirty):
+        y = torch.empty_like(x)
+        rm, rv, sm, si = (torch.full((C,), v, device="cuda") for v in (0.0, 1.0, 7.0, 7.0))
+        hk.batch_norm_fwd(x, scale, bias, y, 0.1, 1e-5, rm, rv, sm, si)
+        torch.cuda.synchronize()
+        out.append((y.transpose(0, 1), rm, rv, sm, si))
+    for k, (a, b) in enumerate(zip(*out)):
+        assert torch.equal(a[~hit], b[~hit]), k
+    y, rm, rv, sm, si = (t[hit] for t in out[1])
+    assert bool(torch.isnan(y).all()) and bool(torch.isnan(rv).all()) and bool(torch.isnan(si).all())
+    assert not bool(torch.isfinite(rm).any()) and not bool(torch.isfinite(sm).any())
