@@ -289,14 +289,12 @@ void norm_fwd_any_kernel(NormFwdArgs a) {
       }
     }
   };
-  auto store_sum = [&] {
-    if constexpr (HAS_RES) {
-      if (a.x_out) {
-        T* xo = static_cast<T*>(a.x_out) + row * a.xout_pitch + outer_level_offset(a.xout_lv);
+  auto store_sum = [&] {   // (without a residual: a copy of the input)
+    if (a.x_out) {         // uniform
+      T* xo = static_cast<T*>(a.x_out) + row * a.xout_pitch + outer_level_offset(a.xout_lv);
 #pragma unroll
-        for (int i = 0; i < NV; ++i)
-          if (i * tpr + t < a.nvec) store_row_vec<T, true, true>(xo, i * tpr + t, v[i], a.cols);
-      }
+      for (int i = 0; i < NV; ++i)
+        if (i * tpr + t < a.nvec) store_row_vec<T, true, true>(xo, i * tpr + t, v[i], a.cols);
     }
   };
 
@@ -627,7 +625,9 @@ int norm_fwd_typed(NormFwdArgs a, hipStream_t s) {
   // rows of up to 32 vectors share a wavefront (LayerNorm of 32768 rows of 256 bf16: 13.1 us with one to each, 10.7
   // so); at 96 vectors norm_fwd_kernel is the faster one (20.1 against 25.5 us)
   const bool short_rows = a.nvec <= 32 && tune_get(TUNE_NORM_FWD_THREADS) == 0;
-  if (vec_ok && !short_rows &&
+  // norm_fwd_kernel writes the pre-norm sum beside the residual it reads, the others without one as well
+  const bool sum_alone = a.x_out != nullptr && !has_res;
+  if (vec_ok && !short_rows && !sum_alone &&
       pick_row_shape(a.nvec, tune_get(TUNE_NORM_FWD_THREADS), max_nv, wave_nv, many_rows, &threads, &nv)) {
     if (threads == 64) {
       dim3 grid(unsigned((a.n0 + 3) / 4), unsigned(a.n1), unsigned(a.n2)), block(256);

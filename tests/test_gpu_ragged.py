@@ -443,3 +443,32 @@ def test_cross_entropy_of_highest_values(hk, cuda, dtype, cols):
     top = x[:5].double().max(-1).values
     assert torch.equal(stats[0, :5].double(), top)
     helpers.assert_close(stats[1, :5], (x[:5].double() - top[:, None]).exp().sum(-1).cpu().numpy(), "fp32", "stats")
+
+
+@pytest.mark.parametrize("dtype", ["fp32", "bf16", "fp16"])
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("is_rms", [True, False])
+def test_pre_norm_sum_without_a_residual(hk, cuda, dtype, shift, is_rms):
+    """x_out is written whether a residual is added or not: then it is the input, in a buffer of its own and in place."""
+    import torch
+    eps = 1e-6
+    for cols in (3, 40, 41, 256, 520, 1021, 4096, 4099, 40000):
+        rows, pitch = 5, cols + (0 if shift == 0 else 5)
+        x0 = helpers.draw(150 + cols, (rows, cols), dtype=dtype)
+        gamma = helpers.draw(550 + cols, (cols,), "uniform", 0.5, 1.5, dtype)
+        place = lambda a, fill=None: _placed(cuda, a, dtype, shift, pitch, fill)
+        tg = helpers.to_torch(gamma, dtype, cuda)
+        _, tx0 = place(x0)
+        zb, tz = place(x0, 0.0)
+        xb, tx = place(x0, 0.0)
+        mu, rs = torch.empty(rows, device=cuda), torch.empty(rows, device=cuda)
+        hk.dropout_add_ln_fwd(tx0, None, tg, None, tz, tx, mu, rs, eps, is_rms)
+        torch.cuda.synchronize()
+        assert torch.equal(tx.contiguous(), tx0.contiguous()), cols
+        helpers.assert_close(tz.contiguous(), oracle.dropout_add_ln_fwd(x0, None, gamma, None, eps, is_rms)[0], dtype,
+                             "z %d" % cols)
+        assert _guards_untouched(zb, tz) and _guards_untouched(xb, tx), cols
+        z2, before = torch.empty_like(tz.contiguous()), tx0.clone()
+        hk.dropout_add_ln_fwd(tx0, None, tg, None, z2, tx0, mu, rs, eps, is_rms)
+        torch.cuda.synchronize()
+        assert torch.equal(tx0.contiguous(), before) and torch.equal(z2, tz.contiguous()), cols
