@@ -109,17 +109,16 @@ void copy_out(const NDArray& result, HtArray* out, const Stream& stream) {
 }
 
 // The caller's buffer as the place of an accelerator's loss, if the loss can be written there directly (the copy of one
-// value from a pool array took longer than the kernels of a 256 x 1000 loss): dense, of the loss's type and extent, apart
-// from the inputs.  Undefined otherwise: the loss goes through copy_out() and its checks.
+// value from a pool array took longer than the kernels of a 256 x 1000 loss): dense, of the loss's own shape and type,
+// apart from the inputs.  Undefined otherwise: the loss goes through copy_out() and its checks.
 NDArray loss_buffer(const NDArray& preds, const NDArray& labels, const HtArray* out, ReductionType reduction,
                     const Stream& stream) {
   if (!stream.device().is_cuda() || out == nullptr || !preds.is_defined() || !labels.is_defined() || preds->ndim() == 0)
     return NDArray();
   NDArray dst = wrap(out);
-  size_t rows = 1;
-  for (size_t i = 0; i + 1 < preds->ndim(); ++i) rows *= size_t(preds->shape(i));
-  const size_t numel = reduction == kNONE ? rows : 1;
-  if (numel == 0 || dst->numel() != numel || dst->ndim() != 1 || !dst->is_contiguous() || dst->dtype() != preds->dtype() ||
+  HTShape shape = {1};
+  if (reduction == kNONE && preds->ndim() > 1) shape = HTShape(preds->shape().begin(), preds->shape().end() - 1);
+  if (dst->numel() == 0 || dst->shape() != shape || !dst->is_contiguous() || dst->dtype() != preds->dtype() ||
       dst->device() != preds->device())
     return NDArray();
   auto first = [](const NDArray& a) { return reinterpret_cast<uintptr_t>(a->storage()->data_ptr().ptr); };

@@ -1146,3 +1146,29 @@ def test_ndarray_sceloss_buffers(ops, cuda, reduction):
     for bad in (torch.empty(n + 1, device=cuda), torch.empty(n, device=cuda, dtype=torch.bfloat16)):
         with pytest.raises(Exception):
             ops.ndarray_sceloss(tx, tl, bad, reduction, ignored_index=-100)
+
+
+@pytest.mark.parametrize("sparse", [True, False])
+@pytest.mark.parametrize("reduction", ["none", "mean", "sum"])
+def test_ndarray_sceloss_of_rank_3(ops, cuda, sparse, reduction):
+    """Predictions of three dimensions: a loss buffer of the loss's shape, a flat one and one with a dimension more get the
+    same values."""
+    import torch
+    a, b, cols = 3, 4, 40
+    x = helpers.draw(78, (a, b, cols), dtype="fp32")
+    lab = (np.arange(a * b, dtype=np.int64) * 3).reshape(a, b)
+    dense = np.abs(helpers.draw(79, (a, b, cols), dtype="fp32"))
+    tx = helpers.to_torch(x, "fp32", cuda)
+    tl = torch.from_numpy(lab).to(cuda) if sparse else helpers.to_torch(dense, "fp32", cuda)
+    flat = x.reshape(-1, cols)
+    want = oracle.sce_sparse_fwd(flat, lab.ravel(), -100) if sparse else oracle.sce_dense_fwd(flat, dense.reshape(-1, cols))
+    want = want if reduction == "none" else np.array([want.mean() if reduction == "mean" else want.sum()])
+    shapes = [(a, b), (a * b,), (1, a, b)] if reduction == "none" else [(1,), (1, 1)]
+    outs = [torch.full(s, 7.0, device=cuda) for s in shapes]
+    _sync_in()
+    for out in outs:
+        if sparse:
+            ops.ndarray_sceloss(tx, tl, out, reduction, ignored_index=-100)
+        else:
+            ops.ndarray_sceloss(tx, tl, out, reduction)
+        helpers.assert_close(out.view(-1), want, "fp32", "loss %s" % (tuple(out.shape),))
