@@ -288,7 +288,7 @@ struct BnVecWalk {
   __device__ __forceinline__ bool live() const { return index < r.total; }
   // offset of the loaded vector (the channel's first one past the end), and how many of its elements belong to others
   __device__ __forceinline__ int64_t off() const { return live() ? plane + vec_column<T, true>(v, r.HW) : 0; }
-  __device__ __forceinline__ int skip() const { return live() ? (v + 1) * VEC - r.HW : VEC; }
+  __device__ __forceinline__ int skip() const { return live() ? VEC - (r.HW - v * VEC) : VEC; }
   __device__ __forceinline__ void next() {
     index += stride;
     v += step_v;

@@ -149,3 +149,70 @@ def test_batch_norm_past_2_31_elements(hk, cuda):
         want = (x[img, ch].double() - mean[ch]) / torch.sqrt(var[ch] + 1e-5) * scale[ch].double() + bias[ch].double()
         got = y[img, ch].double()
         assert ((got - want).abs() <= 1e-2 * (want.abs() + 1.0)).all()
+
+
+# the last, partial vector of such a plane ends past element 2^31
+LONGEST_PLANE = (1 << 31) - 3
+
+
+def _guarded(torch, n, cuda):
+    buf = torch.full((n + 64,), 7.0, dtype=torch.bfloat16, device=cuda)
+    return buf, buf[32:32 + n]
+
+
+def test_softmax_over_planes_that_end_below_2_31_elements(hk, cuda):
+    import torch
+    n = LONGEST_PLANE
+    x = _randn(torch, (2 * n,), 11, 2.0).view(1, 2, n)
+    dy = _randn(torch, (2 * n,), 12).view(1, 2, n)
+    yb, y = _guarded(torch, 2 * n, cuda)
+    hk.softmax_fwd(x, y.view(1, 2, n), 1)
+    db, dx = _guarded(torch, 2 * n, cuda)
+    hk.softmax_bwd(y.view(1, 2, n), dy, dx.view(1, 2, n), 1)
+    torch.cuda.synchronize()
+    for buf in (yb, db):
+        assert bool((buf[:32] == 7.0).all()) and bool((buf[-32:] == 7.0).all())
+    y, dx = y.view(2, n), dx.view(2, n)
+    for lo in (0, n // 2, n - 1000):
+        at = slice(lo, lo + 1000)
+        helpers.assert_close(y[:, at].contiguous(), torch.softmax(x[0, :, at].double(), 0).cpu().numpy(), "bf16", "softmax")
+        yd = y[:, at].double()
+        want = yd * (dy[0, :, at].double() - (yd * dy[0, :, at].double()).sum(0))
+        helpers.assert_close(dx[:, at].contiguous(), want.cpu().numpy(), "bf16", "softmax gradient")
+
+
+def test_batch_norm_of_a_plane_that_ends_below_2_31_elements(hk, cuda):
+    import torch
+    n = LONGEST_PLANE
+    x = _randn(torch, (n,), 13, 2.0).add_(3.0)
+    total = squares = 0.0
+    for part in x.split(1 << 28):
+        d = part.double()
+        total += float(d.sum())
+        squares += float(((d - 3.0) ** 2).sum())
+    mean = total / n
+    var = squares / n - (mean - 3.0) ** 2
+    scale, bias = torch.full((1,), 1.5, device=cuda), torch.full((1,), 0.25, device=cuda)
+    sm, si = torch.empty(1, device=cuda), torch.empty(1, device=cuda)
+    yb, y = _guarded(torch, n, cuda)
+    hk.batch_norm_fwd(x.view(1, 1, n), scale, bias, y.view(1, 1, n), 0.1, 1e-5, None, None, sm, si)
+    db, dx = _guarded(torch, n, cuda)
+    dy = _randn(torch, (n,), 14)
+    hk.batch_norm_bwd(dy.view(1, 1, n), x.view(1, 1, n), scale, dx.view(1, 1, n), None, None, sm, si)
+    torch.cuda.synchronize()
+    for buf in (yb, db):
+        assert bool((buf[:32] == 7.0).all()) and bool((buf[-32:] == 7.0).all())
+    inv = (var + 1e-5) ** -0.5
+    helpers.assert_close(sm, np.array([mean]), "fp32", "save_mean")
+    helpers.assert_close(si, np.array([inv]), "fp32", "save_invstd")
+    mean_dy = mean_dyx = 0.0
+    for lo in range(0, n, 1 << 28):
+        d, xhat = dy[lo:lo + (1 << 28)].double(), (x[lo:lo + (1 << 28)].double() - mean) * inv
+        mean_dy += float(d.sum()) / n
+        mean_dyx += float((d * xhat).sum()) / n
+    for lo in (0, n // 2, n - 1000):
+        at = slice(lo, lo + 1000)
+        xhat = (x[at].double() - mean) * inv
+        helpers.assert_close(y[at], (xhat * 1.5 + 0.25).cpu().numpy(), "bf16", "batch norm")
+        want = 1.5 * inv * (dy[at].double() - mean_dy - xhat * mean_dyx)
+        helpers.assert_close(dx[at], want.cpu().numpy(), "bf16", "batch norm gradient")
