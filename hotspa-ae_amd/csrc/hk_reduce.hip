@@ -671,9 +671,11 @@ static InnerShape shape_inner(const ReducePlan& p, bool split) {
   const int64_t groups = tpr <= 64 ? (p.rows * tpr + 255) / 256 : p.rows;
   const int64_t want = p.nruns > 1 ? std::max<int64_t>(cus, want_blocks * 256 / std::max(tpr, 256)) : want_blocks;
   const int64_t rounds = p.nruns > 1 ? 8 : 16;   // vectors per thread below which a split is not worth its fold
+  // counted in whole vectors: a partial one more must not make a row need scratch (see scratch_required)
+  const int64_t whole = p.nruns * (p.cols / VEC);
   int64_t nsplit = 1;
-  if (split && groups < want && nvec > int64_t(tpr) * rounds * 2) {
-    nsplit = std::min<int64_t>((want + groups - 1) / groups, nvec / (int64_t(tpr) * rounds));
+  if (split && groups < want && whole > int64_t(tpr) * rounds * 2) {
+    nsplit = std::min<int64_t>((want + groups - 1) / groups, whole / (int64_t(tpr) * rounds));
     nsplit = std::max<int64_t>(1, std::min<int64_t>(nsplit, 1024));
   }
   s.chunk = std::max<int64_t>(1, (nvec + nsplit - 1) / nsplit);

@@ -472,3 +472,18 @@ def test_pre_norm_sum_without_a_residual(hk, cuda, dtype, shift, is_rms):
         hk.dropout_add_ln_fwd(tx0, None, tg, None, z2, tx0, mu, rs, eps, is_rms)
         torch.cuda.synchronize()
         assert torch.equal(tx0.contiguous(), before) and torch.equal(z2, tz.contiguous()), cols
+
+
+@pytest.mark.parametrize("dtype", ["fp32", "bf16", "fp16"])
+def test_rows_that_need_no_scratch(hk, cuda, dtype):
+    """A row of the most whole vectors that one workgroup takes, and a partial one more, on the 16-byte grid."""
+    import torch
+    dt = {"fp32": torch.float32, "bf16": torch.bfloat16, "fp16": torch.float16}[dtype]
+    vec = 16 // ES[dtype]
+    for cols in [32768 * vec + k for k in range(vec)]:
+        a = np.random.default_rng(cols).integers(-3, 4, cols)
+        x, out = torch.from_numpy(a).to(dt).to(cuda), torch.empty(1, dtype=dt, device=cuda)
+        assert hk.reduce_workspace_bytes(hk.dtype_code(x), [cols], [1], [0]) == 0, cols
+        hk.reduce(x, out, [0], "sum", workspace=torch.empty(1, device=cuda))
+        torch.cuda.synchronize()
+        assert float(out) == float(oracle.round_to(np.asarray([a.sum()], np.float32), dtype)[0]), cols
