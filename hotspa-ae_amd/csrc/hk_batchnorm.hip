@@ -8,7 +8,7 @@
 //    channel reads it once, agrees on its statistics and writes the result;
 //  - longer ones: partial statistics from several workgroups per channel, then a pass whose workgroups merge their
 //    channel's partials themselves (the input is read twice, the second time from the memory-side cache where it fits);
-//  - fp64, planes shorter than a 16-byte vector and arrays past 2^31 elements: element by element, three launches.
+//  - fp64 and planes shorter than a 16-byte vector: element by element, three launches.
 // The first two take planes of any length and alignment: the partial last vector of a run is read as the run's last whole
 // one, the elements it shares with the vector before it are left out of the sums.
 #include "hk_common.h"
@@ -254,10 +254,13 @@ void bn_bwd_apply_kernel(const T* dy, const T* x, T* dx, const CT* __restrict__ 
 // ---------------------------------------------------------------------------
 // planes as 16-byte vectors
 // ---------------------------------------------------------------------------
+// IT: what counts a channel's vectors and a plane's elements, 32 bits unless the array is past 2^31 elements
+template <typename IT>
 struct BnRuns {
-  int C, HW;
-  int run_vecs;        // vectors per run, the partial one included
-  int total;           // vectors per channel
+  int C;
+  IT HW;
+  IT run_vecs;         // vectors per run, the partial one included
+  IT total;            // vectors per channel
   int64_t image;       // C * HW
 };
 struct BnParams {
@@ -270,25 +273,29 @@ struct BnParams {
 };
 
 // A thread's walk over the vectors v0, v0 + stride, ... of a channel
-template <typename T>
+template <typename T, typename IT>
 struct BnVecWalk {
   static constexpr int VEC = VecIO<T>::N;
-  const BnRuns& r;
-  int index, v;          // vector in the channel, and in its run
+  using UT = typename std::make_unsigned<IT>::type;
+  const BnRuns<IT>& r;
+  IT index, v;           // vector in the channel, and in its run
   int64_t plane;         // offset of the run from the channel's first
-  int stride, step_v;
+  IT stride, step_v;
   int64_t step_plane;
-  __device__ __forceinline__ BnVecWalk(const BnRuns& runs, int v0, int by) : r(runs), index(v0), stride(by) {
-    const uint32_t n = uint32_t(v0) / uint32_t(r.run_vecs), q = uint32_t(by) / uint32_t(r.run_vecs);
-    v = v0 - int(n) * r.run_vecs;
+  __device__ __forceinline__ BnVecWalk(const BnRuns<IT>& runs, IT v0, int by) : r(runs), index(v0), stride(by) {
+    const UT n = UT(v0) / UT(r.run_vecs), q = UT(by) / UT(r.run_vecs);
+    v = v0 - IT(n) * r.run_vecs;
     plane = int64_t(n) * r.image;
-    step_v = by - int(q) * r.run_vecs;
+    step_v = by - IT(q) * r.run_vecs;
     step_plane = int64_t(q) * r.image;
   }
   __device__ __forceinline__ bool live() const { return index < r.total; }
   // offset of the loaded vector (the channel's first one past the end), and how many of its elements belong to others
   __device__ __forceinline__ int64_t off() const { return live() ? plane + vec_column<T, true>(v, r.HW) : 0; }
-  __device__ __forceinline__ int skip() const { return live() ? VEC - (r.HW - v * VEC) : VEC; }
+  __device__ __forceinline__ int skip() const {
+    const IT left = r.HW - v * VEC;
+    return !live() ? VEC : left >= VEC ? 0 : VEC - int(left);
+  }
   __device__ __forceinline__ void next() {
     index += stride;
     v += step_v;
@@ -304,19 +311,20 @@ struct BnVecWalk {
 // Three launches and two reads of the input before (bf16, forward / backward): 64 x 256 x 196 24.4 / 23.6 us -> 11.2 /
 // 10.3, of which 10 are the call's own; 2 x 512 x 3969 27.9 / 27.0 -> 10.5 / 10.1.  Short odd planes are bound by cache
 // lines that neighbouring channels share (256 x 1024 x 49: 63 / 68 -> 34 / 44 us, 1.5 TB/s).
-template <typename T, int NV>
+template <typename T, int NV, typename IT>
 __global__ __launch_bounds__(1024)
-void bn_fwd_channel_kernel(const T* x, T* y, BnRuns r, BnParams p) {
+void bn_fwd_channel_kernel(const T* x, T* y, BnRuns<IT> r, BnParams p) {
   constexpr int VEC = VecIO<T>::N;
   __shared__ float red[2][kMaxWaves * 2];
   const int c = blockIdx.x, nwaves = int(blockDim.x >> 6);
   const int64_t base = int64_t(c) * r.HW;
   u32x4 raw[NV];
-  int off[NV], skip[NV];
-  BnVecWalk<T> w(r, int(threadIdx.x), int(blockDim.x));
+  IT off[NV];
+  int skip[NV];
+  BnVecWalk<T, IT> w(r, IT(threadIdx.x), int(blockDim.x));
 #pragma unroll
   for (int i = 0; i < NV; ++i, w.next()) {
-    off[i] = int(w.off());
+    off[i] = IT(w.off());
     skip[i] = w.skip();
     raw[i] = ld16_any<T>(x + base + off[i]);
   }
@@ -374,19 +382,20 @@ struct BnBwdCoef {
   __device__ __forceinline__ float operator()(float g, float x) const { return k0 * g + (k1 * (x - mean) + k2); }
 };
 
-template <typename T, int NV>
+template <typename T, int NV, typename IT>
 __global__ __launch_bounds__(1024)
-void bn_bwd_channel_kernel(const T* dy, const T* x, T* dx, BnRuns r, BnParams p) {
+void bn_bwd_channel_kernel(const T* dy, const T* x, T* dx, BnRuns<IT> r, BnParams p) {
   constexpr int VEC = VecIO<T>::N;
   __shared__ float red[kMaxWaves * 2];
   const int c = blockIdx.x, nwaves = int(blockDim.x >> 6);
   const int64_t base = int64_t(c) * r.HW;
   u32x4 rg[NV], rx[NV];
-  int off[NV], skip[NV];
-  BnVecWalk<T> w(r, int(threadIdx.x), int(blockDim.x));
+  IT off[NV];
+  int skip[NV];
+  BnVecWalk<T, IT> w(r, IT(threadIdx.x), int(blockDim.x));
 #pragma unroll
   for (int i = 0; i < NV; ++i, w.next()) {
-    off[i] = int(w.off());
+    off[i] = IT(w.off());
     skip[i] = w.skip();
     rg[i] = ld16_any<T>(dy + base + off[i]);
     rx[i] = ld16_any<T>(x + base + off[i]);
@@ -430,14 +439,14 @@ void bn_bwd_channel_kernel(const T* dy, const T* x, T* dx, BnRuns r, BnParams p)
 constexpr int kBnVecs = 4;
 
 // (count, mean, M2) of the slice blockIdx.y of channel blockIdx.x -> part[(c * splits + split) * 3 ..]
-template <typename T>
+template <typename T, typename IT>
 __global__ __launch_bounds__(256)
-void bn_fwd_partial_kernel(const T* __restrict__ x, BnRuns r, int splits, float* __restrict__ part) {
+void bn_fwd_partial_kernel(const T* __restrict__ x, BnRuns<IT> r, int splits, float* __restrict__ part) {
   constexpr int VEC = VecIO<T>::N, U = kBnVecs;
   __shared__ float red[2][kMaxWaves * 2];
   const int64_t c = blockIdx.x;
   const T* base = x + c * r.HW;
-  BnVecWalk<T> w(r, int(blockIdx.y) * 256 + int(threadIdx.x), splits * 256);
+  BnVecWalk<T, IT> w(r, IT(blockIdx.y) * 256 + IT(threadIdx.x), splits * 256);
   // sums about a pivot K, the mean of the thread's first vector: a large common offset never enters a sum
   float K = 0.f, s1 = 0.f, s2 = 0.f, cnt = 0.f;
   while (w.live()) {
@@ -481,16 +490,16 @@ void bn_fwd_partial_kernel(const T* __restrict__ x, BnRuns r, int splits, float*
 
 // Workgroup (chunk, channel) = divmod(blockIdx.x, C): kBnVecs vectors per thread, loaded before the channel's partials
 // are merged; every wavefront merges them for itself.  The first chunk's workgroup writes the statistics.
-template <typename T>
+template <typename T, typename IT>
 __global__ __launch_bounds__(256)
-void bn_fwd_merge_apply_kernel(const T* x, T* y, BnRuns r, BnParams p, int splits, const float* __restrict__ part) {
+void bn_fwd_merge_apply_kernel(const T* x, T* y, BnRuns<IT> r, BnParams p, int splits, const float* __restrict__ part) {
   constexpr int VEC = VecIO<T>::N, U = kBnVecs;
   const int chunk = int(blockIdx.x / uint32_t(r.C)), c = int(blockIdx.x - uint32_t(chunk) * uint32_t(r.C));
   const int64_t base = int64_t(c) * r.HW;
   u32x4 raw[U];
-  int v[U];
+  IT v[U];
   int64_t plane[U];
-  BnVecWalk<T> w(r, chunk * (256 * U) + int(threadIdx.x), 256);
+  BnVecWalk<T, IT> w(r, IT(chunk) * (256 * U) + IT(threadIdx.x), 256);
 #pragma unroll
   for (int i = 0; i < U; ++i, w.next()) {
     raw[i] = ld16_any<T>(x + base + w.off());
@@ -525,9 +534,9 @@ void bn_fwd_merge_apply_kernel(const T* x, T* y, BnRuns r, BnParams p, int split
 }
 
 // sums of dy and dy * xhat of a slice -> part[(c * splits + split) * 2 ..]
-template <typename T>
+template <typename T, typename IT>
 __global__ __launch_bounds__(256)
-void bn_bwd_partial_kernel(const T* __restrict__ dy, const T* __restrict__ x, BnRuns r, BnParams p, int splits,
+void bn_bwd_partial_kernel(const T* __restrict__ dy, const T* __restrict__ x, BnRuns<IT> r, BnParams p, int splits,
                            float* __restrict__ part) {
   constexpr int VEC = VecIO<T>::N, U = kBnVecs / 2;
   __shared__ float red[kMaxWaves * 2];
@@ -535,7 +544,7 @@ void bn_bwd_partial_kernel(const T* __restrict__ dy, const T* __restrict__ x, Bn
   const int64_t base = c * r.HW;
   const float mean = p.mean[c], invstd = p.invstd[c];
   SumTuple<2> s = SumTuple<2>::identity();
-  BnVecWalk<T> w(r, int(blockIdx.y) * 256 + int(threadIdx.x), splits * 256);
+  BnVecWalk<T, IT> w(r, IT(blockIdx.y) * 256 + IT(threadIdx.x), splits * 256);
   while (w.live()) {
     u32x4 rg[U], rx[U];
     int skip[U];
@@ -566,17 +575,17 @@ void bn_bwd_partial_kernel(const T* __restrict__ dy, const T* __restrict__ x, Bn
   }
 }
 
-template <typename T>
+template <typename T, typename IT>
 __global__ __launch_bounds__(256)
-void bn_bwd_merge_apply_kernel(const T* dy, const T* x, T* dx, BnRuns r, BnParams p, int splits,
+void bn_bwd_merge_apply_kernel(const T* dy, const T* x, T* dx, BnRuns<IT> r, BnParams p, int splits,
                                const float* __restrict__ part) {
   constexpr int VEC = VecIO<T>::N, U = kBnVecs / 2;
   const int chunk = int(blockIdx.x / uint32_t(r.C)), c = int(blockIdx.x - uint32_t(chunk) * uint32_t(r.C));
   const int64_t base = int64_t(c) * r.HW;
   u32x4 rg[U], rx[U];
-  int v[U];
+  IT v[U];
   int64_t plane[U];
-  BnVecWalk<T> w(r, chunk * (256 * U) + int(threadIdx.x), 256);
+  BnVecWalk<T, IT> w(r, IT(chunk) * (256 * U) + IT(threadIdx.x), 256);
 #pragma unroll
   for (int i = 0; i < U; ++i, w.next()) {
     const int64_t off = base + w.off();
@@ -631,22 +640,24 @@ static size_t bn_ws_bytes(int64_t N, int64_t C, int64_t HW, size_t ct_size) {
 }
 
 // How the vector kernels take an [N, C, HW] array; form 0: they don't
+template <typename IT>
 struct BnPlan {
   int form;            // 1: a workgroup per channel; 2: partials and merge
-  BnRuns runs;
+  BnRuns<IT> runs;
   int threads, nv;     // form 1
   int splits;          // form 2
 };
-template <typename T>
-static BnPlan bn_plan(int64_t N, int64_t C, int64_t HW, int max_splits, int max_nv) {
+template <typename T, typename IT>
+static BnPlan<IT> bn_plan(int64_t N, int64_t C, int64_t HW, int max_splits, int max_nv) {
   constexpr int VEC = VecIO<T>::N;
-  BnPlan b{};
-  if (HW < VEC || N * C * HW > 0x7fffffffLL) return b;
-  b.runs.C = int(C); b.runs.HW = int(HW); b.runs.image = C * HW;
-  b.runs.run_vecs = int((HW + VEC - 1) / VEC);
-  const int64_t total = N * b.runs.run_vecs;
-  if (total > 0x3fffffff) return b;
-  b.runs.total = int(total);
+  BnPlan<IT> b{};
+  const int64_t run_vecs = (HW + VEC - 1) / VEC, total = N * run_vecs;
+  // the walk's count of vectors and its steps stay below IT's most, the workgroups of either form below the grid's
+  if (HW < VEC || (sizeof(IT) == 4 && (N * C * HW > 0x7fffffffLL || total > 0x3fffffff))) return b;
+  if (C > 0x7fffffffLL || (total / (128 * kBnVecs) + 1) * C > 0x7fffffffLL) return b;
+  b.runs.C = int(C); b.runs.HW = IT(HW); b.runs.image = C * HW;
+  b.runs.run_vecs = IT(run_vecs);
+  b.runs.total = IT(total);
   for (int nv = 1; nv <= max_nv; nv <<= 1) {
     // one vector a thread while there are fewer channels than two workgroups per compute unit, else two at least
     if (total > int64_t(nv) * 1024 || (nv == 1 && total > 64 && C > 2 * device_cu_count())) continue;
@@ -660,8 +671,67 @@ static BnPlan bn_plan(int64_t N, int64_t C, int64_t HW, int max_splits, int max_
   b.splits = int(std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(want, most), std::min(max_splits, 256))));
   return b;
 }
-static inline unsigned bn_chunks(const BnRuns& r, int per_thread) {
+template <typename IT>
+static inline unsigned bn_chunks(const BnRuns<IT>& r, int per_thread) {
   return unsigned((int64_t(r.total) + 256 * per_thread - 1) / (256 * per_thread)) * unsigned(r.C);
+}
+
+// the vector kernels' launches; *handled: they take the array
+template <typename T, typename IT>
+static int bn_fwd_vec(const T* x, T* y, const BnParams& p, int64_t N, int64_t C, int64_t HW, int max_splits, float* part,
+                      hipStream_t st, bool* handled) {
+  const BnPlan<IT> b = bn_plan<T, IT>(N, C, HW, max_splits, 8);
+  *handled = b.form != 0;
+  if (b.form == 1) {
+    const dim3 grid{unsigned(C)}, block{unsigned(b.threads)};
+    profile_before(st);
+    switch (b.nv) {
+      case 1: HK_LAUNCH((bn_fwd_channel_kernel<T, 1, IT>), grid, block, 0, st, x, y, b.runs, p); break;
+      case 2: HK_LAUNCH((bn_fwd_channel_kernel<T, 2, IT>), grid, block, 0, st, x, y, b.runs, p); break;
+      case 4: HK_LAUNCH((bn_fwd_channel_kernel<T, 4, IT>), grid, block, 0, st, x, y, b.runs, p); break;
+      default: HK_LAUNCH((bn_fwd_channel_kernel<T, 8, IT>), grid, block, 0, st, x, y, b.runs, p);
+    }
+    profile_after(st);
+    return launch_check("bn_fwd_channel_kernel");
+  }
+  if (b.form == 2) {
+    HK_LAUNCH((bn_fwd_partial_kernel<T, IT>), dim3(unsigned(C), unsigned(b.splits)), dim3(256), 0, st, x, b.runs, b.splits, part);
+    const int rc = launch_check("bn_fwd_partial_kernel");
+    if (rc != HK_OK) return rc;
+    profile_before(st);
+    HK_LAUNCH((bn_fwd_merge_apply_kernel<T, IT>), dim3(bn_chunks(b.runs, kBnVecs)), dim3(256), 0, st, x, y, b.runs, p, b.splits, part);
+    profile_after(st);
+    return launch_check("bn_fwd_merge_apply_kernel");
+  }
+  return HK_OK;
+}
+
+template <typename T, typename IT>
+static int bn_bwd_vec(const T* dy, const T* x, T* dx, const BnParams& p, int64_t N, int64_t C, int64_t HW, int max_splits,
+                      float* part, hipStream_t st, bool* handled) {
+  const BnPlan<IT> b = bn_plan<T, IT>(N, C, HW, max_splits, 4);
+  *handled = b.form != 0;
+  if (b.form == 1) {
+    const dim3 grid{unsigned(C)}, block{unsigned(b.threads)};
+    profile_before(st);
+    switch (b.nv) {
+      case 1: HK_LAUNCH((bn_bwd_channel_kernel<T, 1, IT>), grid, block, 0, st, dy, x, dx, b.runs, p); break;
+      case 2: HK_LAUNCH((bn_bwd_channel_kernel<T, 2, IT>), grid, block, 0, st, dy, x, dx, b.runs, p); break;
+      default: HK_LAUNCH((bn_bwd_channel_kernel<T, 4, IT>), grid, block, 0, st, dy, x, dx, b.runs, p);
+    }
+    profile_after(st);
+    return launch_check("bn_bwd_channel_kernel");
+  }
+  if (b.form == 2) {
+    HK_LAUNCH((bn_bwd_partial_kernel<T, IT>), dim3(unsigned(C), unsigned(b.splits)), dim3(256), 0, st, dy, x, b.runs, p, b.splits, part);
+    const int rc = launch_check("bn_bwd_partial_kernel");
+    if (rc != HK_OK) return rc;
+    profile_before(st);
+    HK_LAUNCH((bn_bwd_merge_apply_kernel<T, IT>), dim3(bn_chunks(b.runs, kBnVecs / 2)), dim3(256), 0, st, dy, x, dx, b.runs, p, b.splits, part);
+    profile_after(st);
+    return launch_check("bn_bwd_merge_apply_kernel");
+  }
+  return HK_OK;
 }
 
 template <typename T, typename PT>
@@ -674,33 +744,15 @@ static int bn_fwd_typed(const void* x, const void* scale, const void* bias, void
   T* yp = static_cast<T*>(y);
   const BnShape s = bn_shape(N, C, HW);
   if constexpr (!std::is_same<T, double>::value) {
-    const BnPlan b = bn_plan<T>(N, C, HW, s.splits, 8);
     BnParams p{};
     p.scale = static_cast<const float*>(scale); p.bias = static_cast<const float*>(bias);
     p.running_mean = static_cast<float*>(running_mean); p.running_var = static_cast<float*>(running_var);
     p.save_mean = static_cast<float*>(save_mean); p.save_invstd = static_cast<float*>(save_invstd);
     p.momentum = momentum; p.eps = eps; p.count = float(N * HW);
-    if (b.form == 1) {
-      const dim3 grid{unsigned(C)}, block{unsigned(b.threads)};
-      profile_before(st);
-      switch (b.nv) {
-        case 1: HK_LAUNCH((bn_fwd_channel_kernel<T, 1>), grid, block, 0, st, xp, yp, b.runs, p); break;
-        case 2: HK_LAUNCH((bn_fwd_channel_kernel<T, 2>), grid, block, 0, st, xp, yp, b.runs, p); break;
-        case 4: HK_LAUNCH((bn_fwd_channel_kernel<T, 4>), grid, block, 0, st, xp, yp, b.runs, p); break;
-        default: HK_LAUNCH((bn_fwd_channel_kernel<T, 8>), grid, block, 0, st, xp, yp, b.runs, p);
-      }
-      profile_after(st);
-      return launch_check("bn_fwd_channel_kernel");
-    }
-    if (b.form == 2) {
-      HK_LAUNCH((bn_fwd_partial_kernel<T>), dim3(unsigned(C), unsigned(b.splits)), dim3(256), 0, st, xp, b.runs, b.splits, part);
-      const int rc = launch_check("bn_fwd_partial_kernel");
-      if (rc != HK_OK) return rc;
-      profile_before(st);
-      HK_LAUNCH((bn_fwd_merge_apply_kernel<T>), dim3(bn_chunks(b.runs, kBnVecs)), dim3(256), 0, st, xp, yp, b.runs, p, b.splits, part);
-      profile_after(st);
-      return launch_check("bn_fwd_merge_apply_kernel");
-    }
+    bool handled = false;
+    int rc = bn_fwd_vec<T, int>(xp, yp, p, N, C, HW, s.splits, part, st, &handled);
+    if (!handled) rc = bn_fwd_vec<T, int64_t>(xp, yp, p, N, C, HW, s.splits, part, st, &handled);
+    if (handled) return rc;
   }
   CT* coef = part + size_t(C) * size_t(s.splits) * 3;
   const int64_t total = N * C * HW;
@@ -734,32 +786,15 @@ static int bn_bwd_typed(const void* dy, const void* x, const void* scale, void* 
   T* op = static_cast<T*>(dx);
   const BnShape s = bn_shape(N, C, HW);
   if constexpr (!std::is_same<T, double>::value) {
-    const BnPlan b = bn_plan<T>(N, C, HW, s.splits, 4);
     BnParams p{};
     p.scale = static_cast<const float*>(scale);
     p.mean = static_cast<const float*>(save_mean); p.invstd = static_cast<const float*>(save_invstd);
     p.dscale = static_cast<float*>(dscale); p.dbias = static_cast<float*>(dbias);
     p.count = float(N * HW);
-    if (b.form == 1) {
-      const dim3 grid{unsigned(C)}, block{unsigned(b.threads)};
-      profile_before(st);
-      switch (b.nv) {
-        case 1: HK_LAUNCH((bn_bwd_channel_kernel<T, 1>), grid, block, 0, st, gp, xp, op, b.runs, p); break;
-        case 2: HK_LAUNCH((bn_bwd_channel_kernel<T, 2>), grid, block, 0, st, gp, xp, op, b.runs, p); break;
-        default: HK_LAUNCH((bn_bwd_channel_kernel<T, 4>), grid, block, 0, st, gp, xp, op, b.runs, p);
-      }
-      profile_after(st);
-      return launch_check("bn_bwd_channel_kernel");
-    }
-    if (b.form == 2) {
-      HK_LAUNCH((bn_bwd_partial_kernel<T>), dim3(unsigned(C), unsigned(b.splits)), dim3(256), 0, st, gp, xp, b.runs, p, b.splits, part);
-      const int rc = launch_check("bn_bwd_partial_kernel");
-      if (rc != HK_OK) return rc;
-      profile_before(st);
-      HK_LAUNCH((bn_bwd_merge_apply_kernel<T>), dim3(bn_chunks(b.runs, kBnVecs / 2)), dim3(256), 0, st, gp, xp, op, b.runs, p, b.splits, part);
-      profile_after(st);
-      return launch_check("bn_bwd_merge_apply_kernel");
-    }
+    bool handled = false;
+    int rc = bn_bwd_vec<T, int>(gp, xp, op, p, N, C, HW, s.splits, part, st, &handled);
+    if (!handled) rc = bn_bwd_vec<T, int64_t>(gp, xp, op, p, N, C, HW, s.splits, part, st, &handled);
+    if (handled) return rc;
   }
   CT* coef = part + size_t(C) * size_t(s.splits) * 3;
   const int64_t total = N * C * HW;

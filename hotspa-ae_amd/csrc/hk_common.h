@@ -226,16 +226,16 @@ __device__ __forceinline__ void st16_any(T* p, const u32x4& v) {
   __builtin_nontemporal_store(v, reinterpret_cast<typename AnyBoundary<T>::vec*>(p));
 }
 // first column that vector v loads (compared as what is left of the row: v * N + N may be past 2^31)
-template <typename T, bool RAGGED>
-__device__ __forceinline__ int vec_column(int v, int cols) {
+template <typename T, bool RAGGED, typename I>
+__device__ __forceinline__ I vec_column(I v, I cols) {
   constexpr int N = VecIO<T>::N;
   if constexpr (!RAGGED) return v * N;
   return cols - v * N >= N ? v * N : cols - N;
 }
 // Stores vector v of a row.  SAME: an element that two vectors hold was computed to the same bits in both, so the
 // partial vector is stored whole over its neighbour's end; otherwise its own elements go out one by one.
-template <typename T, bool RAGGED, bool SAME>
-__device__ __forceinline__ void store_row_vec(T* row, int v, const float* f, int cols) {
+template <typename T, bool RAGGED, bool SAME, typename I>
+__device__ __forceinline__ void store_row_vec(T* row, I v, const float* f, I cols) {
   constexpr int N = VecIO<T>::N;
   if constexpr (!RAGGED) {
     __builtin_nontemporal_store(VecIO<T>::pack(f), reinterpret_cast<u32x4*>(row + v * N));
@@ -244,7 +244,7 @@ __device__ __forceinline__ void store_row_vec(T* row, int v, const float* f, int
   } else if (cols - v * N >= N) {
     st16_any(row + v * N, VecIO<T>::pack(f));
   } else if (v * N < cols) {
-    const int skip = N - (cols - v * N);
+    const int skip = N - int(cols - v * N);
 #pragma unroll
     for (int j = 1; j < N; ++j)
       if (j >= skip) Cvt<T>::store(row + cols - N + j, f[j]);

@@ -216,3 +216,71 @@ def test_batch_norm_of_a_plane_that_ends_below_2_31_elements(hk, cuda):
         helpers.assert_close(y[at], (xhat * 1.5 + 0.25).cpu().numpy(), "bf16", "batch norm")
         want = 1.5 * inv * (dy[at].double() - mean_dy - xhat * mean_dyx)
         helpers.assert_close(dx[at], want.cpu().numpy(), "bf16", "batch norm gradient")
+
+
+def _batch_norm_time(torch, hk, cuda, N, C, HW):
+    """us of a forward and a backward, the best of three."""
+    x, y = torch.ones((N, C, HW), dtype=torch.bfloat16, device=cuda), torch.empty((N, C, HW), dtype=torch.bfloat16, device=cuda)
+    scale, bias, sm, si = (torch.ones(C, device=cuda) for _ in range(4))
+    workspace = torch.empty(hk.batch_norm_workspace_bytes(x) // 4 + 1, device=cuda)
+    best = [1e9, 1e9]
+    for _ in range(4):
+        at = [torch.cuda.Event(enable_timing=True) for _ in range(3)]
+        at[0].record()
+        hk.batch_norm_fwd(x, scale, bias, y, 0.1, 1e-5, None, None, sm, si, workspace=workspace)
+        at[1].record()
+        hk.batch_norm_bwd(x, x, scale, y, None, None, sm, si, workspace=workspace)
+        at[2].record()
+        torch.cuda.synchronize()
+        best = [min(b, at[i].elapsed_time(at[i + 1]) * 1e3) for i, b in enumerate(best)]
+    return best
+
+
+# channels of the two-launch form and of one workgroup
+@pytest.mark.parametrize("half,C,HW", [(90, 1024, 112 * 112), (16, 168000, 28 * 28)])
+def test_batch_norm_past_2_31_elements_is_no_slower_by_element(hk, cuda, half, C, HW):
+    """Twice the array costs about twice the time: the same kernels take it past element 2^31 (element by element it
+    was eight times)."""
+    import torch
+    assert half * C * HW < (1 << 31) < 2 * half * C * HW
+    small, large = _batch_norm_time(torch, hk, cuda, half, C, HW), _batch_norm_time(torch, hk, cuda, 2 * half, C, HW)
+    assert large[0] < 3 * small[0] and large[1] < 3 * small[1], (small, large)
+
+
+# of both forms, whole vectors and ragged planes, and a plane of more than 2^31 elements
+@pytest.mark.parametrize("N,C,HW", [(180, 1024, 112 * 112), (32, 90000, 28 * 28 + 1), (2, 1, (1 << 31) + 5)])
+def test_batch_norm_past_2_31_elements_of_every_form(hk, cuda, N, C, HW):
+    import torch
+    gen = torch.Generator(device="cuda").manual_seed(21)
+    x, dy = (_randn(torch, (N, C, HW), 31 + k, 2.0) for k in range(2))
+    x += 3.0
+    scale, bias = (torch.rand(C, generator=gen, device=cuda) + 0.5 for _ in range(2))
+    y, dx = torch.empty_like(x), torch.empty_like(x)
+    sm, si, ds, db = (torch.empty(C, device=cuda) for _ in range(4))
+    hk.batch_norm_fwd(x, scale, bias, y, 0.1, 1e-5, None, None, sm, si)
+    hk.batch_norm_bwd(dy, x, scale, dx, ds, db, sm, si)
+    torch.cuda.synchronize()
+    m = N * HW
+    for c in sorted({0, 1 % C, C // 2, C - 1}):
+        def mean_of(fn):
+            total = 0.0
+            for n in range(N):
+                for lo in range(0, HW, 1 << 28):
+                    at = slice(lo, min(HW, lo + (1 << 28)))
+                    total += float(fn(x[n, c, at].double(), dy[n, c, at].double()).sum())
+            return total / m
+        mean = mean_of(lambda a, g: a)
+        inv = (mean_of(lambda a, g: (a - mean) ** 2) + 1e-5) ** -0.5
+        helpers.assert_close(sm[c:c + 1], np.array([mean]), "fp32", "save_mean")
+        helpers.assert_close(si[c:c + 1], np.array([inv]), "fp32", "save_invstd")
+        mean, inv = float(sm[c]), float(si[c])
+        mg, mgx = mean_of(lambda a, g: g), mean_of(lambda a, g: g * (a - mean) * inv)
+        # sums of m terms of both signs: the rounding error is that of the terms
+        helpers.assert_close(db[c:c + 1], np.array([mg * m]), "fp32", "dbias", scale=float(np.sqrt(m)))
+        helpers.assert_close(ds[c:c + 1], np.array([mgx * m]), "fp32", "dscale", scale=float(np.sqrt(m)))
+        for n in sorted({0, 1, N // 2, N - 1}):
+            for at in (slice(0, 700), slice(HW - 700, HW)):
+                xhat = (x[n, c, at].double() - mean) * inv
+                helpers.assert_close(y[n, c, at], (xhat * float(scale[c]) + float(bias[c])).cpu().numpy(), "bf16", "y")
+                want = float(scale[c]) * inv * (dy[n, c, at].double() - mg - xhat * mgx)
+                helpers.assert_close(dx[n, c, at], want.cpu().numpy(), "bf16", "dx")
