@@ -151,7 +151,7 @@ __device__ __forceinline__ ACC block_reduce_lds(ACC v, ACC* lds) {
 // inner reduction, vector path (fp32 / bf16 / fp16 input, fp32 accumulate)
 // grid = (row groups, nsplit); `lanes` lanes of a wavefront (LANES) or a whole workgroup take one row chunk.
 //
-// A row is one run of `cols` contiguous elements or, with RUNS, `nruns` of them a fixed step apart (the sum over the
+// A row is one run of `cols` contiguous elements or, in the RUNS form, `nruns` of them a fixed step apart (the sum over the
 // first and the last dimension of [N, C, H * W]: row = channel, run = image).  Rows start anywhere (see ld16_any in
 // hk_common.h); the last, partial vector of a run is loaded as the run's last whole one and the elements that the
 // vector before it holds are left out.  Bound by HBM: what counts is that every lane has eight 16-byte loads in
@@ -160,6 +160,11 @@ __device__ __forceinline__ ACC block_reduce_lds(ACC v, ACC* lds) {
 // 87 ms (one thread per channel) -> 17.0 us (6.0 TB/s), of [12, 16, 16000] 72.7 ms -> 12.0 us; 16384 rows of 1021
 // elements (before: one workgroup per row, element by element) 20.9 -> 9.4 us, 524288 rows of 9 (9 MB) 364 -> 9.5 us,
 // 524288 aligned rows of 64 (a wavefront per row before) 93 -> 14.5 us; 32768 x 4096 unchanged at 40.1 us.
+// Eight wavefronts per SIMD are asked for: left to itself the compiler takes up to 158 registers for the fp32 rows that
+// lanes share, and three wavefronts do not cover the loads.  Rows of whole vectors have a form of their own, without the
+// partial vector's selects, and a wavefront's row its width at compile time (loads off one address).  GPU time alone,
+// fp32, without / with all of it: 16384 x 1000 20.2 / 10.4 us, 16384 x 1021 20.2 / 11.0, 8192 x 1024 11.3 / 6.0 (6.2 TB/s),
+// 524288 x 64 42.2 / 20.5; bf16: 16384 x 1000 7.7 / 6.7, 524288 x 64 13.4 / 11.8.
 // ---------------------------------------------------------------------------
 struct InnerArgs {
   const void* in;
@@ -189,13 +194,18 @@ __device__ __forceinline__ float lanes_reduce(float v, int lanes) {
   return v;
 }
 
-template <typename T, typename OUT_T, bool LANES, bool RUNS, typename R>
-__global__ __launch_bounds__(LANES ? 256 : 1024)
+// one run of whole vectors in rows on one level, one run of any length, several of any length
+enum InnerRow { ROW_WHOLE, ROW_RAGGED, ROW_RUNS };
+
+template <typename T, typename OUT_T, bool LANES, InnerRow ROW, typename R, bool WAVE = false>
+__global__ __launch_bounds__(LANES ? 256 : 1024, 8)
 void reduce_inner_vec_kernel(InnerArgs a) {
+  constexpr bool RUNS = ROW == ROW_RUNS, WHOLE = ROW == ROW_WHOLE;
+  static_assert(!WAVE || LANES, "all lanes of a wavefront");
   constexpr int VEC = VecIO<T>::N;
   constexpr int U = 8;
   __shared__ float red[kMaxWaves];
-  const int tpr = LANES ? a.lanes : int(blockDim.x);
+  const int tpr = WAVE ? kWave : LANES ? a.lanes : int(blockDim.x);
   const int t = LANES ? int(threadIdx.x) & (tpr - 1) : int(threadIdx.x);
   const int64_t row = !LANES ? int64_t(blockIdx.x)
                     : tpr == kWave ? int64_t(blockIdx.x) * (blockDim.x >> 6) + wave_index()
@@ -203,13 +213,13 @@ void reduce_inner_vec_kernel(InnerArgs a) {
   if (LANES && row >= a.rows) return;   // whole groups of lanes leave
   const int split = blockIdx.y;
   int64_t base = row * a.row_stride;
-  if (a.level_rows != a.rows) {
+  if (!WHOLE && a.level_rows != a.rows) {
     const uint32_t q = uint32_t(row) / uint32_t(a.level_rows);
     base = int64_t(uint32_t(row) - q * uint32_t(a.level_rows)) * a.row_stride + int64_t(q) * a.level_stride;
   }
   const T* p = static_cast<const T*>(a.in) + base;
   const int64_t nvec = (a.cols + VEC - 1) / VEC;          // of one run
-  const int skip = int(nvec * VEC - a.cols);              // elements of a run's last load that the one before it holds
+  const int skip = WHOLE ? 0 : int(nvec * VEC - a.cols);  // elements of a run's last load that the one before it holds
   const int64_t total = RUNS ? a.nruns * nvec : nvec;
   const int64_t end = (split + 1) * a.chunk < total ? (split + 1) * a.chunk : total;
   int64_t i = split * a.chunk + t;                        // place in the row, in vectors
@@ -226,7 +236,7 @@ void reduce_inner_vec_kernel(InnerArgs a) {
   }
   auto load = [&]() {
     const T* at = p + off;
-    if (skip != 0 && v == nvec - 1) at -= skip;
+    if (!WHOLE && skip != 0 && v == nvec - 1) at -= skip;
     return ld16_any(at);
   };
   auto step = [&]() {
@@ -255,10 +265,11 @@ void reduce_inner_vec_kernel(InnerArgs a) {
     bool last[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      last[u] = skip != 0 && v == nvec - 1;
+      last[u] = !WHOLE && skip != 0 && v == nvec - 1;
       r[u] = load();
       step();
     }
+    __builtin_amdgcn_sched_barrier(0);   // all loads before the first wait
 #pragma unroll
     for (int u = 0; u < U; ++u) add(acc[u], r[u], last[u]);
   }
@@ -268,7 +279,7 @@ void reduce_inner_vec_kernel(InnerArgs a) {
     bool last[U - 1];
 #pragma unroll
     for (int u = 0; u < U - 1; ++u) {
-      last[u] = skip != 0 && v == nvec - 1;
+      last[u] = !WHOLE && skip != 0 && v == nvec - 1;
       r[u] = u32x4{0, 0, 0, 0};
       if (i + int64_t(u) * tpr < end) r[u] = load();
       step();
@@ -783,8 +794,10 @@ static int launch_inner(const ReducePlan& p, const InnerShape& s, const void* in
   const bool lanes = s.tpr <= kWave;
   const int64_t groups = lanes ? (p.rows * s.tpr + 255) / 256 : p.rows;
   dim3 grid(unsigned(groups), unsigned(s.nsplit)), block(lanes ? 256u : unsigned(s.tpr));
-  auto kernel = p.nruns > 1 ? (lanes ? reduce_inner_vec_kernel<T, OUT_T, true, true, R> : reduce_inner_vec_kernel<T, OUT_T, false, true, R>)
-                            : (lanes ? reduce_inner_vec_kernel<T, OUT_T, true, false, R> : reduce_inner_vec_kernel<T, OUT_T, false, false, R>);
+  auto kernel = p.nruns > 1 ? (lanes ? reduce_inner_vec_kernel<T, OUT_T, true, ROW_RUNS, R> : reduce_inner_vec_kernel<T, OUT_T, false, ROW_RUNS, R>)
+      : p.cols % VecIO<T>::N || p.level_rows != p.rows ? (lanes ? reduce_inner_vec_kernel<T, OUT_T, true, ROW_RAGGED, R> : reduce_inner_vec_kernel<T, OUT_T, false, ROW_RAGGED, R>)
+      : s.tpr == kWave ? reduce_inner_vec_kernel<T, OUT_T, true, ROW_WHOLE, R, true>
+                       : (lanes ? reduce_inner_vec_kernel<T, OUT_T, true, ROW_WHOLE, R> : reduce_inner_vec_kernel<T, OUT_T, false, ROW_WHOLE, R>);
   profile_before(st);
   HK_LAUNCH(kernel, grid, block, 0, st, a);
   profile_after(st);
