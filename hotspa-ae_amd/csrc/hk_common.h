@@ -622,7 +622,8 @@ constexpr float kLog2Bound = 3.402823466e38f;
 __device__ __forceinline__ float log2_of_max(float m) {
   return fminf(fmaxf(m * 1.4426950408889634f, -kLog2Bound), kLog2Bound);
 }
-__device__ __forceinline__ bool past_log2_range(float ml) { return fabsf(ml) == kLog2Bound; }
+// (rare: what follows it is kept out of the way of the other rows' code)
+__device__ __forceinline__ bool past_log2_range(float ml) { return __builtin_expect(fabsf(ml) == kLog2Bound, 0); }
 
 // Rows whose maximum's magnitude is past kLog2Bound / log2(e): two different values out there lie so far apart that the
 // softmax is 1 / count at the maximum and 0 elsewhere.  M = the row's maximum, returned: how many elements equal it (NaN

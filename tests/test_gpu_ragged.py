@@ -487,3 +487,24 @@ def test_rows_that_need_no_scratch(hk, cuda, dtype):
         hk.reduce(x, out, [0], "sum", workspace=torch.empty(1, device=cuda))
         torch.cuda.synchronize()
         assert float(out) == float(oracle.round_to(np.asarray([a.sum()], np.float32), dtype)[0]), cols
+
+
+# a wavefront's rows, a workgroup's, rows kept packed (16-bit) and streamed ones, whole vectors and ragged
+@pytest.mark.parametrize("dtype", ["fp32", "bf16", "fp16"])
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("cols", [5, 40, 41, 1031, 4096, 40001, 70001])
+def test_cross_entropy_gradient_at_every_edge_column(hk, cuda, dtype, shift, cols):
+    """Equal logits, the label on each of the first and last 20 columns: 1 / cols, less one at the label and nowhere else."""
+    import torch
+    dt = {"fp32": torch.float32, "bf16": torch.bfloat16, "fp16": torch.float16}[dtype]
+    lab = torch.tensor(sorted(set(range(min(cols, 20))) | set(range(max(cols - 20, 0), cols))), device=cuda)
+    rows = len(lab)
+    pitch = cols + (0 if shift == 0 else 5)
+    _, x = _placed(cuda, np.zeros((rows, cols), np.float32), dtype, shift, pitch)
+    db, dx = _placed(cuda, np.zeros((rows, cols), np.float32), dtype, shift, pitch, 3.0)
+    hk.sce_sparse_bwd(x, lab, torch.ones(rows, dtype=dt, device=cuda), dx, -100)
+    torch.cuda.synchronize()
+    want = np.full((rows, cols), 1.0 / cols)
+    want[np.arange(rows), lab.cpu().numpy()] -= 1.0
+    helpers.assert_close(dx.contiguous(), want, dtype, "dlogits")
+    assert _guards_untouched(db, dx)
