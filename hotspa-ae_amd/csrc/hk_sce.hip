@@ -154,9 +154,9 @@ __device__ __forceinline__ void sce_store_loss(const SceArgs& a, int64_t row, in
                                                const MaxSumMaxTuple& p) {
   const float M = p.v[2];
   if (a.stats) {
-    // sum exp(x - M) = S * 2^(ML - M * log2e)
+    // sum exp(x - M) = S * 2^(ML - M * log2e); 0 where nothing but -inf is, NaN where a NaN is among it
     a.stats[row] = M;
-    a.stats[a.rows + row] = (M == kNegInf) ? 0.f
+    a.stats[a.rows + row] = (M == kNegInf) ? p.v[1] * 0.f
         : past_log2_range(p.v[0]) ? p.v[1] : p.v[1] * __builtin_amdgcn_exp2f(-fmaf(M, kLog2e, -p.v[0]));
     const int64_t local = label - a.vocab_start;
     a.stats[2 * a.rows + row] = (local >= 0 && local < a.cols) ? Cvt<T>::load(xr + local) : 0.f;

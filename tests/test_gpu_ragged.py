@@ -508,3 +508,19 @@ def test_cross_entropy_gradient_at_every_edge_column(hk, cuda, dtype, shift, col
     want[np.arange(rows), lab.cpu().numpy()] -= 1.0
     helpers.assert_close(dx.contiguous(), want, dtype, "dlogits")
     assert _guards_untouched(db, dx)
+
+
+@pytest.mark.parametrize("dtype", ["fp32", "bf16", "fp16"])
+@pytest.mark.parametrize("cols", [5, 40, 41, 1001, 4096, 40001, 70001])
+def test_shard_statistics_keep_a_nan(hk, cuda, dtype, cols):
+    """A column shard of nothing but -inf adds nothing to the row's sum; one that holds a NaN as well, or nothing else,
+    makes it NaN."""
+    import torch
+    dt = {"fp32": torch.float32, "bf16": torch.bfloat16, "fp16": torch.float16}[dtype]
+    x = torch.full((3, cols), -float("inf"), dtype=dt, device=cuda)
+    x[1, cols // 2] = float("nan")
+    x[2, :] = float("nan")
+    stats = torch.full((3, 3), 7.0, device=cuda)
+    hk.vocab_parallel_ce_stats(x, torch.zeros(3, dtype=torch.int64, device=cuda), stats, 0, -100)
+    torch.cuda.synchronize()
+    assert float(stats[1, 0]) == 0.0 and bool(torch.isnan(stats[1, 1:]).all()), stats
