@@ -623,8 +623,12 @@ int norm_fwd_typed(NormFwdArgs a, hipStream_t s) {
   const int want_rows = tune_get(TUNE_NORM_FWD_ROWS);
   const bool many_rows = want_rows > 0 ? want_rows >= 2 : a.rows >= 16 * int64_t(device_cu_count());
   // rows of up to 32 vectors share a wavefront (LayerNorm of 32768 rows of 256 bf16: 13.1 us with one to each, 10.7
-  // so); at 96 vectors norm_fwd_kernel is the faster one (20.1 against 25.5 us)
-  const bool short_rows = a.nvec <= 32 && tune_get(TUNE_NORM_FWD_THREADS) == 0;
+  // so); at 96 vectors norm_fwd_kernel is the faster one (20.1 against 25.5 us).  So it is for a few rows, whose
+  // wavefronts all run at once and leave nothing to share: GPU time alone, LayerNorm of 64 to 256 columns, shared / a
+  // wavefront each, bf16 128 rows 3.3 / 2.85 us, 2048 3.4 / 3.2, 4096 3.4 to 3.9 / 3.7 to 3.9, 16384 3.7 to 5.4 / 6.4 to
+  // 7.6; fp32 128 rows 2.9 / 2.75, 1024 2.9 / 2.85, 2048 3.0 / 3.2.
+  const bool short_rows = a.nvec <= 32 && tune_get(TUNE_NORM_FWD_THREADS) == 0 &&
+                          a.rows > (VEC == 8 ? 8 : 4) * int64_t(device_cu_count());
   // norm_fwd_kernel writes the pre-norm sum beside the residual it reads, the others without one as well
   const bool sum_alone = a.x_out != nullptr && !has_res;
   if (vec_ok && !short_rows && !sum_alone &&
