@@ -609,7 +609,19 @@ static int softmax_strided_typed(const void* x, const void* dy, void* out, int64
   }
   if constexpr (!std::is_same<T, double>::value) {
     constexpr int VEC = VecIO<T>::N;
-    if (inner >= VEC && inner <= 0x7fffffff && dim <= 32 * kDimVecs) {
+    // One thread per position stays the faster one (GPU us, one thread per position / the kernels above)
+    //  - where the device has positions enough for it and planes are so short that every lane's vector has a cache line
+    //    to itself: 32000 x 64 x 8 bf16 40.9 / 82.9, backward 37.8 / 113.3, and 8000 x 64 x 8 17.1 / 27.8 (one vector a
+    //    plane: sooner); 32000 x 64 x 8 fp32 61.6 / 69.8 and 50.6 / 102.4; 16000 x 64 x 16 bf16 53.9 / 36.4 and 43.9 /
+    //    47.1.  Odd planes, 28444 x 64 x 9 bf16, 63 / 50 and 70 / 69, and fewer positions, 2000 x 64 x 8 bf16 half the
+    //    time with the kernels above, do not belong to them;
+    //  - for a few positions of two to four entries on planes that share cache lines, where it is the shorter program:
+    //    1306 x 2 x 49 bf16 2.9 / 3.45 and 2.75 / 3.3, 64 x 2 x 1000 2.8 / 3.2 (64 positions a plane 2.9 / 2.9).
+    const int64_t positions = outer * inner, cus = device_cu_count(), bytes = inner * int64_t(sizeof(T));
+    const bool short_planes = inner % 4 == 0 && (BWD ? bytes < 64 : inner < 16) &&
+                              positions > cus * (BWD && bytes == 16 ? 192 : 512);
+    const bool few_narrow = positions <= cus * 512 && bytes % 128 != 0 && dim <= 4;
+    if (inner >= VEC && inner <= 0x7fffffff && dim <= 32 * kDimVecs && !short_planes && !few_narrow) {
       SoftmaxDimArgs a{};
       a.x = x; a.dy = dy; a.out = out; a.inner = inner; a.dim = int(dim);
       a.run_vecs = int((inner + VEC - 1) / VEC);
