@@ -815,10 +815,10 @@ static int sce_typed(SceArgs a, hipStream_t s) {
     HK_LAUNCH((sce_long_kernel<T, MODE == 1>), levels, dim3(unsigned(threads)), 0, s, a);
     profile_after(s);
     return launch_check("sce_long_kernel");
+  } else {
+    HK_LAUNCH((sce_generic_kernel<T, float, MODE>), levels, dim3(256), 0, s, a);
+    return launch_check("sce_generic_kernel");
   }
-  HK_LAUNCH((sce_generic_kernel<T, float, MODE>), dim3(unsigned(a.n0), unsigned(a.n1), unsigned(a.n2)), dim3(256), 0,
-            s, a);
-  return launch_check("sce_generic_kernel");
 }
 
 template <int MODE>
