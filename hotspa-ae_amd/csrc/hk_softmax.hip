@@ -439,13 +439,16 @@ static bool pick_softmax_shape(int nvec, bool aligned, bool odd, int max_nv, boo
   // measured on MI355X at 2048 bf16 columns: forward is fastest with two
   // vectors per thread (128 threads per row), backward with one (256 threads)
   const int want = bwd ? 1 : 2;
+  // a forced width is rounded up to one that exists; a wavefront's lanes hold up to four vectors each
   if (forced > 0 && forced <= 64) {
-    *threads = forced;
-    *nv = (nvec + forced - 1) / forced;
-    return (forced == 8 || forced == 16 || forced == 32 || forced == 64) && *nv <= 4;
+    const int lanes = std::max(8, pow2_ceil_sm(forced)), n = (nvec + lanes - 1) / lanes;
+    if (n <= 4) {
+      *threads = lanes; *nv = n;
+      return true;
+    }
   }
   if (forced > 0) {
-    int t = std::min(1024, std::max(64, (forced + 63) / 64 * 64));
+    int t = std::min(1024, std::max(128, (forced + 63) / 64 * 64));
     int n = pow2_ceil_sm((nvec + t - 1) / t);
     if (n > max_nv) return false;
     *threads = t; *nv = n;

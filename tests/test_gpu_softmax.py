@@ -132,3 +132,23 @@ def test_short_planes_cost_their_bytes(hk, cuda):
 
     short, long = replay_time((32000, 64, 8)), replay_time((4000, 64, 64))
     assert short[0] < 5 * long[0] and short[1] < 4 * long[1], (short, long)
+
+
+@pytest.mark.parametrize("width", [1, 8, 24, 40, 64, 100, 256])
+@pytest.mark.parametrize("cols", [64, 256, 1024, 2048, 4096])
+def test_forced_widths(hk, cuda, width, cols):
+    """Any width may be asked for, on rows of one level and of two: it is rounded to one that exists."""
+    import torch
+    x = helpers.draw(50 + cols, (6, 4, cols), dtype="bf16")
+    base = helpers.to_torch(x, "bf16", cuda)
+    y, y2 = torch.empty_like(base), torch.empty(4, 6, cols, dtype=base.dtype, device=cuda)
+    hk.tune_set("softmax_threads", width)
+    try:
+        hk.softmax_fwd(base, y)
+        hk.softmax_fwd(base.transpose(0, 1), y2)
+        torch.cuda.synchronize()
+    finally:
+        hk.tune_set("softmax_threads", 0)
+    want = torch.softmax(base.double(), -1)
+    helpers.assert_close(y, want.cpu().numpy(), "bf16", "y")
+    helpers.assert_close(y2, want.transpose(0, 1).contiguous().cpu().numpy(), "bf16", "y of a view")
