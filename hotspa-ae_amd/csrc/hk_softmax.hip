@@ -322,9 +322,9 @@ void softmax_bwd_dim_kernel(SoftmaxDimArgs a) {
   }
 }
 
-// Softmax along a dimension of extent `dim` with element stride `inner`, longer or with shorter planes than the kernels
-// above take, and fp64
-// (inner == 1: rows too long or too unaligned for the register kernels).
+// Softmax along a dimension of extent `dim` with element stride `inner`: longer dimensions than the kernels above take,
+// shorter planes, those that softmax_strided_typed leaves to it, and fp64; for inner == 1, rows longer than a
+// workgroup's registers hold or shorter than a vector, and fp64.
 // One thread walks one (outer, inner) position, threads of a wave sit on
 // neighbouring inner positions; for inner == 1 one workgroup takes one row.
 template <typename T, typename CT>

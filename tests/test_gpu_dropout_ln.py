@@ -239,12 +239,14 @@ def test_parallel_residual(hk, cuda, combo, has_x1, tied, p, is_rms, shape):
 
 @pytest.mark.parametrize("combo", COMBOS, ids=lambda c: "w%s-i%s-r%s" % c)
 @pytest.mark.parametrize("rows,cols,blocks", [(1, 512, 0), (61, 512, 2), (50, 4096, 3), (2500, 4096, 0),
-                                               (37, 5120, 5), (19, 8192, 4), (23, 1000, 2)])
+                                               (37, 5120, 5), (19, 8192, 4), (23, 1000, 2), (61, 520, 2),
+                                               (23, 4104, 2)])
 @pytest.mark.parametrize("is_rms", [False, True])
 def test_prenorm_block_backward(hk, cuda, combo, rows, cols, blocks, is_rms):
     """Dropout + incoming and outgoing residual-stream gradients and nothing else: the form with a kernel of
-    its own when the row fills every thread (cols = 1000 does not and takes the general kernel).  A forced
-    small grid makes every thread group walk many rows, through full rounds and the guarded tail."""
+    its own, for rows that fill every thread and rows that leave some idle (520 and 1000 columns in several
+    groups of a workgroup, 4104 in its only one).  A forced small grid makes every thread group walk many rows,
+    through full rounds and the guarded tail."""
     import torch
     wt, it, rt = combo
     p = 0.15

@@ -1138,6 +1138,7 @@ def test_ndarray_sceloss_buffers(ops, cuda, reduction):
     n = want.size
     tl = torch.from_numpy(lab).to(cuda)
     inside_labels, inside_preds = torch.from_numpy(lab).to(cuda), tx.clone()
+    _sync_in()
     for out, labels, preds in ((torch.empty(n, device=cuda), tl, tx), (torch.empty(1, n, device=cuda), tl, tx),
                                (inside_labels.view(torch.float32)[:n], inside_labels, tx),
                                (inside_preds.view(-1)[5:5 + n], tl, inside_preds)):
