@@ -670,7 +670,10 @@ static InnerShape shape_inner(const ReducePlan& p, bool split) {
       tpr = 1;
       while (int64_t(tpr) * 2 < nvec) tpr <<= 1;
     } else {
-      tpr = nvec <= 64 * 32 ? 64 : (nvec <= 256 * 32 ? 256 : 1024);
+      // a wavefront for up to two rounds of 8 loads per lane; its third and fourth wait behind each other (GPU us, 64 / 256
+      // threads, fp32 rows of 1500 vectors: 1100 of them 7.4 / 6.2, 8192 31.7 / 29.4; of 2048: 1024 7.4 / 7.0, 8192
+      // 42.4 / 40.3; of 1000: 8192 21.2 / 21.3; of 512: 4096 6.9 / 7.0)
+      tpr = nvec <= 64 * 16 ? 64 : (nvec <= 256 * 32 ? 256 : 1024);
       // too few rows to fill the chip: widen the group until a thread has at most one round of 8 loads,
       // so that a short row costs one memory round trip instead of several dependent ones
       if (p.rows < want_blocks) tpr = int(std::max<int64_t>(tpr, std::min<int64_t>(1024, (nvec + 7) / 8)));
