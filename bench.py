@@ -606,8 +606,8 @@ CASES = [
     ("next: 2-norm of rows, gradient bf16 [32768x4096]", lambda hk, t, n: case_p_norm(hk, t, n, "bwd")),
     ("next: gradient of mean axis0 bf16 [32768x4096] (write only)", lambda hk, t, n: case_reduce_gradient(hk, t, n, 0)),
     ("next: gradient of mean axis1 bf16 [32768x4096] (write only)", lambda hk, t, n: case_reduce_gradient(hk, t, n, 1)),
-    ("next: batch norm fwd bf16 [256,256,56,56] (2R+1W, 3 launches)", lambda hk, t, n: case_batch_norm(hk, t, n, "fwd")),
-    ("next: batch norm bwd bf16 [256,256,56,56] (4R+1W, 3 launches)", lambda hk, t, n: case_batch_norm(hk, t, n, "bwd")),
+    ("next: batch norm fwd bf16 [256,256,56,56] (2R+1W, 2 launches)", lambda hk, t, n: case_batch_norm(hk, t, n, "fwd")),
+    ("next: batch norm bwd bf16 [256,256,56,56] (4R+1W, 2 launches)", lambda hk, t, n: case_batch_norm(hk, t, n, "bwd")),
     ("next: gather of a transposed view fp32 [8192x4096]", lambda hk, t, n: case_strided(hk, t, n, "transposed fp32")),
     ("next: gather of a view with the last two dimensions swapped bf16 [32x2048x2048]",
      lambda hk, t, n: case_strided(hk, t, n, "swapped bf16")),
