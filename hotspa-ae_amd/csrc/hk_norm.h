@@ -61,7 +61,8 @@ struct NormBwdArgs {
   int cols;
   int nvec;
   int part_pitch;       // elements between partial rows: cols rounded up to whole vectors
-  int tpr;              // threads per row (multiple of 64)
+  int tpr;              // threads per row
+  int fold_both;        // the staging area of the column sums' fold holds both of them
   float eps;
   float inv_cols;
   int stat_kind;
@@ -72,7 +73,9 @@ struct NormBwdArgs {
 struct BwdPlan {
   bool reg_path;
   bool any;             // the instance for rows of any length and alignment
+  int lpr;              // lanes of a wavefront that hold a row; 0: whole wavefronts, with a barrier per row
   int tpr, nv, rpb, grid;
+  bool fold_both;
   int block;
   size_t lds_bytes;
   size_t ws_bytes;
@@ -114,6 +117,7 @@ struct GenericIO {
 // Per-type entry points (T = float, bf16, fp16), defined by the explicit instantiations.
 template <typename T> int norm_fwd_typed(NormFwdArgs a, hipStream_t s);
 template <typename T> BwdPlan plan_norm_bwd(int64_t rows, int cols, bool aligned);
+template <typename T> BwdPlan plan_norm_bwd_lanes(int64_t rows, int cols);
 template <typename T> int norm_bwd_typed(NormBwdArgs a, int mode, void* dgamma, void* dbeta, void* ws,
                                           size_t ws_bytes, hipStream_t s);
 // double precision: one workgroup per row, arithmetic in double (with the fp32 instantiations)

@@ -173,15 +173,16 @@ int hk_norm_bwd_workspace_bytes(int dtype, int64_t rows, int64_t cols, size_t* b
              "hk_norm_bwd_workspace_bytes: bad shape");
   *bytes = 0;
   if (rows == 0 || cols == 0) return HK_OK;
-  // for operands on the 16-byte grid and off it
-  auto need = [&](auto plan) {
+  // for operands on the 16-byte grid and off it, and for the rows of a wavefront's lanes
+  auto need = [&](auto plan, auto plan_lanes) {
     const BwdPlan on = plan(rows, int(cols), true), off = plan(rows, int(cols), false);
-    return std::max(on.reg_path ? on.ws_bytes : 0, off.reg_path ? off.ws_bytes : 0);
+    const BwdPlan lanes = plan_lanes(rows, int(cols));
+    return std::max({on.reg_path ? on.ws_bytes : 0, off.reg_path ? off.ws_bytes : 0, lanes.reg_path ? lanes.ws_bytes : 0});
   };
   switch (dtype) {
-    case HK_FLOAT32: *bytes = need(plan_norm_bwd<float>); return HK_OK;
-    case HK_BFLOAT16: *bytes = need(plan_norm_bwd<bf16>); return HK_OK;
-    case HK_FLOAT16: *bytes = need(plan_norm_bwd<fp16>); return HK_OK;
+    case HK_FLOAT32: *bytes = need(plan_norm_bwd<float>, plan_norm_bwd_lanes<float>); return HK_OK;
+    case HK_BFLOAT16: *bytes = need(plan_norm_bwd<bf16>, plan_norm_bwd_lanes<bf16>); return HK_OK;
+    case HK_FLOAT16: *bytes = need(plan_norm_bwd<fp16>, plan_norm_bwd_lanes<fp16>); return HK_OK;
     case HK_FLOAT64: return HK_OK;
     default:
       set_last_error("hk_norm_bwd_workspace_bytes: not implemented for dtype %d", dtype);

@@ -3,5 +3,6 @@
 
 namespace hk {
 template BwdPlan plan_norm_bwd<bf16>(int64_t, int, bool);
+template BwdPlan plan_norm_bwd_lanes<bf16>(int64_t, int);
 template int norm_bwd_typed<bf16>(NormBwdArgs, int, void*, void*, void*, size_t, hipStream_t);
 } // namespace hk

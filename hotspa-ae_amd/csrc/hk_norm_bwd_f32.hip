@@ -3,6 +3,7 @@
 
 namespace hk {
 template BwdPlan plan_norm_bwd<float>(int64_t, int, bool);
+template BwdPlan plan_norm_bwd_lanes<float>(int64_t, int);
 template int norm_bwd_typed<float>(NormBwdArgs, int, void*, void*, void*, size_t, hipStream_t);
 
 int norm_bwd_f64(const NormBwdArgs& a, int mode, void* dgamma, void* dbeta, hipStream_t s) {

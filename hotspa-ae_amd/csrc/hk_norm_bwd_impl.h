@@ -57,15 +57,18 @@ __device__ __forceinline__ float clamp_by_magnitude(float g, float eps) {
 // optional operands, by splitting each row number with two divisions.
 //
 // RAGGED: rows of any length and alignment, see AnyBoundary.  The row's partial last vector is
-// read as its last whole one; the elements that it shares with the vector before it are zeroed in x and dy, add nothing
-// and are not stored.  The partial rows of the column sums keep whole vectors (part_pitch).  LayerNorm backward of
-// 8191 x 1021 bf16: 1114 us element by element -> 22.5 us, of 10000 x 8191 2121 -> 142 us (3.5 TB/s; 8192 columns on
-// the 16-byte grid 93 us: what is left is the extra cache lines of accesses on odd 2-byte boundaries), of
-// 8192 x 8191 fp32 1328 -> 150 us (5.4 TB/s).
+// read as its last whole one; the elements that it shares with the vector before it are left out of the row sums, their
+// dx comes out of both to the same bits and is stored twice, in whole vectors (element by element, up to seven stores
+// per row: 14549 x 3579 bf16 68.5 us instead of 57.2).  The partial rows of the column sums keep whole vectors
+// (part_pitch), of which the fold takes every column once.  LayerNorm backward of 8191 x 1021 bf16: 1114 us element by
+// element, 13.8 us so (8192 x 1024 on the 16-byte grid: 12.9); of 8192 x 8191 fp32 1328 -> 150 us (5.4 TB/s).
+//
+// LPR: that many lanes of a wavefront hold a row (plan_norm_bwd_lanes); 0 for whole wavefronts.
 template <typename T, int NV, int MODE, int PF, bool EXACT, bool STATS_F32, bool EXTRA, int MAXT, bool FIXED,
-          bool CLAMP, bool LEVELS = false, bool RAGGED = false>
+          bool CLAMP, bool LEVELS = false, bool RAGGED = false, int LPR = 0>
 __global__ __launch_bounds__(MAXT)
 void norm_bwd_kernel(NormBwdArgs a) {
+  static_assert(LPR == 0 || (RAGGED && LPR < kWave && NV == 1), "several rows to a wavefront: any boundary, a vector per lane");
   static_assert(!LEVELS || (FIXED && !EXTRA && EXACT), "the running walk index is built for the lean instances");
   static_assert(!RAGGED || (!FIXED && !EXACT), "rows of any boundary: any group width, a partial last vector");
   constexpr int VEC = VecIO<T>::N;
@@ -74,12 +77,12 @@ void norm_bwd_kernel(NormBwdArgs a) {
   constexpr bool WITH_DB = EXTRA || MODE != BWD_RMS;   // column sums of dy (dbeta)
   using StatT = typename std::conditional<STATS_F32, float, T>::type;
   using RowSums = SumTuple<KS>;
-  extern __shared__ float lds[];            // [rows_per_block, cols] column-sum staging
+  extern __shared__ __align__(16) float lds[];   // [rows_per_block, part_pitch] column-sum staging, of one sum or both
   __shared__ __align__(16) float red[2][kMaxWaves * KS];  // double-buffered by step parity
 
-  const int tpr = FIXED ? MAXT : a.tpr;    // multiple of 64: a wavefront never straddles two rows
+  const int tpr = FIXED ? MAXT : LPR ? LPR : a.tpr;   // without LPR a multiple of 64: a wavefront never straddles two rows
   const int rpb = FIXED ? 1 : int(blockDim.x) / tpr;
-  const int group = FIXED ? 0 : __builtin_amdgcn_readfirstlane(int(threadIdx.x) / tpr);
+  const int group = FIXED ? 0 : LPR ? int(threadIdx.x) / tpr : __builtin_amdgcn_readfirstlane(int(threadIdx.x) / tpr);
   const int t = int(threadIdx.x) - group * tpr;
   const int waves_per_group = tpr >> 6;
   const int first_wave = group * waves_per_group;
@@ -89,7 +92,7 @@ void norm_bwd_kernel(NormBwdArgs a) {
   int vidx[NV];
   bool vin[NV];
   int col[NV];                            // first column that vector i loads
-  [[maybe_unused]] u32x4 own[NV];         // RAGGED: the bits of a loaded vector that belong to this thread
+  [[maybe_unused]] uint32_t own[VEC];     // RAGGED: which elements of the last loaded vector count in the row sums
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
     const int v = i * tpr + t;
@@ -97,33 +100,16 @@ void norm_bwd_kernel(NormBwdArgs a) {
     vidx[i] = vin[i] ? v : a.nvec - 1;
     col[i] = vec_column<T, RAGGED>(vidx[i], a.cols);
     if constexpr (RAGGED) {
-      const int skip = (v + 1) * VEC - a.cols;
-      constexpr int PER = 4 / int(sizeof(T));   // elements per dword
+      const int skip = (v + 1) * VEC - a.cols;   // VEC or more past the row's end
+      if (i == NV - 1) {
 #pragma unroll
-      for (int d = 0; d < 4; ++d) own[i][d] = skip >= (d + 1) * PER ? 0u : (skip <= d * PER ? 0xffffffffu : 0xffff0000u);
+        for (int j = 0; j < VEC; ++j) own[j] = skip > j ? 0u : 0xffffffffu;
+      }
     }
   }
   auto ld_row = [](const T* p) { if constexpr (RAGGED) return ld16_any<T>(p); else return ld16(p); };
   auto ld_par = [](const T* p) { if constexpr (RAGGED) return ld16_any_keep<T>(p); else return ld16_keep(p); };
 
-  // gamma (and beta) of this thread's columns as fp32; a missing gamma is all ones
-  float gm[NE];
-  [[maybe_unused]] float bt[MODE == BWD_LN_MEMEFF ? NE : 1];
-  {
-    const T* gp = static_cast<const T*>(a.gamma);
-    const T* bp = static_cast<const T*>(a.beta);
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-#pragma unroll
-      for (int j = 0; j < VEC; ++j) gm[i * VEC + j] = 1.f;
-      if (gp) VecIO<T>::unpack(ld_par(gp + col[i]), &gm[i * VEC]);
-      if constexpr (MODE == BWD_LN_MEMEFF) {
-#pragma unroll
-        for (int j = 0; j < VEC; ++j) bt[i * VEC + j] = 0.f;
-        if (bp) VecIO<T>::unpack(ld_par(bp + col[i]), &bt[i * VEC]);
-      }
-    }
-  }
   [[maybe_unused]] const bool clamp = MODE == BWD_LN_MEMEFF || CLAMP || (EXTRA && a.clamp_gamma != 0);
 
   float dg[NE], db[NE];
@@ -188,6 +174,26 @@ void norm_bwd_kernel(NormBwdArgs a) {
   int64_t row0 = int64_t(blockIdx.x) * rpb + group;
   static_for<PF>([&](auto slot) { issue(slot, row0 + decltype(slot)::value * stride); });
 
+  // gamma (and beta) of this thread's columns as fp32, after the first rows' loads so that one latency
+  // covers both; a missing gamma is all ones
+  float gm[NE];
+  [[maybe_unused]] float bt[MODE == BWD_LN_MEMEFF ? NE : 1];
+  {
+    const T* gp = static_cast<const T*>(a.gamma);
+    const T* bp = static_cast<const T*>(a.beta);
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) gm[i * VEC + j] = 1.f;
+      if (gp) VecIO<T>::unpack(ld_par(gp + col[i]), &gm[i * VEC]);
+      if constexpr (MODE == BWD_LN_MEMEFF) {
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) bt[i * VEC + j] = 0.f;
+        if (bp) VecIO<T>::unpack(ld_par(bp + col[i]), &bt[i * VEC]);
+      }
+    }
+  }
+
   int parity = 0;
   // guarded: check that the slot's row exists (the tail); otherwise it is known to
   auto step = [&](auto slot, auto guarded) {
@@ -198,10 +204,6 @@ void norm_bwd_kernel(NormBwdArgs a) {
     float xs[NE], ts[NE];                 // xc (x_hat in the memory-efficient mode) and dy * gamma
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
-      if constexpr (RAGGED) {
-        nx[d][i] &= own[i];
-        ndy[d][i] &= own[i];
-      }
       VecIO<T>::unpack(nx[d][i], &xs[i * VEC]);
       VecIO<T>::unpack(ndy[d][i], &ts[i * VEC]);
       if (!EXACT && !RAGGED) {
@@ -219,6 +221,12 @@ void norm_bwd_kernel(NormBwdArgs a) {
     // the slot is free again: refill it with the row PF steps ahead
     issue(slot, row + int64_t(PF) * stride);
 
+    // an element that the row's last vector shares with the one before it counts once in the row sums; its column
+    // sums stay with the fold, which takes each column from one of them
+    auto in_sums = [&](float v, int e) {
+      if constexpr (RAGGED) return e >= NE - VEC ? u2f(f2u(v) & own[e - (NE - VEC)]) : v;
+      else return v;
+    };
     RowSums s = RowSums::identity();
     float& s_prod = s.v[KS - 1];            // sum(dy g xc) (sum(dy (y - beta)) in the memory-efficient mode)
     // new column sums go to copies first: a guarded step of a missing row must leave dg / db alone
@@ -231,8 +239,8 @@ void norm_bwd_kernel(NormBwdArgs a) {
           const float yb = xs[e] - bt[e];
           const float kg = clamp_by_magnitude(gm[e], a.eps);
           const float xhat = yb / kg;
-          s.v[0] = fmaf(dz, gm[e], s.v[0]);
-          s_prod = fmaf(dz, yb, s_prod);
+          s.v[0] = fmaf(in_sums(dz, e), gm[e], s.v[0]);
+          s_prod = fmaf(in_sums(dz, e), in_sums(yb, e), s_prod);
           dg[e] = fmaf(dz, xhat, dg[e]);
           if constexpr (WITH_DB) db[e] += dz;
           xs[e] = xhat;
@@ -241,8 +249,8 @@ void norm_bwd_kernel(NormBwdArgs a) {
           const float xc = (MODE == BWD_RMS) ? xs[e] : xs[e] - mu;
           const float dzr = dz * rs;
           const float q = dzr * gm[e];
-          s_prod = fmaf(q, xc, s_prod);
-          if constexpr (MODE != BWD_RMS) s.v[0] += q;
+          s_prod = fmaf(in_sums(q, e), in_sums(xc, e), s_prod);
+          if constexpr (MODE != BWD_RMS) s.v[0] += in_sums(q, e);
           dg[e] = fmaf(dzr, xc, dg[e]);
           if constexpr (WITH_DB) db[e] += dz;
           xs[e] = xc;
@@ -256,7 +264,18 @@ void norm_bwd_kernel(NormBwdArgs a) {
     else if (clamp) accumulate(std::true_type{});   // uniform
     else accumulate(std::false_type{});
 
-    if constexpr (FIXED) s = group_allreduce_tuple_fixed<RowSums, MAXT / 64>(s, red[parity]);
+    if constexpr (LPR != 0) {
+      // No barrier separates the steps of a lane group: without this the column sums of every step of a round are
+      // formed at the round's end, and each step's row stays in registers until then (LayerNorm, bf16: 123 registers
+      // instead of 94).
+#pragma unroll
+      for (int e = 0; e < NE; ++e) {
+        asm volatile("" : "+v"(dg[e]));
+        if constexpr (WITH_DB) asm volatile("" : "+v"(db[e]));
+      }
+    }
+    if constexpr (LPR != 0) s = lanes_allreduce_tuple<LPR>(s);
+    else if constexpr (FIXED) s = group_allreduce_tuple_fixed<RowSums, MAXT / 64>(s, red[parity]);
     else s = group_allreduce_tuple(s, red[parity], first_wave, waves_per_group);
     parity ^= 1;
     if (valid) {
@@ -305,7 +324,8 @@ void norm_bwd_kernel(NormBwdArgs a) {
             }
           }
           if constexpr (RAGGED) {
-            store_row_vec<T, true, false>(dxr, v, o, a.cols);
+            // (an upstream gradient that is added in place must not be read after a neighbour has stored over it)
+            store_row_vec<T, true, !EXTRA>(dxr, v, o, a.cols);
             if (drr) store_row_vec<T, true, false>(drr, v, o, a.cols);
           } else {
             const u32x4 pk = VecIO<T>::pack(o);
@@ -334,61 +354,57 @@ void norm_bwd_kernel(NormBwdArgs a) {
     row0 += round;
   }
 
-  // fold the row groups of this block, then write one partial row per block
-  float* outs[2] = {a.part_dgamma, a.part_dbeta};
-  if constexpr (FIXED) {
-    // one group: every thread writes its own sums, as 16-byte streaming stores (the partial rows are read by the
-    // fold kernel, never again by this one; left in the cache they would only wait for the write-back at the
-    // kernel's end)
-    static_assert(VEC % 4 == 0, "whole float4 vectors per 16-byte vector of the data type");
+  // fold the row groups of this block, then write one partial row per block, as 16-byte streaming stores (the partial
+  // rows are read by the fold kernel, never again by this one; left in the cache they would only wait for the
+  // write-back at the kernel's end)
+  static_assert(VEC % 4 == 0, "whole float4 vectors per 16-byte vector of the data type");
+  float* outs[2] = {a.part_dgamma, WITH_DB ? a.part_dbeta : nullptr};
+  auto put = [&](float* dst, const float* acc, bool stream) {
 #pragma unroll
-    for (int which = 0; which < (WITH_DB ? 2 : 1); ++which) {
-      if (outs[which] == nullptr) continue;
-      const float* acc = which == 0 ? dg : db;
-      float* dst = outs[which] + int64_t(blockIdx.x) * a.cols;   // whole vectors: part_pitch == cols
+    for (int i = 0; i < NV; ++i) {
+      if (!EXACT && !vin[i]) continue;
 #pragma unroll
-      for (int i = 0; i < NV; ++i) {
-#pragma unroll
-        for (int j = 0; j < VEC; j += 4) {
-          const u32x4 pk = {f2u(acc[i * VEC + j]), f2u(acc[i * VEC + j + 1]), f2u(acc[i * VEC + j + 2]),
-                            f2u(acc[i * VEC + j + 3])};
-          st16_stream(dst + vidx[i] * VEC + j, pk);
-        }
+      for (int j = 0; j < VEC; j += 4) {
+        const u32x4 pk = {f2u(acc[i * VEC + j]), f2u(acc[i * VEC + j + 1]), f2u(acc[i * VEC + j + 2]),
+                          f2u(acc[i * VEC + j + 3])};
+        if (stream) st16_stream(dst + vidx[i] * VEC + j, pk);
+        else st16(dst + vidx[i] * VEC + j, pk);
       }
     }
+  };
+  if (FIXED || rpb == 1) {   // every thread writes its own sums
+    if (outs[0]) put(outs[0] + int64_t(blockIdx.x) * a.part_pitch, dg, true);
+    if (WITH_DB && outs[1]) put(outs[1] + int64_t(blockIdx.x) * a.part_pitch, db, true);
     return;
   }
-#pragma unroll
-  for (int which = 0; which < (WITH_DB ? 2 : 1); ++which) {
-    if (outs[which] == nullptr) continue;
-    float* acc = which == 0 ? dg : db;
-    __syncthreads();
-    if (rpb > 1) {
-#pragma unroll
-      for (int i = 0; i < NV; ++i) {
-        const int v = i * tpr + t;
-        if (v < a.nvec) {
-#pragma unroll
-          for (int j = 0; j < VEC; ++j) lds[group * a.part_pitch + v * VEC + j] = acc[i * VEC + j];
-        }
+  // Several groups: every group stages its sums, then neighbouring threads fold neighbouring columns, 16 bytes each.
+  // (Folded by the first group alone, element by element, either sum took 4 us of a kernel that has 2 us of rows:
+  // LayerNorm of 1218 x 92 fp16 11.3 us.)
+  const int pitch = a.part_pitch, region = rpb * pitch;
+  auto fold = [&](const float* src, float* dst) {
+    if (dst == nullptr) return;
+    for (int c = int(threadIdx.x) * 4; c < pitch; c += int(blockDim.x) * 4) {
+      float r[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+      for (int g = 0; g < rpb; ++g) {
+        const u32x4 v = *reinterpret_cast<const u32x4*>(src + g * pitch + c);
+        r[0] += u2f(v.x); r[1] += u2f(v.y); r[2] += u2f(v.z); r[3] += u2f(v.w);
       }
+      st16(dst + int64_t(blockIdx.x) * pitch + c, u32x4{f2u(r[0]), f2u(r[1]), f2u(r[2]), f2u(r[3])});
+    }
+  };
+  const bool both = WITH_DB && a.fold_both;   // uniform: the staging area holds both sums
+  put(lds + group * pitch, dg, false);
+  if (both) put(lds + region + group * pitch, db, false);
+  __syncthreads();
+  fold(lds, outs[0]);
+  if constexpr (WITH_DB) {
+    if (!both) {
+      __syncthreads();
+      put(lds + group * pitch, db, false);
       __syncthreads();
     }
-    if (group == 0) {
-      float* dst = outs[which] + int64_t(blockIdx.x) * a.part_pitch;
-#pragma unroll
-      for (int i = 0; i < NV; ++i) {
-        const int v = i * tpr + t;
-        if (v < a.nvec) {
-#pragma unroll
-          for (int j = 0; j < VEC; ++j) {
-            float r = acc[i * VEC + j];
-            for (int g = 1; g < rpb; ++g) r += lds[g * a.part_pitch + v * VEC + j];
-            dst[v * VEC + j] = r;
-          }
-        }
-      }
-    }
+    fold(both ? lds + region : lds, outs[1]);
   }
 }
 
@@ -396,14 +412,14 @@ void norm_bwd_kernel(NormBwdArgs a) {
 // pitch == cols; otherwise the last vector of a partial row holds the row's last columns, the first pitch - cols of
 // its elements being another vector's.
 // blockIdx.y picks dgamma / dbeta; a block covers 128 columns as 32 float4
-// column groups x 16 row slices, every slice keeps 8 independent loads in
-// flight, slices are folded through LDS.
+// column groups x 16 row slices, every slice keeps 16 independent loads in
+// flight (256 partial rows in one round), slices are folded through LDS.
 template <typename T>
 __global__ __launch_bounds__(512)
 void norm_bwd_finalize_kernel(const float* __restrict__ part_dgamma,
                               const float* __restrict__ part_dbeta, T* dgamma, T* dbeta,
                               int nparts, int cols, int pitch) {
-  constexpr int U = 8;
+  constexpr int U = 16;
   __shared__ float lds[16][32][4];
   const float* part = blockIdx.y == 0 ? part_dgamma : part_dbeta;
   T* out = blockIdx.y == 0 ? dgamma : dbeta;
@@ -412,19 +428,19 @@ void norm_bwd_finalize_kernel(const float* __restrict__ part_dgamma,
   const int c = (blockIdx.x * 32 + cg) * 4;
   float acc[4] = {0.f, 0.f, 0.f, 0.f};
   if (c < pitch) {                                    // a multiple of 4
-    int r = slice;
-    for (; r + (U - 1) * 16 < nparts; r += U * 16) {
+    for (int r = slice; r < nparts; r += U * 16) {
       u32x4 v[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) v[u] = ld16_keep(part + int64_t(r + u * 16) * pitch + c);
+      for (int u = 0; u < U; ++u) {   // a row past the end reads the last one
+        const int rr = r + u * 16;
+        v[u] = ld16_keep(part + int64_t(rr < nparts ? rr : nparts - 1) * pitch + c);
+      }
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        acc[0] += u2f(v[u].x); acc[1] += u2f(v[u].y); acc[2] += u2f(v[u].z); acc[3] += u2f(v[u].w);
+        const bool in = r + u * 16 < nparts;
+        acc[0] += in ? u2f(v[u].x) : 0.f; acc[1] += in ? u2f(v[u].y) : 0.f;
+        acc[2] += in ? u2f(v[u].z) : 0.f; acc[3] += in ? u2f(v[u].w) : 0.f;
       }
-    }
-    for (; r < nparts; r += 16) {
-      const u32x4 v = ld16_keep(part + int64_t(r) * pitch + c);
-      acc[0] += u2f(v.x); acc[1] += u2f(v.y); acc[2] += u2f(v.z); acc[3] += u2f(v.w);
     }
   }
 #pragma unroll
@@ -563,6 +579,34 @@ void norm_bwd_generic_cols_kernel(NormBwdArgs a, int mode, T* dgamma, T* dbeta) 
   }
 }
 
+// Many rows of up to 32 vectors, dense or pitched, on any boundary, without optional operands: 16 or 32 lanes to a row,
+// a vector per lane, two rows in flight per group.  A wavefront to a row leaves half of its lanes and more idle; that
+// shows once its workgroups, 16 rows each on every compute unit, have to walk (LayerNorm bf16, 32768 x 64 12.9 -> 8.1 us,
+// 32768 x 256 14.3 -> 12.9, 10490 x 80 7.1 -> 6.2), and not before (2530 x 71 5.8 against 6.1, 1218 x 92 5.1 against 5.8).
+// Longer rows do not gain from a wavefront of their own either, although it needs no barrier: 31451 x 1792 58.2 -> 63.7,
+// 8191 x 1021 13.3 -> 14.7, 4002 x 904 8.4 -> 9.0.
+template <typename T>
+BwdPlan plan_norm_bwd_lanes(int64_t rows, int cols) {
+  constexpr int VEC = VecIO<T>::N;
+  BwdPlan p{};
+  const int nvec = (cols + VEC - 1) / VEC, pitch = nvec * VEC;
+  if (cols < VEC || nvec > 32 || rows <= int64_t(device_cu_count()) * 16) return p;
+  p.lpr = nvec <= 16 ? 16 : 32;
+  p.nv = 1;
+  p.tpr = p.lpr;
+  p.block = 512;
+  p.rpb = p.block / p.lpr;
+  int64_t grid = tune_get(TUNE_NORM_BWD_BLOCKS);
+  if (grid <= 0) grid = device_cu_count();
+  p.grid = int(std::max<int64_t>(1, std::min<int64_t>(grid, (rows + p.rpb - 1) / p.rpb)));
+  p.reg_path = true;
+  const size_t one = size_t(p.rpb) * pitch * sizeof(float);   // at most 64 KiB
+  p.fold_both = 2 * one <= 65536;
+  p.lds_bytes = p.fold_both ? 2 * one : one;
+  p.ws_bytes = size_t(2) * size_t(p.grid) * pitch * sizeof(float);
+  return p;
+}
+
 // Rows that the aligned plan does not take: the general instance at 8 columns per thread (bf16, fp16; 4 for short fp32
 // rows), one 1024-thread workgroup per compute unit, as many rows per step as fit it.  The partial rows stay within
 // 16 MiB (what the library's own scratch holds) by using fewer workgroups for the longest rows.
@@ -584,7 +628,9 @@ BwdPlan plan_norm_bwd_any(int64_t rows, int cols) {
   if (grid < 1) grid = 1;
   p.reg_path = p.any = true;
   p.tpr = tpr; p.nv = nv; p.rpb = rpb; p.grid = int(grid); p.block = tpr * rpb;
-  p.lds_bytes = rpb > 1 ? size_t(rpb) * pitch * sizeof(float) : 0;
+  const size_t one = size_t(rpb) * pitch * sizeof(float);
+  p.fold_both = rpb > 1 && 2 * one <= 65536;
+  p.lds_bytes = rpb > 1 ? (p.fold_both ? 2 : 1) * one : 0;
   p.ws_bytes = size_t(2) * size_t(grid) * pitch * sizeof(float);
   return p;
 }
@@ -632,7 +678,9 @@ BwdPlan plan_norm_bwd(int64_t rows, int cols, bool aligned) {
   if (grid < 1) grid = 1;
   p.reg_path = true;
   p.tpr = tpr; p.nv = nv; p.rpb = rpb; p.grid = grid; p.block = tpr * rpb;
-  p.lds_bytes = rpb > 1 ? size_t(rpb) * cols * sizeof(float) : 0;
+  const size_t one = size_t(rpb) * cols * sizeof(float);
+  p.fold_both = rpb > 1 && 2 * one <= 65536;
+  p.lds_bytes = rpb > 1 ? (p.fold_both ? 2 : 1) * one : 0;
   p.ws_bytes = size_t(2) * grid * cols * sizeof(float);
   return p;
 }
@@ -695,6 +743,16 @@ static int launch_norm_bwd_inst(const NormBwdArgs& a, const BwdPlan& p, int pf, 
   return HK_OK;
 }
 
+template <typename T, int MODE, bool CLAMP, int MAXT>
+static void launch_norm_bwd_lanes(const NormBwdArgs& a, const BwdPlan& p, hipStream_t s) {
+  const dim3 grid{unsigned(p.grid)}, block{unsigned(p.block)};
+#define HK_BWD_LANES(NV, LPR) \
+  HK_LAUNCH((norm_bwd_kernel<T, NV, MODE, 2, false, true, false, MAXT, false, CLAMP, false, true, LPR>), grid, block, \
+            p.lds_bytes, s, a)
+  if (p.lpr == 16) HK_BWD_LANES(1, 16); else HK_BWD_LANES(1, 32);
+#undef HK_BWD_LANES
+}
+
 template <typename T, int MODE>
 static int launch_norm_bwd_any(const NormBwdArgs& a, const BwdPlan& p, hipStream_t s) {
   const dim3 grid{unsigned(p.grid)}, block{unsigned(p.block)};
@@ -745,6 +803,19 @@ static int launch_norm_bwd_nv(const NormBwdArgs& a, const BwdPlan& p, hipStream_
     set_last_error("norm_bwd: this mode keeps its statistics in float32");
     return HK_ERR_INVALID;
   }
+  if constexpr (MODE != BWD_LN_MEMEFF) {
+    if (p.lpr) {
+      profile_before(s);
+      if constexpr (MODE == BWD_LN) {
+        if (a.clamp_gamma) launch_norm_bwd_lanes<T, MODE, true, 512>(a, p, s);
+        else launch_norm_bwd_lanes<T, MODE, false, 512>(a, p, s);
+      } else {
+        launch_norm_bwd_lanes<T, MODE, false, 512>(a, p, s);
+      }
+      profile_after(s);
+      return launch_check("norm_bwd_kernel");
+    }
+  }
   if (p.any) return launch_norm_bwd_any<T, MODE>(a, p, s);
   const int bound = bound_for(p.block);
   const bool have_kernel = p.nv == 1 || p.nv == 2 || (p.nv == 4 && VecIO<T>::N == 4);
@@ -785,6 +856,13 @@ int norm_bwd_typed(NormBwdArgs a, int mode, void* dgamma, void* dbeta, void* ws,
   // rows that once took no scratch do without it still
   if (p.any && want_cols && (ws == nullptr || ws_bytes < p.ws_bytes || !aligned16(ws))) p.reg_path = false;
   if (p.any && !a.stats_f32 && mode != BWD_LN) p.reg_path = false;
+  if (p.reg_path && tune_get(TUNE_NORM_BWD_THREADS) <= 0) {
+    const bool lean = mode != BWD_LN_MEMEFF && a.stats_f32 && !a.dx_in && !a.dres && a.n0 == a.rows &&
+                      !(mode == BWD_RMS && (dbeta != nullptr || a.clamp_gamma));
+    const BwdPlan q = lean ? plan_norm_bwd_lanes<T>(a.rows, a.cols) : BwdPlan{};
+    // (a scratch that was sized for the other plans alone still serves them)
+    if (q.reg_path && (!want_cols || (ws != nullptr && ws_bytes >= q.ws_bytes && aligned16(ws)))) p = q;
+  }
   if (!p.reg_path) {
     HK_LAUNCH((norm_bwd_generic_dx_kernel<T, float>), dim3(unsigned(a.n0), unsigned(a.n1), unsigned(a.n2)), dim3(256),
               0, s, a, mode);
@@ -810,6 +888,7 @@ int norm_bwd_typed(NormBwdArgs a, int mode, void* dgamma, void* dbeta, void* ws,
     a.part_dbeta = nullptr;
   }
   a.tpr = p.tpr;
+  a.fold_both = p.fold_both;
   {
     // the walking kernel's row stride, split over the walk levels (used by the instances with a running walk index)
     const uint64_t stride = uint64_t(p.grid) * uint64_t(p.rpb);

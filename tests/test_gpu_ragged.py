@@ -367,6 +367,43 @@ def test_layer_norm_bwd_any_length_modes(hk, cuda, dtype, cols):
         helpers.assert_close(got, want, dtype, what, scale=None if what == "dx" else many)
 
 
+@pytest.mark.parametrize("dtype", ["fp32", "bf16", "fp16"])
+@pytest.mark.parametrize("is_rms", [True, False])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_norm_bwd_without_options(hk, cuda, dtype, is_rms, shift):
+    """Several rows to a wavefront (short rows, more of them than one step of the other kernels' workgroups takes) at
+    the edges of a lane group, and the longer rows' folds of one, several and many groups, dx in place of dz."""
+    import torch
+    vec, many_rows = 16 // ES[dtype], torch.cuda.get_device_properties(0).multi_processor_count * 16
+    shapes = [(many_rows + k, v * vec + j) for k, v in ((1, 1), (300, 15), (77, 16), (1, 17), (33, 31))
+              for j in (0, 1, vec - 1)] + [(many_rows, 9 * vec + 1), (many_rows + 1, 32 * vec), (3 * many_rows, 8 * vec + 3)] + \
+             [(1, 3 * vec), (600, 40 * vec + 1), (900, 128 * vec), (513, 129 * vec + 3), (300, 300 * vec + 1)]
+    for rows, cols in shapes:
+        pitch = cols + (0 if shift == 0 else 5)
+        x, dz = (helpers.draw(s + cols, (rows, cols), dtype=dtype) for s in (1100, 1200))
+        gamma = helpers.draw(1300 + cols, (cols,), "uniform", 0.5, 1.5, dtype)
+        mean = None if is_rms else x.astype(np.float64).mean(-1).astype(np.float32)
+        centred = x.astype(np.float64) - (0 if is_rms else mean[:, None])
+        rs = (1.0 / np.sqrt(np.square(centred).mean(-1) + 1e-5)).astype(np.float32)
+        edx, edg, edb = oracle.dropout_add_ln_bwd(dz, None, x, np.zeros_like(rs) if is_rms else mean, rs, gamma, is_rms)
+        tx = _placed(cuda, x, dtype, shift, pitch)[1]
+        zb, tz = _placed(cuda, dz, dtype, shift, pitch)
+        tg = _placed(cuda, gamma[None], dtype, shift, cols)[1][0]
+        (gb, dg), (bb, db) = (_placed(cuda, gamma[None], dtype, shift, cols, 0.0) for _ in range(2))
+        tmean = None if is_rms else helpers.to_torch(mean, "fp32", cuda)
+        hk.dropout_add_ln_bwd(tz, None, tx, tmean, helpers.to_torch(rs, "fp32", cuda), tg, tz, None, dg[0],
+                              None if is_rms else db[0], is_rms)
+        torch.cuda.synchronize()
+        what = "%d x %d" % (rows, cols)
+        helpers.assert_close(tz.contiguous(), edx, dtype, "dx0 " + what)
+        # column sums over `rows` terms: their rounding error is that of the terms
+        helpers.assert_close(dg[0].contiguous(), edg, dtype, "dgamma " + what, scale=float(np.sqrt(rows)))
+        if not is_rms:
+            helpers.assert_close(db[0].contiguous(), edb, dtype, "dbeta " + what, scale=float(np.sqrt(rows)))
+        for b, v in ((zb, tz), (gb, dg), (bb, db)):
+            assert _guards_untouched(b, v), what
+
+
 def _highest_rows(torch, cuda, seed, cols, dt):
     """Six rows: one element of the type's highest value, two of them, all of them, one above a second highest, highest
     beside lowest, and +inf beside the highest.  softmax is 1 / count at the row's maximum but for the last, all NaN."""
