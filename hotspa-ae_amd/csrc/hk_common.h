@@ -233,8 +233,9 @@ __device__ __forceinline__ I vec_column(I v, I cols) {
   return cols - v * N >= N ? v * N : cols - N;
 }
 // Stores vector v of a row.  SAME: an element that two vectors hold was computed to the same bits in both, so the
-// partial vector is stored whole over its neighbour's end; otherwise its own elements go out one by one.
-template <typename T, bool RAGGED, bool SAME, typename I>
+// partial vector is stored whole over its neighbour's end; otherwise its own elements go out one by one.  PLAIN: whole
+// vectors go through the cache.
+template <typename T, bool RAGGED, bool SAME, bool PLAIN = false, typename I = int>
 __device__ __forceinline__ void store_row_vec(T* row, I v, const float* f, I cols) {
   constexpr int N = VecIO<T>::N;
   if constexpr (!RAGGED) {
@@ -242,13 +243,23 @@ __device__ __forceinline__ void store_row_vec(T* row, I v, const float* f, I col
   } else if constexpr (SAME) {
     st16_any(row + vec_column<T, true>(v, cols), VecIO<T>::pack(f));
   } else if (cols - v * N >= N) {
-    st16_any(row + v * N, VecIO<T>::pack(f));
+    if constexpr (PLAIN) *reinterpret_cast<typename AnyBoundary<T>::vec*>(row + v * N) = VecIO<T>::pack(f);
+    else st16_any(row + v * N, VecIO<T>::pack(f));
   } else if (v * N < cols) {
     const int skip = N - int(cols - v * N);
 #pragma unroll
     for (int j = 1; j < N; ++j)
       if (j >= skip) Cvt<T>::store(row + cols - N + j, f[j]);
   }
+}
+
+// Workgroups are handed to the 8 XCDs in turn.  Where neighbouring workgroups share cache lines, runs of RUN of them go
+// to one XCD instead, whose L2 then holds each line whole; what is left over at the grid's end keeps its place.
+template <int RUN>
+__device__ __forceinline__ int64_t xcd_run_block(uint32_t block, uint32_t blocks) {
+  if (block >= blocks / (8 * RUN) * (8 * RUN)) return block;
+  const uint32_t turn = block / 8;
+  return int64_t(turn / RUN * 8 + block % 8) * RUN + turn % RUN;
 }
 
 __device__ __forceinline__ u32x4 ld16_stream(const void* p) {

@@ -177,27 +177,37 @@ void softmax_bwd_kernel(SoftmaxArgs a) {
 // plane is read as its last whole one, its own elements are stored one by one (in place, a neighbour may have replaced
 // the others before they were read).  The exponentials are formed twice, once for the sum and once on the way out:
 // holding them in fp32 would cost twice the registers.
-// Bound by HBM and, on odd planes, by the extra cache lines of accesses that straddle them; one thread per column that
-// passed over it three times measured (forward / backward, us) 150 / 160 at 8 x 21 x 263169 fp32, now 81 / 113 (4.4 and 4.7
-// TB/s; 5.3 and 5.5 at 263168); 81 / 77 at 8 x 21 x 263168 bf16, now 34.6 / 48.8; 143 / 103 at 16 x 150 x 16384 bf16, now
-// 44 / 46.5; 447 / 356 at 8 x 256 x 40000 fp32, now 124 / 183.
+// Bound by HBM and, on odd planes, by the cache lines that neighbouring workgroups share: runs of 8 or 16 of them stay
+// on one XCD, whose L2 then sees each line whole (8 x 21 x 263169 fp32, forward / backward: 82 / 117 -> 72 / 106 us).  One
+// thread per column that passed over it three times measured (forward / backward, us) 150 / 160 at 8 x 21 x 263169 fp32,
+// now 71 / 96 (5.0 and 5.5 TB/s; 65 / 91 at 263168); 81 / 77 at 8 x 21 x 263168 bf16, now 33 / 45; 143 / 103 at 16 x 150 x
+// 16384 bf16, now 37 / 43; 447 / 356 at 8 x 256 x 40000 fp32, now 123 / 180.
 constexpr int kDimVecs = 8;      // most entries per lane
-template <int N> __device__ __forceinline__ void slices_share(float* f, float* lds, int lx, int lane, int slices, bool take_max) {
-  // lds: [slices][N / 4][lx] 16-byte vectors
-  u32x4* mine = reinterpret_cast<u32x4*>(lds);
+// f[0..N): this lane's values; on return the slices' maximum or sum (in slice order) of each, the same in every slice.
+// lds: [slices + 1][LX * N].  A thread merges the slices of one value (every thread merging all of its lane's values
+// takes slices * N steps: 65 entries of 355 bf16 positions 9.0 us, so 5.5); calls may follow one another.
+template <int N, int LX> __device__ __forceinline__ void slices_share(float* f, float* lds, int slices, bool take_max) {
+  u32x4* mine = reinterpret_cast<u32x4*>(lds + (int(threadIdx.y) * LX + int(threadIdx.x)) * N);
 #pragma unroll
-  for (int q = 0; q < N / 4; ++q)
-    mine[(int(threadIdx.y) * (N / 4) + q) * lx + lane] = u32x4{f2u(f[4 * q]), f2u(f[4 * q + 1]), f2u(f[4 * q + 2]), f2u(f[4 * q + 3])};
+  for (int q = 0; q < N / 4; ++q) mine[q] = u32x4{f2u(f[4 * q]), f2u(f[4 * q + 1]), f2u(f[4 * q + 2]), f2u(f[4 * q + 3])};
   __syncthreads();
-#pragma unroll
-  for (int j = 0; j < N; ++j) f[j] = take_max ? kNegInf : 0.f;
-  for (int s = 0; s < slices; ++s) {   // the same order in every slice
-#pragma unroll
-    for (int q = 0; q < N / 4; ++q) {
-      const u32x4 o = mine[(s * (N / 4) + q) * lx + lane];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) f[4 * q + j] = take_max ? fmaxf(f[4 * q + j], u2f(o[j])) : f[4 * q + j] + u2f(o[j]);
+  float* merged = lds + slices * LX * N;
+  for (int i = int(threadIdx.y) * LX + int(threadIdx.x); i < LX * N; i += slices * LX) {
+    float r = lds[i];
+#pragma unroll 4
+    for (int s = 1; s < slices; ++s) {
+      const float o = lds[s * LX * N + i];
+      r = take_max ? fmaxf(r, o) : r + o;
     }
+    merged[i] = r;
+  }
+  __syncthreads();
+  const u32x4* got = reinterpret_cast<const u32x4*>(merged + int(threadIdx.x) * N);
+#pragma unroll
+  for (int q = 0; q < N / 4; ++q) {
+    const u32x4 o = got[q];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) f[4 * q + j] = u2f(o[j]);
   }
 }
 
@@ -215,22 +225,22 @@ struct DimColumn {
   int v, first, count;
   bool live;
   __device__ __forceinline__ DimColumn(const SoftmaxDimArgs& a, int nk) {
-    const int64_t id = int64_t(blockIdx.x) * LX + int(threadIdx.x);
+    const int64_t id = xcd_run_block<LX == 256 ? 8 : 16>(blockIdx.x, gridDim.x) * LX + int(threadIdx.x);
     live = id < a.total;
     const uint32_t i = uint32_t(live ? id : a.total - 1), o = i / uint32_t(a.run_vecs);
     v = int(i - o * uint32_t(a.run_vecs));
     base = int64_t(o) * a.dim * a.inner + vec_column<T, true>(v, int(a.inner));
-    // a slice of a whole wavefront: its entries' addresses are scalar
-    first = (LX == kWave ? __builtin_amdgcn_readfirstlane(int(threadIdx.y)) : int(threadIdx.y)) * nk;
+    // a slice of whole wavefronts: its entries' addresses are scalar
+    first = (LX >= kWave ? __builtin_amdgcn_readfirstlane(int(threadIdx.y)) : int(threadIdx.y)) * nk;
     count = min(nk, a.dim - first);        // entries of this slice, at least one
   }
 };
 
-template <typename T, int NK, int LX>
+template <typename T, int NK, int LX, bool PLAIN>
 __global__ __launch_bounds__(1024)
 void softmax_fwd_dim_kernel(SoftmaxDimArgs a) {
   constexpr int VEC = VecIO<T>::N;
-  extern __shared__ __align__(16) float shared[];   // two [slices][LX][VEC] arrays
+  extern __shared__ __align__(16) float shared[];   // [slices + 1][LX][VEC]
   const DimColumn<T, LX> c(a, NK);
   const T* xp = static_cast<const T*>(a.x) + c.base;
   u32x4 raw[NK];
@@ -247,7 +257,7 @@ void softmax_fwd_dim_kernel(SoftmaxDimArgs a) {
 #pragma unroll
     for (int j = 0; j < VEC; ++j) m[j] = max3(m[j], f[j], g[j]);
   }
-  if (a.slices > 1) slices_share<VEC>(m, shared, LX, int(threadIdx.x), a.slices, true);
+  if (a.slices > 1) slices_share<VEC, LX>(m, shared, a.slices, true);
   float base2[VEC], ml[VEC], s[VEC];
 #pragma unroll
   for (int j = 0; j < VEC; ++j) {
@@ -265,7 +275,7 @@ void softmax_fwd_dim_kernel(SoftmaxDimArgs a) {
       s[j] += k < c.count ? e : 0.f;
     }
   }
-  if (a.slices > 1) slices_share<VEC>(s, shared + a.slices * LX * VEC, LX, int(threadIdx.x), a.slices, false);
+  if (a.slices > 1) slices_share<VEC, LX>(s, shared, a.slices, false);
   if (!c.live) return;
 #pragma unroll
   for (int j = 0; j < VEC; ++j) s[j] = 1.0f / s[j];
@@ -277,16 +287,16 @@ void softmax_fwd_dim_kernel(SoftmaxDimArgs a) {
       VecIO<T>::unpack(raw[k], f);
 #pragma unroll
       for (int j = 0; j < VEC; ++j) f[j] = __builtin_amdgcn_exp2f(fmaf(f[j], base2[j], -ml[j])) * s[j];
-      store_row_vec<T, true, false>(yp + int64_t(c.first + k) * a.inner, c.v, f, int(a.inner));
+      store_row_vec<T, true, false, PLAIN>(yp + int64_t(c.first + k) * a.inner, c.v, f, int(a.inner));
     }
   }
 }
 
-template <typename T, int NK, int LX>
+template <typename T, int NK, int LX, bool PLAIN>
 __global__ __launch_bounds__(1024)
 void softmax_bwd_dim_kernel(SoftmaxDimArgs a) {
   constexpr int VEC = VecIO<T>::N;
-  extern __shared__ __align__(16) float shared[];   // [slices][LX][VEC]
+  extern __shared__ __align__(16) float shared[];   // [slices + 1][LX][VEC]
   const DimColumn<T, LX> c(a, NK);
   const T* yp = static_cast<const T*>(a.x) + c.base;
   const T* dyp = static_cast<const T*>(a.dy) + c.base;
@@ -306,7 +316,7 @@ void softmax_bwd_dim_kernel(SoftmaxDimArgs a) {
 #pragma unroll
     for (int j = 0; j < VEC; ++j) dot[j] = k < c.count ? fmaf(y[j], d[j], dot[j]) : dot[j];
   }
-  if (a.slices > 1) slices_share<VEC>(dot, shared, LX, int(threadIdx.x), a.slices, false);
+  if (a.slices > 1) slices_share<VEC, LX>(dot, shared, a.slices, false);
   if (!c.live) return;
   T* dxp = static_cast<T*>(a.out) + c.base - vec_column<T, true>(c.v, int(a.inner));
 #pragma unroll
@@ -317,7 +327,7 @@ void softmax_bwd_dim_kernel(SoftmaxDimArgs a) {
       VecIO<T>::unpack(rd[k], d);
 #pragma unroll
       for (int j = 0; j < VEC; ++j) d[j] = y[j] * (d[j] - dot[j]);
-      store_row_vec<T, true, false>(dxp + int64_t(c.first + k) * a.inner, c.v, d, int(a.inner));
+      store_row_vec<T, true, false, PLAIN>(dxp + int64_t(c.first + k) * a.inner, c.v, d, int(a.inner));
     }
   }
 }
@@ -578,14 +588,14 @@ static int softmax_lastdim_typed(SoftmaxArgs a, hipStream_t s) {
   }
 }
 
-template <typename T, bool BWD, int LX>
+template <typename T, bool BWD, int LX, bool PLAIN>
 static void launch_softmax_dim(const SoftmaxDimArgs& a, int nk, hipStream_t s) {
   const dim3 grid{unsigned((a.total + LX - 1) / LX)}, block{unsigned(LX), unsigned(a.slices)};
-  const size_t lds = a.slices > 1 ? size_t(BWD ? 1 : 2) * a.slices * LX * VecIO<T>::N * sizeof(float) : 0;
+  const size_t lds = a.slices > 1 ? size_t(a.slices + 1) * LX * VecIO<T>::N * sizeof(float) : 0;
 #define HK_DIM_CASE(N)                                                              \
   case N:                                                                           \
-    if constexpr (BWD) HK_LAUNCH((softmax_bwd_dim_kernel<T, N, LX>), grid, block, lds, s, a); \
-    else HK_LAUNCH((softmax_fwd_dim_kernel<T, N, LX>), grid, block, lds, s, a);     \
+    if constexpr (BWD) HK_LAUNCH((softmax_bwd_dim_kernel<T, N, LX, PLAIN>), grid, block, lds, s, a); \
+    else HK_LAUNCH((softmax_fwd_dim_kernel<T, N, LX, PLAIN>), grid, block, lds, s, a);     \
     break;
   profile_before(s);
   switch (nk) {
@@ -630,14 +640,31 @@ static int softmax_strided_typed(const void* x, const void* dy, void* out, int64
       a.run_vecs = int((inner + VEC - 1) / VEC);
       a.total = outer * a.run_vecs;
       // 8 entries a lane; 6 where that holds two 16-bit operands in fewer registers (8 x 21 x 263168 bf16 backward
-      // 56.1 -> 48.8 us, 16 x 150 x 16384 86.7 -> 46.5; forward 34.6 / 34.1 and 43.8 / 47.4 us), if 32 slices do then
-      const int most = std::max(BWD && VEC == 8 ? 6 : kDimVecs, int(dim + 31) / 32);
+      // 56.1 -> 48.8 us, 16 x 150 x 16384 86.7 -> 46.5; forward 34.6 / 34.1 and 43.8 / 47.4 us), if 32 slices do then.
+      // A problem that leaves most wavefront slots empty takes 2 entries a lane, in workgroups of half a wavefront's
+      // vectors (a quarter's, up to 64 slices, for the longer dimensions of the smallest): its time is one lane's chain
+      // of instructions.  GPU us, forward / backward, with 6 to 8 entries in a wavefront's and so: 4 x 65 x 355 bf16
+      // 8.6 / 7.5 and 4.4 / 3.6, 2 x 250 x 200 fp32 9.4 / 10.7 and 5.8 / 5.9, 3 x 57 x 5877 fp32 5.8 / 6.3 and 4.5 / 4.4,
+      // 4 x 100 x 10000 bf16 10.1 / 8.0 and 7.8 / 6.8; at 2 x 128 x 16384 fp32 they meet, 8.9 / 11.1 and 9.9 / 10.8.
+      const bool few = a.total <= cus * 64 && a.total * dim <= cus * 3072;
+      const int lx = few && a.total <= cus * 16 && dim > 64 ? 16 : 32, fewest = int((dim + 1024 / lx - 1) / (1024 / lx));
+      const int most = std::max(few ? 2 : BWD && VEC == 8 ? 6 : kDimVecs, fewest);
       const int slices = int((dim + most - 1) / most), nk = int((dim + slices - 1) / slices);
       a.slices = int((dim + nk - 1) / nk);
       if (a.total <= 0x7fffffffLL) {
-        // up to 16 slices of a wavefront each, up to 32 of half a wavefront
-        if (a.slices <= 16) launch_softmax_dim<T, BWD, 64>(a, nk, s);
-        else launch_softmax_dim<T, BWD, 32>(a, nk, s);
+        // fp32 planes that fill the device many times over, up to 32 entries: runs of 2 KiB and 4 KiB of an entry per
+        // workgroup instead of 1 KiB share fewer lines (8 x 21 x 263169 forward 71.8 / 69.7 / 69.0, backward 106 / 103 /
+        // 96 us with runs of 64 / 128 / 256 lanes; 8 x 21 x 263168 62.9 / 64.0 / 65.5 and 93.1 / 93.1 / 90.3); not 16-bit
+        // ones (8 x 21 x 263169 35.3 / 37.8 / 48.1 and 50.3 / 51.0 / 55.8)
+        const bool wide = VEC == 4 && a.slices <= 4 && a.total >= cus * 2048;
+        // PLAIN: 16-bit entries in runs of 1 KiB, and the few, are stored through the cache (8 x 21 x 263170 bf16 35.5 /
+        // 48.8 -> 33.9 / 44.4, 4 x 65 x 355 5.9 / 5.1 -> 5.4 / 4.4; fp32 70.8 / 104 -> 73.2 / 112, and 16-bit ones in runs of
+        // 512 bytes, 16 x 150 x 16384, 37.2 / 42.3 -> 39.9 / 47.1 us, are not)
+        if (lx == 16) launch_softmax_dim<T, BWD, 16, true>(a, nk, s);
+        else if (few) launch_softmax_dim<T, BWD, 32, true>(a, nk, s);
+        else if (a.slices > 16) launch_softmax_dim<T, BWD, 32, false>(a, nk, s);
+        else if (wide) launch_softmax_dim<T, BWD, (VEC == 4 ? (BWD ? 256 : 128) : 64), VEC == 8>(a, nk, s);
+        else launch_softmax_dim<T, BWD, 64, VEC == 8>(a, nk, s);
         return launch_check("softmax_dim_kernel");
       }
     }

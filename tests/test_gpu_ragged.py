@@ -270,6 +270,39 @@ def test_cross_entropy_of_lowest_values(hk, cuda, dtype, cols):
     helpers.assert_close(dx[ok], p[ok].cpu().numpy(), dtype, "dlogits")
 
 
+# one of every launch of the kernels above: many fp32 planes (runs of 128 and 256 lanes), 16-bit ones with blocks left over
+# after the runs that stay on one XCD, more than 16 slices, and few positions with up to and more than 64 entries
+@pytest.mark.parametrize("dtype,outer,dim,inner", [("fp32", 1, 9, 4 * 524288 + 3), ("fp32", 2, 32, 1048577), ("bf16", 8, 21, 40961),
+                                                   ("fp16", 8, 21, 40960), ("bf16", 16, 150, 8191), ("fp32", 4, 129, 8003),
+                                                   ("bf16", 4, 65, 355), ("fp32", 2, 250, 203), ("fp16", 5, 256, 15),
+                                                   ("bf16", 5, 8, 4111), ("fp32", 3, 57, 5877), ("bf16", 2, 17, 8)])
+def test_softmax_dim_launches(hk, cuda, dtype, outer, dim, inner):
+    import torch
+    dt = {"fp32": torch.float32, "bf16": torch.bfloat16, "fp16": torch.float16}[dtype]
+    gen = torch.Generator(device=cuda).manual_seed(dim * 1000003 + inner)
+    guard = lambda: torch.full((outer * dim * inner + 2 * GUARD,), 7.0, dtype=dt, device=cuda)
+    x, dy = (torch.randn(outer, dim, inner, generator=gen, device=cuda).to(dt) for _ in range(2))
+    yb, db = guard(), guard()
+    y, dx = (b[GUARD:-GUARD].view(outer, dim, inner) for b in (yb, db))
+    hk.softmax_fwd(x, y, 1)
+    hk.softmax_bwd(y, dy, dx, 1)
+    torch.cuda.synchronize()
+    assert bool((yb[:GUARD] == 7).all() and (yb[-GUARD:] == 7).all() and (db[:GUARD] == 7).all() and (db[-GUARD:] == 7).all())
+    # every element against 64 bits: half a unit in the last place of the stored type (8, 11 and 24 bits), and roundings of
+    # 2^-24: 12 for the exponents (arguments up to 16, half a unit of which is 16 of these, times log 2) of the element
+    # and of the sum, dim additions, exp2 and the quotient; dx carries the dot product's error, dim roundings at most
+    unit = {"fp32": 2.0 ** -24, "bf16": 2.0 ** -8, "fp16": 2.0 ** -11}[dtype]
+    for o in range(outer):
+        want = torch.softmax(x[o].double(), 0)
+        assert bool(((y[o].double() - want).abs() <= want * (unit + (28 + dim) * 2.0 ** -24) + 2.0 ** -25 * (dtype == "fp16")).all()), o
+        yo, do = y[o].double(), dy[o].double()
+        dot = (yo * do).sum(0, keepdim=True)
+        want = yo * (do - dot)
+        terms = yo * (do.abs() + (yo * do.abs()).sum(0, keepdim=True))
+        assert bool(((dx[o].double() - want).abs() <= want.abs() * unit + terms * (dim + 4) * 2.0 ** -24 +
+                     2.0 ** -25 * (dtype == "fp16")).all()), o
+
+
 def _norm_lengths(dtype):
     vec = 16 // ES[dtype]
     out = {v * vec + k for v in (1, 2, 8, 16, 32, 64, 65, 128, 192, 256, 300, 512, 1024) for k in (0, 1, vec - 1)}
