@@ -8,8 +8,8 @@
 // writes the row once.  Rows whose label equals the ignored index are not read
 // at all: loss 0 / a zero gradient row is written.
 //
-// Sparse labels take rows of any length and alignment this way (see RowSpan); 16-bit rows of 32768 to 65536 columns are
-// kept packed (sce_packed_kernel), longer ones are streamed (sce_long_kernel).
+// Sparse labels take rows of any length and alignment this way (see RowSpan); 16-bit rows of 32768 to 98304 columns keep
+// a part in LDS (RowTail, sce_packed_kernel), longer ones are streamed (sce_long_kernel).
 #include "hk_common.h"
 
 #include <algorithm>
@@ -248,10 +248,39 @@ __device__ __forceinline__ void sce_store_zero_row(T* dxr, int cols, int t, int 
   span.store_edge(dxr, 0.f);
 }
 
-template <typename T, int NV, bool WAVE_ROW, bool RAGGED>
+// The vectors of a row past NV per thread, kept in LDS as they were loaded: [rounds][threads].  A wavefront reads back what
+// it loaded itself (directly, through no register), so there is no barrier; `arrived` waits for it.
+template <typename T, int NV>
+struct RowTail {
+  const RowSpan<T, true>& span;
+  u32x4* lds;
+  int t, tpr;
+  __device__ __forceinline__ void load(const T* row) const {
+    for (int v = NV * tpr, k = 0; v < span.nvec; v += tpr, k += tpr) {
+      if (v + t < span.nvec) {   // lane i's 16 bytes go to the wavefront's address + 16 i
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(row + span.head + (v + t) * span.N),
+                                         (__attribute__((address_space(3))) void*)(lds + k + wave_index() * kWave), 16, 0,
+                                         kBufStream);
+      }
+    }
+  }
+  static __device__ __forceinline__ void arrived() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+  // f(unpacked elements, index of the vector) for this thread's share
+  template <typename F>
+  __device__ __forceinline__ void each(F&& f) const {
+    for (int v = NV * tpr + t, k = t; v < span.nvec; v += tpr, k += tpr) {
+      float e[RowSpan<T, true>::N];
+      VecIO<T>::unpack(lds[k], e);
+      f(e, v);
+    }
+  }
+};
+
+template <typename T, int NV, bool WAVE_ROW, bool RAGGED, bool TAIL = false>
 __global__ __launch_bounds__(WAVE_ROW ? 256 : 1024, (sce_min_waves<T, NV>(WAVE_ROW)))
 void sce_sparse_bwd_kernel(SceArgs a) {
   constexpr int VEC = VecIO<T>::N;
+  extern __shared__ __align__(16) u32x4 tail_lds[];   // TAIL: the row's vectors past NV per thread
   __shared__ float red[kMaxWaves * 2];
   int tpr, t, nwaves;
   int64_t i0, row;
@@ -272,6 +301,8 @@ void sce_sparse_bwd_kernel(SceArgs a) {
   for (int i = 0; i < NV; ++i)
     raw[i] = span.template load<false>(xr, i * tpr + t, (i + 1) * tpr <= span.nvec);
   [[maybe_unused]] float edge = span.load_edge(xr);
+  const auto tail = [&] { if constexpr (TAIL) return RowTail<T, NV>{span, tail_lds, t, tpr}; else return 0; }();
+  if constexpr (TAIL) tail.load(xr);
   const float g = sce_row_grad<T, float>(a, row);
   float e[NV * VEC];
 #pragma unroll
@@ -280,6 +311,13 @@ void sce_sparse_bwd_kernel(SceArgs a) {
   float m = RAGGED ? max3(edge, e[0], e[1]) : fmaxf(e[0], e[1]);
 #pragma unroll
   for (int k = 2; k < NV * VEC; k += 2) m = max3(m, e[k], e[k + 1]);
+  if constexpr (TAIL) {
+    tail.arrived();
+    tail.each([&](const float* f, int) {
+#pragma unroll
+      for (int j = 0; j < VEC; j += 2) m = max3(m, f[j], f[j + 1]);
+    });
+  }
   const float ml = log2_of_max(m);
   // four independent chains, as in the forward kernel
   float s4[4] = {0.f, 0.f, 0.f, 0.f};
@@ -291,6 +329,12 @@ void sce_sparse_bwd_kernel(SceArgs a) {
   if constexpr (RAGGED) {
     edge = __builtin_amdgcn_exp2f(fmaf(edge, kLog2e, -ml));
     s4[0] += edge;
+  }
+  if constexpr (TAIL) {
+    tail.each([&](const float* f, int) {
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) s4[j & 3] += __builtin_amdgcn_exp2f(fmaf(f[j], kLog2e, -ml));
+    });
   }
   const float s = (s4[0] + s4[1]) + (s4[2] + s4[3]);
   MaxSumTuple p;
@@ -317,16 +361,29 @@ void sce_sparse_bwd_kernel(SceArgs a) {
       span.store(dxr, v, &e[i * VEC]);
     }
   }
+  if constexpr (TAIL) {
+    const float inv = g / p.v[1];
+    tail.each([&](float* f, int v) {
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) f[j] = __builtin_amdgcn_exp2f(fmaf(f[j], kLog2e, -p.v[0])) * inv;
+      if (v == place.vec) {
+#pragma unroll
+        for (int j = 0; j < VEC; ++j)
+          if (j == place.element) f[j] -= g;
+      }
+      span.store(dxr, v, f);
+    });
+  }
   if constexpr (RAGGED) span.store_edge(dxr, edge * scale - (span.edge == lab ? g : 0.f));
 }
 
 // ------------------------------- long rows ---------------------------------
-// Sparse labels, rows that do not fit a workgroup's registers (65536 16-bit elements, 32768 fp32): the workgroup streams the row, kLongVecs vectors per
-// thread and step, and every thread keeps a running (maximum, sum of exponentials) that it re-bases once per step.
+// Sparse labels, rows that do not fit a workgroup's registers (32768 fp32 elements) and LDS (98304 16-bit ones): the workgroup
+// streams the row, kLongVecs vectors per thread and step, and every thread keeps a running (maximum, sum of exponentials) that it re-bases once per step.
 // The backward reads the row a second time, from its end, so that what was read last is found in the nearest cache
 // (1024 x 128256 bf16 116 -> 111 us), and is bound by what that second read costs: 1024 x 128256 bf16 679 us by
 // elements -> 111 us (4.7 TB/s of row and gradient), forward 307 -> 48 us (5.5 TB/s).  Every step has as many threads
-// as its share of the row needs (4096 x 50257 bf16, which sce_packed_kernel takes now: 160 and 83 us, with 1024
+// as its share of the row needs (4096 x 50257 bf16, which has kernels of its own now: 160 and 83 us, with 1024
 // throughout 167 and 86 us).
 constexpr int kLongThreads = 1024;
 constexpr int kLongVecs = 4;
@@ -423,13 +480,13 @@ void sce_long_kernel(SceArgs a) {
 }
 
 // --------------------------- rows kept as loaded ---------------------------
-// Sparse labels, 16-bit rows of more than kLongVecs and up to kPackedVecs vectors per thread of a 1024-thread workgroup:
-// the vectors stay in registers as they were loaded and are unpacked three times (maximum, sum, gradient), so that twice
-// the elements fit the 64 registers at which two such workgroups share a compute unit (43 forward, 56 backward), and the
-// row is read once.  Bound by HBM and by the two rows that a compute unit has under way, whose loads, arithmetic and
-// stores overlap less than four would.  Against sce_long_kernel, bf16, forward / backward: 4096 x 50257 83.9 / 164.5 ->
-// 78.3 / 152.9 us (5.4 TB/s backward), x 50304 81.6 / 159.7 -> 78.0 / 146.8, x 65536 88.5 / 202.5 -> 88.6 / 182.4,
-// x 33000 49.2 / 106.6 -> 47.0 / 99.6.
+// Sparse labels, 16-bit rows longer than 32768 columns: kPackedVecs vectors per thread stay in registers as they were loaded
+// and are unpacked once per pass (maximum, sum, gradient), the rest of the row is kept in LDS (RowTail), so that the row is
+// read once and four, three or two rows share a compute unit (pick_sce_long_shape; 64 registers or fewer: 46 forward, 58
+// backward).  Bound by HBM in the forward, and by how far the loads, the arithmetic (two exponentials an element) and the
+// stores of two rows overlap in the backward.  us, forward / backward, streamed by sce_long_kernel and so: 4096 x 50257 bf16
+// 95 / 168 and 65 / 145 (sce_sparse_bwd_kernel), 2500 x 80000 74 / 164 and 68 / 145, 4096 x 65536 102 / 200 and 86 / 181
+// (sce_sparse_bwd_kernel).
 constexpr int kPackedVecs = 8;
 
 // The compiler would keep the unpacked elements from one pass to the next otherwise: twice the registers.
@@ -443,6 +500,7 @@ template <typename T, bool BWD>
 __global__ __launch_bounds__(1024, 8)
 void sce_packed_kernel(SceArgs a) {
   constexpr int VEC = VecIO<T>::N, NV = kPackedVecs;
+  extern __shared__ __align__(16) u32x4 tail_lds[];   // the vectors past NV per thread
   __shared__ float red[kMaxWaves * 3];
   const int t = int(threadIdx.x), tpr = int(blockDim.x), nwaves = tpr >> 6;
   const int64_t i0 = blockIdx.x, row = dense_row_index(i0, a.rn);
@@ -460,6 +518,8 @@ void sce_packed_kernel(SceArgs a) {
   for (int i = 0; i < NV; ++i)
     raw[i] = span.template load<false>(xr, i * tpr + t, (i + 1) * tpr <= span.nvec);
   const float edge = span.load_edge(xr);
+  const RowTail<T, NV> tail{span, tail_lds, t, tpr};
+  tail.load(xr);
   float m = edge;
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
@@ -468,6 +528,11 @@ void sce_packed_kernel(SceArgs a) {
 #pragma unroll
     for (int j = 0; j < VEC; j += 2) m = max3(m, f[j], f[j + 1]);
   }
+  tail.arrived();
+  tail.each([&](const float* f, int) {
+#pragma unroll
+    for (int j = 0; j < VEC; j += 2) m = max3(m, f[j], f[j + 1]);
+  });
   const float ml = log2_of_max(m);
   unpack_again(raw);
   float s4[4] = {__builtin_amdgcn_exp2f(fmaf(edge, kLog2e, -ml)), 0.f, 0.f, 0.f};
@@ -478,6 +543,10 @@ void sce_packed_kernel(SceArgs a) {
 #pragma unroll
     for (int j = 0; j < VEC; ++j) s4[j & 3] += __builtin_amdgcn_exp2f(fmaf(f[j], kLog2e, -ml));
   }
+  tail.each([&](const float* f, int) {
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) s4[j & 3] += __builtin_amdgcn_exp2f(fmaf(f[j], kLog2e, -ml));
+  });
   const float s = (s4[0] + s4[1]) + (s4[2] + s4[3]);
   if constexpr (!BWD) {
     MaxSumMaxTuple p;
@@ -497,6 +566,16 @@ void sce_packed_kernel(SceArgs a) {
     }
     const auto place = span.place_of(lab);
     const float ML = p.v[0], scale = g / p.v[1];
+    const auto put = [&](float* o, int v) {
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) o[j] = __builtin_amdgcn_exp2f(fmaf(o[j], kLog2e, -ML)) * scale;
+      if (v == place.vec) {
+#pragma unroll
+        for (int j = 0; j < VEC; ++j)
+          if (j == place.element) o[j] -= g;
+      }
+      span.store(dxr, v, o);
+    };
     unpack_again(raw);
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
@@ -504,16 +583,10 @@ void sce_packed_kernel(SceArgs a) {
       if (v < span.nvec) {
         float o[VEC];
         VecIO<T>::unpack(raw[i], o);
-#pragma unroll
-        for (int j = 0; j < VEC; ++j) o[j] = __builtin_amdgcn_exp2f(fmaf(o[j], kLog2e, -ML)) * scale;
-        if (v == place.vec) {
-#pragma unroll
-          for (int j = 0; j < VEC; ++j)
-            if (j == place.element) o[j] -= g;
-        }
-        span.store(dxr, v, o);
+        put(o, v);
       }
     }
+    tail.each(put);
     span.store_edge(dxr, __builtin_amdgcn_exp2f(fmaf(edge, kLog2e, -ML)) * scale - (span.edge == lab ? g : 0.f));
   }
 }
@@ -730,16 +803,52 @@ static bool pick_sce_shape(int nvec, int max_nv_wave, int max_nv, int* threads, 
     return true;
   }
   // long rows, measured at 32000 bf16 columns: the widest vector count the
-  // kernel is built for wins (512 threads x 8 vectors beat 1024 x 4 forward)
+  // kernel is built for wins (512 threads x 8 vectors beat 1024 x 4 forward).  Fewer than 256 threads, three wavefronts
+  // that is, are still better than half the vectors in more of them, most of all where those leave a wavefront idle: us at
+  // 8000 x 4100 bf16 forward 192 x 4 15.6, 320 x 2 20.7 (128 x 8 15.8), 6000 x 6144 14.0 and 19.5, 8000 x 2464 fp32 13.8
+  // and 18.6; backward, 10326 x 2112 bf16, 192 x 2 16.9, 320 x 1 26.8, 8000 x 4100 192 x 4 24.6, 320 x 2 27.4.
   for (int n = max_nv; n >= 1; n >>= 1) {
     int t = ((nvec + n - 1) / n + 63) / 64 * 64;
-    if (t <= 1024 && (t >= 256 || n == 1)) { *threads = t; *nv = n; return true; }
+    if (t <= 1024 && (t >= (n > 4 ? 256 : 192) || n == 1)) { *threads = t; *nv = n; return true; }
   }
   for (int n = 1; n <= max_nv; n <<= 1) {
     int t = ((nvec + n - 1) / n + 63) / 64 * 64;
     if (t <= 1024) { *threads = t; *nv = n; return true; }
   }
   return false;
+}
+
+// 16-bit rows with a tail in LDS (threads 0: none).  The forward keeps four rows under way per compute unit where that
+// fits (512 threads and up to 39 KiB of LDS each), then three, then two; the backward, whose reads and writes do not like
+// company, two (4096 x 50257 bf16, rows per compute unit 2 / 3 / 4: forward 78.3 / 69.0 / 65, backward 152 / 154 / 163 us),
+// with the exponentials of 4 vectors per thread in registers as far as two tails of 64 KiB reach (against packed rows x 33000
+// 102 -> 94, x 50257 152 -> 145, x 65536 183 -> 181 us).  Longer than 98304 columns: streamed (x 80000, 2500 rows, streamed
+// 74 / 164, so 68 / 145 us).  fp32 rows, 4096 x 32000 and x 20001, gain nothing: 175 / 178 and 116 / 113 us.
+struct SceLongShape {
+  int threads;
+  bool packed;        // sce_packed_kernel, else sce_sparse_bwd_kernel
+  size_t lds_bytes;
+};
+template <bool BWD>
+static SceLongShape pick_sce_long_shape(int nvec) {
+  SceLongShape l{0, false, 0};
+  if (nvec <= 4 * 1024) return l;
+  size_t per_cu = 0, per_block = 0;
+  device_lds_bytes(&per_cu, &per_block);
+  per_block = std::min<size_t>(per_block, 65536);
+  const size_t red = 512;   // the reduction's own array
+  const auto fits = [&](int vectors, int rows_per_cu) {
+    l.lds_bytes = size_t(std::max(0, vectors) + 63) / 64 * 64 * 16;   // a wavefront's share is whole
+    return l.lds_bytes <= per_block - red && l.lds_bytes + red <= per_cu / size_t(rows_per_cu);
+  };
+  if (BWD && fits(nvec - 4 * 1024, 2)) { l.threads = 1024; return l; }
+  l.packed = true;
+  for (int rows = BWD ? 2 : 4; rows >= 2; --rows) {
+    const int most = rows == 4 ? 512 : rows == 3 ? 640 : 1024;   // 32 wavefronts in all
+    const int threads = std::min(most, ((nvec + kPackedVecs - 1) / kPackedVecs + 63) / 64 * 64);
+    if (fits(nvec - kPackedVecs * threads, rows)) { l.threads = threads; return l; }
+  }
+  return l;
 }
 
 // MODE as in sce_generic_kernel
@@ -777,9 +886,10 @@ static int sce_typed(SceArgs a, hipStream_t s) {
                       (MODE == 0 || MODE == 2 || (aligned16(a.out) && steps_ok(a.out_pitch, a.out_lv))) &&
                       steps_ok(a.x_pitch, a.x_lv) && (MODE < 2 || steps_ok(a.lab_pitch, a.lab_lv));
   a.nvec = (a.cols + VEC - 1) / VEC;
-  // sparse forward only keeps the packed row; the others keep 32 floats or two rows
+  // sparse forward only keeps the packed row; the others keep 32 floats or two rows, in a wavefront 16 floats of fp32
+  // (10000 x 1634 backward 64 x 8 25.5, 256 x 2 23.4; x 1100 17.5, 192 x 2 16.2 us)
   const int max_nv = (MODE == 0) ? 8 : 32 / VEC;
-  const int max_nv_wave = (MODE == 0) ? 8 : 32 / VEC;
+  const int max_nv_wave = (MODE == 0) ? 8 : 4;
   int threads = 0, nv = 0;
   const bool shaped = pick_sce_shape(a.nvec, max_nv_wave, max_nv, &threads, &nv);
   const dim3 levels{unsigned(a.n0), unsigned(a.n1), unsigned(a.n2)};
@@ -792,16 +902,18 @@ static int sce_typed(SceArgs a, hipStream_t s) {
     return launch_sce_nv<T, MODE, false, RAGGED>(a, nv, levels, dim3{unsigned(threads)}, s);
   };
   if constexpr (MODE < 2 && VEC == 8) {
-    // The forward with 64 floats a thread in more than 512 threads is slower (4096 x 50304 bf16 94 us, kept packed 78,
-    // x 65536 105 against 89; 32000 columns, 512 threads, stay with it: 155 us, streamed 230), the backward does not fit
-    // that.  fp32 vectors have nothing to unpack: 4096 x 32000 78.0 / 177.7 us against 79.0 / 177.4, x 20001 48.3 / 114.9
-    // against 48.5 / 116.2, so they stay with the kernels above.
-    if (a.nvec > kLongVecs * 1024 && a.nvec <= kPackedVecs * 1024 && tune_get(TUNE_SCE_THREADS) <= 0) {
-      threads = ((a.nvec + kPackedVecs - 1) / kPackedVecs + 63) / 64 * 64;
+    const SceLongShape l = pick_sce_long_shape<MODE == 1>(a.nvec);
+    if (l.threads > 0 && tune_get(TUNE_SCE_THREADS) <= 0) {
+      const dim3 block{unsigned(l.threads)};
       profile_before(s);
-      HK_LAUNCH((sce_packed_kernel<T, MODE == 1>), levels, dim3(unsigned(threads)), 0, s, a);
+      if constexpr (MODE == 1) {
+        if (l.packed) HK_LAUNCH((sce_packed_kernel<T, true>), levels, block, l.lds_bytes, s, a);
+        else HK_LAUNCH((sce_sparse_bwd_kernel<T, 4, false, true, true>), levels, block, l.lds_bytes, s, a);
+      } else {
+        HK_LAUNCH((sce_packed_kernel<T, false>), levels, block, l.lds_bytes, s, a);
+      }
       profile_after(s);
-      return launch_check("sce_packed_kernel");
+      return launch_check("sce kernel");
     }
   }
   if (vec_ok && shaped) return launch(std::false_type{});

@@ -594,3 +594,35 @@ def test_shard_statistics_keep_a_nan(hk, cuda, dtype, cols):
     hk.vocab_parallel_ce_stats(x, torch.zeros(3, dtype=torch.int64, device=cuda), stats, 0, -100)
     torch.cuda.synchronize()
     assert float(stats[1, 0]) == 0.0 and bool(torch.isnan(stats[1, 1:]).all()), stats
+
+
+# 16-bit rows with a part in LDS: the most vectors of four, three and two rows per compute unit (6592, 8448, 12224) and of a
+# gradient row with exponentials in registers (8128), one more each, and the first rows past registers alone (4097)
+@pytest.mark.parametrize("dtype", ["bf16", "fp16"])
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("vectors", [4097, 4160, 6592, 6593, 8128, 8129, 8448, 8449, 12224, 12225])
+def test_cross_entropy_rows_with_a_tail(hk, cuda, dtype, shift, vectors):
+    import torch
+    rows = 5
+    for cols in (8 * vectors, 8 * vectors - 7):
+        pitch = cols + (0 if shift == 0 else 5)
+        x = helpers.draw(9100 + cols, (rows, cols), dtype=dtype)
+        _, tx = _placed(cuda, x, dtype, shift, pitch)
+        lab = torch.tensor([0, cols - 1, -100, 32768, cols - 9], device=cuda)     # the first and last column, one in the tail
+        g = torch.tensor([1.0, -2.0, 3.0, 0.5, 1.5], dtype=tx.dtype, device=cuda)
+        loss = torch.empty(rows, dtype=tx.dtype, device=cuda)
+        db, dx = _placed(cuda, x, dtype, shift, pitch, 3.0)
+        hk.sce_sparse_fwd(tx, lab, loss, -100)
+        hk.sce_sparse_bwd(tx, lab, g, dx, -100)
+        torch.cuda.synchronize()
+        p = torch.softmax(tx.double(), -1)
+        want = torch.logsumexp(tx.double(), -1) - tx.double().gather(1, lab.clamp(min=0)[:, None])[:, 0]
+        p[torch.arange(rows, device=cuda), lab.clamp(min=0)] -= 1
+        want[2] = 0
+        p[2] = 0
+        helpers.assert_close(loss, want.cpu().numpy(), dtype, "loss %d" % cols)
+        helpers.assert_close(dx.contiguous(), (p * g.double()[:, None]).cpu().numpy(), dtype, "dlogits %d" % cols)
+        assert _guards_untouched(db, dx), cols
+        hk.sce_sparse_bwd(tx, lab, g, tx, -100)     # in place
+        torch.cuda.synchronize()
+        assert torch.equal(tx.contiguous(), dx.contiguous()), cols
