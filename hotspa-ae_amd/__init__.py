@@ -1,13 +1,15 @@
 """MI355X-native row-wise operator kernels behind Hetu's kernel interface.
 
-The compute lives in two native libraries built in-tree by ``build.py``:
+The compute lives in native libraries built in-tree by ``build.py``:
 
 * ``lib/libhk_rowwise.so``   — C-ABI device layer + hand-written gfx950 kernels
   (``include/hk_rowwise.h``);
 * ``lib/libhetu_rowwise.so`` — C++ host layer with Hetu's own types and kernel
   entry points (``hetu::impl::LayerNormCuda`` ...).
 
-This Python package is only the thin ctypes harness used by the tests and the
+* ``lib/hk_call.so``          — the CPython binding of both.
+
+This Python package is only the thin harness used by the tests and the
 benchmark: it loads the libraries and passes raw device pointers.  There is no
 CPU fallback: if the library is missing, loading fails with an error.
 

@@ -1,4 +1,5 @@
-"""ctypes bindings of include/hk_rowwise.h operating on torch CUDA tensors.
+"""Bindings of include/hk_rowwise.h operating on torch CUDA tensors: the operators that programs call in every step
+through lib/hk_call.so, the others through ctypes.
 
 torch is used for device memory and streams only; every computation goes
 through the C-ABI entry points.
@@ -63,10 +64,40 @@ def check(rc):
         raise HkError(rc, lib().hk_last_error().decode("utf-8", "replace"))
 
 
+_CALL = os.path.join(_HERE, "lib", "hk_call.so")
+_call = None
+_codes = None
+
+
+def _dtype_codes():
+    global _codes
+    if _codes is None:
+        import torch
+        _codes = {torch.float16: 5, torch.float32: 6, torch.float64: 7, torch.bfloat16: 8, torch.int64: 4,
+                  torch.int32: 3, torch.int16: 2, torch.int8: 1, torch.uint8: 0, torch.bool: 9}
+    return _codes
+
+
+def native():
+    """hk_call.so: entry points that take tensors and numbers as they are; raises if it has not been built."""
+    global _call
+    if _call is None:
+        if not os.path.exists(_CALL):
+            raise HkError(-100, "native library %s is missing: run __graft_entry__.build() first" % _CALL)
+        import importlib.util
+        import torch
+        lib()
+        spec = importlib.util.spec_from_file_location("hk_call", _CALL)
+        call = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(call)
+        call.setup(_dtype_codes(), lambda: torch.cuda.current_stream().cuda_stream,
+                   getattr(torch._C, "_cuda_getDevice", None), getattr(torch._C, "_cuda_getCurrentRawStream", None))
+        _call = call
+    return _call
+
+
 def dtype_code(t):
-    import torch
-    return {torch.float16: 5, torch.float32: 6, torch.float64: 7, torch.bfloat16: 8, torch.int64: 4,
-            torch.int32: 3, torch.int16: 2, torch.int8: 1, torch.uint8: 0, torch.bool: 9}[t.dtype]
+    return (_codes or _dtype_codes())[t.dtype]
 
 
 def torch_dtype(name):
@@ -195,9 +226,10 @@ def _multi_level(tensors):
 
 
 def layer_norm_fwd(x, gamma, beta, y, mean, stat, eps, stat_kind=HK_STAT_RSTD, stream=None):
-    rows = x.numel() // x.shape[-1] if x.numel() else 0
-    cols = x.shape[-1]
-    lv = _multi_level([x, y])
+    n = _call or native()
+    rows, cols = n.rows_cols(x)
+    dense = n.dense(x, y)
+    lv = None if dense else _multi_level([x, y])
     if lv is not None:
         counts, (xs, ys) = lv
         check(lib().hk_layer_norm_fwd_strided_rows(dtype_code(x), _ptr(x), _steps(xs), _ptr(gamma), _ptr(beta), _ptr(y),
@@ -207,11 +239,9 @@ def layer_norm_fwd(x, gamma, beta, y, mean, stat, eps, stat_kind=HK_STAT_RSTD, s
                                                    ctypes.c_float(eps),
                                                    stream if stream is not None else current_stream()))
         return
-    check(lib().hk_layer_norm_fwd_pitched(dtype_code(x), _ptr(x), _i64(_pitch(x, cols)), _ptr(gamma), _ptr(beta),
-                                          _ptr(y), _i64(_pitch(y, cols)), _ptr(mean), _ptr(stat),
-                                          dtype_code(mean if mean is not None else stat), ctypes.c_int(stat_kind),
-                                          _i64(rows), _i64(cols), ctypes.c_float(eps),
-                                          stream if stream is not None else current_stream()))
+    xp, yp = (cols, cols) if dense else (_pitch(x, cols), _pitch(y, cols))
+    check(n.hk_layer_norm_fwd_pitched(dtype_code(x), x, xp, gamma, beta, y, yp, mean, stat,
+                                      dtype_code(mean if mean is not None else stat), stat_kind, rows, cols, eps, stream))
 
 
 def norm_bwd_workspace_bytes(dtype, rows, cols):
@@ -229,12 +259,13 @@ def _workspace(nbytes, device):
 
 def layer_norm_bwd(dy, x_or_y, gamma, beta, mean, stat, dx, dgamma, dbeta, eps, stat_kind=HK_STAT_RSTD,
                    memory_efficient=False, clamp_gamma=False, workspace=None, stream=None):
-    cols = dy.shape[-1]
-    rows = dy.numel() // cols if dy.numel() else 0
+    n = _call or native()
+    rows, cols = n.rows_cols(dy)
     if workspace is None:
         workspace = _workspace(norm_bwd_workspace_bytes(dtype_code(dy), rows, cols), dy.device)
     wsb = 0 if workspace is None else workspace.numel() * workspace.element_size()
-    lv = _multi_level([dy, x_or_y, dx])
+    dense = n.dense(dy, x_or_y, dx)
+    lv = None if dense else _multi_level([dy, x_or_y, dx])
     if lv is not None:
         counts, (dys, xs, dxs) = lv
         check(lib().hk_layer_norm_bwd_strided_rows(dtype_code(dy), _ptr(dy), _steps(dys), _ptr(x_or_y), _steps(xs),
@@ -245,21 +276,19 @@ def layer_norm_bwd(dy, x_or_y, gamma, beta, mean, stat, dx, dgamma, dbeta, eps, 
                                                    _ptr(workspace), ctypes.c_size_t(wsb),
                                                    stream if stream is not None else current_stream()))
         return workspace
-    check(lib().hk_layer_norm_bwd_pitched(dtype_code(dy), _ptr(dy), _i64(_pitch(dy, cols)), _ptr(x_or_y),
-                                          _i64(_pitch(x_or_y, cols)), _ptr(gamma), _ptr(beta), _ptr(mean),
-                                          _ptr(stat), dtype_code(stat), ctypes.c_int(stat_kind), _ptr(dx),
-                                          _i64(_pitch(dx, cols)), _ptr(dgamma), _ptr(dbeta), _i64(rows), _i64(cols),
-                                          ctypes.c_float(eps), ctypes.c_int(int(memory_efficient)),
-                                          ctypes.c_int(int(clamp_gamma)), _ptr(workspace), ctypes.c_size_t(wsb),
-                                          stream if stream is not None else current_stream()))
+    dyp, xp, dxp = (cols,) * 3 if dense else [_pitch(t, cols) for t in (dy, x_or_y, dx)]
+    check(n.hk_layer_norm_bwd_pitched(dtype_code(dy), dy, dyp, x_or_y, xp, gamma, beta, mean, stat, dtype_code(stat),
+                                      stat_kind, dx, dxp, dgamma, dbeta, rows, cols, eps, memory_efficient, clamp_gamma,
+                                      workspace, wsb, stream))
     return workspace
 
 
 def dropout_add_ln_fwd(x0, residual, gamma, beta, z, x_out, mu, rsigma, eps, is_rms, stream=None):
-    cols = x0.shape[-1]
-    rows = x0.numel() // cols if x0.numel() else 0
+    n = _call or native()
+    rows, cols = n.rows_cols(x0)
     rtype = dtype_code(residual) if residual is not None else dtype_code(x0)
-    lv = _multi_level([x0, residual, z, x_out])
+    dense = n.dense(x0, residual, z, x_out)
+    lv = None if dense else _multi_level([x0, residual, z, x_out])
     if lv is not None:
         counts, (xs, rs_, zs, xos) = lv
         check(lib().hk_dropout_add_ln_fwd_strided_rows(dtype_code(x0), rtype, dtype_code(gamma), _ptr(x0), _steps(xs),
@@ -269,22 +298,20 @@ def dropout_add_ln_fwd(x0, residual, gamma, beta, z, x_out, mu, rsigma, eps, is_
                                                        ctypes.c_int(int(is_rms)),
                                                        stream if stream is not None else current_stream()))
         return
-    check(lib().hk_dropout_add_ln_fwd_pitched(dtype_code(x0), rtype, dtype_code(gamma), _ptr(x0),
-                                              _i64(_pitch(x0, cols)), _ptr(residual), _i64(_pitch(residual, cols)),
-                                              _ptr(gamma), _ptr(beta), _ptr(z), _i64(_pitch(z, cols)), _ptr(x_out),
-                                              _i64(_pitch(x_out, cols)), _ptr(mu), _ptr(rsigma), _i64(rows),
-                                              _i64(cols), ctypes.c_float(eps), ctypes.c_int(int(is_rms)),
-                                              stream if stream is not None else current_stream()))
+    xp, rp, zp, op = (cols,) * 4 if dense else [_pitch(t, cols) for t in (x0, residual, z, x_out)]
+    check(n.hk_dropout_add_ln_fwd_pitched(dtype_code(x0), rtype, dtype_code(gamma), x0, xp, residual, rp, gamma, beta, z, zp,
+                                          x_out, op, mu, rsigma, rows, cols, eps, is_rms, stream))
 
 
 def dropout_add_ln_bwd(dz, dx_in, x, mu, rsigma, gamma, dx0, dresidual, dgamma, dbeta, is_rms,
                        workspace=None, stream=None):
-    cols = x.shape[-1]
-    rows = x.numel() // cols if x.numel() else 0
+    n = _call or native()
+    rows, cols = n.rows_cols(x)
     if workspace is None:
         workspace = _workspace(norm_bwd_workspace_bytes(dtype_code(dz), rows, cols), dz.device)
     wsb = 0 if workspace is None else workspace.numel() * workspace.element_size()
-    lv = _multi_level([dz, dx_in, x, dx0, dresidual])
+    dense = n.dense(dz, dx_in, x, dx0, dresidual)
+    lv = None if dense else _multi_level([dz, dx_in, x, dx0, dresidual])
     if lv is not None:
         counts, (dzs, dis, xs, dxs, drs) = lv
         check(lib().hk_dropout_add_ln_bwd_strided_rows(dtype_code(dz), dtype_code(x), dtype_code(gamma), _ptr(dz),
@@ -295,14 +322,10 @@ def dropout_add_ln_bwd(dz, dx_in, x, mu, rsigma, gamma, dx0, dresidual, dgamma, 
                                                        _ptr(workspace), ctypes.c_size_t(wsb),
                                                        stream if stream is not None else current_stream()))
         return workspace
-    check(lib().hk_dropout_add_ln_bwd_pitched(dtype_code(dz), dtype_code(x), dtype_code(gamma), _ptr(dz),
-                                              _i64(_pitch(dz, cols)), _ptr(dx_in), _i64(_pitch(dx_in, cols)),
-                                              _ptr(x), _i64(_pitch(x, cols)), _ptr(mu), _ptr(rsigma), _ptr(gamma),
-                                              _ptr(dx0), _i64(_pitch(dx0, cols)), _ptr(dresidual),
-                                              _i64(_pitch(dresidual, cols)), _ptr(dgamma), _ptr(dbeta), _i64(rows),
-                                              _i64(cols), ctypes.c_int(int(is_rms)), _ptr(workspace),
-                                              ctypes.c_size_t(wsb),
-                                              stream if stream is not None else current_stream()))
+    zp, ip, xp, dxp, rp = (cols,) * 5 if dense else [_pitch(t, cols) for t in (dz, dx_in, x, dx0, dresidual)]
+    check(n.hk_dropout_add_ln_bwd_pitched(dtype_code(dz), dtype_code(x), dtype_code(gamma), dz, zp, dx_in, ip, x, xp, mu,
+                                          rsigma, gamma, dx0, dxp, dresidual, rp, dgamma, dbeta, rows, cols, is_rms,
+                                          workspace, wsb, stream))
     return workspace
 
 
@@ -352,27 +375,18 @@ def dropout_add_ln_fwd_ex(x0, gamma, z, mu, rs, *, x1=None, residual=None, beta=
                           seed=0, offset=0, rtype=None, stream=None):
     """hk_dropout_add_ln_fwd_ex on torch tensors; rows is the length of the subsets when they are given.
     rtype (a dtype code) names the residual type when neither residual nor x is passed."""
-    p = DropoutAddLnFwdParams()
-    p.itype = dtype_code(x0)
-    p.wtype = dtype_code(gamma)
+    itype = dtype_code(x0)
     if residual is not None:
-        p.rtype = dtype_code(residual)
+        rtype = dtype_code(residual)
     elif x is not None:
-        p.rtype = dtype_code(x)
-    else:
-        p.rtype = p.itype if rtype is None else rtype
-    p.cols = x0.shape[1]
-    p.rows = x0.shape[0] if x0_subset is None else x0_subset.numel()
-    p.x0_numrows = x0.shape[0]
-    p.z_numrows = z.shape[0]
-    for name, t in (("x0", x0), ("x1", x1), ("residual", residual), ("gamma", gamma), ("beta", beta),
-                    ("gamma1", gamma1), ("beta1", beta1), ("rowscale", rowscale), ("colscale", colscale),
-                    ("x0_subset", x0_subset), ("z_subset", z_subset), ("z", z), ("z1", z1), ("x", x),
-                    ("dmask", dmask), ("dmask1", dmask1), ("mu", mu), ("rs", rs)):
-        setattr(p, name, _addr(t))
-    p.dropout_p = dropout_p; p.epsilon = eps; p.rowscale_const = rowscale_const
-    p.is_rms_norm = int(is_rms); p.seed = seed; p.offset = offset
-    check(lib().hk_dropout_add_ln_fwd_ex(ctypes.byref(p), stream if stream is not None else current_stream()))
+        rtype = dtype_code(x)
+    elif rtype is None:
+        rtype = itype
+    numrows, cols = x0.shape[:2]
+    check((_call or native()).dropout_fwd_ex(
+        itype, rtype, dtype_code(gamma), numrows if x0_subset is None else x0_subset.numel(), cols, numrows, z.shape[0], x0, x1,
+        residual, gamma, beta, gamma1, beta1, rowscale, colscale, x0_subset, z_subset, z, z1, x, dmask, dmask1, mu, rs,
+        dropout_p, eps, rowscale_const, is_rms, seed, offset, stream))
 
 
 def dropout_add_ln_bwd_ex(dz, x, mu, rs, gamma, dx0, *, dz1=None, dx=None, x0=None, dmask=None, dmask1=None,
@@ -380,26 +394,27 @@ def dropout_add_ln_bwd_ex(dz, x, mu, rs, gamma, dx0, *, dz1=None, dx=None, x0=No
                           dresidual=None, dgamma=None, dbeta=None, dgamma1=None, dbeta1=None, dcolscale=None,
                           dropout_p=0.0, rowscale_const=1.0, is_rms=False, workspace=None, stream=None):
     """hk_dropout_add_ln_bwd_ex on torch tensors; allocates the workspace when none is passed."""
-    p = DropoutAddLnBwdParams()
-    p.itype = dtype_code(dz); p.rtype = dtype_code(x); p.wtype = dtype_code(gamma)
-    p.rows, p.cols = x.shape
-    p.x0_numrows = dx0.shape[0]
-    p.z_numrows = dz.shape[0]
-    for name, t in (("dz", dz), ("dz1", dz1), ("dx", dx), ("x", x), ("x0", x0), ("dmask", dmask),
-                    ("dmask1", dmask1), ("mu", mu), ("rs", rs), ("gamma", gamma), ("gamma1", gamma1),
-                    ("rowscale", rowscale), ("colscale", colscale), ("x0_subset", x0_subset),
-                    ("z_subset", z_subset), ("dx0", dx0), ("dx1", dx1), ("dresidual", dresidual),
-                    ("dgamma", dgamma), ("dbeta", dbeta), ("dgamma1", dgamma1), ("dbeta1", dbeta1),
-                    ("dcolscale", dcolscale)):
-        setattr(p, name, _addr(t))
-    p.dropout_p = dropout_p; p.rowscale_const = rowscale_const; p.is_rms_norm = int(is_rms)
+    itype, rtype, wtype = dtype_code(dz), dtype_code(x), dtype_code(gamma)
+    rows, cols = x.shape
     if workspace is None:
+        p = DropoutAddLnBwdParams()
+        p.itype, p.rtype, p.wtype, p.rows, p.cols, p.x0_numrows, p.z_numrows = itype, rtype, wtype, rows, cols, dx0.shape[0], dz.shape[0]
+        for name, t in (("dz", dz), ("dz1", dz1), ("dx", dx), ("x", x), ("x0", x0), ("dmask", dmask),
+                        ("dmask1", dmask1), ("mu", mu), ("rs", rs), ("gamma", gamma), ("gamma1", gamma1),
+                        ("rowscale", rowscale), ("colscale", colscale), ("x0_subset", x0_subset),
+                        ("z_subset", z_subset), ("dx0", dx0), ("dx1", dx1), ("dresidual", dresidual),
+                        ("dgamma", dgamma), ("dbeta", dbeta), ("dgamma1", dgamma1), ("dbeta1", dbeta1),
+                        ("dcolscale", dcolscale)):
+            setattr(p, name, _addr(t))
+        p.dropout_p = dropout_p; p.rowscale_const = rowscale_const; p.is_rms_norm = int(is_rms)
         need = ctypes.c_size_t(0)
         check(lib().hk_dropout_add_ln_bwd_ex_workspace_bytes(ctypes.byref(p), ctypes.byref(need)))
         workspace = _workspace(need.value, dz.device)
-    p.workspace = _addr(workspace)
-    p.workspace_bytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
-    check(lib().hk_dropout_add_ln_bwd_ex(ctypes.byref(p), stream if stream is not None else current_stream()))
+    wsb = 0 if workspace is None else workspace.numel() * workspace.element_size()
+    check((_call or native()).dropout_bwd_ex(
+        itype, rtype, wtype, rows, cols, dx0.shape[0], dz.shape[0], dz, dz1, dx, x, x0, dmask, dmask1, mu, rs, gamma, gamma1,
+        rowscale, colscale, x0_subset, z_subset, dx0, dx1, dresidual, dgamma, dbeta, dgamma1, dbeta1, dcolscale, workspace,
+        wsb, dropout_p, rowscale_const, is_rms, stream))
     return workspace
 
 
@@ -409,15 +424,12 @@ BINARY_OPS = {"add": 0, "sub": 1, "mul": 2, "div": 3}
 
 def unary(op, x, out, stream=None):
     """hk_unary: out = op(x), dense arrays of one dtype (out may be x)."""
-    check(lib().hk_unary(UNARY_OPS[op], dtype_code(x), _ptr(x), _ptr(out), _i64(x.numel()),
-                         stream if stream is not None else current_stream()))
+    check((_call or native()).hk_unary(UNARY_OPS[op], dtype_code(x), x, out, x.numel(), stream))
 
 
 def binary_const(op, x, scalar, out, scalar_first=False, stream=None):
     """hk_binary_const: out = x op scalar (scalar op x when scalar_first)."""
-    check(lib().hk_binary_const(BINARY_OPS[op], dtype_code(x), _ptr(x), ctypes.c_double(scalar),
-                                ctypes.c_int(int(scalar_first)), _ptr(out), _i64(x.numel()),
-                                stream if stream is not None else current_stream()))
+    check((_call or native()).hk_binary_const(BINARY_OPS[op], dtype_code(x), x, scalar, scalar_first, out, x.numel(), stream))
 
 
 def binary(op, a, b, out, stream=None):
@@ -519,18 +531,15 @@ def batch_norm_fwd(x, scale, bias, y, momentum, eps, running_mean, running_var, 
     """hk_batch_norm_fwd on a dense [N, C, ...] tensor; allocates the workspace when none is passed."""
     n, c, hw, ws = _bn_workspace(x, workspace)
     wsb = 0 if ws is None else ws.numel() * ws.element_size()
-    check(lib().hk_batch_norm_fwd(dtype_code(x), _ptr(x), _ptr(scale), _ptr(bias), _ptr(y), ctypes.c_double(momentum),
-                                  ctypes.c_double(eps), _ptr(running_mean), _ptr(running_var), _ptr(save_mean),
-                                  _ptr(save_invstd), _i64(n), _i64(c), _i64(hw), _ptr(ws), ctypes.c_size_t(wsb),
-                                  stream if stream is not None else current_stream()))
+    check((_call or native()).hk_batch_norm_fwd(dtype_code(x), x, scale, bias, y, momentum, eps, running_mean, running_var,
+                                                save_mean, save_invstd, n, c, hw, ws, wsb, stream))
 
 
 def batch_norm_bwd(dy, x, scale, dx, dscale, dbias, save_mean, save_invstd, workspace=None, stream=None):
     n, c, hw, ws = _bn_workspace(x, workspace)
     wsb = 0 if ws is None else ws.numel() * ws.element_size()
-    check(lib().hk_batch_norm_bwd(dtype_code(x), _ptr(dy), _ptr(x), _ptr(scale), _ptr(dx), _ptr(dscale), _ptr(dbias),
-                                  _ptr(save_mean), _ptr(save_invstd), _i64(n), _i64(c), _i64(hw), _ptr(ws),
-                                  ctypes.c_size_t(wsb), stream if stream is not None else current_stream()))
+    check((_call or native()).hk_batch_norm_bwd(dtype_code(x), dy, x, scale, dx, dscale, dbias, save_mean, save_invstd, n, c,
+                                                hw, ws, wsb, stream))
 
 
 def _odi(shape, dim):
@@ -545,7 +554,9 @@ def _odi(shape, dim):
 
 
 def softmax_fwd(x, y, dim=-1, stream=None):
-    if dim in (-1, x.dim() - 1):
+    n = _call or native()
+    dense = n.dense(x, y)
+    if not dense and dim in (-1, x.dim() - 1):
         lv = _multi_level([x, y])
         if lv is not None:
             counts, (xs, ys) = lv
@@ -553,19 +564,18 @@ def softmax_fwd(x, y, dim=-1, stream=None):
                                                     _arr(counts), _i64(x.shape[-1]),
                                                     stream if stream is not None else current_stream()))
             return
-    if x.dim() == 2 and dim in (-1, 1) and not (x.is_contiguous() and y.is_contiguous()):
+    if not dense and x.dim() == 2 and dim in (-1, 1):
         rows, cols = x.shape
-        check(lib().hk_softmax_fwd_pitched(dtype_code(x), _ptr(x), _i64(_pitch(x, cols)), _ptr(y),
-                                           _i64(_pitch(y, cols)), _i64(rows), _i64(cols),
-                                           stream if stream is not None else current_stream()))
+        check(n.hk_softmax_fwd_pitched(dtype_code(x), x, _pitch(x, cols), y, _pitch(y, cols), rows, cols, stream))
         return
-    o, d, i = _odi(list(x.shape), dim)
-    check(lib().hk_softmax_fwd(dtype_code(x), _ptr(x), _ptr(y), _i64(o), _i64(d), _i64(i),
-                               stream if stream is not None else current_stream()))
+    o, d, i = _odi(x.shape, dim)
+    check(n.hk_softmax_fwd(dtype_code(x), x, y, o, d, i, stream))
 
 
 def softmax_bwd(y, dy, dx, dim=-1, stream=None):
-    if dim in (-1, y.dim() - 1):
+    n = _call or native()
+    dense = n.dense(y, dy, dx)
+    if not dense and dim in (-1, y.dim() - 1):
         lv = _multi_level([y, dy, dx])
         if lv is not None:
             counts, (ys, dys, dxs) = lv
@@ -573,36 +583,35 @@ def softmax_bwd(y, dy, dx, dim=-1, stream=None):
                                                     _steps(dxs), _arr(counts), _i64(y.shape[-1]),
                                                     stream if stream is not None else current_stream()))
             return
-    if y.dim() == 2 and dim in (-1, 1) and not (y.is_contiguous() and dy.is_contiguous() and dx.is_contiguous()):
+    if not dense and y.dim() == 2 and dim in (-1, 1):
         rows, cols = y.shape
-        check(lib().hk_softmax_bwd_pitched(dtype_code(y), _ptr(y), _i64(_pitch(y, cols)), _ptr(dy),
-                                           _i64(_pitch(dy, cols)), _ptr(dx), _i64(_pitch(dx, cols)), _i64(rows),
-                                           _i64(cols), stream if stream is not None else current_stream()))
+        check(n.hk_softmax_bwd_pitched(dtype_code(y), y, _pitch(y, cols), dy, _pitch(dy, cols), dx, _pitch(dx, cols), rows, cols,
+                                       stream))
         return
-    o, d, i = _odi(list(y.shape), dim)
-    check(lib().hk_softmax_bwd(dtype_code(y), _ptr(y), _ptr(dy), _ptr(dx), _i64(o), _i64(d), _i64(i),
-                               stream if stream is not None else current_stream()))
+    o, d, i = _odi(y.shape, dim)
+    check(n.hk_softmax_bwd(dtype_code(y), y, dy, dx, o, d, i, stream))
 
 
 def sce_sparse_fwd(logits, labels, loss, ignored_index, stream=None):
-    cols = logits.shape[-1]
-    rows = logits.numel() // cols if logits.numel() else 0
-    lv = _multi_level([logits])
+    n = _call or native()
+    rows, cols = n.rows_cols(logits)
+    dense = n.dense(logits)
+    lv = None if dense else _multi_level([logits])
     if lv is not None:
         counts, (xs,) = lv
         check(lib().hk_sce_sparse_fwd_strided_rows(dtype_code(logits), _ptr(logits), _steps(xs), _ptr(labels),
                                                    _ptr(loss), _arr(counts), _i64(cols), _i64(ignored_index),
                                                    stream if stream is not None else current_stream()))
         return
-    check(lib().hk_sce_sparse_fwd_pitched(dtype_code(logits), _ptr(logits), _i64(_pitch(logits, cols)), _ptr(labels),
-                                          _ptr(loss), _i64(rows), _i64(cols), _i64(ignored_index),
-                                          stream if stream is not None else current_stream()))
+    check(n.hk_sce_sparse_fwd_pitched(dtype_code(logits), logits, cols if dense else _pitch(logits, cols), labels, loss, rows,
+                                      cols, ignored_index, stream))
 
 
 def sce_sparse_bwd(logits, labels, grad_loss, dlogits, ignored_index, stream=None):
-    cols = logits.shape[-1]
-    rows = logits.numel() // cols if logits.numel() else 0
-    lv = _multi_level([logits, dlogits])
+    n = _call or native()
+    rows, cols = n.rows_cols(logits)
+    dense = n.dense(logits, dlogits)
+    lv = None if dense else _multi_level([logits, dlogits])
     if lv is not None:
         counts, (xs, ds) = lv
         check(lib().hk_sce_sparse_bwd_strided_rows(dtype_code(logits), _ptr(logits), _steps(xs), _ptr(labels),
@@ -610,40 +619,34 @@ def sce_sparse_bwd(logits, labels, grad_loss, dlogits, ignored_index, stream=Non
                                                    _i64(cols), _i64(ignored_index),
                                                    stream if stream is not None else current_stream()))
         return
-    check(lib().hk_sce_sparse_bwd_pitched(dtype_code(logits), _ptr(logits), _i64(_pitch(logits, cols)), _ptr(labels),
-                                          _ptr(grad_loss), _ptr(dlogits), _i64(_pitch(dlogits, cols)), _i64(rows),
-                                          _i64(cols), _i64(ignored_index),
-                                          stream if stream is not None else current_stream()))
+    xp, dp = (cols, cols) if dense else (_pitch(logits, cols), _pitch(dlogits, cols))
+    check(n.hk_sce_sparse_bwd_pitched(dtype_code(logits), logits, xp, labels, grad_loss, dlogits, dp, rows, cols, ignored_index,
+                                      stream))
 
 
 def sce_sparse_bwd_reduced(logits, labels, grad_output, scale, dlogits, ignored_index, stream=None):
-    cols = logits.shape[-1]
-    rows = logits.numel() // cols if logits.numel() else 0
-    check(lib().hk_sce_sparse_bwd_reduced(dtype_code(logits), _ptr(logits), _ptr(labels), _ptr(grad_output),
-                                          ctypes.c_double(scale), _ptr(dlogits), _i64(rows), _i64(cols),
-                                          _i64(ignored_index), stream if stream is not None else current_stream()))
+    n = _call or native()
+    rows, cols = n.rows_cols(logits)
+    check(n.hk_sce_sparse_bwd_reduced(dtype_code(logits), logits, labels, grad_output, scale, dlogits, rows, cols, ignored_index,
+                                      stream))
 
 
 def sce_dense_bwd_reduced(logits, labels, grad_output, scale, dlogits, stream=None):
-    cols = logits.shape[-1]
-    rows = logits.numel() // cols if logits.numel() else 0
-    check(lib().hk_sce_dense_bwd_reduced(dtype_code(logits), _ptr(logits), _ptr(labels), _ptr(grad_output),
-                                         ctypes.c_double(scale), _ptr(dlogits), _i64(rows), _i64(cols),
-                                         stream if stream is not None else current_stream()))
+    n = _call or native()
+    rows, cols = n.rows_cols(logits)
+    check(n.hk_sce_dense_bwd_reduced(dtype_code(logits), logits, labels, grad_output, scale, dlogits, rows, cols, stream))
 
 
 def sce_dense_fwd(logits, labels, loss, stream=None):
-    cols = logits.shape[-1]
-    rows = logits.numel() // cols if logits.numel() else 0
-    check(lib().hk_sce_dense_fwd(dtype_code(logits), _ptr(logits), _ptr(labels), _ptr(loss), _i64(rows), _i64(cols),
-                                 stream if stream is not None else current_stream()))
+    n = _call or native()
+    rows, cols = n.rows_cols(logits)
+    check(n.hk_sce_dense_fwd(dtype_code(logits), logits, labels, loss, rows, cols, stream))
 
 
 def sce_dense_bwd(logits, labels, grad_loss, dlogits, stream=None):
-    cols = logits.shape[-1]
-    rows = logits.numel() // cols if logits.numel() else 0
-    check(lib().hk_sce_dense_bwd(dtype_code(logits), _ptr(logits), _ptr(labels), _ptr(grad_loss), _ptr(dlogits),
-                                 _i64(rows), _i64(cols), stream if stream is not None else current_stream()))
+    n = _call or native()
+    rows, cols = n.rows_cols(logits)
+    check(n.hk_sce_dense_bwd(dtype_code(logits), logits, labels, grad_loss, dlogits, rows, cols, stream))
 
 
 def nll_loss_fwd(pred, labels, loss, stream=None):
@@ -669,14 +672,12 @@ def reduce_workspace_bytes(dtype, shape, strides, axes):
 
 def reduce(x, out, axes, op="sum", workspace=None, stream=None):
     """x may be any strided torch view; axes already wrapped to [0, ndim)."""
-    shape, strides = list(x.shape), list(x.stride())
+    shape, strides = x.shape, x.stride()
     if workspace is None:
         workspace = _workspace(reduce_workspace_bytes(dtype_code(x), shape, strides, axes), x.device)
     wsb = 0 if workspace is None else workspace.numel() * workspace.element_size()
-    check(lib().hk_reduce(dtype_code(x), dtype_code(out), _ptr(x), _ptr(out), ctypes.c_int(len(shape)), _arr(shape),
-                          _arr(strides), ctypes.c_int(len(axes)), _arr(axes),
-                          ctypes.c_int(REDUCE_OPS[op]), _ptr(workspace),
-                          ctypes.c_size_t(wsb), stream if stream is not None else current_stream()))
+    check((_call or native()).hk_reduce(dtype_code(x), dtype_code(out), x, out, len(shape), shape, strides, len(axes),
+                                        list(axes), REDUCE_OPS[op], workspace, wsb, stream))
     return workspace
 
 
