@@ -310,13 +310,15 @@ struct BnVecWalk {
 // left out is kept as a second term, so that elements near the mean keep their digits.
 // Three launches and two reads of the input before (bf16, forward / backward): 64 x 256 x 196 24.4 / 23.6 us -> 11.2 /
 // 10.3, of which 10 are the call's own; 2 x 512 x 3969 27.9 / 27.0 -> 10.5 / 10.1.  Short odd planes are bound by cache
-// lines that neighbouring channels share (256 x 1024 x 49: 63 / 68 -> 34 / 44 us, 1.5 TB/s).
+// lines that neighbouring channels share: 16 of them stay on one XCD (channels handed out in turn / in runs of 4 / 16 / 32, GPU
+// us: 256 x 1024 x 49 34.4, 43.7 / 29.8, 38.1 / 27.5, 35.7 / 27.0, 35.1, 1.8 TB/s; 64 x 1000 x 49 fp32 9.6, 12.0 / 8.1, 10.4 /
+// 7.9, 10.3 / 8.0, 10.2; 64 x 256 x 196 6.7, 6.3 / 6.5, 6.3 / 6.2, 6.0 / 6.2, 6.0; planes of whole lines do not care).
 template <typename T, int NV, typename IT>
 __global__ __launch_bounds__(1024)
 void bn_fwd_channel_kernel(const T* x, T* y, BnRuns<IT> r, BnParams p) {
   constexpr int VEC = VecIO<T>::N;
   __shared__ float red[2][kMaxWaves * 2];
-  const int c = blockIdx.x, nwaves = int(blockDim.x >> 6);
+  const int c = int(xcd_run_block<16>(blockIdx.x, gridDim.x)), nwaves = int(blockDim.x >> 6);
   const int64_t base = int64_t(c) * r.HW;
   u32x4 raw[NV];
   IT off[NV];
@@ -387,7 +389,7 @@ __global__ __launch_bounds__(1024)
 void bn_bwd_channel_kernel(const T* dy, const T* x, T* dx, BnRuns<IT> r, BnParams p) {
   constexpr int VEC = VecIO<T>::N;
   __shared__ float red[kMaxWaves * 2];
-  const int c = blockIdx.x, nwaves = int(blockDim.x >> 6);
+  const int c = int(xcd_run_block<16>(blockIdx.x, gridDim.x)), nwaves = int(blockDim.x >> 6);
   const int64_t base = int64_t(c) * r.HW;
   u32x4 rg[NV], rx[NV];
   IT off[NV];

@@ -232,6 +232,37 @@ __device__ __forceinline__ I vec_column(I v, I cols) {
   if constexpr (!RAGGED) return v * N;
   return cols - v * N >= N ? v * N : cols - N;
 }
+// A ragged row whose 16-bit elements start on an odd 2-byte boundary: its vectors from the second on start one element
+// earlier, on a 4-byte boundary.  skip(v) of a loaded vector's first elements belong to vectors before it.
+template <typename T>
+struct RaggedRow {
+  static constexpr int N = VecIO<T>::N;
+  int cols, lead;
+  __device__ __forceinline__ RaggedRow(const T* row, int cols_) : cols(cols_), lead(0) {
+    if constexpr (sizeof(T) == 2) lead = int(reinterpret_cast<uintptr_t>(row) >> 1) & 1;
+  }
+  __device__ __forceinline__ bool live(int v) const { return v * N - lead < cols; }
+  __device__ __forceinline__ int column(int v) const { return min(max(v * N - lead, 0), cols - N); }
+  __device__ __forceinline__ int skip(int v) const { return (v == 1 ? N : v * N - (v ? lead : 0)) - column(v); }
+  // SAME: an element that two vectors hold was computed to the same bits in both
+  template <bool SAME>
+  __device__ __forceinline__ void store(T* row, int v, const float* f) const {
+    if (SAME || skip(v) <= 0) {
+      st16_any(row + column(v), VecIO<T>::pack(f));
+    } else {
+#pragma unroll
+      for (int j = 1; j < N; ++j)
+        if (j >= skip(v)) Cvt<T>::store(row + column(v) + j, f[j]);
+    }
+  }
+};
+// vectors of a ragged row's plan: one more where a row may start on an odd boundary
+template <typename T>
+inline int ragged_vectors(int64_t cols, bool odd) {
+  constexpr int N = VecIO<T>::N;
+  return int((cols + (sizeof(T) == 2 && odd ? 1 : 0) + N - 1) / N);
+}
+
 // Stores vector v of a row.  SAME: an element that two vectors hold was computed to the same bits in both, so the
 // partial vector is stored whole over its neighbour's end; otherwise its own elements go out one by one.  PLAIN: whole
 // vectors go through the cache.

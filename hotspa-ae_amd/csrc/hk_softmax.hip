@@ -40,12 +40,13 @@ void softmax_fwd_kernel(SoftmaxArgs a) {
   const T* xr = static_cast<const T*>(a.x) + row * a.x_pitch + outer_level_offset(a.x_lv);
   // slots past the row's end hold -inf, which changes neither the maximum nor the sum; in a ragged row they hold
   // elements of the row a second time, which the maximum may see and the sum leaves out
+  [[maybe_unused]] const RaggedRow<T> odd(xr, a.cols);
   u32x4 raw[NV];
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
     const int v = i * tpr + t;
     if constexpr (RAGGED) {
-      raw[i] = ld16_any<T>(xr + vec_column<T, true>(v, a.cols));
+      raw[i] = ld16_any<T>(xr + odd.column(v));
     } else if ((i + 1) * tpr <= a.nvec) {       // uniform: every thread's slot i is inside the row
       raw[i] = ld16(xr + v * VEC);
     } else {
@@ -74,7 +75,7 @@ void softmax_fwd_kernel(SoftmaxArgs a) {
   float s = 0.f;
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
-    [[maybe_unused]] const int skip = (i * tpr + t + 1) * VEC - a.cols;   // elements of earlier vectors (ragged)
+    [[maybe_unused]] const int skip = odd.skip(i * tpr + t);   // elements of earlier vectors (ragged)
 #pragma unroll
     for (int j = 0; j < VEC; ++j) {
       float& x = e[i * VEC + j];
@@ -106,10 +107,11 @@ void softmax_fwd_kernel(SoftmaxArgs a) {
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
     const int v = i * tpr + t;
-    if (v < a.nvec) {
+    if (RAGGED ? odd.live(v) : v < a.nvec) {
 #pragma unroll
       for (int j = 0; j < VEC; ++j) e[i * VEC + j] *= scale;
-      store_row_vec<T, RAGGED, (LPR > 0)>(yr, v, &e[i * VEC], a.cols);
+      if constexpr (RAGGED) odd.template store<(LPR > 0)>(yr, v, &e[i * VEC]);
+      else st16_stream(yr + v * VEC, VecIO<T>::pack(&e[i * VEC]));
     }
   }
 }
@@ -126,12 +128,13 @@ void softmax_bwd_kernel(SoftmaxArgs a) {
 
   const T* yr = static_cast<const T*>(a.x) + row * a.x_pitch + outer_level_offset(a.x_lv);
   const T* dyr = static_cast<const T*>(a.dy) + row * a.dy_pitch + outer_level_offset(a.dy_lv);
+  [[maybe_unused]] const RaggedRow<T> odd(yr, a.cols);
   u32x4 ry[NV], rdy[NV];
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
     const int v = i * tpr + t;
     if constexpr (RAGGED) {
-      const int c = vec_column<T, true>(v, a.cols);
+      const int c = odd.column(v);
       ry[i] = ld16_any<T>(yr + c);
       rdy[i] = ld16_any<T>(dyr + c);
     } else {
@@ -147,7 +150,7 @@ void softmax_bwd_kernel(SoftmaxArgs a) {
     float y[VEC], d[VEC];
     VecIO<T>::unpack(ry[i], y);
     VecIO<T>::unpack(rdy[i], d);
-    [[maybe_unused]] const int skip = (i * tpr + t + 1) * VEC - a.cols;
+    [[maybe_unused]] const int skip = odd.skip(i * tpr + t);
 #pragma unroll
     for (int j = 0; j < VEC; ++j) {
       if constexpr (RAGGED) s.v[0] = j < skip ? s.v[0] : fmaf(y[j], d[j], s.v[0]);
@@ -160,13 +163,14 @@ void softmax_bwd_kernel(SoftmaxArgs a) {
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
     const int v = i * tpr + t;
-    if (v < a.nvec) {
+    if (RAGGED ? odd.live(v) : v < a.nvec) {
       float y[VEC], d[VEC];
       VecIO<T>::unpack(ry[i], y);
       VecIO<T>::unpack(rdy[i], d);
 #pragma unroll
       for (int j = 0; j < VEC; ++j) d[j] = y[j] * (d[j] - dot);
-      store_row_vec<T, RAGGED, true>(dxr, v, d, a.cols);
+      if constexpr (RAGGED) odd.template store<true>(dxr, v, d);
+      else st16_stream(dxr + v * VEC, VecIO<T>::pack(d));
     }
   }
 }
@@ -560,7 +564,6 @@ static int softmax_lastdim_typed(SoftmaxArgs a, hipStream_t s) {
   const bool vec_ok = a.cols % VEC == 0 && aligned16(a.x) && aligned16(a.dy) && aligned16(a.out) &&
                       steps_ok(a.x_pitch, a.x_lv) && steps_ok(a.out_pitch, a.out_lv) &&
                       (!BWD || steps_ok(a.dy_pitch, a.dy_lv));
-  a.nvec = (a.cols + VEC - 1) / VEC;
   // forward keeps NV*VEC exponentials per thread: at most 64 floats
   // backward holds y and dy: at most 4 vectors of each per thread
   const int max_nv = BWD ? 4 : 64 / VEC;
@@ -568,6 +571,7 @@ static int softmax_lastdim_typed(SoftmaxArgs a, hipStream_t s) {
   const uintptr_t boundary = reinterpret_cast<uintptr_t>(a.x) | reinterpret_cast<uintptr_t>(a.dy) |
                              reinterpret_cast<uintptr_t>(a.out) | uintptr_t(a.x_pitch * int64_t(sizeof(T))) |
                              uintptr_t(a.out_pitch * int64_t(sizeof(T)));
+  a.nvec = ragged_vectors<T>(a.cols, (boundary & 3) != 0);
   const bool shaped = pick_softmax_shape(a.nvec, vec_ok, (boundary & 3) != 0, max_nv, BWD, &threads, &nv);
   if (vec_ok && shaped) return launch_softmax<T, BWD, false>(a, threads, nv, s);
   if (a.n0 != a.rows) {
