@@ -240,12 +240,16 @@ void norm_fwd_kernel(NormFwdArgs a) {
 // before it are left out of the sums and stored twice, to the same bits.  The residual sum goes out after the first
 // reduction: it may replace x or the residual in place, and every lane of the row has read its vectors by then.
 // Bound by HBM and, for odd rows, by the extra cache lines of accesses that straddle them (LayerNorm, bf16:
-// 8191 x 1021 30.7 us element by element -> 11.4 us, of which 10 are the call's own; 16384 x 2047 100 -> 30.5 us, 4.4
-// TB/s, 2048 columns 25 us; 10000 x 8191 290 -> 81 us; 8192 x 8191 fp32 219 -> 99 us, 5.4 TB/s).
+// 8191 x 1021 30.7 us element by element -> 8.1 us; 16384 x 2047 100 -> 30.5 us, 4.4 TB/s, 2048 columns 25 us; 10000 x 8191
+// 290 -> 81 us; 8192 x 8191 fp32 219 -> 99 us, 5.4 TB/s; accesses on 4-byte boundaries (RaggedRow): 9000 x 7001 72 -> 66 us,
+// 14549 x 3579 57 -> 53, RMSNorm 47 -> 41; stored through the cache 8191 x 1021 takes 10.3).
 template <typename T, int NV, int LPR, bool HAS_RES, bool IS_RMS>
 __global__ __launch_bounds__(LPR ? 256 : 1024)
 void norm_fwd_any_kernel(NormFwdArgs a) {
   constexpr int VEC = VecIO<T>::N;
+  // (a LayerNorm row of a wavefront pays more for gamma and beta off their 16-byte boundaries: 16000 x 2047 29.4 us, 31.0
+  // with its own accesses on 4 bytes)
+  constexpr bool kShift = IS_RMS || LPR == 0;
   using Lanes = RowLanes<LPR>;
   __shared__ float red[2][kMaxWaves * 2];
   const int tpr = Lanes::count(), t = Lanes::lane();
@@ -253,14 +257,15 @@ void norm_fwd_any_kernel(NormFwdArgs a) {
   if (LPR && row >= a.n0) return;   // row counts within the innermost level
 
   float v[NV][VEC];
+  const T* xr = static_cast<const T*>(a.x) + row * a.x_pitch + outer_level_offset(a.x_lv);
+  const RaggedRow<T, kShift> odd(xr, a.cols);
   {
-    const T* xr = static_cast<const T*>(a.x) + row * a.x_pitch + outer_level_offset(a.x_lv);
     const T* rr = HAS_RES ? static_cast<const T*>(a.residual) + row * a.res_pitch + outer_level_offset(a.res_lv) : nullptr;
     u32x4 raw[NV];
     [[maybe_unused]] u32x4 res[NV];
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
-      const int c = vec_column<T, true>(i * tpr + t, a.cols);
+      const int c = odd.column(i * tpr + t);
       raw[i] = ld16_any<T>(xr + c);
       if constexpr (HAS_RES) res[i] = ld16_any<T>(rr + c);
     }
@@ -279,11 +284,12 @@ void norm_fwd_any_kernel(NormFwdArgs a) {
   auto each = [&](auto f) {
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
-      if ((i + 1) * tpr * VEC <= a.cols) {   // uniform: whole vectors in every lane
+      if ((i + 1) * tpr * VEC - odd.lead <= a.cols) {   // uniform: whole vectors in every lane
 #pragma unroll
-        for (int j = 0; j < VEC; ++j) f(v[i][j]);
+        for (int j = 0; j < VEC; ++j)                   // (the second one's first element may be the first one's)
+          f(i == 0 && j == 0 && odd.lead != 0 && t == 1 ? 0.f : v[i][j]);
       } else {
-        const int skip = (i * tpr + t + 1) * VEC - a.cols;   // elements of earlier vectors
+        const int skip = odd.skip(i * tpr + t);   // elements of earlier vectors
 #pragma unroll
         for (int j = 0; j < VEC; ++j) f(j < skip ? 0.f : v[i][j]);
       }
@@ -294,7 +300,7 @@ void norm_fwd_any_kernel(NormFwdArgs a) {
       T* xo = static_cast<T*>(a.x_out) + row * a.xout_pitch + outer_level_offset(a.xout_lv);
 #pragma unroll
       for (int i = 0; i < NV; ++i)
-        if (i * tpr + t < a.nvec) store_row_vec<T, true, true>(xo, i * tpr + t, v[i], a.cols);
+        if (odd.live(i * tpr + t)) odd.template store<true>(xo, i * tpr + t, v[i]);
     }
   };
 
@@ -334,11 +340,13 @@ void norm_fwd_any_kernel(NormFwdArgs a) {
   T* yr = static_cast<T*>(a.y) + row * a.y_pitch + outer_level_offset(a.y_lv);
   const T* gp = static_cast<const T*>(a.gamma);
   const T* bp = static_cast<const T*>(a.beta);
+  int again = t;   // the vectors' places are formed anew: kept from the loads on they cost the eighth wavefront per SIMD
+  asm volatile("" : "+v"(again));
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
-    const int vec = i * tpr + t;
-    if (vec < a.nvec) {
-      const int c = vec_column<T, true>(vec, a.cols);
+    const int vec = i * tpr + again;
+    if (odd.live(vec)) {
+      const int c = odd.column(vec);
       float g[VEC], b[VEC], f[VEC];
       if (gp) VecIO<T>::unpack(ld16_any_keep<T>(gp + c), g);   // uniform
       if (bp) VecIO<T>::unpack(ld16_any_keep<T>(bp + c), b);
@@ -347,7 +355,7 @@ void norm_fwd_any_kernel(NormFwdArgs a) {
         const float n = rs * v[i][j];
         f[j] = gp ? (bp ? fmaf(g[j], n, b[j]) : g[j] * n) : (bp ? n + b[j] : n);
       }
-      store_row_vec<T, true, true>(yr, vec, f, a.cols);
+      odd.template store<true>(yr, vec, f);
     }
   }
 }
@@ -650,7 +658,9 @@ int norm_fwd_typed(NormFwdArgs a, hipStream_t s) {
                    : launch_norm_fwd_nv<T, false, false>(a, nv, rpb, grid, block, s);
   }
   int lanes = 0;
-  if (a.cols >= VEC && pick_any_shape(a.nvec, &lanes, &nv)) {
+  const uintptr_t starts = reinterpret_cast<uintptr_t>(a.x) |
+                           uintptr_t((a.x_pitch | a.x_lv.p1 | a.x_lv.p2) * int64_t(sizeof(T)));
+  if (a.cols >= VEC && pick_any_shape(ragged_vectors<T>(a.cols, (starts & 3) != 0), &lanes, &nv)) {
     if (a.is_rms) return has_res ? launch_norm_fwd_any<T, true, true>(a, lanes, nv, s) : launch_norm_fwd_any<T, false, true>(a, lanes, nv, s);
     return has_res ? launch_norm_fwd_any<T, true, false>(a, lanes, nv, s) : launch_norm_fwd_any<T, false, false>(a, lanes, nv, s);
   }

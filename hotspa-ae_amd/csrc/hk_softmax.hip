@@ -5,7 +5,8 @@
 // thread folds its elements into a (max, sum-of-exp) pair and the pairs are merged online across wavefronts (LDS).
 // The stored exponentials are rescaled on the way out, so exp is evaluated once per element.
 // Bound by HBM: what a row costs is its bytes and, for ragged rows, the extra cache lines of misaligned accesses
-// (192 x 577 x 577 bf16, forward + backward: 508 us with element-wise passes, 118 us so).
+// (192 x 577 x 577 bf16, forward + backward: 508 us with element-wise passes, 118 us with vectors counted from the row's start,
+// 107 us with those of odd rows on 4-byte boundaries; stored through the cache, 110).
 #include "hk_common.h"
 
 #include <algorithm>
@@ -40,7 +41,7 @@ void softmax_fwd_kernel(SoftmaxArgs a) {
   const T* xr = static_cast<const T*>(a.x) + row * a.x_pitch + outer_level_offset(a.x_lv);
   // slots past the row's end hold -inf, which changes neither the maximum nor the sum; in a ragged row they hold
   // elements of the row a second time, which the maximum may see and the sum leaves out
-  [[maybe_unused]] const RaggedRow<T> odd(xr, a.cols);
+  [[maybe_unused]] const RaggedRow<T, true> odd(xr, a.cols);
   u32x4 raw[NV];
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
@@ -128,7 +129,7 @@ void softmax_bwd_kernel(SoftmaxArgs a) {
 
   const T* yr = static_cast<const T*>(a.x) + row * a.x_pitch + outer_level_offset(a.x_lv);
   const T* dyr = static_cast<const T*>(a.dy) + row * a.dy_pitch + outer_level_offset(a.dy_lv);
-  [[maybe_unused]] const RaggedRow<T> odd(yr, a.cols);
+  [[maybe_unused]] const RaggedRow<T, true> odd(yr, a.cols);
   u32x4 ry[NV], rdy[NV];
 #pragma unroll
   for (int i = 0; i < NV; ++i) {

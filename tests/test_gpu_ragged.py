@@ -626,3 +626,43 @@ def test_cross_entropy_rows_with_a_tail(hk, cuda, dtype, shift, vectors):
         hk.sce_sparse_bwd(tx, lab, g, tx, -100)     # in place
         torch.cuda.synchronize()
         assert torch.equal(tx.contiguous(), dx.contiguous()), cols
+
+
+# operands whose rows start on different boundaries: x on even ones, on odd ones, on both in turn (an odd pitch), the others
+# the other way round; one vector, the edges of a lane group's and of a wavefront's shares, a workgroup
+@pytest.mark.parametrize("dtype", ["bf16", "fp16"])
+@pytest.mark.parametrize("x_at,other_at", [((0, 6), (1, 6)), ((1, 6), (0, 6)), ((0, 5), (1, 5)), ((1, 5), (0, 6)), ((0, 6), (0, 5))])
+def test_rows_on_different_boundaries(hk, cuda, dtype, x_at, other_at):
+    import torch
+    rows = 21
+    for cols in (8, 9, 15, 16, 17, 63, 64, 65, 128, 257, 512, 519, 1024, 2047, 2048, 2055, 4096, 8190):
+        x, dy = (helpers.draw(s + cols, (rows, cols), dtype=dtype) for s in (9500, 9600))
+        at = lambda a, where, fill=None: _placed(cuda, a, dtype, where[0], cols + where[1], fill)
+        tx = at(x, x_at)[1]
+        yb, ty = at(x, other_at, 0.0)
+        hk.softmax_fwd(tx, ty)
+        tdy = at(dy, other_at)[1]
+        yx = at(x, x_at)[1]
+        yx.copy_(ty)
+        db, dx = at(x, other_at, 0.0)
+        hk.softmax_bwd(yx, tdy, dx)
+        torch.cuda.synchronize()
+        assert _guards_untouched(yb, ty) and _guards_untouched(db, dx), cols
+        helpers.assert_close(ty.contiguous(), oracle.softmax_fwd(x), dtype, "softmax y %d" % cols)
+        y = helpers.to_numpy(ty.contiguous())
+        helpers.assert_close(dx.contiguous(), oracle.softmax_bwd(y, dy), dtype, "softmax dx %d" % cols,
+                             scale=float(np.sqrt(np.mean(np.square(y * dy)))),
+                             ordinary_rtol=helpers.SOFTMAX_GRADIENT_ORDINARY_RTOL)
+        gamma = helpers.draw(9700 + cols, (cols,), "uniform", 0.5, 1.5, dtype)
+        tg = _placed(cuda, gamma[None], dtype, other_at[0], cols)[1][0]
+        for is_rms in (True, False):
+            zb, tz = at(x, other_at, 0.0)
+            xb, tsum = at(x, x_at, 0.0)
+            mu, rs = torch.empty(rows, device=cuda), torch.empty(rows, device=cuda)
+            hk.dropout_add_ln_fwd(tx, tdy, tg, None, tz, tsum, mu, rs, 1e-6, is_rms)
+            torch.cuda.synchronize()
+            ez, ex, _, ers = oracle.dropout_add_ln_fwd(x, dy, gamma, None, 1e-6, is_rms)
+            helpers.assert_close(tz.contiguous(), ez, dtype, "z %d" % cols)
+            helpers.assert_close(tsum.contiguous(), ex, dtype, "x %d" % cols)
+            helpers.assert_close(rs, ers, "fp32", "rsigma %d" % cols)
+            assert _guards_untouched(zb, tz) and _guards_untouched(xb, tsum), cols
