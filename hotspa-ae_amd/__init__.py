@@ -7,7 +7,7 @@ The compute lives in native libraries built in-tree by ``build.py``:
 * ``lib/libhetu_rowwise.so`` — C++ host layer with Hetu's own types and kernel
   entry points (``hetu::impl::LayerNormCuda`` ...).
 
-* ``lib/hk_call.so``          — the CPython binding of both.
+* ``lib/hk_call.so``, ``lib/ht_call.so`` — their CPython bindings.
 
 This Python package is only the thin harness used by the tests and the
 benchmark: it loads the libraries and passes raw device pointers.  There is no

@@ -3,7 +3,7 @@
   lib/libhk_rowwise.so   C-ABI device layer + HIP kernels (hipcc, gfx950)
   lib/libhk_bench.so     the streaming yardstick bench.py measures against (hipcc, gfx950); not an operator
   lib/libhetu_rowwise.so C++ host layer mirroring Hetu's operator interface (g++)
-  lib/hk_call.so         CPython binding of both (g++)
+  lib/hk_call.so, lib/ht_call.so   CPython bindings of the two (g++)
 
 Run as ``python hotspa-ae_amd/build.py`` or through ``__graft_entry__.build()``.
 """
@@ -127,12 +127,13 @@ def build_host(verbose=True):
          ["-L" + LIB, "-lhk_rowwise", "-Wl,-rpath,$ORIGIN"])
     if verbose:
         print("[build] linked", out, flush=True)
-    call = os.path.join(LIB, "hk_call.so")
-    _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-I" + INCLUDE,
-          "-I" + sysconfig.get_paths()["include"], os.path.join(HERE, "pybind", "hk_call.cc"), "-o", call, "-L" + LIB,
-          "-lhetu_rowwise", "-lhk_rowwise", "-Wl,-rpath,$ORIGIN"])
-    if verbose:
-        print("[build] linked", call, flush=True)
+    for name, extra in (("hk_call", ["-lhk_rowwise"]), ("ht_call", ["-DHT_CALL", "-lhetu_rowwise", "-lhk_rowwise"])):
+        call = os.path.join(LIB, name + ".so")
+        _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-I" + INCLUDE,
+              "-I" + sysconfig.get_paths()["include"], os.path.join(HERE, "pybind", "hk_call.cc"), "-o", call, "-L" + LIB] +
+             extra + ["-Wl,-rpath,$ORIGIN"])
+        if verbose:
+            print("[build] linked", call, flush=True)
     for name in ("host_selftest", "gpu_selftest"):
         selftest = os.path.join(ROOT, "tests", "cpp", name + ".cc")
         if os.path.exists(selftest):

@@ -78,21 +78,26 @@ def _dtype_codes():
     return _codes
 
 
+def load_binding(path, missing):
+    """The binding at `path`: entry points that take tensors and numbers as they are; `missing` is raised without it."""
+    if not os.path.exists(path):
+        raise missing
+    import importlib.util
+    import torch
+    spec = importlib.util.spec_from_file_location(os.path.basename(path)[:-3], path)
+    call = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(call)
+    call.setup(_dtype_codes(), lambda: torch.cuda.current_stream().cuda_stream,
+               getattr(torch._C, "_cuda_getDevice", None), getattr(torch._C, "_cuda_getCurrentRawStream", None))
+    return call
+
+
 def native():
-    """hk_call.so: entry points that take tensors and numbers as they are; raises if it has not been built."""
+    """hk_call.so; raises if it has not been built."""
     global _call
     if _call is None:
-        if not os.path.exists(_CALL):
-            raise HkError(-100, "native library %s is missing: run __graft_entry__.build() first" % _CALL)
-        import importlib.util
-        import torch
         lib()
-        spec = importlib.util.spec_from_file_location("hk_call", _CALL)
-        call = importlib.util.module_from_spec(spec)
-        spec.loader.exec_module(call)
-        call.setup(_dtype_codes(), lambda: torch.cuda.current_stream().cuda_stream,
-                   getattr(torch._C, "_cuda_getDevice", None), getattr(torch._C, "_cuda_getCurrentRawStream", None))
-        _call = call
+        _call = load_binding(_CALL, HkError(-100, "native library %s is missing: run __graft_entry__.build() first" % _CALL))
     return _call
 
 

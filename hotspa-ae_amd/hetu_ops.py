@@ -1,5 +1,5 @@
 """Bindings of include/hetu_ops_c.h: the C++ operator layer (libhetu_rowwise.so)
-called, through lib/hk_call.so, with torch tensors as borrowed arrays.
+called, through lib/ht_call.so, with torch tensors as borrowed arrays.
 
 Errors of the C++ layer come back as Python exceptions named after the C++
 ones (AssertionError_, NotImplemented_, ValueError_, RuntimeError_).
@@ -90,8 +90,21 @@ def desc(t):
     return a
 
 
+_CALL = os.path.join(_HERE, "lib", "ht_call.so")
+_native = None
+
+
+def native():
+    """ht_call.so; raises if it has not been built."""
+    global _native
+    if _native is None:
+        lib()
+        _native = capi.load_binding(_CALL, HetuError("native library %s is missing: run __graft_entry__.build() first" % _CALL))
+    return _native
+
+
 def _call(name, *args):
-    check(getattr(capi.native(), name)(*args))
+    check(getattr(_native or native(), name)(*args))
 
 
 def stream_sync(stream=DEFAULT_STREAM, device=0):

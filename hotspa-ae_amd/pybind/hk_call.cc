@@ -1,4 +1,5 @@
-// CPython binding of the operator entry points of hk_rowwise.h and hetu_ops_c.h: lib/hk_call.so.
+// CPython binding of the operator entry points of hk_rowwise.h, lib/hk_call.so, and, compiled with HT_CALL, of hetu_ops_c.h,
+// lib/ht_call.so (two modules, so that a program without the operator layer does not load it).
 //
 // A call takes the C arguments in order and returns the entry point's code.  Tensors are handed over as they are and
 // asked for what is needed (data_ptr(), shape, stride(), dtype, ...): a pointer argument is None or a tensor, an HtArray
@@ -244,6 +245,7 @@ template <typename... A, int (*F)(A...), bool LABELS> struct Entry<F, LABELS> {
   }
 };
 
+#ifndef HT_CALL
 // the entry points that take a block of parameters, with its members as arguments
 int dropout_fwd_ex(int itype, int rtype, int wtype, int64_t rows, int64_t cols, int64_t x0_numrows, int64_t z_numrows,
                    const void* x0, const void* x1, const void* residual, const void* gamma, const void* beta,
@@ -271,6 +273,8 @@ int dropout_bwd_ex(int itype, int rtype, int wtype, int64_t rows, int64_t cols, 
                                      dropout_p, rowscale_const, is_rms_norm};
   return hk_dropout_add_ln_bwd_ex(&p, stream);
 }
+
+#endif
 
 // dense(a, b, ...): whether every operand is None or contiguous
 PyObject* dense(PyObject*, PyObject* const* args, Py_ssize_t n) {
@@ -314,12 +318,14 @@ PyMethodDef methods[] = {
     {"setup", setup, METH_VARARGS, nullptr},
     {"dense", (PyCFunction)(void (*)())dense, METH_FASTCALL, nullptr},
     {"rows_cols", rows_cols, METH_O, nullptr},
+#ifndef HT_CALL
     ENTRY(dropout_fwd_ex), ENTRY(dropout_bwd_ex), ENTRY(hk_batch_norm_bwd), ENTRY(hk_batch_norm_fwd),
     ENTRY(hk_binary_const), ENTRY(hk_dropout_add_ln_bwd_pitched), ENTRY(hk_dropout_add_ln_fwd_pitched),
     ENTRY(hk_layer_norm_bwd_pitched), ENTRY(hk_layer_norm_fwd_pitched), ENTRY(hk_reduce), ENTRY(hk_sce_dense_bwd),
     ENTRY(hk_sce_dense_bwd_reduced), ENTRY(hk_sce_dense_fwd), LABELS(hk_sce_sparse_bwd_pitched),
     LABELS(hk_sce_sparse_bwd_reduced), LABELS(hk_sce_sparse_fwd_pitched), ENTRY(hk_softmax_bwd),
     ENTRY(hk_softmax_bwd_pitched), ENTRY(hk_softmax_fwd), ENTRY(hk_softmax_fwd_pitched), ENTRY(hk_unary),
+#else
     ENTRY(ht_batch_norm), ENTRY(ht_batch_norm_gradient), ENTRY(ht_binary), ENTRY(ht_binary_const),
     ENTRY(ht_broadcast_shape), ENTRY(ht_dropout_add_ln_bwd), ENTRY(ht_dropout_add_ln_fwd),
     ENTRY(ht_dropout_add_ln_parallel_residual_bwd), ENTRY(ht_dropout_add_ln_parallel_residual_fwd),
@@ -332,13 +338,21 @@ PyMethodDef methods[] = {
     ENTRY(ht_softmax_cross_entropy_gradient), ENTRY(ht_softmax_cross_entropy_sparse),
     ENTRY(ht_softmax_cross_entropy_sparse_gradient), ENTRY(ht_softmax_gradient), ENTRY(ht_unary),
     ENTRY(ht_vocab_parallel_cross_entropy), ENTRY(ht_vocab_parallel_cross_entropy_gradient),
+#endif
     {nullptr, nullptr, 0, nullptr}};
 
-PyModuleDef module = {PyModuleDef_HEAD_INIT, "hk_call", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+#ifndef HT_CALL
+#define MODULE_INIT PyInit_hk_call
+#define MODULE_NAME "hk_call"
+#else
+#define MODULE_INIT PyInit_ht_call
+#define MODULE_NAME "ht_call"
+#endif
+PyModuleDef module = {PyModuleDef_HEAD_INIT, MODULE_NAME, nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 } // namespace
 
-PyMODINIT_FUNC PyInit_hk_call(void) {
+PyMODINIT_FUNC MODULE_INIT(void) {
   const std::pair<PyObject**, const char*> names[] = {
       {&s_data_ptr, "data_ptr"}, {&s_is_contiguous, "is_contiguous"}, {&s_shape, "shape"}, {&s_stride, "stride"},
       {&s_dtype, "dtype"}, {&s_is_cuda, "is_cuda"}, {&s_get_device, "get_device"}, {&s_value, "value"}};

@@ -1,4 +1,4 @@
-"""lib/hk_call.so: what an argument may be, and that what is no such thing is refused before the entry point runs."""
+"""lib/hk_call.so and lib/ht_call.so: what an argument may be, and that what is no such thing is refused before the entry point runs."""
 import importlib
 
 import pytest
@@ -27,7 +27,7 @@ def test_values_are_refused_before_the_call(hk, call):
     with pytest.raises(AttributeError):
         hk.sce_sparse_fwd(x, [0, 1], out, -100, stream=0)          # labels lie on the device
     with pytest.raises(TypeError):
-        call.ht_reduce(x, out, torch.tensor([1]), 1, 0, 1)         # axes do not
+        ops.native().ht_reduce(x, out, torch.tensor([1]), 1, 0, 1)         # axes do not
     with pytest.raises(TypeError):
         call.hk_unary(0, 6, x, x)
     with pytest.raises(AssertionError):
