@@ -377,3 +377,19 @@ def test_refused_calls(hk, cuda):
     hk.dropout_add_ln_bwd_ex(e0, e0, mu[:0], rs[:0], g, e0.clone(), dmask=m[:0], dropout_p=0.1, dgamma=dg)
     torch.cuda.synchronize()
     assert (dg == 0).all()
+
+
+@pytest.mark.parametrize("p", [2.0 ** -33, 2.0 ** -25, 2.0 ** -24, 1e-7, 0.1, 1.0 / 3, 0.5, 0.75, 0.999, 1 - 2.0 ** -23, 1 - 2.0 ** -24])
+def test_mask_at_every_probability(hk, cuda, p):
+    """The largest random bits that are kept, against the comparison of the draw itself, bit for bit; the probabilities
+    where 1 - p rounds to one, and the smallest and largest that it does not round to one or zero."""
+    import torch
+    from oracle import dropout_add_ln as dal
+    rows, cols, seed = 512, 4096, 77
+    x = torch.ones(rows, cols, dtype=torch.bfloat16, device=cuda)
+    z, mask = torch.empty_like(x), torch.full((rows, cols), 9, dtype=torch.uint8, device=cuda)
+    mu, rs = torch.empty(rows, device=cuda), torch.empty(rows, device=cuda)
+    hk.dropout_add_ln_fwd_ex(x, x[0], z, mu, rs, dmask=mask, dropout_p=p, is_rms=True, seed=seed)
+    torch.cuda.synchronize()
+    want = dal.dropout_keep(seed, 0, rows * cols, np.float32(1) - np.float32(p)).reshape(rows, cols)
+    assert np.array_equal(mask.cpu().numpy(), want)
