@@ -172,13 +172,10 @@ void norm_bwd_kernel(NormBwdArgs a) {
     }
   };
   int64_t row0 = int64_t(blockIdx.x) * rpb + group;
-  static_for<PF>([&](auto slot) { issue(slot, row0 + decltype(slot)::value * stride); });
-
-  // gamma (and beta) of this thread's columns as fp32, after the first rows' loads so that one latency
-  // covers both; a missing gamma is all ones
+  // gamma (and beta) of this thread's columns as fp32; a missing gamma is all ones
   float gm[NE];
   [[maybe_unused]] float bt[MODE == BWD_LN_MEMEFF ? NE : 1];
-  {
+  auto load_parameters = [&] {
     const T* gp = static_cast<const T*>(a.gamma);
     const T* bp = static_cast<const T*>(a.beta);
 #pragma unroll
@@ -192,7 +189,12 @@ void norm_bwd_kernel(NormBwdArgs a) {
         if (bp) VecIO<T>::unpack(ld_par(bp + col[i]), &bt[i * VEC]);
       }
     }
-  }
+  };
+  // behind the first rows' loads, so that one latency covers both; the longest walks (one group of a whole workgroup) are
+  // the better for it the other way round (32768 x 4096, forward and backward: 0.2 % of 216 us)
+  if constexpr (FIXED) load_parameters();
+  static_for<PF>([&](auto slot) { issue(slot, row0 + decltype(slot)::value * stride); });
+  if constexpr (!FIXED) load_parameters();
 
   int parity = 0;
   // guarded: check that the slot's row exists (the tail); otherwise it is known to
