@@ -498,7 +498,7 @@ static int launch_norm_fwd_nv(const NormFwdArgs& a, int nv, int rpb, dim3 grid, 
 // Picks threads-per-row and vectors-per-thread for a row of `nvec` 16-byte
 // vectors.  Returns false when the row does not fit the register kernels.
 static bool pick_row_shape(int nvec, int forced_threads, int max_nv, int wave_row_max_nv, bool many_rows,
-                           int* threads, int* nv) {
+                           bool two_waves, int* threads, int* nv) {
   if (forced_threads > 0) {
     int t = std::min(1024, std::max(64, (forced_threads + 63) / 64 * 64));
     int n = pow2_ceil((nvec + t - 1) / t);
@@ -507,8 +507,11 @@ static bool pick_row_shape(int nvec, int forced_threads, int max_nv, int wave_ro
     *nv = n;
     return true;
   }
-  // short rows: one wavefront per row
-  if (nvec <= 64 * wave_row_max_nv && nvec <= 256) {
+  // short rows: one wavefront per row; the longest of them, when there are many and no residual comes with them, two (us, one
+  // wavefront x 4 vectors / two x 2 with one row per workgroup / with two: 16384 x 2048 bf16 25.2 / 24.6 / 24.0, 31451 x 1792
+  // 40.2 / 40.0 / 38.7, RMSNorm of 31000 x 2000 48.0 / 44.3 / 45.4, 12135 x 1768 18.4 / 17.6 / 18.3, 13454 x 1000 fp32 22.2 /
+  // 20.8 / 21.6; 20000 x 1536, 192 vectors, 23.3 / 23.7 / 22.7, 4000 x 1600 5.7 / 5.9 / 6.2 and 5000 x 1664 6.4 / - / 7.5 stay)
+  if (nvec <= 64 * wave_row_max_nv && nvec <= (two_waves ? 192 : 256)) {
     *threads = 64;
     *nv = pow2_ceil((nvec + 63) / 64);
     return true;
@@ -630,6 +633,7 @@ int norm_fwd_typed(NormFwdArgs a, hipStream_t s) {
   // large inputs take two rows per workgroup (below), which also changes the best width of some rows
   const int want_rows = tune_get(TUNE_NORM_FWD_ROWS);
   const bool many_rows = want_rows > 0 ? want_rows >= 2 : a.rows >= 16 * int64_t(device_cu_count());
+  const bool two_waves = !has_res && a.rows >= 40 * int64_t(device_cu_count());
   // rows of up to 32 vectors share a wavefront (LayerNorm of 32768 rows of 256 bf16: 13.1 us with one to each, 10.7
   // so); at 96 vectors norm_fwd_kernel is the faster one (20.1 against 25.5 us).  So it is for a few rows, whose
   // wavefronts all run at once and leave nothing to share: GPU time alone, LayerNorm of 64 to 256 columns, shared / a
@@ -640,7 +644,7 @@ int norm_fwd_typed(NormFwdArgs a, hipStream_t s) {
   // norm_fwd_kernel writes the pre-norm sum beside the residual it reads, the others without one as well
   const bool sum_alone = a.x_out != nullptr && !has_res;
   if (vec_ok && !short_rows && !sum_alone &&
-      pick_row_shape(a.nvec, tune_get(TUNE_NORM_FWD_THREADS), max_nv, wave_nv, many_rows, &threads, &nv)) {
+      pick_row_shape(a.nvec, tune_get(TUNE_NORM_FWD_THREADS), max_nv, wave_nv, many_rows, two_waves, &threads, &nv)) {
     if (threads == 64) {
       dim3 grid(unsigned((a.n0 + 3) / 4), unsigned(a.n1), unsigned(a.n2)), block(256);
       return has_res ? launch_norm_fwd_nv<T, true, true>(a, nv, 1, grid, block, s)
@@ -651,7 +655,9 @@ int norm_fwd_typed(NormFwdArgs a, hipStream_t s) {
     int rpb = 1;
     if (threads <= 512) {
       const int most = max_rows_per_block<T>(nv, has_res);
-      rpb = std::min(many_rows ? 2 : 1, most);
+      // (of two wavefronts' rows only those of whole 128-byte lines, see pick_row_shape)
+      const bool pairs = many_rows && (threads > 128 || a.nvec % 8 == 0 || want_rows > 0);
+      rpb = std::min(pairs ? 2 : 1, most);
     }
     dim3 grid{unsigned((a.n0 + rpb - 1) / rpb), unsigned(a.n1), unsigned(a.n2)}, block{unsigned(threads)};
     return has_res ? launch_norm_fwd_nv<T, false, true>(a, nv, rpb, grid, block, s)

@@ -442,3 +442,36 @@ def test_few_short_rows_take_a_wavefront_each(hk, cuda, rows, cols):
     finally:
         hk.tune_set("norm_fwd_threads", 0)
     assert chosen < 1.1 * forced, (chosen, forced)
+
+
+@pytest.mark.parametrize("dtype,cols", [("bf16", 2048), ("bf16", 1544), ("bf16", 2000), ("fp16", 1792), ("fp32", 1024), ("fp32", 772), ("fp32", 1000)])
+def test_norm_fwd_of_many_rows_on_two_wavefronts(hk, cuda, dtype, cols):
+    """Rows of 193 to 256 vectors: few of them on a wavefront each, many on two; rows of whole 128-byte lines two to a
+    workgroup (an odd number of them leaves one alone).  The same rows either way, within the sums' order."""
+    import torch
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    rows, few = 40 * cus + 1, 512
+    gen = torch.Generator(device=cuda).manual_seed(cols)
+    dt = {"fp32": torch.float32, "bf16": torch.bfloat16, "fp16": torch.float16}[dtype]
+    x = torch.randn(rows, cols, generator=gen, device=cuda).to(dt)
+    g, b = (torch.randn(cols, generator=gen, device=cuda).to(dt) for _ in range(2))
+    y, mean, rstd = torch.full_like(x, 7), torch.empty(rows, device=cuda), torch.empty(rows, device=cuda)
+    hk.layer_norm_fwd(x, g, b, y, mean, rstd, 1e-5)
+    z, mu, rs = torch.full_like(x, 7), torch.empty(rows, device=cuda), torch.empty(rows, device=cuda)
+    hk.dropout_add_ln_fwd(x, None, g, None, z, None, mu, rs, 1e-6, True)
+    torch.cuda.synchronize()
+    pick = torch.tensor([0, 1, 2, 3, rows // 2, rows - 2, rows - 1], device=cuda)
+    xd, gd, bd = x[pick].double(), g.double(), b.double()
+    v = xd.var(-1, unbiased=False, keepdim=True)
+    helpers.assert_close(y[pick], ((xd - xd.mean(-1, keepdim=True)) / (v + 1e-5).sqrt() * gd + bd).cpu().numpy(), dtype, "y")
+    helpers.assert_close(rstd[pick], (1 / (v + 1e-5).sqrt())[:, 0].cpu().numpy(), "fp32", "rstd")
+    helpers.assert_close(z[pick], (xd / (xd.square().mean(-1, keepdim=True) + 1e-6).sqrt() * gd).cpu().numpy(), dtype, "z")
+    # every row against the few-row launch: fp32 sums in another order, then the stored type's rounding
+    for got, run in ((y, lambda o, m, r, a: hk.layer_norm_fwd(a, g, b, o, m, r, 1e-5)),
+                     (z, lambda o, m, r, a: hk.dropout_add_ln_fwd(a, None, g, None, o, None, m, r, 1e-6, True))):
+        for at in range(0, rows, few):
+            part = x[at:at + few]
+            o, m, r = torch.empty_like(part), torch.empty(len(part), device=cuda), torch.empty(len(part), device=cuda)
+            run(o, m, r, part)
+            d = (o.float() - got[at:at + few].float()).abs().max()
+            assert d <= {"fp32": 2e-5, "bf16": 7e-2, "fp16": 1e-2}[dtype], (at, float(d))   # two units of values up to 16
