@@ -415,8 +415,9 @@ void norm_bwd_kernel(NormBwdArgs a) {
 // its elements being another vector's.
 // blockIdx.y picks dgamma / dbeta; a block covers 128 columns as 32 float4
 // column groups x 16 row slices, every slice keeps 8 independent loads in
-// flight (with 16 a pass over 32768 x 4096 took 0.2 % longer), the last ones guarded by their row's number and not by a loop of single loads
-// (39 partial rows 3.5 -> 2.9 us), slices are folded through LDS.
+// flight (with 16 a pass over 32768 x 4096 took 0.2 % longer), the last ones
+// guarded by their row's number and not by a loop of single loads (39 partial
+// rows 3.5 -> 2.9 us), slices are folded through LDS.
 template <typename T>
 __global__ __launch_bounds__(512)
 void norm_bwd_finalize_kernel(const float* __restrict__ part_dgamma,
