@@ -13,6 +13,7 @@
 #include <Python.h>
 
 #include <array>
+#include <new>
 #include <tuple>
 #include <type_traits>
 #include <utility>
@@ -56,17 +57,21 @@ template <typename F>
 Py_ssize_t each_i64(PyObject* seq, F&& f) {
   PyObject* fast = PySequence_Fast(seq, "a sequence of integers is expected");
   if (fast == nullptr) return -1;
-  const Py_ssize_t n = PySequence_Fast_GET_SIZE(fast);
-  for (Py_ssize_t i = 0; i < n; ++i) {
+  Py_ssize_t i = 0;
+  for (; i < PySequence_Fast_GET_SIZE(fast); ++i) {   // (an item's conversion may change a list)
     int64_t v;
-    if (!to_i64(PySequence_Fast_GET_ITEM(fast, i), &v)) {
+    PyObject* item = PySequence_Fast_GET_ITEM(fast, i);
+    Py_INCREF(item);
+    const bool ok = to_i64(item, &v);
+    Py_DECREF(item);
+    if (!ok) {
       Py_DECREF(fast);
       return -1;
     }
     f(i, v);
   }
   Py_DECREF(fast);
-  return n;
+  return i;
 }
 
 int dtype_code_of(PyObject* tensor) {
@@ -150,9 +155,10 @@ template <typename I> struct HostArray {
       many.resize(size_t(n));
       dst = many.data();
     }
-    if (each_i64(o, [&](Py_ssize_t i, int64_t x) { if (i < n) dst[i] = I(x); }) < 0) return false;
+    const Py_ssize_t got = each_i64(o, [&](Py_ssize_t i, int64_t x) { if (i < n) dst[i] = I(x); });
+    if (got >= 0 && got != n) PyErr_SetString(PyExc_ValueError, "a list of integers changed while it was read");
     v = dst;
-    return true;
+    return got == n;
   }
   const I* get() { return v; }
 };
@@ -188,7 +194,7 @@ template <> struct Arg<HtArray*> {
       PyErr_Format(PyExc_AssertionError, "an array of %zd dimensions, at most %d are taken", n, HT_C_MAX_NDIM);
       return false;
     }
-    n = n < 0 ? n : each_i64(shape, [&](Py_ssize_t i, int64_t x) { a.shape[i] = x; });
+    n = n < 0 ? n : each_i64(shape, [&](Py_ssize_t i, int64_t x) { if (i < n) a.shape[i] = x; });
     Py_DECREF(shape);
     if (n < 0) return false;
     a.ndim = int32_t(n);
@@ -241,7 +247,11 @@ template <typename... A, int (*F)(A...), bool LABELS> struct Entry<F, LABELS> {
       PyErr_Format(PyExc_TypeError, "%zd arguments are expected, %zd given", Py_ssize_t(sizeof...(A)), n);
       return nullptr;
     }
-    return run(args, std::index_sequence_for<A...>{});
+    try {
+      return run(args, std::index_sequence_for<A...>{});
+    } catch (const std::bad_alloc&) {
+      return PyErr_NoMemory();
+    }
   }
 };
 

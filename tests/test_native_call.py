@@ -51,3 +51,18 @@ def test_numbers_convert_like_c(call):
         ops.ndarray_reduce(x, "sum", axes, np.bool_(True), s)
         assert torch.allclose(s[0], x.sum(0), atol=1e-5)
     ops.ndarray_binary("add", x[:, ::2], x[:, ::2], out[:, :3].contiguous())   # strided operands are described as they are
+
+
+def test_a_long_or_changing_list_of_integers(call):
+    ops = importlib.import_module("hotspa-ae_amd.hetu_ops")
+    x, s = torch.randn(4, 6), torch.empty(6)
+    ops.ndarray_reduce(x, "sum", [0] * 40, False, s)     # more of them than the fixed array holds; duplicates are one axis
+    assert torch.allclose(s, x.sum(0), atol=1e-5)
+
+    class Shrinks:
+        def __int__(self):
+            axes.clear()
+            return 0
+    axes = [Shrinks(), 1]
+    with pytest.raises(ValueError):
+        ops.native().ht_reduce(x, s, axes, 2, 0, 1)
