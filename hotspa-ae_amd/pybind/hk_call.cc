@@ -13,6 +13,8 @@
 #include <Python.h>
 
 #include <array>
+#include <cstdio>
+#include <exception>
 #include <new>
 #include <tuple>
 #include <type_traits>
@@ -235,11 +237,32 @@ template <typename... A, int (*F)(A...), bool LABELS> struct Entry<F, LABELS> {
   template <size_t... I>
   static PyObject* run(PyObject* const* args, std::index_sequence<I...>) {
     std::tuple<ArgOf<A>...> conv;
-    if (!(std::get<I>(conv).from(args[I]) && ...)) return nullptr;
-    int rc;
+    try {
+      if (!(std::get<I>(conv).from(args[I]) && ...)) return nullptr;
+    } catch (const std::bad_alloc&) {
+      return PyErr_NoMemory();
+    }
+    int rc = 0;
+    const char* thrown = nullptr;   // an exception of the entry point ends before the lock is taken again
+    char text[256];
+    bool no_memory = false;
     Py_BEGIN_ALLOW_THREADS
-    rc = F(std::get<I>(conv).get()...);
+    try {
+      rc = F(std::get<I>(conv).get()...);
+    } catch (const std::bad_alloc&) {
+      no_memory = true;
+    } catch (const std::exception& e) {
+      std::snprintf(text, sizeof text, "%s", e.what());
+      thrown = text;
+    } catch (...) {
+      thrown = "an entry point ended with an exception";
+    }
     Py_END_ALLOW_THREADS
+    if (no_memory) return PyErr_NoMemory();
+    if (thrown != nullptr) {
+      PyErr_SetString(PyExc_RuntimeError, thrown);
+      return nullptr;
+    }
     return PyLong_FromLong(rc);
   }
   static PyObject* call(PyObject*, PyObject* const* args, Py_ssize_t n) {
@@ -247,11 +270,7 @@ template <typename... A, int (*F)(A...), bool LABELS> struct Entry<F, LABELS> {
       PyErr_Format(PyExc_TypeError, "%zd arguments are expected, %zd given", Py_ssize_t(sizeof...(A)), n);
       return nullptr;
     }
-    try {
-      return run(args, std::index_sequence_for<A...>{});
-    } catch (const std::bad_alloc&) {
-      return PyErr_NoMemory();
-    }
+    return run(args, std::index_sequence_for<A...>{});
   }
 };
 

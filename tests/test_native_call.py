@@ -1,5 +1,9 @@
 """lib/hk_call.so and lib/ht_call.so: what an argument may be, and that what is no such thing is refused before the entry point runs."""
 import importlib
+import os
+import subprocess
+import sys
+import sysconfig
 
 import pytest
 import torch
@@ -66,3 +70,37 @@ def test_a_long_or_changing_list_of_integers(call):
     axes = [Shrinks(), 1]
     with pytest.raises(ValueError):
         ops.native().ht_reduce(x, s, axes, 2, 0, 1)
+
+
+def test_an_exception_of_an_entry_point_is_raised_with_the_lock_held(tmp_path):
+    """In a process of its own: what leaves an entry point without the interpreter's lock ends the program."""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    lib = os.path.join(root, "hotspa-ae_amd", "lib")
+    out = str(tmp_path / "throwing_entries.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-I" + os.path.join(root, "include"),
+                    "-I" + sysconfig.get_paths()["include"], os.path.join(root, "tests", "cpp", "throwing_entries.cc"), "-o", out,
+                    "-L" + lib, "-lhk_rowwise", "-Wl,-rpath," + lib], check=True)
+    code = """
+import importlib.util, threading
+spec = importlib.util.spec_from_file_location("throwing_entries", %r)
+m = importlib.util.module_from_spec(spec)
+spec.loader.exec_module(m)
+def raised(what, *args):
+    try:
+        return m.throws(what, *args)
+    except Exception as e:
+        return type(e).__name__, str(e)
+def check():
+    for _ in range(100):
+        assert raised(0, [7]) == 7
+        assert raised(1, None)[0] == "MemoryError"
+        assert raised(2, list(range(40))) == ("RuntimeError", "a list too long")
+        assert raised(3, None)[0] == "RuntimeError"
+threads = [threading.Thread(target=check) for _ in range(4)]
+[t.start() for t in threads]
+[t.join() for t in threads]
+check()
+print("done")
+""" % out
+    done = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120)
+    assert done.returncode == 0 and done.stdout == "done\n" and "Error" not in done.stderr, (done.returncode, done.stderr)
