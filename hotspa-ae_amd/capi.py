@@ -283,7 +283,7 @@ def layer_norm_bwd(dy, x_or_y, gamma, beta, mean, stat, dx, dgamma, dbeta, eps, 
         return workspace
     dyp, xp, dxp = (cols,) * 3 if dense else [_pitch(t, cols) for t in (dy, x_or_y, dx)]
     check(n.hk_layer_norm_bwd_pitched(dtype_code(dy), dy, dyp, x_or_y, xp, gamma, beta, mean, stat, dtype_code(stat),
-                                      stat_kind, dx, dxp, dgamma, dbeta, rows, cols, eps, memory_efficient, clamp_gamma,
+                                      stat_kind, dx, dxp, dgamma, dbeta, rows, cols, eps, int(memory_efficient), int(clamp_gamma),
                                       workspace, wsb, stream))
     return workspace
 
@@ -305,7 +305,7 @@ def dropout_add_ln_fwd(x0, residual, gamma, beta, z, x_out, mu, rsigma, eps, is_
         return
     xp, rp, zp, op = (cols,) * 4 if dense else [_pitch(t, cols) for t in (x0, residual, z, x_out)]
     check(n.hk_dropout_add_ln_fwd_pitched(dtype_code(x0), rtype, dtype_code(gamma), x0, xp, residual, rp, gamma, beta, z, zp,
-                                          x_out, op, mu, rsigma, rows, cols, eps, is_rms, stream))
+                                          x_out, op, mu, rsigma, rows, cols, eps, int(is_rms), stream))
 
 
 def dropout_add_ln_bwd(dz, dx_in, x, mu, rsigma, gamma, dx0, dresidual, dgamma, dbeta, is_rms,
@@ -329,7 +329,7 @@ def dropout_add_ln_bwd(dz, dx_in, x, mu, rsigma, gamma, dx0, dresidual, dgamma, 
         return workspace
     zp, ip, xp, dxp, rp = (cols,) * 5 if dense else [_pitch(t, cols) for t in (dz, dx_in, x, dx0, dresidual)]
     check(n.hk_dropout_add_ln_bwd_pitched(dtype_code(dz), dtype_code(x), dtype_code(gamma), dz, zp, dx_in, ip, x, xp, mu,
-                                          rsigma, gamma, dx0, dxp, dresidual, rp, dgamma, dbeta, rows, cols, is_rms,
+                                          rsigma, gamma, dx0, dxp, dresidual, rp, dgamma, dbeta, rows, cols, int(is_rms),
                                           workspace, wsb, stream))
     return workspace
 
@@ -391,7 +391,7 @@ def dropout_add_ln_fwd_ex(x0, gamma, z, mu, rs, *, x1=None, residual=None, beta=
     check((_call or native()).dropout_fwd_ex(
         itype, rtype, dtype_code(gamma), numrows if x0_subset is None else x0_subset.numel(), cols, numrows, z.shape[0], x0, x1,
         residual, gamma, beta, gamma1, beta1, rowscale, colscale, x0_subset, z_subset, z, z1, x, dmask, dmask1, mu, rs,
-        dropout_p, eps, rowscale_const, is_rms, seed, offset, stream))
+        dropout_p, eps, rowscale_const, int(is_rms), seed, offset, stream))
 
 
 def dropout_add_ln_bwd_ex(dz, x, mu, rs, gamma, dx0, *, dz1=None, dx=None, x0=None, dmask=None, dmask1=None,
@@ -419,7 +419,7 @@ def dropout_add_ln_bwd_ex(dz, x, mu, rs, gamma, dx0, *, dz1=None, dx=None, x0=No
     check((_call or native()).dropout_bwd_ex(
         itype, rtype, wtype, rows, cols, dx0.shape[0], dz.shape[0], dz, dz1, dx, x, x0, dmask, dmask1, mu, rs, gamma, gamma1,
         rowscale, colscale, x0_subset, z_subset, dx0, dx1, dresidual, dgamma, dbeta, dgamma1, dbeta1, dcolscale, workspace,
-        wsb, dropout_p, rowscale_const, is_rms, stream))
+        wsb, dropout_p, rowscale_const, int(is_rms), stream))
     return workspace
 
 
@@ -434,7 +434,7 @@ def unary(op, x, out, stream=None):
 
 def binary_const(op, x, scalar, out, scalar_first=False, stream=None):
     """hk_binary_const: out = x op scalar (scalar op x when scalar_first)."""
-    check((_call or native()).hk_binary_const(BINARY_OPS[op], dtype_code(x), x, scalar, scalar_first, out, x.numel(), stream))
+    check((_call or native()).hk_binary_const(BINARY_OPS[op], dtype_code(x), x, scalar, int(scalar_first), out, x.numel(), stream))
 
 
 def binary(op, a, b, out, stream=None):
@@ -609,7 +609,7 @@ def sce_sparse_fwd(logits, labels, loss, ignored_index, stream=None):
                                                    stream if stream is not None else current_stream()))
         return
     check(n.hk_sce_sparse_fwd_pitched(dtype_code(logits), logits, cols if dense else _pitch(logits, cols), labels, loss, rows,
-                                      cols, ignored_index, stream))
+                                      cols, int(ignored_index), stream))
 
 
 def sce_sparse_bwd(logits, labels, grad_loss, dlogits, ignored_index, stream=None):
@@ -625,14 +625,14 @@ def sce_sparse_bwd(logits, labels, grad_loss, dlogits, ignored_index, stream=Non
                                                    stream if stream is not None else current_stream()))
         return
     xp, dp = (cols, cols) if dense else (_pitch(logits, cols), _pitch(dlogits, cols))
-    check(n.hk_sce_sparse_bwd_pitched(dtype_code(logits), logits, xp, labels, grad_loss, dlogits, dp, rows, cols, ignored_index,
+    check(n.hk_sce_sparse_bwd_pitched(dtype_code(logits), logits, xp, labels, grad_loss, dlogits, dp, rows, cols, int(ignored_index),
                                       stream))
 
 
 def sce_sparse_bwd_reduced(logits, labels, grad_output, scale, dlogits, ignored_index, stream=None):
     n = _call or native()
     rows, cols = n.rows_cols(logits)
-    check(n.hk_sce_sparse_bwd_reduced(dtype_code(logits), logits, labels, grad_output, scale, dlogits, rows, cols, ignored_index,
+    check(n.hk_sce_sparse_bwd_reduced(dtype_code(logits), logits, labels, grad_output, scale, dlogits, rows, cols, int(ignored_index),
                                       stream))
 
 

@@ -133,24 +133,24 @@ def synchronize_all():
 
 # ---- kernel entry points --------------------------------------------------
 def layer_norm(x, scale, bias, mean, var, out, reduce_dims, eps, stream=DEFAULT_STREAM):
-    _call("ht_layer_norm", x, scale, bias, mean, var, out, reduce_dims,
-          eps, stream)
+    _call("ht_layer_norm", x, scale, bias, mean, var, out, int(reduce_dims),
+          float(eps), stream)
 
 
 def layer_norm_gradient(dy, x, scale, dx, dscale, dbias, mean, var, reduce_dims, eps, stream=DEFAULT_STREAM):
     _call("ht_layer_norm_gradient", dy, x, scale, dx, dscale, dbias, mean,
-          var, reduce_dims, eps, stream)
+          var, int(reduce_dims), float(eps), stream)
 
 
 def fused_layer_norm(x, scale, bias, mean, invvar, out, reduce_dims, eps, stream=DEFAULT_STREAM):
     _call("ht_fused_layer_norm", x, scale, bias, mean, invvar, out,
-          reduce_dims, eps, stream)
+          int(reduce_dims), float(eps), stream)
 
 
 def fused_layer_norm_gradient(dy, x_or_y, scale, bias, dx, dscale, dbias, mean, invvar, reduce_dims, eps, inplace,
                               stream=DEFAULT_STREAM):
     _call("ht_fused_layer_norm_gradient", dy, x_or_y, scale, bias, dx, dscale,
-          dbias, mean, invvar, reduce_dims, eps, int(inplace),
+          dbias, mean, invvar, int(reduce_dims), float(eps), int(inplace),
           stream)
 
 
@@ -159,7 +159,7 @@ def dropout_add_ln_fwd(x0, residual, gamma, beta, z, x, mu, rsigma, eps, is_rms_
                        dmask=None, rowscale_const=1.0, z_numrows=0, stream=DEFAULT_STREAM):
     _call("ht_dropout_add_ln_fwd", x0, residual, gamma, beta, rowscale,
           colscale, x0_subset, z_subset, z, x, dmask, mu, rsigma,
-          dropout_p, eps, rowscale_const, z_numrows, int(residual_in_fp32),
+          float(dropout_p), float(eps), float(rowscale_const), int(z_numrows), int(residual_in_fp32),
           int(is_rms_norm), stream)
 
 
@@ -168,8 +168,8 @@ def dropout_add_ln_bwd(dz, dx, x, mu, rsigma, gamma, dx0, dresidual, dgamma, dbe
                        z_subset=None, dcolscale=None, rowscale_const=1.0, x0_numrows=0, stream=DEFAULT_STREAM):
     _call("ht_dropout_add_ln_bwd", dz, dx, x, x0, dmask, mu, rsigma,
           gamma, rowscale, colscale, x0_subset, z_subset, dx0,
-          dresidual, dgamma, dbeta, dcolscale, dropout_p, rowscale_const,
-          x0_numrows, int(has_residual), int(is_rms_norm), stream)
+          dresidual, dgamma, dbeta, dcolscale, float(dropout_p), float(rowscale_const),
+          int(x0_numrows), int(has_residual), int(is_rms_norm), stream)
 
 
 def dropout_add_ln_parallel_residual_fwd(x0, x1, residual, gamma0, beta0, gamma1, beta1, z0, z1, x, dmask0, dmask1,
@@ -177,7 +177,7 @@ def dropout_add_ln_parallel_residual_fwd(x0, x1, residual, gamma0, beta0, gamma1
                                          stream=DEFAULT_STREAM):
     _call("ht_dropout_add_ln_parallel_residual_fwd", x0, x1, residual, gamma0, beta0,
           gamma1, beta1, z0, z1, x, dmask0, dmask1, mu,
-          rsigma, dropout_p, eps, int(residual_in_fp32),
+          rsigma, float(dropout_p), float(eps), int(residual_in_fp32),
           int(is_rms_norm), stream)
 
 
@@ -186,7 +186,7 @@ def dropout_add_ln_parallel_residual_bwd(dz0, dz1, dx, x, dmask0, dmask1, mu, rs
                                          has_residual, is_rms_norm=False, stream=DEFAULT_STREAM):
     _call("ht_dropout_add_ln_parallel_residual_bwd", dz0, dz1, dx, x, dmask0,
           dmask1, mu, rsigma, gamma0, gamma1, dx0, dx1, dresidual,
-          dgamma0, dbeta0, dgamma1, dbeta1, dropout_p, int(has_x1),
+          dgamma0, dbeta0, dgamma1, dbeta1, float(dropout_p), int(has_x1),
           int(has_residual), int(is_rms_norm), stream)
 
 
@@ -220,26 +220,26 @@ def ndarray_unary(op, x, out=None, in_place=False, stream=DEFAULT_STREAM):
 
 def vocab_parallel_cross_entropy(logits, labels, vocab_start, vocab_end, ignored_index, picked, lse,
                                  stream=DEFAULT_STREAM):
-    _call("ht_vocab_parallel_cross_entropy", logits, labels, vocab_start, vocab_end,
-          ignored_index, picked, lse, stream)
+    _call("ht_vocab_parallel_cross_entropy", logits, labels, int(vocab_start), int(vocab_end),
+          int(ignored_index), picked, lse, stream)
 
 
 def vocab_parallel_cross_entropy_gradient(softmax, labels, vocab_start, vocab_end, ignored_index, grad_loss, out,
                                           stream=DEFAULT_STREAM):
-    _call("ht_vocab_parallel_cross_entropy_gradient", softmax, labels, vocab_start,
-          vocab_end, ignored_index, grad_loss, out, stream)
+    _call("ht_vocab_parallel_cross_entropy_gradient", softmax, labels, int(vocab_start),
+          int(vocab_end), int(ignored_index), grad_loss, out, stream)
 
 
 def norm(x, out, dim, p, stream=DEFAULT_STREAM):
-    _call("ht_norm", x, out, dim, p, stream)
+    _call("ht_norm", x, out, int(dim), int(p), stream)
 
 
 def norm_gradient(x, norm_out, grad, dx, dim, p, stream=DEFAULT_STREAM):
-    _call("ht_norm_gradient", x, norm_out, grad, dx, dim, p, stream)
+    _call("ht_norm_gradient", x, norm_out, grad, dx, int(dim), int(p), stream)
 
 
 def ndarray_norm(x, p, dim, keepdim, out, stream=DEFAULT_STREAM):
-    _call("ht_ndarray_norm", x, p, dim, int(keepdim), out, stream)
+    _call("ht_ndarray_norm", x, int(p), int(dim), int(keepdim), out, stream)
 
 
 def batch_norm(x, scale, bias, y, momentum, eps, running_mean, running_var, save_mean, save_var,
@@ -258,20 +258,20 @@ def set_random_seed(seed):
 
 
 def instance_norm(x, mean, var, out, eps, stream=DEFAULT_STREAM):
-    _call("ht_instance_norm", x, mean, var, out, eps, stream)
+    _call("ht_instance_norm", x, mean, var, out, float(eps), stream)
 
 
 def instance_norm_gradient(dy, x, dx, mean, var, eps, stream=DEFAULT_STREAM):
-    _call("ht_instance_norm_gradient", dy, x, dx, mean, var, eps,
+    _call("ht_instance_norm_gradient", dy, x, dx, mean, var, float(eps),
           stream)
 
 
 def softmax(x, out, dim, stream=DEFAULT_STREAM):
-    _call("ht_softmax", x, out, dim, stream)
+    _call("ht_softmax", x, out, int(dim), stream)
 
 
 def softmax_gradient(y, dy, dx, dim, stream=DEFAULT_STREAM):
-    _call("ht_softmax_gradient", y, dy, dx, dim, stream)
+    _call("ht_softmax_gradient", y, dy, dx, int(dim), stream)
 
 
 def softmax_cross_entropy(pred, label, loss, stream=DEFAULT_STREAM):
@@ -284,13 +284,13 @@ def softmax_cross_entropy_gradient(pred, label, grad_loss, out, stream=DEFAULT_S
 
 
 def softmax_cross_entropy_sparse(pred, label, loss, ignored_index, stream=DEFAULT_STREAM):
-    _call("ht_softmax_cross_entropy_sparse", pred, label, loss, ignored_index,
+    _call("ht_softmax_cross_entropy_sparse", pred, label, loss, int(ignored_index),
           stream)
 
 
 def softmax_cross_entropy_sparse_gradient(pred, label, grad_loss, out, ignored_index, stream=DEFAULT_STREAM):
     _call("ht_softmax_cross_entropy_sparse_gradient", pred, label, grad_loss, out,
-          ignored_index, stream)
+          int(ignored_index), stream)
 
 
 def nll_loss(pred, label, loss, stream=DEFAULT_STREAM):
@@ -314,7 +314,7 @@ def ndarray_reduce(x, red_type, axes, keepdims, out, stream=DEFAULT_STREAM):
 
 
 def ndarray_softmax(x, dim, out, stream=DEFAULT_STREAM):
-    _call("ht_ndarray_softmax", x, dim, out, stream)
+    _call("ht_ndarray_softmax", x, int(dim), out, stream)
 
 
 def ndarray_layernorm(x, scale, bias, normalized_ndim, eps, fused, out, mean=None, var=None,
@@ -326,7 +326,7 @@ def ndarray_layernorm(x, scale, bias, normalized_ndim, eps, fused, out, mean=Non
 def ndarray_sceloss(preds, labels, out, reduction="mean", ignored_index=None, stream=DEFAULT_STREAM):
     sparse = ignored_index is not None
     _call("ht_ndarray_sceloss", preds, labels, int(sparse),
-          ignored_index if sparse else 0, RED[reduction], out, stream)
+          int(ignored_index) if sparse else 0, RED[reduction], out, stream)
 
 
 # ---- gradients of the reductions and of the reduced losses ----------------
@@ -340,7 +340,7 @@ def broadcast_shape(x, out, add_axes=(), const_value=None, stream=DEFAULT_STREAM
 def reduce_gradient(grad_output, out, reduction, axes, keepdims, stream=DEFAULT_STREAM):
     ax = list(axes)
     keep = [keepdims] if isinstance(keepdims, bool) else list(keepdims)
-    _call("ht_reduce_gradient", grad_output, RED[reduction], ax, len(ax), keep,
+    _call("ht_reduce_gradient", grad_output, RED[reduction], ax, len(ax), [int(k) for k in keep],
           len(keep), out, stream)
 
 
@@ -348,7 +348,7 @@ def sceloss_gradient(preds, labels, grad_output, out, reduction="mean", ignored_
                      stream=DEFAULT_STREAM):
     sparse = ignored_index is not None
     _call("ht_sceloss_gradient", preds, labels, grad_output, int(sparse),
-          ignored_index if sparse else 0, RED[reduction], int(fused), out,
+          int(ignored_index) if sparse else 0, RED[reduction], int(fused), out,
           stream)
 
 

@@ -4,8 +4,8 @@
 // A call takes the C arguments in order and returns the entry point's code.  Tensors are handed over as they are and
 // asked for what is needed (data_ptr(), shape, stride(), dtype, ...): a pointer argument is None or a tensor, an HtArray
 // argument likewise (described for the length of the call), an array of integers a tuple or list, a stream None (torch's
-// current one), a ctypes.c_void_p or an address.  Integers wrap like C's.  The interpreter's lock is released while the entry point
-// runs.  Built without torch's headers: it calls the methods that a Python caller would.
+// current one), a ctypes.c_void_p or an address.  Integers wrap like C's; a fraction or a text is refused as one.  The interpreter's
+// lock is released while the entry point runs.  Built without torch's headers: it calls the methods that a Python caller would.
 //
 // A small call is bound by this path: with a ctypes object built per argument, RMSNorm with a residual of 16 x 4096 bf16
 // (3.4 us of kernel) took 10.0 us a call, so it takes 5.0; a 256 x 1000 mean loss and its gradient 43.7 and 33.8.
@@ -37,7 +37,7 @@ bool to_i64(PyObject* o, int64_t* v) {
     *v = int64_t(PyLong_AsUnsignedLongLongMask(o));
     return !(*v == -1 && PyErr_Occurred());
   }
-  PyObject* i = PyNumber_Long(o);
+  PyObject* i = PyNumber_Index(o);   // an integer of any type; a fraction or a text is none
   if (i == nullptr) return false;
   *v = int64_t(PyLong_AsUnsignedLongLongMask(i));
   Py_DECREF(i);

@@ -64,12 +64,47 @@ def test_a_long_or_changing_list_of_integers(call):
     assert torch.allclose(s, x.sum(0), atol=1e-5)
 
     class Shrinks:
-        def __int__(self):
+        def __index__(self):
             axes.clear()
             return 0
     axes = [Shrinks(), 1]
     with pytest.raises(ValueError):
         ops.native().ht_reduce(x, s, axes, 2, 0, 1)
+
+
+def test_what_is_no_integer_is_refused(hk, call):
+    """Axes, flags, streams, the numbers that ctypes took as they are: an integer of any type and nothing else.  Where
+    the wrappers call int() or float() themselves (dim, eps, the truth values), what these take goes through."""
+    import numpy as np
+    ops = importlib.import_module("hotspa-ae_amd.hetu_ops")
+    x, out = torch.randn(4, 6), torch.full((4,), 5.0)
+
+    class One:
+        def __index__(self):
+            return 1
+    for no in (1.9, 1.0, "1", np.float32(1), None, torch.tensor(1.5)):
+        for refused in (lambda: ops.reduce(x, out, [no], "sum"), lambda: ops.reduce(x, out, [1], "sum", stream=no),
+                        lambda: ops.ndarray_reduce(x, "sum", [no], False, out),
+                        lambda: ops.reduce_gradient(out, x.clone(), "sum", [no], [False]),
+                        lambda: ops.broadcast_shape(out, x.clone(), [no]),
+                        lambda: ops.ndarray_layernorm(x, x[0], x[0], no, 1e-5, True, x.clone()),
+                        lambda: call.hk_unary(0, 6, x, x, no, 0)):
+            with pytest.raises(TypeError):
+                refused()
+        with pytest.raises((TypeError, AttributeError)):
+            hk.unary("exp", x[:0], x[:0], stream=1.5)
+    assert (out == 5.0).all()
+    for yes in (1, True, np.int8(1), np.uint64(1), One(), torch.tensor(1), -1):
+        ops.reduce(x, out.fill_(0), [yes], "sum")
+        assert torch.allclose(out, x.sum(1), atol=1e-5)
+    y, want = torch.empty(4, 6), torch.softmax(x, 1)
+    for dim in (1, 1.0, "1", np.float32(1.0)):
+        ops.softmax(x, y.fill_(0), dim)
+        assert torch.allclose(y, want, atol=1e-6)
+    mean, var = torch.empty(4), torch.empty(4)
+    for eps in (1e-5, "1e-5", np.float64(1e-5), 0):
+        ops.layer_norm(x, x[0].contiguous(), x[1].contiguous(), mean, var, y, 1, eps)
+        assert torch.allclose(y, torch.nn.functional.layer_norm(x, (6,), x[0], x[1], float(eps)), atol=1e-5)
 
 
 def test_an_exception_of_an_entry_point_is_raised_with_the_lock_held(tmp_path):
