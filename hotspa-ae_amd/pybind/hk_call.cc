@@ -11,6 +11,7 @@
 // (3.4 us of kernel) took 10.0 us a call, so it takes 5.0; a 256 x 1000 mean loss and its gradient 43.7 and 33.8.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
+#include <pthread.h>
 
 #include <array>
 #include <cstdio>
@@ -30,7 +31,7 @@ PyObject *s_data_ptr, *s_is_contiguous, *s_shape, *s_stride, *s_dtype, *s_is_cud
 PyObject* g_dtype_codes;      // {torch dtype: code}
 PyObject* g_current_stream;   // () -> address of torch's current stream (initialises the device if need be)
 PyObject *g_get_device, *g_raw_stream;   // torch's own two steps of the same, once the device is initialised
-bool g_initialised = false;
+bool g_initialised = false;   // in this process: a child of fork() asks g_current_stream again, which refuses there
 
 bool to_i64(PyObject* o, int64_t* v) {
   if (PyLong_CheckExact(o)) {
@@ -387,5 +388,6 @@ PyMODINIT_FUNC MODULE_INIT(void) {
       {&s_dtype, "dtype"}, {&s_is_cuda, "is_cuda"}, {&s_get_device, "get_device"}, {&s_value, "value"}};
   for (const auto& n : names)
     if ((*n.first = PyUnicode_InternFromString(n.second)) == nullptr) return nullptr;
+  pthread_atfork(nullptr, nullptr, [] { g_initialised = false; });
   return PyModule_Create(&module);
 }

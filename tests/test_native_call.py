@@ -139,3 +139,35 @@ print("done")
 """ % out
     done = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120)
     assert done.returncode == 0 and done.stdout == "done\n" and "Error" not in done.stderr, (done.returncode, done.stderr)
+
+
+def test_a_forked_child_asks_for_the_stream_anew():
+    """A child of fork() cannot use its parent's device: torch's current_stream() refuses there, so it has to be asked, as
+    before the first call.  With stand-ins for torch's functions, in a process of its own, without a device."""
+    code = """
+import importlib, os
+capi = importlib.import_module("hotspa-ae_amd.capi")
+call, parent, asked = capi.native(), os.getpid(), []
+def current_stream():
+    if os.getpid() != parent:
+        raise RuntimeError("a forked child")
+    asked.append(1)
+    return 0
+call.setup(capi._dtype_codes(), current_stream, lambda: 0, lambda device: 0)
+for _ in range(3):
+    assert call.hk_unary(0, 6, None, None, 0, None) == 0     # no elements: nothing is launched
+assert asked == [1]
+pid = os.fork()
+if pid == 0:
+    try:
+        call.hk_unary(0, 6, None, None, 0, None)
+    except RuntimeError as e:
+        os._exit(7 if "a forked child" in str(e) else 1)
+    os._exit(0)
+assert os.waitstatus_to_exitcode(os.waitpid(pid, 0)[1]) == 7
+assert call.hk_unary(0, 6, None, None, 0, None) == 0 and asked == [1]
+print("done")
+"""
+    done = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120,
+                          cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+    assert done.returncode == 0 and done.stdout == "done\n", done.stderr
