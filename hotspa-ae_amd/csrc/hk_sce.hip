@@ -374,7 +374,13 @@ void sce_sparse_bwd_kernel(SceArgs a) {
       span.store(dxr, v, f);
     });
   }
-  if constexpr (RAGGED) span.store_edge(dxr, edge * scale - (span.edge == lab ? g : 0.f));
+  if constexpr (RAGGED) {
+    float d = edge * scale - (span.edge == lab ? g : 0.f);
+    // a row of one class (uniform; such a row has no vectors): the element over itself is exactly one and its gradient
+    // exactly zero, where the line above, contracted, leaves the rounding error of 1 / edge
+    if (a.cols == 1) d = edge / p.v[1] * g - (lab == 0 ? g : 0.f);
+    span.store_edge(dxr, d);
+  }
 }
 
 // ------------------------------- long rows ---------------------------------

@@ -152,3 +152,25 @@ def test_large_common_offset(hk, cuda):
         helpers.assert_close(tloss, oracle.sce_sparse_fwd(x, lab, IGN), "fp32", "loss")
         edx = oracle.sce_sparse_bwd(x, lab, g, IGN)
         helpers.assert_close(tdx, edx, "fp32", "dlogits")
+
+
+@pytest.mark.parametrize("dtype", ["fp32", "bf16", "fp16"])
+def test_gradient_of_one_class_is_exactly_zero(hk, cuda, dtype):
+    """A row of one class: its probability is the element over itself, whatever is left of the exponent's rounding in it."""
+    import torch
+    dt = {"fp32": torch.float32, "bf16": torch.bfloat16, "fp16": torch.float16}[dtype]
+    x = torch.cat([torch.linspace(-700, 700, 20011), torch.linspace(-4, 4, 4001)]).to(dt)[:, None].to(cuda)
+    rows = x.shape[0]
+    labels = torch.zeros(rows, dtype=torch.int64, device=cuda)
+    for shift in (0, 1):                             # rows one after the other, and an element apart
+        tx = x if shift == 0 else torch.cat([x, x], 1)[:, 1:]
+        for g in (1.0, 0.3, -1.7e-3, 123.0):
+            grad = torch.full((rows,), g, dtype=dt, device=cuda)
+            out = torch.full((rows, 1), 5.0, dtype=dt, device=cuda)
+            hk.sce_sparse_bwd(tx, labels, grad, out, IGN)
+            torch.cuda.synchronize()
+            assert torch.count_nonzero(out) == 0, (g, int(torch.count_nonzero(out)))
+            out.fill_(5.0)
+            hk.sce_sparse_bwd_reduced(x, labels, grad[:1], 0.25, out, IGN)
+            torch.cuda.synchronize()
+            assert torch.count_nonzero(out) == 0, (g, int(torch.count_nonzero(out)))
