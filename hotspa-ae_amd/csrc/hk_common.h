@@ -241,8 +241,9 @@ template <typename T, bool SHIFT>
 struct RaggedRow {
   static constexpr int N = VecIO<T>::N;
   int cols, lead;
-  __device__ __forceinline__ RaggedRow(const T* row, int cols_) : cols(cols_), lead(0) {
-    if constexpr (SHIFT && sizeof(T) == 2) lead = int(reinterpret_cast<uintptr_t>(row) >> 1) & 1;
+  // spare: 1 where the plan's vectors hold an element more than the row (see plan_spare), else 0: no shift
+  __device__ __forceinline__ RaggedRow(const T* row, int cols_, int spare) : cols(cols_), lead(0) {
+    if constexpr (SHIFT && sizeof(T) == 2) lead = int(reinterpret_cast<uintptr_t>(row) >> 1) & spare;
   }
   __device__ __forceinline__ bool live(int v) const { return v * N - lead < cols; }
   __device__ __forceinline__ int column(int v) const {
@@ -265,11 +266,18 @@ struct RaggedRow {
     }
   }
 };
-// vectors of a ragged row's plan: one more where a row may start on an odd boundary
-template <typename T>
-inline int ragged_vectors(int64_t cols, bool odd) {
-  constexpr int N = VecIO<T>::N;
-  return int((cols + (sizeof(T) == 2 && odd ? 1 : 0) + N - 1) / N);
+// The plan (threads, vectors per thread) of a ragged row of whole vectors: `worth(threads, nv)` says whether the plan of a
+// vector more, which RaggedRow's shift needs there, is the better one where rows start on odd boundaries (shape(nvec,
+// &threads, &nv) picks a plan).  nvec, *threads and *nv become what is taken; returns RaggedRow's `spare`.
+template <typename T, typename Shape, typename Worth>
+inline int plan_spare(int cols, bool odd, int& nvec, int& threads, int& nv, Shape&& shape, Worth&& worth) {
+  if (cols % VecIO<T>::N != 0) return 1;
+  int t = 0, n = 0;
+  if (sizeof(T) != 2 || !odd || !shape(nvec + 1, &t, &n) || !worth(t, n)) return 0;
+  ++nvec;
+  threads = t;
+  nv = n;
+  return 1;
 }
 
 // Stores vector v of a row.  SAME: an element that two vectors hold was computed to the same bits in both, so the

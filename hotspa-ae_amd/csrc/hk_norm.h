@@ -30,6 +30,7 @@ struct NormFwdArgs {
   LevelSteps x_lv, res_lv, y_lv, xout_lv;
   int cols;
   int nvec;
+  int spare;             // see RaggedRow
   float eps;
   float inv_cols;
   int is_rms;

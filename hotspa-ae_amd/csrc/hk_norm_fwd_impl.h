@@ -258,7 +258,7 @@ void norm_fwd_any_kernel(NormFwdArgs a) {
 
   float v[NV][VEC];
   const T* xr = static_cast<const T*>(a.x) + row * a.x_pitch + outer_level_offset(a.x_lv);
-  const RaggedRow<T, kShift> odd(xr, a.cols);
+  const RaggedRow<T, kShift> odd(xr, a.cols, a.spare);
   {
     const T* rr = HAS_RES ? static_cast<const T*>(a.residual) + row * a.res_pitch + outer_level_offset(a.res_lv) : nullptr;
     u32x4 raw[NV];
@@ -666,7 +666,21 @@ int norm_fwd_typed(NormFwdArgs a, hipStream_t s) {
   int lanes = 0;
   const uintptr_t starts = reinterpret_cast<uintptr_t>(a.x) |
                            uintptr_t((a.x_pitch | a.x_lv.p1 | a.x_lv.p2) * int64_t(sizeof(T)));
-  if (a.cols >= VEC && pick_any_shape(ragged_vectors<T>(a.cols, (starts & 3) != 0), &lanes, &nv)) {
+  if (a.cols >= VEC && pick_any_shape(a.nvec, &lanes, &nv)) {
+    // The vector more is for free where a wavefront has the lanes (LayerNorm does not shift there, see kShift); from a
+    // wavefront to a workgroup it pays for few rows, which then have more wavefronts each; between workgroups where the row
+    // is long enough to be bound by its accesses and does not go to half as many threads of twice the vectors for it.
+    // bf16 us without / with it, LayerNorm: 40000 x 64 5.1 / 7.0, x 256 12.8 / 20.6, 256 x 2048 6.0 / 4.8, 12288 x 2048
+    // 24.5 / 31.5, x 4096 48 / 58, 4096 x 8192 35.6 / 36.0, 1024 x 16384 19.1 / 27.9, x 24576 37 / 27; RMSNorm: 40000 x 192
+    // 11.8 / 10.8, x 256 12.2 / 18.0, 256 x 2048 5.1 / 4.2, 12288 x 2048 22.0 / 24.8, x 4096 43 / 46, x 6144 67 / 62, 4096 x
+    // 8192 30.9 / 29.0, 256 x 8192 5.3 / 5.9, 1024 x 16384 17.4 / 22.1, x 24576 32 / 22; 256 x 65536, which no workgroup
+    // holds with a vector more, 20 / 304 and 19 / 226.
+    a.spare = plan_spare<T>(a.cols, (starts & 3) != 0, a.nvec, lanes, nv, pick_any_shape, [&](int l, int n) {
+      if (l <= kWave) return a.is_rms && l == lanes && n == nv;
+      if (lanes <= kWave) return a.rows <= 4 * int64_t(device_cu_count());
+      if (lanes % 512 == 0) return a.is_rms && nv == 2 && a.rows > 2 * int64_t(device_cu_count());
+      return a.nvec > (a.is_rms ? 512 : 1024);
+    });
     if (a.is_rms) return has_res ? launch_norm_fwd_any<T, true, true>(a, lanes, nv, s) : launch_norm_fwd_any<T, false, true>(a, lanes, nv, s);
     return has_res ? launch_norm_fwd_any<T, true, false>(a, lanes, nv, s) : launch_norm_fwd_any<T, false, false>(a, lanes, nv, s);
   }

@@ -26,6 +26,7 @@ struct SoftmaxArgs {
   LevelSteps x_lv, dy_lv, out_lv;
   int cols;
   int nvec;
+  int spare;        // see RaggedRow
 };
 
 template <typename T, int NV, int LPR, bool RAGGED>
@@ -41,7 +42,7 @@ void softmax_fwd_kernel(SoftmaxArgs a) {
   const T* xr = static_cast<const T*>(a.x) + row * a.x_pitch + outer_level_offset(a.x_lv);
   // slots past the row's end hold -inf, which changes neither the maximum nor the sum; in a ragged row they hold
   // elements of the row a second time, which the maximum may see and the sum leaves out
-  [[maybe_unused]] const RaggedRow<T, true> odd(xr, a.cols);
+  [[maybe_unused]] const RaggedRow<T, true> odd(xr, a.cols, a.spare);
   u32x4 raw[NV];
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
@@ -129,7 +130,7 @@ void softmax_bwd_kernel(SoftmaxArgs a) {
 
   const T* yr = static_cast<const T*>(a.x) + row * a.x_pitch + outer_level_offset(a.x_lv);
   const T* dyr = static_cast<const T*>(a.dy) + row * a.dy_pitch + outer_level_offset(a.dy_lv);
-  [[maybe_unused]] const RaggedRow<T, true> odd(yr, a.cols);
+  [[maybe_unused]] const RaggedRow<T, true> odd(yr, a.cols, a.spare);
   u32x4 ry[NV], rdy[NV];
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
@@ -572,8 +573,22 @@ static int softmax_lastdim_typed(SoftmaxArgs a, hipStream_t s) {
   const uintptr_t boundary = reinterpret_cast<uintptr_t>(a.x) | reinterpret_cast<uintptr_t>(a.dy) |
                              reinterpret_cast<uintptr_t>(a.out) | uintptr_t(a.x_pitch * int64_t(sizeof(T))) |
                              uintptr_t(a.out_pitch * int64_t(sizeof(T)));
-  a.nvec = ragged_vectors<T>(a.cols, (boundary & 3) != 0);
-  const bool shaped = pick_softmax_shape(a.nvec, vec_ok, (boundary & 3) != 0, max_nv, BWD, &threads, &nv);
+  a.nvec = (a.cols + VEC - 1) / VEC;
+  const auto shape = [&](int nvec, int* t, int* n) {
+    return pick_softmax_shape(nvec, vec_ok, (boundary & 3) != 0, max_nv, BWD, t, n);
+  };
+  const bool shaped = shape(a.nvec, &threads, &nv);
+  if (shaped && !vec_ok) {
+    const bool odd = ((reinterpret_cast<uintptr_t>(a.x) | uintptr_t(a.x_pitch * int64_t(sizeof(T)))) & 3) != 0;
+    // The vector more is for free where the lanes are there.  Past a wavefront the backward, whose two operands pay for
+    // accesses off 4 bytes, is the better for it, the forward only in a wavefront and where few wide threads hold the row.
+    // bf16 us without / with it, forward: 40000 x 64 4.1 / 5.3, x 192 9.4 / 8.5, 4096 x 1024 5.8 / 5.3, 12288 x 2048 19.5 /
+    // 22.6, 4096 x 4096 16 / 17, x 8192 28.7 / 30.4, x 16384 60 / 54; backward: 40000 x 64 4.9 / 6.3, x 192 12.0 / 10.4,
+    // x 512 22.0 / 22.9, 4096 x 4096 22.0 / 18.9, x 8192 42.6 / 33.4, 1000 x 32768 (no workgroup holds a vector more) 47 / 124.
+    a.spare = plan_spare<T>(a.cols, odd, a.nvec, threads, nv, shape, [&](int t, int n) {
+      return a.nvec <= 64 ? t == threads && n == nv : BWD || t == 64 || threads == 1024 || nv == 8;
+    });
+  }
   if (vec_ok && shaped) return launch_softmax<T, BWD, false>(a, threads, nv, s);
   if (a.n0 != a.rows) {
     set_last_error("softmax: rows on several levels need 16-byte aligned rows and steps");

@@ -666,3 +666,71 @@ def test_rows_on_different_boundaries(hk, cuda, dtype, x_at, other_at):
             helpers.assert_close(tsum.contiguous(), ex, dtype, "x %d" % cols)
             helpers.assert_close(rs, ers, "fp32", "rsigma %d" % cols)
             assert _guards_untouched(zb, tz) and _guards_untouched(xb, tsum), cols
+
+
+# whole vectors that start on odd boundaries, where a start one element earlier needs a vector more: rows with lanes to spare
+# for it and without, a wavefront's longest (few rows and many), workgroups, and the most that a workgroup holds
+@pytest.mark.parametrize("rows,cols", [(33, 64), (33, 192), (33, 512), (9, 2048), (1100, 2048), (9, 4096), (7, 8192), (600, 8192),
+                                       (5, 12288), (5, 16384), (3, 24576), (3, 32768), (3, 40960), (3, 65536)])
+@pytest.mark.parametrize("pitch", [1, 8])
+def test_whole_vectors_on_odd_boundaries(hk, cuda, rows, cols, pitch):
+    import torch
+    x, dy = (helpers.draw(s + cols + rows, (rows, cols), dtype="bf16") for s in (9800, 9900))
+    at = lambda a, fill=None: _placed(cuda, a, "bf16", 1, cols + pitch, fill)
+    tx, tdy = at(x)[1], at(dy)[1]
+    yb, ty = at(x, 0.0)
+    db, dx = at(x, 0.0)
+    hk.softmax_fwd(tx, ty)
+    hk.softmax_bwd(ty, tdy, dx)
+    torch.cuda.synchronize()
+    assert _guards_untouched(yb, ty) and _guards_untouched(db, dx)
+    helpers.assert_close(ty.contiguous(), torch.softmax(tx.double(), -1).cpu().numpy(), "bf16", "softmax y")
+    yd, dd = ty.double(), tdy.double()
+    helpers.assert_close(dx.contiguous(), (yd * (dd - (yd * dd).sum(-1, keepdim=True))).cpu().numpy(), "bf16", "softmax dx",
+                         scale=float((yd * dd).square().mean().sqrt()))
+    g, b = (helpers.to_torch(helpers.draw(s, (cols,), "uniform", 0.5, 1.5, "bf16"), "bf16", cuda) for s in (9701, 9702))
+    xd = tx.double()
+    mean, var = xd.mean(-1, keepdim=True), xd.var(-1, unbiased=False, keepdim=True)
+    mu, rs = torch.empty(rows, device=cuda), torch.empty(rows, device=cuda)
+    zb, tz = at(x, 0.0)
+    hk.layer_norm_fwd(tx, g, b, tz, mu, rs, 1e-5)
+    torch.cuda.synchronize()
+    helpers.assert_close(tz.contiguous(), ((xd - mean) / (var + 1e-5).sqrt() * g.double() + b.double()).cpu().numpy(), "bf16", "z")
+    helpers.assert_close(rs, (1 / (var + 1e-5).sqrt())[:, 0].cpu().numpy(), "fp32", "rsigma")
+    assert _guards_untouched(zb, tz)
+    zb, tz = at(x, 0.0)
+    hk.dropout_add_ln_fwd(tx, None, g, None, tz, None, mu, rs, 1e-5, True)
+    torch.cuda.synchronize()
+    want = 1 / (xd.square().mean(-1, keepdim=True) + 1e-5).sqrt()
+    helpers.assert_close(tz.contiguous(), (xd * want * g.double()).cpu().numpy(), "bf16", "z")
+    helpers.assert_close(rs, want[:, 0].cpu().numpy(), "fp32", "rsigma")
+    assert _guards_untouched(zb, tz)
+
+
+@pytest.mark.parametrize("what,rows,cols", [("softmax_bwd", 256, 32768), ("softmax_fwd", 256, 65536), ("layer_norm", 256, 65536),
+                                            ("rms_norm", 256, 65536), ("layer_norm", 40000, 256), ("rms_norm", 40000, 256)])
+def test_whole_vectors_on_odd_boundaries_cost_no_more(hk, cuda, what, rows, cols):
+    """A row of whole vectors against the row one vector shorter, which has one to spare: it took 1.6 times as long, and 8 to 17
+    times where the vector more did not fit a workgroup.  Without the shift a gradient's accesses lie off 4 bytes, for which it takes 1.33 times as long (11.5 against 8.6 us at 256 x 32768); the others take the same time."""
+    import torch
+
+    def time_of(n, calls=20):
+        x, y, z = (torch.randn(rows * (n + 1) + 1, device=cuda).bfloat16()[1:].view(rows, n + 1)[:, :n] for _ in range(3))
+        g, m, r = torch.ones(n, device=cuda).bfloat16(), torch.empty(rows, device=cuda), torch.empty(rows, device=cuda)
+        run = {"softmax_fwd": lambda: hk.softmax_fwd(x, y), "softmax_bwd": lambda: hk.softmax_bwd(x, y, z),
+               "layer_norm": lambda: hk.layer_norm_fwd(x, g, g, y, m, r, 1e-5),
+               "rms_norm": lambda: hk.dropout_add_ln_fwd(x, None, g, None, y, None, m, r, 1e-5, True)}[what]
+        best = 1e9
+        for _ in range(8):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            run()
+            a.record()
+            for _ in range(calls):
+                run()
+            b.record()
+            torch.cuda.synchronize()
+            best = min(best, a.elapsed_time(b) * 1e3 / calls)
+        return best
+
+    whole, shorter = time_of(cols), time_of(cols - 8)
+    assert whole < 1.5 * shorter, (whole, shorter)
