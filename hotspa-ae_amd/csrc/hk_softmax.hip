@@ -186,7 +186,7 @@ void softmax_bwd_kernel(SoftmaxArgs a) {
 // Bound by HBM and, on odd planes, by the cache lines that neighbouring workgroups share: runs of 8 or 16 of them stay
 // on one XCD, whose L2 then sees each line whole (8 x 21 x 263169 fp32, forward / backward: 82 / 117 -> 72 / 106 us).  One
 // thread per column that passed over it three times measured (forward / backward, us) 150 / 160 at 8 x 21 x 263169 fp32,
-// now 71 / 96 (5.0 and 5.5 TB/s; 65 / 91 at 263168); 81 / 77 at 8 x 21 x 263168 bf16, now 33 / 45; 143 / 103 at 16 x 150 x
+// now 69 / 92 (5.1 and 5.8 TB/s; 62 / 91 at 263168); 81 / 77 at 8 x 21 x 263168 bf16, now 33 / 45; 143 / 103 at 16 x 150 x
 // 16384 bf16, now 37 / 43; 447 / 356 at 8 x 256 x 40000 fp32, now 123 / 180.
 constexpr int kDimVecs = 8;      // most entries per lane
 // f[0..N): this lane's values; on return the slices' maximum or sum (in slice order) of each, the same in every slice.
@@ -672,11 +672,13 @@ static int softmax_strided_typed(const void* x, const void* dy, void* out, int64
       const int slices = int((dim + most - 1) / most), nk = int((dim + slices - 1) / slices);
       a.slices = int((dim + nk - 1) / nk);
       if (a.total <= 0x7fffffffLL) {
-        // fp32 planes that fill the device many times over, up to 32 entries: runs of 2 KiB and 4 KiB of an entry per
-        // workgroup instead of 1 KiB share fewer lines (8 x 21 x 263169 forward 71.8 / 69.7 / 69.0, backward 106 / 103 /
-        // 96 us with runs of 64 / 128 / 256 lanes; 8 x 21 x 263168 62.9 / 64.0 / 65.5 and 93.1 / 93.1 / 90.3); not 16-bit
-        // ones (8 x 21 x 263169 35.3 / 37.8 / 48.1 and 50.3 / 51.0 / 55.8)
-        const bool wide = VEC == 4 && a.slices <= 4 && a.total >= cus * 2048;
+        // fp32 planes that share cache lines and fill the device many times over, up to 32 entries: runs of 2 KiB and 4 KiB
+        // of an entry per workgroup instead of 1 KiB share fewer lines (8 x 21 x 263169 forward 71.8 / 69.7 / 69.0, backward
+        // 106 / 103 / 96 us with runs of 64 / 128 / 256 lanes).  Planes of whole lines have nothing to gain (runs of 64 lanes
+        // / of 128 forward, 256 backward: 16 x 2 x 1048576 42.3 / 44.3 and 60.9 / 62.7 us, 8 x 9 x 524288 49.4 / 49.4 and 70.8 /
+        // 73.3, 8 x 21 x 263168 62.3 / 63.8 and 90.7 / 88.7), nor 16-bit ones (8 x 21 x 263169 35.3 / 37.8 / 48.1 and 50.3 /
+        // 51.0 / 55.8)
+        const bool wide = VEC == 4 && a.slices <= 4 && a.total >= cus * 2048 && bytes % 128 != 0;
         // PLAIN: 16-bit entries in runs of 1 KiB, and the few, are stored through the cache (8 x 21 x 263170 bf16 35.5 /
         // 48.8 -> 33.9 / 44.4, 4 x 65 x 355 5.9 / 5.1 -> 5.4 / 4.4; fp32 70.8 / 104 -> 73.2 / 112, and 16-bit ones in runs of
         // 512 bytes, 16 x 150 x 16384, 37.2 / 42.3 -> 39.9 / 47.1 us, are not)
