@@ -170,10 +170,12 @@ struct DalFwdArgs {
 // IT / RT / WT: input, residual and weight element types; NC: chunks per thread.  A block holds
 // blockDim.x / tpr row groups; every group takes part in the (block-wide) reduction barrier, a group
 // past the last row works on a copy of the last row and stores nothing.
-template <typename IT, typename RT, typename WT, int NC>
-// (one chunk a thread: 8 wavefronts per SIMD, where the kept elements' lane masks would take scalar registers for 7, 6578 x 512
-// fp32 both ways 36.8 -> 36.5 us; two chunks are the better for 7, 8192 x 4096 bf16 113.8 against 115.1)
-__global__ __launch_bounds__(256, NC == 1 ? 8 : 1)
+// DROP == false, built for one chunk: nothing is dropped.  Without the kept elements' lane masks 8 wavefronts fit a SIMD (60
+// scalar registers instead of 103; 40000 x 256 bf16 with an fp32 weight 30.7 -> 25.4 us, with an fp32 residual 33.4 -> 30.2).
+// Asked for 8 of them with the masks, the compiler spills scalars: 1190 x 1104 bf16 7.5 against 6.8 us, 16384 x 1024 37.1
+// against 35.0, and only 6578 x 512 with an fp32 residual 12.2 against 12.6.
+template <typename IT, typename RT, typename WT, int NC, bool DROP>
+__global__ __launch_bounds__(256)
 void dal_fwd_kernel(DalFwdArgs a) {
   __shared__ float red[kMaxWaves * 3];
   const int tpr = a.tpr;
@@ -196,7 +198,7 @@ void dal_fwd_kernel(DalFwdArgs a) {
     rowscale_val = Cvt<IT>::load(static_cast<const IT*>(a.rowscale) + row);
   }
   const bool load_x0 = row_x0 > 0;
-  const bool dropout = a.dropout != 0;
+  const bool dropout = DROP && a.dropout != 0;
 
   // Every load of the row is issued before the first one is waited for (the optional operands sit behind
   // uniform branches; unpacking inside those branches would serialise the loads).  A thread past the row's
@@ -885,9 +887,12 @@ int hk_dropout_add_ln_fwd_ex(const hkDropoutAddLnFwdParams* pp, hkStream_t strea
     using WT = typename decltype(wt)::type;
     profile_before(s);
     switch (nc) {
-      case 1: HK_LAUNCH((dal_fwd_kernel<IT, RT, WT, 1>), grid, block, 0, s, a); break;
-      case 2: HK_LAUNCH((dal_fwd_kernel<IT, RT, WT, 2>), grid, block, 0, s, a); break;
-      default: HK_LAUNCH((dal_fwd_kernel<IT, RT, WT, 4>), grid, block, 0, s, a); break;
+      case 1:
+        if (dropout) HK_LAUNCH((dal_fwd_kernel<IT, RT, WT, 1, true>), grid, block, 0, s, a);
+        else HK_LAUNCH((dal_fwd_kernel<IT, RT, WT, 1, false>), grid, block, 0, s, a);
+        break;
+      case 2: HK_LAUNCH((dal_fwd_kernel<IT, RT, WT, 2, true>), grid, block, 0, s, a); break;
+      default: HK_LAUNCH((dal_fwd_kernel<IT, RT, WT, 4, true>), grid, block, 0, s, a); break;
     }
     profile_after(s);
     return launch_check("dal_fwd_kernel");
