@@ -518,10 +518,9 @@ static int launch_softmax_nv(const SoftmaxArgs& a, int nv, dim3 grid, dim3 block
       }
       [[fallthrough]];
     case 8:
-      if constexpr (LPR == 0) {
+      if constexpr (!BWD && LPR == 0) {
         if (nv == 8) {
-          if constexpr (BWD) HK_LAUNCH((softmax_bwd_kernel<T, 8, LPR, RAGGED>), grid, block, 0, s, a);
-          else HK_LAUNCH((softmax_fwd_kernel<T, 8, LPR, RAGGED>), grid, block, 0, s, a);
+          HK_LAUNCH((softmax_fwd_kernel<T, 8, LPR, RAGGED>), grid, block, 0, s, a);
           break;
         }
       }
@@ -608,14 +607,21 @@ static int softmax_lastdim_typed(SoftmaxArgs a, hipStream_t s) {
   }
 }
 
-template <typename T, bool BWD, int LX, bool PLAIN>
-static void launch_softmax_dim(const SoftmaxDimArgs& a, int nk, hipStream_t s) {
+// LEAST, MOST: the entries per lane that the plan gives this launch
+template <typename T, bool BWD, int LX, bool PLAIN, int LEAST, int MOST>
+static int launch_softmax_dim(const SoftmaxDimArgs& a, int nk, hipStream_t s) {
+  if (nk < LEAST || nk > MOST) {
+    set_last_error("softmax: no kernel for %d entries per lane", nk);
+    return HK_ERR_UNSUPPORTED;
+  }
   const dim3 grid{unsigned((a.total + LX - 1) / LX)}, block{unsigned(LX), unsigned(a.slices)};
   const size_t lds = a.slices > 1 ? size_t(a.slices + 1) * LX * VecIO<T>::N * sizeof(float) : 0;
 #define HK_DIM_CASE(N)                                                              \
   case N:                                                                           \
-    if constexpr (BWD) HK_LAUNCH((softmax_bwd_dim_kernel<T, N, LX, PLAIN>), grid, block, lds, s, a); \
-    else HK_LAUNCH((softmax_fwd_dim_kernel<T, N, LX, PLAIN>), grid, block, lds, s, a);     \
+    if constexpr (N >= LEAST && N <= MOST) {                                        \
+      if constexpr (BWD) HK_LAUNCH((softmax_bwd_dim_kernel<T, N, LX, PLAIN>), grid, block, lds, s, a); \
+      else HK_LAUNCH((softmax_fwd_dim_kernel<T, N, LX, PLAIN>), grid, block, lds, s, a);   \
+    }                                                                               \
     break;
   profile_before(s);
   switch (nk) {
@@ -623,6 +629,7 @@ static void launch_softmax_dim(const SoftmaxDimArgs& a, int nk, hipStream_t s) {
   }
 #undef HK_DIM_CASE
   profile_after(s);
+  return launch_check("softmax_dim_kernel");
 }
 
 template <typename T, typename CT, bool BWD>
@@ -666,9 +673,10 @@ static int softmax_strided_typed(const void* x, const void* dy, void* out, int64
       // of instructions.  GPU us, forward / backward, with 6 to 8 entries in a wavefront's and so: 4 x 65 x 355 bf16
       // 8.6 / 7.5 and 4.4 / 3.6, 2 x 250 x 200 fp32 9.4 / 10.7 and 5.8 / 5.9, 3 x 57 x 5877 fp32 5.8 / 6.3 and 4.5 / 4.4,
       // 4 x 100 x 10000 bf16 10.1 / 8.0 and 7.8 / 6.8; at 2 x 128 x 16384 fp32 they meet, 8.9 / 11.1 and 9.9 / 10.8.
+      constexpr int kFull = BWD && VEC == 8 ? 6 : kDimVecs;
       const bool few = a.total <= cus * 64 && a.total * dim <= cus * 3072;
       const int lx = few && a.total <= cus * 16 && dim > 64 ? 16 : 32, fewest = int((dim + 1024 / lx - 1) / (1024 / lx));
-      const int most = std::max(few ? 2 : BWD && VEC == 8 ? 6 : kDimVecs, fewest);
+      const int most = std::max(few ? 2 : kFull, fewest);
       const int slices = int((dim + most - 1) / most), nk = int((dim + slices - 1) / slices);
       a.slices = int((dim + nk - 1) / nk);
       if (a.total <= 0x7fffffffLL) {
@@ -682,12 +690,15 @@ static int softmax_strided_typed(const void* x, const void* dy, void* out, int64
         // PLAIN: 16-bit entries in runs of 1 KiB, and the few, are stored through the cache (8 x 21 x 263170 bf16 35.5 /
         // 48.8 -> 33.9 / 44.4, 4 x 65 x 355 5.9 / 5.1 -> 5.4 / 4.4; fp32 70.8 / 104 -> 73.2 / 112, and 16-bit ones in runs of
         // 512 bytes, 16 x 150 x 16384, 37.2 / 42.3 -> 39.9 / 47.1 us, are not)
-        if (lx == 16) launch_softmax_dim<T, BWD, 16, true>(a, nk, s);
-        else if (few) launch_softmax_dim<T, BWD, 32, true>(a, nk, s);
-        else if (a.slices > 16) launch_softmax_dim<T, BWD, 32, false>(a, nk, s);
-        else if (wide) launch_softmax_dim<T, BWD, (VEC == 4 ? (BWD ? 256 : 128) : 64), VEC == 8>(a, nk, s);
-        else launch_softmax_dim<T, BWD, 64, VEC == 8>(a, nk, s);
-        return launch_check("softmax_dim_kernel");
+        // What nk can be.  64 slices: 2 to 4, for 65 to 256 entries.  The few in 32: up to 6, because at 192 entries and past 16
+        // vectors per compute unit they are no longer few.  More than 16 slices are full ones, of `most` entries each.
+        if (lx == 16) return launch_softmax_dim<T, BWD, 16, true, 2, 4>(a, nk, s);
+        if (few) return launch_softmax_dim<T, BWD, 32, true, 1, 6>(a, nk, s);
+        if (a.slices > 16) return launch_softmax_dim<T, BWD, 32, false, kFull, kDimVecs>(a, nk, s);
+        if constexpr (VEC == 4) {
+          if (wide) return launch_softmax_dim<T, BWD, (BWD ? 256 : 128), false, 1, kDimVecs>(a, nk, s);
+        }
+        return launch_softmax_dim<T, BWD, 64, VEC == 8, 1, kFull>(a, nk, s);
       }
     }
   }

@@ -303,6 +303,32 @@ def test_softmax_dim_launches(hk, cuda, dtype, outer, dim, inner):
                      2.0 ** -25 * (dtype == "fp16")).all()), o
 
 
+@pytest.mark.parametrize("dtype", ["fp32", "bf16", "fp16"])
+def test_softmax_dim_of_every_length(hk, cuda, dtype):
+    """Every number of entries, with the fewest positions, some more, the most that count as few, and one more: the plans
+    name kernels that are built."""
+    import torch
+    dt = {"fp32": torch.float32, "bf16": torch.bfloat16, "fp16": torch.float16}[dtype]
+    vec, cus = 16 // ES[dtype], torch.cuda.get_device_properties(0).multi_processor_count
+    unit = {"fp32": 2.0 ** -24, "bf16": 2.0 ** -8, "fp16": 2.0 ** -11}[dtype]
+    gen = torch.Generator(device=cuda).manual_seed(3)
+    for dim in range(1, 257):
+        for vectors in {3, 16 * cus, 16 * cus + 1, min(64 * cus, 3072 * cus // dim), min(64 * cus, 3072 * cus // dim) + 1}:
+            x, dy = (torch.randn(1, dim, vectors * vec - 1, generator=gen, device=cuda).to(dt) for _ in range(2))
+            y, dx = torch.empty_like(x), torch.empty_like(x)
+            hk.softmax_fwd(x, y, 1)
+            hk.softmax_bwd(y, dy, dx, 1)
+            # against fp32: both round each of dim terms and their quotient, and the argument of the exponential (up to 16)
+            # half a unit of 2^-20; dx the same of its terms
+            eps = (2 * dim + 64) * 2.0 ** -24
+            want = torch.softmax(x.float(), 1)
+            assert bool(((y.float() - want).abs() <= want * (unit + eps) + 2.0 ** -25).all()), (dim, vectors)
+            yf, df = y.float(), dy.float()
+            dot = (yf * df).sum(1, keepdim=True)
+            terms = yf * (df.abs() + (yf * df.abs()).sum(1, keepdim=True))
+            assert bool(((dx.float() - yf * (df - dot)).abs() <= terms * (unit + eps) + 2.0 ** -25).all()), (dim, vectors)
+
+
 def _norm_lengths(dtype):
     vec = 16 // ES[dtype]
     out = {v * vec + k for v in (1, 2, 8, 16, 32, 64, 65, 128, 192, 256, 300, 512, 1024) for k in (0, 1, vec - 1)}
