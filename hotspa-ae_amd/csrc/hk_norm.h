@@ -63,7 +63,6 @@ struct NormBwdArgs {
   int nvec;
   int part_pitch;       // elements between partial rows: cols rounded up to whole vectors
   int tpr;              // threads per row
-  int fold_both;        // the staging area of the column sums' fold holds both of them
   float eps;
   float inv_cols;
   int stat_kind;
@@ -76,7 +75,6 @@ struct BwdPlan {
   bool any;             // the instance for rows of any length and alignment
   int lpr;              // lanes of a wavefront that hold a row; 0: whole wavefronts, with a barrier per row
   int tpr, nv, rpb, grid;
-  bool fold_both;
   int block;
   size_t lds_bytes;
   size_t ws_bytes;

@@ -77,7 +77,7 @@ void norm_bwd_kernel(NormBwdArgs a) {
   constexpr bool WITH_DB = EXTRA || MODE != BWD_RMS;   // column sums of dy (dbeta)
   using StatT = typename std::conditional<STATS_F32, float, T>::type;
   using RowSums = SumTuple<KS>;
-  extern __shared__ __align__(16) float lds[];   // [rows_per_block, part_pitch] column-sum staging, of one sum or both
+  extern __shared__ __align__(16) float lds[];   // [2][rows_per_block, part_pitch] staging of both column sums (staging_bytes)
   __shared__ __align__(16) float red[2][kMaxWaves * KS];  // double-buffered by step parity
 
   const int tpr = FIXED ? MAXT : LPR ? LPR : a.tpr;   // without LPR a multiple of 64: a wavefront never straddles two rows
@@ -395,19 +395,11 @@ void norm_bwd_kernel(NormBwdArgs a) {
       st16(dst + int64_t(blockIdx.x) * pitch + c, u32x4{f2u(r[0]), f2u(r[1]), f2u(r[2]), f2u(r[3])});
     }
   };
-  const bool both = WITH_DB && a.fold_both;   // uniform: the staging area holds both sums
   put(lds + group * pitch, dg, false);
-  if (both) put(lds + region + group * pitch, db, false);
+  if constexpr (WITH_DB) put(lds + region + group * pitch, db, false);
   __syncthreads();
   fold(lds, outs[0]);
-  if constexpr (WITH_DB) {
-    if (!both) {
-      __syncthreads();
-      put(lds + group * pitch, db, false);
-      __syncthreads();
-    }
-    fold(both ? lds + region : lds, outs[1]);
-  }
+  if constexpr (WITH_DB) fold(lds + region, outs[1]);
 }
 
 // Folds the [nparts, pitch] fp32 partial rows into dgamma / dbeta of type T.  Rows of whole 16-byte vectors of T:
@@ -583,6 +575,14 @@ void norm_bwd_generic_cols_kernel(NormBwdArgs a, int mode, T* dgamma, T* dbeta) 
   }
 }
 
+// LDS in which the row groups of a workgroup stage both column sums.  A thread has 8 columns in workgroups of up to 1024
+// threads, or 16 in up to 512, so that this is at most 64 KiB (8 groups of 1021 to 1024 columns, say); with the 256 bytes of
+// the reductions' own array it is within the 160 KiB that a workgroup may have, one workgroup being all that a compute
+// unit is given.
+static inline size_t staging_bytes(int groups, int pitch) {
+  return groups > 1 ? size_t(2) * size_t(groups) * size_t(pitch) * sizeof(float) : 0;
+}
+
 // Many rows of up to 32 vectors, dense or pitched, on any boundary, without optional operands: 16 or 32 lanes to a row,
 // a vector per lane, two rows in flight per group.  A wavefront to a row leaves half of its lanes and more idle; that
 // shows once its workgroups, 16 rows each on every compute unit, have to walk (LayerNorm bf16, 32768 x 64 12.9 -> 8.1 us,
@@ -604,9 +604,7 @@ BwdPlan plan_norm_bwd_lanes(int64_t rows, int cols) {
   if (grid <= 0) grid = device_cu_count();
   p.grid = int(std::max<int64_t>(1, std::min<int64_t>(grid, (rows + p.rpb - 1) / p.rpb)));
   p.reg_path = true;
-  const size_t one = size_t(p.rpb) * pitch * sizeof(float);   // at most 64 KiB
-  p.fold_both = 2 * one <= 65536;
-  p.lds_bytes = p.fold_both ? 2 * one : one;
+  p.lds_bytes = staging_bytes(p.rpb, pitch);
   p.ws_bytes = size_t(2) * size_t(p.grid) * pitch * sizeof(float);
   return p;
 }
@@ -623,8 +621,7 @@ BwdPlan plan_norm_bwd_any(int64_t rows, int cols) {
   const int nv = VEC == 4 && nvec > 1024 ? 2 : 1;
   const int tpr = ((nvec + nv - 1) / nv + 63) / 64 * 64;
   if (tpr > 1024) return p;
-  int rpb = std::max(1, 1024 / tpr);
-  while (rpb > 1 && size_t(rpb) * pitch * sizeof(float) > 65536) --rpb;
+  const int rpb = std::max(1, 1024 / tpr);
   int64_t grid = tune_get(TUNE_NORM_BWD_BLOCKS);
   if (grid <= 0) grid = device_cu_count();
   grid = std::min<int64_t>(grid, (rows + rpb - 1) / rpb);
@@ -632,9 +629,7 @@ BwdPlan plan_norm_bwd_any(int64_t rows, int cols) {
   if (grid < 1) grid = 1;
   p.reg_path = p.any = true;
   p.tpr = tpr; p.nv = nv; p.rpb = rpb; p.grid = int(grid); p.block = tpr * rpb;
-  const size_t one = size_t(rpb) * pitch * sizeof(float);
-  p.fold_both = rpb > 1 && 2 * one <= 65536;
-  p.lds_bytes = rpb > 1 ? (p.fold_both ? 2 : 1) * one : 0;
+  p.lds_bytes = staging_bytes(rpb, pitch);
   p.ws_bytes = size_t(2) * size_t(grid) * pitch * sizeof(float);
   return p;
 }
@@ -673,8 +668,6 @@ BwdPlan plan_norm_bwd(int64_t rows, int cols, bool aligned) {
     if (tpr >= 512) rpb = 1;
   }
   rpb = std::max(1, std::min(rpb, max_block / tpr));
-  // staging buffer of the final fold must fit 64 KiB of LDS
-  while (rpb > 1 && size_t(rpb) * cols * sizeof(float) > 65536) --rpb;
   int grid = tune_get(TUNE_NORM_BWD_BLOCKS);
   if (grid <= 0) grid = device_cu_count();   // one 1024-thread workgroup per CU measured fastest
   const int64_t max_useful = (rows + rpb - 1) / rpb;
@@ -682,9 +675,7 @@ BwdPlan plan_norm_bwd(int64_t rows, int cols, bool aligned) {
   if (grid < 1) grid = 1;
   p.reg_path = true;
   p.tpr = tpr; p.nv = nv; p.rpb = rpb; p.grid = grid; p.block = tpr * rpb;
-  const size_t one = size_t(rpb) * cols * sizeof(float);
-  p.fold_both = rpb > 1 && 2 * one <= 65536;
-  p.lds_bytes = rpb > 1 ? (p.fold_both ? 2 : 1) * one : 0;
+  p.lds_bytes = staging_bytes(rpb, cols);
   p.ws_bytes = size_t(2) * grid * cols * sizeof(float);
   return p;
 }
@@ -892,7 +883,6 @@ int norm_bwd_typed(NormBwdArgs a, int mode, void* dgamma, void* dbeta, void* ws,
     a.part_dbeta = nullptr;
   }
   a.tpr = p.tpr;
-  a.fold_both = p.fold_both;
   {
     // the walking kernel's row stride, split over the walk levels (used by the instances with a running walk index)
     const uint64_t stride = uint64_t(p.grid) * uint64_t(p.rpb);
