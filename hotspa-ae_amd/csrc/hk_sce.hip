@@ -8,7 +8,7 @@
 // writes the row once.  Rows whose label equals the ignored index are not read
 // at all: loss 0 / a zero gradient row is written.
 //
-// Sparse labels take rows of any length and alignment this way (see RowSpan); 16-bit rows of 32768 to 98304 columns keep
+// Sparse labels take rows of any length and alignment this way (see RowSpan); 16-bit rows of 32768 to 97792 columns keep
 // a part in LDS (RowTail, sce_packed_kernel), longer ones are streamed (sce_long_kernel).
 #include "hk_common.h"
 
@@ -384,7 +384,7 @@ void sce_sparse_bwd_kernel(SceArgs a) {
 }
 
 // ------------------------------- long rows ---------------------------------
-// Sparse labels, rows that do not fit a workgroup's registers (32768 fp32 elements) and LDS (98304 16-bit ones): the workgroup
+// Sparse labels, rows that do not fit a workgroup's registers (32768 fp32 elements) and LDS (97792 16-bit ones): the workgroup
 // streams the row, kLongVecs vectors per thread and step, and every thread keeps a running (maximum, sum of exponentials) that it re-bases once per step.
 // The backward reads the row a second time, from its end, so that what was read last is found in the nearest cache
 // (1024 x 128256 bf16 116 -> 111 us), and is bound by what that second read costs: 1024 x 128256 bf16 679 us by
@@ -491,8 +491,8 @@ void sce_long_kernel(SceArgs a) {
 // read once and four, three or two rows share a compute unit (pick_sce_long_shape; 64 registers or fewer: 46 forward, 58
 // backward).  Bound by HBM in the forward, and by how far the loads, the arithmetic (two exponentials an element) and the
 // stores of two rows overlap in the backward.  us, forward / backward, streamed by sce_long_kernel and so: 4096 x 50257 bf16
-// 95 / 168 and 65 / 145 (sce_sparse_bwd_kernel), 2500 x 80000 74 / 164 and 68 / 145, 4096 x 65536 102 / 200 and 86 / 181
-// (sce_sparse_bwd_kernel).
+// 95 / 168 and 65 / 145 (up to 65024 columns the backward is sce_sparse_bwd_kernel's), 2500 x 80000 74 / 164 and 68 / 145, 4096 x
+// 65536 102 / 200 and 86 / 183.
 constexpr int kPackedVecs = 8;
 
 // The compiler would keep the unpacked elements from one pass to the next otherwise: twice the registers.
@@ -827,9 +827,10 @@ static bool pick_sce_shape(int nvec, int max_nv_wave, int max_nv, int* threads, 
 // 16-bit rows with a tail in LDS (threads 0: none).  The forward keeps four rows under way per compute unit where that
 // fits (512 threads and up to 39 KiB of LDS each), then three, then two; the backward, whose reads and writes do not like
 // company, two (4096 x 50257 bf16, rows per compute unit 2 / 3 / 4: forward 78.3 / 69.0 / 65, backward 152 / 154 / 163 us),
-// with the exponentials of 4 vectors per thread in registers as far as two tails of 64 KiB reach (against packed rows x 33000
-// 102 -> 94, x 50257 152 -> 145, x 65536 183 -> 181 us).  Longer than 98304 columns: streamed (x 80000, 2500 rows, streamed
-// 74 / 164, so 68 / 145 us).  fp32 rows, 4096 x 32000 and x 20001, gain nothing: 175 / 178 and 116 / 113 us.
+// with the exponentials of 4 vectors per thread in registers as far as two tails of less than 64 KiB reach, 65024 columns
+// (against packed rows x 33000 102 -> 94, x 50257 152 -> 145; x 65024 181, x 65025 packed 193, x 65536, without a tail, 183
+// us).  Longer than 97792 columns, 8 vectors and such a tail: streamed (x 80000, 2500 rows, streamed 74 / 164, so 68 / 145;
+// x 97792 79 / 175, x 97793 streamed 80 / 208 us).  fp32 rows, 4096 x 32000 and x 20001, gain nothing: 175 / 178 and 116 / 113 us.
 struct SceLongShape {
   int threads;
   bool packed;        // sce_packed_kernel, else sce_sparse_bwd_kernel
