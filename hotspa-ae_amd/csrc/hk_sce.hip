@@ -794,7 +794,8 @@ static inline int pow2_ceil_sce(int v) {
   return p;
 }
 
-static bool pick_sce_shape(int nvec, int max_nv_wave, int max_nv, int* threads, int* nv) {
+// least4: the fewest threads that take 4 vectors each
+static bool pick_sce_shape(int nvec, int max_nv_wave, int max_nv, int least4, int* threads, int* nv) {
   const int forced = tune_get(TUNE_SCE_THREADS);
   if (forced > 0) {
     int t = std::min(1024, std::max(64, (forced + 63) / 64 * 64));
@@ -815,7 +816,7 @@ static bool pick_sce_shape(int nvec, int max_nv_wave, int max_nv, int* threads, 
   // and 18.6; backward, 10326 x 2112 bf16, 192 x 2 16.9, 320 x 1 26.8, 8000 x 4100 192 x 4 24.6, 320 x 2 27.4.
   for (int n = max_nv; n >= 1; n >>= 1) {
     int t = ((nvec + n - 1) / n + 63) / 64 * 64;
-    if (t <= 1024 && (t >= (n > 4 ? 256 : 192) || n == 1)) { *threads = t; *nv = n; return true; }
+    if (t <= 1024 && (t >= (n > 4 ? 256 : n == 4 ? least4 : 192) || n == 1)) { *threads = t; *nv = n; return true; }
   }
   for (int n = 1; n <= max_nv; n <<= 1) {
     int t = ((nvec + n - 1) / n + 63) / 64 * 64;
@@ -896,9 +897,15 @@ static int sce_typed(SceArgs a, hipStream_t s) {
   // sparse forward only keeps the packed row; the others keep 32 floats or two rows, in a wavefront 16 floats of fp32
   // (10000 x 1634 backward 64 x 8 25.5, 256 x 2 23.4; x 1100 17.5, 192 x 2 16.2 us)
   const int max_nv = (MODE == 0) ? 8 : 32 / VEC;
+  // (dense labels, fp32, 64 x 8 / as now, forward and backward: 10000 x 1100 64 / 16 and 64 / 24, x 2048 86 / 26 and 89 / 40)
   const int max_nv_wave = (MODE == 0) ? 8 : 4;
+  // Three wavefronts of 4 vectors, 513 to 768 in all, against five or six of 2, us at 16000 rows of 514, 576 and 700 vectors: bf16
+  // sparse backward 46.2 / 47.5, 47.6 / 50.4 and 62.3 / 60.6, dense forward 42.3 / 46.4, 45.0 / 46.5 and 55.6 / 60.6, dense backward
+  // 69.8 / 65.9, 70.0 / 69.6 and 93.2 / 87.1; fp32 sparse backward 46.6 / 44.9, 47.3 / 47.5 and 61.7 / 58.0, dense forward 42.3 /
+  // 39.5, 44.2 / 42.4 and 56.0 / 52.1, dense backward 68.4 / 65.0, 71.0 / 68.3 and 93.8 / 88.1.
+  const int least4 = MODE == 0 || (VEC == 8 && MODE != 3) ? 192 : 256;
   int threads = 0, nv = 0;
-  const bool shaped = pick_sce_shape(a.nvec, max_nv_wave, max_nv, &threads, &nv);
+  const bool shaped = pick_sce_shape(a.nvec, max_nv_wave, max_nv, least4, &threads, &nv);
   const dim3 levels{unsigned(a.n0), unsigned(a.n1), unsigned(a.n2)};
   auto launch = [&](auto ragged) {
     constexpr bool RAGGED = decltype(ragged)::value;

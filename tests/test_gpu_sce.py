@@ -174,3 +174,12 @@ def test_gradient_of_one_class_is_exactly_zero(hk, cuda, dtype):
             hk.sce_sparse_bwd_reduced(x, labels, grad[:1], 0.25, out, IGN)
             torch.cuda.synchronize()
             assert torch.count_nonzero(out) == 0, (g, int(torch.count_nonzero(out)))
+
+
+# vectors on both sides of a wavefront's most and of what three wavefronts of 2 and of 4 hold
+@pytest.mark.parametrize("dtype", ["fp32", "bf16", "fp16"])
+@pytest.mark.parametrize("vectors", [256, 257, 384, 385, 512, 513, 576, 640, 768, 769])
+def test_rows_of_a_few_wavefronts(hk, cuda, dtype, vectors):
+    shape = (7, vectors * (4 if dtype == "fp32" else 8))
+    test_sce_sparse(hk, cuda, dtype, shape)
+    test_sce_dense(hk, cuda, dtype, shape)
