@@ -217,6 +217,43 @@ template <int N, int LX> __device__ __forceinline__ void slices_share(float* f, 
   }
 }
 
+// The same for few slices: every thread merges its own lane's values, without a second barrier and without the merged copy, in
+// the same order (4 x 5 x 5904 bf16 forward 3.7 -> 3.0 us).
+// lds: [slices][N / 4][LX] 16-byte vectors; a call that follows another takes an area of its own.
+template <int N, int LX> __device__ __forceinline__ void few_slices_share(float* f, float* lds, int slices, bool take_max) {
+  u32x4* area = reinterpret_cast<u32x4*>(lds) + int(threadIdx.x);
+#pragma unroll
+  for (int q = 0; q < N / 4; ++q)
+    area[(int(threadIdx.y) * (N / 4) + q) * LX] = u32x4{f2u(f[4 * q]), f2u(f[4 * q + 1]), f2u(f[4 * q + 2]), f2u(f[4 * q + 3])};
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < N / 4; ++q) {
+    const u32x4 o = area[q * LX];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) f[4 * q + j] = u2f(o[j]);
+  }
+  for (int s = 1; s < slices; ++s) {
+#pragma unroll
+    for (int q = 0; q < N / 4; ++q) {
+      const u32x4 o = area[(s * (N / 4) + q) * LX];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) f[4 * q + j] = take_max ? fmaxf(f[4 * q + j], u2f(o[j])) : f[4 * q + j] + u2f(o[j]);
+    }
+  }
+}
+constexpr int kFewSlices = 6;
+// LDS of a workgroup, in floats: the forward shares twice
+template <int N, int LX, bool FEW, bool BWD>
+static inline size_t share_floats(int slices) {
+  return size_t(FEW ? (BWD ? slices : 2 * slices) : slices + 1) * LX * N;
+}
+template <int N, int LX, bool FEW>
+__device__ __forceinline__ void share(float* f, float* lds, int slices, bool take_max, int call) {
+  if (slices <= 1) return;   // uniform
+  if constexpr (FEW) few_slices_share<N, LX>(f, lds + call * slices * LX * N, slices, take_max);
+  else slices_share<N, LX>(f, lds, slices, take_max);
+}
+
 struct SoftmaxDimArgs {
   const void* x;       // forward: input;  backward: y
   const void* dy;
@@ -242,11 +279,11 @@ struct DimColumn {
   }
 };
 
-template <typename T, int NK, int LX, bool PLAIN>
+template <typename T, int NK, int LX, bool PLAIN, bool FEW>
 __global__ __launch_bounds__(1024)
 void softmax_fwd_dim_kernel(SoftmaxDimArgs a) {
   constexpr int VEC = VecIO<T>::N;
-  extern __shared__ __align__(16) float shared[];   // [slices + 1][LX][VEC]
+  extern __shared__ __align__(16) float shared[];   // share_floats
   const DimColumn<T, LX> c(a, NK);
   const T* xp = static_cast<const T*>(a.x) + c.base;
   u32x4 raw[NK];
@@ -263,7 +300,7 @@ void softmax_fwd_dim_kernel(SoftmaxDimArgs a) {
 #pragma unroll
     for (int j = 0; j < VEC; ++j) m[j] = max3(m[j], f[j], g[j]);
   }
-  if (a.slices > 1) slices_share<VEC, LX>(m, shared, a.slices, true);
+  share<VEC, LX, FEW>(m, shared, a.slices, true, 0);
   float base2[VEC], ml[VEC], s[VEC];
 #pragma unroll
   for (int j = 0; j < VEC; ++j) {
@@ -281,7 +318,7 @@ void softmax_fwd_dim_kernel(SoftmaxDimArgs a) {
       s[j] += k < c.count ? e : 0.f;
     }
   }
-  if (a.slices > 1) slices_share<VEC, LX>(s, shared, a.slices, false);
+  share<VEC, LX, FEW>(s, shared, a.slices, false, 1);
   if (!c.live) return;
 #pragma unroll
   for (int j = 0; j < VEC; ++j) s[j] = 1.0f / s[j];
@@ -298,11 +335,11 @@ void softmax_fwd_dim_kernel(SoftmaxDimArgs a) {
   }
 }
 
-template <typename T, int NK, int LX, bool PLAIN>
+template <typename T, int NK, int LX, bool PLAIN, bool FEW>
 __global__ __launch_bounds__(1024)
 void softmax_bwd_dim_kernel(SoftmaxDimArgs a) {
   constexpr int VEC = VecIO<T>::N;
-  extern __shared__ __align__(16) float shared[];   // [slices + 1][LX][VEC]
+  extern __shared__ __align__(16) float shared[];   // share_floats
   const DimColumn<T, LX> c(a, NK);
   const T* yp = static_cast<const T*>(a.x) + c.base;
   const T* dyp = static_cast<const T*>(a.dy) + c.base;
@@ -322,7 +359,7 @@ void softmax_bwd_dim_kernel(SoftmaxDimArgs a) {
 #pragma unroll
     for (int j = 0; j < VEC; ++j) dot[j] = k < c.count ? fmaf(y[j], d[j], dot[j]) : dot[j];
   }
-  if (a.slices > 1) slices_share<VEC, LX>(dot, shared, a.slices, false);
+  share<VEC, LX, FEW>(dot, shared, a.slices, false, 0);
   if (!c.live) return;
   T* dxp = static_cast<T*>(a.out) + c.base - vec_column<T, true>(c.v, int(a.inner));
 #pragma unroll
@@ -607,20 +644,20 @@ static int softmax_lastdim_typed(SoftmaxArgs a, hipStream_t s) {
   }
 }
 
-// LEAST, MOST: the entries per lane that the plan gives this launch
-template <typename T, bool BWD, int LX, bool PLAIN, int LEAST, int MOST>
+// FEW: up to kFewSlices slices.  LEAST, MOST: the entries per lane that the plan gives this launch
+template <typename T, bool BWD, int LX, bool PLAIN, bool FEW, int LEAST, int MOST>
 static int launch_softmax_dim(const SoftmaxDimArgs& a, int nk, hipStream_t s) {
   if (nk < LEAST || nk > MOST) {
     set_last_error("softmax: no kernel for %d entries per lane", nk);
     return HK_ERR_UNSUPPORTED;
   }
   const dim3 grid{unsigned((a.total + LX - 1) / LX)}, block{unsigned(LX), unsigned(a.slices)};
-  const size_t lds = a.slices > 1 ? size_t(a.slices + 1) * LX * VecIO<T>::N * sizeof(float) : 0;
+  const size_t lds = a.slices > 1 ? share_floats<VecIO<T>::N, LX, FEW, BWD>(a.slices) * sizeof(float) : 0;
 #define HK_DIM_CASE(N)                                                              \
   case N:                                                                           \
     if constexpr (N >= LEAST && N <= MOST) {                                        \
-      if constexpr (BWD) HK_LAUNCH((softmax_bwd_dim_kernel<T, N, LX, PLAIN>), grid, block, lds, s, a); \
-      else HK_LAUNCH((softmax_fwd_dim_kernel<T, N, LX, PLAIN>), grid, block, lds, s, a);   \
+      if constexpr (BWD) HK_LAUNCH((softmax_bwd_dim_kernel<T, N, LX, PLAIN, FEW>), grid, block, lds, s, a); \
+      else HK_LAUNCH((softmax_fwd_dim_kernel<T, N, LX, PLAIN, FEW>), grid, block, lds, s, a);   \
     }                                                                               \
     break;
   profile_before(s);
@@ -687,18 +724,36 @@ static int softmax_strided_typed(const void* x, const void* dy, void* out, int64
         // 73.3, 8 x 21 x 263168 62.3 / 63.8 and 90.7 / 88.7), nor 16-bit ones (8 x 21 x 263169 35.3 / 37.8 / 48.1 and 50.3 /
         // 51.0 / 55.8)
         const bool wide = VEC == 4 && a.slices <= 4 && a.total >= cus * 2048 && bytes % 128 != 0;
-        // PLAIN: 16-bit entries in runs of 1 KiB, and the few, are stored through the cache (8 x 21 x 263170 bf16 35.5 /
-        // 48.8 -> 33.9 / 44.4, 4 x 65 x 355 5.9 / 5.1 -> 5.4 / 4.4; fp32 70.8 / 104 -> 73.2 / 112, and 16-bit ones in runs of
-        // 512 bytes, 16 x 150 x 16384, 37.2 / 42.3 -> 39.9 / 47.1 us, are not)
+        // PLAIN: the few and, of 16-bit entries in runs of 1 KiB, the backward, forwards of 64 MiB and more, and of 24 MiB and
+        // more where planes share lines and one or two slices hold the dimension, are stored through the cache (streamed /
+        // so, forward: 8 x 21 x 263169 36.2 / 33.9, 2 x 6 x 3000000 27.4 / 26.3, 64 x 10 x 50177 26.4 / 25.5, 32 x 12 x 40001 14.6 / 13.2,
+        // but 16 x 60 x 30001 26.5 / 28.4, 4 x 21 x 263169 20.2 / 21.5, 32 x 12 x 40000 11.7 / 13.3, 32 x 19 x 16384 9.3 / 11.4; backward of
+        // 8 x 21 x 263169 50.0 / 46.8, 32 x 19 x 16385 13.6 / 13.1; fp32 70.8 / 73.2 and 104 / 112, and 16-bit ones in runs of 512
+        // bytes, 16 x 150 x 16384, 37.2 / 39.9 and 42.3 / 47.1 us, are not)
+        const int64_t plain_from = int64_t(bytes % 128 != 0 && a.slices <= 2 ? 24 : 64) << 20;
+        const bool plain = VEC == 8 && (BWD || a.total * dim * 16 >= plain_from);
+        // Up to kFewSlices slices every thread merges its own values, GPU us, with slices_share / so: 64 x 10 x 12544 bf16 (2
+        // slices) forward 8.3 / 7.2, 32 x 12 x 40000 11.7 / 11.1, 4 x 5 x 5904 (3) 3.7 / 3.0, 32 x 40 x 6401 (5) 10.4 / 10.2, 4 x 12 x 5904 (6) 3.6 /
+        // 3.35, 16 x 60 x 30001 (8) 25.9 / 27.3.
         // What nk can be.  64 slices: 2 to 4, for 65 to 256 entries.  The few in 32: up to 6, because at 192 entries and past 16
-        // vectors per compute unit they are no longer few.  More than 16 slices are full ones, of `most` entries each.
-        if (lx == 16) return launch_softmax_dim<T, BWD, 16, true, 2, 4>(a, nk, s);
-        if (few) return launch_softmax_dim<T, BWD, 32, true, 1, 6>(a, nk, s);
-        if (a.slices > 16) return launch_softmax_dim<T, BWD, 32, false, kFull, kDimVecs>(a, nk, s);
+        // vectors per compute unit they are no longer few; 1 or 2 in few slices.  More than 16 slices are full ones, of `most`
+        // entries each, and more than 6 of them full ones or one entry short of it.
+        const bool few_slices = a.slices <= kFewSlices;
+        if (lx == 16) return launch_softmax_dim<T, BWD, 16, true, false, 2, 4>(a, nk, s);
+        if (few && few_slices) return launch_softmax_dim<T, BWD, 32, true, true, 1, 2>(a, nk, s);
+        if (few) return launch_softmax_dim<T, BWD, 32, true, false, 2, 6>(a, nk, s);
+        if (a.slices > 16) return launch_softmax_dim<T, BWD, 32, false, false, kFull, kDimVecs>(a, nk, s);
         if constexpr (VEC == 4) {
-          if (wide) return launch_softmax_dim<T, BWD, (BWD ? 256 : 128), false, 1, kDimVecs>(a, nk, s);
+          if (wide) return launch_softmax_dim<T, BWD, (BWD ? 256 : 128), false, true, 1, kDimVecs>(a, nk, s);
         }
-        return launch_softmax_dim<T, BWD, 64, VEC == 8, 1, kFull>(a, nk, s);
+        if constexpr (VEC == 8) {
+          if (plain && few_slices) return launch_softmax_dim<T, BWD, 64, true, true, 1, kFull>(a, nk, s);
+          if (plain) return launch_softmax_dim<T, BWD, 64, true, false, kFull - 1, kFull>(a, nk, s);
+        }
+        if constexpr (VEC == 4 || !BWD) {
+          if (few_slices) return launch_softmax_dim<T, BWD, 64, false, true, 1, kFull>(a, nk, s);
+          return launch_softmax_dim<T, BWD, 64, false, false, kFull - 1, kFull>(a, nk, s);
+        }
       }
     }
   }

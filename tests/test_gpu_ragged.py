@@ -271,10 +271,12 @@ def test_cross_entropy_of_lowest_values(hk, cuda, dtype, cols):
 
 
 # one of every launch of the kernels above: many fp32 planes (runs of 128 and 256 lanes, of 64 where planes are whole lines), 16-bit ones with blocks left over
-# after the runs that stay on one XCD, more than 16 slices, and few positions with up to and more than 64 entries
+# after the runs that stay on one XCD, more than 16 slices, 64 MiB and more of them in up to 6 slices and in 13, 7 slices and more
+# of less, and few positions with up to and more than 64 entries
 @pytest.mark.parametrize("dtype,outer,dim,inner", [("fp32", 1, 9, 4 * 524288 + 3), ("fp32", 1, 9, 4 * 524288), ("fp32", 2, 32, 1048577), ("bf16", 8, 21, 40961),
                                                    ("fp16", 8, 21, 40960), ("bf16", 16, 150, 8191), ("fp32", 4, 129, 8003),
                                                    ("bf16", 4, 65, 355), ("fp32", 2, 250, 203), ("fp16", 5, 256, 15),
+                                                   ("bf16", 8, 21, 200001), ("fp16", 8, 100, 42001), ("bf16", 16, 60, 20001), ("fp32", 16, 60, 10001),
                                                    ("bf16", 5, 8, 4111), ("fp32", 3, 57, 5877), ("bf16", 2, 17, 8)])
 def test_softmax_dim_launches(hk, cuda, dtype, outer, dim, inner):
     import torch
