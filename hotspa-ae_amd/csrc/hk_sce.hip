@@ -826,8 +826,11 @@ static bool pick_sce_shape(int nvec, int max_nv_wave, int max_nv, int least4, in
 }
 
 // 16-bit rows with a tail in LDS (threads 0: none).  The forward keeps four rows under way per compute unit where that
-// fits (512 threads and up to 39 KiB of LDS each), then three, then two; the backward, whose reads and writes do not like
-// company, two (4096 x 50257 bf16, rows per compute unit 2 / 3 / 4: forward 78.3 / 69.0 / 65, backward 152 / 154 / 163 us),
+// fits (512 threads and up to 39 KiB of LDS each), then three where rows are many and two would leave wavefronts idle (rows x
+// 58000, three / two: 750 22.2 / 19.3, 1300 31.7 / 31.6, 4096 80 / 87 us; 4096 x 61000, 960 threads for two, 84 / 89, x 62000, 1024
+// threads, 85.0 / 83.4; x 66688 88.5 / 86.6), then two; past 8 vectors in 1024 threads one or two rows per compute unit are
+// streamed (packed / streamed: 300 x 66688 14.6 / 13.6, 500 x 97000 21.5 / 20.7, 1024 x 75000 30.5 / 35.2 us); the backward, whose reads and
+// writes do not like company, two (4096 x 50257 bf16, rows per compute unit 2 / 3 / 4: forward 78.3 / 69.0 / 65, backward 152 / 154 / 163 us),
 // with the exponentials of 4 vectors per thread in registers as far as two tails of less than 64 KiB reach, 65024 columns
 // (against packed rows x 33000 102 -> 94, x 50257 152 -> 145; x 65024 181, x 65025 packed 193, x 65536, without a tail, 183
 // us).  Longer than 97792 columns, 8 vectors and such a tail: streamed (x 80000, 2500 rows, streamed 74 / 164, so 68 / 145;
@@ -838,9 +841,10 @@ struct SceLongShape {
   size_t lds_bytes;
 };
 template <bool BWD>
-static SceLongShape pick_sce_long_shape(int nvec) {
+static SceLongShape pick_sce_long_shape(int nvec, int64_t rows) {
   SceLongShape l{0, false, 0};
-  if (nvec <= 4 * 1024) return l;
+  const int64_t cus = device_cu_count();
+  if (nvec <= 4 * 1024 || (!BWD && nvec > kPackedVecs * 1024 && rows <= 2 * cus)) return l;
   size_t per_cu = 0, per_block = 0;
   device_lds_bytes(&per_cu, &per_block);
   per_block = std::min<size_t>(per_block, 65536);
@@ -851,10 +855,11 @@ static SceLongShape pick_sce_long_shape(int nvec) {
   };
   if (BWD && fits(nvec - 4 * 1024, 2)) { l.threads = 1024; return l; }
   l.packed = true;
-  for (int rows = BWD ? 2 : 4; rows >= 2; --rows) {
-    const int most = rows == 4 ? 512 : rows == 3 ? 640 : 1024;   // 32 wavefronts in all
+  for (int per = BWD ? 2 : 4; per >= 2; --per) {
+    if (per == 3 && (nvec > kPackedVecs * 960 || rows <= 4 * cus)) continue;
+    const int most = per == 4 ? 512 : per == 3 ? 640 : 1024;   // 32 wavefronts in all
     const int threads = std::min(most, ((nvec + kPackedVecs - 1) / kPackedVecs + 63) / 64 * 64);
-    if (fits(nvec - kPackedVecs * threads, rows)) { l.threads = threads; return l; }
+    if (fits(nvec - kPackedVecs * threads, per)) { l.threads = threads; return l; }
   }
   return l;
 }
@@ -916,7 +921,7 @@ static int sce_typed(SceArgs a, hipStream_t s) {
     return launch_sce_nv<T, MODE, false, RAGGED>(a, nv, levels, dim3{unsigned(threads)}, s);
   };
   if constexpr (MODE < 2 && VEC == 8) {
-    const SceLongShape l = pick_sce_long_shape<MODE == 1>(a.nvec);
+    const SceLongShape l = pick_sce_long_shape<MODE == 1>(a.nvec, a.rows);
     if (l.threads > 0 && tune_get(TUNE_SCE_THREADS) <= 0) {
       const dim3 block{unsigned(l.threads)};
       profile_before(s);

@@ -624,7 +624,7 @@ def test_shard_statistics_keep_a_nan(hk, cuda, dtype, cols):
     assert float(stats[1, 0]) == 0.0 and bool(torch.isnan(stats[1, 1:]).all()), stats
 
 
-# 16-bit rows with a part in LDS: the most vectors of four, three and two rows per compute unit (6592, 8448, 12224) and of a
+# 16-bit rows with a part in LDS: the most vectors of four and two rows per compute unit (6592, 12224) and of a
 # gradient row with exponentials in registers (8128), one more each, and the first rows past registers alone (4097)
 @pytest.mark.parametrize("dtype", ["bf16", "fp16"])
 @pytest.mark.parametrize("shift", [0, 1])
@@ -654,6 +654,26 @@ def test_cross_entropy_rows_with_a_tail(hk, cuda, dtype, shift, vectors):
         hk.sce_sparse_bwd(tx, lab, g, tx, -100)     # in place
         torch.cuda.synchronize()
         assert torch.equal(tx.contiguous(), dx.contiguous()), cols
+
+
+# the same in as many rows as take a plan of their own: more than two and than four per compute unit, three rows' longest and one
+# vector more, past registers, the longest and one more
+@pytest.mark.parametrize("vectors", [6593, 7680, 7681, 8192, 8193, 12224, 12225])
+def test_cross_entropy_of_many_rows_with_a_tail(hk, cuda, vectors):
+    import torch
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    cols = 8 * vectors - 3
+    x = helpers.to_torch(helpers.draw(9150 + cols, (5, cols), dtype="bf16"), "bf16", cuda)
+    lab = torch.tensor([0, cols - 1, -100, 32768, cols - 9], device=cuda)
+    want = torch.logsumexp(x.double(), -1) - x.double().gather(1, lab.clamp(min=0)[:, None])[:, 0]
+    want[2] = 0
+    for times in (2 * cus // 5, 2 * cus // 5 + 1, 4 * cus // 5 + 1):
+        loss = torch.full((5 * times,), 5.0, dtype=torch.bfloat16, device=cuda)
+        hk.sce_sparse_fwd(x.repeat(times, 1), lab.repeat(times), loss, -100)
+        torch.cuda.synchronize()
+        loss = loss.view(times, 5)
+        helpers.assert_close(loss[0], want.cpu().numpy(), "bf16", "loss %d" % times)
+        assert torch.equal(loss, loss[:1].expand(times, 5)), times
 
 
 # operands whose rows start on different boundaries: x on even ones, on odd ones, on both in turn (an odd pitch), the others
