@@ -697,8 +697,8 @@ void dal_bwd_stream_kernel(DalBwdArgs a) {
   put_column_sums(a.part[1], db0, stage, group, rpb, in, a.cols, col);
 }
 
-// Folds [nparts, cols] fp32 partial rows into a [cols] vector of WT; blockIdx.y picks which of the
-// (up to five) sums.  A block covers 128 columns as 32 float4 column groups x 16 row slices.
+// Folds [nparts, cols] fp32 partial rows into a [cols] vector of WT (fold_partial_rows); blockIdx.y picks which of the (up to
+// five) sums that are wanted.
 struct DalFoldArgs {
   const float* part[kMaxParts];
   void* out[kMaxParts];
@@ -706,43 +706,11 @@ struct DalFoldArgs {
 };
 
 template <typename WT>
-__global__ __launch_bounds__(512)
+__global__ __launch_bounds__(kFoldThreads)
 void dal_fold_kernel(DalFoldArgs a) {
-  __shared__ float lds[16][32][4];
-  const float* part = a.part[blockIdx.y];
-  WT* out = static_cast<WT*>(a.out[blockIdx.y]);
-  if (part == nullptr || out == nullptr) return;   // uniform over the block
-  const int cg = threadIdx.x & 31, slice = threadIdx.x >> 5;
-  const int c = (blockIdx.x * 32 + cg) * 4;
-  float acc[4] = {0.f, 0.f, 0.f, 0.f};
-  if (c < a.cols) {
-    constexpr int U = 8;   // loads in flight
-    int r = slice;
-    for (; r + (U - 1) * 16 < a.nparts; r += U * 16) {
-      u32x4 v[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) v[u] = ld16_keep(part + int64_t(r + u * 16) * a.cols + c);
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        acc[0] += u2f(v[u].x); acc[1] += u2f(v[u].y); acc[2] += u2f(v[u].z); acc[3] += u2f(v[u].w);
-      }
-    }
-    for (; r < a.nparts; r += 16) {
-      const u32x4 v = ld16_keep(part + int64_t(r) * a.cols + c);
-      acc[0] += u2f(v.x); acc[1] += u2f(v.y); acc[2] += u2f(v.z); acc[3] += u2f(v.w);
-    }
-  }
-#pragma unroll
-  for (int k = 0; k < 4; ++k) lds[slice][cg][k] = acc[k];
-  __syncthreads();
-  if (threadIdx.x < 128) {
-    const int g = threadIdx.x >> 2, k = threadIdx.x & 3;
-    const int oc = (blockIdx.x * 32 + g) * 4 + k;
-    float s = 0.f;
-#pragma unroll
-    for (int sl = 0; sl < 16; ++sl) s += lds[sl][g][k];
-    if (oc < a.cols) Cvt<WT>::store(out + oc, s);
-  }
+  const float s = fold_partial_rows(a.part[blockIdx.y], a.nparts, a.cols, int(blockIdx.x));
+  const int oc = int(blockIdx.x) * kFoldCols + int(threadIdx.x);
+  if (threadIdx.x < kFoldCols && oc < a.cols) Cvt<WT>::store(static_cast<WT*>(a.out[blockIdx.y]) + oc, s);
 }
 
 // ---------------------------------------------------------------------------
@@ -1008,7 +976,9 @@ int hk_dropout_add_ln_bwd_ex(const hkDropoutAddLnBwdParams* pp, hkStream_t strea
   a.is_rms = p.is_rms_norm ? 1 : 0; a.dropout = dropout ? 1 : 0;
 
   DalFoldArgs f{};
-  for (int k = 0; k < kMaxParts; ++k) { f.part[k] = a.part[k]; f.out[k] = outs[k]; }
+  int wanted = 0;
+  for (int k = 0; k < kMaxParts; ++k)
+    if (outs[k]) { f.part[wanted] = a.part[k]; f.out[wanted++] = outs[k]; }
   f.nparts = int(sh.nparts); f.cols = int(p.cols);
 
   const dim3 grid{unsigned(sh.grid)}, block{unsigned(sh.block)};
@@ -1028,8 +998,9 @@ int hk_dropout_add_ln_bwd_ex(const hkDropoutAddLnBwdParams* pp, hkStream_t strea
     else HK_LAUNCH((dal_bwd_kernel<IT, RT, WT, false, false>), grid, block, lds, s, a);
     profile_after(s);
     int r = launch_check("dal_bwd_kernel");
-    if (r != HK_OK || nslots == 0) return r;
-    HK_LAUNCH((dal_fold_kernel<WT>), dim3(unsigned((p.cols + 127) / 128), kMaxParts), dim3(512), 0, s, f);
+    if (r != HK_OK || wanted == 0) return r;
+    HK_LAUNCH((dal_fold_kernel<WT>), dim3(unsigned((p.cols + kFoldCols - 1) / kFoldCols), unsigned(wanted)),
+              dim3(kFoldThreads), 0, s, f);
     return launch_check("dal_fold_kernel");
   });
 }

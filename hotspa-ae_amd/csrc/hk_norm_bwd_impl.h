@@ -402,56 +402,19 @@ void norm_bwd_kernel(NormBwdArgs a) {
   if constexpr (WITH_DB) fold(lds + region, outs[1]);
 }
 
-// Folds the [nparts, pitch] fp32 partial rows into dgamma / dbeta of type T.  Rows of whole 16-byte vectors of T:
-// pitch == cols; otherwise the last vector of a partial row holds the row's last columns, the first pitch - cols of
-// its elements being another vector's.
-// blockIdx.y picks dgamma / dbeta; a block covers 128 columns as 32 float4
-// column groups x 16 row slices, every slice keeps 8 independent loads in
-// flight (with 16 a pass over 32768 x 4096 took 0.2 % longer), the last ones
-// guarded by their row's number and not by a loop of single loads (39 partial
-// rows 3.5 -> 2.9 us), slices are folded through LDS.
+// Folds the [nparts, pitch] fp32 partial rows into dgamma / dbeta of type T (fold_partial_rows); blockIdx.y picks which.  Rows
+// of whole 16-byte vectors of T: pitch == cols; otherwise the last vector of a partial row holds the row's last columns, the
+// first pitch - cols of its elements being another vector's.
 template <typename T>
-__global__ __launch_bounds__(512)
-void norm_bwd_finalize_kernel(const float* __restrict__ part_dgamma,
-                              const float* __restrict__ part_dbeta, T* dgamma, T* dbeta,
-                              int nparts, int cols, int pitch) {
-  constexpr int U = 8;
-  __shared__ float lds[16][32][4];
-  const float* part = blockIdx.y == 0 ? part_dgamma : part_dbeta;
-  T* out = blockIdx.y == 0 ? dgamma : dbeta;
-  if (part == nullptr || out == nullptr) return;     // uniform over the block
-  const int cg = threadIdx.x & 31, slice = threadIdx.x >> 5;
-  const int c = (blockIdx.x * 32 + cg) * 4;
-  float acc[4] = {0.f, 0.f, 0.f, 0.f};
-  if (c < pitch) {                                    // a multiple of 4
-    for (int r = slice; r < nparts; r += U * 16) {
-      u32x4 v[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {   // a row past the end reads the last one
-        const int rr = r + u * 16;
-        v[u] = ld16_keep(part + int64_t(rr < nparts ? rr : nparts - 1) * pitch + c);
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const bool in = r + u * 16 < nparts;
-        acc[0] += in ? u2f(v[u].x) : 0.f; acc[1] += in ? u2f(v[u].y) : 0.f;
-        acc[2] += in ? u2f(v[u].z) : 0.f; acc[3] += in ? u2f(v[u].w) : 0.f;
-      }
-    }
-  }
-#pragma unroll
-  for (int k = 0; k < 4; ++k) lds[slice][cg][k] = acc[k];
-  __syncthreads();
-  if (threadIdx.x < 128) {
-    const int g = threadIdx.x >> 2, k = threadIdx.x & 3;
-    const int oc = (blockIdx.x * 32 + g) * 4 + k;
-    float s = 0.f;
-#pragma unroll
-    for (int sl = 0; sl < 16; ++sl) s += lds[sl][g][k];
-    const int shift = pitch - cols, tail = pitch - VecIO<T>::N;   // shift > 0: the partial last vector
-    if (shift == 0 || oc < tail) { if (oc < cols) Cvt<T>::store(out + oc, s); }
-    else if (oc >= tail + shift && oc < pitch) Cvt<T>::store(out + oc - shift, s);
-  }
+__global__ __launch_bounds__(kFoldThreads)
+void norm_bwd_finalize_kernel(const float* part0, const float* part1, T* out0, T* out1, int nparts, int cols, int pitch) {
+  T* out = blockIdx.y == 0 ? out0 : out1;
+  const float s = fold_partial_rows(blockIdx.y == 0 ? part0 : part1, nparts, pitch, int(blockIdx.x));
+  const int oc = int(blockIdx.x) * kFoldCols + int(threadIdx.x);
+  if (threadIdx.x >= kFoldCols || oc >= pitch) return;
+  const int shift = pitch - cols, tail = pitch - VecIO<T>::N;   // shift > 0: the partial last vector
+  if (shift == 0 || oc < tail) Cvt<T>::store(out + oc, s);
+  else if (oc >= tail + shift) Cvt<T>::store(out + oc - shift, s);
 }
 
 // Fallback backward for rows the register kernel cannot take (shorter than a 16-byte vector, more than 8192 columns,
@@ -898,9 +861,10 @@ int norm_bwd_typed(NormBwdArgs a, int mode, void* dgamma, void* dbeta, void* ws,
     default: rc = launch_norm_bwd_nv<T, BWD_LN_MEMEFF>(a, p, s); break;
   }
   if (rc != HK_OK || !want_cols) return rc;
-  HK_LAUNCH((norm_bwd_finalize_kernel<T>), dim3(unsigned((a.part_pitch + 127) / 128), 2), dim3(512), 0, s,
-                     a.part_dgamma, a.part_dbeta, static_cast<T*>(dgamma), static_cast<T*>(dbeta),
-                     p.grid, a.cols, a.part_pitch);
+  const bool both = dgamma != nullptr && dbeta != nullptr;
+  HK_LAUNCH((norm_bwd_finalize_kernel<T>), dim3(unsigned((a.part_pitch + kFoldCols - 1) / kFoldCols), both ? 2 : 1),
+            dim3(kFoldThreads), 0, s, dgamma ? a.part_dgamma : a.part_dbeta, a.part_dbeta,
+            static_cast<T*>(dgamma ? dgamma : dbeta), static_cast<T*>(dbeta), p.grid, a.cols, a.part_pitch);
   return launch_check("norm_bwd_finalize_kernel");
 }
 
