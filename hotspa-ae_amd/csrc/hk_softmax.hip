@@ -181,14 +181,17 @@ void softmax_bwd_kernel(SoftmaxArgs a) {
 // inner positions; the dimension is cut into slices of NK entries, LX lanes per slice, so that the whole column stays in
 // registers: one read, one write.  Slices agree on the maximum and the sum through LDS.  The partial last vector of a
 // plane is read as its last whole one, its own elements are stored one by one (in place, a neighbour may have replaced
-// the others before they were read).  The exponentials are formed twice, once for the sum and once on the way out:
-// holding them in fp32 would cost twice the registers.
-// Bound by HBM and, on odd planes, by the cache lines that neighbouring workgroups share: runs of 8 or 16 of them stay
-// on one XCD, whose L2 then sees each line whole (8 x 21 x 263169 fp32, forward / backward: 82 / 117 -> 72 / 106 us).  One
-// thread per column that passed over it three times measured (forward / backward, us) 150 / 160 at 8 x 21 x 263169 fp32,
-// now 69 / 92 (5.1 and 5.8 TB/s; 62 / 91 at 263168); 81 / 77 at 8 x 21 x 263168 bf16, now 33 / 45; 143 / 103 at 16 x 150 x
-// 16384 bf16, now 37 / 43; 447 / 356 at 8 x 256 x 40000 fp32, now 123 / 180.
-constexpr int kDimVecs = 8;      // most entries per lane
+// the others before they were read).
+// Bound by HBM, by how many workgroups a compute unit has under way (one loads while another stores: hence at most 512
+// threads a workgroup where the plan does not say otherwise) and, on odd planes, by the cache lines that neighbouring
+// workgroups share: runs of 8 or 16 of them stay on one XCD, whose L2 then sees each line whole.  Forward / backward, us:
+// 8 x 21 x 263169 fp32 66 / 94 (5.4 and 5.6 TB/s), 263168 62 / 89; 232 x 21 x 16384 bf16 52.6 / 75.5 (6.1 and 6.4 TB/s).
+// AGAIN: the compiler keeps what it has formed of the vectors, exponentials or unpacked elements in fp32, from one step to the next.
+// That is the faster program while it fits (10 entries of bf16 forward 118 registers, of which 40 hold them as loaded; 32 x 150 x
+// 16384 56 us kept, 60 formed again).  Past it, it costs a compute unit its second workgroup or spills (12 forward 136 registers, 16
+// backward 256 and 41 spilled), and what is needed again is formed again: forward 25 x 256 x 12101 87 -> 77, backward 19 x 256 x 16384
+// 152 -> 85, 38 x 128 x 16384 87 -> 81.
+constexpr int kDimVecs = 8;      // most entries per lane of a wavefront's run; of half a wavefront's, 16
 // f[0..N): this lane's values; on return the slices' maximum or sum (in slice order) of each, the same in every slice.
 // lds: [slices + 1][LX * N].  A thread merges the slices of one value (every thread merging all of its lane's values
 // takes slices * N steps: 65 entries of 355 bf16 positions 9.0 us, so 5.5); calls may follow one another.
@@ -261,6 +264,12 @@ struct SoftmaxDimArgs {
   int64_t inner, total;   // total: vectors of all planes, outer * run_vecs
   int dim, run_vecs, slices;
 };
+// What is formed from these vectors after this point is formed from them again, not kept in registers since before it.
+template <int N>
+__device__ __forceinline__ void form_again(u32x4 (&raw)[N]) {
+#pragma unroll
+  for (int k = 0; k < N; ++k) asm volatile("" : "+v"(raw[k]));
+}
 // this lane's column: element offset of its vector in entry 0 of the plane, its place in the run, whether it exists
 template <typename T, int LX>
 struct DimColumn {
@@ -279,8 +288,8 @@ struct DimColumn {
   }
 };
 
-template <typename T, int NK, int LX, bool PLAIN, bool FEW>
-__global__ __launch_bounds__(1024)
+template <typename T, int NK, int LX, bool PLAIN, bool FEW, int MAXT, bool AGAIN>
+__global__ __launch_bounds__(MAXT)
 void softmax_fwd_dim_kernel(SoftmaxDimArgs a) {
   constexpr int VEC = VecIO<T>::N;
   extern __shared__ __align__(16) float shared[];   // share_floats
@@ -301,6 +310,7 @@ void softmax_fwd_dim_kernel(SoftmaxDimArgs a) {
     for (int j = 0; j < VEC; ++j) m[j] = max3(m[j], f[j], g[j]);
   }
   share<VEC, LX, FEW>(m, shared, a.slices, true, 0);
+  if constexpr (AGAIN) form_again(raw);
   float base2[VEC], ml[VEC], s[VEC];
 #pragma unroll
   for (int j = 0; j < VEC; ++j) {
@@ -319,6 +329,7 @@ void softmax_fwd_dim_kernel(SoftmaxDimArgs a) {
     }
   }
   share<VEC, LX, FEW>(s, shared, a.slices, false, 1);
+  if constexpr (AGAIN) form_again(raw);
   if (!c.live) return;
 #pragma unroll
   for (int j = 0; j < VEC; ++j) s[j] = 1.0f / s[j];
@@ -335,8 +346,8 @@ void softmax_fwd_dim_kernel(SoftmaxDimArgs a) {
   }
 }
 
-template <typename T, int NK, int LX, bool PLAIN, bool FEW>
-__global__ __launch_bounds__(1024)
+template <typename T, int NK, int LX, bool PLAIN, bool FEW, int MAXT, bool AGAIN>
+__global__ __launch_bounds__(MAXT)
 void softmax_bwd_dim_kernel(SoftmaxDimArgs a) {
   constexpr int VEC = VecIO<T>::N;
   extern __shared__ __align__(16) float shared[];   // share_floats
@@ -360,6 +371,7 @@ void softmax_bwd_dim_kernel(SoftmaxDimArgs a) {
     for (int j = 0; j < VEC; ++j) dot[j] = k < c.count ? fmaf(y[j], d[j], dot[j]) : dot[j];
   }
   share<VEC, LX, FEW>(dot, shared, a.slices, false, 0);
+  if constexpr (AGAIN) { form_again(ry); form_again(rd); }
   if (!c.live) return;
   T* dxp = static_cast<T*>(a.out) + c.base - vec_column<T, true>(c.v, int(a.inner));
 #pragma unroll
@@ -644,25 +656,28 @@ static int softmax_lastdim_typed(SoftmaxArgs a, hipStream_t s) {
   }
 }
 
-// FEW: up to kFewSlices slices.  LEAST, MOST: the entries per lane that the plan gives this launch
-template <typename T, bool BWD, int LX, bool PLAIN, bool FEW, int LEAST, int MOST>
+// FEW: up to kFewSlices slices.  MAXT: the most threads that its plans have.  LEAST, MOST:
+// the entries per lane that they give (of 16-bit types from 8 on even numbers).  LEAST_AGAIN: from how many on AGAIN; 14 backward just fit without
+template <typename T, bool BWD, int LX, bool PLAIN, bool FEW, int MAXT, int LEAST, int MOST, int LEAST_AGAIN = 17>
 static int launch_softmax_dim(const SoftmaxDimArgs& a, int nk, hipStream_t s) {
-  if (nk < LEAST || nk > MOST) {
+  if (nk < LEAST || nk > MOST || (nk > kDimVecs && nk % 2 != 0 && VecIO<T>::N == 8) || a.slices * LX > MAXT) {
     set_last_error("softmax: no kernel for %d entries per lane", nk);
     return HK_ERR_UNSUPPORTED;
   }
   const dim3 grid{unsigned((a.total + LX - 1) / LX)}, block{unsigned(LX), unsigned(a.slices)};
   const size_t lds = a.slices > 1 ? share_floats<VecIO<T>::N, LX, FEW, BWD>(a.slices) * sizeof(float) : 0;
-#define HK_DIM_CASE(N)                                                              \
-  case N:                                                                           \
-    if constexpr (N >= LEAST && N <= MOST) {                                        \
-      if constexpr (BWD) HK_LAUNCH((softmax_bwd_dim_kernel<T, N, LX, PLAIN, FEW>), grid, block, lds, s, a); \
-      else HK_LAUNCH((softmax_fwd_dim_kernel<T, N, LX, PLAIN, FEW>), grid, block, lds, s, a);   \
+#define HK_DIM_CASE(NK)                                                             \
+  case NK:                                                                          \
+    if constexpr (NK >= LEAST && NK <= MOST && (NK <= kDimVecs || NK % 2 == 0 || VecIO<T>::N == 4)) { \
+      constexpr bool AGAIN = NK >= LEAST_AGAIN && !(BWD && NK == 14);               \
+      if constexpr (BWD) HK_LAUNCH((softmax_bwd_dim_kernel<T, NK, LX, PLAIN, FEW, MAXT, AGAIN>), grid, block, lds, s, a); \
+      else HK_LAUNCH((softmax_fwd_dim_kernel<T, NK, LX, PLAIN, FEW, MAXT, AGAIN>), grid, block, lds, s, a); \
     }                                                                               \
     break;
   profile_before(s);
   switch (nk) {
     HK_DIM_CASE(1) HK_DIM_CASE(2) HK_DIM_CASE(3) HK_DIM_CASE(4) HK_DIM_CASE(5) HK_DIM_CASE(6) HK_DIM_CASE(7) HK_DIM_CASE(8)
+    HK_DIM_CASE(9) HK_DIM_CASE(10) HK_DIM_CASE(11) HK_DIM_CASE(12) HK_DIM_CASE(13) HK_DIM_CASE(14) HK_DIM_CASE(15) HK_DIM_CASE(16)
   }
 #undef HK_DIM_CASE
   profile_after(s);
@@ -703,57 +718,103 @@ static int softmax_strided_typed(const void* x, const void* dy, void* out, int64
       a.x = x; a.dy = dy; a.out = out; a.inner = inner; a.dim = int(dim);
       a.run_vecs = int((inner + VEC - 1) / VEC);
       a.total = outer * a.run_vecs;
-      // 8 entries a lane; 6 where that holds two 16-bit operands in fewer registers (8 x 21 x 263168 bf16 backward
-      // 56.1 -> 48.8 us, 16 x 150 x 16384 86.7 -> 46.5; forward 34.6 / 34.1 and 43.8 / 47.4 us), if 32 slices do then.
       // A problem that leaves most wavefront slots empty takes 2 entries a lane, in workgroups of half a wavefront's
       // vectors (a quarter's, up to 64 slices, for the longer dimensions of the smallest): its time is one lane's chain
       // of instructions.  GPU us, forward / backward, with 6 to 8 entries in a wavefront's and so: 4 x 65 x 355 bf16
       // 8.6 / 7.5 and 4.4 / 3.6, 2 x 250 x 200 fp32 9.4 / 10.7 and 5.8 / 5.9, 3 x 57 x 5877 fp32 5.8 / 6.3 and 4.5 / 4.4,
       // 4 x 100 x 10000 bf16 10.1 / 8.0 and 7.8 / 6.8; at 2 x 128 x 16384 fp32 they meet, 8.9 / 11.1 and 9.9 / 10.8.
-      constexpr int kFull = BWD && VEC == 8 ? 6 : kDimVecs;
       const bool few = a.total <= cus * 64 && a.total * dim <= cus * 3072;
-      const int lx = few && a.total <= cus * 16 && dim > 64 ? 16 : 32, fewest = int((dim + 1024 / lx - 1) / (1024 / lx));
-      const int most = std::max(few ? 2 : kFull, fewest);
-      const int slices = int((dim + most - 1) / most), nk = int((dim + slices - 1) / slices);
+      const bool odd = bytes % 128 != 0;   // planes share cache lines
+      const int64_t array = a.total * dim * 16;
+      // More entries than that: runs of half a wavefront's vectors in up to 16 slices; forward, of the longest dimensions of 16-bit
+      // entries, a quarter's in up to 32 where planes are whole lines or the array is small.  A workgroup then has at most 512
+      // threads and several share a compute unit (runs of 64 lanes in up to 16 slices of 8 or 6 entries, as before, / 32 / 16
+      // lanes; forward, bf16: 122 x 40 x 16384 66 / 54 / 54, 76 x 64 61 / 55 / 55, 55 x 88 72 / 54 / 56, 38 x 128 72 / 57 / 55, 32 x
+      // 150 73 / 56 / 56, 26 x 182 71 / 60 / 56, 19 x 256 73 / 69 / 58; odd planes, 75 x 88 x 12101 81 / 69 / 72, 36 x 182 90 / 75 / 80,
+      // 25 x 256 89 / 77 / 86; backward: 76 x 64 x 16384 90 / 76 / 78, 55 x 88 89 / 78 / 78, 4 x 224 x 12288 13.5 / 12.2 / 14.4, 19 x 256 147 / 85 /
+      // 85, 3 x 256 x 12288 21 / 15 / 15).  Odd planes of up to
+      // 48 entries keep their runs longer (300 x 33 x 8191 forward 65 / 73).  In the 16-bit backward of 129 to 192 entries (5 x 182 x
+      // 12288, 6 entries in 31 slices 12.1, 12 in 16 12.7) and of fp32 (13 x 167 x 3648 forward 11.7 / 12.1), slices are the 32 that a
+      // workgroup can have; fp32 up to 128 entries stays with runs of 64 lanes, up to 16 slices (64 / 32 lanes, 4 x 60 x 263169 115 / 132
+      // and 168 / 196, 39 x 70 x 3264 forward 12.6 / 13.9, 38 x 64 x 16384 56 / 55).
+      const bool many = !few && dim > (VEC == 4 ? 128 : odd ? 48 : 32);
+      const bool tall = many && dim > 128 && (VEC == 4 || (BWD && dim <= 192));
+      const bool quarter = VEC == 8 && !BWD && dim > 160 && many && (!odd || array < (int64_t(48) << 20));
+      const int lx = few ? (a.total <= cus * 16 && dim > 64 ? 16 : 32) : quarter ? 16 : 32;
+      const int most_slices = (few || tall ? 1024 : 512) / lx, fewest = int((dim + most_slices - 1) / most_slices);
+      int nk;
+      if (many) {
+        // (up to 80 entries forward 8 or a little less: 12 x 52 x 40554 22.5 us, of 5 entries 24.8)
+        nk = std::max(tall ? (VEC == 4 ? 8 : 6) : BWD ? 4 : dim <= 80 ? int((dim + (dim + 7) / 8 - 1) / ((dim + 7) / 8)) : 5, fewest);
+        if (nk > kDimVecs) nk = (nk + 1) / 2 * 2;
+        if (BWD && nk > kDimVecs) nk = std::max(nk, 14);
+      } else {
+        // the 16-bit backward of small arrays and of odd planes takes as few as 6 (22 x 8 x 20059 6.4 / 7.0 us, 310 x 46 x 3005 53 / 64)
+        const int full = VEC == 8 && BWD && (array < (int64_t(48) << 20) || odd) ? 6 : kDimVecs;
+        const int most = few ? std::max(2, fewest) : full, slices = int((dim + most - 1) / most);
+        nk = int((dim + slices - 1) / slices);
+      }
       a.slices = int((dim + nk - 1) / nk);
       if (a.total <= 0x7fffffffLL) {
-        // fp32 planes that share cache lines and fill the device many times over, up to 32 entries: runs of 2 KiB and 4 KiB
-        // of an entry per workgroup instead of 1 KiB share fewer lines (8 x 21 x 263169 forward 71.8 / 69.7 / 69.0, backward
-        // 106 / 103 / 96 us with runs of 64 / 128 / 256 lanes).  Planes of whole lines have nothing to gain (runs of 64 lanes
-        // / of 128 forward, 256 backward: 16 x 2 x 1048576 42.3 / 44.3 and 60.9 / 62.7 us, 8 x 9 x 524288 49.4 / 49.4 and 70.8 /
-        // 73.3, 8 x 21 x 263168 62.3 / 63.8 and 90.7 / 88.7), nor 16-bit ones (8 x 21 x 263169 35.3 / 37.8 / 48.1 and 50.3 /
-        // 51.0 / 55.8)
-        const bool wide = VEC == 4 && a.slices <= 4 && a.total >= cus * 2048 && bytes % 128 != 0;
-        // PLAIN: the few and, of 16-bit entries in runs of 1 KiB, the backward, forwards of 64 MiB and more, and of 24 MiB and
-        // more where planes share lines and one or two slices hold the dimension, are stored through the cache (streamed /
-        // so, forward: 8 x 21 x 263169 36.2 / 33.9, 2 x 6 x 3000000 27.4 / 26.3, 64 x 10 x 50177 26.4 / 25.5, 32 x 12 x 40001 14.6 / 13.2,
-        // but 16 x 60 x 30001 26.5 / 28.4, 4 x 21 x 263169 20.2 / 21.5, 32 x 12 x 40000 11.7 / 13.3, 32 x 19 x 16384 9.3 / 11.4; backward of
-        // 8 x 21 x 263169 50.0 / 46.8, 32 x 19 x 16385 13.6 / 13.1; fp32 70.8 / 73.2 and 104 / 112, and 16-bit ones in runs of 512
-        // bytes, 16 x 150 x 16384, 37.2 / 39.9 and 42.3 / 47.1 us, are not)
-        const int64_t plain_from = int64_t(bytes % 128 != 0 && a.slices <= 2 ? 24 : 64) << 20;
-        const bool plain = VEC == 8 && (BWD || a.total * dim * 16 >= plain_from);
+        // fp32 planes that fill the device many times over take longer runs, which share fewer lines: 9 to 32 entries, on planes of
+        // whole lines 24, two slices of 128 lanes (slices of up to 8 entries of 64 lanes / of 128 forward and 256 backward / so: 8 x 21 x 263169 forward 71.8 / 69.7 / 66.1,
+        // backward 106 / 96.6 / 94.5 us; 8 x 21 x 263168 62.7 / - / 61.7 and 95.6 / - / 89.1, 2 x 30 x 1000001 forward - / 98.7 / 94.4, 4 x 17 x
+        // 400003 backward - / 64.6 / 60.1, but 128 x 32 x 16384 87 / - / 89 and 129 / - / 134), fewer entries one slice of 128 forward, 256 backward where planes share lines.  Runs of 64 lanes
+        // are as good on planes of whole lines (16 x 2 x 1048576 42.3 / 44.3 and 60.9 / 62.7 us) and better for 16-bit entries
+        // (8 x 21 x 263169 35.3 / 37.8 / 48.1 and 50.3 / 51.0 / 55.8).
+        const bool wide = VEC == 4 && dim <= (odd ? 32 : 24) && a.total >= cus * 2048 && (odd || dim > kDimVecs);
+        if (wide && dim > kDimVecs) { nk = int((dim + 1) / 2); a.slices = 2; }
+        // PLAIN: stored through the cache, where lines that two workgroups share meet.  Larger arrays and planes of whole lines are
+        // streamed (streamed / so, bf16 forward: 60 x 5 x 263169 56.9 / 58.7, 413 x 5 x 12101 20.9 / 19.8, 1322 x 5 x 12101 61.1 / 63.5,
+        // 232 x 21 x 16384 52.6 / 57.4, 18 x 16 x 263169 55.7 / 58.7, 13 x 220 x 4093 15.5 / 16, 13 x 150 x 12101 25.6 / 25.1, 44 x 150 x 12101
+        // 73.7 / 69.7, 30 x 220 x 12101 89 / 85, planes of less than 4 KiB, 1567813 x 4 x 17, 188 / 180, 3043 x 26 x 1033 77 / 68; backward: 976 x 5 x 16384
+        // 74 / 80, 232 x 21 x 16384 75.5 / 82, 15 x 19 x 44480 15.6 / 15.0, 98 x 21 x 12101 29 / 28, 314 x 21 x 12101 85 / 89, 51 x 128 x 12101 98.6 / 103,
+        // 214 x 2 x 1427 3.55 / 3.1, 17 x 11 x 52027 13.0 / 12.5, 5 x 153 x 10427 12.5 / 13.1; fp32, 2 x 193 x 21456 forward 13.0 / 14.8,
+        // 5 x 98 x 12304 backward 13.0 / 15.2, planes of less than 4 KiB, 6614 x 187 x 29, 87 / 75 and 135 / 121).
+        const bool plain = VEC == 8 && BWD && tall                                           ? false
+                           : odd && bytes < 4096 && (BWD || array >= (int64_t(24) << 20)) ? true
+                           : VEC == 4                                                     ? false
+                           : BWD && !many ? array < (int64_t(odd ? 128 : 48) << 20)
+                                               : odd && array >= (int64_t(24) << 20) && ((!BWD && many) || array < (int64_t(128) << 20));
         // Up to kFewSlices slices every thread merges its own values, GPU us, with slices_share / so: 64 x 10 x 12544 bf16 (2
         // slices) forward 8.3 / 7.2, 32 x 12 x 40000 11.7 / 11.1, 4 x 5 x 5904 (3) 3.7 / 3.0, 32 x 40 x 6401 (5) 10.4 / 10.2, 4 x 12 x 5904 (6) 3.6 /
         // 3.35, 16 x 60 x 30001 (8) 25.9 / 27.3.
         // What nk can be.  64 slices: 2 to 4, for 65 to 256 entries.  The few in 32: up to 6, because at 192 entries and past 16
-        // vectors per compute unit they are no longer few; 1 or 2 in few slices.  More than 16 slices are full ones, of `most`
-        // entries each, and more than 6 of them full ones or one entry short of it.
-        const bool few_slices = a.slices <= kFewSlices;
-        if (lx == 16) return launch_softmax_dim<T, BWD, 16, true, false, 2, 4>(a, nk, s);
-        if (few && few_slices) return launch_softmax_dim<T, BWD, 32, true, true, 1, 2>(a, nk, s);
-        if (few) return launch_softmax_dim<T, BWD, 32, true, false, 2, 6>(a, nk, s);
-        if (a.slices > 16) return launch_softmax_dim<T, BWD, 32, false, false, kFull, kDimVecs>(a, nk, s);
-        if constexpr (VEC == 4) {
-          if (wide) return launch_softmax_dim<T, BWD, (BWD ? 256 : 128), false, true, 1, kDimVecs>(a, nk, s);
+        // vectors per compute unit they are no longer few; 1 or 2 in few slices.  32 slices of a quarter's run: 6 to 8, as in 32 of half one.  fp32 in more than six
+        // slices of 64 lanes: 7 or 8; the 16-bit backward of 37 to 48 entries on odd planes: 5 or 6.
+        constexpr int kLeast = BWD ? 4 : 5, kLeastAgain = BWD ? 7 : 12;
+        if (few) {
+          if (lx == 16) return launch_softmax_dim<T, BWD, 16, true, false, 1024, 2, 4>(a, nk, s);
+          if (a.slices <= kFewSlices) return launch_softmax_dim<T, BWD, 32, true, true, 1024, 1, 2>(a, nk, s);
+          return launch_softmax_dim<T, BWD, 32, true, false, 1024, 2, 6>(a, nk, s);
+        }
+        if constexpr (VEC == 8 && !BWD) {
+          if (quarter) return launch_softmax_dim<T, BWD, 16, false, false, 512, 6, 8>(a, nk, s);
+        }
+        if (tall && plain) return launch_softmax_dim<T, BWD, 32, true, false, 1024, 6, kDimVecs>(a, nk, s);
+        if (tall) return launch_softmax_dim<T, BWD, 32, false, false, 1024, 6, kDimVecs>(a, nk, s);
+        if constexpr (BWD && VEC == 8) {
+          // (24 MB / 64 MB of 128 entries 16.6 / 35.9 formed again, 15.4 / 36.8 kept; 160 MB 81.5 / 87.4)
+          if (many && nk <= kDimVecs && array < (int64_t(48) << 20)) {
+            if (plain) return launch_softmax_dim<T, BWD, 32, true, false, 512, kLeast, kDimVecs>(a, nk, s);
+            return launch_softmax_dim<T, BWD, 32, false, false, 512, kLeast, kDimVecs>(a, nk, s);
+          }
         }
         if constexpr (VEC == 8) {
-          if (plain && few_slices) return launch_softmax_dim<T, BWD, 64, true, true, 1, kFull>(a, nk, s);
-          if (plain) return launch_softmax_dim<T, BWD, 64, true, false, kFull - 1, kFull>(a, nk, s);
+          if (many && plain) return launch_softmax_dim<T, BWD, 32, true, false, 512, kLeast, 16, kLeastAgain>(a, nk, s);
+          if (many) return launch_softmax_dim<T, BWD, 32, false, false, 512, kLeast, 16, kLeastAgain>(a, nk, s);
         }
-        if constexpr (VEC == 4 || !BWD) {
-          if (few_slices) return launch_softmax_dim<T, BWD, 64, false, true, 1, kFull>(a, nk, s);
-          return launch_softmax_dim<T, BWD, 64, false, false, kFull - 1, kFull>(a, nk, s);
+        if constexpr (VEC == 4) {
+          if (wide && a.slices == 2) return launch_softmax_dim<T, BWD, 128, false, true, 256, 5, 16>(a, nk, s);
+          if (wide) return launch_softmax_dim<T, BWD, (BWD ? 256 : 128), false, true, 256, 1, kDimVecs>(a, nk, s);
+          if (a.slices > kFewSlices) return launch_softmax_dim<T, BWD, 64, false, false, 1024, kDimVecs - 1, kDimVecs>(a, nk, s);
         }
+        if constexpr (VEC == 8 && BWD) {
+          if (a.slices > kFewSlices && plain) return launch_softmax_dim<T, BWD, 64, true, false, 512, 5, 6>(a, nk, s);
+          if (a.slices > kFewSlices) return launch_softmax_dim<T, BWD, 64, false, false, 512, 5, 6>(a, nk, s);
+        }
+        if (plain) return launch_softmax_dim<T, BWD, 64, true, true, 512, 1, kDimVecs>(a, nk, s);
+        return launch_softmax_dim<T, BWD, 64, false, true, 512, 1, kDimVecs>(a, nk, s);
       }
     }
   }

@@ -152,3 +152,41 @@ def test_forced_widths(hk, cuda, width, cols):
     want = torch.softmax(base.double(), -1)
     helpers.assert_close(y, want.cpu().numpy(), "bf16", "y")
     helpers.assert_close(y2, want.transpose(0, 1).contiguous().cpu().numpy(), "bf16", "y of a view")
+
+
+@pytest.mark.parametrize("dtype,shape", [
+    # slices of 4 to 16 entries, in runs of half and of a quarter of a wavefront's vectors, whole and odd planes, streamed
+    # and through the cache, elements formed again or kept: the edges of the rules on entries and on the array's bytes
+    ("bf16", (68, 32, 2048)), ("bf16", (70, 33, 1984)), ("fp16", (33, 48, 4099)), ("bf16", (33, 49, 4099)),
+    ("bf16", (34, 80, 4096)), ("fp16", (34, 81, 4100)), ("bf16", (32, 96, 4224)), ("bf16", (9, 97, 16383)),
+    ("bf16", (60, 112, 4601)), ("bf16", (60, 128, 4608)), ("fp16", (9, 129, 8185)), ("bf16", (7, 160, 12001)),
+    ("bf16", (6, 161, 8192)), ("fp16", (6, 192, 8190)), ("bf16", (5, 193, 8192)), ("bf16", (6, 208, 21001)),
+    ("bf16", (4, 224, 8777)), ("fp16", (4, 225, 8192)), ("bf16", (3, 256, 11001)), ("bf16", (20, 256, 4992)),
+    ("bf16", (6, 26, 90001)), ("bf16", (6, 40, 60001)), ("bf16", (3000, 21, 403)), ("fp32", (9, 48, 8193)), ("fp32", (2, 9, 1048577)),
+    ("fp32", (3, 21, 700001)), ("fp32", (3, 32, 699904)), ("fp32", (3, 8, 700001)),
+    ("fp32", (9, 64, 8193)), ("fp32", (7, 128, 4100)), ("fp32", (5, 129, 5001)), ("fp32", (4, 256, 4099)),
+    ("fp32", (700, 150, 85))])
+def test_dimension_shapes(hk, cuda, dtype, shape):
+    import torch
+    g = torch.Generator(device=cuda).manual_seed(sum(shape))
+    tt = {"fp32": torch.float32, "bf16": torch.bfloat16, "fp16": torch.float16}[dtype]
+    x = (torch.randn(shape, generator=g, device=cuda) * 3.0).to(tt)
+    x[:, :, 0] = torch.finfo(tt).min           # nothing but the lowest value: uniform
+    x[:, 1:, 1] = -float("inf")                # one finite entry: one-hot
+    dy = torch.randn(shape, generator=g, device=cuda).to(tt)
+    y, dx = torch.empty_like(x), torch.empty_like(x)
+    hk.softmax_fwd(x, y, 1)
+    hk.softmax_bwd(y, dy, dx, 1)
+    ey = torch.softmax(x.double(), 1)
+    d = dy.double()
+    s = y.double()
+    edx = s * (d - (s * d).sum(1, keepdim=True))
+    # the rounding of what is stored (twice half an ulp, for a value that fp32 puts on the other side of a tie), and fp32's:
+    # forward, exponents of up to 32 in magnitude are rounded to 2^-20 and x times the rounded log2(e) is off by 2^-20, times
+    # ln 2, and the exponential and the sum by 2^-22 each: 2^-19 of the result; backward, of the products that the bracket is the
+    # difference of, of which there are up to 256
+    ulp = {"fp32": 2.0 ** -19, "bf16": 2.0 ** -8, "fp16": 2.0 ** -10}[dtype]
+    tiny = 2.0 ** -24 if dtype == "fp16" else 0.0   # fp16 results below its smallest normal number
+    assert bool(((y.double() - ey).abs() <= ulp * ey + tiny).all()), shape
+    size = s * (d.abs() + (s * d.abs()).sum(1, keepdim=True))
+    assert bool(((dx.double() - edx).abs() <= ulp * edx.abs() + 2.0 ** -19 * size + tiny).all()), shape
