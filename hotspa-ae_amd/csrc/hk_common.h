@@ -677,16 +677,17 @@ using MaxSumMaxTuple = OnlineSoftmaxTuple<3>;
 // multiple of 4) apart.  A workgroup of kFoldThreads takes 32 neighbouring columns, one 128-byte line of every row, as 8 float4
 // groups x 32 row slices, so that 256 partial rows, one per compute unit, are 8 loads a thread that are all under way at once:
 // what it costs is one trip to memory, and the columns spread over as many compute units as there are lines.  Slices 8 lanes
-// apart meet in their wavefront, the rest in LDS.  Returned in the first 32 threads: the sum of column 32 * tile + t (0 past
-// pitch).  (128 columns a workgroup, 16 rows a thread in two rounds, as
+// apart meet in their wavefront, the rest in LDS.  Summed in 64 bits, which costs nothing beside that trip: what is left of the
+// rounding is that of the partial rows (900 x 512 fp32, 2-norm 7.8e-8 instead of 1.2e-7).  Returned in the first 32 threads: the
+// sum of column 32 * tile + t (0 past pitch).  (128 columns a workgroup, 16 rows a thread in two rounds, as
 // before: LayerNorm forward and backward of 8191 x 1021 bf16 24.1 us, RMSNorm of 32768 x 4096 216.5; so 23.3 and 214.4.)
 constexpr int kFoldThreads = 256, kFoldCols = 32;
 __device__ __forceinline__ float fold_partial_rows(const float* part, int nparts, int pitch, int tile) {
   constexpr int U = 8, SLICES = kFoldThreads / 8;
-  __shared__ float lds[SLICES / 2][kFoldCols];
+  __shared__ double lds[SLICES / 2][kFoldCols];
   const int cg = int(threadIdx.x) & 7, slice = int(threadIdx.x) >> 3;
   const int c = tile * kFoldCols + cg * 4;
-  float acc[4] = {0.f, 0.f, 0.f, 0.f};
+  double acc[4] = {0., 0., 0., 0.};
   if (c < pitch) {
     for (int r = slice; r < nparts; r += U * SLICES) {
       u32x4 v[U];
@@ -705,16 +706,18 @@ __device__ __forceinline__ float fold_partial_rows(const float* part, int nparts
   }
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
-    acc[k] += dpp_perm<kDppRor8>(acc[k]);
+    const uint64_t bits = uint64_t(__double_as_longlong(acc[k]));
+    const uint32_t lo = f2u(dpp_perm<kDppRor8>(u2f(uint32_t(bits)))), hi = f2u(dpp_perm<kDppRor8>(u2f(uint32_t(bits >> 32))));
+    acc[k] += __longlong_as_double(int64_t(uint64_t(hi) << 32 | lo));
     if ((slice & 1) == 0) lds[slice >> 1][cg * 4 + k] = acc[k];
   }
   __syncthreads();
-  float s = 0.f;
+  double s = 0.;
   if (threadIdx.x < kFoldCols) {
 #pragma unroll
     for (int i = 0; i < SLICES / 2; ++i) s += lds[i][threadIdx.x];
   }
-  return s;
+  return float(s);
 }
 
 // The maximum of a thread's elements in the log2 domain, kept finite.  Below: a maximum near the type's lowest value
