@@ -329,11 +329,15 @@ __device__ __forceinline__ u32x4 ld16_stream(const void* p) {
 struct LevelSteps {
   int64_t p1, p2;   // elements between consecutive j1 / j2; the step of j0 is the operand's pitch
 };
+struct ShortLevelSteps {   // the same below 2^31
+  int p1, p2;
+};
 struct RowNumbering {
   int64_t rn0, rn1, rn2;
 };
 // offset of this workgroup's rows along the two outer walk levels, in elements
-__device__ __forceinline__ int64_t outer_level_offset(const LevelSteps& l) {
+template <typename L>
+__device__ __forceinline__ int64_t outer_level_offset(const L& l) {
   return int64_t(blockIdx.y) * l.p1 + int64_t(blockIdx.z) * l.p2;
 }
 // number of the row (j0, blockIdx.y, blockIdx.z)
@@ -555,7 +559,8 @@ __device__ __forceinline__ P group_allreduce_tuple_fixed(P a, float* scratch) {
 // workgroup; LPR == 0: the whole workgroup.
 template <int LPR>
 struct RowLanes {
-  static __device__ __forceinline__ int count() { return LPR ? LPR : int(blockDim.x); }
+  // threads: the workgroup's
+  static __device__ __forceinline__ int count(int threads) { return LPR ? LPR : threads; }
   static __device__ __forceinline__ int lane() { return LPR ? int(threadIdx.x) & (LPR - 1) : int(threadIdx.x); }
   static __device__ __forceinline__ int64_t row() {
     if constexpr (LPR == 0) return int64_t(blockIdx.x);
@@ -563,8 +568,8 @@ struct RowLanes {
     else return int64_t(blockIdx.x) * (256 / LPR) + int(threadIdx.x) / LPR;
   }
   template <typename P>
-  static __device__ __forceinline__ P allreduce(P p, float* red) {
-    if constexpr (LPR == 0) return group_allreduce_tuple(p, red, 0, int(blockDim.x >> 6));
+  static __device__ __forceinline__ P allreduce(P p, float* red, int threads) {
+    if constexpr (LPR == 0) return group_allreduce_tuple(p, red, 0, threads >> 6);
     else return lanes_allreduce_tuple<LPR>(p);
   }
 };
@@ -917,6 +922,13 @@ static inline bool lds_bytes_for_residency(int workgroups, size_t static_bytes, 
   return true;
 }
 
+//
+// What a launch costs the host depends on how many bytes of arguments it writes: 64 to 112 of them 2.65 to 2.8 us a launch
+// among others, 120 to 512 3.5 to 3.8 in a program that does nothing else (on one host of several 2.33 and 2.45; from Python
+// about 0.3 us a launch).  A kernel that reads blockDim or gridDim has 66 more written beside its own.  Kernels that are
+// launched for small work take what they need in kCheapArgs bytes, their threads and blocks among it: steps and counts that
+// fit 32 bits, without what only some instances use.
+constexpr size_t kCheapArgs = 112;
 #define HK_LAUNCH(kernel, grid, block, lds_bytes, stream, ...)                                                  \
   do {                                                                                                          \
     hipEvent_t hk_ev_before_, hk_ev_after_;                                                                     \

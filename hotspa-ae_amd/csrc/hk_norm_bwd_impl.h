@@ -67,7 +67,8 @@ __device__ __forceinline__ float clamp_by_magnitude(float g, float eps) {
 template <typename T, int NV, int MODE, int PF, bool EXACT, bool STATS_F32, bool EXTRA, int MAXT, bool FIXED,
           bool CLAMP, bool LEVELS = false, bool RAGGED = false, int LPR = 0>
 __global__ __launch_bounds__(MAXT)
-void norm_bwd_kernel(NormBwdArgs a) {
+void norm_bwd_kernel(typename std::conditional<LEVELS || EXTRA, NormBwdArgs, NormBwdFlat>::type given) {
+  const NormBwdArgs a = given.template args<T, MODE>();
   static_assert(LPR == 0 || (RAGGED && LPR < kWave && NV == 1), "several rows to a wavefront: any boundary, a vector per lane");
   static_assert(!LEVELS || (FIXED && !EXTRA && EXACT), "the running walk index is built for the lean instances");
   static_assert(!RAGGED || (!FIXED && !EXACT), "rows of any boundary: any group width, a partial last vector");
@@ -81,7 +82,7 @@ void norm_bwd_kernel(NormBwdArgs a) {
   __shared__ __align__(16) float red[2][kMaxWaves * KS];  // double-buffered by step parity
 
   const int tpr = FIXED ? MAXT : LPR ? LPR : a.tpr;   // without LPR a multiple of 64: a wavefront never straddles two rows
-  const int rpb = FIXED ? 1 : int(blockDim.x) / tpr;
+  const int rpb = FIXED ? 1 : a.threads / tpr;
   const int group = FIXED ? 0 : LPR ? int(threadIdx.x) / tpr : __builtin_amdgcn_readfirstlane(int(threadIdx.x) / tpr);
   const int t = int(threadIdx.x) - group * tpr;
   const int waves_per_group = tpr >> 6;
@@ -116,7 +117,7 @@ void norm_bwd_kernel(NormBwdArgs a) {
 #pragma unroll
   for (int e = 0; e < NE; ++e) { dg[e] = 0.f; db[e] = 0.f; }
 
-  const int64_t stride = int64_t(gridDim.x) * rpb;
+  const int64_t stride = int64_t(a.blocks) * rpb;
   const int64_t last_row = a.rows - 1;
   u32x4 nx[PF][NV], ndy[PF][NV];
   StatT nmu[PF], nsv[PF];
@@ -385,7 +386,7 @@ void norm_bwd_kernel(NormBwdArgs a) {
   const int pitch = a.part_pitch, region = rpb * pitch;
   auto fold = [&](const float* src, float* dst) {
     if (dst == nullptr) return;
-    for (int c = int(threadIdx.x) * 4; c < pitch; c += int(blockDim.x) * 4) {
+    for (int c = int(threadIdx.x) * 4; c < pitch; c += a.threads * 4) {
       float r[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 8
       for (int g = 0; g < rpb; ++g) {
@@ -452,7 +453,7 @@ void norm_bwd_generic_dx_kernel(NormBwdArgs a, int mode) {
     return rs * (xv - mu);
   };
   CT s1 = 0, s2 = 0;
-  for (int c = threadIdx.x; c < a.cols; c += blockDim.x) {
+  for (int c = threadIdx.x; c < a.cols; c += 256) {
     const CT g = gp ? GenericIO<T, CT>::ld(gp + c) : CT(1);
     const CT d = GenericIO<T, CT>::ld(dyr + c);
     if (mode == BWD_LN_MEMEFF) {
@@ -470,7 +471,7 @@ void norm_bwd_generic_dx_kernel(NormBwdArgs a, int mode) {
   T* dxr = static_cast<T*>(a.dx) + i0 * a.dx_pitch + outer_level_offset(a.dx_lv);
   T* drr = a.dres ? static_cast<T*>(a.dres) + i0 * a.dres_pitch + outer_level_offset(a.dres_lv) : nullptr;
   const T* dir = a.dx_in ? static_cast<const T*>(a.dx_in) + i0 * a.dxin_pitch + outer_level_offset(a.dxin_lv) : nullptr;
-  for (int c = threadIdx.x; c < a.cols; c += blockDim.x) {
+  for (int c = threadIdx.x; c < a.cols; c += 256) {
     const CT g = gp ? GenericIO<T, CT>::ld(gp + c) : CT(1);
     const CT d = GenericIO<T, CT>::ld(dyr + c);
     CT o = rs * (d * kgamma(g) - c1 - xhat_of(c, g) * c2);
@@ -664,11 +665,14 @@ static int launch_norm_bwd_inst(const NormBwdArgs& a, const BwdPlan& p, int pf, 
   // (dbeta under RMSNorm counts as optional: the lean RMSNorm instances do not form it)
   const bool optional = a.dx_in != nullptr || a.dres != nullptr || (want_clamp && MODE != BWD_LN) ||
                         (MODE == BWD_RMS && a.part_dbeta != nullptr);
-  const bool extra = optional || (levels && !(fixed && exact));
+  const bool extra = optional || (levels ? !(fixed && exact) : !NormBwdFlat::holds(a));
   // the deep ring exists for the plain case only: full rows, no optional operands
   if (!exact || extra) pf = 1;
-#define HK_BWD_LAUNCH_L(P, E, F, X, FX, C, L) \
-  HK_LAUNCH((norm_bwd_kernel<T, NV, MODE, P, E, F, X, MAXT, FX, C, L>), grid, block, p.lds_bytes, s, a)
+#define HK_BWD_LAUNCH_L(P, E, F, X, FX, C, L)                                                                            \
+  do {                                                                                                                  \
+    if constexpr (X || L) HK_LAUNCH((norm_bwd_kernel<T, NV, MODE, P, E, F, X, MAXT, FX, C, L>), grid, block, p.lds_bytes, s, a); \
+    else HK_LAUNCH((norm_bwd_kernel<T, NV, MODE, P, E, F, X, MAXT, FX, C, L>), grid, block, p.lds_bytes, s, NormBwdFlat(a, MODE)); \
+  } while (0)
 #define HK_BWD_LAUNCH(P, E, F, X, FX, C) HK_BWD_LAUNCH_L(P, E, F, X, FX, C, false)
 #define HK_BWD_LEAN_L(P, F, FX, L)                                          \
   do {                                                                      \
@@ -706,7 +710,7 @@ static void launch_norm_bwd_lanes(const NormBwdArgs& a, const BwdPlan& p, hipStr
   const dim3 grid{unsigned(p.grid)}, block{unsigned(p.block)};
 #define HK_BWD_LANES(NV, LPR) \
   HK_LAUNCH((norm_bwd_kernel<T, NV, MODE, 2, false, true, false, MAXT, false, CLAMP, false, true, LPR>), grid, block, \
-            p.lds_bytes, s, a)
+            p.lds_bytes, s, NormBwdFlat(a, MODE))
   if (p.lpr == 16) HK_BWD_LANES(1, 16); else HK_BWD_LANES(1, 32);
 #undef HK_BWD_LANES
 }
@@ -714,10 +718,13 @@ static void launch_norm_bwd_lanes(const NormBwdArgs& a, const BwdPlan& p, hipStr
 template <typename T, int MODE>
 static int launch_norm_bwd_any(const NormBwdArgs& a, const BwdPlan& p, hipStream_t s) {
   const dim3 grid{unsigned(p.grid)}, block{unsigned(p.block)};
-#define HK_BWD_ANY_P(P, NV, F, X) \
-  HK_LAUNCH((norm_bwd_kernel<T, NV, MODE, P, false, F, X, 1024, false, false, false, true>), grid, block, p.lds_bytes, s, a)
+#define HK_BWD_ANY_P(P, NV, F, X)                                                                                            \
+  do {                                                                                                                    \
+    if constexpr (X) HK_LAUNCH((norm_bwd_kernel<T, NV, MODE, P, false, F, X, 1024, false, false, false, true>), grid, block, p.lds_bytes, s, a); \
+    else HK_LAUNCH((norm_bwd_kernel<T, NV, MODE, P, false, F, X, 1024, false, false, false, true>), grid, block, p.lds_bytes, s, NormBwdFlat(a, MODE)); \
+  } while (0)
 #define HK_BWD_ANY(NV, F) HK_BWD_ANY_P(1, NV, F, true)
-  const bool extra = a.dx_in != nullptr || a.dres != nullptr || a.clamp_gamma != 0 || a.n0 != a.rows ||
+  const bool extra = a.dx_in != nullptr || a.dres != nullptr || a.clamp_gamma != 0 || !NormBwdFlat::holds(a) ||
                      (MODE == BWD_RMS && a.part_dbeta != nullptr) || !a.stats_f32;
   profile_before(s);
   if constexpr (MODE != BWD_LN_MEMEFF) {
@@ -815,7 +822,7 @@ int norm_bwd_typed(NormBwdArgs a, int mode, void* dgamma, void* dbeta, void* ws,
   if (p.any && want_cols && (ws == nullptr || ws_bytes < p.ws_bytes || !aligned16(ws))) p.reg_path = false;
   if (p.any && !a.stats_f32 && mode != BWD_LN) p.reg_path = false;
   if (p.reg_path && tune_get(TUNE_NORM_BWD_THREADS) <= 0) {
-    const bool lean = mode != BWD_LN_MEMEFF && a.stats_f32 && !a.dx_in && !a.dres && a.n0 == a.rows &&
+    const bool lean = mode != BWD_LN_MEMEFF && a.stats_f32 && !a.dx_in && !a.dres && NormBwdFlat::holds(a) &&
                       !(mode == BWD_RMS && (dbeta != nullptr || a.clamp_gamma));
     const BwdPlan q = lean ? plan_norm_bwd_lanes<T>(a.rows, a.cols) : BwdPlan{};
     // (a scratch that was sized for the other plans alone still serves them)
@@ -846,6 +853,8 @@ int norm_bwd_typed(NormBwdArgs a, int mode, void* dgamma, void* dbeta, void* ws,
     a.part_dbeta = nullptr;
   }
   a.tpr = p.tpr;
+  a.threads = uint16_t(p.block);
+  a.blocks = p.grid;
   {
     // the walking kernel's row stride, split over the walk levels (used by the instances with a running walk index)
     const uint64_t stride = uint64_t(p.grid) * uint64_t(p.rpb);

@@ -29,22 +29,24 @@ namespace hk {
 // the normalisation costs one multiply and one multiply-add per element.  Which values stay in registers across
 // the reductions is written out here rather than left to the compiler: with the row kept packed and unpacked again
 // per pass, unrelated edits moved the 5120-column bf16 kernel between 57.7 and 61 us.
-template <typename T, int NV, bool WAVE_ROW, bool HAS_RES, bool IS_RMS, int R>
+// A: NormFwdArgs, or NormFwdFlat where that holds the arguments
+template <typename T, int NV, bool WAVE_ROW, bool HAS_RES, bool IS_RMS, int R, typename A>
 __global__ __launch_bounds__(WAVE_ROW ? 256 : (R >= 2 ? 512 : 1024))   // several rows: at most 512 threads
-void norm_fwd_kernel(NormFwdArgs a) {
+void norm_fwd_kernel(A given) {
+  const NormFwdArgs a = given.args();
   static_assert(R == 1 || !WAVE_ROW, "a wavefront takes one row");
   constexpr int VEC = VecIO<T>::N;
   constexpr int NE = NV * VEC;
   __shared__ __align__(16) float red[2][kMaxWaves * 2 * R];   // one slot per reduction of the kernel
 
-  const int tpr = WAVE_ROW ? kWave : int(blockDim.x);
+  const int tpr = WAVE_ROW ? kWave : a.threads;
   const int t = WAVE_ROW ? int(threadIdx.x & 63) : int(threadIdx.x);
   const int64_t row0 = WAVE_ROW
-      ? int64_t(blockIdx.x) * (blockDim.x >> 6) + wave_index()
+      ? int64_t(blockIdx.x) * (256 / kWave) + wave_index()
       : int64_t(blockIdx.x) * R;
   // row0 counts along the first walk level; blockIdx.y / z are the other two (one level: both 0)
   if (WAVE_ROW && row0 >= a.n0) return;  // wave-uniform; no block barrier in this mode
-  const int nwaves = WAVE_ROW ? 1 : int(blockDim.x >> 6);
+  const int nwaves = WAVE_ROW ? 1 : tpr >> 6;
   auto off = [&](int i) { return uint32_t(i * tpr + t) * 16u; };   // vector i of thread t, in bytes from the row's start
   // long rows: stops the scheduler from unpacking every vector of a pass before the first one is consumed
   auto fence = [] { if constexpr (NV * R >= 8) __builtin_amdgcn_sched_barrier(0); };
@@ -243,16 +245,17 @@ void norm_fwd_kernel(NormFwdArgs a) {
 // 8191 x 1021 30.7 us element by element -> 8.1 us; 16384 x 2047 100 -> 30.5 us, 4.4 TB/s, 2048 columns 25 us; 10000 x 8191
 // 290 -> 81 us; 8192 x 8191 fp32 219 -> 99 us, 5.4 TB/s; accesses on 4-byte boundaries (RaggedRow): 9000 x 7001 72 -> 66 us,
 // 14549 x 3579 57 -> 53, RMSNorm 47 -> 41; stored through the cache 8191 x 1021 takes 10.3).
-template <typename T, int NV, int LPR, bool HAS_RES, bool IS_RMS>
+template <typename T, int NV, int LPR, bool HAS_RES, bool IS_RMS, typename A>
 __global__ __launch_bounds__(LPR ? 256 : 1024)
-void norm_fwd_any_kernel(NormFwdArgs a) {
+void norm_fwd_any_kernel(A given) {
+  const NormFwdArgs a = given.args();
   constexpr int VEC = VecIO<T>::N;
   // (a LayerNorm row of a wavefront pays more for gamma and beta off their 16-byte boundaries: 16000 x 2047 29.4 us, 31.0
   // with its own accesses on 4 bytes)
   constexpr bool kShift = IS_RMS || LPR == 0;
   using Lanes = RowLanes<LPR>;
   __shared__ float red[2][kMaxWaves * 2];
-  const int tpr = Lanes::count(), t = Lanes::lane();
+  const int tpr = Lanes::count(a.threads), t = Lanes::lane();
   const int64_t row = Lanes::row();
   if (LPR && row >= a.n0) return;   // row counts within the innermost level
 
@@ -308,7 +311,7 @@ void norm_fwd_any_kernel(NormFwdArgs a) {
   if constexpr (IS_RMS) {
     SumTuple<2> both = SumTuple<2>::identity();
     each([&](float x) { both.v[0] = fmaf(x, x, both.v[0]); both.v[1] += x; });
-    both = Lanes::allreduce(both, red[0]);
+    both = Lanes::allreduce(both, red[0], tpr);
     const float ms = both.v[0] * a.inv_cols;   // mean(x^2) = var + mu^2
     mu = both.v[1] * a.inv_cols;
     var = fmaxf(ms - mu * mu, 0.f);
@@ -318,7 +321,7 @@ void norm_fwd_any_kernel(NormFwdArgs a) {
     // the mean first, then the sum of squares about it, as in norm_fwd_kernel
     SumTuple<1> s = SumTuple<1>::identity();
     each([&](float x) { s.v[0] += x; });
-    s = Lanes::allreduce(s, red[0]);
+    s = Lanes::allreduce(s, red[0], tpr);
     mu = s.v[0] * a.inv_cols;
     store_sum();
     s = SumTuple<1>::identity();
@@ -327,7 +330,7 @@ void norm_fwd_any_kernel(NormFwdArgs a) {
 #pragma unroll
       for (int j = 0; j < VEC; ++j) v[i][j] -= mu;
     each([&](float x) { s.v[0] = fmaf(x, x, s.v[0]); });
-    s = Lanes::allreduce(s, red[1]);
+    s = Lanes::allreduce(s, red[1], tpr);
     var = s.v[0] * a.inv_cols;
     rs = 1.0f / sqrtf(var + a.eps);
   }
@@ -380,7 +383,7 @@ void norm_fwd_generic_kernel(NormFwdArgs a) {
     return v;
   };
   CT s = 0, ss = 0;
-  for (int c = threadIdx.x; c < a.cols; c += blockDim.x) {
+  for (int c = threadIdx.x; c < a.cols; c += 256) {
     const CT v = ldx(c);
     if (xo) GenericIO<T, CT>::st(xo + c, v);
     s += v;
@@ -398,7 +401,7 @@ void norm_fwd_generic_kernel(NormFwdArgs a) {
     rs = CT(1) / sqrt(ms + CT(a.eps));
   } else {
     CT m2 = 0;
-    for (int c = threadIdx.x; c < a.cols; c += blockDim.x) {
+    for (int c = threadIdx.x; c < a.cols; c += 256) {
       const CT d = ldx(c) - mu;
       m2 += d * d;
     }
@@ -421,7 +424,7 @@ void norm_fwd_generic_kernel(NormFwdArgs a) {
   T* yr = static_cast<T*>(a.y) + i0 * a.y_pitch + outer_level_offset(a.y_lv);
   const T* gp = static_cast<const T*>(a.gamma);
   const T* bp = static_cast<const T*>(a.beta);
-  for (int c = threadIdx.x; c < a.cols; c += blockDim.x) {
+  for (int c = threadIdx.x; c < a.cols; c += 256) {
     const CT g = gp ? GenericIO<T, CT>::ld(gp + c) : CT(1);
     const CT b = bp ? GenericIO<T, CT>::ld(bp + c) : CT(0);
     GenericIO<T, CT>::st(yr + c, g * (rs * (ldx(c) - shift)) + b);
@@ -439,7 +442,8 @@ static constexpr int max_rows_per_block(int nv, bool has_res) {
 
 // rows_per_block: 1 or 2 (one-wavefront rows always 1)
 template <typename T, int NV, bool WAVE_ROW, bool HAS_RES, bool IS_RMS>
-static int launch_norm_fwd_width(const NormFwdArgs& a, int rows_per_block, dim3 grid, dim3 block, hipStream_t s) {
+static int launch_norm_fwd_width(NormFwdArgs a, int rows_per_block, dim3 grid, dim3 block, hipStream_t s) {
+  a.threads = uint16_t(block.x);
   if constexpr (!WAVE_ROW && max_rows_per_block<T>(NV, HAS_RES) >= 2) {
     if (rows_per_block == 2) {
       // two rows of several vectors per thread: fewer workgroups per compute unit than the thread limit admits
@@ -451,13 +455,14 @@ static int launch_norm_fwd_width(const NormFwdArgs& a, int rows_per_block, dim3 
       HK_REQUIRE(lds_bytes_for_residency(resident, sizeof(float) * 2 * kMaxWaves * 2 * 2, &lds), HK_ERR_INVALID,
                  "norm_fwd: 'norm_fwd_resident' = %d needs more dynamic LDS than one workgroup may ask for", resident);
       profile_before(s);
-      HK_LAUNCH((norm_fwd_kernel<T, NV, false, HAS_RES, IS_RMS, 2>), grid, block, lds, s, a);
+      HK_LAUNCH((norm_fwd_kernel<T, NV, false, HAS_RES, IS_RMS, 2, NormFwdArgs>), grid, block, lds, s, a);
       profile_after(s);
       return HK_OK;
     }
   }
   profile_before(s);
-  HK_LAUNCH((norm_fwd_kernel<T, NV, WAVE_ROW, HAS_RES, IS_RMS, 1>), grid, block, 0, s, a);
+  if (NormFwdFlat::holds(a)) HK_LAUNCH((norm_fwd_kernel<T, NV, WAVE_ROW, HAS_RES, IS_RMS, 1, NormFwdFlat>), grid, block, 0, s, NormFwdFlat(a));
+  else HK_LAUNCH((norm_fwd_kernel<T, NV, WAVE_ROW, HAS_RES, IS_RMS, 1, NormFwdArgs>), grid, block, 0, s, a);
   profile_after(s);
   return HK_OK;
 }
@@ -559,17 +564,25 @@ static bool pick_row_shape(int nvec, int forced_threads, int max_nv, int wave_ro
 }
 
 template <typename T, int LPR, bool HAS_RES, bool IS_RMS>
-static int launch_norm_fwd_any_nv(const NormFwdArgs& a, int nv, dim3 grid, dim3 block, hipStream_t s) {
-#define HK_ANY_CASE(N) case N: HK_LAUNCH((norm_fwd_any_kernel<T, N, LPR, HAS_RES, IS_RMS>), grid, block, 0, s, a); break;
+static int launch_norm_fwd_any_nv(NormFwdArgs a, int nv, dim3 grid, dim3 block, hipStream_t s) {
+  a.threads = uint16_t(block.x);
+  const bool flat = NormFwdFlat::holds(a);
+#define HK_ANY_LAUNCH(N)                                                                                                          \
+  do {                                                                                                                            \
+    if (flat) HK_LAUNCH((norm_fwd_any_kernel<T, N, LPR, HAS_RES, IS_RMS, NormFwdFlat>), grid, block, 0, s, NormFwdFlat(a)); \
+    else HK_LAUNCH((norm_fwd_any_kernel<T, N, LPR, HAS_RES, IS_RMS, NormFwdArgs>), grid, block, 0, s, a);                      \
+  } while (0)
+#define HK_ANY_CASE(N) case N: HK_ANY_LAUNCH(N); break;
   profile_before(s);
   if constexpr (LPR == kWave) {
     switch (nv) { HK_ANY_CASE(1) HK_ANY_CASE(2) HK_ANY_CASE(3) default: HK_ANY_CASE(4) }
   } else if constexpr (LPR == 0) {
     switch (nv) { HK_ANY_CASE(2) HK_ANY_CASE(4) default: HK_ANY_CASE(8) }
   } else {
-    HK_LAUNCH((norm_fwd_any_kernel<T, 1, LPR, HAS_RES, IS_RMS>), grid, block, 0, s, a);
+    HK_ANY_LAUNCH(1);
   }
 #undef HK_ANY_CASE
+#undef HK_ANY_LAUNCH
   profile_after(s);
   return launch_check("norm_fwd_any_kernel");
 }

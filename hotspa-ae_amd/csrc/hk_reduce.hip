@@ -138,7 +138,7 @@ __device__ __forceinline__ ACC block_reduce_lds(ACC v, ACC* lds) {
   const int tid = threadIdx.x;
   lds[tid] = v;
   __syncthreads();
-  for (int s = blockDim.x >> 1; s > 0; s >>= 1) {
+  for (int s = 256 >> 1; s > 0; s >>= 1) {
     if (tid < s) lds[tid] = R::template apply<ACC>(lds[tid], lds[tid + s]);
     __syncthreads();
   }
@@ -178,7 +178,7 @@ struct InnerArgs {
   int64_t run_stride;
   int64_t chunk;      // vectors per split, out of nruns * ceil(cols / vector)
   int nsplit;
-  int lanes;          // LANES: 1, 2, 4, ... 64 lanes take a row
+  int lanes;          // threads that take a row: LANES 1, 2, 4, ... 64, else the workgroup's
   float factor;
   int is_mean;
 };
@@ -205,11 +205,11 @@ void reduce_inner_vec_kernel(InnerArgs a) {
   constexpr int VEC = VecIO<T>::N;
   constexpr int U = 8;
   __shared__ float red[kMaxWaves];
-  const int tpr = WAVE ? kWave : LANES ? a.lanes : int(blockDim.x);
+  const int tpr = WAVE ? kWave : a.lanes;
   const int t = LANES ? int(threadIdx.x) & (tpr - 1) : int(threadIdx.x);
   const int64_t row = !LANES ? int64_t(blockIdx.x)
-                    : tpr == kWave ? int64_t(blockIdx.x) * (blockDim.x >> 6) + wave_index()
-                                   : (int64_t(blockIdx.x) * blockDim.x + threadIdx.x) >> __builtin_ctz(tpr);
+                    : tpr == kWave ? int64_t(blockIdx.x) * (256 / kWave) + wave_index()
+                                   : (int64_t(blockIdx.x) * 256 + threadIdx.x) >> __builtin_ctz(tpr);
   if (LANES && row >= a.rows) return;   // whole groups of lanes leave
   const int split = blockIdx.y;
   int64_t base = row * a.row_stride;
@@ -293,7 +293,7 @@ void reduce_inner_vec_kernel(InnerArgs a) {
   if constexpr (LANES) {
     s = lanes_reduce<R>(s, tpr);
   } else {
-    s = block_allreduce<AsFloatOp<R>>(s, red, int(blockDim.x >> 6));
+    s = block_allreduce<AsFloatOp<R>>(s, red, tpr >> 6);
   }
   if (t == 0) {
     if (a.nsplit == 1) st_acc<OUT_T, float>(static_cast<OUT_T*>(a.out) + row, R::template post<float>(s, a.factor, a.is_mean));
@@ -329,7 +329,7 @@ void reduce_inner_scalar_kernel(const T* in, OUT_T* out, int64_t rows, int64_t r
   const int64_t row = blockIdx.x;
   const T* p = in + row * row_stride;
   ACC acc = R::template identity<ACC>();
-  for (int64_t c = threadIdx.x; c < cols; c += blockDim.x) acc = R::template apply<ACC>(acc, R::template pre<ACC>(ld_acc<T, ACC>(p + c), factor));
+  for (int64_t c = threadIdx.x; c < cols; c += 256) acc = R::template apply<ACC>(acc, R::template pre<ACC>(ld_acc<T, ACC>(p + c), factor));
   acc = block_reduce_lds<R, ACC>(acc, lds);
   if (threadIdx.x == 0) st_acc<OUT_T, ACC>(out + row, R::template post<ACC>(acc, factor, is_mean));
 }
@@ -345,7 +345,7 @@ struct OuterArgs {
   int64_t b_stride, r_stride;   // elements
   int64_t rows_per_split;
   int rsplit;
-  int wx;               // wavefronts of a workgroup side by side across columns (the others stack over rows)
+  int wx, wy;           // wavefronts of a workgroup side by side across columns, and stacked over rows
   float factor;
   int is_mean;
   int split_major;      // grid = (row splits, column tiles, batch) instead of (column tiles, row splits, batch)
@@ -363,7 +363,7 @@ void reduce_outer_vec_kernel(OuterArgs a) {
   const int wx = a.wx;
   const int wc = wave % wx;        // this wavefront's place across columns ...
   const int w = wave / wx;         // ... and over rows
-  const int wy = int(blockDim.x >> 6) / wx;
+  const int wy = a.wy;
   // Row splits along the grid's x (whenever the column tiles fit its y): workgroups are dealt to the XCDs round
   // robin in x-major order, so the workgroups of one XCD then take whole runs of rows (every column tile of a few
   // row splits) rather than one column tile of every row split -- the same bytes in flight at any time, 1 % faster
@@ -509,7 +509,7 @@ template <typename T, typename ACC, typename OUT_T, typename R>
 __global__ __launch_bounds__(256)
 void reduce_outer_scalar_kernel(const T* in, OUT_T* out, int64_t B, int64_t NR, int64_t C,
                                 int64_t b_stride, int64_t r_stride, float factor, int is_mean) {
-  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
   if (i >= B * C) return;
   const int64_t b = i / C, c = i - b * C;
   const T* p = in + b * b_stride + c;
@@ -532,7 +532,7 @@ struct GenericMeta {
 template <typename T, typename ACC, typename OUT_T, typename R>
 __global__ __launch_bounds__(256)
 void reduce_generic_kernel(const T* in, OUT_T* out, GenericMeta m, float factor, int is_mean) {
-  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
   if (i >= m.n_out) return;
   int64_t rem = i, base = 0;
   for (int d = m.n_keep - 1; d >= 0; --d) {
@@ -813,7 +813,7 @@ static int launch_outer(const ReducePlan& p, const OuterShape& s, const void* in
   constexpr int VEC = 16 / sizeof(T);
   OuterArgs a{};
   a.in = in; a.out = out; a.B = p.B; a.R = p.R; a.C = p.C; a.b_stride = p.b_stride; a.r_stride = p.r_stride;
-  a.rows_per_split = s.rows_per_split; a.rsplit = s.rsplit; a.wx = s.wx; a.factor = factor; a.is_mean = is_mean;
+  a.rows_per_split = s.rows_per_split; a.rsplit = s.rsplit; a.wx = s.wx; a.wy = s.wy; a.factor = factor; a.is_mean = is_mean;
   a.partial = partial;
   const int64_t col_tiles = (((p.C + VEC - 1) / VEC + 63) / 64 + s.wx - 1) / s.wx;
   a.split_major = col_tiles <= 65535 ? 1 : 0;

@@ -16,7 +16,7 @@ namespace hk {
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kNegInf = -__builtin_huge_valf();
 
-struct SoftmaxArgs {
+struct SoftmaxRows {
   const void* x;    // forward: input;  backward: y
   const void* dy;   // backward only
   void* out;        // forward: y;      backward: dx
@@ -28,6 +28,18 @@ struct SoftmaxArgs {
   int nvec;
   int spare;        // see RaggedRow
 };
+// What the kernels take of it (see kCheapArgs).  Steps below 2^31 elements; what lies further apart goes out in several launches
+// (launch_softmax), of which there are few, as so much memory lies between them.
+struct SoftmaxArgs {
+  const void* x;
+  const void* dy;
+  void* out;
+  int n0, x_pitch, dy_pitch, out_pitch;
+  ShortLevelSteps x_lv, dy_lv, out_lv;
+  int cols, nvec, spare;
+  int threads;      // of a workgroup
+};
+static_assert(sizeof(SoftmaxArgs) <= kCheapArgs, "");
 
 template <typename T, int NV, int LPR, bool RAGGED>
 __global__ __launch_bounds__(LPR ? 256 : 1024)
@@ -35,7 +47,7 @@ void softmax_fwd_kernel(SoftmaxArgs a) {
   constexpr int VEC = VecIO<T>::N;
   using Lanes = RowLanes<LPR>;
   __shared__ float red[kMaxWaves * 2];
-  const int tpr = Lanes::count(), t = Lanes::lane();
+  const int tpr = Lanes::count(a.threads), t = Lanes::lane();
   const int64_t row = Lanes::row();
   if (LPR && row >= a.n0) return;   // row counts within the innermost level
 
@@ -67,7 +79,7 @@ void softmax_fwd_kernel(SoftmaxArgs a) {
   // row's maximum first: its butterfly is cheaper than merging (maximum, sum) pairs, whose every step takes two
   // exponentials, and an element held twice then comes out the same twice.  Across wavefronts each thread keeps its
   // own maximum and the pairs are merged, which costs one barrier instead of two.
-  if constexpr (LPR > 0) m = Lanes::allreduce(MaxTuple{{m}}, red).v[0];
+  if constexpr (LPR > 0) m = Lanes::allreduce(MaxTuple{{m}}, red, a.threads).v[0];
   // A row whose maximum lies at the type's lowest values (scores masked with it) or at its highest would overflow in the
   // log2 domain: two different values out there are so far apart that any base gives 1 at the maximum and 0 elsewhere, so
   // lanes that agree on the row's maximum take base 2 for such a row.  A whole workgroup's threads have maxima of their
@@ -88,16 +100,16 @@ void softmax_fwd_kernel(SoftmaxArgs a) {
   T* yr = static_cast<T*>(a.out) + row * a.out_pitch + outer_level_offset(a.out_lv);
   float scale;
   if constexpr (LPR > 0) {
-    scale = 1.0f / Lanes::allreduce(SumTuple<1>{{s}}, red).v[0];
+    scale = 1.0f / Lanes::allreduce(SumTuple<1>{{s}}, red, a.threads).v[0];
   } else {
     MaxSumTuple p;
     p.v[0] = ml; p.v[1] = s;
-    p = Lanes::allreduce(p, red);
+    p = Lanes::allreduce(p, red, a.threads);
     if (past_log2_range(p.v[0])) {   // uniform
       float M;
       const float n = row_max_count<T>(xr, a.cols, t, tpr, [&](auto v) {
         __syncthreads();   // red may still be read
-        return Lanes::allreduce(v, red);
+        return Lanes::allreduce(v, red, a.threads);
       }, M);
       const float inv = 1.0f / (M == kNegInf ? __builtin_nanf("") : n);   // nothing but -inf has no softmax
       for (int c = t; c < a.cols; c += tpr) Cvt<T>::store(yr + c, (Cvt<T>::load(xr + c) == M ? 1.f : 0.f) * inv);
@@ -124,7 +136,7 @@ void softmax_bwd_kernel(SoftmaxArgs a) {
   constexpr int VEC = VecIO<T>::N;
   using Lanes = RowLanes<LPR>;
   __shared__ float red[kMaxWaves];
-  const int tpr = Lanes::count(), t = Lanes::lane();
+  const int tpr = Lanes::count(a.threads), t = Lanes::lane();
   const int64_t row = Lanes::row();
   if (LPR && row >= a.n0) return;   // row counts within the innermost level
 
@@ -159,7 +171,7 @@ void softmax_bwd_kernel(SoftmaxArgs a) {
       else s.v[0] = fmaf(y[j], d[j], s.v[0]);   // padding is zero
     }
   }
-  s = Lanes::allreduce(s, red);
+  s = Lanes::allreduce(s, red, a.threads);
   const float dot = s.v[0];
   T* dxr = static_cast<T*>(a.out) + row * a.out_pitch + outer_level_offset(a.out_lv);
 #pragma unroll
@@ -263,7 +275,9 @@ struct SoftmaxDimArgs {
   void* out;
   int64_t inner, total;   // total: vectors of all planes, outer * run_vecs
   int dim, run_vecs, slices;
+  int blocks;             // of the launch
 };
+static_assert(sizeof(SoftmaxDimArgs) <= kCheapArgs, "");
 // What is formed from these vectors after this point is formed from them again, not kept in registers since before it.
 template <int N>
 __device__ __forceinline__ void form_again(u32x4 (&raw)[N]) {
@@ -277,7 +291,7 @@ struct DimColumn {
   int v, first, count;
   bool live;
   __device__ __forceinline__ DimColumn(const SoftmaxDimArgs& a, int nk) {
-    const int64_t id = xcd_run_block<LX == 256 ? 8 : 16>(blockIdx.x, gridDim.x) * LX + int(threadIdx.x);
+    const int64_t id = xcd_run_block<LX == 256 ? 8 : 16>(blockIdx.x, uint32_t(a.blocks)) * LX + int(threadIdx.x);
     live = id < a.total;
     const uint32_t i = uint32_t(live ? id : a.total - 1), o = i / uint32_t(a.run_vecs);
     v = int(i - o * uint32_t(a.run_vecs));
@@ -405,7 +419,7 @@ template <> __device__ __forceinline__ double exp_ct<double>(double v) { return 
 template <typename T, typename CT>
 __global__ __launch_bounds__(256)
 void softmax_fwd_strided_kernel(const T* x, T* y, int64_t outer, int64_t dim, int64_t inner) {
-  const int64_t pos = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  const int64_t pos = int64_t(blockIdx.x) * 256 + threadIdx.x;
   if (pos >= outer * inner) return;
   const int64_t o = pos / inner, in = pos - o * inner;
   const T* xp = x + o * dim * inner + in;
@@ -425,7 +439,7 @@ template <typename T, typename CT>
 __global__ __launch_bounds__(256)
 void softmax_bwd_strided_kernel(const T* y, const T* dy, T* dx, int64_t outer, int64_t dim,
                                 int64_t inner) {
-  const int64_t pos = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  const int64_t pos = int64_t(blockIdx.x) * 256 + threadIdx.x;
   if (pos >= outer * inner) return;
   const int64_t o = pos / inner, in = pos - o * inner;
   const int64_t base = o * dim * inner + in;
@@ -443,7 +457,7 @@ __device__ __forceinline__ CT block_reduce_generic(CT v, CT* lds, bool is_max) {
   const int tid = threadIdx.x;
   lds[tid] = v;
   __syncthreads();
-  for (int s = blockDim.x >> 1; s > 0; s >>= 1) {
+  for (int s = 256 >> 1; s > 0; s >>= 1) {
     if (tid < s) lds[tid] = is_max ? (lds[tid] > lds[tid + s] ? lds[tid] : lds[tid + s])
                                    : lds[tid] + lds[tid + s];
     __syncthreads();
@@ -460,16 +474,16 @@ void softmax_fwd_longrow_kernel(const T* x, T* y, int64_t cols, int64_t x_pitch,
   const T* xr = x + int64_t(blockIdx.x) * x_pitch;
   T* yr = y + int64_t(blockIdx.x) * y_pitch;
   CT m = -__builtin_huge_val();
-  for (int64_t c = threadIdx.x; c < cols; c += blockDim.x) {
+  for (int64_t c = threadIdx.x; c < cols; c += 256) {
     const CT v = SmIO<T, CT>::ld(xr + c);
     m = v > m ? v : m;
   }
   m = block_reduce_generic<CT>(m, lds, true);
   CT s = 0;
-  for (int64_t c = threadIdx.x; c < cols; c += blockDim.x) s += exp_ct<CT>(SmIO<T, CT>::ld(xr + c) - m);
+  for (int64_t c = threadIdx.x; c < cols; c += 256) s += exp_ct<CT>(SmIO<T, CT>::ld(xr + c) - m);
   s = block_reduce_generic<CT>(s, lds, false);
   const CT inv = CT(1) / s;
-  for (int64_t c = threadIdx.x; c < cols; c += blockDim.x)
+  for (int64_t c = threadIdx.x; c < cols; c += 256)
     SmIO<T, CT>::st(yr + c, exp_ct<CT>(SmIO<T, CT>::ld(xr + c) - m) * inv);
 }
 
@@ -482,10 +496,10 @@ void softmax_bwd_longrow_kernel(const T* y, const T* dy, T* dx, int64_t cols, in
   const T* dyr = dy + int64_t(blockIdx.x) * dy_pitch;
   T* dxr = dx + int64_t(blockIdx.x) * dx_pitch;
   CT dot = 0;
-  for (int64_t c = threadIdx.x; c < cols; c += blockDim.x)
+  for (int64_t c = threadIdx.x; c < cols; c += 256)
     dot += SmIO<T, CT>::ld(yr + c) * SmIO<T, CT>::ld(dyr + c);
   dot = block_reduce_generic<CT>(dot, lds, false);
-  for (int64_t c = threadIdx.x; c < cols; c += blockDim.x) {
+  for (int64_t c = threadIdx.x; c < cols; c += 256) {
     const CT yv = SmIO<T, CT>::ld(yr + c);
     SmIO<T, CT>::st(dxr + c, yv * (SmIO<T, CT>::ld(dyr + c) - dot));
   }
@@ -592,23 +606,52 @@ static int launch_softmax_nv(const SoftmaxArgs& a, int nv, dim3 grid, dim3 block
 }
 
 template <typename T, bool BWD, bool RAGGED>
-static int launch_softmax(const SoftmaxArgs& a, int threads, int nv, hipStream_t s) {
-  if (threads > 64) {
-    dim3 grid{unsigned(a.n0), unsigned(a.n1), unsigned(a.n2)}, block{unsigned(threads)};
-    return launch_softmax_nv<T, BWD, 0, RAGGED>(a, nv, grid, block, s);
+static int launch_softmax(const SoftmaxRows& r, int threads, int nv, hipStream_t s) {
+  constexpr int64_t kMost = 0x7fffffff;
+  const auto far = [&](int64_t n, int64_t x, int64_t dy, int64_t out) {
+    return n > 1 && (std::max(std::max(x, BWD ? dy : 0), out) > kMost || std::min(std::min(x, BWD ? dy : 0), out) < -kMost);
+  };
+  const bool far0 = far(r.n0, r.x_pitch, r.dy_pitch, r.out_pitch), far1 = far(r.n1, r.x_lv.p1, r.dy_lv.p1, r.out_lv.p1),
+             far2 = far(r.n2, r.x_lv.p2, r.dy_lv.p2, r.out_lv.p2);
+  if (far0 || far1 || far2) {   // a launch for each step of the levels whose rows lie that far apart
+    SoftmaxRows part = r;
+    if (far0) part.n0 = 1;
+    if (far1) part.n1 = 1;
+    if (far2) part.n2 = 1;
+    for (int64_t k = 0; k < (far2 ? r.n2 : 1); ++k) {
+      for (int64_t j = 0; j < (far1 ? r.n1 : 1); ++j) {
+        for (int64_t i = 0; i < (far0 ? r.n0 : 1); ++i) {
+          const auto at = [&](int64_t pitch, const LevelSteps& l) { return i * pitch + j * l.p1 + k * l.p2; };
+          part.x = static_cast<const T*>(r.x) + at(r.x_pitch, r.x_lv);
+          if constexpr (BWD) part.dy = static_cast<const T*>(r.dy) + at(r.dy_pitch, r.dy_lv);
+          part.out = static_cast<T*>(r.out) + at(r.out_pitch, r.out_lv);
+          const int rc = launch_softmax<T, BWD, RAGGED>(part, threads, nv, s);
+          if (rc != HK_OK) return rc;
+        }
+      }
+    }
+    return HK_OK;
   }
-  const int rows_per_block = 256 / threads;
-  dim3 grid(unsigned((a.n0 + rows_per_block - 1) / rows_per_block), unsigned(a.n1), unsigned(a.n2)), block(256);
+  const int rows_per_block = threads > 64 ? 1 : 256 / threads;
+  const dim3 grid(unsigned((r.n0 + rows_per_block - 1) / rows_per_block), unsigned(r.n1), unsigned(r.n2));
+  const dim3 block(threads > 64 ? unsigned(threads) : 256u);
+  SoftmaxArgs a{};   // (a step of a level of one row is not taken)
+  a.x = r.x; a.dy = r.dy; a.out = r.out; a.n0 = int(r.n0);
+  if (r.n0 > 1) { a.x_pitch = int(r.x_pitch); a.dy_pitch = int(BWD ? r.dy_pitch : 0); a.out_pitch = int(r.out_pitch); }
+  if (r.n1 > 1) { a.x_lv.p1 = int(r.x_lv.p1); a.dy_lv.p1 = int(BWD ? r.dy_lv.p1 : 0); a.out_lv.p1 = int(r.out_lv.p1); }
+  if (r.n2 > 1) { a.x_lv.p2 = int(r.x_lv.p2); a.dy_lv.p2 = int(BWD ? r.dy_lv.p2 : 0); a.out_lv.p2 = int(r.out_lv.p2); }
+  a.cols = r.cols; a.nvec = r.nvec; a.spare = r.spare; a.threads = int(block.x);
   switch (threads) {
     case 8: return launch_softmax_nv<T, BWD, 8, RAGGED>(a, nv, grid, block, s);
     case 16: return launch_softmax_nv<T, BWD, 16, RAGGED>(a, nv, grid, block, s);
     case 32: return launch_softmax_nv<T, BWD, 32, RAGGED>(a, nv, grid, block, s);
-    default: return launch_softmax_nv<T, BWD, 64, RAGGED>(a, nv, grid, block, s);
+    case 64: return launch_softmax_nv<T, BWD, 64, RAGGED>(a, nv, grid, block, s);
+    default: return launch_softmax_nv<T, BWD, 0, RAGGED>(a, nv, grid, block, s);
   }
 }
 
 template <typename T, bool BWD>
-static int softmax_lastdim_typed(SoftmaxArgs a, hipStream_t s) {
+static int softmax_lastdim_typed(SoftmaxRows a, hipStream_t s) {
   constexpr int VEC = VecIO<T>::N;
   auto steps_ok = [](int64_t pitch, const LevelSteps& l) { return pitch % VEC == 0 && l.p1 % VEC == 0 && l.p2 % VEC == 0; };
   const bool vec_ok = a.cols % VEC == 0 && aligned16(a.x) && aligned16(a.dy) && aligned16(a.out) &&
@@ -659,12 +702,13 @@ static int softmax_lastdim_typed(SoftmaxArgs a, hipStream_t s) {
 // FEW: up to kFewSlices slices.  MAXT: the most threads that its plans have.  LEAST, MOST:
 // the entries per lane that they give (of 16-bit types from 8 on even numbers).  LEAST_AGAIN: from how many on AGAIN; 14 backward just fit without
 template <typename T, bool BWD, int LX, bool PLAIN, bool FEW, int MAXT, int LEAST, int MOST, int LEAST_AGAIN = 17>
-static int launch_softmax_dim(const SoftmaxDimArgs& a, int nk, hipStream_t s) {
+static int launch_softmax_dim(SoftmaxDimArgs a, int nk, hipStream_t s) {
   if (nk < LEAST || nk > MOST || (nk > kDimVecs && nk % 2 != 0 && VecIO<T>::N == 8) || a.slices * LX > MAXT) {
     set_last_error("softmax: no kernel for %d entries per lane", nk);
     return HK_ERR_UNSUPPORTED;
   }
-  const dim3 grid{unsigned((a.total + LX - 1) / LX)}, block{unsigned(LX), unsigned(a.slices)};
+  a.blocks = int((a.total + LX - 1) / LX);
+  const dim3 grid{unsigned(a.blocks)}, block{unsigned(LX), unsigned(a.slices)};
   const size_t lds = a.slices > 1 ? share_floats<VecIO<T>::N, LX, FEW, BWD>(a.slices) * sizeof(float) : 0;
 #define HK_DIM_CASE(NK)                                                             \
   case NK:                                                                          \
@@ -856,7 +900,7 @@ static int softmax_dispatch(int dtype, const void* x, const void* dy, void* out,
   HK_REQUIRE(outer <= 0x7fffffffLL && (outer * inner + 255) / 256 <= 0x7fffffffLL, HK_ERR_INVALID,
              "%s: too many rows", who);
   if (inner == 1 && dim <= 0x3fffffff && dtype != HK_FLOAT64) {
-    SoftmaxArgs a{};
+    SoftmaxRows a{};
     a.x = x; a.dy = dy; a.out = out; a.rows = outer; a.cols = int(dim);
     a.x_pitch = x_pitch; a.dy_pitch = dy_pitch; a.out_pitch = out_pitch;
     a.n0 = outer; a.n1 = a.n2 = 1;

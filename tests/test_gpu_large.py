@@ -284,3 +284,49 @@ def test_batch_norm_past_2_31_elements_of_every_form(hk, cuda, N, C, HW):
                 helpers.assert_close(y[n, c, at], (xhat * float(scale[c]) + float(bias[c])).cpu().numpy(), "bf16", "y")
                 want = float(scale[c]) * inv * (dy[n, c, at].double() - mg - xhat * mgx)
                 helpers.assert_close(dx[n, c, at], want.cpu().numpy(), "bf16", "dx")
+
+
+@pytest.mark.parametrize("cols", [64, 61, 1000, 1021])
+def test_rows_2_31_elements_apart(hk, cuda, cols):
+    """Steps between rows that 32 bits do not hold, on one level and as one of three, against the same rows side by side."""
+    import torch
+    far = (1 << 31) + 8
+    block = 3 * 5 * 1024
+    base = torch.empty(far + block, dtype=torch.bfloat16, device=cuda)
+
+    def check(shape, strides):
+        def far_copy(t, off):
+            v = base.as_strided(shape, strides, off)
+            v.copy_(t)
+            return v
+        g = torch.Generator(device=cuda).manual_seed(cols)
+        x, dy = (torch.randn(shape, generator=g, device=cuda).to(torch.bfloat16) for _ in range(2))
+        y, dx = torch.empty_like(x), torch.empty_like(x)
+        hk.softmax_fwd(x, y, -1)
+        hk.softmax_bwd(y, dy, dx, -1)
+        fy, fdx = torch.empty_like(x), torch.empty_like(x)
+        hk.softmax_fwd(far_copy(x, 0), fy, -1)
+        assert torch.equal(fy, y), shape
+        hk.softmax_bwd(far_copy(y, 0), dy, fdx, -1)
+        assert torch.equal(fdx, dx), shape
+        fout = base.as_strided(shape, strides, 0)
+        hk.softmax_fwd(x, fout, -1)
+        assert torch.equal(fout, y), shape
+        rows = x.numel() // cols
+        w = torch.rand(cols, generator=g, device=cuda).to(torch.bfloat16)
+        mu, rs, z = torch.empty(rows, device=cuda), torch.empty(rows, device=cuda), torch.empty_like(x)
+        fmu, frs, fz = torch.empty(rows, device=cuda), torch.empty(rows, device=cuda), torch.empty_like(x)
+        hk.layer_norm_fwd(x, w, w, z, mu, rs, 1e-5)
+        hk.layer_norm_fwd(far_copy(x, 0), w, w, fz, fmu, frs, 1e-5)
+        helpers.assert_close(fz, helpers.to_numpy(z).astype(np.float64), "bf16", "z")
+        helpers.assert_close(frs, helpers.to_numpy(rs).astype(np.float64), "fp32", "rstd")
+        dg, db, fdg, fdb = (torch.empty_like(w) for _ in range(4))
+        hk.layer_norm_bwd(dy, x, w, w, mu, rs, dx, dg, db, 1e-5)
+        hk.layer_norm_bwd(far_copy(dy, 0), x, w, w, mu, rs, fdx, fdg, fdb, 1e-5)
+        for got, want, what in ((fdx, dx, "dx"), (fdg, dg, "dgamma"), (fdb, db, "dbeta")):
+            helpers.assert_close(got, helpers.to_numpy(want).astype(np.float64), "bf16", what)
+
+    check((2, cols), (far, 1))
+    if cols % 8 == 0:
+        check((3, 2, 5, cols), (5 * cols, far, cols, 1))
+        check((2, 5, 3, cols), (far, cols, 5 * cols, 1))
