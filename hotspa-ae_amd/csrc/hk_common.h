@@ -6,6 +6,7 @@
 // v_cvt_pk_bf16_f32 conversion are assumed.
 #pragma once
 
+#include <initializer_list>
 #include <hip/hip_runtime.h>
 #include <hip/hip_ext.h>
 #include <type_traits>
@@ -332,6 +333,26 @@ struct LevelSteps {
 struct ShortLevelSteps {   // the same below 2^31
   int p1, p2;
 };
+// whether some of the steps between the n rows of a level is none that 32 bits hold
+inline bool far_level(int64_t n, std::initializer_list<int64_t> steps) {
+  for (const int64_t p : steps)
+    if (n > 1 && (p > 0x7fffffffLL || p < -0x7fffffffLL)) return true;
+  return false;
+}
+// one(part, i, j, k) for every step of the far levels, with part's far levels cut to the one row: few, as so much memory lies
+// between them
+template <typename Rows, typename F>
+inline int each_near_part(const Rows& r, bool far0, bool far1, bool far2, F&& one) {
+  Rows part = r;
+  if (far0) part.n0 = 1;
+  if (far1) part.n1 = 1;
+  if (far2) part.n2 = 1;
+  int rc = 0;
+  for (int64_t k = 0; k < (far2 ? r.n2 : 1) && rc == 0; ++k)
+    for (int64_t j = 0; j < (far1 ? r.n1 : 1) && rc == 0; ++j)
+      for (int64_t i = 0; i < (far0 ? r.n0 : 1) && rc == 0; ++i) rc = one(part, i, j, k);
+  return rc;
+}
 struct RowNumbering {
   int64_t rn0, rn1, rn2;
 };

@@ -141,6 +141,10 @@ __device__ __forceinline__ int64_t subset_row(const int32_t* subset, int64_t row
 // ===========================================================================
 // forward
 // ===========================================================================
+// threads per row of nchunks chunks, nc to a thread
+__host__ __device__ __forceinline__ int dal_fwd_threads(int nchunks, int nc) {
+  return int((uint32_t(nchunks + nc - 1) / uint32_t(nc) + 63u) / 64u * 64u);
+}
 struct DalFwdArgs {
   const void* x0;
   const void* x1;
@@ -165,7 +169,44 @@ struct DalFwdArgs {
   float eps, inv_cols, scale, rowscale_const;
   int is_rms, dropout;
   DropArgs drop;
+  template <int NC> __device__ __forceinline__ DalFwdArgs args() const { return *this; }
 };
+// The same with one input and one affine pair, no scaling and no subsets (see kCheapArgs: 1528 x 1104 fp16, forward and backward,
+// 17.2 -> 16.3 us, the fold of the partial rows among it)
+struct DalFwdFlat {
+  const void* x0;
+  const void* residual;
+  const void* gamma;
+  const void* beta;
+  void* z;
+  void* x;
+  uint8_t* dmask;
+  float* mu;
+  float* rs;
+  uint32_t rows, cols;   // the highest bits: is_rms, dropout
+  float eps, inv_cols, scale;
+  DropArgs drop;
+  static bool holds(const DalFwdArgs& a) {
+    return !a.x1 && !a.gamma1 && !a.beta1 && !a.rowscale && !a.colscale && !a.x0_subset && !a.z_subset && !a.z1 && !a.dmask1;
+  }
+  explicit DalFwdFlat(const DalFwdArgs& a)
+      : x0(a.x0), residual(a.residual), gamma(a.gamma), beta(a.beta), z(a.z), x(a.x), dmask(a.dmask), mu(a.mu), rs(a.rs),
+        rows(uint32_t(a.rows) | (a.is_rms ? 0x80000000u : 0u)), cols(uint32_t(a.cols) | (a.dropout ? 0x80000000u : 0u)),
+        eps(a.eps), inv_cols(a.inv_cols), scale(a.scale), drop(a.drop) {}
+  template <int NC>
+  __device__ __forceinline__ DalFwdArgs args() const {
+    DalFwdArgs a{};
+    a.x0 = x0; a.residual = residual; a.gamma = gamma; a.beta = beta; a.z = z; a.x = x; a.dmask = dmask; a.mu = mu; a.rs = rs;
+    a.rows = a.x0_numrows = a.z_numrows = rows & 0x7fffffffu;
+    a.cols = int(cols & 0x7fffffffu);
+    a.nchunks = int(uint32_t(a.cols) / uint32_t(kChunk));
+    a.tpr = dal_fwd_threads(a.nchunks, NC);
+    a.eps = eps; a.inv_cols = inv_cols; a.scale = scale; a.is_rms = int(rows >> 31); a.dropout = int(cols >> 31);
+    a.drop = drop;
+    return a;
+  }
+};
+static_assert(sizeof(DalFwdFlat) <= kCheapArgs, "");
 
 // IT / RT / WT: input, residual and weight element types; NC: chunks per thread.  A block holds
 // blockDim.x / tpr row groups; every group takes part in the (block-wide) reduction barrier, a group
@@ -174,14 +215,16 @@ struct DalFwdArgs {
 // scalar registers instead of 103; 40000 x 256 bf16 with an fp32 weight 30.7 -> 25.4 us, with an fp32 residual 33.4 -> 30.2).
 // Asked for 8 of them with the masks, the compiler spills scalars: 1190 x 1104 bf16 7.5 against 6.8 us, 16384 x 1024 37.1
 // against 35.0, and only 6578 x 512 with an fp32 residual 12.2 against 12.6.
-template <typename IT, typename RT, typename WT, int NC, bool DROP>
+// A: DalFwdArgs, or DalFwdFlat where that holds the arguments.
+template <typename IT, typename RT, typename WT, int NC, bool DROP, typename A>
 __global__ __launch_bounds__(256)
-void dal_fwd_kernel(DalFwdArgs a) {
+void dal_fwd_kernel(A given) {
+  const DalFwdArgs a = given.template args<NC>();
   __shared__ float red[kMaxWaves * 3];
   const int tpr = a.tpr;
   const int group = __builtin_amdgcn_readfirstlane(int(threadIdx.x) / tpr);
   const int t = int(threadIdx.x) - group * tpr;
-  const int rpb = int(blockDim.x) / tpr;
+  const int rpb = max(1, 256 / tpr);
   const int wpg = tpr >> 6;
   const int64_t row_raw = int64_t(blockIdx.x) * rpb + group;
   const bool row_ok = row_raw < a.rows;
@@ -397,6 +440,25 @@ struct DalBwdArgs {
   int is_rms, dropout;
 };
 
+// What dal_bwd_stream_kernel takes of it (see kCheapArgs)
+struct DalStreamArgs {
+  const void* dz;
+  const void* dx;
+  const void* x;
+  const uint8_t* dmask;
+  const float* mu;
+  const float* rs;
+  const void* gamma;
+  void* dx0;
+  void* dresidual;
+  float* part[2];
+  uint32_t rows_rms, cols;   // the highest bit of the rows: is_rms
+  float inv_cols, scale;
+  uint16_t tpr, threads;
+  uint32_t blocks;
+};
+static_assert(sizeof(DalStreamArgs) <= kCheapArgs, "");
+
 // A thread's column sums acc -> the partial row of its block.  The block's row groups are folded through LDS first: one
 // partial row per group took the fold kernel longer than the backward itself (16384 x 768 bf16 73 us, 30 us now,
 // with the rows that do not fill their threads on the streaming kernel; 8192 x 4104 110 -> 70 us).
@@ -585,18 +647,21 @@ void dal_bwd_kernel(DalBwdArgs a) {
 // (512 threads = 4096 columns), else 0: the launch bound and the cross-wavefront step of the row sums follow it.
 template <typename IT, typename RT, typename WT, int PF, int TPR>
 __global__ __launch_bounds__(TPR ? TPR : 1024)
-void dal_bwd_stream_kernel(DalBwdArgs a) {
+void dal_bwd_stream_kernel(DalStreamArgs a) {
+  const int64_t rows = a.rows_rms & 0x7fffffffu;
+  const bool is_rms = a.rows_rms >> 31 != 0;
+  const int cols = int(a.cols), nchunks = int(a.cols / uint32_t(kChunk));
   constexpr int NI = kChunk / VecIO<IT>::N;   // 16-byte vectors per chunk of the input type
   constexpr int NR = kChunk / VecIO<RT>::N;   //                       ... of the residual type
   __shared__ __align__(16) float red[2][kMaxWaves * 2];
   const int tpr = TPR ? TPR : a.tpr;
   const int group = TPR ? 0 : __builtin_amdgcn_readfirstlane(int(threadIdx.x) / tpr);
   const int t = int(threadIdx.x) - group * tpr;
-  const int rpb = TPR ? 1 : int(blockDim.x) / tpr;
+  const int rpb = TPR ? 1 : a.threads / tpr;
   const int wpg = tpr >> 6;
   const int first_wave = group * wpg;
-  const bool in = TPR || t < a.nchunks;
-  const int col = (in ? t : a.nchunks - 1) * kChunk;
+  const bool in = TPR || t < nchunks;
+  const int col = (in ? t : nchunks - 1) * kChunk;
   extern __shared__ __align__(16) float stage[];
 
   float g0[kChunk];
@@ -605,15 +670,15 @@ void dal_bwd_stream_kernel(DalBwdArgs a) {
 #pragma unroll
   for (int j = 0; j < kChunk; ++j) { dg0[j] = 0.f; db0[j] = 0.f; }
 
-  const int64_t stride = int64_t(gridDim.x) * rpb;
-  const int64_t last_row = a.rows - 1;
+  const int64_t stride = int64_t(a.blocks) * rpb;
+  const int64_t last_row = rows - 1;
   u32x4 ndz[PF][NI], nx[PF][NR], ndx[PF][NR];
   u32x2 nm[PF];
   float nmu[PF], nrs[PF];
   auto issue = [&](auto slot, int64_t r) {
     constexpr int d = decltype(slot)::value;
     const int64_t rc = r < last_row ? r : last_row;
-    const int64_t e = rc * int64_t(a.cols) + col;
+    const int64_t e = rc * int64_t(cols) + col;
     nmu[d] = a.mu[rc];
     nrs[d] = a.rs[rc];
 #pragma unroll
@@ -633,7 +698,7 @@ void dal_bwd_stream_kernel(DalBwdArgs a) {
     constexpr int d = decltype(slot)::value;
     constexpr bool GUARD = decltype(guarded)::value;
     const int64_t row = row0 + d * stride;
-    const bool valid = !GUARD || row < a.rows;
+    const bool valid = !GUARD || row < rows;
     float dz[kChunk], y[kChunk], u[kChunk];
 #pragma unroll
     for (int i = 0; i < NI; ++i) VecIO<IT>::unpack(ndz[d][i], &dz[i * VecIO<IT>::N]);
@@ -643,7 +708,7 @@ void dal_bwd_stream_kernel(DalBwdArgs a) {
       VecIO<RT>::unpack(ndx[d][i], &u[i * VecIO<RT>::N]);
     }
     const u32x2 mw = nm[d];
-    const float mu = a.is_rms ? 0.f : nmu[d];
+    const float mu = is_rms ? 0.f : nmu[d];
     const float rs = nrs[d];
     issue(slot, row + int64_t(PF) * stride);   // the slot is free again
 
@@ -664,7 +729,7 @@ void dal_bwd_stream_kernel(DalBwdArgs a) {
     else s = group_allreduce_tuple(s, red[parity], first_wave, wpg);
     parity ^= 1;
     if (valid && in) {
-      const float mdy = a.is_rms ? 0.f : s.v[0] * a.inv_cols;
+      const float mdy = is_rms ? 0.f : s.v[0] * a.inv_cols;
       const float mdyy = s.v[1] * a.inv_cols;
       float o[kChunk];
 #pragma unroll
@@ -673,7 +738,7 @@ void dal_bwd_stream_kernel(DalBwdArgs a) {
         const uint32_t byte = ((j < 4 ? mw.x : mw.y) >> (8 * (j & 3))) & 0xffu;
         o[j] = byte ? u[j] * a.scale : 0.f;
       }
-      const int64_t e = row * int64_t(a.cols) + col;
+      const int64_t e = row * int64_t(cols) + col;
       store8<RT, false>(static_cast<RT*>(a.dresidual) + e, u);
       store8<IT, true>(static_cast<IT*>(a.dx0) + e, o);
     }
@@ -683,18 +748,18 @@ void dal_bwd_stream_kernel(DalBwdArgs a) {
   // rounds in which every slot of every group of this block holds an existing row, then the guarded tail;
   // both bounds are block-uniform, so every thread reaches the barrier of every step
 #pragma nounroll
-  for (; base + int64_t(PF - 1) * stride + rpb <= a.rows; base += round) {
+  for (; base + int64_t(PF - 1) * stride + rpb <= rows; base += round) {
     static_for<PF>([&](auto slot) { step(slot, std::false_type{}); });
     row0 += round;
   }
 #pragma nounroll
-  for (; base < a.rows; base += round) {
+  for (; base < rows; base += round) {
     static_for<PF>([&](auto slot) { step(slot, std::true_type{}); });
     row0 += round;
   }
 
-  put_column_sums(a.part[0], dg0, stage, group, rpb, in, a.cols, col);
-  put_column_sums(a.part[1], db0, stage, group, rpb, in, a.cols, col);
+  put_column_sums(a.part[0], dg0, stage, group, rpb, in, cols, col);
+  put_column_sums(a.part[1], db0, stage, group, rpb, in, cols, col);
 }
 
 // Folds [nparts, cols] fp32 partial rows into a [cols] vector of WT (fold_partial_rows); blockIdx.y picks which of the (up to
@@ -845,7 +910,7 @@ int hk_dropout_add_ln_fwd_ex(const hkDropoutAddLnFwdParams* pp, hkStream_t strea
 
   // chunks per thread: the fewest that keep a row within 256 threads
   const int nc = a.nchunks <= 256 ? 1 : (a.nchunks <= 512 ? 2 : 4);
-  a.tpr = ((a.nchunks + nc - 1) / nc + 63) / 64 * 64;
+  a.tpr = dal_fwd_threads(a.nchunks, nc);
   const int rpb = std::max(1, 256 / a.tpr);
   const dim3 block{unsigned(a.tpr * rpb)}, grid{unsigned((p.rows + rpb - 1) / rpb)};
   hipStream_t s = as_hip(stream);
@@ -853,15 +918,20 @@ int hk_dropout_add_ln_fwd_ex(const hkDropoutAddLnFwdParams* pp, hkStream_t strea
     using IT = typename decltype(it)::type;
     using RT = typename decltype(rt)::type;
     using WT = typename decltype(wt)::type;
+    auto launch = [&](const auto& given) {
+      using A = typename std::decay<decltype(given)>::type;
+      switch (nc) {
+        case 1:
+          if (dropout) HK_LAUNCH((dal_fwd_kernel<IT, RT, WT, 1, true, A>), grid, block, 0, s, given);
+          else HK_LAUNCH((dal_fwd_kernel<IT, RT, WT, 1, false, A>), grid, block, 0, s, given);
+          break;
+        case 2: HK_LAUNCH((dal_fwd_kernel<IT, RT, WT, 2, true, A>), grid, block, 0, s, given); break;
+        default: HK_LAUNCH((dal_fwd_kernel<IT, RT, WT, 4, true, A>), grid, block, 0, s, given); break;
+      }
+    };
     profile_before(s);
-    switch (nc) {
-      case 1:
-        if (dropout) HK_LAUNCH((dal_fwd_kernel<IT, RT, WT, 1, true>), grid, block, 0, s, a);
-        else HK_LAUNCH((dal_fwd_kernel<IT, RT, WT, 1, false>), grid, block, 0, s, a);
-        break;
-      case 2: HK_LAUNCH((dal_fwd_kernel<IT, RT, WT, 2, true>), grid, block, 0, s, a); break;
-      default: HK_LAUNCH((dal_fwd_kernel<IT, RT, WT, 4, true>), grid, block, 0, s, a); break;
-    }
+    if (DalFwdFlat::holds(a)) launch(DalFwdFlat(a));
+    else launch(a);
     profile_after(s);
     return launch_check("dal_fwd_kernel");
   });
@@ -975,11 +1045,11 @@ int hk_dropout_add_ln_bwd_ex(const hkDropoutAddLnBwdParams* pp, hkStream_t strea
   a.inv_cols = 1.0f / float(p.cols); a.scale = 1.0f / (1.0f - p.dropout_p); a.rowscale_const = p.rowscale_const;
   a.is_rms = p.is_rms_norm ? 1 : 0; a.dropout = dropout ? 1 : 0;
 
-  DalFoldArgs f{};
+  DalFoldArgs fold{};
   int wanted = 0;
   for (int k = 0; k < kMaxParts; ++k)
-    if (outs[k]) { f.part[wanted] = a.part[k]; f.out[wanted++] = outs[k]; }
-  f.nparts = int(sh.nparts); f.cols = int(p.cols);
+    if (outs[k]) { fold.part[wanted] = a.part[k]; fold.out[wanted++] = outs[k]; }
+  fold.nparts = int(sh.nparts); fold.cols = int(p.cols);
 
   const dim3 grid{unsigned(sh.grid)}, block{unsigned(sh.block)};
   return dispatch_types(p.wtype, p.itype, p.rtype, who, [&](auto it, auto rt, auto wt) {
@@ -991,8 +1061,11 @@ int hk_dropout_add_ln_bwd_ex(const hkDropoutAddLnBwdParams* pp, hkStream_t strea
     constexpr int PF = sizeof(RT) == 2 ? 2 : 1;
     const bool full = int(p.cols) / kChunk == sh.tpr;
     const size_t lds = sh.rpb > 1 ? size_t(sh.rpb) * size_t(p.cols) * sizeof(float) : 0;
-    if (stream_form && full && sh.tpr == 512 && sh.block == 512) HK_LAUNCH((dal_bwd_stream_kernel<IT, RT, WT, PF, 512>), grid, block, lds, s, a);
-    else if (stream_form) HK_LAUNCH((dal_bwd_stream_kernel<IT, RT, WT, PF, 0>), grid, block, lds, s, a);
+    const DalStreamArgs f{a.dz, a.dx, a.x, a.dmask, a.mu, a.rs, a.gamma, a.dx0, a.dresidual, {a.part[0], a.part[1]},
+                          uint32_t(a.rows) | (a.is_rms ? 0x80000000u : 0u), uint32_t(a.cols), a.inv_cols, a.scale,
+                          uint16_t(a.tpr), uint16_t(sh.block), uint32_t(sh.grid)};
+    if (stream_form && full && sh.tpr == 512 && sh.block == 512) HK_LAUNCH((dal_bwd_stream_kernel<IT, RT, WT, PF, 512>), grid, block, lds, s, f);
+    else if (stream_form) HK_LAUNCH((dal_bwd_stream_kernel<IT, RT, WT, PF, 0>), grid, block, lds, s, f);
     else if (g1) HK_LAUNCH((dal_bwd_kernel<IT, RT, WT, false, true>), grid, block, lds, s, a);
     else if (colscale) HK_LAUNCH((dal_bwd_kernel<IT, RT, WT, true, false>), grid, block, lds, s, a);
     else HK_LAUNCH((dal_bwd_kernel<IT, RT, WT, false, false>), grid, block, lds, s, a);
@@ -1000,7 +1073,7 @@ int hk_dropout_add_ln_bwd_ex(const hkDropoutAddLnBwdParams* pp, hkStream_t strea
     int r = launch_check("dal_bwd_kernel");
     if (r != HK_OK || wanted == 0) return r;
     HK_LAUNCH((dal_fold_kernel<WT>), dim3(unsigned((p.cols + kFoldCols - 1) / kFoldCols), unsigned(wanted)),
-              dim3(kFoldThreads), 0, s, f);
+              dim3(kFoldThreads), 0, s, fold);
     return launch_check("dal_fold_kernel");
   });
 }

@@ -28,8 +28,7 @@ struct SoftmaxRows {
   int nvec;
   int spare;        // see RaggedRow
 };
-// What the kernels take of it (see kCheapArgs).  Steps below 2^31 elements; what lies further apart goes out in several launches
-// (launch_softmax), of which there are few, as so much memory lies between them.
+// What the kernels take of it (see kCheapArgs).  Steps below 2^31 elements; what lies further apart goes out in several launches.
 struct SoftmaxArgs {
   const void* x;
   const void* dy;
@@ -607,39 +606,26 @@ static int launch_softmax_nv(const SoftmaxArgs& a, int nv, dim3 grid, dim3 block
 
 template <typename T, bool BWD, bool RAGGED>
 static int launch_softmax(const SoftmaxRows& r, int threads, int nv, hipStream_t s) {
-  constexpr int64_t kMost = 0x7fffffff;
-  const auto far = [&](int64_t n, int64_t x, int64_t dy, int64_t out) {
-    return n > 1 && (std::max(std::max(x, BWD ? dy : 0), out) > kMost || std::min(std::min(x, BWD ? dy : 0), out) < -kMost);
-  };
-  const bool far0 = far(r.n0, r.x_pitch, r.dy_pitch, r.out_pitch), far1 = far(r.n1, r.x_lv.p1, r.dy_lv.p1, r.out_lv.p1),
-             far2 = far(r.n2, r.x_lv.p2, r.dy_lv.p2, r.out_lv.p2);
-  if (far0 || far1 || far2) {   // a launch for each step of the levels whose rows lie that far apart
-    SoftmaxRows part = r;
-    if (far0) part.n0 = 1;
-    if (far1) part.n1 = 1;
-    if (far2) part.n2 = 1;
-    for (int64_t k = 0; k < (far2 ? r.n2 : 1); ++k) {
-      for (int64_t j = 0; j < (far1 ? r.n1 : 1); ++j) {
-        for (int64_t i = 0; i < (far0 ? r.n0 : 1); ++i) {
-          const auto at = [&](int64_t pitch, const LevelSteps& l) { return i * pitch + j * l.p1 + k * l.p2; };
-          part.x = static_cast<const T*>(r.x) + at(r.x_pitch, r.x_lv);
-          if constexpr (BWD) part.dy = static_cast<const T*>(r.dy) + at(r.dy_pitch, r.dy_lv);
-          part.out = static_cast<T*>(r.out) + at(r.out_pitch, r.out_lv);
-          const int rc = launch_softmax<T, BWD, RAGGED>(part, threads, nv, s);
-          if (rc != HK_OK) return rc;
-        }
-      }
-    }
-    return HK_OK;
+  const int64_t dy0 = BWD ? r.dy_pitch : 0, dy1 = BWD ? r.dy_lv.p1 : 0, dy2 = BWD ? r.dy_lv.p2 : 0;
+  const bool far0 = far_level(r.n0, {r.x_pitch, dy0, r.out_pitch}), far1 = far_level(r.n1, {r.x_lv.p1, dy1, r.out_lv.p1}),
+             far2 = far_level(r.n2, {r.x_lv.p2, dy2, r.out_lv.p2});
+  if (far0 || far1 || far2) {
+    return each_near_part(r, far0, far1, far2, [&](SoftmaxRows part, int64_t i, int64_t j, int64_t k) {
+      const auto at = [&](int64_t pitch, const LevelSteps& l) { return i * pitch + j * l.p1 + k * l.p2; };
+      part.x = static_cast<const T*>(r.x) + at(r.x_pitch, r.x_lv);
+      if constexpr (BWD) part.dy = static_cast<const T*>(r.dy) + at(r.dy_pitch, r.dy_lv);
+      part.out = static_cast<T*>(r.out) + at(r.out_pitch, r.out_lv);
+      return launch_softmax<T, BWD, RAGGED>(part, threads, nv, s);
+    });
   }
   const int rows_per_block = threads > 64 ? 1 : 256 / threads;
   const dim3 grid(unsigned((r.n0 + rows_per_block - 1) / rows_per_block), unsigned(r.n1), unsigned(r.n2));
   const dim3 block(threads > 64 ? unsigned(threads) : 256u);
   SoftmaxArgs a{};   // (a step of a level of one row is not taken)
   a.x = r.x; a.dy = r.dy; a.out = r.out; a.n0 = int(r.n0);
-  if (r.n0 > 1) { a.x_pitch = int(r.x_pitch); a.dy_pitch = int(BWD ? r.dy_pitch : 0); a.out_pitch = int(r.out_pitch); }
-  if (r.n1 > 1) { a.x_lv.p1 = int(r.x_lv.p1); a.dy_lv.p1 = int(BWD ? r.dy_lv.p1 : 0); a.out_lv.p1 = int(r.out_lv.p1); }
-  if (r.n2 > 1) { a.x_lv.p2 = int(r.x_lv.p2); a.dy_lv.p2 = int(BWD ? r.dy_lv.p2 : 0); a.out_lv.p2 = int(r.out_lv.p2); }
+  if (r.n0 > 1) { a.x_pitch = int(r.x_pitch); a.dy_pitch = int(dy0); a.out_pitch = int(r.out_pitch); }
+  if (r.n1 > 1) { a.x_lv.p1 = int(r.x_lv.p1); a.dy_lv.p1 = int(dy1); a.out_lv.p1 = int(r.out_lv.p1); }
+  if (r.n2 > 1) { a.x_lv.p2 = int(r.x_lv.p2); a.dy_lv.p2 = int(dy2); a.out_lv.p2 = int(r.out_lv.p2); }
   a.cols = r.cols; a.nvec = r.nvec; a.spare = r.spare; a.threads = int(block.x);
   switch (threads) {
     case 8: return launch_softmax_nv<T, BWD, 8, RAGGED>(a, nv, grid, block, s);

@@ -330,3 +330,25 @@ def test_rows_2_31_elements_apart(hk, cuda, cols):
     if cols % 8 == 0:
         check((3, 2, 5, cols), (5 * cols, far, cols, 1))
         check((2, 5, 3, cols), (far, cols, 5 * cols, 1))
+
+
+def test_cross_entropy_rows_2_31_elements_apart(hk, cuda):
+    """As above: per token losses, their gradient from gradients of their own, labels by row number."""
+    import torch
+    cols, far = 200, (1 << 31) + 8
+    base = torch.empty(far + 3 * 5 * cols, dtype=torch.bfloat16, device=cuda)
+    for shape, strides in (((2, cols), (far, 1)), ((3, 2, 5, cols), (5 * cols, far, cols, 1)), ((2, 5, 3, cols), (far, cols, 5 * cols, 1))):
+        g = torch.Generator(device=cuda).manual_seed(7)
+        x = torch.randn(shape, generator=g, device=cuda).to(torch.bfloat16)
+        labels = torch.randint(0, cols, shape[:-1], generator=g, device=cuda)
+        labels.view(-1)[1] = -100
+        dloss = torch.rand(shape[:-1], generator=g, device=cuda).to(torch.bfloat16)
+        loss, floss = torch.empty_like(dloss), torch.empty_like(dloss)
+        dx, fdx = torch.empty_like(x), torch.empty_like(x)
+        hk.sce_sparse_fwd(x, labels, loss, -100)
+        hk.sce_sparse_bwd(x, labels, dloss, dx, -100)
+        fx = base.as_strided(shape, strides, 0)
+        fx.copy_(x)
+        hk.sce_sparse_fwd(fx, labels, floss, -100)
+        hk.sce_sparse_bwd(fx, labels, dloss, fdx, -100)
+        assert torch.equal(floss, loss) and torch.equal(fdx, dx), shape
