@@ -402,10 +402,18 @@ __device__ __forceinline__ float dpp_perm(float v) {
   return u2f(uint32_t(__builtin_amdgcn_update_dpp(0, int(f2u(v)), CTRL, 0xf, 0xf, true)));
 }
 
+template <int CTRL>
+__device__ __forceinline__ double dpp_perm_f64(double v) {
+  const uint64_t bits = uint64_t(__double_as_longlong(v));
+  const uint32_t lo = f2u(dpp_perm<CTRL>(u2f(uint32_t(bits)))), hi = f2u(dpp_perm<CTRL>(u2f(uint32_t(bits >> 32))));
+  return __longlong_as_double(int64_t(uint64_t(hi) << 32 | lo));
+}
+
 constexpr int kDppXor1 = 0xB1;        // quad_perm:[1,0,3,2]
 constexpr int kDppXor2 = 0x4E;        // quad_perm:[2,3,0,1]
 constexpr int kDppHalfMirror = 0x141; // row_half_mirror
 constexpr int kDppMirror = 0x140;     // row_mirror
+constexpr int kDppRor4 = 0x124;       // row_ror:4
 constexpr int kDppRor8 = 0x128;       // row_ror:8
 constexpr int kDppBcast15 = 0x142;    // row_bcast:15
 constexpr int kDppBcast31 = 0x143;    // row_bcast:31
@@ -732,9 +740,7 @@ __device__ __forceinline__ float fold_partial_rows(const float* part, int nparts
   }
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
-    const uint64_t bits = uint64_t(__double_as_longlong(acc[k]));
-    const uint32_t lo = f2u(dpp_perm<kDppRor8>(u2f(uint32_t(bits)))), hi = f2u(dpp_perm<kDppRor8>(u2f(uint32_t(bits >> 32))));
-    acc[k] += __longlong_as_double(int64_t(uint64_t(hi) << 32 | lo));
+    acc[k] += dpp_perm_f64<kDppRor8>(acc[k]);
     if ((slice & 1) == 0) lds[slice >> 1][cg * 4 + k] = acc[k];
   }
   __syncthreads();

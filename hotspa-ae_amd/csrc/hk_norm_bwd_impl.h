@@ -418,6 +418,160 @@ void norm_bwd_finalize_kernel(const float* part0, const float* part1, T* out0, T
   else if (oc >= tail + shift) Cvt<T>::store(out + oc - shift, s);
 }
 
+constexpr int small_lanes(bool ragged) { return ragged ? 4 : 8; }
+// The whole backward of a small array in one launch.  Its time is that of launches and trips to memory, of which the kernels above
+// take three (rows, partial rows, their fold), so here the first a.blocks workgroups form the column sums from the operands
+// themselves, LANES vectors of every row each, and the others dx: what is read twice comes from a cache.  dx must not lie over dy
+// or x.  A workgroup of column sums has a slice of rows for every LANES threads, up to four rows of each under way at once; the
+// slices meet in LDS, in 64 bits.  dx comes out to the same bits as from norm_bwd_kernel: the plan's threads and vectors, its
+// order of operations.
+template <typename T, int NV, int MODE, bool RAGGED>
+__global__ __launch_bounds__(kSmallThreads)
+void norm_bwd_small_kernel(NormBwdFlat given) {
+  constexpr int LANES = small_lanes(RAGGED);
+  const NormBwdArgs a = given.template args<T, MODE>();
+  constexpr int VEC = VecIO<T>::N, SLICES = kSmallThreads / LANES, COLS = LANES * VEC;
+  constexpr int SUMS = MODE == BWD_RMS ? 1 : 2;
+  __shared__ __align__(16) float fold[SUMS][kSmallThreads / 16][COLS + 8];
+  __shared__ __align__(16) float red[kMaxWaves * SUMS];
+  auto ld_row = [](const T* p) { if constexpr (RAGGED) return ld16_any_keep<T>(p); else return ld16_keep(p); };
+  auto rs_of = [&](float sv) { return (MODE != BWD_RMS && a.stat_kind == HK_STAT_VAR) ? 1.0f / sqrtf(sv + a.eps) : sv; };
+  const float* meanp = static_cast<const float*>(a.mean);
+  const float* statp = static_cast<const float*>(a.stat);
+  const T* xp = static_cast<const T*>(a.x);
+  const T* dyp = static_cast<const T*>(a.dy);
+  const int rows = int(a.rows);
+  if (int(blockIdx.x) < a.blocks) {
+    const int lane = int(threadIdx.x) & (LANES - 1), slice = int(threadIdx.x) / LANES;
+    const int col = vec_column<T, RAGGED>(min(int(blockIdx.x) * LANES + lane, a.nvec - 1), a.cols);
+    float dg[VEC], db[VEC];
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) dg[j] = db[j] = 0.f;
+    auto round = [&](int base, auto count) {
+      constexpr int U = decltype(count)::value;
+      u32x4 rx[U], rdy[U];
+      float mu[U], sv[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {   // a row past the end reads the last one
+        const int64_t r = min(base + u * SLICES + slice, rows - 1);
+        rx[u] = ld_row(xp + r * a.x_pitch + col);
+        rdy[u] = ld_row(dyp + r * a.dy_pitch + col);
+        mu[u] = MODE == BWD_LN ? meanp[r] : 0.f;
+        sv[u] = statp[r];
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const bool in = base + u * SLICES + slice < rows;
+        const float rs = rs_of(sv[u]);
+        float x[VEC], d[VEC];
+        VecIO<T>::unpack(rx[u], x);
+        VecIO<T>::unpack(rdy[u], d);
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) {
+          const float more = fmaf(d[j] * rs, MODE == BWD_LN ? x[j] - mu[u] : x[j], dg[j]);
+          dg[j] = in ? more : dg[j];
+          if constexpr (SUMS == 2) db[j] += in ? d[j] : 0.f;
+        }
+      }
+    };
+    int base = 0;
+    for (; rows - base > 2 * SLICES; base += 4 * SLICES) round(base, std::integral_constant<int, 4>{});
+    if (rows - base > SLICES) round(base, std::integral_constant<int, 2>{});
+    else if (rows > base) round(base, std::integral_constant<int, 1>{});
+#pragma unroll
+    for (int k = 0; k < SUMS; ++k) {
+      float* acc = k == 0 ? dg : db;
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) {
+        acc[j] += dpp_perm<kDppRor8>(acc[j]);
+        if constexpr (LANES == 4) acc[j] += dpp_perm<kDppRor4>(acc[j]);
+      }
+      if ((int(threadIdx.x) & 15) < LANES) {
+#pragma unroll
+        for (int j = 0; j < VEC; j += 4)
+          st16(&fold[k][threadIdx.x >> 4][lane * VEC + j], u32x4{f2u(acc[j]), f2u(acc[j + 1]), f2u(acc[j + 2]), f2u(acc[j + 3])});
+      }
+    }
+    __syncthreads();
+    const int sub = int(threadIdx.x) & 7, o = int(threadIdx.x) >> 3, k = o / COLS, c = o % COLS;
+    if (k < SUMS) {   // whole wavefronts
+      double s = 0.;
+#pragma unroll
+      for (int i = 0; i < kSmallThreads / 128; ++i) s += fold[k][sub + 8 * i][c];
+      s += dpp_perm_f64<kDppXor1>(s);
+      s += dpp_perm_f64<kDppXor2>(s);
+      s += dpp_perm_f64<kDppHalfMirror>(s);
+      T* out = reinterpret_cast<T*>(k == 0 ? a.part_dgamma : a.part_dbeta);
+      const int v = int(blockIdx.x) * LANES + c / VEC;
+      const int at = vec_column<T, RAGGED>(v, a.cols) + c % VEC;   // a column that two vectors hold: from the first
+      if (sub == 0 && v < a.nvec && out != nullptr && at >= v * VEC) Cvt<T>::store(out + at, float(s));
+    }
+    return;
+  }
+
+  const int tpr = a.tpr, rpb = kSmallThreads / tpr;
+  const int group = __builtin_amdgcn_readfirstlane(int(threadIdx.x) / tpr), t = int(threadIdx.x) - group * tpr;
+  // (the wavefronts that no row is left for work on the last one too and store nothing)
+  const bool idle = group >= rpb;
+  const int64_t wanted = idle ? rows : int64_t(int(blockIdx.x) - a.blocks) * rpb + group, row = wanted < rows ? wanted : rows - 1;
+  const T* xr = xp + row * a.x_pitch;
+  const T* dyr = dyp + row * a.dy_pitch;
+  const T* gp = static_cast<const T*>(a.gamma);
+  u32x4 rx[NV], rdy[NV], rg[NV];
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int c = vec_column<T, RAGGED>(min(i * tpr + t, a.nvec - 1), a.cols);
+    rx[i] = ld_row(xr + c);
+    rdy[i] = ld_row(dyr + c);
+    if (gp) rg[i] = ld_row(gp + c);   // uniform
+  }
+  const float mu = MODE == BWD_LN ? meanp[row] : 0.f, rs = rs_of(statp[row]);
+  float xs[NV][VEC], ts[NV][VEC];
+  SumTuple<SUMS> s = SumTuple<SUMS>::identity();
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    float g[VEC];
+    VecIO<T>::unpack(rx[i], xs[i]);
+    VecIO<T>::unpack(rdy[i], ts[i]);
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) g[j] = 1.f;
+    if (gp) VecIO<T>::unpack(rg[i], g);
+    const int v = i * tpr + t;
+    if constexpr (!RAGGED) {
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) ts[i][j] = v < a.nvec ? ts[i][j] : 0.f;
+    }
+    auto in_sums = [&](float f, int j) {   // as in norm_bwd_kernel
+      if (RAGGED && i == NV - 1) return u2f(f2u(f) & ((v + 1) * VEC - a.cols > j ? 0u : 0xffffffffu));
+      return f;
+    };
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) {
+      const float xc = MODE == BWD_RMS ? xs[i][j] : xs[i][j] - mu;
+      const float dzr = ts[i][j] * rs;
+      const float q = dzr * g[j];
+      s.v[SUMS - 1] = fmaf(in_sums(q, j), in_sums(xc, j), s.v[SUMS - 1]);
+      if constexpr (MODE != BWD_RMS) s.v[0] += in_sums(q, j);
+      xs[i][j] = xc;
+      ts[i][j] = MODE == BWD_LN && a.clamp_gamma ? dzr * clamp_by_magnitude(g[j], a.eps) : q;
+    }
+  }
+  s = group_allreduce_tuple(s, red, idle ? 0 : group * (tpr >> 6), tpr >> 6);
+  if (wanted >= rows) return;
+  const float rc1 = MODE == BWD_RMS ? 0.f : s.v[0] * a.inv_cols, k3 = rs * rs * s.v[SUMS - 1] * a.inv_cols;
+  T* dxr = static_cast<T*>(a.dx) + row * a.dx_pitch;
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int v = i * tpr + t;
+    if (v < a.nvec) {
+      float o[VEC];
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) o[j] = fmaf(-xs[i][j], k3, ts[i][j] - rc1);
+      store_row_vec<T, RAGGED, true>(dxr, v, o, a.cols);
+    }
+  }
+}
+
 // Fallback backward for rows the register kernel cannot take (shorter than a 16-byte vector, more than 8192 columns,
 // no scratch given for rows off the 16-byte grid): one workgroup
 // per row for dx, then a column kernel for dgamma / dbeta (re-reads dy and x).
@@ -807,6 +961,48 @@ static int launch_norm_bwd_nv(const NormBwdArgs& a, const BwdPlan& p, hipStream_
   return launch_check("norm_bwd_kernel");
 }
 
+// norm_bwd_small_kernel where it measured faster: while its column sums take about one trip to memory.  Forward and backward, us,
+// three launches / so, rows of whole vectors: 16 x 640 bf16 12.0 / 8.8, 512 x 4096 12.6 / 10.3 (LayerNorm 14.3 / 10.9), 768 x 2048 11.8
+// / 11.1, x 4096 14.7 / 12.3, x 8192 20.6 / 16.5, fp32 30.1 / 27.9; 1024 x 512 bf16 11.9 / 9.4, x 2048 11.8 / 12.9, fp32 x 8192
+// 36.2 / 37.7, 1536 x 640 bf16 11.9 / 13.0.  Of any boundary, whose columns are split into narrower tiles (4 / 8 vectors, 512 x 1021
+// 10.3 / 10.6, 768 x 1021 12.2 / 14.0): 512 x 1021 bf16 12.4 / 10.3, x 8191 19.8 / 19.0, 256 x 8191 fp32 19.0 / 17.7, 640 x 1021
+// bf16 12.5 / 12.2, 512 x 8191 fp32 25.2 / 28.6.
+template <typename T, int MODE>
+static bool launch_norm_bwd_small(NormBwdArgs a, const BwdPlan& p, void* dgamma, void* dbeta, hipStream_t s) {
+  constexpr int VEC = VecIO<T>::N;
+  const int64_t row_bytes = int64_t(a.cols) * int64_t(sizeof(T));
+  const bool small = p.any ? a.rows <= 512 && a.rows * row_bytes <= (int64_t(8) << 20) : a.rows <= (row_bytes <= 1024 ? 1024 : 768);
+  if (!small || p.lpr || p.nv > (VEC == 4 ? 2 : 1) || tune_get(TUNE_NORM_BWD_ROWS_PER_BLOCK) > 0 || tune_get(TUNE_NORM_BWD_BLOCKS) > 0 ||
+      tune_get(TUNE_NORM_BWD_PREFETCH) > 0) return false;
+  // what is written may not lie over what other workgroups still read
+  const auto apart = [&](const void* out, int64_t n_out, const void* in, int64_t n_in) {
+    const uintptr_t o = reinterpret_cast<uintptr_t>(out), i = reinterpret_cast<uintptr_t>(in);
+    return out == nullptr || in == nullptr || i + uintptr_t(n_in) * sizeof(T) <= o || o + uintptr_t(n_out) * sizeof(T) <= i;
+  };
+  const auto extent = [&](int64_t pitch) { return (a.rows - 1) * pitch + a.cols; };
+  if (!apart(a.dx, extent(a.dx_pitch), a.dy, extent(a.dy_pitch)) || !apart(a.dx, extent(a.dx_pitch), a.x, extent(a.x_pitch)) ||
+      !apart(dgamma, a.cols, a.gamma, a.cols) || !apart(dbeta, a.cols, a.gamma, a.cols)) return false;
+  const int nvec = (a.cols + VEC - 1) / VEC, lanes = small_lanes(p.any), rpb = kSmallThreads / p.tpr;
+  a.tpr = p.tpr;
+  a.threads = kSmallThreads;
+  a.blocks = dgamma || dbeta ? (nvec + lanes - 1) / lanes : 0;
+  a.part_dgamma = static_cast<float*>(dgamma);
+  a.part_dbeta = static_cast<float*>(dbeta);
+  const NormBwdFlat f(a, MODE);
+  const dim3 grid{unsigned(a.blocks) + unsigned((a.rows + rpb - 1) / rpb)}, block{kSmallThreads};
+  profile_before(s);
+#define HK_BWD_SMALL(NV)                                                                              \
+  do {                                                                                                \
+    if (p.any) HK_LAUNCH((norm_bwd_small_kernel<T, NV, MODE, true>), grid, block, 0, s, f);           \
+    else HK_LAUNCH((norm_bwd_small_kernel<T, NV, MODE, false>), grid, block, 0, s, f);                \
+  } while (0)
+  if (p.nv == 1) HK_BWD_SMALL(1);
+  else if constexpr (VEC == 4) HK_BWD_SMALL(2);
+#undef HK_BWD_SMALL
+  profile_after(s);
+  return true;
+}
+
 template <typename T>
 int norm_bwd_typed(NormBwdArgs a, int mode, void* dgamma, void* dbeta, void* ws, size_t ws_bytes,
                    hipStream_t s) {
@@ -821,9 +1017,9 @@ int norm_bwd_typed(NormBwdArgs a, int mode, void* dgamma, void* dbeta, void* ws,
   // rows that once took no scratch do without it still
   if (p.any && want_cols && (ws == nullptr || ws_bytes < p.ws_bytes || !aligned16(ws))) p.reg_path = false;
   if (p.any && !a.stats_f32 && mode != BWD_LN) p.reg_path = false;
+  const bool lean = p.reg_path && tune_get(TUNE_NORM_BWD_THREADS) <= 0 && mode != BWD_LN_MEMEFF && a.stats_f32 && !a.dx_in &&
+                    !a.dres && NormBwdFlat::holds(a) && !(mode == BWD_RMS && (dbeta != nullptr || a.clamp_gamma));
   if (p.reg_path && tune_get(TUNE_NORM_BWD_THREADS) <= 0) {
-    const bool lean = mode != BWD_LN_MEMEFF && a.stats_f32 && !a.dx_in && !a.dres && NormBwdFlat::holds(a) &&
-                      !(mode == BWD_RMS && (dbeta != nullptr || a.clamp_gamma));
     const BwdPlan q = lean ? plan_norm_bwd_lanes<T>(a.rows, a.cols) : BwdPlan{};
     // (a scratch that was sized for the other plans alone still serves them)
     if (q.reg_path && (!want_cols || (ws != nullptr && ws_bytes >= q.ws_bytes && aligned16(ws)))) p = q;
@@ -852,6 +1048,9 @@ int norm_bwd_typed(NormBwdArgs a, int mode, void* dgamma, void* dbeta, void* ws,
     a.part_dgamma = nullptr;
     a.part_dbeta = nullptr;
   }
+  if (lean && (mode == BWD_LN ? launch_norm_bwd_small<T, BWD_LN>(a, p, dgamma, dbeta, s)
+                              : launch_norm_bwd_small<T, BWD_RMS>(a, p, dgamma, dbeta, s)))
+    return launch_check("norm_bwd_small_kernel");
   a.tpr = p.tpr;
   a.threads = uint16_t(p.block);
   a.blocks = p.grid;

@@ -189,6 +189,41 @@ def test_rmsnorm_bwd_without_dbeta(hk, cuda, dtype, rows, cols):
     assert torch.equal(tdx3, tdx)
 
 
+@pytest.mark.parametrize("dtype", ["fp32", "bf16", "fp16"])
+@pytest.mark.parametrize("is_rms", [True, False])
+def test_bwd_of_few_rows(hk, cuda, dtype, is_rms):
+    """One launch for the whole backward: the edges of its slices of rows, of its column tiles and of its rule, on whole vectors
+    and on any boundary; dx over dy or x, and dgamma over gamma, which other launches serve, to the same bits of dx."""
+    import torch
+    shapes = [(1, 8), (2, 64), (127, 72), (128, 520), (129, 64), (255, 1032), (256, 128), (257, 192), (512, 264), (513, 1024),
+              (768, 640), (769, 640), (1024, 256), (1025, 256), (130, 8192), (33, 4104), (3, 9), (1, 13), (255, 33), (257, 1021),
+              (511, 31), (512, 517), (513, 517), (300, 1027), (256, 8191), (70, 4099)]
+    for rows, cols in shapes:
+        x, gamma, _, dz = _inputs(rows, cols, dtype, 6100 + cols + rows)
+        tx, tg, tdz = (helpers.to_torch(v, dtype, cuda) for v in (x, gamma, dz))
+        mean = np.zeros(rows, np.float32) if is_rms else x.astype(np.float64).mean(-1).astype(np.float32)
+        rs = (1.0 / np.sqrt(np.square(x.astype(np.float64) - mean[:, None]).mean(-1) + 1e-2)).astype(np.float32)
+        tmu, trs = helpers.to_torch(mean, "fp32", cuda), helpers.to_torch(rs, "fp32", cuda)
+        tdx, tdg = torch.empty_like(tx), torch.empty_like(tg)
+        tdb = None if is_rms else torch.empty_like(tg)
+        hk.dropout_add_ln_bwd(tdz, None, tx, tmu, trs, tg, tdx, None, tdg, tdb, is_rms)
+        over_dy, over_x, over_g, dg2 = tdz.clone(), tx.clone(), tg.clone(), torch.empty_like(tg)
+        hk.dropout_add_ln_bwd(over_dy, None, tx, tmu, trs, tg, over_dy, None, dg2, tdb, is_rms)
+        hk.dropout_add_ln_bwd(tdz, None, over_x, tmu, trs, tg, over_x, None, dg2, tdb, is_rms)
+        dx2 = torch.empty_like(tx)
+        hk.dropout_add_ln_bwd(tdz, None, tx, tmu, trs, over_g, dx2, None, over_g, tdb, is_rms)
+        torch.cuda.synchronize()
+        what = "%d x %d" % (rows, cols)
+        assert torch.equal(over_dy, tdx) and torch.equal(over_x, tdx) and torch.equal(dx2, tdx), what
+        edx, edg, edb = oracle.dropout_add_ln_bwd(dz, None, x, mean, rs, gamma, is_rms)
+        many = float(np.sqrt(rows))   # column sums over `rows` terms: their rounding error is that of the terms
+        helpers.assert_close(tdx, edx, dtype, "dx0 " + what, scale=1.0)
+        helpers.assert_close(tdg, edg, dtype, "dgamma " + what, scale=many)
+        helpers.assert_close(over_g, edg, dtype, "dgamma " + what, scale=many)
+        if tdb is not None:
+            helpers.assert_close(tdb, edb, dtype, "dbeta " + what, scale=many)
+
+
 def test_rmsnorm_bwd_identity(hk, cuda):
     """sum_cols dx*x = eps * rs^3 * sum_cols (gamma*dz)*x per row: pins where eps sits."""
     import torch
