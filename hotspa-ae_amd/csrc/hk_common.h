@@ -708,20 +708,25 @@ using MaxSumTuple = OnlineSoftmaxTuple<2>;
 using MaxSumMaxTuple = OnlineSoftmaxTuple<3>;
 
 // Column sums of the fp32 partial rows that a backward kernel's workgroups leave behind: `nparts` rows, `pitch` floats (a
-// multiple of 4) apart.  A workgroup of kFoldThreads takes 32 neighbouring columns, one 128-byte line of every row, as 8 float4
-// groups x 32 row slices, so that 256 partial rows, one per compute unit, are 8 loads a thread that are all under way at once:
-// what it costs is one trip to memory, and the columns spread over as many compute units as there are lines.  Slices 8 lanes
-// apart meet in their wavefront, the rest in LDS.  Summed in 64 bits, which costs nothing beside that trip: what is left of the
-// rounding is that of the partial rows (900 x 512 fp32, 2-norm 7.8e-8 instead of 1.2e-7).  Returned in the first 32 threads: the
-// sum of column 32 * tile + t (0 past pitch).  (128 columns a workgroup, 16 rows a thread in two rounds, as
-// before: LayerNorm forward and backward of 8191 x 1021 bf16 24.1 us, RMSNorm of 32768 x 4096 216.5; so 23.3 and 214.4.)
-constexpr int kFoldThreads = 256, kFoldCols = 32;
+// multiple of 4) apart.  A workgroup of 32 * LANES threads takes 4 * LANES neighbouring columns, as LANES float4 groups x 32 row
+// slices, so that 256 partial rows, one per compute unit, are 8 loads a thread that are all under way at once: what it costs is
+// one trip to memory.  8 lanes, one 128-byte line of every row, spread the columns over as many compute units as there are lines;
+// where those are more than the device has, 32 lanes read longer runs (fold_lanes).  Slices meet in LDS.  A thread's rows are added
+// in pairs, the slices in 64 bits: what is left of the rounding is mostly that of the partial rows (900 x 512 fp32, 2-norm 9.4e-8;
+// one after the other 1.2e-7).  Returned in the first 4 * LANES threads: the sum of column 4 * LANES * tile + t (0 past pitch).
+// Forward and backward, us, two rounds of 8 rows by 512 threads to 128 columns / 8 lanes / 32 lanes: LayerNorm of 8191 x 1021 bf16 24.5 /
+// 23.6 / 24.6, of 4096 x 4096 40.3 / 38.9 / 40.7, RMSNorm of 32768 x 4096 215.4 / 213.4 / 215.2, LayerNorm of 1000 x 7202 fp32 (226 lines,
+// two sums) 37.6 / 38.9 / 37.75.
+constexpr int fold_threads(int lanes) { return 32 * lanes; }
+int device_cu_count();
+static inline int fold_lanes(int pitch, int sums) { return (pitch + 31) / 32 * sums > device_cu_count() ? 32 : 8; }
+template <int LANES>
 __device__ __forceinline__ float fold_partial_rows(const float* part, int nparts, int pitch, int tile) {
-  constexpr int U = 8, SLICES = kFoldThreads / 8;
-  __shared__ double lds[SLICES / 2][kFoldCols];
-  const int cg = int(threadIdx.x) & 7, slice = int(threadIdx.x) >> 3;
-  const int c = tile * kFoldCols + cg * 4;
-  double acc[4] = {0., 0., 0., 0.};
+  constexpr int U = 8, SLICES = 32, PAIR = LANES == 8 ? 2 : 1, COLS = 4 * LANES;
+  __shared__ float lds[SLICES / PAIR][COLS];
+  const int cg = int(threadIdx.x) & (LANES - 1), slice = int(threadIdx.x) / LANES;
+  const int c = tile * COLS + cg * 4;
+  float acc[4] = {0.f, 0.f, 0.f, 0.f};
   if (c < pitch) {
     for (int r = slice; r < nparts; r += U * SLICES) {
       u32x4 v[U];
@@ -731,23 +736,28 @@ __device__ __forceinline__ float fold_partial_rows(const float* part, int nparts
         v[u] = ld16_keep(part + int64_t(rr < nparts ? rr : nparts - 1) * pitch + c);
       }
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const bool in = r + u * SLICES < nparts;
-        acc[0] += in ? u2f(v[u].x) : 0.f; acc[1] += in ? u2f(v[u].y) : 0.f;
-        acc[2] += in ? u2f(v[u].z) : 0.f; acc[3] += in ? u2f(v[u].w) : 0.f;
+      for (int k = 0; k < 4; ++k) {
+        float f[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) f[u] = r + u * SLICES < nparts ? u2f(v[u][k]) : 0.f;
+#pragma unroll
+        for (int n = U / 2; n > 0; n /= 2)
+#pragma unroll
+          for (int u = 0; u < n; ++u) f[u] += f[u + n];
+        acc[k] += f[0];
       }
     }
   }
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
-    acc[k] += dpp_perm_f64<kDppRor8>(acc[k]);
-    if ((slice & 1) == 0) lds[slice >> 1][cg * 4 + k] = acc[k];
+    if constexpr (PAIR == 2) acc[k] += dpp_perm<kDppRor8>(acc[k]);   // slices 8 lanes apart
+    if (PAIR == 1 || (slice & 1) == 0) lds[slice / PAIR][cg * 4 + k] = acc[k];
   }
   __syncthreads();
   double s = 0.;
-  if (threadIdx.x < kFoldCols) {
+  if (threadIdx.x < COLS) {
 #pragma unroll
-    for (int i = 0; i < SLICES / 2; ++i) s += lds[i][threadIdx.x];
+    for (int i = 0; i < SLICES / PAIR; ++i) s += lds[i][threadIdx.x];
   }
   return float(s);
 }

@@ -770,12 +770,12 @@ struct DalFoldArgs {
   int nparts, cols;
 };
 
-template <typename WT>
-__global__ __launch_bounds__(kFoldThreads)
+template <typename WT, int LANES>
+__global__ __launch_bounds__(fold_threads(LANES))
 void dal_fold_kernel(DalFoldArgs a) {
-  const float s = fold_partial_rows(a.part[blockIdx.y], a.nparts, a.cols, int(blockIdx.x));
-  const int oc = int(blockIdx.x) * kFoldCols + int(threadIdx.x);
-  if (threadIdx.x < kFoldCols && oc < a.cols) Cvt<WT>::store(static_cast<WT*>(a.out[blockIdx.y]) + oc, s);
+  const float s = fold_partial_rows<LANES>(a.part[blockIdx.y], a.nparts, a.cols, int(blockIdx.x));
+  const int oc = int(blockIdx.x) * (4 * LANES) + int(threadIdx.x);
+  if (threadIdx.x < 4 * LANES && oc < a.cols) Cvt<WT>::store(static_cast<WT*>(a.out[blockIdx.y]) + oc, s);
 }
 
 // ---------------------------------------------------------------------------
@@ -1072,8 +1072,12 @@ int hk_dropout_add_ln_bwd_ex(const hkDropoutAddLnBwdParams* pp, hkStream_t strea
     profile_after(s);
     int r = launch_check("dal_bwd_kernel");
     if (r != HK_OK || wanted == 0) return r;
-    HK_LAUNCH((dal_fold_kernel<WT>), dim3(unsigned((p.cols + kFoldCols - 1) / kFoldCols), unsigned(wanted)),
-              dim3(kFoldThreads), 0, s, fold);
+    auto launch_fold = [&](auto kernel, int lanes) {
+      HK_LAUNCH(kernel, dim3(unsigned((p.cols + 4 * lanes - 1) / (4 * lanes)), unsigned(wanted)), dim3(unsigned(fold_threads(lanes))), 0, s,
+                fold);
+    };
+    if (fold_lanes(int(p.cols), wanted) == 8) launch_fold(dal_fold_kernel<WT, 8>, 8);
+    else launch_fold(dal_fold_kernel<WT, 32>, 32);
     return launch_check("dal_fold_kernel");
   });
 }

@@ -406,13 +406,13 @@ void norm_bwd_kernel(typename std::conditional<LEVELS || EXTRA, NormBwdArgs, Nor
 // Folds the [nparts, pitch] fp32 partial rows into dgamma / dbeta of type T (fold_partial_rows); blockIdx.y picks which.  Rows
 // of whole 16-byte vectors of T: pitch == cols; otherwise the last vector of a partial row holds the row's last columns, the
 // first pitch - cols of its elements being another vector's.
-template <typename T>
-__global__ __launch_bounds__(kFoldThreads)
+template <typename T, int LANES>
+__global__ __launch_bounds__(fold_threads(LANES))
 void norm_bwd_finalize_kernel(const float* part0, const float* part1, T* out0, T* out1, int nparts, int cols, int pitch) {
   T* out = blockIdx.y == 0 ? out0 : out1;
-  const float s = fold_partial_rows(blockIdx.y == 0 ? part0 : part1, nparts, pitch, int(blockIdx.x));
-  const int oc = int(blockIdx.x) * kFoldCols + int(threadIdx.x);
-  if (threadIdx.x >= kFoldCols || oc >= pitch) return;
+  const float s = fold_partial_rows<LANES>(blockIdx.y == 0 ? part0 : part1, nparts, pitch, int(blockIdx.x));
+  const int oc = int(blockIdx.x) * (4 * LANES) + int(threadIdx.x);
+  if (int(threadIdx.x) >= 4 * LANES || oc >= pitch) return;
   const int shift = pitch - cols, tail = pitch - VecIO<T>::N;   // shift > 0: the partial last vector
   if (shift == 0 || oc < tail) Cvt<T>::store(out + oc, s);
   else if (oc >= tail + shift) Cvt<T>::store(out + oc - shift, s);
@@ -1070,9 +1070,13 @@ int norm_bwd_typed(NormBwdArgs a, int mode, void* dgamma, void* dbeta, void* ws,
   }
   if (rc != HK_OK || !want_cols) return rc;
   const bool both = dgamma != nullptr && dbeta != nullptr;
-  HK_LAUNCH((norm_bwd_finalize_kernel<T>), dim3(unsigned((a.part_pitch + kFoldCols - 1) / kFoldCols), both ? 2 : 1),
-            dim3(kFoldThreads), 0, s, dgamma ? a.part_dgamma : a.part_dbeta, a.part_dbeta,
-            static_cast<T*>(dgamma ? dgamma : dbeta), static_cast<T*>(dbeta), p.grid, a.cols, a.part_pitch);
+  auto fold = [&](auto kernel, int lanes) {
+    HK_LAUNCH(kernel, dim3(unsigned((a.part_pitch + 4 * lanes - 1) / (4 * lanes)), both ? 2 : 1), dim3(unsigned(fold_threads(lanes))), 0, s,
+              dgamma ? a.part_dgamma : a.part_dbeta, a.part_dbeta, static_cast<T*>(dgamma ? dgamma : dbeta), static_cast<T*>(dbeta),
+              p.grid, a.cols, a.part_pitch);
+  };
+  if (fold_lanes(a.part_pitch, both ? 2 : 1) == 8) fold(norm_bwd_finalize_kernel<T, 8>, 8);
+  else fold(norm_bwd_finalize_kernel<T, 32>, 32);
   return launch_check("norm_bwd_finalize_kernel");
 }
 
