@@ -762,6 +762,66 @@ __device__ __forceinline__ float fold_partial_rows(const float* part, int nparts
   return float(s);
 }
 
+// Column sums of an array of few rows, by one workgroup of kSmallThreads threads for LANES * N columns: a slice of rows for every
+// LANES threads, N columns a thread, up to four rows of each slice under way at once.  load(row) fetches what a thread needs of a
+// row, add(fetched, whether the row exists, sums) adds it; slices meet in LDS, in 64 bits.  put(k, c, sum) gets sum k of column c
+// from one thread each.
+constexpr int kSmallThreads = 1024;
+template <int SUMS, int N, int LANES, typename Load, typename Add, typename Put>
+__device__ __forceinline__ void column_sums_of_few_rows(int rows, Load&& load, Add&& add, Put&& put) {
+  static_assert((LANES == 8 || LANES == 4) && N % 4 == 0 && SUMS * N * LANES * 8 <= kSmallThreads && N * LANES % 8 == 0, "");
+  constexpr int SLICES = kSmallThreads / LANES, COLS = LANES * N;
+  __shared__ __align__(16) float fold[SUMS][kSmallThreads / 16][COLS + 8];
+  const int lane = int(threadIdx.x) & (LANES - 1), slice = int(threadIdx.x) / LANES;
+  float acc[SUMS][N];
+#pragma unroll
+  for (int k = 0; k < SUMS; ++k)
+#pragma unroll
+    for (int j = 0; j < N; ++j) acc[k][j] = 0.f;
+  auto round = [&](int base, auto count) {
+    constexpr int U = decltype(count)::value;
+    decltype(load(int64_t(0))) raw[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) raw[u] = load(int64_t(min(base + u * SLICES + slice, rows - 1)));   // past the end: the last one
+#pragma unroll
+    for (int u = 0; u < U; ++u) add(raw[u], base + u * SLICES + slice < rows, acc);
+  };
+  int base = 0;
+  for (; rows - base > 2 * SLICES; base += 4 * SLICES) round(base, std::integral_constant<int, 4>{});
+  if (rows - base > SLICES) round(base, std::integral_constant<int, 2>{});
+  else if (rows > base) round(base, std::integral_constant<int, 1>{});
+#pragma unroll
+  for (int k = 0; k < SUMS; ++k) {
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      acc[k][j] += dpp_perm<kDppRor8>(acc[k][j]);
+      if constexpr (LANES == 4) acc[k][j] += dpp_perm<kDppRor4>(acc[k][j]);
+    }
+    if ((int(threadIdx.x) & 15) < LANES) {
+#pragma unroll
+      for (int j = 0; j < N; j += 4)
+        *reinterpret_cast<u32x4*>(&fold[k][threadIdx.x >> 4][lane * N + j]) =
+            u32x4{f2u(acc[k][j]), f2u(acc[k][j + 1]), f2u(acc[k][j + 2]), f2u(acc[k][j + 3])};
+    }
+  }
+  __syncthreads();
+  const int sub = int(threadIdx.x) & 7, o = int(threadIdx.x) >> 3, k = o / COLS, c = o % COLS;
+  if (k < SUMS) {   // whole wavefronts
+    double s = 0.;
+#pragma unroll
+    for (int i = 0; i < kSmallThreads / 128; ++i) s += fold[k][sub + 8 * i][c];
+    s += dpp_perm_f64<kDppXor1>(s);
+    s += dpp_perm_f64<kDppXor2>(s);
+    s += dpp_perm_f64<kDppHalfMirror>(s);
+    if (sub == 0) put(k, c, float(s));
+  }
+}
+// whether what is written is no byte of what is read (either may be null)
+inline bool apart(const void* out, int64_t out_bytes, const void* in, int64_t in_bytes) {
+  const uintptr_t o = reinterpret_cast<uintptr_t>(out), i = reinterpret_cast<uintptr_t>(in);
+  return out == nullptr || in == nullptr || i + uintptr_t(in_bytes) <= o || o + uintptr_t(out_bytes) <= i;
+}
+
 // The maximum of a thread's elements in the log2 domain, kept finite.  Below: a maximum near the type's lowest value
 // (logits masked with it) would overflow to -inf and turn 0 * inf into the row's sum, an empty maximum would need a
 // select; elements at such a maximum come out as 0, as they should next to any ordinary element of the row.  Above: a

@@ -762,6 +762,99 @@ void dal_bwd_stream_kernel(DalStreamArgs a) {
   put_column_sums(a.part[1], db0, stage, group, rpb, in, cols, col);
 }
 
+// The same for few rows, in one launch: three trips to memory otherwise (rows, partial rows, their fold).  The first a.blocks
+// workgroups form the column sums from the operands themselves (column_sums_of_few_rows), the others dx0 and dresidual, to the same
+// bits; part: dgamma and dbeta.  dx0 and dresidual must not lie over dz or x.
+template <typename IT, typename RT, typename WT>
+__global__ __launch_bounds__(kSmallThreads)
+void dal_bwd_small_kernel(DalStreamArgs a) {
+  constexpr int NI = kChunk / VecIO<IT>::N, NR = kChunk / VecIO<RT>::N, LANES = NR == 1 ? 8 : 4;
+  __shared__ __align__(16) float red[kMaxWaves * 2];
+  const int rows = int(a.rows_rms & 0x7fffffffu), cols = int(a.cols), nchunks = int(a.cols / uint32_t(kChunk));
+  const bool is_rms = a.rows_rms >> 31 != 0;
+  struct Fetched {
+    u32x4 dz[NI], x[NR];
+    float mu, rs;
+  };
+  const auto fetch = [&](int64_t r, int col) {
+    Fetched f;
+    const int64_t e = r * int64_t(cols) + col;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) f.dz[i] = ld16_keep(static_cast<const IT*>(a.dz) + e + i * VecIO<IT>::N);
+#pragma unroll
+    for (int i = 0; i < NR; ++i) f.x[i] = ld16_keep(static_cast<const RT*>(a.x) + e + i * VecIO<RT>::N);
+    f.mu = is_rms ? 0.f : a.mu[r];
+    f.rs = a.rs[r];
+    return f;
+  };
+  const auto unpack = [&](const Fetched& f, float* dz, float* y) {
+#pragma unroll
+    for (int i = 0; i < NI; ++i) VecIO<IT>::unpack(f.dz[i], dz + i * VecIO<IT>::N);
+#pragma unroll
+    for (int i = 0; i < NR; ++i) VecIO<RT>::unpack(f.x[i], y + i * VecIO<RT>::N);
+#pragma unroll
+    for (int j = 0; j < kChunk; ++j) y[j] = f.rs * (y[j] - f.mu);
+  };
+  if (blockIdx.x < a.blocks) {
+    const int first = int(blockIdx.x) * LANES, col = min(first + (int(threadIdx.x) & (LANES - 1)), nchunks - 1) * kChunk;
+    column_sums_of_few_rows<2, kChunk, LANES>(
+        rows, [&](int64_t r) { return fetch(r, col); },
+        [&](const Fetched& f, bool in, float (&acc)[2][kChunk]) {
+          float dz[kChunk], y[kChunk];
+          unpack(f, dz, y);
+#pragma unroll
+          for (int j = 0; j < kChunk; ++j) {
+            acc[0][j] = in ? fmaf(dz[j], y[j], acc[0][j]) : acc[0][j];
+            acc[1][j] += in ? dz[j] : 0.f;
+          }
+        },
+        [&](int k, int c, float sum) {
+          WT* out = reinterpret_cast<WT*>(a.part[k]);
+          if (out != nullptr && first * kChunk + c < cols) Cvt<WT>::store(out + first * kChunk + c, sum);
+        });
+    return;
+  }
+  const int tpr = a.tpr, rpb = kSmallThreads / tpr;
+  const int group = __builtin_amdgcn_readfirstlane(int(threadIdx.x) / tpr), t = int(threadIdx.x) - group * tpr;
+  // (the wavefronts that no row is left for work on the last one too and store nothing)
+  const bool idle = group >= rpb, in = t < nchunks;
+  const int64_t wanted = idle ? rows : int64_t(blockIdx.x - a.blocks) * rpb + group, row = wanted < rows ? wanted : rows - 1;
+  const int col = (in ? t : nchunks - 1) * kChunk;
+  const int64_t e = row * int64_t(cols) + col;
+  const Fetched f = fetch(row, col);
+  u32x4 ndx[NR];
+#pragma unroll
+  for (int i = 0; i < NR; ++i) ndx[i] = ld16(static_cast<const RT*>(a.dx) + e + i * VecIO<RT>::N);
+  const u32x2 mw = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(a.dmask + e));
+  float g0[kChunk], dz[kChunk], y[kChunk], u[kChunk];
+  load8_keep<WT>(static_cast<const WT*>(a.gamma) + col, g0);
+  unpack(f, dz, y);
+#pragma unroll
+  for (int i = 0; i < NR; ++i) VecIO<RT>::unpack(ndx[i], &u[i * VecIO<RT>::N]);
+  SumTuple<2> s;
+  s.v[0] = 0.f; s.v[1] = 0.f;
+  float dy[kChunk];
+#pragma unroll
+  for (int j = 0; j < kChunk; ++j) {
+    dy[j] = g0[j] * (in ? dz[j] : 0.f);
+    s.v[0] += dy[j];
+    s.v[1] = fmaf(dy[j], y[j], s.v[1]);
+  }
+  s = group_allreduce_tuple(s, red, idle ? 0 : group * (tpr >> 6), tpr >> 6);
+  if (wanted >= rows || !in) return;
+  const float mdy = is_rms ? 0.f : s.v[0] * a.inv_cols;
+  const float mdyy = s.v[1] * a.inv_cols;
+  float o[kChunk];
+#pragma unroll
+  for (int j = 0; j < kChunk; ++j) {
+    u[j] += f.rs * (dy[j] - fmaf(mdyy, y[j], mdy));
+    const uint32_t byte = ((j < 4 ? mw.x : mw.y) >> (8 * (j & 3))) & 0xffu;
+    o[j] = byte ? u[j] * a.scale : 0.f;
+  }
+  store8<RT, false>(static_cast<RT*>(a.dresidual) + e, u);
+  store8<IT, true>(static_cast<IT*>(a.dx0) + e, o);
+}
+
 // Folds [nparts, cols] fp32 partial rows into a [cols] vector of WT (fold_partial_rows); blockIdx.y picks which of the (up to
 // five) sums that are wanted.
 struct DalFoldArgs {
@@ -1064,6 +1157,24 @@ int hk_dropout_add_ln_bwd_ex(const hkDropoutAddLnBwdParams* pp, hkStream_t strea
     const DalStreamArgs f{a.dz, a.dx, a.x, a.dmask, a.mu, a.rs, a.gamma, a.dx0, a.dresidual, {a.part[0], a.part[1]},
                           uint32_t(a.rows) | (a.is_rms ? 0x80000000u : 0u), uint32_t(a.cols), a.inv_cols, a.scale,
                           uint16_t(a.tpr), uint16_t(sh.block), uint32_t(sh.grid)};
+    // dal_bwd_small_kernel where it measured faster, forward and backward, us, two launches of the backward / one: bf16 64 x 512 12.5 /
+    // 9.7, 256 x 4096 15.8 / 10.4, 768 x 2048 15.5 / 12.3, x 8192 36.6 / 29.6, 1024 x 512 12.5 / 10.8, x 8192 40.8 / 37.6, 1500 x 1024
+    // 15.1 / 15.5, x 8192 53.6 / 51.6; fp32 256 x 8192 28.8 / 24.1, 768 x 1024 15.8 / 12.4, x 4096 31.2 / 28.9, x 6144 45.6 / 47.8, 1024 x
+    // 2048 23.2 / 22.7, x 4096 38.7 / 39.0.
+    const int64_t n = p.rows * p.cols, ni = n * int64_t(sizeof(IT)), nr = n * int64_t(sizeof(RT));
+    if (stream_form && p.rows <= (sizeof(RT) == 2 ? 1024 : 768) && nr <= (int64_t(16) << 20) && tune_get(TUNE_NORM_BWD_BLOCKS) <= 0 && tune_get(TUNE_NORM_BWD_ROWS_PER_BLOCK) <= 0 &&
+        apart(p.dx0, ni, p.dz, ni) && apart(p.dx0, ni, p.x, nr) && apart(p.dresidual, nr, p.dz, ni) && apart(p.dresidual, nr, p.x, nr) &&
+        apart(p.dx0, ni, p.dx, nr) && apart(p.dgamma, p.cols * int64_t(sizeof(WT)), p.gamma, p.cols * int64_t(sizeof(WT))) &&
+        apart(p.dbeta, p.cols * int64_t(sizeof(WT)), p.gamma, p.cols * int64_t(sizeof(WT)))) {
+      const int lanes = sizeof(RT) == 2 ? 8 : 4, rpb = kSmallThreads / sh.tpr;
+      DalStreamArgs few = f;
+      few.part[0] = static_cast<float*>(p.dgamma);
+      few.part[1] = static_cast<float*>(p.dbeta);
+      few.blocks = wanted ? uint32_t((a.nchunks + lanes - 1) / lanes) : 0;   // (the rest to the same bits without them)
+      HK_LAUNCH((dal_bwd_small_kernel<IT, RT, WT>), dim3(few.blocks + unsigned((p.rows + rpb - 1) / rpb)), dim3(kSmallThreads), 0, s, few);
+      profile_after(s);
+      return launch_check("dal_bwd_small_kernel");
+    }
     if (stream_form && full && sh.tpr == 512 && sh.block == 512) HK_LAUNCH((dal_bwd_stream_kernel<IT, RT, WT, PF, 512>), grid, block, lds, s, f);
     else if (stream_form) HK_LAUNCH((dal_bwd_stream_kernel<IT, RT, WT, PF, 0>), grid, block, lds, s, f);
     else if (g1) HK_LAUNCH((dal_bwd_kernel<IT, RT, WT, false, true>), grid, block, lds, s, a);

@@ -115,8 +115,6 @@ struct NormBwdArgs {
   template <typename T, int MODE> __device__ __forceinline__ const NormBwdArgs& args() const { return *this; }
 };
 
-constexpr int kSmallThreads = 1024;   // of a workgroup of norm_bwd_small_kernel
-
 // What the lean instances take of it: rows on one level, no optional operands (see kCheapArgs)
 struct NormBwdFlat {
   const void* dy;

@@ -422,17 +422,14 @@ constexpr int small_lanes(bool ragged) { return ragged ? 4 : 8; }
 // The whole backward of a small array in one launch.  Its time is that of launches and trips to memory, of which the kernels above
 // take three (rows, partial rows, their fold), so here the first a.blocks workgroups form the column sums from the operands
 // themselves, LANES vectors of every row each, and the others dx: what is read twice comes from a cache.  dx must not lie over dy
-// or x.  A workgroup of column sums has a slice of rows for every LANES threads, up to four rows of each under way at once; the
-// slices meet in LDS, in 64 bits.  dx comes out to the same bits as from norm_bwd_kernel: the plan's threads and vectors, its
+// or x (see column_sums_of_few_rows).  dx comes out to the same bits as from norm_bwd_kernel: the plan's threads and vectors, its
 // order of operations.
 template <typename T, int NV, int MODE, bool RAGGED>
 __global__ __launch_bounds__(kSmallThreads)
 void norm_bwd_small_kernel(NormBwdFlat given) {
   constexpr int LANES = small_lanes(RAGGED);
   const NormBwdArgs a = given.template args<T, MODE>();
-  constexpr int VEC = VecIO<T>::N, SLICES = kSmallThreads / LANES, COLS = LANES * VEC;
-  constexpr int SUMS = MODE == BWD_RMS ? 1 : 2;
-  __shared__ __align__(16) float fold[SUMS][kSmallThreads / 16][COLS + 8];
+  constexpr int VEC = VecIO<T>::N, SUMS = MODE == BWD_RMS ? 1 : 2;
   __shared__ __align__(16) float red[kMaxWaves * SUMS];
   auto ld_row = [](const T* p) { if constexpr (RAGGED) return ld16_any_keep<T>(p); else return ld16_keep(p); };
   auto rs_of = [&](float sv) { return (MODE != BWD_RMS && a.stat_kind == HK_STAT_VAR) ? 1.0f / sqrtf(sv + a.eps) : sv; };
@@ -442,70 +439,35 @@ void norm_bwd_small_kernel(NormBwdFlat given) {
   const T* dyp = static_cast<const T*>(a.dy);
   const int rows = int(a.rows);
   if (int(blockIdx.x) < a.blocks) {
-    const int lane = int(threadIdx.x) & (LANES - 1), slice = int(threadIdx.x) / LANES;
-    const int col = vec_column<T, RAGGED>(min(int(blockIdx.x) * LANES + lane, a.nvec - 1), a.cols);
-    float dg[VEC], db[VEC];
-#pragma unroll
-    for (int j = 0; j < VEC; ++j) dg[j] = db[j] = 0.f;
-    auto round = [&](int base, auto count) {
-      constexpr int U = decltype(count)::value;
-      u32x4 rx[U], rdy[U];
-      float mu[U], sv[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {   // a row past the end reads the last one
-        const int64_t r = min(base + u * SLICES + slice, rows - 1);
-        rx[u] = ld_row(xp + r * a.x_pitch + col);
-        rdy[u] = ld_row(dyp + r * a.dy_pitch + col);
-        mu[u] = MODE == BWD_LN ? meanp[r] : 0.f;
-        sv[u] = statp[r];
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const bool in = base + u * SLICES + slice < rows;
-        const float rs = rs_of(sv[u]);
-        float x[VEC], d[VEC];
-        VecIO<T>::unpack(rx[u], x);
-        VecIO<T>::unpack(rdy[u], d);
-#pragma unroll
-        for (int j = 0; j < VEC; ++j) {
-          const float more = fmaf(d[j] * rs, MODE == BWD_LN ? x[j] - mu[u] : x[j], dg[j]);
-          dg[j] = in ? more : dg[j];
-          if constexpr (SUMS == 2) db[j] += in ? d[j] : 0.f;
-        }
-      }
+    struct Fetched {
+      u32x4 x, dy;
+      float mu, sv;
     };
-    int base = 0;
-    for (; rows - base > 2 * SLICES; base += 4 * SLICES) round(base, std::integral_constant<int, 4>{});
-    if (rows - base > SLICES) round(base, std::integral_constant<int, 2>{});
-    else if (rows > base) round(base, std::integral_constant<int, 1>{});
+    const int first = int(blockIdx.x) * LANES;
+    const int col = vec_column<T, RAGGED>(min(first + (int(threadIdx.x) & (LANES - 1)), a.nvec - 1), a.cols);
+    column_sums_of_few_rows<SUMS, VEC, LANES>(
+        rows,
+        [&](int64_t r) {
+          return Fetched{ld_row(xp + r * a.x_pitch + col), ld_row(dyp + r * a.dy_pitch + col), MODE == BWD_LN ? meanp[r] : 0.f, statp[r]};
+        },
+        [&](const Fetched& f, bool in, float (&acc)[SUMS][VEC]) {
+          const float rs = rs_of(f.sv);
+          float x[VEC], d[VEC];
+          VecIO<T>::unpack(f.x, x);
+          VecIO<T>::unpack(f.dy, d);
 #pragma unroll
-    for (int k = 0; k < SUMS; ++k) {
-      float* acc = k == 0 ? dg : db;
-#pragma unroll
-      for (int j = 0; j < VEC; ++j) {
-        acc[j] += dpp_perm<kDppRor8>(acc[j]);
-        if constexpr (LANES == 4) acc[j] += dpp_perm<kDppRor4>(acc[j]);
-      }
-      if ((int(threadIdx.x) & 15) < LANES) {
-#pragma unroll
-        for (int j = 0; j < VEC; j += 4)
-          st16(&fold[k][threadIdx.x >> 4][lane * VEC + j], u32x4{f2u(acc[j]), f2u(acc[j + 1]), f2u(acc[j + 2]), f2u(acc[j + 3])});
-      }
-    }
-    __syncthreads();
-    const int sub = int(threadIdx.x) & 7, o = int(threadIdx.x) >> 3, k = o / COLS, c = o % COLS;
-    if (k < SUMS) {   // whole wavefronts
-      double s = 0.;
-#pragma unroll
-      for (int i = 0; i < kSmallThreads / 128; ++i) s += fold[k][sub + 8 * i][c];
-      s += dpp_perm_f64<kDppXor1>(s);
-      s += dpp_perm_f64<kDppXor2>(s);
-      s += dpp_perm_f64<kDppHalfMirror>(s);
-      T* out = reinterpret_cast<T*>(k == 0 ? a.part_dgamma : a.part_dbeta);
-      const int v = int(blockIdx.x) * LANES + c / VEC;
-      const int at = vec_column<T, RAGGED>(v, a.cols) + c % VEC;   // a column that two vectors hold: from the first
-      if (sub == 0 && v < a.nvec && out != nullptr && at >= v * VEC) Cvt<T>::store(out + at, float(s));
-    }
+          for (int j = 0; j < VEC; ++j) {
+            const float more = fmaf(d[j] * rs, MODE == BWD_LN ? x[j] - f.mu : x[j], acc[0][j]);
+            acc[0][j] = in ? more : acc[0][j];
+            if constexpr (SUMS == 2) acc[1][j] += in ? d[j] : 0.f;
+          }
+        },
+        [&](int k, int c, float sum) {
+          T* out = reinterpret_cast<T*>(k == 0 ? a.part_dgamma : a.part_dbeta);
+          const int v = first + c / VEC;
+          const int at = vec_column<T, RAGGED>(v, a.cols) + c % VEC;   // a column that two vectors hold: from the first
+          if (v < a.nvec && out != nullptr && at >= v * VEC) Cvt<T>::store(out + at, sum);
+        });
     return;
   }
 
@@ -974,14 +936,9 @@ static bool launch_norm_bwd_small(NormBwdArgs a, const BwdPlan& p, void* dgamma,
   const bool small = p.any ? a.rows <= 512 && a.rows * row_bytes <= (int64_t(8) << 20) : a.rows <= (row_bytes <= 1024 ? 1024 : 768);
   if (!small || p.lpr || p.nv > (VEC == 4 ? 2 : 1) || tune_get(TUNE_NORM_BWD_ROWS_PER_BLOCK) > 0 || tune_get(TUNE_NORM_BWD_BLOCKS) > 0 ||
       tune_get(TUNE_NORM_BWD_PREFETCH) > 0) return false;
-  // what is written may not lie over what other workgroups still read
-  const auto apart = [&](const void* out, int64_t n_out, const void* in, int64_t n_in) {
-    const uintptr_t o = reinterpret_cast<uintptr_t>(out), i = reinterpret_cast<uintptr_t>(in);
-    return out == nullptr || in == nullptr || i + uintptr_t(n_in) * sizeof(T) <= o || o + uintptr_t(n_out) * sizeof(T) <= i;
-  };
-  const auto extent = [&](int64_t pitch) { return (a.rows - 1) * pitch + a.cols; };
+  const auto extent = [&](int64_t pitch) { return ((a.rows - 1) * pitch + a.cols) * int64_t(sizeof(T)); };
   if (!apart(a.dx, extent(a.dx_pitch), a.dy, extent(a.dy_pitch)) || !apart(a.dx, extent(a.dx_pitch), a.x, extent(a.x_pitch)) ||
-      !apart(dgamma, a.cols, a.gamma, a.cols) || !apart(dbeta, a.cols, a.gamma, a.cols)) return false;
+      !apart(dgamma, row_bytes, a.gamma, row_bytes) || !apart(dbeta, row_bytes, a.gamma, row_bytes)) return false;
   const int nvec = (a.cols + VEC - 1) / VEC, lanes = small_lanes(p.any), rpb = kSmallThreads / p.tpr;
   a.tpr = p.tpr;
   a.threads = kSmallThreads;

@@ -393,3 +393,46 @@ def test_mask_at_every_probability(hk, cuda, p):
     torch.cuda.synchronize()
     want = dal.dropout_keep(seed, 0, rows * cols, np.float32(1) - np.float32(p)).reshape(rows, cols)
     assert np.array_equal(mask.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("combo", [("fp32", "fp32", "fp32"), ("bf16", "bf16", "bf16"), ("fp32", "fp16", "fp32"),
+                                   ("fp16", "fp16", "fp16"), ("fp16", "fp32", "fp32")], ids=lambda c: "w%s-i%s-r%s" % c)
+@pytest.mark.parametrize("is_rms", [False, True])
+def test_block_backward_of_few_rows(hk, cuda, combo, is_rms):
+    """One launch for the whole backward of the dropout block: the edges of its slices of rows, column tiles and rule; gradients
+    written over dz, x or the residual stream's gradient, and dgamma over gamma, to the same bits of the gradients."""
+    import torch
+    wt, it, rt = combo
+    for rows, cols in [(1, 8), (2, 64), (127, 72), (128, 520), (255, 1032), (257, 192), (512, 264), (513, 640), (768, 128),
+                       (769, 128), (1024, 264), (1025, 136), (130, 8192), (40, 4104)]:
+        x, dx_in, dz = helpers.draw(71, (rows, cols), dtype=rt), helpers.draw(72, (rows, cols), dtype=rt), helpers.draw(73, (rows, cols), dtype=it)
+        gamma = helpers.draw(74, (cols,), "uniform", 0.5, 1.5, wt)
+        mask = _mask(rows * cols, 0.3).reshape(rows, cols)
+        xd = x.astype(np.float64)
+        mean = np.zeros(rows, np.float32) if is_rms else xd.mean(-1).astype(np.float32)
+        rs = (1.0 / np.sqrt(np.square(xd - mean[:, None]).mean(-1) + 1e-2)).astype(np.float32)
+        edx0, edres, edg, edb, _ = dal.bwd(dz, dx_in, x, None, mask, mean, rs, gamma, None, None, dropout_p=0.3, is_rms=is_rms)
+        tx, tdxin, tdz, tg = _tt(x, rt, cuda), _tt(dx_in, rt, cuda), _tt(dz, it, cuda), _tt(gamma, wt, cuda)
+        tmask, tmu, trs = _tt(mask, "uint8", cuda), _tt(mean, "fp32", cuda), _tt(rs, "fp32", cuda)
+        what = "%d x %d" % (rows, cols)
+
+        def run(x=tx, dxin=tdxin, dz=tdz, g=tg, dx0=None, dres=None, dg=None):
+            dx0 = torch.empty_like(tdz) if dx0 is None else dx0
+            dres = torch.empty_like(tx) if dres is None else dres
+            dg, db = torch.empty_like(tg) if dg is None else dg, torch.empty_like(tg)
+            hk.dropout_add_ln_bwd_ex(dz, x, tmu, trs, g, dx0, dx=dxin, dmask=tmask, dresidual=dres, dgamma=dg, dbeta=db,
+                                     dropout_p=0.3, is_rms=is_rms)
+            return dx0, dres, dg, db
+        dx0, dres, dg, db = run()
+        over = tdz.clone(), tx.clone(), tdxin.clone(), tg.clone()
+        outs = [run(dz=over[0], dx0=over[0])[:2], run(x=over[1], dres=over[1])[:2], run(dxin=over[2], dres=over[2])[:2],
+                run(g=over[3], dg=over[3])[:2]]
+        torch.cuda.synchronize()
+        for o in outs:
+            assert torch.equal(o[0], dx0) and torch.equal(o[1], dres), what
+        many = float(np.sqrt(rows))   # column sums over `rows` terms: their rounding error is that of the terms
+        helpers.assert_close(dx0, edx0, it, "dx0 " + what)
+        helpers.assert_close(dres, edres, rt, "dresidual " + what)
+        for got in (dg, over[3]):
+            helpers.assert_close(got, edg, wt, "dgamma " + what, scale=many)
+        helpers.assert_close(db, edb, wt, "dbeta " + what, scale=many)
