@@ -680,9 +680,21 @@ static BnPlan<IT> bn_plan(int64_t N, int64_t C, int64_t HW, int max_splits, int 
   b.runs.C = int(C); b.runs.HW = IT(HW); b.runs.image = C * HW;
   b.runs.run_vecs = IT(run_vecs);
   b.runs.total = IT(total);
+  // workgroups of nv vectors a thread that a compute unit runs at once: 32 wavefronts, fewer past 64 registers a thread
+  const auto at_once = [&](int nv) {
+    const int waves = nv == 8 ? (VEC == 8 ? 16 : 24) : max_nv == 4 && nv == 4 && VEC == 8 ? 20 : 32;
+    return waves / int(((total + nv - 1) / nv + 63) / 64);
+  };
+  const int64_t cus = device_cu_count();
   for (int nv = 1; nv <= max_nv; nv <<= 1) {
     // one vector a thread while there are fewer channels than two workgroups per compute unit, else two at least
     if (total > int64_t(nv) * 1024 || (nv == 1 && total > 64 && C > 2 * device_cu_count())) continue;
+    // and twice the fewest where not all channels run at once so and more of them do then, backward as many (forward and backward, us,
+    // fewest / twice: 64 x 600 x 196 bf16 25.0 / 21.5, 10 x 900 x 1024 24.7 / 20.4, 30 x 999 x 441 39.8 / 33.8, backward as it was 35.4, 40 x
+    // 1000 x 144 fp32 27.3 / 22.6; where all run at once or no more do, 2 x 600 x 3000 fp16 12.2 / 12.65, 100 x 1024 x 49 20.1 / 20.6, 38 x
+    // 587 x 576, forward, of 33.7 both ways, 2.5 more)
+    const bool more = max_nv == 4 ? at_once(2 * nv) >= at_once(nv) : at_once(2 * nv) > at_once(nv);
+    if (2 * nv <= max_nv && C > cus * at_once(nv) && more) nv *= 2;
     b.form = 1;
     b.nv = nv;
     b.threads = int(((total + nv - 1) / nv + 63) / 64 * 64);
@@ -691,10 +703,11 @@ static BnPlan<IT> bn_plan(int64_t N, int64_t C, int64_t HW, int max_splits, int 
   b.form = 2;
   const int64_t want = (int64_t(device_cu_count()) * 8 + C - 1) / C, round = 256 * kBnVecs;
   const int64_t most = std::max<int64_t>(1, std::min<int64_t>(std::min(want, (total + round - 1) / round), std::min(max_splits, 256)));
-  // as few slices as take that many rounds of loads: a last one that is nearly empty costs a trip to memory like any other (us:
-  // 31 x 404 x 2304 fp16 32.8 / 48.4 -> 30.1 / 45.9, 107 x 26 x 2601 bf16 forward 15.0 -> 14.0, 128 x 27 x 6084 fp32 backward 71.4 -> 67.7)
+  // as few slices as take one or two rounds of loads: a last one that is nearly empty costs a trip to memory like any other (us: 31 x 404
+  // x 2304 fp16 32.8 / 48.4 -> 30.1 / 45.9, 107 x 26 x 2601 bf16 forward 15.0 -> 14.0, 200 x 100 x 1000 both ways 65.0 -> 60.8).  Where they
+  // take more, the compute units' room counts (140 x 65 x 4761 bf16, 32 slices / 28 119.4 / 124.0, 128 x 27 x 6084 fp32 112.4 / 111.2).
   const int64_t rounds = (total + round * most - 1) / (round * most);
-  b.splits = int((total + round * rounds - 1) / (round * rounds));
+  b.splits = int(rounds > 2 ? most : (total + round * rounds - 1) / (round * rounds));
   return b;
 }
 template <typename IT>

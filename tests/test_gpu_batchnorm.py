@@ -215,3 +215,48 @@ def test_channels_that_hold_a_nan_or_an_infinity(hk, cuda, dtype, shape):
     y, rm, rv, sm, si = (t[hit] for t in out[1])
     assert bool(torch.isnan(y).all()) and bool(torch.isnan(rv).all()) and bool(torch.isnan(si).all())
     assert not bool(torch.isfinite(rm).any()) and not bool(torch.isfinite(sm).any())
+
+
+@pytest.mark.parametrize("dtype", ["fp32", "bf16", "fp16"])
+@pytest.mark.parametrize("shape", [(64, 513, 25), (10, 600, 1041), (40, 530, 144), (3, 700, 2003), (38, 587, 576), (30, 65, 2001),
+                                   (13, 65, 9001)])
+def test_many_channels(hk, cuda, dtype, shape):
+    """More channels than run at once in their smallest number of vectors a thread, and one to three rounds of loads a slice."""
+    import torch
+    dt = {"fp32": torch.float32, "bf16": torch.bfloat16, "fp16": torch.float16}[dtype]
+    gen = torch.Generator(device="cuda").manual_seed(23)
+    x = (torch.randn(shape, generator=gen, device=cuda) * 2 + 3).to(dt)
+    dy = torch.randn(shape, generator=gen, device=cuda).to(dt)
+    C, m = shape[1], shape[0] * shape[2]
+    scale, bias = torch.rand(C, generator=gen, device=cuda) + 0.5, torch.randn(C, generator=gen, device=cuda)
+    rm, rv = torch.zeros(C, device=cuda), torch.ones(C, device=cuda)
+    y, dx = torch.empty_like(x), torch.empty_like(x)
+    mean, invstd, ds, db = (torch.empty(C, device=cuda) for _ in range(4))
+    hk.batch_norm_fwd(x, scale, bias, y, 0.1, 1e-5, rm, rv, mean, invstd)
+    hk.batch_norm_bwd(dy, x, scale, dx, ds, db, mean, invstd)
+    xd, gd = x.double(), dy.double()
+    mu = xd.mean((0, 2))
+    var = xd.var((0, 2), unbiased=False)
+    istd = 1 / torch.sqrt(var + 1e-5)
+    v = lambda t: t.double()[None, :, None]
+    xhat = (xd - v(mu)) * v(istd)
+    sdy, sdyx = gd.sum((0, 2)), (gd * xhat).sum((0, 2))
+    host = lambda t: t.cpu().numpy()
+    helpers.assert_close(mean, host(mu), "fp32", "mean", scale=3.0)
+    helpers.assert_close(invstd, host(istd), "fp32", "invstd")
+    helpers.assert_close(rv, host(0.9 + 0.1 * var * m / (m - 1)), "fp32", "running_var")
+    # the rounding of what is stored, and fp32's of the terms that each element is the sum of: the statistics' own (2^-22), and
+    # one for every operation
+    ulp = {"fp32": 2.0 ** -23, "bf16": 2.0 ** -8, "fp16": 2.0 ** -10}[dtype]
+    tiny = 2.0 ** -24 if dtype == "fp16" else 0.0
+    # (the mean's rounding is that of terms of a standard deviation)
+    ey, size = xhat * v(scale) + v(bias), (xhat.abs() + 1) * v(scale) + v(bias).abs()
+    assert bool(((y.double() - ey).abs() <= ulp * ey.abs() + 2.0 ** -20 * size + tiny).all())
+    # sums over m terms: their rounding error is that of the terms
+    helpers.assert_close(db, host(sdy), "fp32", "dbias", scale=float(np.sqrt(m)))
+    helpers.assert_close(ds, host(sdyx), "fp32", "dscale", scale=float(np.sqrt(m)))
+    # (of a sum, the terms'; of xhat, the saved mean's as well, which is of fp32)
+    k = v(scale) * v(istd)
+    edx = k * (gd - v(sdy / m) - xhat * v(sdyx / m))
+    size = k * (gd.abs() + v(gd.abs().mean((0, 2))) + (xhat.abs() + v(mu * istd)) * v((gd * xhat).abs().mean((0, 2))))
+    assert bool(((dx.double() - edx).abs() <= ulp * edx.abs() + 2.0 ** -20 * size + tiny).all())
