@@ -816,10 +816,19 @@ __device__ __forceinline__ void column_sums_of_few_rows(int rows, Load&& load, A
     if (sub == 0) put(k, c, float(s));
   }
 }
-// whether what is written is no byte of what is read (either may be null)
-inline bool apart(const void* out, int64_t out_bytes, const void* in, int64_t in_bytes) {
-  const uintptr_t o = reinterpret_cast<uintptr_t>(out), i = reinterpret_cast<uintptr_t>(in);
-  return out == nullptr || in == nullptr || i + uintptr_t(in_bytes) <= o || o + uintptr_t(out_bytes) <= i;
+struct Span {
+  const void* at;   // may be null
+  int64_t bytes;
+};
+// whether nothing that is written shares a byte with anything that is read: what one launch that stores before all of its
+// workgroups have read needs, where launches one after the other need nothing of the kind
+inline bool apart(std::initializer_list<Span> written, std::initializer_list<Span> read) {
+  for (const Span& w : written)
+    for (const Span& r : read) {
+      const uintptr_t o = reinterpret_cast<uintptr_t>(w.at), i = reinterpret_cast<uintptr_t>(r.at);
+      if (w.at != nullptr && r.at != nullptr && i + uintptr_t(r.bytes) > o && o + uintptr_t(w.bytes) > i) return false;
+    }
+  return true;
 }
 
 // The maximum of a thread's elements in the log2 domain, kept finite.  Below: a maximum near the type's lowest value

@@ -764,7 +764,8 @@ void dal_bwd_stream_kernel(DalStreamArgs a) {
 
 // The same for few rows, in one launch: three trips to memory otherwise (rows, partial rows, their fold).  The first a.blocks
 // workgroups form the column sums from the operands themselves (column_sums_of_few_rows), the others dx0 and dresidual, to the same
-// bits; part: dgamma and dbeta.  dx0 and dresidual must not lie over dz or x.
+// bits; part: dgamma and dbeta.  Nothing that is written may lie over what is read, but
+// dresidual may be dx.
 template <typename IT, typename RT, typename WT>
 __global__ __launch_bounds__(kSmallThreads)
 void dal_bwd_small_kernel(DalStreamArgs a) {
@@ -1161,11 +1162,16 @@ int hk_dropout_add_ln_bwd_ex(const hkDropoutAddLnBwdParams* pp, hkStream_t strea
     // 9.7, 256 x 4096 15.8 / 10.4, 768 x 2048 15.5 / 12.3, x 8192 36.6 / 29.6, 1024 x 512 12.5 / 10.8, x 8192 40.8 / 37.6, 1500 x 1024
     // 15.1 / 15.5, x 8192 53.6 / 51.6; fp32 256 x 8192 28.8 / 24.1, 768 x 1024 15.8 / 12.4, x 4096 31.2 / 28.9, x 6144 45.6 / 47.8, 1024 x
     // 2048 23.2 / 22.7, x 4096 38.7 / 39.0.
-    const int64_t n = p.rows * p.cols, ni = n * int64_t(sizeof(IT)), nr = n * int64_t(sizeof(RT));
-    if (stream_form && p.rows <= (sizeof(RT) == 2 ? 1024 : 768) && nr <= (int64_t(16) << 20) && tune_get(TUNE_NORM_BWD_BLOCKS) <= 0 && tune_get(TUNE_NORM_BWD_ROWS_PER_BLOCK) <= 0 &&
-        apart(p.dx0, ni, p.dz, ni) && apart(p.dx0, ni, p.x, nr) && apart(p.dresidual, nr, p.dz, ni) && apart(p.dresidual, nr, p.x, nr) &&
-        apart(p.dx0, ni, p.dx, nr) && apart(p.dgamma, p.cols * int64_t(sizeof(WT)), p.gamma, p.cols * int64_t(sizeof(WT))) &&
-        apart(p.dbeta, p.cols * int64_t(sizeof(WT)), p.gamma, p.cols * int64_t(sizeof(WT)))) {
+    const int64_t n = p.rows * p.cols, ni = n * int64_t(sizeof(IT)), nr = n * int64_t(sizeof(RT)), nw = p.cols * int64_t(sizeof(WT)),
+                  ns = p.rows * int64_t(sizeof(float));
+    const Span dz{p.dz, ni}, dx{p.dx, nr}, x{p.x, nr}, mask{p.dmask, n}, mu{p.mu, ns}, rs{p.rs, ns}, gamma{p.gamma, nw};
+    const Span dx0{p.dx0, ni}, dresidual{p.dresidual, nr}, dgamma{p.dgamma, nw}, dbeta{p.dbeta, nw};
+    // (dresidual may be dx: an element of it is read by the thread that stores it.  What two launches write over each other, the
+    // column sums win.)
+    const bool one_launch = apart({dx0, dgamma, dbeta}, {dz, dx, x, mask, mu, rs, gamma}) && apart({dresidual}, {dz, x, mask, mu, rs, gamma}) &&
+                            apart({dgamma, dbeta}, {dx0, dresidual});
+    if (stream_form && one_launch && p.rows <= (sizeof(RT) == 2 ? 1024 : 768) && nr <= (int64_t(16) << 20) &&
+        tune_get(TUNE_NORM_BWD_BLOCKS) <= 0 && tune_get(TUNE_NORM_BWD_ROWS_PER_BLOCK) <= 0) {
       const int lanes = sizeof(RT) == 2 ? 8 : 4, rpb = kSmallThreads / sh.tpr;
       DalStreamArgs few = f;
       few.part[0] = static_cast<float*>(p.dgamma);

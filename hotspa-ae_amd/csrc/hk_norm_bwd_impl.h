@@ -421,9 +421,9 @@ void norm_bwd_finalize_kernel(const float* part0, const float* part1, T* out0, T
 constexpr int small_lanes(bool ragged) { return ragged ? 4 : 8; }
 // The whole backward of a small array in one launch.  Its time is that of launches and trips to memory, of which the kernels above
 // take three (rows, partial rows, their fold), so here the first a.blocks workgroups form the column sums from the operands
-// themselves, LANES vectors of every row each, and the others dx: what is read twice comes from a cache.  dx must not lie over dy
-// or x (see column_sums_of_few_rows).  dx comes out to the same bits as from norm_bwd_kernel: the plan's threads and vectors, its
-// order of operations.
+// themselves, LANES vectors of every row each, and the others dx: what is read twice comes from a cache.  Nothing that
+// is written may lie over what is read (see column_sums_of_few_rows).  dx comes out to the same bits as from norm_bwd_kernel: the
+// plan's threads and vectors, its order of operations.
 template <typename T, int NV, int MODE, bool RAGGED>
 __global__ __launch_bounds__(kSmallThreads)
 void norm_bwd_small_kernel(NormBwdFlat given) {
@@ -936,9 +936,11 @@ static bool launch_norm_bwd_small(NormBwdArgs a, const BwdPlan& p, void* dgamma,
   const bool small = p.any ? a.rows <= 512 && a.rows * row_bytes <= (int64_t(8) << 20) : a.rows <= (row_bytes <= 1024 ? 1024 : 768);
   if (!small || p.lpr || p.nv > (VEC == 4 ? 2 : 1) || tune_get(TUNE_NORM_BWD_ROWS_PER_BLOCK) > 0 || tune_get(TUNE_NORM_BWD_BLOCKS) > 0 ||
       tune_get(TUNE_NORM_BWD_PREFETCH) > 0) return false;
-  const auto extent = [&](int64_t pitch) { return ((a.rows - 1) * pitch + a.cols) * int64_t(sizeof(T)); };
-  if (!apart(a.dx, extent(a.dx_pitch), a.dy, extent(a.dy_pitch)) || !apart(a.dx, extent(a.dx_pitch), a.x, extent(a.x_pitch)) ||
-      !apart(dgamma, row_bytes, a.gamma, row_bytes) || !apart(dbeta, row_bytes, a.gamma, row_bytes)) return false;
+  const auto rows_of = [&](const void* at, int64_t pitch) { return Span{at, ((a.rows - 1) * pitch + a.cols) * int64_t(sizeof(T))}; };
+  const Span dy = rows_of(a.dy, a.dy_pitch), x = rows_of(a.x, a.x_pitch), dx = rows_of(a.dx, a.dx_pitch), gamma{a.gamma, row_bytes};
+  const Span mean{a.mean, a.rows * int64_t(sizeof(float))}, stat{a.stat, mean.bytes}, dg{dgamma, row_bytes}, db{dbeta, row_bytes};
+  // (what two launches write over each other, the column sums win)
+  if (!apart({dx, dg, db}, {dy, x, gamma, mean, stat}) || !apart({dg, db}, {dx})) return false;
   const int nvec = (a.cols + VEC - 1) / VEC, lanes = small_lanes(p.any), rpb = kSmallThreads / p.tpr;
   a.tpr = p.tpr;
   a.threads = kSmallThreads;

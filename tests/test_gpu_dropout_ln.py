@@ -436,3 +436,50 @@ def test_block_backward_of_few_rows(hk, cuda, combo, is_rms):
         for got in (dg, over[3]):
             helpers.assert_close(got, edg, wt, "dgamma " + what, scale=many)
         helpers.assert_close(db, edb, wt, "dbeta " + what, scale=many)
+
+
+@pytest.mark.parametrize("combo", [("fp32", "fp32", "fp32"), ("bf16", "bf16", "bf16"), ("fp16", "fp32", "fp32")],
+                         ids=lambda c: "w%s-i%s-r%s" % c)
+def test_block_backward_of_few_rows_column_sums_over_operands(hk, cuda, combo):
+    """dgamma or dbeta in the memory of an input or of another gradient: they are stored when every row has been read and every
+    other gradient written."""
+    import torch
+    wt, it, rt = combo
+    for rows, cols in [(1, 64), (8, 8192), (300, 64), (512, 1032), (768, 256)]:
+        x, dx_in, dz = helpers.draw(81, (rows, cols), dtype=rt), helpers.draw(82, (rows, cols), dtype=rt), helpers.draw(83, (rows, cols), dtype=it)
+        gamma = helpers.draw(84, (cols,), "uniform", 0.5, 1.5, wt)
+        mask = _mask(rows * cols, 0.3).reshape(rows, cols)
+        xd = x.astype(np.float64)
+        mean = xd.mean(-1).astype(np.float32)
+        rs = (1.0 / np.sqrt(np.square(xd - mean[:, None]).mean(-1) + 1e-2)).astype(np.float32)
+        _, _, edg, edb, _ = dal.bwd(dz, dx_in, x, None, mask, mean, rs, gamma, None, None, dropout_p=0.3, is_rms=False)
+        tg = _tt(gamma, wt, cuda)
+        want = {"dz": _tt(dz, it, cuda), "x": _tt(x, rt, cuda), "dx": _tt(dx_in, rt, cuda), "mask": _tt(mask, "uint8", cuda),
+                "mu": _tt(mean, "fp32", cuda), "rs": _tt(rs, "fp32", cuda)}
+
+        def run(t, dg, db):
+            hk.dropout_add_ln_bwd_ex(t["dz"], t["x"], t["mu"], t["rs"], tg, t["dx0"], dx=t["dx"], dmask=t["mask"],
+                                     dresidual=t["dresidual"], dgamma=dg, dbeta=db, dropout_p=0.3, is_rms=False)
+        want["dx0"], want["dresidual"] = torch.empty_like(want["dz"]), torch.empty_like(want["x"])
+        run(want, torch.empty_like(tg), torch.empty_like(tg))
+        many = float(np.sqrt(rows))   # column sums over `rows` terms: their rounding error is that of the terms
+        for over in want:
+            if want[over].numel() * want[over].element_size() < cols * tg.element_size():
+                continue
+            for which in (0, 1):
+                for last in (False, True):
+                    t = {k: v.clone() for k, v in want.items()}
+                    memory = t[over].view(-1).view(tg.dtype)
+                    sums = [torch.empty_like(tg), torch.empty_like(tg)]
+                    sums[which] = memory[memory.numel() - cols:] if last else memory[:cols]
+                    t["dx0"].view(-1)[0] = t["dresidual"].view(-1)[0] = -77.0
+                    run(t, *sums)
+                    what = "%s over %s, %d x %d" % (("dgamma", "dbeta")[which], over, rows, cols)
+                    helpers.assert_close(sums[0], edg, wt, "dgamma " + what, scale=many)
+                    helpers.assert_close(sums[1], edb, wt, "dbeta " + what, scale=many)
+                    for k in ("dx0", "dresidual"):
+                        got, expected = t[k].view(-1), want[k].view(-1)
+                        if k == over:   # all but the memory of the sums
+                            n = cols * tg.element_size() // got.element_size()
+                            got, expected = (got[:-n], expected[:-n]) if last else (got[n:], expected[n:])
+                        assert torch.equal(got, expected), what

@@ -224,6 +224,47 @@ def test_bwd_of_few_rows(hk, cuda, dtype, is_rms):
             helpers.assert_close(tdb, edb, dtype, "dbeta " + what, scale=many)
 
 
+@pytest.mark.parametrize("dtype", ["fp32", "bf16", "fp16"])
+@pytest.mark.parametrize("is_rms", [True, False])
+def test_bwd_of_few_rows_column_sums_over_operands(hk, cuda, dtype, is_rms):
+    """dgamma or dbeta in the memory of dy, x, the statistics or dx: they are stored when every row has been read and every dx
+    written."""
+    import torch
+    for rows, cols in [(1, 64), (1, 1021), (7, 8192), (300, 64), (257, 37), (512, 1024), (511, 1021)]:
+        x, gamma, _, dz = _inputs(rows, cols, dtype, 6200 + cols + rows)
+        mean = np.zeros(rows, np.float32) if is_rms else x.astype(np.float64).mean(-1).astype(np.float32)
+        rs = (1.0 / np.sqrt(np.square(x.astype(np.float64) - mean[:, None]).mean(-1) + 1e-2)).astype(np.float32)
+        tg = helpers.to_torch(gamma, dtype, cuda)
+        given = {"x": (x, dtype), "dy": (dz, dtype), "mean": (mean, "fp32"), "stat": (rs, "fp32")}
+        want = {k: helpers.to_torch(v, d, cuda) for k, (v, d) in given.items()}
+        edx = torch.empty_like(want["x"])
+        hk.dropout_add_ln_bwd(want["dy"], None, want["x"], want["mean"], want["stat"], tg, edx, None, torch.empty_like(tg),
+                              None if is_rms else torch.empty_like(tg), is_rms)
+        _, edg, edb = oracle.dropout_add_ln_bwd(dz, None, x, mean, rs, gamma, is_rms)
+        many = float(np.sqrt(rows))   # column sums over `rows` terms: their rounding error is that of the terms
+        for over in ("dy", "x", "mean", "stat", "dx"):
+            for which in ("dgamma",) if is_rms else ("dgamma", "dbeta"):
+                t = {k: v.clone() for k, v in want.items()}
+                t["dx"] = torch.empty_like(edx)
+                if t[over].numel() * t[over].element_size() < cols * tg.element_size():
+                    continue
+                for last in (False, True):
+                    for k, v in want.items():
+                        t[k].copy_(v)
+                    memory = t[over].view(-1).view(tg.dtype)
+                    sums = {"dgamma": torch.empty_like(tg), "dbeta": None if is_rms else torch.empty_like(tg)}
+                    sums[which] = memory[memory.numel() - cols:] if last else memory[:cols]
+                    hk.dropout_add_ln_bwd(t["dy"], None, t["x"], t["mean"], t["stat"], tg, t["dx"], None, sums["dgamma"],
+                                          sums["dbeta"], is_rms)
+                    what = "%s over %s, %d x %d" % (which, over, rows, cols)
+                    helpers.assert_close(sums["dgamma"], edg, dtype, "dgamma " + what, scale=many)
+                    if not is_rms:
+                        helpers.assert_close(sums["dbeta"], edb, dtype, "dbeta " + what, scale=many)
+                    dx, kept = t["dx"].view(-1), edx.numel() - (cols if over == "dx" else 0)
+                    at = cols if over == "dx" and not last else 0
+                    assert torch.equal(dx[at:at + kept], edx.view(-1)[at:at + kept]), what
+
+
 def test_rmsnorm_bwd_identity(hk, cuda):
     """sum_cols dx*x = eps * rs^3 * sum_cols (gamma*dz)*x per row: pins where eps sits."""
     import torch
