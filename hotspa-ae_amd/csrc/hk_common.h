@@ -357,9 +357,12 @@ struct RowNumbering {
   int64_t rn0, rn1, rn2;
 };
 // offset of this workgroup's rows along the two outer walk levels, in elements
-template <typename L>
-__device__ __forceinline__ int64_t outer_level_offset(const L& l) {
+__device__ __forceinline__ int64_t outer_level_offset(const LevelSteps& l) {
   return int64_t(blockIdx.y) * l.p1 + int64_t(blockIdx.z) * l.p2;
+}
+// (both factors 32 bits of one kind: two multiplications, where a sign extended to 64 bits makes it five instructions)
+__device__ __forceinline__ int64_t outer_level_offset(const ShortLevelSteps& l) {
+  return int64_t(int(blockIdx.y)) * l.p1 + int64_t(int(blockIdx.z)) * l.p2;
 }
 // number of the row (j0, blockIdx.y, blockIdx.z)
 __device__ __forceinline__ int64_t dense_row_index(int64_t j0, const RowNumbering& rn) {
