@@ -165,6 +165,10 @@ __device__ __forceinline__ ACC block_reduce_lds(ACC v, ACC* lds) {
 // partial vector's selects, and a wavefront's row its width at compile time (loads off one address).  GPU time alone,
 // fp32, without / with all of it: 16384 x 1000 20.2 / 10.4 us, 16384 x 1021 20.2 / 11.0, 8192 x 1024 11.3 / 6.0 (6.2 TB/s),
 // 524288 x 64 42.2 / 20.5; bf16: 16384 x 1000 7.7 / 6.7, 524288 x 64 13.4 / 11.8.
+// LARGE: the workgroup's width is read from the launch's own dimensions.  Small calls take the host's time and go without, in fewer
+// arguments (see kCheapArgs: axes (0, 2) of [32, 64, 1024] bf16 4.2 us, 4.6 with).  Calls that wait for the device measured faster with
+// them, one after another: [64, 256, 3136] 16.98 us, 17.15 without (the same instructions, 96 bytes of arguments instead of 352),
+// [32, 512, 784] 5.98 / 6.07; last axis of [4, 64, 65536] 6.65 / 6.73, of [33, 116, 4336] 7.21 / 7.42, of [50, 716, 1272] 14.8 / 15.05.
 // ---------------------------------------------------------------------------
 struct InnerArgs {
   const void* in;
@@ -197,7 +201,7 @@ __device__ __forceinline__ float lanes_reduce(float v, int lanes) {
 // one run of whole vectors in rows on one level, one run of any length, several of any length
 enum InnerRow { ROW_WHOLE, ROW_RAGGED, ROW_RUNS };
 
-template <typename T, typename OUT_T, bool LANES, InnerRow ROW, typename R, bool WAVE = false>
+template <typename T, typename OUT_T, bool LANES, InnerRow ROW, typename R, bool WAVE = false, bool LARGE = false>
 __global__ __launch_bounds__(LANES ? 256 : 1024, 8)
 void reduce_inner_vec_kernel(InnerArgs a) {
   constexpr bool RUNS = ROW == ROW_RUNS, WHOLE = ROW == ROW_WHOLE;
@@ -205,11 +209,12 @@ void reduce_inner_vec_kernel(InnerArgs a) {
   constexpr int VEC = VecIO<T>::N;
   constexpr int U = 8;
   __shared__ float red[kMaxWaves];
-  const int tpr = WAVE ? kWave : a.lanes;
+  const int width = LARGE ? int(blockDim.x) : LANES ? 256 : a.lanes;   // of the workgroup
+  const int tpr = WAVE ? kWave : LANES ? a.lanes : width;
   const int t = LANES ? int(threadIdx.x) & (tpr - 1) : int(threadIdx.x);
   const int64_t row = !LANES ? int64_t(blockIdx.x)
-                    : tpr == kWave ? int64_t(blockIdx.x) * (256 / kWave) + wave_index()
-                                   : (int64_t(blockIdx.x) * 256 + threadIdx.x) >> __builtin_ctz(tpr);
+                    : tpr == kWave ? int64_t(blockIdx.x) * (width >> 6) + wave_index()
+                                   : (int64_t(blockIdx.x) * width + threadIdx.x) >> __builtin_ctz(tpr);
   if (LANES && row >= a.rows) return;   // whole groups of lanes leave
   const int split = blockIdx.y;
   int64_t base = row * a.row_stride;
@@ -797,10 +802,20 @@ static int launch_inner(const ReducePlan& p, const InnerShape& s, const void* in
   const bool lanes = s.tpr <= kWave;
   const int64_t groups = lanes ? (p.rows * s.tpr + 255) / 256 : p.rows;
   dim3 grid(unsigned(groups), unsigned(s.nsplit)), block(lanes ? 256u : unsigned(s.tpr));
-  auto kernel = p.nruns > 1 ? (lanes ? reduce_inner_vec_kernel<T, OUT_T, true, ROW_RUNS, R> : reduce_inner_vec_kernel<T, OUT_T, false, ROW_RUNS, R>)
-      : p.cols % VecIO<T>::N || p.level_rows != p.rows ? (lanes ? reduce_inner_vec_kernel<T, OUT_T, true, ROW_RAGGED, R> : reduce_inner_vec_kernel<T, OUT_T, false, ROW_RAGGED, R>)
-      : s.tpr == kWave ? reduce_inner_vec_kernel<T, OUT_T, true, ROW_WHOLE, R, true>
-                       : (lanes ? reduce_inner_vec_kernel<T, OUT_T, true, ROW_WHOLE, R> : reduce_inner_vec_kernel<T, OUT_T, false, ROW_WHOLE, R>);
+  // 24 MiB take the device 5.5 us, more than the host needs for a launch
+  const bool large = p.rows * p.nruns * p.cols * int64_t(sizeof(T)) >= int64_t(24) << 20;
+  auto workgroup = [&](auto row) {
+    constexpr InnerRow ROW = decltype(row)::value;
+    return large ? reduce_inner_vec_kernel<T, OUT_T, false, ROW, R, false, true> : reduce_inner_vec_kernel<T, OUT_T, false, ROW, R>;
+  };
+  constexpr std::integral_constant<InnerRow, ROW_RUNS> runs;
+  constexpr std::integral_constant<InnerRow, ROW_RAGGED> ragged;
+  constexpr std::integral_constant<InnerRow, ROW_WHOLE> whole;
+  auto kernel = p.nruns > 1 ? (lanes ? reduce_inner_vec_kernel<T, OUT_T, true, ROW_RUNS, R> : workgroup(runs))
+      : p.cols % VecIO<T>::N || p.level_rows != p.rows ? (lanes ? reduce_inner_vec_kernel<T, OUT_T, true, ROW_RAGGED, R> : workgroup(ragged))
+      : s.tpr == kWave ? (large ? reduce_inner_vec_kernel<T, OUT_T, true, ROW_WHOLE, R, true, true>
+                                : reduce_inner_vec_kernel<T, OUT_T, true, ROW_WHOLE, R, true>)
+                       : (lanes ? reduce_inner_vec_kernel<T, OUT_T, true, ROW_WHOLE, R> : workgroup(whole));
   profile_before(st);
   HK_LAUNCH(kernel, grid, block, 0, st, a);
   profile_after(st);

@@ -325,3 +325,23 @@ def test_long_rows_take_more_than_a_wavefront(hk, cuda):
         finally:
             hk.tune_set("reduce_inner_threads", 0)
     assert times[0] < 0.95 * times[64], times
+
+
+@pytest.mark.parametrize("dtype,shape,axes", [
+    ("bf16", (12, 256, 4096), [0, 2]), ("bf16", (12, 256, 4095), [0, 2]), ("fp32", (6, 256, 4100), [0, 2]), ("fp32", (2, 3071, 1024), [0, 2]),
+    ("fp16", (24, 1031, 520), [0, 2]), ("bf16", (3072, 4096), [1]), ("bf16", (3071, 4096), [1]), ("fp32", (1537, 4096), [1]),
+    ("fp16", (24577, 520), [1])])
+def test_rows_of_large_arrays(hk, cuda, dtype, shape, axes):
+    """Both sides of the 24 MiB from which on the width comes with the launch: whole numbers, whose sums are exact in fp32."""
+    import torch
+    tt = {"fp32": torch.float32, "bf16": torch.bfloat16, "fp16": torch.float16}[dtype]
+    g = torch.Generator(device=cuda).manual_seed(sum(shape))
+    x = torch.randint(-3, 4, shape, generator=g, device=cuda).to(tt)
+    kept = [n for i, n in enumerate(shape) if i not in axes]
+    ws = torch.empty(hk.reduce_workspace_bytes(hk.dtype_code(x), list(shape), list(x.stride()), axes) // 4 + 1, device=cuda)
+    out = torch.empty(kept, dtype=torch.float32, device=cuda)
+    hk.reduce(x, out, axes, "sum", workspace=ws)
+    assert torch.equal(out.double(), x.double().sum(axes))
+    most = torch.empty(kept, dtype=tt, device=cuda)
+    hk.reduce(x, most, axes, "max", workspace=ws)
+    assert torch.equal(most, x.amax(axes))
