@@ -793,13 +793,19 @@ static int softmax_strided_typed(const void* x, const void* dy, void* out, int64
       }
       a.slices = int((dim + nk - 1) / nk);
       if (a.total <= 0x7fffffffLL) {
-        // fp32 planes that fill the device many times over take longer runs, which share fewer lines: 9 to 32 entries, on planes of
-        // whole lines 24, two slices of 128 lanes (slices of up to 8 entries of 64 lanes / of 128 forward and 256 backward / so: 8 x 21 x 263169 forward 71.8 / 69.7 / 66.1,
-        // backward 106 / 96.6 / 94.5 us; 8 x 21 x 263168 62.7 / - / 61.7 and 95.6 / - / 89.1, 2 x 30 x 1000001 forward - / 98.7 / 94.4, 4 x 17 x
-        // 400003 backward - / 64.6 / 60.1, but 128 x 32 x 16384 87 / - / 89 and 129 / - / 134), fewer entries one slice of 128 forward, 256 backward where planes share lines.  Runs of 64 lanes
-        // are as good on planes of whole lines (16 x 2 x 1048576 42.3 / 44.3 and 60.9 / 62.7 us) and better for 16-bit entries
-        // (8 x 21 x 263169 35.3 / 37.8 / 48.1 and 50.3 / 51.0 / 55.8).
-        const bool wide = VEC == 4 && dim <= (odd ? 32 : 24) && a.total >= cus * 2048 && (odd || dim > kDimVecs);
+        // fp32 planes that fill the device many times over take longer runs, which share fewer lines: 9 to 24 entries, on odd planes
+        // of 256 KiB 32, two slices of 128 lanes; fewer one of 128 forward, 256 backward on odd planes.  Time of slices of up to 8
+        // entries of 64 lanes over that of the two, forward and backward, geometric means of 9 to 24 entries: odd planes of 5001
+        // to 263169, by vectors per compute unit, 300 0.94 and 0.93, 500 0.99 and 1.00, 780 1.00 and 1.00, 1030 to 1170 1.02 and 1.03, 1550 1.03 and
+        // 1.05, 2100 1.03 and 1.06, 7800 1.05 and 1.10; planes of whole lines 1030 to 1150 0.99 and 1.00, 1550 1.00 and 1.01, 2100 1.00 and 1.02,
+        // 4700 1.01 and 1.02.  28 and 32 entries: odd planes of 5001 at 2100 0.96 and 0.98, of 20001 at 1130 1.00 and 0.99, 2100 0.98 and
+        // 0.99, of 100003 at 780 0.99 and 0.99, 1170 1.00 and 1.00, 2100 1.01 and 1.02, of 263169 at 1030 1.07 and 1.07, 2100 1.11 and 1.12; whole
+        // lines, 128 x 32 x 16384, 0.98 and 0.96.
+        // Runs of 64 lanes are as good for few entries on planes of whole lines (16 x 2 x 1048576 42.3 / 44.3 and 60.9 / 62.7 us) and
+        // better for 16-bit entries (8 x 21 x 263169 35.3 / 37.8 / 48.1 and 50.3 / 51.0 / 55.8).
+        const bool wide = VEC == 4 && (dim <= kDimVecs ? odd && a.total >= cus * 2048
+                                       : dim <= 24     ? a.total >= cus * (odd ? 1024 : 2048)
+                                                       : dim <= 32 && odd && bytes >= (256 << 10) && a.total >= cus * 1024);
         if (wide && dim > kDimVecs) { nk = int((dim + 1) / 2); a.slices = 2; }
         // PLAIN: stored through the cache, where lines that two workgroups share meet.  Larger arrays and planes of whole lines are
         // streamed (streamed / so, bf16 forward: 60 x 5 x 263169 56.9 / 58.7, 413 x 5 x 12101 20.9 / 19.8, 1322 x 5 x 12101 61.1 / 63.5,

@@ -190,3 +190,11 @@ def test_dimension_shapes(hk, cuda, dtype, shape):
     assert bool(((y.double() - ey).abs() <= ulp * ey + tiny).all()), shape
     size = s * (d.abs() + (s * d.abs()).sum(1, keepdim=True))
     assert bool(((dx.double() - edx).abs() <= ulp * edx.abs() + 2.0 ** -19 * size + tiny).all()), shape
+
+
+@pytest.mark.parametrize("dtype,shape", [
+    # fp32 in two slices of 128 lanes: the edges of the planes' length and of the vectors per compute unit
+    ("fp32", (105, 21, 10001)), ("fp32", (104, 9, 10001)), ("fp32", (4, 24, 262145)), ("fp32", (4, 32, 262145)), ("fp32", (5, 25, 209713)),
+    ("fp32", (4, 26, 262144)), ("fp32", (16, 28, 65533))])
+def test_dimension_shapes_at_the_edges_of_the_rules(hk, cuda, dtype, shape):
+    test_dimension_shapes(hk, cuda, dtype, shape)
