@@ -195,6 +195,9 @@ def test_dimension_shapes(hk, cuda, dtype, shape):
 @pytest.mark.parametrize("dtype,shape", [
     # fp32 in two slices of 128 lanes: the edges of the planes' length and of the vectors per compute unit
     ("fp32", (105, 21, 10001)), ("fp32", (104, 9, 10001)), ("fp32", (4, 24, 262145)), ("fp32", (4, 32, 262145)), ("fp32", (5, 25, 209713)),
-    ("fp32", (4, 26, 262144)), ("fp32", (16, 28, 65533))])
+    ("fp32", (4, 26, 262144)), ("fp32", (16, 28, 65533)),
+    # 16 bits: what is streamed and what is stored through the cache, on both sides of 24, 32, 48 and 64 MiB
+    ("bf16", (37, 24, 18999)), ("fp16", (46, 40, 18999)), ("bf16", (16, 56, 15001)), ("bf16", (20, 64, 14001)), ("bf16", (14, 128, 15001)),
+    ("fp16", (12, 176, 14001)), ("bf16", (14, 250, 8001)), ("bf16", (8, 90, 14400)), ("bf16", (16, 90, 14400)), ("bf16", (6, 200, 14001))])
 def test_dimension_shapes_at_the_edges_of_the_rules(hk, cuda, dtype, shape):
     test_dimension_shapes(hk, cuda, dtype, shape)
