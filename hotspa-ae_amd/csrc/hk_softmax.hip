@@ -692,11 +692,14 @@ static int softmax_lastdim_typed(SoftmaxRows a, hipStream_t s) {
   }
 }
 
-// FEW: up to kFewSlices slices.  MAXT: the most threads that its plans have.  LEAST, MOST:
-// the entries per lane that they give (of 16-bit types from 8 on even numbers).  LEAST_AGAIN: from how many on AGAIN; 14 backward just fit without
+// FEW: up to kFewSlices slices.  MAXT: the most threads that its plans have.  LEAST, MOST: the entries per lane that they give (of
+// 16-bit types from 8 on even numbers, backward 14 and 16).  LEAST_AGAIN: from how many on AGAIN; 14 backward just fit without
 template <typename T, bool BWD, int LX, bool PLAIN, bool FEW, int MAXT, int LEAST, int MOST, int LEAST_AGAIN = 17>
 static int launch_softmax_dim(SoftmaxDimArgs a, int nk, hipStream_t s) {
-  if (nk < LEAST || nk > MOST || (nk > kDimVecs && nk % 2 != 0 && VecIO<T>::N == 8) || a.slices * LX > MAXT) {
+  const auto built = [](int n) {
+    return n >= LEAST && n <= MOST && (n <= kDimVecs || VecIO<T>::N == 4 || (n % 2 == 0 && (!BWD || n >= 14)));
+  };
+  if (!built(nk) || a.slices * LX > MAXT) {
     set_last_error("softmax: no kernel for %d entries per lane", nk);
     return HK_ERR_UNSUPPORTED;
   }
@@ -705,7 +708,7 @@ static int launch_softmax_dim(SoftmaxDimArgs a, int nk, hipStream_t s) {
   const size_t lds = a.slices > 1 ? share_floats<VecIO<T>::N, LX, FEW, BWD>(a.slices) * sizeof(float) : 0;
 #define HK_DIM_CASE(NK)                                                             \
   case NK:                                                                          \
-    if constexpr (NK >= LEAST && NK <= MOST && (NK <= kDimVecs || NK % 2 == 0 || VecIO<T>::N == 4)) { \
+    if constexpr (built(NK)) {                                                      \
       constexpr bool AGAIN = NK >= LEAST_AGAIN && !(BWD && NK == 14);               \
       if constexpr (BWD) HK_LAUNCH((softmax_bwd_dim_kernel<T, NK, LX, PLAIN, FEW, MAXT, AGAIN>), grid, block, lds, s, a); \
       else HK_LAUNCH((softmax_fwd_dim_kernel<T, NK, LX, PLAIN, FEW, MAXT, AGAIN>), grid, block, lds, s, a); \
@@ -831,9 +834,13 @@ static int softmax_strided_typed(const void* x, const void* dy, void* out, int64
         // slices) forward 8.3 / 7.2, 32 x 12 x 40000 11.7 / 11.1, 4 x 5 x 5904 (3) 3.7 / 3.0, 32 x 40 x 6401 (5) 10.4 / 10.2, 4 x 12 x 5904 (6) 3.6 /
         // 3.35, 16 x 60 x 30001 (8) 25.9 / 27.3.
         // What nk can be.  64 slices: 2 to 4, for 65 to 256 entries.  The few in 32: up to 6, because at 192 entries and past 16
-        // vectors per compute unit they are no longer few; 1 or 2 in few slices.  32 slices of a quarter's run: 6 to 8, as in 32 of half one.  fp32 in more than six
-        // slices of 64 lanes: 7 or 8; the 16-bit backward of 37 to 48 entries on odd planes: 5 or 6.
-        constexpr int kLeast = BWD ? 4 : 5, kLeastAgain = BWD ? 7 : 12;
+        // vectors per compute unit they are no longer few; 1 or 2 in few slices.  32 slices of a quarter's run: 6 to 8; of half
+        // one 8, in the 16-bit backward 6.  16 of half one: forward 6 to 16, backward 4 to 8, 14 and 16.  fp32 in more than
+        // six slices of 64 lanes: 7 or 8; the 16-bit backward of 37 to 48 entries on odd planes: 6.  Of those in few slices
+        // through the cache, the 16-bit backward's are on odd planes or small, the fp32 forward's of 24 MiB and more in less
+        // than 2048 vectors per compute unit.
+        constexpr int kLeastPlain = VEC == 4 && !BWD ? 3 : 1, kMostPlain = VEC == 8 && BWD ? 6 : kDimVecs;
+        constexpr int kLeast = BWD ? 4 : 6, kLeastAgain = BWD ? 7 : 12;
         if (few) {
           if (lx == 16) return launch_softmax_dim<T, BWD, 16, true, false, 1024, 2, 4>(a, nk, s);
           if (a.slices <= kFewSlices) return launch_softmax_dim<T, BWD, 32, true, true, 1024, 1, 2>(a, nk, s);
@@ -842,8 +849,12 @@ static int softmax_strided_typed(const void* x, const void* dy, void* out, int64
         if constexpr (VEC == 8 && !BWD) {
           if (quarter) return launch_softmax_dim<T, BWD, 16, false, false, 512, 6, 8>(a, nk, s);
         }
-        if (tall && plain) return launch_softmax_dim<T, BWD, 32, true, false, 1024, 6, kDimVecs>(a, nk, s);
-        if (tall) return launch_softmax_dim<T, BWD, 32, false, false, 1024, 6, kDimVecs>(a, nk, s);
+        if constexpr (VEC == 4) {
+          if (tall && plain) return launch_softmax_dim<T, BWD, 32, true, false, 1024, kDimVecs, kDimVecs>(a, nk, s);
+          if (tall) return launch_softmax_dim<T, BWD, 32, false, false, 1024, kDimVecs, kDimVecs>(a, nk, s);
+        } else if constexpr (BWD) {
+          if (tall) return launch_softmax_dim<T, BWD, 32, false, false, 1024, 6, 6>(a, nk, s);
+        }
         if constexpr (BWD && VEC == 8) {
           // (24 MB / 64 MB of 128 entries 16.6 / 35.9 formed again, 15.4 / 36.8 kept; 160 MB 81.5 / 87.4)
           if (many && nk <= kDimVecs && array < (int64_t(48) << 20)) {
@@ -861,10 +872,10 @@ static int softmax_strided_typed(const void* x, const void* dy, void* out, int64
           if (a.slices > kFewSlices) return launch_softmax_dim<T, BWD, 64, false, false, 1024, kDimVecs - 1, kDimVecs>(a, nk, s);
         }
         if constexpr (VEC == 8 && BWD) {
-          if (a.slices > kFewSlices && plain) return launch_softmax_dim<T, BWD, 64, true, false, 512, 5, 6>(a, nk, s);
-          if (a.slices > kFewSlices) return launch_softmax_dim<T, BWD, 64, false, false, 512, 5, 6>(a, nk, s);
+          if (a.slices > kFewSlices && plain) return launch_softmax_dim<T, BWD, 64, true, false, 512, 6, 6>(a, nk, s);
+          if (a.slices > kFewSlices) return launch_softmax_dim<T, BWD, 64, false, false, 512, 6, 6>(a, nk, s);
         }
-        if (plain) return launch_softmax_dim<T, BWD, 64, true, true, 512, 1, kDimVecs>(a, nk, s);
+        if (plain) return launch_softmax_dim<T, BWD, 64, true, true, 512, kLeastPlain, kMostPlain>(a, nk, s);
         return launch_softmax_dim<T, BWD, 64, false, true, 512, 1, kDimVecs>(a, nk, s);
       }
     }
