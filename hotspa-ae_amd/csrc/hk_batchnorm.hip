@@ -690,11 +690,19 @@ static BnPlan<IT> bn_plan(int64_t N, int64_t C, int64_t HW, int max_splits, int 
     // one vector a thread while there are fewer channels than two workgroups per compute unit, else two at least
     if (total > int64_t(nv) * 1024 || (nv == 1 && total > 64 && C > 2 * device_cu_count())) continue;
     // and twice the fewest where not all channels run at once so and more of them do then, backward as many (forward and backward, us,
-    // fewest / twice: 64 x 600 x 196 bf16 25.0 / 21.5, 10 x 900 x 1024 24.7 / 20.4, 30 x 999 x 441 39.8 / 33.8, backward as it was 35.4, 40 x
+    // fewest / twice: 64 x 600 x 196 bf16 25.4 / 22.2, 10 x 900 x 1024 24.7 / 20.4, 30 x 999 x 441 39.8 / 33.8, backward as it was 35.4, 40 x
     // 1000 x 144 fp32 27.3 / 22.6; where all run at once or no more do, 2 x 600 x 3000 fp16 12.2 / 12.65, 100 x 1024 x 49 20.1 / 20.6, 38 x
     // 587 x 576, forward, of 33.7 both ways, 2.5 more)
     const bool more = max_nv == 4 ? at_once(2 * nv) >= at_once(nv) : at_once(2 * nv) > at_once(nv);
-    if (2 * nv <= max_nv && C > cus * at_once(nv) && more) nv *= 2;
+    // the 16-bit backward of two vectors: not in every width.  Fewest / twice, by wavefronts of the fewest, 800 channels of planes off
+    // the vectors' boundaries and on them: 9 20 x 413 13.0 / 13.8 and 4 x 2064 10.1 / 10.5, 10 20 x 477 14.7 / 14.5 and 4 x 2400 11.5 / 11.05, 11
+    // 20 x 533 15.8 / 17.3 and 4 x 2680 12.4 / 13.3, 12 20 x 573 17.0 / 18.0 and 4 x 2896 13.3 / 14.2, 15 20 x 717 20.4 / 21.3 and 4 x 3600 15.9 /
+    // 16.1, 16 20 x 757 21.35 / 22.4; 13 20 x 621 18.15 / 18.95, of 1000 channels 22.7 / 21.0; 64 x 196 of 768, 860 and 1024 14.2 / 14.75, 19.5 / 17.8
+    // and 20.3 / 19.5, 14 30 x 441 17.4 / 17.5, 21.0 / 20.5 and 25.0 / 22.7
+    const int waves = int(((total + nv - 1) / nv + 63) / 64);
+    const bool pays = max_nv != 4 || VEC != 8 || nv != 2 || waves <= 8 || waves == 10 ||
+                      ((waves == 13 || waves == 14) && 4 * C > 13 * cus);
+    if (2 * nv <= max_nv && C > cus * at_once(nv) && more && pays) nv *= 2;
     b.form = 1;
     b.nv = nv;
     b.threads = int(((total + nv - 1) / nv + 63) / 64 * 64);

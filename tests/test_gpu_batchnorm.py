@@ -260,3 +260,9 @@ def test_many_channels(hk, cuda, dtype, shape):
     edx = k * (gd - v(sdy / m) - xhat * v(sdyx / m))
     size = k * (gd.abs() + v(gd.abs().mean((0, 2))) + (xhat.abs() + v(mu * istd)) * v((gd * xhat).abs().mean((0, 2))))
     assert bool(((dx.double() - edx).abs() <= ulp * edx.abs() + 2.0 ** -20 * size + tiny).all())
+
+
+@pytest.mark.parametrize("shape", [(4, 800, 2300), (4, 800, 2310), (20, 800, 533), (20, 833, 621), (20, 832, 621), (4, 900, 3584), (4, 900, 3592)])
+def test_many_channels_of_two_or_four_vectors_a_thread(hk, cuda, shape):
+    """16-bit backward: both sides of the widths that take four."""
+    test_many_channels(hk, cuda, "bf16", shape)
