@@ -953,20 +953,20 @@ template <typename T, int MODE>
 static int sce_typed(SceArgs a, hipStream_t s) {
   constexpr int VEC = VecIO<T>::N;
   constexpr bool BWD = (MODE & 1) != 0;
-  const bool far0 = far_level(a.n0, {a.x_pitch, MODE < 2 ? 0 : a.lab_pitch, BWD ? a.out_pitch : 0}),
-             far1 = far_level(a.n1, {a.x_lv.p1, BWD ? a.out_lv.p1 : 0}), far2 = far_level(a.n2, {a.x_lv.p2, BWD ? a.out_lv.p2 : 0});
-  if (far0 || far1 || far2) {
-    return each_near_part(a, far0, far1, far2, [&](SceArgs part, int64_t i, int64_t j, int64_t k) {
-      const auto at = [&](int64_t pitch, const LevelSteps& l) { return i * pitch + j * l.p1 + k * l.p2; };
-      const int64_t number = i * a.rn.rn0 + j * a.rn.rn1 + k * a.rn.rn2;
-      part.logits = static_cast<const T*>(a.logits) + at(a.x_pitch, a.x_lv);
-      if constexpr (MODE < 2) part.labels = a.labels + number;
-      else part.dlabels = static_cast<const T*>(a.dlabels) + at(a.lab_pitch, a.lab_lv);
-      if (BWD && !a.grad_scalar) part.grad_loss = static_cast<const T*>(a.grad_loss) + number;
-      part.out = static_cast<T*>(a.out) + (BWD ? at(a.out_pitch, a.out_lv) : number);
-      if (a.stats) part.stats = a.stats + number;
-      return sce_typed<T, MODE>(part, s);
-    });
+  if constexpr (MODE < 2) {   // (dense labels, a reduced loss and the statistics of a shard come with rows side by side)
+    const bool far0 = far_level(a.n0, {a.x_pitch, BWD ? a.out_pitch : 0}), far1 = far_level(a.n1, {a.x_lv.p1, BWD ? a.out_lv.p1 : 0}),
+               far2 = far_level(a.n2, {a.x_lv.p2, BWD ? a.out_lv.p2 : 0});
+    if (far0 || far1 || far2) {
+      return each_near_part(a, far0, far1, far2, [&](SceArgs part, int64_t i, int64_t j, int64_t k) {
+        const auto at = [&](int64_t pitch, const LevelSteps& l) { return i * pitch + j * l.p1 + k * l.p2; };
+        const int64_t number = i * a.rn.rn0 + j * a.rn.rn1 + k * a.rn.rn2;
+        part.logits = static_cast<const T*>(a.logits) + at(a.x_pitch, a.x_lv);
+        part.labels = a.labels + number;
+        if (BWD) part.grad_loss = static_cast<const T*>(a.grad_loss) + number;
+        part.out = static_cast<T*>(a.out) + (BWD ? at(a.out_pitch, a.out_lv) : number);
+        return sce_typed<T, MODE>(part, s);
+      });
+    }
   }
   auto steps_ok = [](int64_t pitch, const LevelSteps& l) { return pitch % VEC == 0 && l.p1 % VEC == 0 && l.p2 % VEC == 0; };
   const bool vec_ok = a.cols % VEC == 0 && aligned16(a.logits) && aligned16(a.dlabels) &&

@@ -352,3 +352,33 @@ def test_cross_entropy_rows_2_31_elements_apart(hk, cuda):
         hk.sce_sparse_fwd(fx, labels, floss, -100)
         hk.sce_sparse_bwd(fx, labels, dloss, fdx, -100)
         assert torch.equal(floss, loss) and torch.equal(fdx, dx), shape
+
+
+def test_gradients_of_rows_2_31_elements_apart(hk, cuda):
+    """Gradients that are written so far apart, on one level and as one of three, against the same side by side; logits beside them
+    or as far apart in another order."""
+    import torch
+    cols, far = 200, (1 << 31) + 8
+    room = 3 * 5 * cols
+    base = torch.empty(far + 2 * room, dtype=torch.bfloat16, device=cuda)
+    for shape, strides in (((2, cols), (far, 1)), ((3, 2, 5, cols), (5 * cols, far, cols, 1)), ((2, 5, 3, cols), (far, cols, 5 * cols, 1)),
+                           ((5, 3, 2, cols), (cols, 5 * cols, far, 1))):
+        g = torch.Generator(device=cuda).manual_seed(11)
+        x, dy = (torch.randn(shape, generator=g, device=cuda).to(torch.bfloat16) for _ in range(2))
+        labels = torch.randint(0, cols, shape[:-1], generator=g, device=cuda)
+        labels.view(-1)[1] = -100
+        dloss = torch.rand(shape[:-1], generator=g, device=cuda).to(torch.bfloat16)
+        y, dx = torch.empty_like(x), torch.empty_like(x)
+        out = base.as_strided(shape, strides, room)
+        hk.softmax_fwd(x, y, -1)
+        hk.softmax_bwd(y, dy, dx, -1)
+        hk.softmax_bwd(y, dy, out, -1)
+        assert torch.equal(out, dx), shape
+        hk.sce_sparse_bwd(x, labels, dloss, dx, -100)
+        hk.sce_sparse_bwd(x, labels, dloss, out, -100)
+        assert torch.equal(out, dx), shape
+        fx = base.as_strided(shape, strides, 0)
+        fx.copy_(x)
+        out.zero_()
+        hk.sce_sparse_bwd(fx, labels, dloss, out, -100)
+        assert torch.equal(out, dx), shape
