@@ -925,10 +925,22 @@ template <typename T, int MODE, bool WAVE_ROW, bool RAGGED>
 static int launch_sce_nv(SceArgs given, int nv, dim3 grid, dim3 block, hipStream_t s) {
   given.threads = uint16_t(block.x);
   const SceFlat a = SceFlat::of<MODE>(given);
+  // fp32 rows of 8 vectors a thread, backward: 20 wavefronts a compute unit where rows are of any boundary or 9 or 10 wavefronts, up to
+  // which they fit twice.  56 registers would let 32 in, which the lines that rows share suffer from (us, 32 / 20; with 73 registers
+  // 24 were in): 5307 x 11001 81.2 / 78.3, 79.4, x 14001 107.4 / 100.4, 102.3, 9000 x 13001 169 / 158, 161, 1500 x 9001 20.3 / 19.8, 20.8, x
+  // 10001 22.7 / 23.4, 22.7, 620 x 18113 18.9 / 17.7, 17.3, x 18112 18.0 / 16.2, 16.2, 4000 x 20480 112.9 / 108.2, 110.5.  Whole vectors, 9000 x 9600 109.8 /
+  // 112.9 and x 15104 186.6 / 172.9, are left as they are, and so are longer rows, 620 x 21954 21.3 / 23.6, x 29229 27.9 / 30.8.
+  const auto resident = [&](int n) {
+    size_t lds = 0;
+    const int waves = int(block.x / kWave);
+    if (MODE == 1 && !WAVE_ROW && VecIO<T>::N == 4 && n == 8 && waves <= 10 && (RAGGED || waves >= 9))
+      lds_bytes_for_residency(20 / waves, sizeof(float) * kMaxWaves * 2, &lds);
+    return lds;
+  };
 #define HK_SCE_LAUNCH(N)                                                                         \
   do {                                                                                           \
     if constexpr (MODE == 0) HK_LAUNCH((sce_sparse_fwd_kernel<T, N, WAVE_ROW, RAGGED>), grid, block, 0, s, a); \
-    else if constexpr (MODE == 1) HK_LAUNCH((sce_sparse_bwd_kernel<T, N, WAVE_ROW, RAGGED>), grid, block, 0, s, a); \
+    else if constexpr (MODE == 1) HK_LAUNCH((sce_sparse_bwd_kernel<T, N, WAVE_ROW, RAGGED>), grid, block, resident(N), s, a); \
     else if constexpr (MODE == 2) HK_LAUNCH((sce_dense_kernel<T, N, WAVE_ROW, false>), grid, block, 0, s, a); \
     else HK_LAUNCH((sce_dense_kernel<T, N, WAVE_ROW, true>), grid, block, 0, s, a);       \
   } while (0)

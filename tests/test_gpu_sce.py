@@ -183,3 +183,26 @@ def test_rows_of_a_few_wavefronts(hk, cuda, dtype, vectors):
     shape = (7, vectors * (4 if dtype == "fp32" else 8))
     test_sce_sparse(hk, cuda, dtype, shape)
     test_sce_dense(hk, cuda, dtype, shape)
+
+
+@pytest.mark.parametrize("cols", [8193, 8196, 10239, 10241, 16383, 16385, 16388, 20477, 20480, 20481, 24575])
+def test_fp32_backward_of_eight_vectors_a_thread(hk, cuda, cols):
+    """5 to 12 wavefronts a row, whole vectors and any boundary, more rows than are resident at once."""
+    import torch
+    rows = 700
+    g = torch.Generator(device=cuda).manual_seed(cols)
+    x = torch.randn(rows, cols, generator=g, device=cuda) * 2
+    labels = torch.randint(0, cols, (rows,), generator=g, device=cuda)
+    labels[::7] = -100
+    dloss = torch.rand(rows, generator=g, device=cuda)
+    dx = torch.empty_like(x)
+    hk.sce_sparse_bwd(x, labels, dloss, dx, -100)
+    want = torch.softmax(x.double(), 1)
+    live = labels >= 0
+    want[live.nonzero()[:, 0], labels[live]] -= 1.0
+    want *= (dloss * live).double()[:, None]
+    # fp32: the exponent's rounding (2^-21 at magnitudes below 16), the exponential, the sum and the products; at the label of a
+    # difference of terms below 1
+    bound = 2.0 ** -19 * (want.abs() + dloss.double()[:, None] * torch.nn.functional.one_hot(labels.clamp(min=0), cols))
+    assert bool(((dx.double() - want).abs() <= bound).all())
+    assert bool((dx[~live] == 0).all())
