@@ -1017,16 +1017,19 @@ int hk_dropout_add_ln_fwd_ex(const hkDropoutAddLnFwdParams* pp, hkStream_t strea
       // Rows of four chunks a thread, 16 bits: 20 wavefronts a compute unit of the 32 that the flat arguments' 60 registers let in
       // (us, 32 / 20; the others' 72 registers, 28: bf16 3743 x 5000 32.9 / 31.6, 32.2, x 5648 38.1 / 36.0, 36.8, x 6144 38.7 / 36.6, 37.9, 7600 x
       // 5648 69.3 / 65.4, 66.6, x 7512 92.2 / 89.4, 90.3, 12000 x 5376 101.7 / 99.1, 101.9, x 6144 112.1 / 115.0, 111.3).
-      size_t resident = 0;
-      if (sizeof(A) <= kCheapArgs && sizeof(IT) == 2 && sizeof(RT) == 2)
-        lds_bytes_for_residency(std::max(1, 20 / int(block.x / kWave)), sizeof(float) * kMaxWaves * 3, &resident);
+      const auto resident = [&] {
+        size_t lds = 0;
+        if (sizeof(A) <= kCheapArgs && sizeof(IT) == 2 && sizeof(RT) == 2)
+          lds_bytes_for_residency(std::max(1, 20 / int(block.x / kWave)), sizeof(float) * kMaxWaves * 3, &lds);
+        return lds;
+      };
       switch (nc) {
         case 1:
           if (dropout) HK_LAUNCH((dal_fwd_kernel<IT, RT, WT, 1, true, A>), grid, block, 0, s, given);
           else HK_LAUNCH((dal_fwd_kernel<IT, RT, WT, 1, false, A>), grid, block, 0, s, given);
           break;
         case 2: HK_LAUNCH((dal_fwd_kernel<IT, RT, WT, 2, true, A>), grid, block, 0, s, given); break;
-        default: HK_LAUNCH((dal_fwd_kernel<IT, RT, WT, 4, true, A>), grid, block, resident, s, given); break;
+        default: HK_LAUNCH((dal_fwd_kernel<IT, RT, WT, 4, true, A>), grid, block, resident(), s, given); break;
       }
     };
     profile_before(s);
