@@ -810,32 +810,29 @@ static int softmax_strided_typed(const void* x, const void* dy, void* out, int64
                                        : dim <= 24     ? a.total >= cus * (odd ? 1024 : 2048)
                                                        : dim <= 32 && odd && bytes >= (256 << 10) && a.total >= cus * 1024);
         if (wide && dim > kDimVecs) { nk = int((dim + 1) / 2); a.slices = 2; }
-        // PLAIN: stored through the cache, where lines that two workgroups share meet.  us streamed / so, bf16, or the one over the
-        // other.  Forward in one or two slices: 60 x 5 x 263169 56.9 / 58.7, 413 x 5 x 12101 20.9 / 19.8, 1322 x 5 x 12101 61.1 / 63.5, 18 x
-        // 16 x 263169 55.7 / 58.7.  In more, odd planes of 4099 to 67311: 18 to 48 entries at 29 MiB 0.92 to 1.13, 38 MiB 0.91 to 1.00, 53 MiB 0.90
-        // to 0.94, 8 x 21 x 263169 (85 MiB) 36.2 / 33.9, 150 MiB 0.95 to 0.98; 49 to 64 at 29 MiB 1.04 to 1.14, 38 MiB 0.95 to 1.02, 53 MiB 0.91 to
-        // 0.94; 72 to 160 at 29 MiB 0.94 to 1.04, 38 MiB 0.93 to 1.06, 53 MiB 0.85 to 0.97, 44 x 150 x 12101 (152 MiB) 73.7 / 69.7.  Backward, up
-        // to 48 entries: 976 x 5 x 16384 74 / 80, 232 x 21 x 16384 75.5 / 82, 15 x 19 x 44480 15.6 / 15.0, 98 x 21 x 12101 29 / 28, 314 x 21 x 12101 85 / 89, 214 x 2
-        // x 1427 3.55 / 3.1, 17 x 11 x 52027 13.0 / 12.5.  Of more, odd planes: 49 to 96 at 13 and 19 MiB 1.02 to 1.10, 29 MiB 1.03 to 1.07, 38 MiB
-        // 0.97 to 1.03, from 53 MiB on 0.93 to 0.97; 104 to 128 at 13 MiB 0.93 to 1.01, 19 and 29 MiB 1.00 to 1.03, from 38 MiB on 0.94 to
-        // 1.00; 5 x 153 x 10427 12.5 / 13.1; 208 and 240 at 13 MiB 0.93 to 0.95, 19 MiB 0.94 to 1.03, 29 MiB 1.06 to 1.10, 38 MiB 1.03 to 1.08, from 53
-        // MiB on 0.96 to 1.00.  Whole lines: 232 x 21 x 16384 forward 52.6 / 57.4, backward of 33 to 64 entries at 13 to 29 MiB 0.94 to 1.06, 80 to 96
-        // 1.00 to 1.11, 104 to 128 0.85 to 0.95.  Planes of less than 4 KiB: 1567813 x 4 x 17 forward 188 / 180, 3043 x 26 x 1033 77 / 68, fp32, 6614 x
-        // 187 x 29, 87 / 75 and backward 135 / 121; longer ones of fp32, 2 x 193 x 21456 forward 13.0 / 14.8, 5 x 98 x 12304 backward 13.0 / 15.2.
+        // PLAIN: stored through the cache, where lines that two workgroups share meet and a call that follows may find them.  Larger arrays
+        // and planes of whole lines are streamed (streamed / so, bf16 forward: 60 x 5 x 263169 56.9 / 58.7, 413 x 5 x 12101 20.9 / 19.8, 1322 x 5 x 12101 61.1 / 63.5,
+        // 232 x 21 x 16384 52.6 / 57.4, 18 x 16 x 263169 55.7 / 58.7, 13 x 220 x 4093 15.5 / 16, 13 x 150 x 12101 25.6 / 25.1, 44 x 150 x 12101
+        // 73.7 / 69.7, 30 x 220 x 12101 89 / 85, planes of less than 4 KiB, 1567813 x 4 x 17, 188 / 180, 3043 x 26 x 1033 77 / 68; backward: 976 x 5 x 16384
+        // 74 / 80, 232 x 21 x 16384 75.5 / 82, 15 x 19 x 44480 15.6 / 15.0, 98 x 21 x 12101 29 / 28, 51 x 128 x 12101 98.6 / 103,
+        // 214 x 2 x 1427 3.55 / 3.1, 17 x 11 x 52027 13.0 / 12.5, 5 x 153 x 10427 12.5 / 13.1; fp32, 2 x 193 x 21456 forward 13.0 / 14.8,
+        // 5 x 98 x 12304 backward 13.0 / 15.2, planes of less than 4 KiB, 6614 x 187 x 29, 87 / 75 and 135 / 121).
+        // Odd planes whose forward and backward follow one another, three sets of buffers in turn: 18 to 48 entries at 35 to 62 MiB 1.00 to
+        // 1.08 of the speed with the forward streamed, at 128 to 176 MiB 1.01 to 1.09 with both streamed (13 x 21 x 271110 132 / 124, 30 x 9 x 263349 122 /
+        // 117); by itself a forward of 32 to 64 MiB takes up to 10 % longer so, and both directions up to 8 % past 128 MiB.
         const auto mib = [&](int n) { return int64_t(n) << 20; };
-        const bool plain = VEC == 8 && BWD && tall                                    ? false
-                           : odd && bytes < 4096 && (BWD || array >= mib(24))         ? true
-                           : VEC == 4                                                 ? false
-                           : BWD && many ? (dim <= 96 ? array < mib(odd ? 48 : dim > 72 ? 32 : 0) : odd && dim > 192 && array >= mib(24) && array < mib(48))
-                           : BWD         ? array < mib(odd ? 128 : 48)
-                                         : odd && (many || array < mib(128)) &&
-                                               (array >= mib(64) || (array >= mib(24) && (array < mib(32) || a.slices <= 2)));
+        const bool plain = VEC == 8 && BWD && tall                            ? false
+                           : odd && bytes < 4096 && (BWD || array >= mib(24)) ? true
+                           : VEC == 4                                         ? false
+                           : BWD && !many                                     ? odd || array < mib(48)
+                                                                              : odd && array >= mib(24) && (!BWD || array < mib(128));
         // Up to kFewSlices slices every thread merges its own values, GPU us, with slices_share / so: 64 x 10 x 12544 bf16 (2
         // slices) forward 8.3 / 7.2, 32 x 12 x 40000 11.7 / 11.1, 4 x 5 x 5904 (3) 3.7 / 3.0, 32 x 40 x 6401 (5) 10.4 / 10.2, 4 x 12 x 5904 (6) 3.6 /
         // 3.35, 16 x 60 x 30001 (8) 25.9 / 27.3.
         // What nk can be.  64 slices: 2 to 4, for 65 to 256 entries.  The few in 32: up to 6, because at 192 entries and past 16
         // vectors per compute unit they are no longer few; 1 or 2 in few slices.  32 slices of a quarter's run: 6 to 8; of half
-        // one 8, in the 16-bit backward 6.  16 of half one: forward 6 to 16, backward 4 to 8, 14 and 16.  fp32 in more than
+        // one 8, in the 16-bit backward 6.  16 of half one: forward 6 to 16, streamed,
+        // which odd planes of 24 MiB and more are not, 10, backward 4 to 8, 14 and 16.  fp32 in more than
         // six slices of 64 lanes: 7 or 8; the 16-bit backward of 37 to 48 entries on odd planes: 6.  Of those in few slices
         // through the cache, the 16-bit backward's are on odd planes or small, the fp32 forward's of 24 MiB and more in less
         // than 2048 vectors per compute unit.
@@ -864,7 +861,7 @@ static int softmax_strided_typed(const void* x, const void* dy, void* out, int64
         }
         if constexpr (VEC == 8) {
           if (many && plain) return launch_softmax_dim<T, BWD, 32, true, false, 512, kLeast, 16, kLeastAgain>(a, nk, s);
-          if (many) return launch_softmax_dim<T, BWD, 32, false, false, 512, kLeast, 16, kLeastAgain>(a, nk, s);
+          if (many) return launch_softmax_dim<T, BWD, 32, false, false, 512, kLeast, (BWD ? 16 : 10), kLeastAgain>(a, nk, s);
         }
         if constexpr (VEC == 4) {
           if (wide && a.slices == 2) return launch_softmax_dim<T, BWD, 128, false, true, 256, 5, 16>(a, nk, s);
@@ -872,8 +869,7 @@ static int softmax_strided_typed(const void* x, const void* dy, void* out, int64
           if (a.slices > kFewSlices) return launch_softmax_dim<T, BWD, 64, false, false, 1024, kDimVecs - 1, kDimVecs>(a, nk, s);
         }
         if constexpr (VEC == 8 && BWD) {
-          if (a.slices > kFewSlices && plain) return launch_softmax_dim<T, BWD, 64, true, false, 512, 6, 6>(a, nk, s);
-          if (a.slices > kFewSlices) return launch_softmax_dim<T, BWD, 64, false, false, 512, 6, 6>(a, nk, s);
+          if (a.slices > kFewSlices) return launch_softmax_dim<T, BWD, 64, true, false, 512, 6, 6>(a, nk, s);   // odd planes
         }
         if (plain) return launch_softmax_dim<T, BWD, 64, true, true, 512, kLeastPlain, kMostPlain>(a, nk, s);
         return launch_softmax_dim<T, BWD, 64, false, true, 512, 1, kDimVecs>(a, nk, s);
